@@ -1,5 +1,6 @@
 // C ABI of libtrittention_hip.so: argument checks, scratch layout, dispatch.
 // Declarations and the contract of each entry point: include/trittention_hip.h.
+#include <algorithm>
 #include <atomic>
 #include <cstdint>
 #include <cstdlib>
@@ -62,11 +63,12 @@ hipError_t ensure_dynamic_smem(const void* kernel, size_t bytes) {
 
 namespace {
 
-// Bump allocator over the caller's workspace; with base == nullptr it only measures.
+// Bump allocator over the caller's workspace; with base == nullptr it only measures (every take() is then null: what is
+// taken must never depend on what an earlier take() returned).
 struct Arena {
     char* base;
-    size_t off = 0;
-    explicit Arena(void* b) : base(static_cast<char*>(b)) {}
+    size_t capacity, off = 0;
+    explicit Arena(void* b, size_t cap = 0) : base(static_cast<char*>(b)), capacity(cap) {}
     template <typename T>
     T* take(size_t count) {
         off = (off + 255) & ~size_t(255);
@@ -75,6 +77,7 @@ struct Arena {
         return p;
     }
     size_t bytes() const { return (off + 255) & ~size_t(255); }
+    bool overflows() const { return base && off > capacity; }  // a plan that does not match its query: refuse, launch nothing
 };
 
 size_t elem_size(int dtype) { return dtype == TRITT_F32 ? 4 : 2; }
@@ -191,12 +194,22 @@ void fill_inputs(const void* q, const void* k1, const void* k2, const void* v1, 
 
 int clampw(int w, int T) { return w > T ? T : w; }
 
-// The fp32 path has two sets of kernels: on the matrix cores (v_mfma_f32_32x32x2_f32; a workgroup per 32 queries)
-// and on the vector ALUs (a wave per query: far more workgroups, the better shape for problems of a few tiles).
-bool use_f32_mfma(int BH, int T, bool backward = false) {
-    if (knobs().f32_valu) return false;
-    // the backward deals the rounds of a tile out to workgroups when the tiles alone leave the chip idle
-    return (long long)BH * ((T + 31) / 32) >= (backward ? 8 : 64);
+// The fp32 path has two sets of kernels: on the matrix cores (v_mfma_f32_32x32x2_f32; D = 32, 64 and 128), which deal the
+// rounds of a query tile out over workgroups and are the faster ones at every size (B=1 H=1 T=16 D=64: forward 14 against
+// 27 us, backward 32 against 200 us), and on the vector ALUs (D = 8 and 16, and TRITT_TUNE_F32_VALU).
+bool use_f32_mfma() { return knobs().f32_valu == 0; }
+// room for the parts of a split fp32 matrix-core forward; a problem whose other scratch fits the library's static buffer
+// (tritt_tdp_fwd_static_scratch) takes no more parts than still fit
+void plan_f32_parts(Arena& ar, GenericTdpArgs& a) {
+    a.fwd_parts = 1;
+    a.part = nullptr;
+    if (!f32_mfma_tdp_supported(a.D) || !use_f32_mfma()) return;
+    const size_t per_part = (size_t)a.BH * a.T * f32_fwd_part_floats(a.D) * sizeof(float), used = ar.bytes();
+    size_t parts = (size_t)f32_fwd_parts(a);
+    if (used <= TRITT_STATIC_SCRATCH_BYTES) parts = std::min(parts, (TRITT_STATIC_SCRATCH_BYTES - used) / per_part);
+    if (parts < 2) return;
+    a.fwd_parts = (int)parts;
+    a.part = ar.take<float>(parts * per_part / sizeof(float));
 }
 
 // ---------------------------------------------------------------- triple-dot, fp32 VALU path
@@ -207,15 +220,22 @@ int tdp_fwd_generic(Arena& ar, bool run, const void* q, const void* k1, const vo
     float *copies[4], *u;
     F32Inputs in = plan_inputs(ar, q, k1, k2, v2, n, dtype, copies, &u);
     float* o32 = dtype == TRITT_F32 ? (float*)o : ar.take<float>(n);
-    if (!run) return TRITT_OK;
-    fill_inputs(q, k1, k2, v1, v2, n, dtype, copies, u, st);
     GenericTdpArgs a{};
-    a.q = in.q; a.k1 = in.k1; a.k2 = in.k2; a.u = in.u; a.v2 = in.v2;
-    a.o = o32; a.lse = lse;
     a.BH = B * H; a.T = T; a.D = D; a.alpha = alpha;
     a.causal = causal; a.k1_window = w1; a.k2_window = w2; a.kk_left = kl; a.kk_right = kr;
-    // fp32 on the matrix cores where a kernel exists (D = 32, 64), fp32 VALU kernels otherwise
-    hipError_t e = (f32_mfma_tdp_supported(D) && use_f32_mfma(B * H, T)) ? f32_mfma_tdp_fwd(a, st) : generic_tdp_fwd(a, st);
+    plan_f32_parts(ar, a);
+    if (!run) return TRITT_OK;
+    if (ar.overflows()) return TRITT_ERR_WORKSPACE;
+    const bool mfma32 = f32_mfma_tdp_supported(D) && use_f32_mfma();
+    a.q = in.q; a.k1 = in.k1; a.k2 = in.k2; a.u = in.u; a.v2 = in.v2;
+    a.o = o32; a.lse = lse;
+    if (mfma32 && dtype == TRITT_F32 && f32_fwd_takes_v1(a)) {
+        a.u = (const float*)v1;
+        a.u_is_v1 = 1;
+    } else {
+        fill_inputs(q, k1, k2, v1, v2, n, dtype, copies, u, st);
+    }
+    hipError_t e = mfma32 ? f32_mfma_tdp_fwd(a, st) : generic_tdp_fwd(a, st);
     if (e != hipSuccess) return (int)e;
     if (dtype != TRITT_F32) from_f32(o32, nullptr, o, n, dtype, st);
     return (int)hipGetLastError();
@@ -226,55 +246,67 @@ int tdp_bwd_generic(Arena& ar, bool run, const void* q, const void* k1, const vo
                     void* dk2, void* dv1, void* dv2, int B, int H, int T, int D, int dtype, float alpha, int causal,
                     int w1, int w2, int kl, int kr, hipStream_t st) {
     const size_t n = (size_t)B * H * T * D;
+    const bool mfma32 = f32_mfma_tdp_supported(D) && use_f32_mfma();
     float *copies[4], *u;
     F32Inputs in = plan_inputs(ar, q, k1, k2, v2, n, dtype, copies, &u);
     float* do32 = dtype == TRITT_F32 ? (float*)d_o : ar.take<float>(n);
     float* delta = ar.take<float>((size_t)B * H * T);
-    float* du = ar.take<float>(n);
-    // fp32 results: the caller's tensors when they are fp32, scratch otherwise; `spare` stands in for the
-    // unwanted (null) half of a gradient pair whose other half is wanted (one kernel writes both halves)
-    float *dq32 = (float*)dq, *dk132 = (float*)dk1, *dk232 = (float*)dk2, *dv232 = (float*)dv2;
-    float* spare = nullptr;
-    if (dtype != TRITT_F32) {
-        dq32 = ar.take<float>(n); dk132 = ar.take<float>(n); dk232 = ar.take<float>(n); dv232 = ar.take<float>(n);
-    } else {
-        spare = ar.take<float>(n);
-    }
-    long long* fixed = f32_mfma_tdp_supported(D) ? ar.take<long long>(f32_mfma_tdp_bwd_scratch_elems(B * H, T, D)) : nullptr;
     // 16-bit tensors on the fp32 path: the output and the log-sum-exp are formed once more in fp32, because Delta =
     // rowsum(dO * O) from the stored 16-bit output carries that output's rounding, which nearly one-hot softmax
     // rows (large scores, first causal rows) turn into gradient errors far above it
     float* o32 = dtype != TRITT_F32 ? ar.take<float>(n) : nullptr;
     float* lse32 = dtype != TRITT_F32 ? ar.take<float>((size_t)B * H * T) : nullptr;
+    GenericTdpArgs a{};
+    a.BH = B * H; a.T = T; a.D = D; a.alpha = alpha;
+    a.causal = causal; a.k1_window = w1; a.k2_window = w2; a.kk_left = kl; a.kk_right = kr;
+    if (dtype != TRITT_F32) plan_f32_parts(ar, a);  // (o32 is null while measuring)
+    long long* fixed = mfma32 ? ar.take<long long>(f32_mfma_tdp_bwd_scratch_elems(B * H, T, D)) : nullptr;
+    // VALU kernels: fp32 results, the caller's tensors when they are fp32, scratch otherwise; `spare` stands in for the
+    // unwanted (null) half of a gradient pair whose other half is wanted (one kernel writes both halves)
+    float *dq32 = (float*)dq, *dk132 = (float*)dk1, *dk232 = (float*)dk2, *dv232 = (float*)dv2;
+    float *spare = nullptr, *du = nullptr;
+    if (!mfma32) {
+        du = ar.take<float>(n);
+        if (dtype != TRITT_F32) {
+            dq32 = ar.take<float>(n); dk132 = ar.take<float>(n); dk232 = ar.take<float>(n); dv232 = ar.take<float>(n);
+        } else {
+            spare = ar.take<float>(n);
+        }
+    }
     if (!run) return TRITT_OK;
+    if (ar.overflows()) return TRITT_ERR_WORKSPACE;
+    if (dtype != TRITT_F32 || !mfma32) fill_inputs(q, k1, k2, v1, v2, n, dtype, copies, u, st);
+    if (dtype != TRITT_F32) to_f32<false>(d_o, do32, n, dtype, st);
+    a.q = in.q; a.k1 = in.k1; a.k2 = in.k2; a.u = in.u; a.v2 = in.v2;
+    if (o32) {
+        a.o = o32; a.lse = lse32;
+        hipError_t ef = mfma32 ? f32_mfma_tdp_fwd(a, st) : generic_tdp_fwd(a, st);
+        if (ef != hipSuccess) return (int)ef;
+        lse = lse32;
+    }
+    a.lse_in = lse; a.d_o = do32;
+    if (mfma32) {
+        F32BwdCall c{};
+        c.a = a; c.o = o32 ? o32 : (const float*)o;
+        c.v1_f32 = dtype == TRITT_F32 ? (const float*)v1 : nullptr; c.u_out = u;
+        c.delta = delta; c.scratch = fixed; c.v1 = v1;
+        c.dq = dq; c.dk1 = dk1; c.dk2 = dk2; c.dv1 = dv1; c.dv2 = dv2;
+        c.elem = dtype == TRITT_F32 ? 0 : dtype == TRITT_BF16 ? 1 : 2;
+        return (int)f32_mfma_tdp_bwd(c, st);
+    }
+    if (o32) rowdot(do32, o32, delta, B * H * T, D, TRITT_F32, st);
+    else rowdot(d_o, o, delta, B * H * T, D, dtype, st);
+    a.delta = delta;
     const bool want_k2 = dk2 || dv2, want_k1 = dk1 || dv1;
     if (dtype == TRITT_F32) {
         if (want_k2 && !dk2) dk232 = spare;
         if (want_k2 && !dv2) dv232 = spare;
         if (want_k1 && !dk1) dk132 = spare;
     }
-    fill_inputs(q, k1, k2, v1, v2, n, dtype, copies, u, st);
-    if (dtype != TRITT_F32) to_f32<false>(d_o, do32, n, dtype, st);
-    GenericTdpArgs a{};
-    a.q = in.q; a.k1 = in.k1; a.k2 = in.k2; a.u = in.u; a.v2 = in.v2;
-    a.BH = B * H; a.T = T; a.D = D; a.alpha = alpha;
-    a.causal = causal; a.k1_window = w1; a.k2_window = w2; a.kk_left = kl; a.kk_right = kr;
-    const bool mfma32 = fixed && use_f32_mfma(B * H, T, true);
-    if (o32) {
-        a.o = o32; a.lse = lse32;
-        hipError_t ef = (fixed && use_f32_mfma(B * H, T)) ? f32_mfma_tdp_fwd(a, st) : generic_tdp_fwd(a, st);
-        if (ef != hipSuccess) return (int)ef;
-        rowdot(do32, o32, delta, B * H * T, D, TRITT_F32, st);
-        lse = lse32;
-    } else {
-        rowdot(d_o, o, delta, B * H * T, D, dtype, st);
-    }
-    a.lse_in = lse; a.d_o = do32; a.delta = delta;
     a.dq = dq ? dq32 : nullptr;
     a.dk2 = want_k2 ? dk232 : nullptr; a.dv2 = want_k2 ? dv232 : nullptr;
     a.dk1 = want_k1 ? dk132 : nullptr; a.du = want_k1 ? du : nullptr;
-    hipError_t e = mfma32 ? f32_mfma_tdp_bwd(a, fixed, st) : generic_tdp_bwd(a, st);
-    if (e != hipSuccess) return (int)e;
+    if (hipError_t e = generic_tdp_bwd(a, st); e != hipSuccess) return (int)e;
     if (dv1) from_f32(du, v1, dv1, n, dtype, st);
     if (dtype != TRITT_F32) {
         if (dq) from_f32(dq32, nullptr, dq, n, dtype, st);
@@ -302,6 +334,7 @@ int dps_fwd_impl(Arena& ar, bool run, const void* q, const void* k1, const void*
     a.w = ar.take<float>(n);
     a.lse1 = ar.take<float>(rows);
     if (!run) return TRITT_OK;
+    if (ar.overflows()) return TRITT_ERR_WORKSPACE;
     fill_inputs(q, k1, k2, v1, v2, n, dtype, copies, u, st);
     a.q = in.q; a.k1 = in.k1; a.k2 = in.k2; a.u = in.u; a.v2 = in.v2;
     a.o = o32; a.lse = lse;
@@ -336,6 +369,7 @@ int dps_bwd_impl(Arena& ar, bool run, const void* q, const void* k1, const void*
     float* o32 = dtype != TRITT_F32 ? ar.take<float>(n) : nullptr;
     float* lse32 = dtype != TRITT_F32 ? ar.take<float>(rows) : nullptr;
     if (!run) return TRITT_OK;
+    if (ar.overflows()) return TRITT_ERR_WORKSPACE;
     fill_inputs(q, k1, k2, v1, v2, n, dtype, copies, u, st);
     if (dtype != TRITT_F32) to_f32<false>(d_o, do32, n, dtype, st);
     a.q = in.q; a.k1 = in.k1; a.k2 = in.k2; a.u = in.u; a.v2 = in.v2;
@@ -594,7 +628,7 @@ int tritt_tdp_fwd(const void* q, const void* k1, const void* k2, const void* v1,
         a.alpha = alpha;
         return (int)mfma_tdp_fwd(a, (hipStream_t)stream);
     }
-    Arena ar(workspace);
+    Arena ar(workspace, workspace_bytes);
     return tdp_fwd_generic(ar, true, q, k1, k2, v1, v2, o, lse, B, H, T, D, dtype, alpha, causal, w1, w2, kl, kr,
                            (hipStream_t)stream);
 }
@@ -662,7 +696,7 @@ int tritt_tdp_bwd(const void* q, const void* k1, const void* k2, const void* v1,
         a.split = use_split(D, dtype, flags) ? 1 : 0;
         return (int)mfma_tdp_bwd(a, (hipStream_t)stream);
     }
-    Arena ar(workspace);
+    Arena ar(workspace, workspace_bytes);
     return tdp_bwd_generic(ar, true, q, k1, k2, v1, v2, o, lse, d_o, dq, dk1, dk2, dv1, dv2, B, H, T, D, dtype, alpha,
                            causal, w1, w2, kl, kr, (hipStream_t)stream);
 }
@@ -697,7 +731,7 @@ int tritt_dps_fwd(const void* q, const void* k1, const void* k2, const void* v1,
         a.is_bf16 = dtype == TRITT_BF16;
         return (int)mfma_dps_fwd(a, (hipStream_t)stream);
     }
-    Arena ar(workspace);
+    Arena ar(workspace, workspace_bytes);
     return dps_fwd_impl(ar, true, q, k1, k2, v1, v2, o, lse, B, H, T, D, dtype, alpha, causal, clampw(k_diff, T),
                         (hipStream_t)stream);
 }
@@ -734,7 +768,7 @@ int tritt_dps_bwd(const void* q, const void* k1, const void* k2, const void* v1,
         a.is_bf16 = dtype == TRITT_BF16;
         return (int)mfma_dps_bwd(a, (hipStream_t)stream);
     }
-    Arena ar(workspace);
+    Arena ar(workspace, workspace_bytes);
     return dps_bwd_impl(ar, true, q, k1, k2, v1, v2, o, lse, d_o, dq, dk1, dk2, dv1, dv2, B, H, T, D, dtype, alpha,
                         causal, clampw(k_diff, T), (hipStream_t)stream);
 }

@@ -43,17 +43,36 @@ struct GenericTdpArgs {
     int BH, T, D;
     float alpha;
     int causal, k1_window, k2_window, kk_left, kk_right;
+    // fp32 MFMA forward: workgroups per query tile at most (f32_fwd_parts) and, above 1, room for that many parts per row
+    int fwd_parts;
+    float* part;
+    int u_is_v1;  // forward: `u` is V1 and the kernel applies SiLU (where f32_fwd_takes_v1 says it may)
 };
 hipError_t generic_tdp_fwd(const GenericTdpArgs& a, hipStream_t st);
 hipError_t generic_tdp_bwd(const GenericTdpArgs& a, hipStream_t st);
 
 // fp32 MFMA triple-dot kernels (D = 32 or 64, any mask): same operands as the VALU kernels
 bool f32_mfma_tdp_supported(int D);
+// workgroups per query tile that the forward of this problem is dealt out to (BH, T, D and the mask of `a`)
+int f32_fwd_parts(const GenericTdpArgs& a);
+bool f32_fwd_takes_v1(const GenericTdpArgs& a);
+size_t f32_fwd_part_floats(int D);  // scratch per row and part
 hipError_t f32_mfma_tdp_fwd(const GenericTdpArgs& a, hipStream_t st);
-// backward: `scratch` = f32_mfma_tdp_bwd_scratch_elems() 64-bit words (fixed-point accumulators of the four
-// key / value gradients; zeroed by the call)
+// The backward: `a` holds the fp32 operands (u: written by the call when v1_f32 is given), lse_in and d_o; the gradients come
+// out in the caller's type.
+struct F32BwdCall {
+    GenericTdpArgs a;
+    const float* o;       // fp32 output of the forward
+    const float* v1_f32;  // with u_out = a.u: fp32 V1, whose SiLU the call forms; null: a.u is there already
+    float* u_out;
+    float* delta;         // scratch [BH, T]
+    long long* scratch;   // f32_mfma_tdp_bwd_scratch_elems() 64-bit words: fixed-point accumulators and what belongs to them
+    const void* v1;       // V1 in the caller's type (SiLU')
+    void *dq, *dk1, *dk2, *dv1, *dv2;  // null: not wanted
+    int elem;             // the caller's type: 0 float, 1 bf16, 2 f16
+};
 size_t f32_mfma_tdp_bwd_scratch_elems(int BH, int T, int D);
-hipError_t f32_mfma_tdp_bwd(const GenericTdpArgs& a, long long* scratch, hipStream_t st);
+hipError_t f32_mfma_tdp_bwd(const F32BwdCall& c, hipStream_t st);
 
 // The first `tiles` query tiles (32 queries each) of a 16-bit triple-dot backward, computed in fp32 from the
 // 16-bit tensors (D = 32, 64 or 128) and added to the accumulators of the 16-bit MFMA backward, which then starts
@@ -80,14 +99,9 @@ struct FirstTileArgs {
     int causal, k1_window, k2_window, kk_left, kk_right;
     bool want_q, want_k2, want_k1;
     int tiles;
-    int round_parts;  // tiles > 1: workgroups per query tile (its rounds of eight rows dealt out); above 1 needs acc_q when dQ is wanted
+    bool split_rounds;  // tiles > 1: the rounds (of eight rows) of a query tile may be dealt out to workgroups; needs acc_q when dQ is wanted
 };
 hipError_t f32_mfma_tdp_bwd_first_tile(const FirstTileArgs& a, hipStream_t st);
-// Workgroups per query tile of the fp32 matrix-core backward over all tiles: one workgroup walks a tile's rounds (of
-// eight rows) one after another, so a grid that leaves most compute units idle (short sequences, few heads) is
-// dealt out by rounds as well.
-int f32_round_parts(int BH, int T);
-
 // fp32 operands of the dot-product-sum kernels (two chained attention passes).
 struct DpsArgs {
     const float *q, *k1, *k2, *u, *v2;

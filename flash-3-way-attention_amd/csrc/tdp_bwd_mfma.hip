@@ -854,7 +854,7 @@ static hipError_t launch_bwd(const MfmaBwdArgs& a, hipStream_t st) {
         f.k1_window = a.k1_window; f.k2_window = a.k2_window; f.kk_left = a.kk_left; f.kk_right = a.kk_right;
         f.want_q = want_q; f.want_k2 = want_k2; f.want_k1 = want_k1;
         f.tiles = all_in_f32 ? p.nqt : 1;
-        f.round_parts = (dqacc || !want_q) ? std::min(splits, f32_round_parts(a.BH, a.T)) : 1;
+        f.split_rounds = dqacc || !want_q;
         if constexpr (D == 64) {
             if (plain64 && !all_in_f32 && p.nqt > 1 && (want_q || want_k2 || want_k1)) {
                 if (hipError_t e = tile0_prepare<E, 64>(f, st, t0_r0, t0_r1, t0_roles, t0_rounds); e != hipSuccess) return e;

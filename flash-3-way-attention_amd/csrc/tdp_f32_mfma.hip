@@ -5,8 +5,10 @@
 // All tensors here are fp32 [BH, T, D]; U = SiLU(V1) (see capi.hip).
 //
 // Formulation (the same virtual-query one as the 16-bit kernels).  A workgroup owns 32 consecutive queries;
-// its eight waves take eight consecutive rows b per round (one per wave; b = k, the K2 / V2 row, in the
-// natural orientation) and sweep the streamed index a (= j, K1 / U rows) in 32-row stages shared through LDS.
+// its waves take consecutive rows b per round (one per wave; b = k, the K2 / V2 row, in the natural orientation) and
+// sweep the streamed index a (= j, K1 / U rows) in 32-row stages shared through LDS.  The rounds of a tile are dealt out
+// over several workgroups by their cost (F32Deal): the forward's parts are joined by f32_merge_kernel, the backward's
+// meet in fixed-point accumulators.
 // For a fixed row b the scores of the 32 queries against 32 streamed rows are one 32x32 tile
 //   S^T[a, q] = sum_d KA[a, d] * (scale * Q[q, d] * KB[b, d])
 // i.e. D / 2 MFMAs (K = 2 each).  The tile leaves the MFMA with lane <-> query and registers <-> streamed rows,
@@ -14,8 +16,7 @@
 //   Tv^T[d, q] += sum_a VA^T[d, a] * P^T[a, q]
 // so P is never moved between lanes, and every per-query quantity (running maximum, row sum, the merge of a
 // finished row b into the output, O^T[d, q] += Tv^T[d, q] * VB[b, d]) is lane-local.
-// With 64-cycle MFMAs the kernels are bound by the matrix pipe; the element-wise work (mask predicate on every
-// element, online softmax) hides under it, so there is one loop body for every mask.
+// One loop body serves every mask; only tiles on its edge evaluate it.
 #include <algorithm>
 
 #include "common.hpp"
@@ -26,114 +27,227 @@
 namespace tritt {
 namespace {
 
-__global__ __launch_bounds__(256) void f32_zero_kernel(long long* __restrict__ a, size_t n) {
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) a[i] = 0;
-}
-// the partial maxima of |dO| that fix the scale of a slice's accumulators: grid (kScaleParts, BH)
-__global__ __launch_bounds__(256) void f32_scale_kernel(const float* __restrict__ d_o, unsigned* __restrict__ parts,
-                                                        size_t per_slice) {
+// One pass ahead of the backward kernels, 64 rows per workgroup: U = SiLU(V1) (u null: the caller has it), Delta =
+// rowsum(dO * O), the partial maxima of |dO| that fix the scale of a slice's accumulators, and the accumulators and poison
+// words cleared.  Five launches of 2-5 us each without it; grid (64-row blocks, BH).
+template <int D>
+__global__ __launch_bounds__(256) void f32_prep_kernel(const float* __restrict__ v1, float* __restrict__ u,
+                                                       const float* __restrict__ o, const float* __restrict__ d_o,
+                                                       float* __restrict__ delta, long long* __restrict__ acc, size_t n,
+                                                       unsigned* __restrict__ scale_parts, unsigned* __restrict__ poison, int T) {
     __shared__ unsigned red[4];
-    const size_t pieces = per_slice / 4, per_part = (pieces + kScaleParts - 1) / kScaleParts;
-    const size_t lo = min(pieces, blockIdx.x * per_part), hi = min(pieces, lo + per_part);
-    const unsigned m = block_absmax_bits<float>(d_o + blockIdx.y * per_slice + lo * 4, hi - lo, red);
-    if (threadIdx.x == 0) parts[blockIdx.y * kScaleParts + blockIdx.x] = m;
-}
-// fixed point -> fp32, one tensor (dQ / alpha accumulated over the workgroups of a tile)
-__global__ __launch_bounds__(256) void f32_finish_q_kernel(const long long* __restrict__ acc, float* __restrict__ dq, size_t n,
-                                                           int T, int D, const unsigned* __restrict__ scale_parts,
-                                                           const unsigned* __restrict__ poison, float alpha) {
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
-        const size_t row = i / D;
-        const double inv = fixed_scale_inverse(fixed_scale_field<false>(scale_parts, (int)(row / T), kF32FixedBias));
-        dq[i] = (poison[row] & kPoisonDQ) ? __builtin_nanf("") : (float)((double)acc[i] * inv) * alpha;
+    constexpr int kPieces = D / 4;
+    const int bh = blockIdx.y, j0 = blockIdx.x * 64;
+    const size_t base = (size_t)bh * T * D;
+    if (threadIdx.x < 64 && j0 + threadIdx.x < T) poison[(size_t)bh * T + j0 + threadIdx.x] = 0;
+    // part s of a slice: its 64-row blocks s, s + kScaleParts, ...
+    for (int part = blockIdx.x; part < kScaleParts; part += gridDim.x) {
+        unsigned m = 0;
+        for (int r0 = part * 64; r0 < T; r0 += kScaleParts * 64)
+            m = max(m, block_absmax_bits<float>(d_o + base + (size_t)r0 * D, (size_t)min(64, T - r0) * kPieces, red));
+        if (threadIdx.x == 0) scale_parts[bh * kScaleParts + part] = m;
+    }
+    for (int idx = threadIdx.x; idx < 64 * kPieces; idx += 256) {  // whole waves: 64 kPieces is a multiple of 256
+        const int j = j0 + idx / kPieces;
+        const size_t off = base + (size_t)j * D + (idx % kPieces) * 4;
+        float dot = 0.f;
+        if (j < T) {
+            if (u) {
+                f32x4v x = *reinterpret_cast<const f32x4v*>(v1 + off);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[e] = silu_f(x[e]);
+                *reinterpret_cast<f32x4v*>(u + off) = x;
+            }
+            const f32x4v x = *reinterpret_cast<const f32x4v*>(o + off), y = *reinterpret_cast<const f32x4v*>(d_o + off);
+            dot = x[0] * y[0] + x[1] * y[1] + (x[2] * y[2] + x[3] * y[3]);
+            const longlong2 z = make_longlong2(0, 0);
+#pragma unroll
+            for (int t = 0; t < 5; ++t) {
+                longlong2* p = reinterpret_cast<longlong2*>(acc + t * n + off);
+                p[0] = z;
+                p[1] = z;
+            }
+        }
+#pragma unroll
+        for (int w = kPieces / 2; w > 0; w >>= 1) dot += __shfl_xor(dot, w, 64);
+        if (idx % kPieces == 0 && j < T) delta[(size_t)bh * T + j] = dot;
     }
 }
-// fixed point -> fp32
-__global__ __launch_bounds__(256) void f32_finish_kernel(const long long* __restrict__ acc, float* __restrict__ dk_rows,
-                                                         float* __restrict__ dv_rows, size_t n, int T, int D,
+// fixed point -> the gradients (null: not wanted); dV1 = dU SiLU'(V1), dQ = alpha times its sum.  Four elements per thread.
+template <typename E>
+__global__ __launch_bounds__(256) void f32_finish_kernel(const long long* __restrict__ acc, const E* __restrict__ v1,
+                                                         E* __restrict__ dq, E* __restrict__ dk1, E* __restrict__ dk2,
+                                                         E* __restrict__ dv1, E* __restrict__ dv2, size_t n, int T, int D,
                                                          const unsigned* __restrict__ scale_parts,
-                                                         const unsigned* __restrict__ poison, unsigned bit_k,
-                                                         unsigned bit_v) {
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
+                                                         const unsigned* __restrict__ poison, float alpha) {
+    typedef __attribute__((ext_vector_type(4))) E e4;
+    for (size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4; i < n; i += (size_t)gridDim.x * 1024) {
         const size_t row = i / D;
         const double inv = fixed_scale_inverse(fixed_scale_field<false>(scale_parts, (int)(row / T), kF32FixedBias));
         const unsigned bad = poison[row];
-        dk_rows[i] = (bad & bit_k) ? __builtin_nanf("") : (float)((double)acc[i] * inv);
-        dv_rows[i] = (bad & bit_v) ? __builtin_nanf("") : (float)((double)acc[n + i] * inv);
+        auto put = [&](E* out, int which, unsigned bit, auto factor) {
+            if (!out) return;
+            const longlong2* p = reinterpret_cast<const longlong2*>(acc + which * n + i);
+            const longlong2 lo = p[0], hi = p[1];
+            const long long v[4] = {lo.x, lo.y, hi.x, hi.y};
+            e4 r;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                r[e] = (E)(((bad & bit) ? __builtin_nanf("") : (float)((double)v[e] * inv)) * factor(e));
+            *reinterpret_cast<e4*>(out + i) = r;
+        };
+        auto one = [](int) { return 1.0f; };
+        put(dk2, 0, kPoisonDK2, one);
+        put(dv2, 1, kPoisonDV2, one);
+        put(dk1, 2, kPoisonDK1, one);
+        if (dv1) {
+            const e4 x = *reinterpret_cast<const e4*>(v1 + i);
+            put(dv1, 3, kPoisonDU, [&](int e) { return silu_grad_f((float)x[e]); });
+        }
+        put(dq, 4, kPoisonDQ, [&](int) { return alpha; });
     }
+}
+
+// waves per workgroup
+constexpr int f32_fwd_waves(int D) { return D > 64 ? 8 : 4; }
+constexpr int f32_bwd_waves(int D) { return D > 64 ? 8 : 4; }
+
+// Joins the parts of a split forward, four columns per thread.
+__global__ __launch_bounds__(256) void f32_merge_kernel(const float* __restrict__ part, float* __restrict__ o,
+                                                        float* __restrict__ lse, size_t rows, int T, int D, TdpMask mask,
+                                                        F32Deal deal) {
+    const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x, row = idx / (D / 4);
+    const int d = (int)(idx % (D / 4)) * 4;
+    if (row >= rows) return;
+    const int parts = f32_tile_parts(deal, mask, (int)(row % T) / 32, T, f32_fwd_waves(D));
+    const float* src = part + row * deal.max_parts * (D + 4);
+    // four parts' loads in flight at a time (a part beyond the last one repeats it with weight zero)
+    float m = kNegBig, l = 0.f;
+    f32x4v acc = {0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < parts; s0 += 4) {
+        float ms[4], ls[4];
+        f32x4v os[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const float* at = src + min(s0 + k, parts - 1) * (D + 4);
+            ms[k] = s0 + k < parts ? at[D] : kNegBig;
+            ls[k] = at[D + 1];
+            os[k] = *reinterpret_cast<const f32x4v*>(at + d);
+        }
+        const float top = fmaxf(fmaxf(fmaxf(ms[0], ms[1]), fmaxf(ms[2], ms[3])), m), keep = fast_exp2(m - top);
+        l *= keep;
+        acc *= keep;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const float w = fast_exp2(ms[k] - top);
+            l += w * ls[k];
+            acc += os[k] * w;
+        }
+        m = top;
+    }
+    *reinterpret_cast<f32x4v*>(o + row * D + d) = acc / l;
+    if (d == 0) lse[row] = (m + fast_log2(l)) * kLn2;
+}
+
+// How the tiles of a problem are dealt out over workgroups.  `slots`: workgroups the chip holds at a time.  About six parts per
+// slot even out a grid whose tiles differ by a factor of hundreds (B=4 H=8 T=512: one workgroup per tile 5.9 ms, a fixed
+// count of 4 / 16 per tile 4.1 / 3.9, by cost 3.3); below sixteen steps per slot a part's own cost (prologue, merge: two
+// or three steps' worth) asks for fewer, two per slot; a problem smaller than that gets one step per part (B=1 H=2 T=64
+// D=32: 27 -> 9 us).  At most sixteen parts per tile: 32 gained nothing and double the scratch of a split forward.
+F32Deal f32_deal(const TdpMask& mask, int BH, int T, int nw, int slots, int most) {
+    const int nqt = (T + 31) / 32;
+    long long total = 0;
+    int rounds;
+    for (int qt = 0; qt < nqt; ++qt) total += f32_tile_steps(mask, qt * 32, std::min(T - 1, qt * 32 + 31), T, nw, &rounds);
+    const double per_slot = (double)total * BH / slots;
+    const double target = std::max({per_slot / 6.0, std::min(16.0, per_slot / 2.0), 1.0});
+    F32Deal d{(float)(1.0 / target), most, 0};
+    int parts = 1;
+    for (int qt = 0; qt < nqt; ++qt) parts = std::max(parts, f32_tile_parts(d, mask, qt, T, nw));
+    d.max_parts = parts;
+    for (int qt = 0; qt < nqt; ++qt) d.items += f32_tile_parts(d, mask, qt, T, nw);
+    return d;
+}
+F32Deal f32_bwd_deal(int BH, int T, int D, const TdpMask& mask) {
+    const int nw = f32_bwd_waves(D);
+    return f32_deal(mask, BH, T, nw, nw == 4 ? 512 : 256, knobs().bwd_splits > 0 ? std::min(knobs().bwd_splits, 16) : 16);
 }
 
 // both launches of the backward over query tiles 0 .. nqt - 1
 template <typename E, int D>
 hipError_t launch_f32_bwd_tiles(F32BwdParams<E> p, const E* k1, const E* u, const E* k2, const E* v2, void* acc_k2,
                                 void* acc_v2, void* acc_k1, void* acc_u, const TdpMask& natural, bool want_q,
-                                bool want_k2, bool want_k1, hipStream_t st, const InputsAt& at) {
+                                bool want_k2, bool want_k1, hipStream_t st, const InputsAt& at, bool split) {
     // a workgroup holds all D gradient columns and forms S and dP once (D = 128: dQ's running sum is kept in LDS)
-    constexpr int DOUT = D, DOUT_NODQ = D;
-    auto kern_dq = tdp_f32_bwd_kernel<E, D, DOUT, true>;
-    auto kern_nodq = tdp_f32_bwd_kernel<E, D, DOUT_NODQ, false>;
-    constexpr size_t smem = f32_bwd_smem<D>();
-    static_assert(DOUT * 33 <= 4 * 32 * (D + 1), "dQ of the tile aliases the stage buffers (D <= 64)");
+    constexpr int DOUT = D;
+    constexpr int NW = f32_bwd_waves(D);
+    auto kern_dq = tdp_f32_bwd_kernel<E, D, DOUT, true, NW>;
+    auto kern_nodq = tdp_f32_bwd_kernel<E, D, DOUT, false, NW>;
+    constexpr size_t smem = f32_bwd_smem<D, NW>();
     if (hipError_t e = ensure_dynamic_smem(reinterpret_cast<const void*>(kern_dq), smem); e != hipSuccess) return e;
     if (hipError_t e = ensure_dynamic_smem(reinterpret_cast<const void*>(kern_nodq), smem); e != hipSuccess) return e;
-    // small grids: the rounds of a tile dealt out to several workgroups (the launch with dQ only when dQ has an accumulator)
-    const int parts = std::max(1, p.round_parts);
-    const dim3 grid(8 * xcd_slots(p.BH, p.nqt), D / DOUT, p.acc_q ? parts : 1), grid_nodq(8 * xcd_slots(p.BH, p.nqt), D / DOUT_NODQ, parts);
+    // The rounds of a tile are dealt out to several workgroups (the launch with dQ: only when dQ has an accumulator).  The list
+    // of parts belongs to the mask it was made for, and the second launch exchanges the two key indices.
+    const TdpMask exchanged{natural.causal, natural.wb, natural.wa, natural.rab, natural.lab};
+    const F32Deal whole{0.f, 1, p.nqt};
+    auto deal_for = [&](const TdpMask& m) { return split ? f32_bwd_deal(p.BH, p.T, D, m) : whole; };
+    auto grid_of = [&](const F32Deal& d) { return dim3(8 * xcd_slots(p.BH, d.items), D / DOUT); };
     // rows = (K2, V2), streamed = (K1, U): dQ, dK2, dV2
     p.ka = k1; p.va = u; p.kb = k2; p.vb = v2;
     place_inputs(p, at, false);
     p.acc_k = acc_k2; p.acc_v = acc_v2; p.bit_k = kPoisonDK2; p.bit_v = kPoisonDV2;
     p.mask = natural;
-    if (want_q) hipLaunchKernelGGL(kern_dq, grid, dim3(512), smem, st, p);
-    else if (want_k2) hipLaunchKernelGGL(kern_nodq, grid_nodq, dim3(512), smem, st, p);
+    p.deal = want_q && !p.acc_q ? whole : deal_for(natural);
+    if (want_q) hipLaunchKernelGGL(kern_dq, grid_of(p.deal), dim3(64 * NW), smem, st, p);
+    else if (want_k2) hipLaunchKernelGGL(kern_nodq, grid_of(p.deal), dim3(64 * NW), smem, st, p);
     // rows = (K1, U), streamed = (K2, V2): dK1, dU (the mask with the two key indices exchanged)
     p.ka = k2; p.va = v2; p.kb = k1; p.vb = u;
     place_inputs(p, at, true);
     p.acc_k = acc_k1; p.acc_v = acc_u; p.bit_k = kPoisonDK1; p.bit_v = kPoisonDU;
-    p.mask = TdpMask{natural.causal, natural.wb, natural.wa, natural.rab, natural.lab};
-    if (want_k1) hipLaunchKernelGGL(kern_nodq, grid_nodq, dim3(512), smem, st, p);
+    p.mask = exchanged;
+    p.deal = deal_for(exchanged);
+    if (want_k1) hipLaunchKernelGGL(kern_nodq, grid_of(p.deal), dim3(64 * NW), smem, st, p);
     return hipGetLastError();
 }
 
 template <int D>
-hipError_t launch_f32_bwd(const GenericTdpArgs& a, long long* acc, hipStream_t st) {
-    const size_t n = (size_t)a.BH * a.T * D;
-    const bool want_q = a.dq != nullptr, want_k2 = a.dk2 && a.dv2, want_k1 = a.dk1 && a.du;
+hipError_t launch_f32_bwd(const F32BwdCall& c, hipStream_t st) {
+    const GenericTdpArgs& a = c.a;
+    const size_t n = (size_t)a.BH * a.T * D, rows = (size_t)a.BH * a.T;
+    const bool want_q = c.dq != nullptr, want_k2 = c.dk2 || c.dv2, want_k1 = c.dk1 || c.dv1;
+    // scratch: the accumulators of dK2, dV2, dK1, dU and dQ, the rows' poison words, the slices' scale partials
+    long long* acc = c.scratch;
+    unsigned* poison = reinterpret_cast<unsigned*>(acc + 5 * n);
+    unsigned* parts = reinterpret_cast<unsigned*>(acc + 5 * n + (rows + 3) / 4 * 2);  // 16-byte aligned
+    hipLaunchKernelGGL(f32_prep_kernel<D>, dim3((a.T + 63) / 64, a.BH), dim3(256), 0, st, c.v1_f32, c.v1_f32 ? c.u_out : nullptr,
+                       c.o, a.d_o, c.delta, acc, n, parts, poison, a.T);
     F32BwdParams<float> p{};
-    p.q = a.q; p.d_o = a.d_o; p.lse = a.lse_in; p.delta = a.delta;
-    p.round_parts = f32_round_parts(a.BH, a.T);
-    const bool q_shared = want_q && p.round_parts > 1;
-    p.dq = a.dq; p.acc_q = q_shared ? acc + 4 * n : nullptr; p.acc_q_rows = 0; p.stats_part = nullptr; p.split_rounds = 0;
-    // scratch: four accumulators (five when the rounds of a tile are dealt out: dQ then has one too), the rows'
-    // poison words, the slices' scale partials
-    const size_t nacc = (p.round_parts > 1 ? 5 : 4) * n;
-    const size_t rows = (size_t)a.BH * a.T, zero_n = nacc + (rows + 3) / 4 * 2;  // 16-byte aligned parts
-    unsigned* poison = reinterpret_cast<unsigned*>(acc + nacc);
-    unsigned* parts = reinterpret_cast<unsigned*>(acc + zero_n);
+    p.q = a.q; p.d_o = a.d_o; p.lse = a.lse_in; p.delta = c.delta;
+    p.dq = nullptr; p.acc_q = acc + 4 * n; p.acc_q_rows = 0; p.stats_part = nullptr; p.split_rounds = 0;
     p.scale_parts = parts; p.poison = poison; p.scale_bias = kF32FixedBias;
     p.T = a.T; p.BH = a.BH; p.nqt = (a.T + 31) / 32;
     p.alpha = a.alpha;
-    size_t gz = (zero_n + 255) / 256;
-    if (gz > 8192) gz = 8192;
-    hipLaunchKernelGGL(f32_zero_kernel, dim3((unsigned)gz), dim3(256), 0, st, acc, zero_n);
-    hipLaunchKernelGGL(f32_scale_kernel, dim3(kScaleParts, a.BH), dim3(256), 0, st, a.d_o, parts, (size_t)a.T * D);
     const TdpMask natural{a.causal, a.k1_window, a.k2_window, a.kk_left, a.kk_right};
     if (hipError_t e = launch_f32_bwd_tiles<float, D>(p, a.k1, a.u, a.k2, a.v2, acc, acc + n, acc + 2 * n, acc + 3 * n,
-                                                      natural, want_q, want_k2, want_k1, st, dense_inputs(a.T, D));
+                                                      natural, want_q, want_k2, want_k1, st, dense_inputs(a.T, D), true);
         e != hipSuccess)
         return e;
-    size_t gf = (n + 255) / 256;
-    if (gf > 4096) gf = 4096;
-    if (q_shared)
-        hipLaunchKernelGGL(f32_finish_q_kernel, dim3((unsigned)gf), dim3(256), 0, st, acc + 4 * n, a.dq, n, a.T, D, parts,
-                           poison, a.alpha);
-    if (want_k2)
-        hipLaunchKernelGGL(f32_finish_kernel, dim3((unsigned)gf), dim3(256), 0, st, acc, a.dk2, a.dv2, n, a.T, D, parts,
-                           poison, kPoisonDK2, kPoisonDV2);
-    if (want_k1)
-        hipLaunchKernelGGL(f32_finish_kernel, dim3((unsigned)gf), dim3(256), 0, st, acc + 2 * n, a.dk1, a.du, n, a.T, D,
-                           parts, poison, kPoisonDK1, kPoisonDU);
+    const dim3 grid((unsigned)std::min<size_t>((n / 4 + 255) / 256, 8192));
+    auto finish = [&](auto zero) {
+        using E = decltype(zero);
+        hipLaunchKernelGGL(f32_finish_kernel<E>, grid, dim3(256), 0, st, acc, (const E*)c.v1, (E*)c.dq, (E*)c.dk1, (E*)c.dk2,
+                           (E*)c.dv1, (E*)c.dv2, n, a.T, D, parts, poison, a.alpha);
+    };
+    if (c.elem == 0) finish(0.f);
+    else if (c.elem == 1) finish((__bf16)0.f);
+    else finish((_Float16)0.f);
     return hipGetLastError();
+}
+
+F32Deal f32_fwd_deal(const GenericTdpArgs& a, int most) {
+    auto w = [&](int x) { return std::min(x, a.T); };
+    const TdpMask mask{a.causal, w(a.k1_window), w(a.k2_window), w(a.kk_left), w(a.kk_right)};
+    return f32_deal(mask, a.BH, a.T, f32_fwd_waves(a.D), a.D > 64 ? 256 : 768, knobs().fwd_splits > 0 ? std::min(knobs().fwd_splits, most) : most);
 }
 
 template <int D>
@@ -142,29 +256,37 @@ hipError_t launch_f32_fwd(const GenericTdpArgs& a, hipStream_t st) {
     p.q = a.q; p.ka = a.k1; p.kb = a.k2; p.va = a.u; p.vb = a.v2;
     place_inputs(p, dense_inputs(a.T, D), false);
     p.o = a.o; p.lse = a.lse;
-    p.d_o = nullptr; p.delta = nullptr; p.split_rounds = 0; p.zero_ptr = nullptr; p.zero_words = 0;
+    p.d_o = nullptr; p.delta = nullptr; p.split_rounds = 0; p.zero_ptr = nullptr; p.zero_words = 0; p.deal = F32Deal{0.f, 1, p.nqt}; p.silu_va = a.u_is_v1 != 0;
     p.T = a.T; p.BH = a.BH; p.nqt = (a.T + 31) / 32;
     p.scale_log2 = a.alpha * kLog2e;
     p.mask = TdpMask{a.causal, a.k1_window, a.k2_window, a.kk_left, a.kk_right};
-    auto kern = tdp_f32_fwd_kernel<float, D, false>;
-    constexpr size_t smem = f32_fwd_smem<D>();
-    static_assert(D * 33 <= 4 * 32 * (D + 1), "the merged output aliases the stage buffers");
+    p.deal = a.part ? f32_fwd_deal(a, a.fwd_parts) : F32Deal{0.f, 1, p.nqt};
+    p.part = a.part;
+    constexpr int NW = f32_fwd_waves(D);
+    auto kern = tdp_f32_fwd_kernel<float, D, false, NW>;
+    constexpr size_t smem = f32_fwd_smem<D, NW>();
     if (hipError_t e = ensure_dynamic_smem(reinterpret_cast<const void*>(kern), smem); e != hipSuccess) return e;
-    hipLaunchKernelGGL(kern, dim3(8 * xcd_slots(a.BH, p.nqt)), dim3(512), smem, st, p);
+    hipLaunchKernelGGL(kern, dim3(8 * xcd_slots(a.BH, p.deal.items)), dim3(64 * NW), smem, st, p);
+    if (p.deal.max_parts > 1) {
+        const size_t rows = (size_t)a.BH * a.T;
+        hipLaunchKernelGGL(f32_merge_kernel, dim3((unsigned)((rows * (D / 4) + 255) / 256)), dim3(256), 0, st, a.part, a.o,
+                           a.lse, rows, a.T, D, p.mask, p.deal);
+    }
     return hipGetLastError();
 }
 
 }  // namespace
 
-bool f32_mfma_tdp_supported(int D) { return D == 32 || D == 64 || D == 128; }
-
-// Measured at D = 64 with narrow windows (seven rounds of two or three stages per tile): a round costs about 25 us and
-// a workgroup about 50 us before its first one, so dealing rounds out pays while the tiles alone leave more than half
-// of the compute units idle (32 tiles: 245 -> 75 us per launch), and not beyond (128 tiles: 245 -> 260 us).
-int f32_round_parts(int BH, int T) {
-    const int tiles = BH * ((T + 31) / 32);
-    return tiles >= 128 ? 1 : std::min(16, (256 + tiles - 1) / tiles);
+// SiLU as the value stages go to LDS costs about 1600 cycles of the waves that move them, every time a tile streams a row;
+// where a workgroup has no more than a few stages to walk that is less than a launch of its own (2-5 us)
+bool f32_fwd_takes_v1(const GenericTdpArgs& a) {
+    const F32Deal d = f32_fwd_deal(a, std::max(1, a.fwd_parts));
+    return d.inv_target >= 0.25f && (long long)a.BH * d.items <= 768;
 }
+int f32_fwd_parts(const GenericTdpArgs& a) { return f32_fwd_deal(a, 16).max_parts; }
+size_t f32_fwd_part_floats(int D) { return D + 4; }
+
+bool f32_mfma_tdp_supported(int D) { return D == 32 || D == 64 || D == 128; }
 
 // The first query tiles of a 16-bit backward, in fp32 (see the comment above tdp_f32_bwd_kernel).
 template <typename E, int D>
@@ -173,12 +295,12 @@ static hipError_t launch_stats(const FirstTileArgs& a, hipStream_t st) {
     p.q = (const E*)a.q; p.ka = (const E*)a.k1; p.kb = (const E*)a.k2; p.va = (const E*)a.u; p.vb = (const E*)a.v2;
     place_inputs(p, inputs_of(a), false);
     p.o = nullptr; p.lse = a.lse_f32; p.d_o = (const E*)a.d_o; p.delta = a.delta_f32;
-    p.split_rounds = 0; p.zero_ptr = nullptr; p.zero_words = 0;
+    p.split_rounds = 0; p.zero_ptr = nullptr; p.zero_words = 0; p.deal = F32Deal{0.f, 1, p.nqt}; p.silu_va = false;
     p.T = a.T; p.BH = a.BH; p.nqt = a.tiles;
     p.scale_log2 = a.alpha * kLog2e;
     p.mask = TdpMask{a.causal, a.k1_window, a.k2_window, a.kk_left, a.kk_right};
-    auto kern = tdp_f32_fwd_kernel<E, D, true>;
-    constexpr size_t smem = f32_fwd_smem<D>();
+    auto kern = tdp_f32_fwd_kernel<E, D, true, kF32Waves>;
+    constexpr size_t smem = f32_fwd_smem<D, kF32Waves>();
     if (hipError_t e = ensure_dynamic_smem(reinterpret_cast<const void*>(kern), smem); e != hipSuccess) return e;
     hipLaunchKernelGGL(kern, dim3(8 * xcd_slots(a.BH, p.nqt)), dim3(512), smem, st, p);
     return hipGetLastError();
@@ -212,7 +334,6 @@ static hipError_t first_tile_typed(const FirstTileArgs& a, hipStream_t st) {
     F32BwdParams<E> p{};
     p.q = (const E*)a.q; p.d_o = (const E*)a.d_o; p.lse = a.lse_f32; p.delta = a.delta_f32;
     p.dq = (E*)a.dq; p.acc_q = a.acc_q; p.acc_q_rows = 0; p.stats_part = nullptr; p.split_rounds = 0;
-    p.round_parts = a.round_parts;
     p.scale_parts = a.scale_parts; p.poison = a.poison; p.scale_bias = a.scale_bias;
     p.T = a.T; p.BH = a.BH; p.nqt = a.tiles;
     p.alpha = a.alpha;
@@ -220,11 +341,11 @@ static hipError_t first_tile_typed(const FirstTileArgs& a, hipStream_t st) {
     const E *k1 = (const E*)a.k1, *u = (const E*)a.u, *k2 = (const E*)a.k2, *v2 = (const E*)a.v2;
     const bool wq = a.want_q, wk2 = a.want_k2, wk1 = a.want_k1;
     if (a.D == 32)
-        return launch_f32_bwd_tiles<E, 32>(p, k1, u, k2, v2, a.acc_k2, a.acc_v2, a.acc_k1, a.acc_u, natural, wq, wk2, wk1, st, inputs_of(a));
+        return launch_f32_bwd_tiles<E, 32>(p, k1, u, k2, v2, a.acc_k2, a.acc_v2, a.acc_k1, a.acc_u, natural, wq, wk2, wk1, st, inputs_of(a), a.split_rounds);
     if (a.D == 64)
-        return launch_f32_bwd_tiles<E, 64>(p, k1, u, k2, v2, a.acc_k2, a.acc_v2, a.acc_k1, a.acc_u, natural, wq, wk2, wk1, st, inputs_of(a));
+        return launch_f32_bwd_tiles<E, 64>(p, k1, u, k2, v2, a.acc_k2, a.acc_v2, a.acc_k1, a.acc_u, natural, wq, wk2, wk1, st, inputs_of(a), a.split_rounds);
     if (a.D == 128)
-        return launch_f32_bwd_tiles<E, 128>(p, k1, u, k2, v2, a.acc_k2, a.acc_v2, a.acc_k1, a.acc_u, natural, wq, wk2, wk1, st, inputs_of(a));
+        return launch_f32_bwd_tiles<E, 128>(p, k1, u, k2, v2, a.acc_k2, a.acc_v2, a.acc_k1, a.acc_u, natural, wq, wk2, wk1, st, inputs_of(a), a.split_rounds);
     return hipErrorInvalidValue;
 }
 hipError_t f32_mfma_tdp_bwd_first_tile(const FirstTileArgs& a, hipStream_t st) {
@@ -239,14 +360,14 @@ hipError_t f32_mfma_tdp_fwd(const GenericTdpArgs& a, hipStream_t st) {
 }
 
 size_t f32_mfma_tdp_bwd_scratch_elems(int BH, int T, int D) {
-    return (f32_round_parts(BH, T) > 1 ? 5 : 4) * (size_t)BH * T * D + ((size_t)BH * T + 3) / 4 * 2 +
+    return 5 * (size_t)BH * T * D + ((size_t)BH * T + 3) / 4 * 2 +
            (size_t)BH * kScaleParts / 2;
 }
 
-hipError_t f32_mfma_tdp_bwd(const GenericTdpArgs& a, long long* scratch, hipStream_t st) {
-    if (a.D == 32) return launch_f32_bwd<32>(a, scratch, st);
-    if (a.D == 64) return launch_f32_bwd<64>(a, scratch, st);
-    if (a.D == 128) return launch_f32_bwd<128>(a, scratch, st);
+hipError_t f32_mfma_tdp_bwd(const F32BwdCall& c, hipStream_t st) {
+    if (c.a.D == 32) return launch_f32_bwd<32>(c, st);
+    if (c.a.D == 64) return launch_f32_bwd<64>(c, st);
+    if (c.a.D == 128) return launch_f32_bwd<128>(c, st);
     return hipErrorInvalidValue;
 }
 

@@ -18,6 +18,59 @@ __device__ __forceinline__ f32x16 mma_f32(float a, float b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
 }
 
+// Ranges of streamed rows / owner rows a tile of queries [q0, q1] can touch.
+struct Range {
+    int lo, hi;
+};
+__host__ __device__ __forceinline__ Range row_range(const TdpMask& m, int q0, int q1, int T) {
+    if (!m.causal) return {0, T - 1};
+    return {q0 - m.wb > 0 ? q0 - m.wb : 0, q1};
+}
+__device__ __forceinline__ Range streamed_range(const TdpMask& m, int q0, int q1, int b, int T) {
+    if (!m.causal) return {0, T - 1};
+    // a <= q, q - a <= wa, b - a <= lab, a - b <= rab
+    return {max(0, max(q0 - m.wa, b - m.lab)), min(q1, b + m.rab)};
+}
+
+// Workgroups per query tile.  The work of a tile is its (round of nw rows, 32-row stage) steps, which under a causal mask
+// grows with the square of its position: a workgroup takes about 1 / inv_target of them, and a tile as many workgroups (its
+// parts) as that asks for.  The grid is the list of all parts, heaviest tiles first, without gaps: workgroups that find
+// nothing to do would land on the same shader engines again and again (the dispatcher takes those in turn), B=4 H=8 T=512
+// 13.8 -> 15-16 ms per backward.
+struct F32Deal {
+    float inv_target;
+    int max_parts, items;  // parts of the heaviest tile, and of all tiles of a slice
+};
+__host__ __device__ __forceinline__ int f32_tile_steps(const TdpMask& m, int q0, int q1, int T, int nw, int* rounds_out) {
+    const Range r = row_range(m, q0, q1, T);
+    const int rounds = r.hi / nw - r.lo / nw + 1;
+    *rounds_out = rounds;
+    if (!m.causal) return rounds * ((T + 31) / 32);
+    const int span = q1 - (q0 - m.wa > 0 ? q0 - m.wa : 0), band = m.lab + m.rab + nw;
+    return rounds * ((span < band ? span : band) / 32 + 1);
+}
+__host__ __device__ __forceinline__ int f32_tile_parts(const F32Deal& d, const TdpMask& m, int qt, int T, int nw) {
+    if (d.max_parts <= 1) return 1;
+    const int q0 = qt * 32, q1 = q0 + 31 < T - 1 ? q0 + 31 : T - 1;
+    int rounds;
+    const int want = 1 + (int)((float)f32_tile_steps(m, q0, q1, T, nw, &rounds) * d.inv_target);
+    const int most = rounds < d.max_parts ? rounds : d.max_parts;
+    return want < most ? want : most;
+}
+// part `item` of a slice's list: its tile, its place among the tile's parts and their number (part >= parts: past the list)
+struct F32Item {
+    int qt, part, parts;
+};
+__device__ __forceinline__ F32Item f32_item(const F32Deal& d, const TdpMask& m, int item, int nqt, int T, int nw) {
+    if (d.max_parts <= 1) return {nqt - 1 - item, 0, 1};
+    F32Item it{nqt - 1, item, f32_tile_parts(d, m, nqt - 1, T, nw)};
+    while (it.part >= it.parts && it.qt > 0) {
+        it.part -= it.parts;
+        it.parts = f32_tile_parts(d, m, --it.qt, T, nw);
+    }
+    return it;
+}
+
 template <typename E>
 struct F32Params {
     const E *q, *ka, *kb, *va, *vb;  // streamed = (ka, va), rows = (kb, vb)
@@ -37,87 +90,168 @@ struct F32Params {
     int split_rounds;
     unsigned* zero_ptr;
     int zero_words;
+    bool silu_va;  // va is V1 itself: SiLU is applied as its stages go to LDS (not with STATS)
+    // deal.max_parts > 1 (never with STATS): the rounds of a tile are dealt out to f32_tile_parts() workgroups; each leaves
+    // its unnormalised output, reference maximum and row sum in part[((bh T + q) max_parts + y) (D + 4)] (O[D], M, L)
+    F32Deal deal;
+    float* part;
     int T, BH, nqt;  // nqt: query tiles this launch covers (tiles 0 .. nqt - 1)
     float scale_log2;
     TdpMask mask;  // in terms of the streamed index a and the row index b
 };
 
-// Ranges of streamed rows / owner rows a tile of queries [q0, q1] can touch.
-struct Range {
-    int lo, hi;
-};
-__device__ __forceinline__ Range row_range(const TdpMask& m, int q0, int q1, int T) {
-    if (!m.causal) return {0, T - 1};
-    return {max(0, q0 - m.wb), q1};
-}
-__device__ __forceinline__ Range streamed_range(const TdpMask& m, int q0, int q1, int b, int T) {
-    if (!m.causal) return {0, T - 1};
-    // a <= q, q - a <= wa, b - a <= lab, a - b <= rab
-    return {max(0, max(q0 - m.wa, b - m.lab)), min(q1, b + m.rab)};
-}
-
 // Staging of 32 x D tiles of E through registers (16-byte pieces), converted to fp32 on the way into LDS.
-template <typename E, int D>
+// NW waves move the two tiles of a stage.
+template <typename E, int D, int NW>
 struct StageE {
     static constexpr int VE = 16 / (int)sizeof(E);           // elements per piece
     static constexpr int kPieces = 32 * D / VE;               // per tensor
-    static constexpr int kPer = (kPieces + 255) / 256;        // per thread
+    static constexpr int kThreads = NW * 32;                  // per tensor: half of the workgroup for each
+    static constexpr int kPer = (kPieces + kThreads - 1) / kThreads;  // per thread
     uint4 x[kPer];
 };
-template <typename E, int D>
-__device__ __forceinline__ void stage_fetch_e(StageE<E, D>& r, const E* __restrict__ ka, const E* __restrict__ va, int a0,
+template <typename E, int D, int NW>
+__device__ __forceinline__ void stage_fetch_e(StageE<E, D, NW>& r, const E* __restrict__ ka, const E* __restrict__ va, int a0,
                                               int T, unsigned pitch_ka, unsigned pitch_va) {
-    using S = StageE<E, D>;
+    using S = StageE<E, D, NW>;
     constexpr int kVec = D / S::VE;
-    const int t = threadIdx.x & 255;
-    const E* src = threadIdx.x < 256 ? ka : va;
-    const unsigned pitch = threadIdx.x < 256 ? pitch_ka : pitch_va;
+    const int t = threadIdx.x & (S::kThreads - 1);
+    const bool first = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) < NW / 2;  // whole waves serve one tensor
+    const E* src = first ? ka : va;
+    const unsigned pitch = first ? pitch_ka : pitch_va;
+    // a whole stage lies at per-lane offsets that never change from its (scalar) first row; 31 pitch < T pitch < 2^31
+    const bool whole = a0 + 31 < T;
+    const E* row0 = src + (size_t)a0 * pitch;
 #pragma unroll
     for (int i = 0; i < S::kPer; ++i) {
-        const int idx = t + i * 256;
-        if (idx < S::kPieces) {
+        const int idx = t + i * S::kThreads;
+        if (S::kPieces % S::kThreads == 0 || idx < S::kPieces) {
             const int row = idx / kVec, c = idx % kVec;
-            r.x[i] = *reinterpret_cast<const uint4*>(src + (size_t)min(a0 + row, T - 1) * pitch + c * S::VE);
+            if (whole) r.x[i] = *reinterpret_cast<const uint4*>(row0 + (unsigned)(row * pitch + c * S::VE));
+            else r.x[i] = *reinterpret_cast<const uint4*>(src + (size_t)min(a0 + row, T - 1) * pitch + c * S::VE);
         }
     }
 }
-template <typename E, int D>
-__device__ __forceinline__ void stage_store_e(const StageE<E, D>& r, float* sk, float* sv) {
-    using S = StageE<E, D>;
-    constexpr int kVec = D / S::VE, LD = D + 1;
-    const int t = threadIdx.x & 255;
-    float* dst = threadIdx.x < 256 ? sk : sv;
+template <typename E, int D, int NW>
+__device__ __forceinline__ void stage_store_e(const StageE<E, D, NW>& r, float* sk, float* sv, bool silu_v = false) {
+    using S = StageE<E, D, NW>;
+    constexpr int kVec = D / S::VE, LD = D + 4;  // f32_pitch<D>()
+    const int t = threadIdx.x & (S::kThreads - 1);
+    const bool first = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) < NW / 2;
+    float* dst = first ? sk : sv;
+    const bool silu = silu_v && !first;
 #pragma unroll
     for (int i = 0; i < S::kPer; ++i) {
-        const int idx = t + i * 256;
-        if (idx < S::kPieces) {
+        const int idx = t + i * S::kThreads;
+        if (S::kPieces % S::kThreads == 0 || idx < S::kPieces) {
             const int row = idx / kVec, c = idx % kVec;
             float* p = dst + row * LD + c * S::VE;
             const E* e = reinterpret_cast<const E*>(&r.x[i]);
 #pragma unroll
-            for (int k = 0; k < S::VE; ++k) p[k] = (float)e[k];
+            for (int k = 0; k < S::VE; k += 4) {
+                typedef __attribute__((ext_vector_type(4))) float f4;
+                f4 v = {(float)e[k], (float)e[k + 1], (float)e[k + 2], (float)e[k + 3]};
+                if (silu) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) v[j] = silu_f(v[j]);
+                }
+                *reinterpret_cast<f4*>(p + k) = v;
+            }
         }
     }
 }
 
+// Row pitch (floats) of the [rows][D] tiles in LDS: rows start on 16-byte boundaries and the pitch is an odd number of
+// 16-byte units, so that the 16-byte operand reads of a wave (32 rows, one piece each) fall on distinct bank groups.
+template <int D>
+constexpr int f32_pitch() {
+    return D + 4;
+}
+template <int N>
+struct VecF {
+    typedef __attribute__((ext_vector_type(N))) float type;
+};
+template <>
+struct VecF<1> {
+    typedef float type;
+};
+template <int N>
+__device__ __forceinline__ float vec_at(const typename VecF<N>::type& v, int i) {
+    if constexpr (N == 1) return v;
+    else return v[i];
+}
+typedef VecF<4>::type f32x4v;
+
+// The valid streamed rows of one (query, row b): a - lo <= span as unsigned numbers; nothing is valid for span 0, lo 2^30
+struct Interval {
+    int lo;
+    unsigned span;
+};
+__device__ __forceinline__ Interval valid_interval(const TdpMask& m, int q, int b, int T) {
+    if (!m.causal) return {0, (unsigned)(T - 1)};
+    const int lo = max(0, max(q - m.wa, b - m.lab)), hi = min(min(q, b + m.rab), T - 1);
+    const bool any = (b <= q) & (q <= b + m.wb) & (lo <= hi);
+    return any ? Interval{lo, (unsigned)(hi - lo)} : Interval{1 << 30, 0u};
+}
+
+// whether all of tile (queries q0 .. q0 + 31, streamed rows a0 .. a0 + 31) of row b is valid
+__device__ __forceinline__ bool all_valid(const TdpMask& m, int q0, int a0, int b, int T) {
+    if (!m.causal) return a0 + 31 < T;
+    return (b <= q0) & (q0 + 31 <= b + m.wb) & (a0 + 31 <= min(q0, b + m.rab)) & (a0 >= max(q0 + 31 - m.wa, b - m.lab));
+}
+
+// The (round of rows, stage of streamed rows) sequence a workgroup walks, one stage per step; rounds whose rows see no
+// streamed row at all are passed over.
+struct Walk {
+    int m, st, st_hi;
+};
+template <int NW>
+__device__ __forceinline__ bool open_round(Walk& w, const TdpMask& mask, int m, int m_hi, int step, int q0, int q1, int T) {
+    for (; m <= m_hi; m += step) {
+        // the union over the round's rows
+        const Range ra = streamed_range(mask, q0, q1, min(m * NW, T - 1), T);
+        const Range rb = streamed_range(mask, q0, q1, min(m * NW + NW - 1, T - 1), T);
+        const int lo = min(ra.lo, rb.lo) / 32, hi = max(ra.hi, rb.hi) / 32;
+        if (lo <= hi) {
+            w = {m, lo, hi};
+            return true;
+        }
+    }
+    return false;
+}
+
 // ------------------------------------------------------------------------------------------ forward
-template <typename E, int D, bool STATS>
-__global__ __launch_bounds__(512) void tdp_f32_fwd_kernel(F32Params<E> p) {
-    constexpr int DT = D / 32, KS = D / 2, LD = D + 1, NW = kF32Waves;
-    constexpr bool FLY = D > 64;  // form the B operand of the score product as it is used
+// What bounds it: the fp32 matrix pipe, which fp32 MFMAs (64 cycles each) and vector instructions use in turn -- measured
+// busy(MFMA) + busy(VALU) = 97 % of the cycles -- so every vector instruction of the loop counts, and waves of different
+// workgroups have to fill each other's waits.  Hence: a workgroup is four waves (D <= 64; one per SIMD) that fit 168
+// registers, three workgroups to a CU; the B operand of the score product is formed once per round and held; the maximum is
+// only formed when a sum outgrows its reference; tiles inside the mask skip it; stages are fetched from a scalar base at
+// constant lane offsets.  Operand reads are as wide as the layout allows: the k-slots of four consecutive MFMAs are four
+// consecutive d (16 bytes of a row), and output row r of value tile dt is column d = DT r + dt, so that the operands of the
+// DT value tiles are DT consecutive columns.  Stages and row operands are fetched one step ahead across the rounds' ends,
+// one barrier per step.  B=4 H=8 T=512 D=64: 5.94 -> 3.26 ms (113 TFLOP/s, 72 % of the fp32 matrix rate), of which the parts
+// (F32Deal) make 2.4; B=2 H=4 T=500: 5.38 -> 0.88 ms.  Eight waves with the operand formed as it is used and 128 registers
+// (two workgroups to a CU) measured 3.49 ms, eight with it held (one workgroup) 3.66.
+template <typename E, int D, bool STATS, int NW>
+__global__ __launch_bounds__(64 * NW, NW == 8 ? 2 : 3) void tdp_f32_fwd_kernel(F32Params<E> p) {
+    constexpr int DT = D / 32, LD = f32_pitch<D>(), NT = 64 * NW;
+    constexpr bool HOLD = D <= 64;
+    using vDT = typename VecF<DT>::type;
     extern __shared__ __align__(16) float smem_f[];
-    float* sK = smem_f;                 // [2][32][LD] streamed key rows
-    float* sV = sK + 2 * 32 * LD;       // [2][32][LD] streamed value rows
-    float* sQ = sV + 2 * 32 * LD;       // [32][LD]    the tile's queries * scale
-    float* sKb = sQ + 32 * LD;          // [NW][D]     row operands of the round
-    float* sVb = sKb + NW * D;          // [NW][D]
-    float* sM = sVb + NW * D;           // [NW][32]    end of kernel: per-wave maxima and sums
+    float* sM = smem_f;                 // [NW][32]    end of kernel: per-wave maxima and sums
     float* sL = sM + NW * 32;           // [NW][32]
-    float* sO = sK;                     // [D][33]     end of kernel: merged output (aliases the stages)
+    float* sQ = sL + NW * 32;           // [32][LD]    the tile's queries * scale
+    float* sK = sQ + 32 * LD;           // [2][32][LD] streamed key rows
+    float* sV = sK + 2 * 32 * LD;       // [2][32][LD] streamed value rows
+    float* sKb = sV + 2 * 32 * LD;      // [2][NW][D]  row operands of a round
+    float* sVb = sKb + 2 * NW * D;      // [2][NW][D]
+    float* sO = sK;                     // [NW][D][33] end of kernel: the waves' outputs (alias everything from the stages on)
 
     int bh, order;
-    if (!xcd_tile(p.BH, p.nqt, blockIdx.x >> 3, blockIdx.x & 7, bh, order)) return;
-    const int qt = p.nqt - 1 - order;  // heaviest query tiles first
+    if (!xcd_tile(p.BH, STATS ? p.nqt : p.deal.items, blockIdx.x >> 3, blockIdx.x & 7, bh, order)) return;
+    const F32Item item = STATS ? F32Item{p.nqt - 1 - order, 0, 1} : f32_item(p.deal, p.mask, order, p.nqt, p.T, NW);
+    const int qt = item.qt, part = item.part, step = item.parts;
+    if (part >= step) return;
 
     const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -134,160 +268,231 @@ __global__ __launch_bounds__(512) void tdp_f32_fwd_kernel(F32Params<E> p) {
 
     const int q0 = qt * 32, q1 = min(T - 1, q0 + 31);
     const int q = q0 + n;  // this lane's query (column of every tile)
-    for (int idx = tid; idx < 32 * D; idx += 512) {
-        const int r = idx / D, d = idx % D;
-        sQ[r * LD + d] = (float)Qs[(size_t)min(q0 + r, T - 1) * p.at_q.st + d] * p.scale_log2;
-    }
-
     const Range rows = row_range(mask, q0, q1, T);
-    int m_lo = rows.lo / NW, m_hi = rows.hi / NW;  // rounds of NW rows
+    // rounds of NW rows: workgroup `part` of a tile takes every step-th one from the part-th on
+    int m_lo = rows.lo / NW + part, m_hi = rows.hi / NW;
     if (STATS && p.split_rounds) {
         m_lo = max(m_lo, (int)blockIdx.y);  // this workgroup's round only (none at all if it is out of range)
         m_hi = min(m_hi, (int)blockIdx.y);
         if (blockIdx.y == 0)
-            for (int idx = tid; idx < p.zero_words; idx += 512) p.zero_ptr[(size_t)bh * p.zero_words + idx] = 0u;
+            for (int idx = tid; idx < p.zero_words; idx += NT) p.zero_ptr[(size_t)bh * p.zero_words + idx] = 0u;
     }
 
-    f32x16 accO[DT];
+    f32x16 accO[DT], accT[DT];
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) accO[dt][i] = 0.f;
+        for (int i = 0; i < 16; ++i) {
+            accO[dt][i] = 0.f;
+            accT[dt][i] = 0.f;
+        }
     float m_run = kNegBig, l_run = 0.f;  // per query, over every (a, b) this wave has seen (l: this lane's half)
 
-    StageE<E, D> regs;
-    for (int m = m_lo; m <= m_hi; ++m) {
-        const int b = m * NW + wave;
-        // the streamed stages this round needs: the union over its rows
-        const Range ra = streamed_range(mask, q0, q1, min(m * NW, T - 1), T);
-        const Range rb = streamed_range(mask, q0, q1, min(m * NW + NW - 1, T - 1), T);
-        const int st_lo = min(ra.lo, rb.lo) / 32, st_hi = max(ra.hi, rb.hi) / 32;
+    StageE<E, D, NW> regs;
+    constexpr int kRowPer = (NW * D + NT - 1) / NT;
+    float row_k[kRowPer], row_v[kRowPer];
+    auto fetch_rows = [&](int m) {
+#pragma unroll
+        for (int i = 0; i < kRowPer; ++i) {
+            const int idx = min(tid + i * NT, NW * D - 1);
+            const size_t row = (size_t)min(m * NW + idx / D, T - 1);
+            row_k[i] = (float)KB[row * p.at_kb.st + idx % D];
+            row_v[i] = (float)VB[row * p.at_vb.st + idx % D];
+        }
+    };
+    auto store_rows = [&](int par) {
+#pragma unroll
+        for (int i = 0; i < kRowPer; ++i)
+            if (tid + i * NT < NW * D) {
+                sKb[par * NW * D + tid + i * NT] = row_k[i];
+                sVb[par * NW * D + tid + i * NT] = row_v[i];
+            }
+    };
+
+    Walk w{};
+    bool have = open_round<NW>(w, mask, m_lo, m_hi, step, q0, q1, T);
+    if (have) {
+        fetch_rows(w.m);
+        stage_fetch_e<E, D, NW>(regs, KA, VA, w.st * 32, T, p.at_ka.st, p.at_va.st);
+    }
+    for (int idx = tid; idx < 32 * D; idx += NT) {
+        const int r = idx / D, d = idx % D;
+        sQ[r * LD + d] = (float)Qs[(size_t)min(q0 + r, T - 1) * p.at_q.st + d] * p.scale_log2;
+    }
+    if (have) {
+        store_rows(0);
+        stage_store_e<E, D, NW>(regs, sK, sV, !STATS && p.silu_va);
+    }
+    __syncthreads();
+
+    int buf = 0, par = 0;
+    float bq[HOLD ? D / 2 : 1];
+    bool fresh = true;  // the first step of a round
+    while (have) {
+        const float* cK = sK + buf * 32 * LD;
+        const float* cV = sV + buf * 32 * LD;
+        const bool last = w.st == w.st_hi;  // of this round
+        Walk nw{w.m, w.st + 1, w.st_hi};
+        const bool more = last ? open_round<NW>(nw, mask, w.m + step, m_hi, step, q0, q1, T) : true;
+        if (more) {
+            stage_fetch_e<E, D, NW>(regs, KA, VA, nw.st * 32, T, p.at_ka.st, p.at_va.st);
+            if (last) fetch_rows(nw.m);
+        }
+        const int b = w.m * NW + wave, a0 = w.st * 32;
         const bool row_ok = b <= rows.hi && b >= rows.lo;
         const Range mine = streamed_range(mask, q0, q1, min(b, T - 1), T);
-
-        __syncthreads();  // previous round: everyone is done with sKb / sVb and the stage buffers
-        for (int idx = tid; idx < NW * D; idx += 512) {
-            const int r = idx / D, d = idx % D;
-            const size_t row = (size_t)min(m * NW + r, T - 1);
-            sKb[idx] = (float)KB[row * p.at_kb.st + d];
-            sVb[idx] = (float)VB[row * p.at_vb.st + d];
-        }
-        if (st_lo <= st_hi) {
-            stage_fetch_e<E, D>(regs, KA, VA, st_lo * 32, T, p.at_ka.st, p.at_va.st);
-            stage_store_e<E, D>(regs, sK, sV);
-        }
-        __syncthreads();
-
-        // B operand of the score product: lane (q, g), step s holds scale * Q[q, g*D/2 + s] * KB[b, g*D/2 + s]
-        float bq[FLY ? 1 : KS];
-        if constexpr (!FLY) {
+        const float* ob = sKb + par * NW * D + wave * D;
+        if constexpr (HOLD) {
+            if (fresh) {
 #pragma unroll
-            for (int s = 0; s < KS; ++s) bq[s] = sQ[n * LD + g * KS + s] * sKb[wave * D + g * KS + s];
-        }
-
-        f32x16 accT[DT];
+                for (int c = 0; c < D / 8; ++c) {
+                    const f32x4v qv = *reinterpret_cast<const f32x4v*>(sQ + n * LD + 4 * g + 8 * c);
+                    const f32x4v kb = *reinterpret_cast<const f32x4v*>(ob + 4 * g + 8 * c);
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) accT[dt][i] = 0.f;
-
-        for (int st = st_lo; st <= st_hi; ++st) {
-            const int buf = (st - st_lo) & 1;
-            const float* cK = sK + buf * 32 * LD;
-            const float* cV = sV + buf * 32 * LD;
-            const bool more = st < st_hi;
-            if (more) stage_fetch_e<E, D>(regs, KA, VA, (st + 1) * 32, T, p.at_ka.st, p.at_va.st);
-            const int a0 = st * 32;
-            if (row_ok && a0 + 31 >= mine.lo && a0 <= mine.hi) {
-                f32x16 s;
-#pragma unroll
-                for (int i = 0; i < 16; ++i) s[i] = 0.f;
-#pragma unroll
-                for (int ks = 0; ks < KS; ++ks) {
-                    const int col = g * KS + ks;
-                    const float oq = FLY ? sQ[n * LD + col] * sKb[wave * D + col] : bq[FLY ? 0 : ks];
-                    s = mma_f32(cK[n * LD + col], oq, s);
+                    for (int e = 0; e < 4; ++e) bq[c * 4 + e] = qv[e] * kb[e];
                 }
-                // mask, tile maximum of this lane's 16 rows
+            }
+            fresh = last;
+        }
+        if (row_ok && a0 + 31 >= mine.lo && a0 <= mine.hi) {
+            f32x16 s;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) s[i] = 0.f;
+            // per-lane parts of the LDS addresses, opaque: every read is one of them plus an immediate offset
+            int row_base = n * LD + 4 * g, own_base = 4 * g, out_base = 4 * g * LD + DT * n;
+            asm volatile("" : "+v"(row_base), "+v"(own_base), "+v"(out_base));
+            // MFMA 4 c + e contracts d = 8 c + e (lanes of half 0) and 8 c + 4 + e (half 1)
+#pragma unroll
+            for (int c = 0; c < D / 8; ++c) {
+                const f32x4v ka = *reinterpret_cast<const f32x4v*>(cK + row_base + 8 * c);
+                if constexpr (HOLD) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) s = mma_f32(ka[e], bq[c * 4 + e], s);
+                } else {
+                    const f32x4v qv = *reinterpret_cast<const f32x4v*>(sQ + row_base + 8 * c);
+                    const f32x4v kb = *reinterpret_cast<const f32x4v*>(ob + own_base + 8 * c);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) s = mma_f32(ka[e], qv[e] * kb[e], s);
+                }
+            }
+            if (!all_valid(mask, q0, a0, b, T)) {
+                const Interval ok = valid_interval(mask, q, b, T);
+                const int x = a0 + 4 * g - ok.lo;
+#pragma unroll
+                for (int i = 0; i < 16; ++i) s[i] = (unsigned)(x + c_row(0, i)) <= ok.span ? s[i] : -INFINITY;
+            }
+            // exponentials relative to the query's reference, which is some earlier tile's maximum: a sum that outgrows it
+            // by 2^40 (or the first one of all) moves it to this tile's maximum.  fp32 sums lose nothing by a loose
+            // reference, and the maximum need not be formed for every tile
+            f32x16 pv;
+            float psum = 0.f;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                pv[i] = fast_exp2(s[i] - m_run);
+                psum += pv[i];
+            }
+            if (__any(!(psum <= 1.0e12f))) {
                 float tmax = kNegBig;
 #pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    const int a = a0 + c_row(g, i);
-                    const bool ok = a < T && tdp_valid(mask, q, a, b);
-                    s[i] = ok ? s[i] : -INFINITY;
-                    tmax = fmaxf(tmax, s[i]);
-                }
+                for (int i = 0; i < 16; ++i) tmax = fmaxf(tmax, s[i]);
                 tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-                const float m_new = fmaxf(m_run, tmax);
-                if (__any(m_new > m_run)) {
-                    const float sc = fast_exp2(m_run - m_new);
-                    l_run *= sc;
-#pragma unroll
-                    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-                        for (int i = 0; i < 16; ++i) {
-                            accT[dt][i] *= sc;
-                            accO[dt][i] *= sc;
-                        }
-                    m_run = m_new;
-                }
-                float psum = 0.f;
-#pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    s[i] = fast_exp2(s[i] - m_run);
-                    psum += s[i];
-                }
-                l_run += psum;
-                // Tv^T[d, q] += VA^T[d, a] P^T[a, q]: step i contracts the two streamed rows c_row(0, i), c_row(1, i)
+                const float m_new = fmaxf(m_run, tmax), sc = fast_exp2(m_run - m_new);
+                l_run *= sc;
 #pragma unroll
                 for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) accT[dt] = mma_f32(cV[c_row(g, i) * LD + dt * 32 + n], s[i], accT[dt]);
+                    for (int i = 0; i < 16; ++i) {
+                        accT[dt][i] *= sc;
+                        accO[dt][i] *= sc;
+                    }
+                m_run = m_new;
+                psum = 0.f;
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    pv[i] = fast_exp2(s[i] - m_run);
+                    psum += pv[i];
+                }
             }
-            if (more) {
-                stage_store_e<E, D>(regs, sK + (buf ^ 1) * 32 * LD, sV + (buf ^ 1) * 32 * LD);
-                __syncthreads();
+            l_run += psum;
+            // Tv^T[d, q] += VA^T[d, a] P^T[a, q]: step i contracts the two streamed rows c_row(0, i), c_row(1, i)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const vDT va = *reinterpret_cast<const vDT*>(cV + out_base + c_row(0, i) * LD);
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt) accT[dt] = mma_f32(vec_at<DT>(va, dt), pv[i], accT[dt]);
             }
         }
-        // the finished row: O^T[d, q] += Tv^T[d, q] * VB[b, d]   (register i of half g is d = 32 dt + c_row(g, i))
-        if (row_ok) {
+        if (last) {
+            // the finished row: O^T[d, q] += Tv^T[d, q] * VB[b, d]   (register i of half g: d = DT c_row(g, i) + dt)
+            if (row_ok) {
+                const float* vb = sVb + par * NW * D + wave * D;
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    const vDT v = *reinterpret_cast<const vDT*>(vb + DT * (c_row(0, i) + 4 * g));
+#pragma unroll
+                    for (int dt = 0; dt < DT; ++dt) accO[dt][i] += accT[dt][i] * vec_at<DT>(v, dt);
+                }
+            }
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-                for (int i = 0; i < 16; ++i) accO[dt][i] += accT[dt][i] * sVb[wave * D + dt * 32 + c_row(g, i)];
+                for (int i = 0; i < 16; ++i) accT[dt][i] = 0.f;
         }
+        if (more) {
+            buf ^= 1;
+            if (last) {
+                par ^= 1;
+                store_rows(par);
+            }
+            stage_store_e<E, D, NW>(regs, sK + buf * 32 * LD, sV + buf * 32 * LD, !STATS && p.silu_va);
+            __syncthreads();
+        }
+        w = nw;
+        have = more;
     }
 
-    // ---- merge the eight waves' partial results (each relative to its own maximum), one wave after another
+    // ---- merge the waves' partial results: each leaves its own, relative to the common maximum, in a [D][33] slice of LDS,
+    // and the slices are added in a fixed order (one wave after another into a common slice put a barrier and a chain of
+    // LDS round trips per wave at the end of every workgroup)
     l_run += __shfl_xor(l_run, 32, 64);
-    __syncthreads();
     if (g == 0) {
         sM[wave * 32 + n] = m_run;
         sL[wave * 32 + n] = l_run;
     }
-    for (int idx = tid; idx < D * 33; idx += 512) sO[idx] = 0.f;
     __syncthreads();
     float M = kNegBig;
 #pragma unroll
     for (int w = 0; w < NW; ++w) M = fmaxf(M, sM[w * 32 + n]);
     const float mine_scale = fast_exp2(m_run - M);
-    for (int w = 0; w < NW; ++w) {
-        if (wave == w) {
 #pragma unroll
-            for (int dt = 0; dt < DT; ++dt)
+    for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-                for (int i = 0; i < 16; ++i) sO[(dt * 32 + c_row(g, i)) * 33 + n] += accO[dt][i] * mine_scale;
-        }
-        __syncthreads();
-    }
+        for (int i = 0; i < 16; ++i) sO[wave * D * 33 + (DT * c_row(g, i) + dt) * 33 + n] = accO[dt][i] * mine_scale;
+    __syncthreads();
+    auto merged = [&](int d, int r) {
+        float v = sO[d * 33 + r];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) v += sO[(w * D + d) * 33 + r];
+        return v;
+    };
     float L = 0.f;
 #pragma unroll
     for (int w = 0; w < NW; ++w) L += sL[w * 32 + n] * fast_exp2(sM[w * 32 + n] - M);
     if constexpr (STATS) {
-        // Delta[q] = sum_d dO[q, d] O[q, d] with O in fp32 (lane n of wave 0 walks its query's row)
+        // Delta[q] = sum_d dO[q, d] O[q, d] with O in fp32: two threads of every wave per query, joined through LDS
+        float* red = sQ;  // [2 NW][32]
+        const int k16 = wave * 2 + g;
+        float dsum = 0.f;
+        if (q < T) {
+            const E* dor = slice(p.d_o, p.at_do) + (size_t)q * p.at_do.st;
+            for (int d = k16; d < D; d += 2 * NW) dsum += (float)dor[d] * merged(d, n);
+        }
+        red[k16 * 32 + n] = dsum;
+        __syncthreads();
         if (wave == 0 && g == 0 && q < T) {
-            float dsum = 0.f;
-            for (int d = 0; d < D; ++d) dsum += (float)slice(p.d_o, p.at_do)[(size_t)q * p.at_do.st + d] * sO[d * 33 + n];
+            dsum = 0.f;
+#pragma unroll
+            for (int k = 0; k < 2 * NW; ++k) dsum += red[k * 32 + n];
             if (p.split_rounds) {
                 float* part = p.delta + (((size_t)bh * 32 + n) * p.split_rounds + blockIdx.y) * 3;
                 part[0] = M; part[1] = L; part[2] = dsum;
@@ -296,8 +501,19 @@ __global__ __launch_bounds__(512) void tdp_f32_fwd_kernel(F32Params<E> p) {
             }
         }
         if (p.split_rounds) return;
+    } else if (p.deal.max_parts > 1) {
+        // perhaps one of several workgroups of the tile: its unnormalised output, reference and sum (f32_merge_kernel)
+        for (int idx = tid; idx < 32 * D; idx += NT) {
+            const int r = idx / D, d = idx % D;
+            if (q0 + r < T) p.part[(((size_t)bh * T + q0 + r) * p.deal.max_parts + part) * (D + 4) + d] = merged(d, r);
+        }
+        if (wave == 0 && g == 0 && q < T) {
+            float* ml = p.part + (((size_t)bh * T + q) * p.deal.max_parts + part) * (D + 4) + D;
+            ml[0] = M; ml[1] = L;
+        }
+        return;
     } else {
-        for (int idx = tid; idx < 32 * D; idx += 512) {
+        for (int idx = tid; idx < 32 * D; idx += NT) {
             const int r = idx / D, d = idx % D;
             if (q0 + r < T) {
                 float Lr = 0.f, Mr = kNegBig;
@@ -305,7 +521,7 @@ __global__ __launch_bounds__(512) void tdp_f32_fwd_kernel(F32Params<E> p) {
                 for (int w = 0; w < NW; ++w) Mr = fmaxf(Mr, sM[w * 32 + r]);
 #pragma unroll
                 for (int w = 0; w < NW; ++w) Lr += sL[w * 32 + r] * fast_exp2(sM[w * 32 + r] - Mr);
-                p.o[base + (size_t)(q0 + r) * D + d] = (E)(sO[d * 33 + r] / Lr);
+                p.o[base + (size_t)(q0 + r) * D + d] = (E)(merged(d, r) / Lr);
             }
         }
     }
@@ -328,8 +544,9 @@ __global__ __launch_bounds__(512) void tdp_f32_fwd_kernel(F32Params<E> p) {
 // fp32.  That is how the 16-bit backward runs its first query tile: for the first few causal queries the softmax
 // is nearly one-hot and dS = P (dP - Delta) cancels two O(10) numbers, which the 16-bit operands of the MFMA
 // kernels (dO * V2 rounded to 16 bit) cannot resolve.
-// D = 128: a workgroup produces DOUT = 64 of the gradient columns (blockIdx.y picks the half), and the B operands
-// of the score products are formed as they are used instead of being held in registers.
+// The operand reads and the walk over rounds and stages are the forward's; four waves per workgroup and two workgroups to a
+// CU at D <= 64 (B=4 H=8 T=512 D=64: 18.5 -> 13.5 ms, B=2 H=4 T=500: 20.0 -> 3.5; eight waves, one workgroup: 15.1 / 4.0).
+// DOUT < D: a workgroup produces DOUT of the gradient columns (blockIdx.y picks them).
 // the fp32 tensors' accumulators resolve 2^-36 of the slice's max |dO| and cover sums up to 2^27 times it
 constexpr int kF32FixedBias = 36;
 
@@ -346,9 +563,9 @@ struct F32BwdParams {
     // when non-null, LSE and Delta of query tile 0 come from the partials the split STATS launch left here
     const float* stats_part;
     int split_rounds;      // tile 0 only: rounds dealt out to workgroups (see tdp_f32_tile0_kernel), else 0
-    // tdp_f32_bwd_kernel: workgroups per query tile (blockIdx.z); workgroup z walks rounds m_lo + z, m_lo + z + parts, ...
-    // More than one needs acc_q where dQ is produced (each workgroup holds a share of it)
-    int round_parts;
+    // tdp_f32_bwd_kernel: the rounds of a tile dealt out to f32_tile_parts() workgroups.  max_parts above one needs acc_q
+    // where dQ is produced (each workgroup holds a share of it)
+    F32Deal deal;
     // fixed-point accumulators (common.hpp); scale_parts null: the accumulators are float
     const unsigned* scale_parts;
     unsigned* poison;
@@ -359,39 +576,58 @@ struct F32BwdParams {
     TdpMask mask;
 };
 
-__device__ __forceinline__ float half_sum(float v) {  // over the 32 lanes of a wave half
+// Sums over the 32 lanes of a wave half, of 16 registers of two tensors at once: lane n ends with the sum of register
+// 8 (n>>4 & 1) + 4 (n>>3 & 1) + 2 (n>>2 & 1) + (n>>1 & 1), of x in even lanes and of y in odd ones.  Every exchange halves
+// what is left to exchange: 31 of them, where register after register takes 160.
+__device__ __forceinline__ float half_sum_16x2(f32x16 x, f32x16 y) {
+    const int n = threadIdx.x & 31;
 #pragma unroll
-    for (int off = 16; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
+    for (int w = 8; w >= 1; w >>= 1) {
+        const bool up = n & (2 * w);
+#pragma unroll
+        for (int i = 0; i < w; ++i) {
+            const float kx = up ? x[i + w] : x[i], sx = up ? x[i] : x[i + w];
+            const float ky = up ? y[i + w] : y[i], sy = up ? y[i] : y[i + w];
+            x[i] = kx + __shfl_xor(sx, 2 * w, 64);
+            y[i] = ky + __shfl_xor(sy, 2 * w, 64);
+        }
+    }
+    const bool odd = n & 1;
+    return (odd ? y[0] : x[0]) + __shfl_xor(odd ? x[0] : y[0], 1, 64);
+}
+__device__ __forceinline__ int half_sum_register() {  // the register whose sum this lane ends with
+    return (threadIdx.x >> 1) & 15;
 }
 
 // `only_round` >= 0: this workgroup walks that round of rows only; else every `parts`-th round from the `part`-th on.
 // `bx` >= 0: the workgroup's place in a grid of its own (a kernel that runs these workgroups beside others passes it);
 // else blockIdx.x, and blockIdx.y picks the gradient columns
-template <typename E, int D, int DOUT, bool WITH_DQ>
-__device__ __forceinline__ void f32_bwd_body(const F32BwdParams<E>& p, int only_round, int part = 0, int parts = 1,
-                                             int bx = -1) {
-    constexpr int DTO = DOUT / 32, KS = D / 2, LD = D + 1, NW = kF32Waves;
-    // form the B operands of the score products as they are used (two LDS reads and a multiply per MFMA) instead of
-    // holding D / 2 of each in registers where the accumulators leave no room for them: both at D = 128, those of
-    // dP alone at D = 64 in the launch that also carries the dQ accumulators
-    constexpr bool FLY = D > 64, FLY_G = FLY || (D == 64 && WITH_DQ);
+template <typename E, int D, int DOUT, bool WITH_DQ, int NW>
+__device__ __forceinline__ void f32_bwd_body(const F32BwdParams<E>& p, int only_round, int bx = -1) {
+    constexpr int DTO = DOUT / 32, LD = f32_pitch<D>(), NT = 64 * NW;
+    using vDT = typename VecF<DTO>::type;
     // dQ of the tile, summed over the rounds: in registers up to 64 columns; beyond that the accumulators of a round
     // leave no room for it and it lives in LDS, where the waves add their round's share one after another
     constexpr bool DQ_LDS = WITH_DQ && DOUT > 64;
+    // B operands of the score products held in registers over a round, where the accumulators leave room for them;
+    // otherwise formed as they are used (two more LDS reads and four multiplies per four MFMAs)
+    constexpr bool HOLD_Q = D < 64 || (D == 64 && !WITH_DQ), HOLD_G = HOLD_Q;
     extern __shared__ __align__(16) float smem_f[];
     float* sK = smem_f;                 // [2][32][LD]
     float* sV = sK + 2 * 32 * LD;       // [2][32][LD]
     float* sQ = sV + 2 * 32 * LD;       // [32][LD]  Q * alpha * log2(e)
     float* sDO = sQ + 32 * LD;          // [32][LD]
-    float* sKb = sDO + 32 * LD;         // [NW][D]
-    float* sVb = sKb + NW * D;          // [NW][D]
-    float* sO = DQ_LDS ? sVb + NW * D : sK;  // [DOUT][33]  dQ of the tile (aliases the stages when it is only formed at the end)
+    float* sKb = sDO + 32 * LD;         // [2][NW][D]
+    float* sVb = sKb + 2 * NW * D;      // [2][NW][D]
+    float* sO = DQ_LDS ? sVb + 2 * NW * D : sK;  // dQ of the tile: [DOUT][33], or at the end [NW][DOUT][33], aliasing everything
 
     int bh, order;
     const int block_x = bx < 0 ? (int)blockIdx.x : bx;
-    if (!xcd_tile(p.BH, p.nqt, block_x >> 3, block_x & 7, bh, order)) return;
-    const int qt = p.nqt - 1 - order;
+    const bool tile0 = only_round >= 0;
+    if (!xcd_tile(p.BH, tile0 ? p.nqt : p.deal.items, block_x >> 3, block_x & 7, bh, order)) return;
+    const F32Item item = tile0 ? F32Item{p.nqt - 1 - order, 0, 1} : f32_item(p.deal, p.mask, order, p.nqt, p.T, NW);
+    const int qt = item.qt, part = item.part, step = item.parts;
+    if (part >= step) return;
     const int c0 = (bx < 0 ? (int)blockIdx.y : 0) * DOUT;  // first gradient column of this workgroup
 
     const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, g = lane >> 5;
@@ -417,8 +653,34 @@ __device__ __forceinline__ void f32_bwd_body(const F32BwdParams<E>& p, int only_
         m_lo = max(m_lo, only_round);
         m_hi = min(m_hi, only_round);
     }
-    if (parts > 1 && m_lo > m_hi) return;  // fewer rounds than workgroups: nothing to add (uniform, before any barrier)
-    for (int idx = tid; idx < 32 * D; idx += 512) {
+
+    StageE<E, D, NW> regs;
+    constexpr int kRowPer = (NW * D + NT - 1) / NT;
+    float row_k[kRowPer], row_v[kRowPer];
+    auto fetch_rows = [&](int m) {
+#pragma unroll
+        for (int i = 0; i < kRowPer; ++i) {
+            const int idx = min(tid + i * NT, NW * D - 1);
+            const size_t row = (size_t)min(m * NW + idx / D, T - 1);
+            row_k[i] = (float)KB[row * p.at_kb.st + idx % D];
+            row_v[i] = (float)VB[row * p.at_vb.st + idx % D];
+        }
+    };
+    auto store_rows = [&](int par) {
+#pragma unroll
+        for (int i = 0; i < kRowPer; ++i)
+            if (tid + i * NT < NW * D) {
+                sKb[par * NW * D + tid + i * NT] = row_k[i];
+                sVb[par * NW * D + tid + i * NT] = row_v[i];
+            }
+    };
+    Walk w{};
+    bool have = open_round<NW>(w, mask, m_lo, m_hi, step, q0, q1, T);
+    if (have) {
+        fetch_rows(w.m);
+        stage_fetch_e<E, D, NW>(regs, KA, VA, w.st * 32, T, p.at_ka.st, p.at_va.st);
+    }
+    for (int idx = tid; idx < 32 * D; idx += NT) {
         const int r = idx / D, d = idx % D;
         const size_t row = (size_t)min(q0 + r, T - 1);
         sQ[r * LD + d] = (float)Qs[row * p.at_q.st + d] * scale_log2;
@@ -428,13 +690,13 @@ __device__ __forceinline__ void f32_bwd_body(const F32BwdParams<E>& p, int only_
     float lse2 = 1.0e30f, delta = 0.f;
     if (q < T) {
         if (p.stats_part) {  // tile 0: join the partials of the rounds
-            const float* part = p.stats_part + ((size_t)bh * 32 + n) * p.split_rounds * 3;
+            const float* sp = p.stats_part + ((size_t)bh * 32 + n) * p.split_rounds * 3;
             float M = kNegBig, L = 0.f, num = 0.f;
-            for (int z = 0; z < p.split_rounds; ++z) M = fmaxf(M, part[z * 3]);
+            for (int z = 0; z < p.split_rounds; ++z) M = fmaxf(M, sp[z * 3]);
             for (int z = 0; z < p.split_rounds; ++z) {
-                const float w = fast_exp2(part[z * 3] - M);
-                L += part[z * 3 + 1] * w;
-                num += part[z * 3 + 2] * w;
+                const float wt = fast_exp2(sp[z * 3] - M);
+                L += sp[z * 3 + 1] * wt;
+                num += sp[z * 3 + 2] * wt;
             }
             lse2 = M + fast_log2(L);
             delta = num / L;
@@ -444,176 +706,231 @@ __device__ __forceinline__ void f32_bwd_body(const F32BwdParams<E>& p, int only_
         }
     }
 
-    f32x16 accDQ[DQ_LDS ? 1 : DTO];
+    f32x16 accDQ[DQ_LDS || !WITH_DQ ? 1 : DTO];
 #pragma unroll
-    for (int dt = 0; dt < (DQ_LDS ? 1 : DTO); ++dt)
+    for (int dt = 0; dt < (DQ_LDS || !WITH_DQ ? 1 : DTO); ++dt)
 #pragma unroll
         for (int i = 0; i < 16; ++i) accDQ[dt][i] = 0.f;
-    if constexpr (DQ_LDS)  // the first round's opening barrier orders this before the first addition
-        for (int idx = tid; idx < DOUT * 33; idx += 512) sO[idx] = 0.f;
+    if constexpr (DQ_LDS)
+        for (int idx = tid; idx < DOUT * 33; idx += NT) sO[idx] = 0.f;
+    f32x16 accQ[DTO], accT[DTO];
+#pragma unroll
+    for (int dt = 0; dt < DTO; ++dt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            accQ[dt][i] = 0.f;
+            accT[dt][i] = 0.f;
+        }
+    if (have) {
+        store_rows(0);
+        stage_store_e<E, D, NW>(regs, sK, sV);
+    }
+    __syncthreads();
 
-    StageE<E, D> regs;
-    for (int m = m_lo; m <= m_hi; m += parts) {
-        const int b = m * NW + wave;
-        const Range ra = streamed_range(mask, q0, q1, min(m * NW, T - 1), T);
-        const Range rb = streamed_range(mask, q0, q1, min(m * NW + NW - 1, T - 1), T);
-        const int st_lo = min(ra.lo, rb.lo) / 32, st_hi = max(ra.hi, rb.hi) / 32;
+    int buf = 0, par = 0;
+    f32x4v bq[HOLD_Q ? D / 8 : 1], bg[HOLD_G ? D / 8 : 1];
+    bool fresh = true;  // the first step of a round
+    while (have) {
+        const float* cK = sK + buf * 32 * LD;
+        const float* cV = sV + buf * 32 * LD;
+        const bool last = w.st == w.st_hi;  // of this round
+        Walk nw{w.m, w.st + 1, w.st_hi};
+        const bool more = last ? open_round<NW>(nw, mask, w.m + step, m_hi, step, q0, q1, T) : true;
+        if (more) {
+            stage_fetch_e<E, D, NW>(regs, KA, VA, nw.st * 32, T, p.at_ka.st, p.at_va.st);
+            if (last) fetch_rows(nw.m);
+        }
+        if (HOLD_Q && fresh) {
+            const float *kr = sKb + par * NW * D + wave * D + 4 * g, *vr = sVb + par * NW * D + wave * D + 4 * g;
+#pragma unroll
+            for (int c = 0; c < D / 8; ++c) {
+                const f32x4v qv = *reinterpret_cast<const f32x4v*>(sQ + n * LD + 4 * g + 8 * c);
+                const f32x4v kb = *reinterpret_cast<const f32x4v*>(kr + 8 * c);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) bq[HOLD_Q ? c : 0][e] = qv[e] * kb[e];
+                if constexpr (HOLD_G) {
+                    const f32x4v gv = *reinterpret_cast<const f32x4v*>(sDO + n * LD + 4 * g + 8 * c);
+                    const f32x4v vb = *reinterpret_cast<const f32x4v*>(vr + 8 * c);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) bg[c][e] = gv[e] * vb[e];
+                }
+            }
+        }
+        fresh = last;
+        const int b = w.m * NW + wave, a0 = w.st * 32;
         const bool row_ok = b <= rows.hi && b >= rows.lo;
         const Range mine = streamed_range(mask, q0, q1, min(b, T - 1), T);
-
-        __syncthreads();
-        for (int idx = tid; idx < NW * D; idx += 512) {
-            const int r = idx / D, d = idx % D;
-            const size_t row = (size_t)min(m * NW + r, T - 1);
-            sKb[idx] = (float)KB[row * p.at_kb.st + d];
-            sVb[idx] = (float)VB[row * p.at_vb.st + d];
-        }
-        if (st_lo <= st_hi) {
-            stage_fetch_e<E, D>(regs, KA, VA, st_lo * 32, T, p.at_ka.st, p.at_va.st);
-            stage_store_e<E, D>(regs, sK, sV);
-        }
-        __syncthreads();
-
-        float bq[FLY ? 1 : KS], bg[FLY_G ? 1 : KS];
-#pragma unroll
-        for (int s = 0; s < KS; ++s) {
-            if constexpr (!FLY) bq[s] = sQ[n * LD + g * KS + s] * sKb[wave * D + g * KS + s];
-            if constexpr (!FLY_G) bg[s] = sDO[n * LD + g * KS + s] * sVb[wave * D + g * KS + s];
-        }
-        f32x16 accQ[DTO], accT[DTO];
-#pragma unroll
-        for (int dt = 0; dt < DTO; ++dt)
+        const float *kb_row = sKb + par * NW * D + wave * D, *vb_row = sVb + par * NW * D + wave * D;
+        if (row_ok && a0 + 31 >= mine.lo && a0 <= mine.hi) {
+            f32x16 s, dp;
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
-                accQ[dt][i] = 0.f;
-                accT[dt][i] = 0.f;
+                s[i] = 0.f;
+                dp[i] = 0.f;
             }
-
-        for (int st = st_lo; st <= st_hi; ++st) {
-            const int buf = (st - st_lo) & 1;
-            const float* cK = sK + buf * 32 * LD;
-            const float* cV = sV + buf * 32 * LD;
-            const bool more = st < st_hi;
-            if (more) stage_fetch_e<E, D>(regs, KA, VA, (st + 1) * 32, T, p.at_ka.st, p.at_va.st);
-            const int a0 = st * 32;
-            if (row_ok && a0 + 31 >= mine.lo && a0 <= mine.hi) {
-                f32x16 s, dp;
+            // The per-lane parts of the LDS addresses, opaque to the compiler from here on: every read below is
+            // then this base plus a compile-time offset (the instruction's immediate field).  Left to itself the
+            // compiler computes the hundreds of addresses of the unrolled loops ahead of the loops and keeps them
+            // in registers (D = 128: 150 of them spilled to scratch memory).
+            int row_base = n * LD + 4 * g, own_base = 4 * g, out_base = 4 * g * LD + c0 + DTO * n;
+            asm volatile("" : "+v"(row_base), "+v"(out_base), "+v"(own_base));
 #pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    s[i] = 0.f;
-                    dp[i] = 0.f;
+            for (int c = 0; c < D / 8; ++c) {
+                const f32x4v ka = *reinterpret_cast<const f32x4v*>(cK + row_base + 8 * c);
+                const f32x4v va = *reinterpret_cast<const f32x4v*>(cV + row_base + 8 * c);
+                f32x4v oq, og;
+                if constexpr (HOLD_Q) {
+                    oq = bq[c];
+                } else {
+                    const f32x4v qv = *reinterpret_cast<const f32x4v*>(sQ + row_base + 8 * c);
+                    const f32x4v kb = *reinterpret_cast<const f32x4v*>(kb_row + own_base + 8 * c);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) oq[e] = qv[e] * kb[e];
                 }
-                // The per-lane parts of the LDS addresses, opaque to the compiler from here on: every read below is
-                // then this base plus a compile-time offset (the instruction's immediate field).  Left to itself the
-                // compiler computes the hundreds of addresses of the unrolled loops ahead of the loops and keeps them
-                // in registers (D = 128: 150 of them spilled to scratch memory).
-                int row_base = n * LD + g * KS, own_base = wave * D + g * KS, out_base = 4 * g * LD + c0 + n;
-                asm volatile("" : "+v"(row_base), "+v"(out_base), "+v"(own_base));
+                if constexpr (HOLD_G) {
+                    og = bg[c];
+                } else {
+                    const f32x4v gv = *reinterpret_cast<const f32x4v*>(sDO + row_base + 8 * c);
+                    const f32x4v vb = *reinterpret_cast<const f32x4v*>(vb_row + own_base + 8 * c);
 #pragma unroll
-                for (int ks = 0; ks < KS; ++ks) {
-                    const float oq = FLY ? sQ[row_base + ks] * sKb[own_base + ks] : bq[FLY ? 0 : ks];
-                    const float og = FLY_G ? sDO[row_base + ks] * sVb[own_base + ks] : bg[FLY_G ? 0 : ks];
-                    s = mma_f32(cK[row_base + ks], oq, s);
-                    dp = mma_f32(cV[row_base + ks], og, dp);
-                    // keep the operand reads of later k-steps from being hoisted over these (they would have to be
-                    // held in registers the accumulators need)
-                    if (FLY_G && (ks & 7) == 7) __builtin_amdgcn_sched_barrier(0);
+                    for (int e = 0; e < 4; ++e) og[e] = gv[e] * vb[e];
                 }
 #pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    const int a = a0 + c_row(g, i);
-                    const bool ok = a < T && tdp_valid(mask, q, a, b);
-                    const float pv = ok ? fast_exp2(s[i] - lse2) : 0.f;
-                    s[i] = pv;
-                    dp[i] = pv * (dp[i] - delta);
+                for (int e = 0; e < 4; ++e) {
+                    s = mma_f32(ka[e], oq[e], s);
+                    dp = mma_f32(va[e], og[e], dp);
                 }
-#pragma unroll
-                for (int dt = 0; dt < DTO; ++dt)
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) {
-                        // row c_row(g, i) = c_row(0, i) + 4 g
-                        accT[dt] = mma_f32(cV[out_base + c_row(0, i) * LD + dt * 32], s[i], accT[dt]);
-                        accQ[dt] = mma_f32(cK[out_base + c_row(0, i) * LD + dt * 32], dp[i], accQ[dt]);
-                        if (FLY_G && (i & 3) == 3) __builtin_amdgcn_sched_barrier(0);
-                    }
+                // operand reads stay within a chunk or two of their use (registers)
+                if (D > 64 || (c & 1)) __builtin_amdgcn_sched_barrier(0);
             }
-            if (more) {
-                stage_store_e<E, D>(regs, sK + (buf ^ 1) * 32 * LD, sV + (buf ^ 1) * 32 * LD);
-                __syncthreads();
+#pragma unroll
+            for (int i = 0; i < 16; ++i) s[i] = fast_exp2(s[i] - lse2);
+            if (!all_valid(mask, q0, a0, b, T)) {
+                const Interval ok = valid_interval(mask, q, b, T);
+                const int x = a0 + 4 * g - ok.lo;
+#pragma unroll
+                for (int i = 0; i < 16; ++i) s[i] = (unsigned)(x + c_row(0, i)) <= ok.span ? s[i] : 0.f;
+            }
+#pragma unroll
+            for (int i = 0; i < 16; ++i) dp[i] = s[i] * (dp[i] - delta);
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                // row c_row(g, i) = c_row(0, i) + 4 g
+                const vDT va = *reinterpret_cast<const vDT*>(cV + out_base + c_row(0, i) * LD);
+                const vDT ka = *reinterpret_cast<const vDT*>(cK + out_base + c_row(0, i) * LD);
+#pragma unroll
+                for (int dt = 0; dt < DTO; ++dt) {
+                    accT[dt] = mma_f32(vec_at<DTO>(va, dt), s[i], accT[dt]);
+                    accQ[dt] = mma_f32(vec_at<DTO>(ka, dt), dp[i], accQ[dt]);
+                }
+                if ((i & (DTO > 2 ? 1 : 3)) == (DTO > 2 ? 1 : 3)) __builtin_amdgcn_sched_barrier(0);
             }
         }
-        if (row_ok) {
-            int q_base = n * LD + c0 + 4 * g, kb_base = wave * D + c0 + 4 * g;  // opaque bases, as in the loop above
-            asm volatile("" : "+v"(q_base), "+v"(kb_base));
+        if (last) {
+            if (row_ok) {
+                int q_base = n * LD + c0 + 4 * DTO * g, kb_base = c0 + 4 * DTO * g;  // opaque bases, as above
+                asm volatile("" : "+v"(q_base), "+v"(kb_base));
+                if constexpr (WITH_DQ && !DQ_LDS) {
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) {
+                        const vDT k = *reinterpret_cast<const vDT*>(kb_row + kb_base + DTO * c_row(0, i));
+#pragma unroll
+                        for (int dt = 0; dt < DTO; ++dt) accDQ[dt][i] += accQ[dt][i] * vec_at<DTO>(k, dt);
+                    }
+                }
+#pragma unroll
+                for (int dt = 0; dt < DTO; ++dt) {
+                    // register i of half g is column d = c0 + DTO c_row(g, i) + dt.  sQ holds Q * alpha * log2(e):
+                    // alpha is wanted, log2(e) is not
+                    f32x16 xk, xv;
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) {
+                        const vDT qv = *reinterpret_cast<const vDT*>(sQ + q_base + DTO * c_row(0, i));
+                        const vDT gv = *reinterpret_cast<const vDT*>(sDO + q_base + DTO * c_row(0, i));
+                        xk[i] = accQ[dt][i] * vec_at<DTO>(qv, dt);
+                        xv[i] = accT[dt][i] * vec_at<DTO>(gv, dt);
+                    }
+                    const float sum = half_sum_16x2(xk, xv);
+                    const bool odd = n & 1;
+                    const int i = half_sum_register(), d = c0 + DTO * c_row(g, i) + dt;
+                    shared_add(odd ? p.acc_v : p.acc_k, base + (size_t)b * D + d, odd ? sum : sum * kLn2, fscale,
+                               p.poison + (size_t)bh * T + b, odd ? p.bit_v : p.bit_k);
+                    __builtin_amdgcn_sched_barrier(0);  // one tile's products and sums in registers at a time
+                }
+            }
+            if constexpr (DQ_LDS) {
+                // dQ[q] += Yq (.) K2[b], one wave after another: a fixed summation order (every wave takes part in the
+                // barriers, whether or not it had a row this round)
+                for (int v = 0; v < NW; ++v) {
+                    if (wave == v && row_ok) {
+                        int kb_base = c0 + 4 * DTO * g, o_base = 4 * DTO * g * 33 + n;
+                        asm volatile("" : "+v"(kb_base), "+v"(o_base));
+#pragma unroll
+                        for (int i = 0; i < 16; ++i) {
+                            const vDT k = *reinterpret_cast<const vDT*>(kb_row + kb_base + DTO * c_row(0, i));
+#pragma unroll
+                            for (int dt = 0; dt < DTO; ++dt)
+                                sO[o_base + (DTO * c_row(0, i) + dt) * 33] += accQ[dt][i] * vec_at<DTO>(k, dt);
+                        }
+                    }
+                    __syncthreads();
+                }
+            }
 #pragma unroll
             for (int dt = 0; dt < DTO; ++dt)
 #pragma unroll
                 for (int i = 0; i < 16; ++i) {
-                    const int d = c0 + dt * 32 + c_row(g, i), dc = dt * 32 + c_row(0, i);
-                    if constexpr (WITH_DQ && !DQ_LDS) accDQ[dt][i] += accQ[dt][i] * sKb[kb_base + dc];
-                    // sQ holds Q * alpha * log2(e): alpha is wanted, log2(e) is not
-                    const float rk = half_sum(accQ[dt][i] * sQ[q_base + dc]) * kLn2;
-                    const float rv = half_sum(accT[dt][i] * sDO[q_base + dc]);
-                    if (n == 0) {
-                        const size_t idx = base + (size_t)b * D + d;
-                        unsigned* prow = p.poison + (size_t)bh * T + b;
-                        shared_add(p.acc_k, idx, rk, fscale, prow, p.bit_k);
-                        shared_add(p.acc_v, idx, rv, fscale, prow, p.bit_v);
-                    }
+                    accQ[dt][i] = 0.f;
+                    accT[dt][i] = 0.f;
                 }
         }
-        if constexpr (DQ_LDS) {
-            // dQ[q] += Yq (.) K2[b], one wave after another: a fixed summation order (every wave takes part in the
-            // barriers, whether or not it had a row this round)
-            for (int w = 0; w < NW; ++w) {
-                if (wave == w && row_ok) {
-                    int kb_base = wave * D + c0 + 4 * g, o_base = 4 * g * 33 + n;
-                    asm volatile("" : "+v"(kb_base), "+v"(o_base));
-#pragma unroll
-                    for (int dt = 0; dt < DTO; ++dt)
-#pragma unroll
-                        for (int i = 0; i < 16; ++i) {
-                            const int dc = dt * 32 + c_row(0, i);
-                            sO[o_base + dc * 33] += accQ[dt][i] * sKb[kb_base + dc];
-                        }
-                }
-                __syncthreads();
+        if (more) {
+            buf ^= 1;
+            if (last) {
+                par ^= 1;
+                store_rows(par);
             }
+            stage_store_e<E, D, NW>(regs, sK + buf * 32 * LD, sV + buf * 32 * LD);
+            __syncthreads();
         }
+        w = nw;
+        have = more;
     }
 
     if constexpr (WITH_DQ) {
         __syncthreads();
-        if constexpr (!DQ_LDS) {
-            for (int idx = tid; idx < DOUT * 33; idx += 512) sO[idx] = 0.f;
+        if constexpr (!DQ_LDS) {  // the waves' shares side by side (sO), added in a fixed order below
+#pragma unroll
+            for (int dt = 0; dt < DTO; ++dt)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) sO[wave * DOUT * 33 + (DTO * c_row(g, i) + dt) * 33 + n] = accDQ[dt][i];
             __syncthreads();
-            for (int w = 0; w < NW; ++w) {  // one wave after another: a fixed summation order
-                if (wave == w) {
-#pragma unroll
-                    for (int dt = 0; dt < DTO; ++dt)
-#pragma unroll
-                        for (int i = 0; i < 16; ++i) sO[(dt * 32 + c_row(g, i)) * 33 + n] += accDQ[dt][i];
-                }
-                __syncthreads();
-            }
         }
-        for (int idx = tid; idx < 32 * DOUT; idx += 512) {
+        auto merged = [&](int d, int r) {
+            float v = sO[d * 33 + r];
+            if constexpr (!DQ_LDS) {
+#pragma unroll
+                for (int w = 1; w < NW; ++w) v += sO[(w * DOUT + d) * 33 + r];
+            }
+            return v;
+        };
+        for (int idx = tid; idx < 32 * DOUT; idx += NT) {
             const int r = idx / DOUT, d = idx % DOUT;
             if (q0 + r < T) {
                 const size_t off = base + (size_t)(q0 + r) * D + c0 + d;
                 if (p.acc_q)
                     shared_add(p.acc_q, p.acc_q_rows ? ((size_t)bh * p.acc_q_rows + q0 + r) * D + c0 + d : off,
-                               sO[d * 33 + r], fscale, p.poison + (size_t)bh * T + q0 + r, kPoisonDQ);
+                               merged(d, r), fscale, p.poison + (size_t)bh * T + q0 + r, kPoisonDQ);
                 else
-                    p.dq[off] = (E)(sO[d * 33 + r] * p.alpha);
+                    p.dq[off] = (E)(merged(d, r) * p.alpha);
             }
         }
     }
 }
 
-template <typename E, int D, int DOUT, bool WITH_DQ>
-__global__ __launch_bounds__(512) void tdp_f32_bwd_kernel(F32BwdParams<E> p) {
-    f32_bwd_body<E, D, DOUT, WITH_DQ>(p, -1, blockIdx.z, gridDim.z);
+template <typename E, int D, int DOUT, bool WITH_DQ, int NW>
+__global__ __launch_bounds__(64 * NW, 2) void tdp_f32_bwd_kernel(F32BwdParams<E> p) {
+    f32_bwd_body<E, D, DOUT, WITH_DQ, NW>(p, -1);
 }
 
 // Query tile 0 of a 16-bit backward, both launches' roles and all rounds at once: blockIdx.z = role * rounds + round
@@ -625,10 +942,10 @@ __device__ __forceinline__ void f32_tile0_block(const F32BwdParams<E>& r0, const
     const int role = z / r0.split_rounds, round = z % r0.split_rounds;
     if (!((roles_mask >> role) & 1)) return;
     if (role == 0) {
-        if (roles_mask & 4) f32_bwd_body<E, D, DOUT, true>(r0, round, 0, 1, bx);
-        else f32_bwd_body<E, D, DOUT, false>(r0, round, 0, 1, bx);
+        if (roles_mask & 4) f32_bwd_body<E, D, DOUT, true, kF32Waves>(r0, round, bx);
+        else f32_bwd_body<E, D, DOUT, false, kF32Waves>(r0, round, bx);
     } else {
-        f32_bwd_body<E, D, DOUT, false>(r1, round, 0, 1, bx);
+        f32_bwd_body<E, D, DOUT, false, kF32Waves>(r1, round, bx);
     }
 }
 template <typename E, int D, int DOUT>
@@ -636,15 +953,17 @@ __global__ __launch_bounds__(512) void tdp_f32_tile0_kernel(F32BwdParams<E> r0, 
     f32_tile0_block<E, D, DOUT>(r0, r1, roles_mask, blockIdx.z);
 }
 
-template <int D>
+template <int D, int NW = kF32Waves>
 constexpr size_t f32_bwd_smem() {
-    // stages, Q and dO, the rows of a round; D = 128: dQ of the tile (f32_bwd_body's DQ_LDS)
-    return sizeof(float) * (size_t)(4 * 32 * (D + 1) + 2 * 32 * (D + 1) + 2 * kF32Waves * D + (D > 64 ? D * 33 : 0));
+    // stages, Q and dO, the rows of two rounds; D = 128: dQ of the tile (f32_bwd_body's DQ_LDS); at the end the waves' dQ
+    constexpr int loop = 6 * 32 * f32_pitch<D>() + 4 * NW * D + (D > 64 ? D * 33 : 0), merge = NW * (D > 64 ? 64 : D) * 33;
+    return sizeof(float) * (size_t)(loop > merge ? loop : merge);
 }
 
-template <int D>
+template <int D, int NW>
 constexpr size_t f32_fwd_smem() {
-    return sizeof(float) * (size_t)(4 * 32 * (D + 1) + 32 * (D + 1) + 2 * kF32Waves * D + 2 * kF32Waves * 32);
+    constexpr int loop = 4 * 32 * f32_pitch<D>() + 4 * NW * D, merge = NW * D * 33;
+    return sizeof(float) * (size_t)(2 * NW * 32 + 32 * f32_pitch<D>() + (loop > merge ? loop : merge));
 }
 
 
@@ -686,17 +1005,18 @@ hipError_t tile0_prepare(const FirstTileArgs& a, hipStream_t st, F32BwdParams<E>
         p.split_rounds = rounds;
         p.zero_ptr = own_dq_acc ? (unsigned*)a.dq0_acc : nullptr;
         p.zero_words = own_dq_acc ? 32 * D * (a.scale_parts ? 2 : 1) : 0;
+        p.deal = F32Deal{0.f, 1, 1}; p.silu_va = false;
         p.T = a.T; p.BH = a.BH; p.nqt = 1;
         p.scale_log2 = a.alpha * kLog2e;
         p.mask = natural;
-        auto kern = tdp_f32_fwd_kernel<E, D, true>;
-        constexpr size_t smem = f32_fwd_smem<D>();
+        auto kern = tdp_f32_fwd_kernel<E, D, true, kF32Waves>;
+        constexpr size_t smem = f32_fwd_smem<D, kF32Waves>();
         if (hipError_t e = ensure_dynamic_smem(reinterpret_cast<const void*>(kern), smem); e != hipSuccess) return e;
         hipLaunchKernelGGL(kern, dim3(8 * xcd_slots(a.BH, 1), rounds), dim3(512), smem, st, p);
     }
     r0 = F32BwdParams<E>{};
     r0.q = (const E*)a.q; r0.d_o = (const E*)a.d_o; r0.lse = nullptr; r0.delta = nullptr;
-    r0.stats_part = a.delta_f32; r0.split_rounds = rounds; r0.round_parts = 1;
+    r0.stats_part = a.delta_f32; r0.split_rounds = rounds; r0.deal = F32Deal{0.f, 1, 1};
     r0.dq = (E*)a.dq; r0.acc_q = a.acc_q ? a.acc_q : a.dq0_acc; r0.acc_q_rows = a.acc_q ? 0 : 32;
     r0.scale_parts = a.scale_parts; r0.poison = a.poison; r0.scale_bias = a.scale_bias;
     r0.T = a.T; r0.BH = a.BH; r0.nqt = 1; r0.alpha = a.alpha;

@@ -74,10 +74,10 @@ const char* tritt_status_string(int status);
  * the same value; tritt_set_tuning changes a knob afterwards, stores its previous value in
  * *previous (which may be NULL) and returns TRITT_OK, or TRITT_ERR_INVALID for an unknown knob.
  * 0 = automatic.  Process-wide: do not change a knob while another thread is inside the library.
- *   TRITT_TUNE_FWD_SPLITS   (env TRITT_FWD_SPLITS)     workgroups per query tile in the triple-dot forward, 1..8
+ *   TRITT_TUNE_FWD_SPLITS   (env TRITT_FWD_SPLITS)     workgroups per query tile in the triple-dot forward, 1..8 (fp32: at most, 1..16)
  *   TRITT_TUNE_FWD_BAND     (env TRITT_FWD_BAND=0)     -1: narrow windowed masks take the streaming forward
  *                                                      instead of the band-resident one
- *   TRITT_TUNE_BWD_SPLITS   (env TRITT_BWD_SPLITS)     workgroups per query tile in the triple-dot backward, 1..16
+ *   TRITT_TUNE_BWD_SPLITS   (env TRITT_BWD_SPLITS)     workgroups per query tile in the triple-dot backward, 1..16 (fp32: at most)
  *   TRITT_TUNE_BWD128_WAVES (env TRITT_BWD128_VARIANT=w8|w4)  the D = 128 backward under full windows: 0 = 16 queries per
  *                           wave on 16x16x32 tiles (the default); 8 | 4 = the 32-query kernels with 8 or 4 waves
  *   TRITT_TUNE_F32_VALU     (env TRITT_F32_VALU=1)     1: the fp32 path runs the VALU kernels at every head dimension (instead of the

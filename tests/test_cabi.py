@@ -35,6 +35,18 @@ def test_version_and_status_strings():
     assert b"head dimension" in lib.tritt_status_string(-2)
 
 
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("T", [31, 449])
+def test_workspace_of_the_fp32_backward_of_16_bit_tensors_holds_a_forward(D, T):
+    """That call forms the output once more in fp32: copies of the inputs, the accumulators and everything the forward
+    itself asks for, the parts of a split forward included."""
+    lib = _lib.lib()
+    shape = (1, 1, T, D, _lib.TRITT_F16, 1, T, T, T, T, _lib.FLAG_FORCE_GENERIC)
+    forward, backward = lib.tritt_tdp_fwd_workspace_bytes(*shape), lib.tritt_tdp_bwd_workspace_bytes(*shape)
+    accumulators = 5 * T * D * 8
+    assert backward >= forward + accumulators + T * D * 4  # ... and dO in fp32
+
+
 def test_workspace_queries_scale_with_problem():
     lib = _lib.lib()
     a = lib.tritt_tdp_bwd_workspace_bytes(1, 2, 64, 32, _lib.TRITT_F32, 1, 64, 64, 64, 64, 1)

@@ -92,6 +92,23 @@ def test_fp32_tensors_on_the_matrix_cores(D, causal, windows, tune):
         util.assert_close(f"{name} vs VALU kernels", a, b, **FP32)
 
 
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("T", [1, 31, 33, 65, 161])
+@pytest.mark.parametrize("splits", [0, 1, 3])
+def test_fp32_rounds_dealt_out_to_workgroups(D, T, splits, tune):
+    """The fp32 matrix-core kernels with the rounds of a query tile in one workgroup, in at most three and in as many as
+    the launcher picks: single rows, tile edges, and a mask whose middle rounds see no key at all (a wide k window over a
+    narrow j window)."""
+    print(f"case fp32 rounds D={D} T={T} splits={splits}", flush=True)
+    tune(_lib.TUNE_FWD_SPLITS, splits)
+    tune(_lib.TUNE_BWD_SPLITS, splits)
+    inputs = orc.make_inputs(1, 3, T, D, torch.float32, seed=T + D)
+    # one row has one (j, k) pair: its dQ, dK1 and dK2 are exactly zero, so only the absolute bar means anything
+    rel = 1e-4 if T > 1 else math.inf
+    for causal, windows in ((True, (None,) * 4), (True, (5, 150, 3, 4)), (False, (None,) * 4)):
+        check_all(inputs, 1 / math.sqrt(D), causal, windows, rel=rel)
+
+
 @pytest.mark.parametrize("causal", [True, False])
 def test_fp32_head_dim_128_large_grid_on_the_matrix_cores(causal, tune):
     """D = 128 with enough query tiles that each is walked by one workgroup (dQ written by that workgroup, its running
