@@ -81,6 +81,24 @@ def lib():
     return _lib
 
 
+_native = None
+
+
+def native():
+    """The extension that takes torch tensors to the library in native code (csrc/torch_front.cpp): `tdp` and `dps`, which
+    return None where the Python autograd Functions have to decide."""
+    global _native
+    if _native is None:
+        lib()  # same error when nothing is built
+        try:
+            from . import _native as module
+        except ImportError as e:
+            raise RuntimeError(f"flash_trittention/_native.so cannot be loaded ({e}): build it with "
+                               f"`make -C {CSRC_DIR}` (there is no fallback implementation)") from e
+        _native = module
+    return _native
+
+
 def exported_symbols():
     return list(_PROTOS)
 

@@ -86,5 +86,12 @@ class TrittentionTriton(nn.Module):
 
     def forward(self, q, k1, k2, v1, v2):
         """q, k1, k2, v1, v2: [B, N, S, D] -> (o [B, N, S, D], m [B, N, S] fp32 logsumexp)."""
+        if not _ops.compiling() and self._function is TrittentionTritonFunction:
+            # the usual call stays in native code, forward and backward (csrc/torch_front.cpp); None: what the Function
+            # below handles or refuses
+            out = _lib.native().dps(q, k1, k2, v1, v2, self.causal, self.softmax_scale, self.k_diff,
+                                    self.convert_to_float32)
+            if out is not None:
+                return out
         return self._function.apply(q, k1, k2, v1, v2, self.causal, self.softmax_scale, self.k_diff,
                                                self.convert_to_float32, self.input_precision)

@@ -116,6 +116,13 @@ def flash_trittention(q, k1, k2, v1, v2, softmax_scale=1 / 8, kk_left=1, kk_righ
         warnings.warn(
             "flash_trittention: `input_precision` is currently unused and has no effect "
             f"(got {input_precision!r}).", stacklevel=2)
+    if not _ops.compiling():
+        # the usual call stays in native code, forward and backward (csrc/torch_front.cpp); None: checks that fail, tensors
+        # that are not on a GPU and the like, which the Function below handles or refuses
+        out = _lib.native().tdp(q, k1, k2, v1, v2, softmax_scale, kk_left, kk_right, k1_window, k2_window, causal,
+                                convert_to_float32)
+        if out is not None:
+            return out
     return FlashTrittention.apply(q, k1, k2, v1, v2, softmax_scale, kk_left, kk_right, k1_window, k2_window, causal,
                                   convert_to_float32)
 
