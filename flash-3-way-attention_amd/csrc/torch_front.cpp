@@ -5,16 +5,20 @@
 // they do (a ctypes call with thirty arguments, five to ten allocations and a dozen tensor queries from the interpreter; for
 // the backward also the hand-over of the engine's thread to the interpreter): 38 us per forward, 100-130 us per backward.
 //
-// tdp() and dps() take the usual case only and return None for everything else -- tensors that are not on a GPU, shapes,
-// types or windows that do not fit, tensor subclasses and functorch wrappers -- which the Python Functions then handle or
-// refuse as they always did.  Nothing is computed here and nothing is kept between calls.
+// tdp() and dps() take the usual case only and return None for everything else -- tensors that are not plain GPU tensors
+// (subclasses, wrappers, tangents), shapes, types or windows that do not fit, calls under a functorch transform or a
+// tracer -- which the Python Functions then handle or refuse as they always did.  Nothing is computed here and nothing is
+// kept between calls.
 #include <Python.h>
 
 #include <ATen/ATen.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include <array>
 #include <optional>
@@ -128,8 +132,10 @@ struct Tdp : torch::autograd::Function<Tdp> {
     static variable_list backward(AutogradContext* ctx, variable_list grad) {
         const variable_list s = ctx->get_saved_variables();
         const Problem p = load(ctx);
-        const std::array<Tensor, 5> in{s[0], s[1], s[2], s[3], s[4]};
-        const Tensor &q = s[0], &o = s[5], &lse = s[6];
+        // a saved-tensor hook may bring a tensor back in another layout
+        const std::array<Tensor, 5> in{view(s[0]), view(s[1]), view(s[2]), view(s[3]), view(s[4])};
+        const Tensor& q = in[0];
+        const Tensor o = s[5].contiguous(), lse = s[6].contiguous();
         const c10::OptionalDeviceGuard guard(q.device());
         const Tensor d_o = view(grad[0].scalar_type() == q.scalar_type() ? grad[0] : grad[0].to(q.scalar_type()));
         const int B = (int)q.size(0), H = (int)q.size(1), T = (int)q.size(2), D = (int)q.size(3);
@@ -195,8 +201,9 @@ struct Dps : torch::autograd::Function<Dps> {
     static variable_list backward(AutogradContext* ctx, variable_list grad) {
         const variable_list s = ctx->get_saved_variables();
         const Problem p = load(ctx);
-        const std::array<Tensor, 5> in{s[0], s[1], s[2], s[3], s[4]};
-        const Tensor &q = s[0], &o = s[5], &m = s[6];
+        const std::array<Tensor, 5> in{view(s[0]), view(s[1]), view(s[2]), view(s[3]), view(s[4])};
+        const Tensor& q = in[0];
+        const Tensor o = s[5].contiguous(), m = s[6].contiguous();
         const c10::OptionalDeviceGuard guard(q.device());
         if (grad[0].sizes() != o.sizes() || grad[0].device() != o.device() || grad[0].scalar_type() != o.scalar_type())
             throw std::runtime_error("TrittentionTriton: dO must have the shape, the device and the dtype of O");
@@ -231,16 +238,26 @@ struct Dps : torch::autograd::Function<Dps> {
 };
 
 // ---- Python entry points -------------------------------------------------------------------------------------------------
+// Whether a Python Function would see its arguments as they are: no functorch transform is active (it refuses or rewrites
+// Functions, also where no argument is wrapped) and torch.jit.trace, which records a Python Function, is not recording.
+bool plain_context() {
+    return !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) &&
+           !torch::jit::tracer::isTracing();
+}
 // the five tensors of a call in the usual case
 std::optional<std::array<Tensor, 5>> usual_tensors(PyObject* const* args) {
+    if (!plain_context()) return std::nullopt;
+    // a GPU tensor with or without autograd; any other key (Python, functorch, Functionalize, Conjugate, Negative,
+    // ZeroTensor, ...) is a wrapper or a lazy form whose storage is not the tensor
+    static const c10::DispatchKeySet plain =
+        c10::DispatchKeySet{c10::DispatchKey::CUDA, c10::DispatchKey::AutogradCUDA, c10::DispatchKey::ADInplaceOrView,
+                            c10::DispatchKey::AutocastCUDA};
     std::array<Tensor, 5> t;
     for (int i = 0; i < 5; ++i) {
-        if (!THPVariable_Check(args[i])) return std::nullopt;
+        if (!THPVariable_CheckExact(args[i])) return std::nullopt;
         t[i] = THPVariable_Unpack(args[i]);
-        const auto keys = t[i].key_set();
-        if (!t[i].is_cuda() || t[i].layout() != at::kStrided || keys.has(c10::DispatchKey::Python) ||
-            keys.has(c10::DispatchKey::FuncTorchBatched) || keys.has(c10::DispatchKey::FuncTorchGradWrapper) ||
-            t[i].is_conj() || t[i].is_neg())
+        if (!t[i].is_cuda() || t[i].layout() != at::kStrided || (t[i].key_set().raw_repr() & ~plain.raw_repr()) ||
+            t[i]._fw_grad(0).defined())
             return std::nullopt;
         if (t[i].dim() != 4 || dtype_code(t[i].scalar_type()) < 0) return std::nullopt;
         if (i && (t[i].sizes() != t[0].sizes() || t[i].scalar_type() != t[0].scalar_type() || t[i].device() != t[0].device()))
@@ -277,32 +294,30 @@ bool number(PyObject* o, double* out) {
     return false;
 }
 
-template <typename F>
-PyObject* guarded(F f) {
-    try {
-        return f();
-    } catch (const std::exception& e) {
-        if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, e.what());
-        return nullptr;
-    }
+bool truth(PyObject* o, bool* out) {
+    const int v = PyObject_IsTrue(o);
+    *out = v == 1;
+    if (v >= 0) return true;
+    PyErr_Clear();
+    return false;
 }
 
 // tdp(q, k1, k2, v1, v2, softmax_scale, kk_left, kk_right, k1_window, k2_window, causal, convert_to_float32) -> O or None
 PyObject* py_tdp(PyObject*, PyObject* const* args, Py_ssize_t n) {
-    return guarded([&]() -> PyObject* {
+    HANDLE_TH_ERRORS  // torch's own exception types, and those of Python code called back (saved-tensor hooks)
         if (n != 12) {
             PyErr_SetString(PyExc_TypeError, "tdp takes 12 arguments");
             return nullptr;
         }
         auto t = usual_tensors(args);
         Problem p{};
-        if (!t || !number(args[5], &p.scale)) Py_RETURN_NONE;
+        bool convert = false;
+        if (!t || !number(args[5], &p.scale) || !truth(args[10], &p.causal) || !truth(args[11], &convert)) Py_RETURN_NONE;
         const int64_t T = (*t)[0].size(2), D = (*t)[0].size(3);
         if (!window(args[8], T, &p.w[0]) || !window(args[9], T, &p.w[1]) || !window(args[6], T, &p.w[2]) ||
             !window(args[7], T, &p.w[3]))
             Py_RETURN_NONE;
-        p.causal = PyObject_IsTrue(args[10]) == 1;
-        if (PyObject_IsTrue(args[11]) == 1)
+        if (convert)
             p.flags = ((*t)[0].scalar_type() != at::kFloat && (D == 32 || D == 64)) ? TRITT_FLAG_SPLIT_OPERANDS
                                                                                      : TRITT_FLAG_FORCE_GENERIC;
         Tensor o;
@@ -311,21 +326,23 @@ PyObject* py_tdp(PyObject*, PyObject* const* args, Py_ssize_t n) {
             o = Tdp::apply((*t)[0], (*t)[1], (*t)[2], (*t)[3], (*t)[4], p);
         }
         return THPVariable_Wrap(std::move(o));
-    });
+    END_HANDLE_TH_ERRORS
 }
 
 // dps(q, k1, k2, v1, v2, causal, softmax_scale, k_diff, convert_to_float32) -> (o, m) or None
 PyObject* py_dps(PyObject*, PyObject* const* args, Py_ssize_t n) {
-    return guarded([&]() -> PyObject* {
+    HANDLE_TH_ERRORS
         if (n != 9) {
             PyErr_SetString(PyExc_TypeError, "dps takes 9 arguments");
             return nullptr;
         }
         auto t = usual_tensors(args);
         Problem p{};
-        if (!t || !number(args[6], &p.scale) || !window(args[7], (*t)[0].size(2), &p.w[0])) Py_RETURN_NONE;
-        p.causal = PyObject_IsTrue(args[5]) == 1;
-        if (PyObject_IsTrue(args[8]) == 1) p.flags = TRITT_FLAG_FORCE_GENERIC;
+        bool convert = false;
+        if (!t || !number(args[6], &p.scale) || !window(args[7], (*t)[0].size(2), &p.w[0]) || !truth(args[5], &p.causal) ||
+            !truth(args[8], &convert))
+            Py_RETURN_NONE;
+        if (convert) p.flags = TRITT_FLAG_FORCE_GENERIC;
         variable_list r;
         {
             pybind11::gil_scoped_release release;
@@ -335,7 +352,7 @@ PyObject* py_dps(PyObject*, PyObject* const* args, Py_ssize_t n) {
         if (!pair) return nullptr;
         for (int i = 0; i < 2; ++i) PyTuple_SET_ITEM(pair, i, THPVariable_Wrap(std::move(r[i])));
         return pair;
-    });
+    END_HANDLE_TH_ERRORS
 }
 
 PyMethodDef methods[] = {

@@ -2,6 +2,7 @@
 so every result is bit for bit the same; and the calls it leaves to them."""
 import pytest
 import torch
+import torch.utils.checkpoint
 
 from flash_trittention import TrittentionTriton, _lib, flash_trittention
 from flash_trittention.dot_product_sum.trittention_triton import TrittentionTritonFunction
@@ -91,3 +92,75 @@ def test_native_backward_takes_another_dtype_and_refuses_changed_inputs():
         a[1].add_(1)
     with pytest.raises(RuntimeError, match="modified by an inplace operation"):
         torch.autograd.grad(out, a, grad)
+
+
+FULL = dict(k1_window=None, k2_window=None, kk_left=None, kk_right=None)
+
+
+def test_native_path_leaves_transforms_traces_and_tangents_to_the_functions():
+    *ins, _ = make(torch.float32, False)
+    native = _lib.native()
+    call = lambda *t: native.tdp(*t, 0.1, None, None, None, None, True, False)
+    assert call(*ins) is not None
+
+    class Tagged(torch.Tensor):
+        pass
+
+    assert call(ins[0].as_subclass(Tagged), *ins[1:]) is None
+    assert call(torch.nn.Parameter(ins[0]), *ins[1:]) is not None
+    seen = []
+
+    def under(x):  # nothing of the call is wrapped, the transform is active all the same
+        seen.append(call(*ins))
+        return x
+
+    torch.func.vmap(under)(torch.zeros(3))
+    assert seen == [None]
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(ins[0], torch.ones_like(ins[0]))
+        assert call(dual, *ins[1:]) is None
+    traced = torch.jit.trace(lambda *t: flash_trittention(*t, **FULL), tuple(ins), check_trace=False)
+    other = [t.flip(2).contiguous() for t in ins]
+    assert torch.equal(traced(*other), flash_trittention(*other, **FULL))  # recorded, not a constant
+
+
+def test_native_path_under_saved_tensor_hooks():
+    """Hooks that move the saved tensors away and back, one that brings them back in another layout, and recomputation
+    (checkpoint stops it with an exception out of a hook)."""
+    *ins, grad = make(torch.bfloat16, False)
+    a = leaves(ins, (1,) * 5)
+    want = torch.autograd.grad(flash_trittention(*a, **FULL), a, grad)
+
+    def other_layout(t):
+        big = torch.empty(t.numel() * 2 + 1, dtype=t.dtype, device=t.device)[1:]
+        wide = big.view(*t.shape, 2)[..., 0]
+        wide.copy_(t)
+        return wide
+
+    for pack, unpack in ((lambda t: t.cpu(), lambda t: t.cuda()), (other_layout, lambda t: t)):
+        with torch.autograd.graph.saved_tensors_hooks(pack, unpack):
+            out = flash_trittention(*a, **FULL)
+            o2, _ = TrittentionTriton(softmax_scale=0.2, k_diff=40)(*a)
+        assert all(torch.equal(x, y) for x, y in zip(want, torch.autograd.grad(out, a, grad)))
+        ref, _ = TrittentionTriton(softmax_scale=0.2, k_diff=40)(*a)
+        assert all(torch.equal(x, y) for x, y in
+                   zip(torch.autograd.grad(o2, a, grad), torch.autograd.grad(ref, a, grad)))
+    out = torch.utils.checkpoint.checkpoint(lambda *t: flash_trittention(*t, **FULL) * 1, *a, use_reentrant=False)
+    assert all(torch.equal(x, y) for x, y in zip(want, torch.autograd.grad(out, a, grad)))
+
+    class Stop(Exception):
+        pass
+
+    def stop(t):
+        raise Stop
+
+    with pytest.raises(Stop), torch.autograd.graph.saved_tensors_hooks(stop, lambda t: t):
+        flash_trittention(*a, **FULL)
+
+
+def test_native_path_arguments_without_a_truth_value():
+    *ins, _ = make(torch.bfloat16, False)
+    with pytest.raises(RuntimeError, match="ambiguous"):
+        flash_trittention(*ins, causal=torch.ones(2), **FULL)
+    with pytest.raises(RuntimeError, match="ambiguous"):
+        flash_trittention(*ins, convert_to_float32=torch.ones(2), **FULL)
