@@ -330,7 +330,7 @@ int dps_fwd_impl(Arena& ar, bool run, const void* q, const void* k1, const void*
     F32Inputs in = plan_inputs(ar, q, k1, k2, v2, n, dtype, copies, &u);
     float* o32 = dtype == TRITT_F32 ? (float*)o : ar.take<float>(n);
     DpsArgs a{};
-    a.r = ar.take<float>(n);
+    if (!use_f32_mfma_dps(D)) a.r = ar.take<float>(n);
     a.w = ar.take<float>(n);
     a.lse1 = ar.take<float>(rows);
     if (!run) return TRITT_OK;
@@ -353,12 +353,16 @@ int dps_bwd_impl(Arena& ar, bool run, const void* q, const void* k1, const void*
     float *copies[4], *u;
     F32Inputs in = plan_inputs(ar, q, k1, k2, v2, n, dtype, copies, &u);
     float* do32 = dtype == TRITT_F32 ? (float*)d_o : ar.take<float>(n);
+    const bool mfma32 = use_f32_mfma_dps(D), in_place = mfma32 && dtype == TRITT_F32;
     DpsArgs a{};
-    a.r = ar.take<float>(n); a.w = ar.take<float>(n); a.dw = ar.take<float>(n); a.dr = ar.take<float>(n);
+    a.r = ar.take<float>(n); a.w = ar.take<float>(n); a.dr = ar.take<float>(n);
     a.dk2_part = ar.take<float>(n);
-    a.lse1 = ar.take<float>(rows); a.delta = ar.take<float>(rows);
-    a.dlse1 = ar.take<float>(rows); a.delta1 = ar.take<float>(rows);
-    float* du = ar.take<float>(n);
+    a.lse1 = ar.take<float>(rows); a.delta = ar.take<float>(rows); a.delta1 = ar.take<float>(rows);
+    if (!mfma32) {
+        a.dw = ar.take<float>(n);
+        a.dlse1 = ar.take<float>(rows);
+    }
+    float* du = in_place ? (float*)dv1 : ar.take<float>(n);
     float *dq32 = (float*)dq, *dk132 = (float*)dk1, *dk232 = (float*)dk2, *dv232 = (float*)dv2;
     if (dtype != TRITT_F32) {
         dq32 = ar.take<float>(n); dk132 = ar.take<float>(n); dk232 = ar.take<float>(n); dv232 = ar.take<float>(n);
@@ -370,24 +374,26 @@ int dps_bwd_impl(Arena& ar, bool run, const void* q, const void* k1, const void*
     float* lse32 = dtype != TRITT_F32 ? ar.take<float>(rows) : nullptr;
     if (!run) return TRITT_OK;
     if (ar.overflows()) return TRITT_ERR_WORKSPACE;
-    fill_inputs(q, k1, k2, v1, v2, n, dtype, copies, u, st);
+    if (!in_place) fill_inputs(q, k1, k2, v1, v2, n, dtype, copies, u, st);
     if (dtype != TRITT_F32) to_f32<false>(d_o, do32, n, dtype, st);
     a.q = in.q; a.k1 = in.k1; a.k2 = in.k2; a.u = in.u; a.v2 = in.v2;
     a.BH = B * H; a.T = T; a.D = D; a.alpha = alpha; a.causal = causal; a.k_diff = k_diff;
     if (o32) {
         a.o = o32; a.lse = lse32;
-        hipError_t ef = use_f32_mfma_dps(D) ? f32_mfma_dps_fwd(a, st) : dps_fwd(a, st);
+        hipError_t ef = mfma32 ? f32_mfma_dps_fwd(a, st) : dps_fwd(a, st);
         if (ef != hipSuccess) return (int)ef;
         rowdot(do32, o32, a.delta, (int)rows, D, TRITT_F32, st);
         lse = lse32;
+    } else if (in_place) {
+        a.v1 = (const float*)v1; a.o_in = (const float*)o;
     } else {
         rowdot(d_o, o, a.delta, (int)rows, D, dtype, st);
     }
     a.lse = const_cast<float*>(lse); a.d_o = do32;
     a.dq = dq32; a.dk1 = dk132; a.dk2 = dk232; a.du = du; a.dv2 = dv232;
-    hipError_t e = use_f32_mfma_dps(D) ? f32_mfma_dps_bwd(a, st) : dps_bwd(a, st);
+    hipError_t e = mfma32 ? f32_mfma_dps_bwd(a, st) : dps_bwd(a, st);
     if (e != hipSuccess) return (int)e;
-    from_f32(du, v1, dv1, n, dtype, st);
+    if (!in_place) from_f32(du, v1, dv1, n, dtype, st);
     if (dtype != TRITT_F32) {
         from_f32(dq32, nullptr, dq, n, dtype, st);
         from_f32(dk132, nullptr, dk1, n, dtype, st);

@@ -2,18 +2,27 @@
 //
 // The same two chained attention passes as dps_kernels.hip (inner: lse1, R = softmax_s(alpha K1_s.K2_t) @ U;
 // outer: softmax_t(alpha Q_q.K2_t + lse1[t]) @ (R * V2); backward = the two attention backwards chained through
-// dR and dlse1) and the same three kernels with the same arguments, "attention with a per-key bias" forward,
-// backward by owner rows and backward by owner columns; only the products run on the fp32 MFMA instead of one
-// lane per row on the vector ALUs.  True fp32 operands, products and accumulation (the 1e-4 bar of fp32 tensors).
+// dR and dlse1): "attention with a per-key bias" forward, backward by owner rows and backward by owner columns, the
+// last two in one launch.  True fp32 operands, products and accumulation (the 1e-4 bar of fp32 tensors).
 //
-// Tiling.  A workgroup = two waves = 64 owner rows (32 per wave, one per MFMA column = lane % 32); the other
-// operand's rows stream through LDS in 32-row tiles shared by the two waves (fetched into registers one tile
-// ahead, row stride D + 1 floats).  A 32x32 score tile is D / 2 MFMAs with the contraction split by lane half:
-//   S^T[a, r] = sum_ks  Ka[a][g D/2 + ks] * Xr[r][g D/2 + ks]        (A from LDS, B from the owner's registers)
+// Tiling.  A workgroup owns 32 rows (one per MFMA column = lane % 32) in all of its waves; the 32-row tiles of the other
+// operand are dealt out to the waves in turn, each wave sums its own share and the shares are joined through LDS at the
+// end.  A step of 32 x 32 pairs is 64-128 MFMAs of 64 cycles, so the serial chain of steps of one wave is what a call
+// of a few hundred owner tiles waits for: with one wave per owner tile and the streamed tiles shared through LDS
+// (B = 2, H = 8, T = 1000, D = 64: half a wave per SIMD, up to 32 steps of 4.4 us one after another) a training step
+// took 589 us, now 205; larger grids gain from the loads and the missing barriers (B = 4, H = 16, T = 2048: 7.1 -> 3.1 ms,
+// 110 TFLOP/s executed of 157).  What bounds it now: the MFMAs at that rate, below it the chain.  Operands come from L2 straight into registers
+// (16 KB per step and wave: a quarter of what L2 gives a CU in the time of the step's MFMAs), without LDS and without a
+// barrier inside the loop; a register set is loaded again as soon as the product that reads it has been issued, so every
+// load has at least one product (2048 cycles) to arrive in.
+//
+// A 32x32 score tile is D / 2 MFMAs with the contraction dealt out to the lane halves in pieces of four,
+//   S^T[a, r] = sum Ka[a][8 j + 4 g + e] * Xr[r][8 j + 4 g + e]       (A: 16-byte loads of a row, B: owner's registers)
 // It leaves the MFMA with lane <-> owner row and registers <-> streamed rows (row c_row(g, i) in register i), which
 // is the B-operand layout of the output products
-//   O^T[d, r] += sum_a V^T[d, a] P^T[a, r]                            (A from LDS, B = the P registers)
+//   O^T[d, r] += sum_a V^T[d, a] P^T[a, r]                            (A: loads along a row, B = the P registers)
 // so P never moves between lanes and every per-owner quantity (running maximum, sums, LSE, Delta) is lane-local.
+// MFMA row n of output tile dt is column d = (D / 32) n + dt, so that a lane's loads are as wide as D allows.
 // One owner per output element: no atomics, bitwise reproducible.
 #include "common.hpp"
 #include "kernels.hpp"
@@ -25,421 +34,572 @@ namespace {
 __device__ __forceinline__ f32x16 mma2(float a, float b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
 }
+__device__ __forceinline__ void pin_order() { __builtin_amdgcn_sched_barrier(0); }
 
-constexpr int kOwnerRows = 64;  // per workgroup
+constexpr int kWaves = 4;  // per workgroup; every wave walks each kWaves-th tile of the workgroup's range
 
 // valid pair (owner-like row r attends key-like row a)
 __device__ __forceinline__ bool pair_valid(int causal, int k_diff, int r, int a) {
     return !causal || ((a <= r) & (r - a <= k_diff));
 }
 
-// Two 32 x D fp32 tiles (rows row0 .. row0 + 31 of A and of B, clamped to T - 1) through registers into LDS.
+// Rows row0 .. row0 + 31 of a head's row-major [T][D] operand (row0 is uniform).  A buffer resource of the rows that
+// exist: rows past T read as zeros, one lane offset serves all loads, and no 64-bit address is kept per lane.
 template <int D>
-struct Stage2 {
-    static constexpr int kPer = 32 * D / 4 / 128;  // float4 pieces per thread and tensor
-    float4 a[kPer], b[kPer];
-};
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rows(const float* src, int row0, int T) {
+    row0 = __builtin_amdgcn_readfirstlane(row0);
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(src) + (size_t)row0 * D, 0, min(32, T - row0) * D * 4, 0x00020000);
+}
+// as A operand of a score product: lane n holds row n
 template <int D>
-__device__ __forceinline__ void stage_fetch2(Stage2<D>& s, const float* __restrict__ A, const float* __restrict__ B,
-                                             int row0, int T) {
-    constexpr int kVec = D / 4;
+__device__ __forceinline__ void load_rows(float (&reg)[D / 2], const float* src, int row0, int T, int n, int g) {
+    const __amdgpu_buffer_rsrc_t rows = tile_rows<D>(src, row0, T);
 #pragma unroll
-    for (int i = 0; i < Stage2<D>::kPer; ++i) {
-        const int idx = threadIdx.x + i * 128, row = min(row0 + idx / kVec, T - 1), c = idx % kVec;
-        s.a[i] = *reinterpret_cast<const float4*>(A + (size_t)row * D + c * 4);
-        s.b[i] = *reinterpret_cast<const float4*>(B + (size_t)row * D + c * 4);
+    for (int j = 0; j < D / 8; ++j) {
+        const auto v = __builtin_amdgcn_raw_buffer_load_b128(rows, (n * D + 4 * g) * 4 + 32 * j, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) reg[4 * j + e] = __uint_as_float(v[e]);
     }
 }
+// as A operand of an output product: lane n holds columns DT n .. DT n + DT - 1 of rows c_row(g, 0 .. 15)
 template <int D>
-__device__ __forceinline__ void stage_store2(const Stage2<D>& s, float* sA, float* sB) {
-    constexpr int kVec = D / 4, LD = D + 1;
-#pragma unroll
-    for (int i = 0; i < Stage2<D>::kPer; ++i) {
-        const int idx = threadIdx.x + i * 128, row = idx / kVec, c = idx % kVec;
-        float* pa = sA + row * LD + c * 4;
-        float* pb = sB + row * LD + c * 4;
-        pa[0] = s.a[i].x; pa[1] = s.a[i].y; pa[2] = s.a[i].z; pa[3] = s.a[i].w;
-        pb[0] = s.b[i].x; pb[1] = s.b[i].y; pb[2] = s.b[i].z; pb[3] = s.b[i].w;
-    }
-}
-
-// With one or two waves per SIMD a chain of MFMAs that accumulate into one tile waits for each result in turn, so
-// every loop below walks two independent accumulators alternately.
-// S^T tile: rows = the 32 staged rows, columns = the wave's owner rows; `own` = the owner's operand registers
-template <int D>
-__device__ __forceinline__ f32x16 score_tile(const float* sT, const float (&own)[D / 2], int n, int g) {
-    constexpr int KS = D / 2, LD = D + 1;
-    f32x16 s, t;
+__device__ __forceinline__ void load_cols(float (&reg)[D / 2], const float* src, int row0, int T, int n, int g) {
+    const __amdgpu_buffer_rsrc_t rows = tile_rows<D>(src, row0, T);
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-        s[i] = 0.f;
-        t[i] = 0.f;
+        const int at = (4 * g * D + D / 32 * n) * 4, row = (8 * (i / 4) + i % 4) * D * 4;
+        if constexpr (D == 64) {
+            const auto v = __builtin_amdgcn_raw_buffer_load_b64(rows, at + row % 4096, row / 4096 * 4096, 0);
+            reg[2 * i] = __uint_as_float(v[0]);
+            reg[2 * i + 1] = __uint_as_float(v[1]);
+        } else {
+            reg[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rows, at + row, 0, 0));
+        }
     }
+}
+// one value per streamed row, lane n <-> row row0 + n (0 past T)
+__device__ __forceinline__ float load_vec(const float* src, int row0, int T, int n) {
+    const __amdgpu_buffer_rsrc_t rows = tile_rows<1>(src, row0, T);
+    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rows, 4 * n, 0, 0));
+}
+template <int D>
+__device__ __forceinline__ f32x16 score_tile(const float (&rows)[D / 2], const float (&own)[D / 2]) {
+    f32x16 s;
 #pragma unroll
-    for (int ks = 0; ks < KS; ks += 2) {
-        s = mma2(sT[n * LD + g * KS + ks], own[ks], s);
-        t = mma2(sT[n * LD + g * KS + ks + 1], own[ks + 1], t);
-    }
+    for (int i = 0; i < 16; ++i) s[i] = 0.f;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) s[i] += t[i];
+    for (int ks = 0; ks < D / 2; ++ks) s = mma2(rows[ks], own[ks], s);
     return s;
 }
-// two score tiles at once (S from sA / ownA, dP from sB / ownB)
+// acc^T[d, owner] += sum over the 32 streamed rows of cols[row, d] * w[row, owner]   (w in score-tile layout)
 template <int D>
-__device__ __forceinline__ void score_tiles(const float* sA, const float (&ownA)[D / 2], const float* sB,
-                                            const float (&ownB)[D / 2], f32x16& s, f32x16& dp, int n, int g) {
-    constexpr int KS = D / 2, LD = D + 1;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        s[i] = 0.f;
-        dp[i] = 0.f;
-    }
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-        s = mma2(sA[n * LD + g * KS + ks], ownA[ks], s);
-        dp = mma2(sB[n * LD + g * KS + ks], ownB[ks], dp);
-    }
-}
-// acc^T[d, owner] += sum over the staged rows of T^T[d, row] * w[row, owner]   (w in score-tile layout)
-template <int D>
-__device__ __forceinline__ void output_tile(f32x16 (&acc)[D / 32], const float* sT, const f32x16& w, int n, int g) {
-    constexpr int LD = D + 1, DT = D / 32;
-    if constexpr (DT == 1) {  // one column tile: split the staged rows over two accumulators
-        f32x16 t;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) t[i] = 0.f;
-#pragma unroll
-        for (int i = 0; i < 16; i += 2) {
-            acc[0] = mma2(sT[c_row(g, i) * LD + n], w[i], acc[0]);
-            t = mma2(sT[c_row(g, i + 1) * LD + n], w[i + 1], t);
-        }
-#pragma unroll
-        for (int i = 0; i < 16; ++i) acc[0][i] += t[i];
-    } else {
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-#pragma unroll
-            for (int dt = 0; dt < DT; ++dt) acc[dt] = mma2(sT[c_row(g, i) * LD + dt * 32 + n], w[i], acc[dt]);
-    }
-}
-// two output products at once
-template <int D>
-__device__ __forceinline__ void output_tiles(f32x16 (&accA)[D / 32], const float* sA, const f32x16& wa,
-                                             f32x16 (&accB)[D / 32], const float* sB, const f32x16& wb, int n, int g) {
-    constexpr int LD = D + 1, DT = D / 32;
+__device__ __forceinline__ void output_tile(f32x16 (&acc)[D / 32], const float (&cols)[D / 2], const f32x16& w) {
+    constexpr int DT = D / 32;
 #pragma unroll
     for (int i = 0; i < 16; ++i)
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) {
-            accA[dt] = mma2(sA[c_row(g, i) * LD + dt * 32 + n], wa[i], accA[dt]);
-            accB[dt] = mma2(sB[c_row(g, i) * LD + dt * 32 + n], wb[i], accB[dt]);
-        }
+        for (int dt = 0; dt < DT; ++dt) acc[dt] = mma2(cols[i * DT + dt], w[i], acc[dt]);
+}
+template <int D>
+__device__ __forceinline__ void clear(f32x16 (&acc)[D / 32]) {
+#pragma unroll
+    for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[dt][i] = 0.f;
 }
 
-// heavy-first tile order under a causal mask (the last owner tiles stream the most rows)
-__device__ __forceinline__ int owner_tile(int causal) { return causal ? gridDim.x - 1 - blockIdx.x : blockIdx.x; }
+// The waves' shares of a 32 x D result, joined in wave order.
+template <int D>
+struct Shares {
+    static constexpr int LD = D + 4, kPieces = 32 * D / 4;  // 16-byte pieces of the result: thread t takes t, t + 256, ...
+    alignas(16) float part[kWaves][32 * LD];
+    float row[kWaves][32], row2[kWaves][32];  // per owner row and wave
+    alignas(16) float vec[kWaves][2][32];                 // one value per streamed row of a wave's step, on its way into the registers
+    alignas(16) float own[32 * LD];                       // the backward's owner rows X or K, scaled
+
+    // lane n's values of the wave's 32 streamed rows, in score-tile order (register i: row c_row(g, i)).  Only the wave
+    // itself writes and reads its slots and its LDS accesses stay in order.
+    __device__ __forceinline__ void vec_put(int which, float v, int wave, int n) {
+        vec[wave][which][n] = v;
+        asm volatile("" ::: "memory");
+    }
+    __device__ __forceinline__ float4 vec_get(int which, int wave, int g, int i4) const {
+        return *reinterpret_cast<const float4*>(&vec[wave][which][8 * i4 + 4 * g]);
+    }
+    // this wave's registers, scaled per owner row
+    __device__ __forceinline__ void put(const f32x16 (&acc)[D / 32], float f, int wave, int n, int g) {
+        float* mine = part[wave] + n * LD;
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4) {
+            const int i = 4 * i4;
+            if constexpr (D == 64) {  // registers i .. i + 3 of both tiles are eight consecutive columns
+                float* p = mine + 16 * i4 + 8 * g;
+                *reinterpret_cast<float4*>(p) = make_float4(acc[0][i] * f, acc[1][i] * f, acc[0][i + 1] * f, acc[1][i + 1] * f);
+                *reinterpret_cast<float4*>(p + 4) =
+                    make_float4(acc[0][i + 2] * f, acc[1][i + 2] * f, acc[0][i + 3] * f, acc[1][i + 3] * f);
+            } else {
+                *reinterpret_cast<float4*>(mine + 8 * i4 + 4 * g) =
+                    make_float4(acc[0][i] * f, acc[0][i + 1] * f, acc[0][i + 2] * f, acc[0][i + 3] * f);
+            }
+        }
+    }
+    __device__ __forceinline__ float4 sum(int piece) const {
+        const int at = piece / (D / 4) * LD + piece % (D / 4) * 4;
+        float4 o = *reinterpret_cast<const float4*>(part[0] + at);
+#pragma unroll
+        for (int w = 1; w < kWaves; ++w) {
+            const float4 e = *reinterpret_cast<const float4*>(part[w] + at);
+            o.x += e.x; o.y += e.y; o.z += e.z; o.w += e.w;
+        }
+        return o;
+    }
+};
 
 // Attention forward with an optional per-key bias (log2 units):
 //   out[r] = softmax_a(scale X[r].K[a] + bias[a]) @ V ;  lse_out[r] = lse_scale * log2-sum-exp2
-//   out_mul[r] = out[r] * mul[r]   (when mul != nullptr)
+//   out_mul[r] = out[r] * mul[r]   (when mul != nullptr; out may then be null)
+struct FwdP {
+    const float *X, *K, *V, *bias, *mul;
+    float *out, *out_mul, *lse_out;
+    float lse_scale, scale_log2;
+    int BH, T, causal, k_diff;
+};
 template <int D>
-__global__ __launch_bounds__(128, 2) void attn_fwd_f32m_kernel(
-    const float* __restrict__ X, const float* __restrict__ K, const float* __restrict__ V,
-    const float* __restrict__ bias, const float* __restrict__ mul, float* __restrict__ out,
-    float* __restrict__ out_mul, float* __restrict__ lse_out, float lse_scale, int T, float scale_log2, int causal,
-    int k_diff) {
-    constexpr int DT = D / 32, KS = D / 2, LD = D + 1;
-    __shared__ float sK[32 * LD], sV[32 * LD], sBias[32];
-    const size_t base = (size_t)blockIdx.y * T * D, vbase = (size_t)blockIdx.y * T;
-    X += base; K += base; V += base;
-    const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, g = lane >> 5, wave = tid >> 6;
-    const int r0 = owner_tile(causal) * kOwnerRows, r = r0 + wave * 32 + n, rc = min(r, T - 1);
-    const int r_hi = min(T - 1, r0 + kOwnerRows - 1);
-    const int a_lo = causal ? max(0, r0 - k_diff) : 0, a_hi = causal ? r_hi : T - 1;
-    // this wave's owner rows and the staged rows they can reach
-    const int wr_lo = r0 + wave * 32, wr_hi = min(T - 1, wr_lo + 31);
+__global__ __launch_bounds__(64 * kWaves, 2) void attn_fwd_f32m_kernel(FwdP p) {
+    constexpr int DT = D / 32, KS = D / 2;
+    __shared__ Shares<D> sh;
+    const int T = p.T, ntiles = (T + 31) / 32;
+    int bh, order;
+    if (!xcd_tile(p.BH, ntiles, blockIdx.x >> 3, blockIdx.x & 7, bh, order)) return;
+    const size_t base = (size_t)bh * T * D, vbase = (size_t)bh * T;
+    const float *X = p.X + base, *K = p.K + base, *V = p.V + base;
+    const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, g = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // heavy first: under a causal mask the last owner tiles stream the most rows
+    const int r0 = (p.causal ? ntiles - 1 - order : order) * 32, r = r0 + n;
+    const int a_lo = p.causal ? max(0, r0 - p.k_diff) & ~31 : 0, a_hi = p.causal ? min(T - 1, r0 + 31) : T - 1;
 
-    float x[KS];
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) x[ks] = X[(size_t)rc * D + g * KS + ks] * scale_log2;
     f32x16 acc[DT];
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) acc[dt][i] = 0.f;
+    clear<D>(acc);
     float m = -INFINITY, l = 0.f;
-
-    Stage2<D> st;
-    const int a_first = a_lo & ~31;
-    stage_fetch2<D>(st, K, V, a_first, T);
-    for (int a0 = a_first; a0 <= a_hi; a0 += 32) {
-        __syncthreads();
-        stage_store2<D>(st, sK, sV);
-        if (tid < 32) sBias[tid] = bias ? bias[vbase + min(a0 + tid, T - 1)] : 0.f;
-        __syncthreads();
-        if (a0 + 32 <= a_hi) stage_fetch2<D>(st, K, V, a0 + 32, T);
-        if (wr_lo >= T) continue;  // a wave with no row inside the sequence (ragged last tile)
-        if (causal && (a0 > wr_hi || a0 + 31 < wr_lo - k_diff)) continue;  // nothing in reach of this wave
-        f32x16 s = score_tile<D>(sK, x, n, g);
-        float mx = -INFINITY;
+    int a0 = a_lo + 32 * wave;
+    if (a0 <= a_hi) {
+        float bias = p.bias ? load_vec(p.bias + vbase, a0, T, n) : 0.f;
+        float x[KS], rows[KS], cols[KS];
+        load_rows<D>(x, X, r0, T, n, g);
+        load_rows<D>(rows, K, a0, T, n, g);
+        load_cols<D>(cols, V, a0, T, n, g);
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int a = a0 + c_row(g, i);
-            const bool ok = (a < T) & (r < T) & pair_valid(causal, k_diff, r, a);
-            s[i] = ok ? s[i] + sBias[c_row(g, i)] : -INFINITY;
-            mx = fmaxf(mx, s[i]);
-        }
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-        const float m_new = fmaxf(m, mx);
-        const float f = m_new == -INFINITY ? 1.f : fast_exp2(m - m_new);  // nothing seen yet: keep the zeros
-        float ps = 0.f;
+        for (int ks = 0; ks < KS; ++ks) x[ks] *= p.scale_log2;
+        for (; a0 <= a_hi; a0 += 32 * kWaves) {
+            const int next = min(a0 + 32 * kWaves, a_hi & ~31);  // (past the end: in bounds, not used)
+            if (p.bias) sh.vec_put(0, bias, wave, n);
+            // two chains: with the one wave per SIMD of a small call an accumulating chain waits for each of its results
+            f32x16 s, t;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            s[i] = s[i] == -INFINITY ? 0.f : fast_exp2(s[i] - m_new);
-            ps += s[i];
-        }
-        ps += __shfl_xor(ps, 32, 64);
-        l = l * f + ps;
-        m = m_new;
+            for (int i = 0; i < 16; ++i) {
+                s[i] = 0.f;
+                t[i] = 0.f;
+            }
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
+            for (int ks = 0; ks < KS; ks += 2) {
+                s = mma2(rows[ks], x[ks], s);
+                t = mma2(rows[ks + 1], x[ks + 1], t);
+            }
+            pin_order();
+            load_rows<D>(rows, K, next, T, n, g);
+            if (p.bias) bias = load_vec(p.bias + vbase, next, T, n);
+            pin_order();
 #pragma unroll
-            for (int i = 0; i < 16; ++i) acc[dt][i] *= f;
-        output_tile<D>(acc, sV, s, n, g);
-    }
-    if (r < T) {
-        const float inv = 1.0f / l;
+            for (int i = 0; i < 16; ++i) s[i] += t[i];
+            if (p.bias) {
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-            for (int i4 = 0; i4 < 4; ++i4) {
-                // registers 4 i4 .. 4 i4 + 3 are four consecutive columns d of row r
-                const size_t off = base + (size_t)r * D + dt * 32 + c_row(g, i4 * 4);
-                const float4 o = make_float4(acc[dt][i4 * 4] * inv, acc[dt][i4 * 4 + 1] * inv, acc[dt][i4 * 4 + 2] * inv,
-                                             acc[dt][i4 * 4 + 3] * inv);
-                *reinterpret_cast<float4*>(out + off) = o;
-                if (mul) {
-                    const float4 mm = *reinterpret_cast<const float4*>(mul + off);
-                    *reinterpret_cast<float4*>(out_mul + off) = make_float4(o.x * mm.x, o.y * mm.y, o.z * mm.z, o.w * mm.w);
+                for (int i4 = 0; i4 < 4; ++i4) {
+                    const float4 b = sh.vec_get(0, wave, g, i4);
+                    s[4 * i4] += b.x; s[4 * i4 + 1] += b.y; s[4 * i4 + 2] += b.z; s[4 * i4 + 3] += b.w;
                 }
             }
-        if (g == 0) lse_out[vbase + r] = (m + fast_log2(l)) * lse_scale;
+            if (a0 + 32 > T || (p.causal && (a0 + 31 > r0 || r0 + 31 - a0 > p.k_diff))) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    const int a = a0 + c_row(g, i);
+                    s[i] = ((a < T) & pair_valid(p.causal, p.k_diff, r, a)) ? s[i] : -INFINITY;
+                }
+            }
+            float mx = s[0];
+#pragma unroll
+            for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
+            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+            const float m_new = fmaxf(m, mx);
+            const float f = m_new == -INFINITY ? 1.f : fast_exp2(m - m_new);  // nothing seen yet: keep the zeros
+            float ps = 0.f;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                s[i] = s[i] == -INFINITY ? 0.f : fast_exp2(s[i] - m_new);
+                ps += s[i];
+            }
+            ps += __shfl_xor(ps, 32, 64);
+            l = l * f + ps;
+            m = m_new;
+            if (__any(f != 1.f)) {
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) acc[dt][i] *= f;
+            }
+            output_tile<D>(acc, cols, s);
+            pin_order();
+            load_cols<D>(cols, V, next, T, n, g);
+            pin_order();
+        }
+    }
+    if (g == 0) sh.row[wave][n] = m;
+    __syncthreads();
+    float M = sh.row[0][n];
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) M = fmaxf(M, sh.row[w][n]);
+    const float f = m == -INFINITY ? 0.f : fast_exp2(m - M);  // a share without a valid pair is zeros
+    sh.put(acc, f, wave, n, g);
+    if (g == 0) sh.row2[wave][n] = l * f;
+    __syncthreads();
+#pragma unroll
+    for (int piece = tid; piece < Shares<D>::kPieces; piece += 64 * kWaves) {
+        const int row = piece / (D / 4), c = piece % (D / 4) * 4;
+        float L = sh.row2[0][row], Mr = sh.row[0][row];
+#pragma unroll
+        for (int w = 1; w < kWaves; ++w) {
+            L += sh.row2[w][row];
+            Mr = fmaxf(Mr, sh.row[w][row]);
+        }
+        if (r0 + row < T) {
+            const float inv = 1.0f / L;
+            float4 o = sh.sum(piece);
+            o.x *= inv; o.y *= inv; o.z *= inv; o.w *= inv;
+            const size_t off = base + (size_t)(r0 + row) * D + c;
+            if (p.out) *reinterpret_cast<float4*>(p.out + off) = o;
+            if (p.mul) {
+                const float4 mm = *reinterpret_cast<const float4*>(p.mul + off);
+                *reinterpret_cast<float4*>(p.out_mul + off) = make_float4(o.x * mm.x, o.y * mm.y, o.z * mm.z, o.w * mm.w);
+            }
+            if (c == 0) p.lse_out[vbase + r0 + row] = (Mr + fast_log2(L)) * p.lse_scale;
+        }
     }
 }
 
-// Attention backward, owner = query-like row r:
-//   P = exp2(scale X[r].K[a] + bias[a] - lse2[r]);  dS = P (G[r].V[a] - delta[r]);
-//   dX[r] = alpha * sum_a dS K[a]  (+ addend[r])
-template <int D>
-__global__ __launch_bounds__(128, 2) void attn_bwd_row_f32m_kernel(
-    const float* __restrict__ X, const float* __restrict__ G, const float* __restrict__ K,
-    const float* __restrict__ V, const float* __restrict__ bias, const float* __restrict__ lse, float lse_to_log2,
-    const float* __restrict__ delta, const float* __restrict__ addend, float* __restrict__ dX, int T, float alpha,
-    int causal, int k_diff) {
-    constexpr int DT = D / 32, KS = D / 2, LD = D + 1;
-    __shared__ float sK[32 * LD], sV[32 * LD], sBias[32];
-    const size_t base = (size_t)blockIdx.y * T * D, vbase = (size_t)blockIdx.y * T;
-    X += base; G += base; K += base; V += base;
-    const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, g = lane >> 5, wave = tid >> 6;
-    const int r0 = owner_tile(causal) * kOwnerRows, r = r0 + wave * 32 + n, rc = min(r, T - 1);
-    const int r_hi = min(T - 1, r0 + kOwnerRows - 1);
-    const int a_lo = causal ? max(0, r0 - k_diff) : 0, a_hi = causal ? r_hi : T - 1;
-    const int wr_lo = r0 + wave * 32, wr_hi = min(T - 1, wr_lo + 31);
-    const float scale_log2 = alpha * kLog2e;
+// Attention backward.  P = exp2(scale X[r].K[a] + bias[a] - lse2[r]);  dS = P (G[r].V[a] - delta[r]).
+//   owner = query-like row r:  dX[r] = alpha * sum_a dS K[a]  (+ addend[r])
+//   owner = key-like row a:    dK[a] = alpha * sum_r dS X[r];  dV[a] = sum_r P G[r];  dbias[a] = sum_r dS
+// Both directions are one launch (neither reads what the other writes); odd places of the grid's order take rows.
+// What becomes of dV is the caller's choice:
+//   mid != nullptr  the outer pass: dV is dW, the gradient of W = R * V2:  mid_out = dW * R,  dR = dW * V2 and
+//                   delta1 = rowsum(dR * R) - dbias
+//   v1 != nullptr   the inner pass of fp32 tensors: dV = the gradient of SiLU(V1), times SiLU'(V1)
+struct BwdP {
+    const float *X, *G, *K, *V, *bias, *lse, *delta, *addend;
+    float *dX, *dK, *dV;
+    const float *mid_r, *mid_v2, *v1;
+    float *dR, *delta1;
+    float lse_to_log2, alpha;
+    int BH, T, causal, k_diff;
+};
 
-    float x[KS], gg[KS];
+// In the backward one of the owner's two operands is read from LDS in every step (8 reads for 32 MFMAs at D = 64): with it
+// in registers beside the accumulators, two operand sets, the other operand and the score tiles the kernel spills at 256.
+template <int D>
+__device__ __forceinline__ void own_put(Shares<D>& sh, const float* src, int row0, int T, float scale, int tid) {
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-        x[ks] = X[(size_t)rc * D + g * KS + ks] * scale_log2;
-        gg[ks] = G[(size_t)rc * D + g * KS + ks];
+    for (int piece = tid; piece < Shares<D>::kPieces; piece += 64 * kWaves) {
+        const int row = piece / (D / 4), c = piece % (D / 4) * 4;
+        float4 x = *reinterpret_cast<const float4*>(src + (size_t)min(row0 + row, T - 1) * D + c);
+        x.x *= scale; x.y *= scale; x.z *= scale; x.w *= scale;
+        *reinterpret_cast<float4*>(sh.own + row * Shares<D>::LD + c) = x;
     }
-    const float lse2 = lse[vbase + rc] * lse_to_log2, dl = delta[vbase + rc];
+}
+template <int D>
+__device__ __forceinline__ f32x16 score_tile(const float (&rows)[D / 2], const Shares<D>& sh, int n, int g) {
+    f32x16 s;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s[i] = 0.f;
+    asm volatile("" ::: "memory");  // (the reads stay inside the caller's loop)
+#pragma unroll
+    for (int j = 0; j < D / 8; ++j) {
+        const float4 x = *reinterpret_cast<const float4*>(sh.own + n * Shares<D>::LD + 8 * j + 4 * g);
+        s = mma2(rows[4 * j], x.x, s);
+        s = mma2(rows[4 * j + 1], x.y, s);
+        s = mma2(rows[4 * j + 2], x.z, s);
+        s = mma2(rows[4 * j + 3], x.w, s);
+    }
+    return s;
+}
+
+template <int D>
+__device__ __forceinline__ void bwd_rows(const BwdP& p, Shares<D>& sh, int bh, int tile, int tid, int wave, int n, int g) {
+    constexpr int DT = D / 32, KS = D / 2;
+    const int T = p.T;
+    const size_t base = (size_t)bh * T * D, vbase = (size_t)bh * T;
+    const float *X = p.X + base, *G = p.G + base, *K = p.K + base, *V = p.V + base;
+    const int r0 = tile * 32, r = r0 + n, rc = min(r, T - 1);
+    const int a_lo = p.causal ? max(0, r0 - p.k_diff) & ~31 : 0, a_hi = p.causal ? min(T - 1, r0 + 31) : T - 1;
+    const float scale_log2 = p.alpha * kLog2e;
     f32x16 acc[DT];
+    clear<D>(acc);
+    int a0 = a_lo + 32 * wave;
+    own_put<D>(sh, X, r0, T, scale_log2, tid);
+    __syncthreads();
+    if (a0 <= a_hi) {
+        float bias = p.bias ? load_vec(p.bias + vbase, a0, T, n) : 0.f;
+        float gg[KS], ra[KS], rb[KS];
+        load_rows<D>(ra, K, a0, T, n, g);
+        load_rows<D>(gg, G, r0, T, n, g);
+        load_rows<D>(rb, V, a0, T, n, g);
+        const float lse2 = p.lse[vbase + rc] * p.lse_to_log2, dl = p.delta[vbase + rc];
+        // two operand sets in turn: the K rows of the next step take the set the V rows are in now
+        auto step = [&](float (&A)[KS], float (&B)[KS]) {
+            const int next = min(a0 + 32 * kWaves, a_hi & ~31);
+            if (p.bias) sh.vec_put(0, bias, wave, n);
+            f32x16 s = score_tile<D>(A, sh, n, g);
+            pin_order();
+            load_cols<D>(A, K, a0, T, n, g);
+            if (p.bias) bias = load_vec(p.bias + vbase, next, T, n);
+            pin_order();
+            const f32x16 dp = score_tile<D>(B, gg);
+            pin_order();
+            load_rows<D>(B, K, next, T, n, g);
+            pin_order();
+            if (p.bias) {
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) acc[dt][i] = 0.f;
-
-    Stage2<D> st;
-    const int a_first = a_lo & ~31;
-    stage_fetch2<D>(st, K, V, a_first, T);
-    for (int a0 = a_first; a0 <= a_hi; a0 += 32) {
-        __syncthreads();
-        stage_store2<D>(st, sK, sV);
-        if (tid < 32) sBias[tid] = bias ? bias[vbase + min(a0 + tid, T - 1)] : 0.f;
-        __syncthreads();
-        if (a0 + 32 <= a_hi) stage_fetch2<D>(st, K, V, a0 + 32, T);
-        if (wr_lo >= T) continue;
-        if (causal && (a0 > wr_hi || a0 + 31 < wr_lo - k_diff)) continue;
-        f32x16 s, dp;
-        score_tiles<D>(sK, x, sV, gg, s, dp, n, g);
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int a = a0 + c_row(g, i);
-            const bool ok = (a < T) & (r < T) & pair_valid(causal, k_diff, r, a);
-            s[i] = ok ? fast_exp2(s[i] + sBias[c_row(g, i)] - lse2) * (dp[i] - dl) : 0.f;
-        }
-        output_tile<D>(acc, sK, s, n, g);
-    }
-    if (r < T) {
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-            for (int i4 = 0; i4 < 4; ++i4) {
-                const size_t off = base + (size_t)r * D + dt * 32 + c_row(g, i4 * 4);
-                float4 o = make_float4(acc[dt][i4 * 4] * alpha, acc[dt][i4 * 4 + 1] * alpha, acc[dt][i4 * 4 + 2] * alpha,
-                                       acc[dt][i4 * 4 + 3] * alpha);
-                if (addend) {
-                    const float4 e = *reinterpret_cast<const float4*>(addend + off);
-                    o.x += e.x; o.y += e.y; o.z += e.z; o.w += e.w;
+                for (int i4 = 0; i4 < 4; ++i4) {
+                    const float4 b = sh.vec_get(0, wave, g, i4);
+                    s[4 * i4] += b.x; s[4 * i4 + 1] += b.y; s[4 * i4 + 2] += b.z; s[4 * i4 + 3] += b.w;
                 }
-                *reinterpret_cast<float4*>(dX + off) = o;
             }
+            const bool edge = a0 + 32 > T || (p.causal && (a0 + 31 > r0 || r0 + 31 - a0 > p.k_diff));
+#pragma unroll
+            for (int i = 0; i < 16; ++i) s[i] = fast_exp2(s[i] - lse2) * (dp[i] - dl);
+            if (edge) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    const int a = a0 + c_row(g, i);
+                    s[i] = ((a < T) & pair_valid(p.causal, p.k_diff, r, a)) ? s[i] : 0.f;
+                }
+            }
+            output_tile<D>(acc, A, s);
+            pin_order();
+            load_rows<D>(A, V, next, T, n, g);
+            pin_order();
+        };
+        while (true) {
+            step(ra, rb);
+            a0 += 32 * kWaves;
+            if (a0 > a_hi) break;
+            step(rb, ra);
+            a0 += 32 * kWaves;
+            if (a0 > a_hi) break;
+        }
+    }
+    sh.put(acc, p.alpha, wave, n, g);
+    __syncthreads();
+#pragma unroll
+    for (int piece = tid; piece < Shares<D>::kPieces; piece += 64 * kWaves) {
+        const int row = piece / (D / 4), c = piece % (D / 4) * 4;
+        if (r0 + row >= T) continue;
+        float4 o = sh.sum(piece);
+        const size_t off = base + (size_t)(r0 + row) * D + c;
+        if (p.addend) {
+            const float4 e = *reinterpret_cast<const float4*>(p.addend + off);
+            o.x += e.x; o.y += e.y; o.z += e.z; o.w += e.w;
+        }
+        *reinterpret_cast<float4*>(p.dX + off) = o;
     }
 }
 
-// Attention backward, owner = key-like row a (the MFMA column); the query-like rows r are staged:
-//   dK[a] = alpha * sum_r dS X[r];  dV[a] = sum_r P G[r];  dbias[a] = sum_r dS
 template <int D>
-__global__ __launch_bounds__(128, (D <= 32 ? 2 : 1)) void attn_bwd_col_f32m_kernel(
-    const float* __restrict__ X, const float* __restrict__ G, const float* __restrict__ K,
-    const float* __restrict__ V, const float* __restrict__ bias, const float* __restrict__ lse, float lse_to_log2,
-    const float* __restrict__ delta, float* __restrict__ dK, float* __restrict__ dV, float* __restrict__ dbias, int T,
-    float alpha, int causal, int k_diff) {
-    constexpr int DT = D / 32, KS = D / 2, LD = D + 1;
-    __shared__ float sX[32 * LD], sG[32 * LD], sL[32], sD[32];
-    const size_t base = (size_t)blockIdx.y * T * D, vbase = (size_t)blockIdx.y * T;
-    X += base; G += base; K += base; V += base;
-    const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, g = lane >> 5, wave = tid >> 6;
-    // heavy first: under a causal mask the FIRST owner columns see the most rows
-    const int c0 = blockIdx.x * kOwnerRows, a = c0 + wave * 32 + n, ac = min(a, T - 1);
-    const int c_hi = min(T - 1, c0 + kOwnerRows - 1);
-    const int r_lo = causal ? c0 : 0;
-    const int r_hi = causal ? (int)min((long)T - 1, (long)c_hi + k_diff) : T - 1;
-    const int wa_lo = c0 + wave * 32, wa_hi = min(T - 1, wa_lo + 31);
-    const float scale_log2 = alpha * kLog2e;
-
-    float k[KS], v[KS];
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-        k[ks] = K[(size_t)ac * D + g * KS + ks] * scale_log2;
-        v[ks] = V[(size_t)ac * D + g * KS + ks];
-    }
-    const float b = bias ? bias[vbase + ac] : 0.f;
+__device__ __forceinline__ void bwd_cols(const BwdP& p, Shares<D>& sh, int bh, int tile, int tid, int wave, int n, int g) {
+    constexpr int DT = D / 32, KS = D / 2;
+    const int T = p.T;
+    const size_t base = (size_t)bh * T * D, vbase = (size_t)bh * T;
+    const float *X = p.X + base, *G = p.G + base, *K = p.K + base, *V = p.V + base;
+    const int c0 = tile * 32, a = c0 + n;
+    const int r_lo = p.causal ? c0 : 0, r_hi = p.causal ? (int)min((long)T - 1, (long)c0 + 31 + p.k_diff) : T - 1;
+    const float scale_log2 = p.alpha * kLog2e;
     f32x16 accK[DT], accV[DT];
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            accK[dt][i] = 0.f;
-            accV[dt][i] = 0.f;
-        }
+    clear<D>(accK);
+    clear<D>(accV);
     float db = 0.f;
-
-    Stage2<D> st;
-    const int r_first = r_lo & ~31;
-    stage_fetch2<D>(st, X, G, r_first, T);
-    for (int rr0 = r_first; rr0 <= r_hi; rr0 += 32) {
-        __syncthreads();
-        stage_store2<D>(st, sX, sG);
-        if (tid < 32) {
-            const int rr = min(rr0 + tid, T - 1);
-            sL[tid] = lse[vbase + rr] * lse_to_log2;
-            sD[tid] = delta[vbase + rr];
-        }
-        __syncthreads();
-        if (rr0 + 32 <= r_hi) stage_fetch2<D>(st, X, G, rr0 + 32, T);
-        if (wa_lo >= T) continue;
-        if (causal && (rr0 + 31 < wa_lo || (long)rr0 > (long)wa_hi + k_diff)) continue;  // nothing in reach
-        f32x16 s, dp;  // rows = staged r, columns = owner a
-        score_tiles<D>(sX, k, sG, v, s, dp, n, g);
+    int rr0 = r_lo + 32 * wave;
+    own_put<D>(sh, K, c0, T, scale_log2, tid);
+    __syncthreads();
+    if (rr0 <= r_hi) {
+        float lse = load_vec(p.lse + vbase, rr0, T, n), delta = load_vec(p.delta + vbase, rr0, T, n);
+        float v[KS], ra[KS], rb[KS];
+        load_rows<D>(ra, X, rr0, T, n, g);
+        load_rows<D>(v, V, c0, T, n, g);
+        load_rows<D>(rb, G, rr0, T, n, g);
+        const float b = p.bias ? p.bias[vbase + min(a, T - 1)] : 0.f;
+        for (; rr0 <= r_hi; rr0 += 32 * kWaves) {
+            const int next = min(rr0 + 32 * kWaves, r_hi & ~31);
+            sh.vec_put(0, lse * p.lse_to_log2, wave, n);
+            sh.vec_put(1, delta, wave, n);
+            f32x16 s = score_tile<D>(ra, sh, n, g);  // rows = streamed r, columns = owner a
+            pin_order();
+            load_cols<D>(ra, X, rr0, T, n, g);
+            lse = load_vec(p.lse + vbase, next, T, n);
+            delta = load_vec(p.delta + vbase, next, T, n);
+            pin_order();
+            f32x16 dp = score_tile<D>(rb, v);
+            pin_order();
+            load_cols<D>(rb, G, rr0, T, n, g);
+            pin_order();
+            const bool edge = rr0 + 32 > T || (p.causal && (rr0 < c0 + 31 || rr0 + 31 - c0 > p.k_diff));
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int rr = rr0 + c_row(g, i);
-            const bool ok = (rr < T) & (a < T) & pair_valid(causal, k_diff, rr, a);
-            const float p = ok ? fast_exp2(s[i] + b - sL[c_row(g, i)]) : 0.f;
-            const float ds = p * (dp[i] - sD[c_row(g, i)]);
-            s[i] = ds;
-            dp[i] = p;
-            db += ds;
+            for (int i4 = 0; i4 < 4; ++i4) {
+                const float4 l2 = sh.vec_get(0, wave, g, i4), dl = sh.vec_get(1, wave, g, i4);
+                const float l2s[4] = {l2.x, l2.y, l2.z, l2.w}, dls[4] = {dl.x, dl.y, dl.z, dl.w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int i = 4 * i4 + e;
+                    const float pr = fast_exp2(s[i] + b - l2s[e]);
+                    s[i] = pr * (dp[i] - dls[e]);
+                    dp[i] = pr;
+                }
+            }
+            if (edge) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    const int rr = rr0 + c_row(g, i);
+                    const bool ok = (rr < T) & pair_valid(p.causal, p.k_diff, rr, a);
+                    s[i] = ok ? s[i] : 0.f;
+                    dp[i] = ok ? dp[i] : 0.f;
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 16; ++i) db += s[i];
+            output_tile<D>(accK, ra, s);
+            pin_order();
+            load_rows<D>(ra, X, next, T, n, g);
+            pin_order();
+            output_tile<D>(accV, rb, dp);
+            pin_order();
+            load_rows<D>(rb, G, next, T, n, g);
+            pin_order();
         }
-        output_tiles<D>(accK, sX, s, accV, sG, dp, n, g);
     }
     db += __shfl_xor(db, 32, 64);
-    if (a < T) {
+    if (g == 0) sh.row[wave][n] = db;
+    sh.put(accK, p.alpha, wave, n, g);
+    __syncthreads();
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
+    for (int piece = tid; piece < Shares<D>::kPieces; piece += 64 * kWaves) {
+        const int row = piece / (D / 4), c = piece % (D / 4) * 4;
+        if (c0 + row < T) *reinterpret_cast<float4*>(p.dK + base + (size_t)(c0 + row) * D + c) = sh.sum(piece);
+    }
+    __syncthreads();
+    sh.put(accV, 1.f, wave, n, g);
+    __syncthreads();
 #pragma unroll
-            for (int i4 = 0; i4 < 4; ++i4) {
-                const size_t off = base + (size_t)a * D + dt * 32 + c_row(g, i4 * 4);
-                *reinterpret_cast<float4*>(dK + off) = make_float4(accK[dt][i4 * 4] * alpha, accK[dt][i4 * 4 + 1] * alpha,
-                                                                   accK[dt][i4 * 4 + 2] * alpha, accK[dt][i4 * 4 + 3] * alpha);
-                *reinterpret_cast<float4*>(dV + off) = make_float4(accV[dt][i4 * 4], accV[dt][i4 * 4 + 1], accV[dt][i4 * 4 + 2],
-                                                                   accV[dt][i4 * 4 + 3]);
+    for (int piece = tid; piece < Shares<D>::kPieces; piece += 64 * kWaves) {
+        const int row = piece / (D / 4), c = piece % (D / 4) * 4;
+        const bool in = c0 + row < T;
+        const size_t off = base + (size_t)(in ? c0 + row : 0) * D + c;
+        float4 o = sh.sum(piece);
+        if (p.mid_r) {
+            const float4 R = *reinterpret_cast<const float4*>(p.mid_r + off), v2 = *reinterpret_cast<const float4*>(p.mid_v2 + off);
+            const float4 dr = make_float4(o.x * v2.x, o.y * v2.y, o.z * v2.z, o.w * v2.w);
+            float dot = dr.x * R.x + dr.y * R.y + dr.z * R.z + dr.w * R.w;  // over the D / 4 lanes of the row
+#pragma unroll
+            for (int d = D / 8; d > 0; d >>= 1) dot += __shfl_xor(dot, d, 64);
+            if (in) {
+                *reinterpret_cast<float4*>(p.dR + off) = dr;
+                if (c == 0) {
+                    float dbias = sh.row[0][row];
+#pragma unroll
+                    for (int w = 1; w < kWaves; ++w) dbias += sh.row[w][row];
+                    p.delta1[vbase + c0 + row] = dot - dbias;
+                }
             }
-        if (dbias && g == 0) dbias[vbase + a] = db;
+            o = make_float4(o.x * R.x, o.y * R.y, o.z * R.z, o.w * R.w);
+        } else if (p.v1) {
+            const float4 v1 = *reinterpret_cast<const float4*>(p.v1 + off);
+            o.x *= silu_grad_f(v1.x); o.y *= silu_grad_f(v1.y); o.z *= silu_grad_f(v1.z); o.w *= silu_grad_f(v1.w);
+        }
+        if (in) *reinterpret_cast<float4*>(p.dV + off) = o;
     }
 }
 
-// dV2 = dW * R;  dR = dW * V2;  delta1 = rowsum(dR * R) - dlse1   (one wave per row)
-__global__ __launch_bounds__(256) void dps_mid_f32m_kernel(const float* __restrict__ dW, const float* __restrict__ R,
-                                                           const float* __restrict__ V2, const float* __restrict__ dlse1,
-                                                           float* __restrict__ dV2, float* __restrict__ dR,
-                                                           float* __restrict__ delta1, int rows, int D) {
-    const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+template <int D>
+__global__ __launch_bounds__(64 * kWaves, 2) void attn_bwd_f32m_kernel(BwdP p) {
+    __shared__ Shares<D> sh;
+    const int ntiles = (p.T + 31) / 32;
+    int bh, order;
+    if (!xcd_tile(p.BH, 2 * ntiles, blockIdx.x >> 3, blockIdx.x & 7, bh, order)) return;
+    const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, g = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // heavy first: under a causal mask the first owner columns see the most rows, the last owner rows the most columns
+    if (order & 1)
+        bwd_rows<D>(p, sh, bh, p.causal ? ntiles - 1 - (order >> 1) : order >> 1, tid, wave, n, g);
+    else
+        bwd_cols<D>(p, sh, bh, order >> 1, tid, wave, n, g);
+}
+
+// what the backward needs ahead of its passes: u = SiLU(v1) (unless the caller has it) and delta = rowsum(dO * O); D / 4 lanes a row
+template <int D>
+__global__ __launch_bounds__(256) void dps_prep_f32m_kernel(const float* __restrict__ v1, float* __restrict__ u,
+                                                            const float* __restrict__ d_o, const float* __restrict__ o,
+                                                            float* __restrict__ delta, size_t rows) {
+    const size_t piece = (size_t)blockIdx.x * 256 + threadIdx.x, row = piece / (D / 4);
     if (row >= rows) return;
-    float part = 0.f;
-    for (int d = lane; d < D; d += 64) {
-        const size_t i = (size_t)row * D + d;
-        const float dw = dW[i], r = R[i];
-        const float dr = dw * V2[i];
-        dV2[i] = dw * r;
-        dR[i] = dr;
-        part += dr * r;
-    }
-    part = wave_sum(part);
-    if (lane == 0) delta1[row] = part - dlse1[row];
+    const float4 x = reinterpret_cast<const float4*>(v1)[piece];
+    reinterpret_cast<float4*>(u)[piece] = make_float4(silu_f(x.x), silu_f(x.y), silu_f(x.z), silu_f(x.w));
+    const float4 a = reinterpret_cast<const float4*>(d_o)[piece], b = reinterpret_cast<const float4*>(o)[piece];
+    float dot = a.x * b.x + a.y * b.y + a.z * b.z + a.w * b.w;
+#pragma unroll
+    for (int d = D / 8; d > 0; d >>= 1) dot += __shfl_xor(dot, d, 64);
+    if (piece % (D / 4) == 0) delta[row] = dot;
+}
+
+template <int D>
+void launch_fwd(const FwdP& p, hipStream_t st) {
+    hipLaunchKernelGGL(attn_fwd_f32m_kernel<D>, dim3(xcd_slots(p.BH, (p.T + 31) / 32) * 8), dim3(64 * kWaves), 0, st, p);
+}
+template <int D>
+void launch_bwd(const BwdP& p, hipStream_t st) {
+    hipLaunchKernelGGL(attn_bwd_f32m_kernel<D>, dim3(xcd_slots(p.BH, 2 * ((p.T + 31) / 32)) * 8), dim3(64 * kWaves), 0, st, p);
+}
+
+// rows = K2[t], keys K1, values U; outputs R (the backward reads it), W = R * V2, lse1 (log2 units)
+FwdP inner_fwd(const DpsArgs& a, float* r) {
+    return {a.k2, a.k1, a.u, nullptr, a.v2, r, a.w, a.lse1, 1.0f, a.alpha * kLog2e, a.BH, a.T, a.causal, a.k_diff};
 }
 
 template <int D>
 hipError_t fwd_impl(const DpsArgs& a, hipStream_t st) {
-    const dim3 grid((a.T + kOwnerRows - 1) / kOwnerRows, a.BH);
-    const float sl2 = a.alpha * kLog2e;
-    // inner: rows = K2[t], keys K1, values U; outputs R, W = R * V2, lse1 (log2 units)
-    hipLaunchKernelGGL(attn_fwd_f32m_kernel<D>, grid, dim3(128), 0, st, a.k2, a.k1, a.u, (const float*)nullptr, a.v2,
-                       a.r, a.w, a.lse1, 1.0f, a.T, sl2, a.causal, a.k_diff);
+    launch_fwd<D>(inner_fwd(a, nullptr), st);
     // outer: rows = Q[q], keys K2 with bias lse1, values W; outputs O, LSE (natural log)
-    hipLaunchKernelGGL(attn_fwd_f32m_kernel<D>, grid, dim3(128), 0, st, a.q, a.k2, (const float*)a.w,
-                       (const float*)a.lse1, (const float*)nullptr, a.o, (float*)nullptr, a.lse, kLn2, a.T, sl2,
-                       a.causal, a.T);
+    launch_fwd<D>({a.q, a.k2, a.w, a.lse1, nullptr, a.o, nullptr, a.lse, kLn2, a.alpha * kLog2e, a.BH, a.T, a.causal, a.T}, st);
     return hipGetLastError();
 }
 
 template <int D>
 hipError_t bwd_impl(const DpsArgs& a, hipStream_t st) {
-    const dim3 grid((a.T + kOwnerRows - 1) / kOwnerRows, a.BH);
-    const float sl2 = a.alpha * kLog2e;
-    const float* nobias = nullptr;
-    // recompute the inner pass: R, W, lse1
-    hipLaunchKernelGGL(attn_fwd_f32m_kernel<D>, grid, dim3(128), 0, st, a.k2, a.k1, a.u, nobias, a.v2, a.r, a.w, a.lse1,
-                       1.0f, a.T, sl2, a.causal, a.k_diff);
-    // outer pass: dQ ; (dK2 part, dW, dlse1)
-    hipLaunchKernelGGL(attn_bwd_row_f32m_kernel<D>, grid, dim3(128), 0, st, a.q, a.d_o, a.k2, (const float*)a.w,
-                       (const float*)a.lse1, (const float*)a.lse, kLog2e, a.delta, nobias, a.dq, a.T, a.alpha, a.causal,
-                       a.T);
-    hipLaunchKernelGGL(attn_bwd_col_f32m_kernel<D>, grid, dim3(128), 0, st, a.q, a.d_o, a.k2, (const float*)a.w,
-                       (const float*)a.lse1, (const float*)a.lse, kLog2e, a.delta, a.dk2_part, a.dw, a.dlse1, a.T,
-                       a.alpha, a.causal, a.T);
-    const int rows = a.BH * a.T;
-    hipLaunchKernelGGL(dps_mid_f32m_kernel, dim3((rows + 3) / 4), dim3(256), 0, st, (const float*)a.dw,
-                       (const float*)a.r, a.v2, (const float*)a.dlse1, a.dv2, a.dr, a.delta1, rows, a.D);
-    // inner pass: dK2 (total) ; (dK1, dU)
-    hipLaunchKernelGGL(attn_bwd_row_f32m_kernel<D>, grid, dim3(128), 0, st, a.k2, (const float*)a.dr, a.k1, a.u, nobias,
-                       (const float*)a.lse1, 1.0f, (const float*)a.delta1, (const float*)a.dk2_part, a.dk2, a.T, a.alpha,
-                       a.causal, a.k_diff);
-    hipLaunchKernelGGL(attn_bwd_col_f32m_kernel<D>, grid, dim3(128), 0, st, a.k2, (const float*)a.dr, a.k1, a.u, nobias,
-                       (const float*)a.lse1, 1.0f, (const float*)a.delta1, a.dk1, a.du, (float*)nullptr, a.T, a.alpha,
-                       a.causal, a.k_diff);
+    if (a.v1) {
+        const size_t rows = (size_t)a.BH * a.T;
+        hipLaunchKernelGGL(dps_prep_f32m_kernel<D>, dim3((unsigned)((rows * (D / 4) + 255) / 256)), dim3(256), 0, st, a.v1,
+                           const_cast<float*>(a.u), a.d_o, a.o_in, a.delta, rows);
+    }
+    launch_fwd<D>(inner_fwd(a, a.r), st);
+    // outer pass: dQ; dK2 part, dV2, dR, delta1
+    BwdP o{};
+    o.X = a.q; o.G = a.d_o; o.K = a.k2; o.V = a.w; o.bias = a.lse1; o.lse = a.lse; o.lse_to_log2 = kLog2e;
+    o.delta = a.delta; o.dX = a.dq; o.dK = a.dk2_part; o.dV = a.dv2;
+    o.mid_r = a.r; o.mid_v2 = a.v2; o.dR = a.dr; o.delta1 = a.delta1;
+    o.alpha = a.alpha; o.BH = a.BH; o.T = a.T; o.causal = a.causal; o.k_diff = a.T;
+    launch_bwd<D>(o, st);
+    // inner pass: dK2 (total); dK1, dU (dV1 for fp32 tensors)
+    BwdP i{};
+    i.X = a.k2; i.G = a.dr; i.K = a.k1; i.V = a.u; i.lse = a.lse1; i.lse_to_log2 = 1.0f;
+    i.delta = a.delta1; i.addend = a.dk2_part; i.dX = a.dk2; i.dK = a.dk1; i.dV = a.du; i.v1 = a.v1;
+    i.alpha = a.alpha; i.BH = a.BH; i.T = a.T; i.causal = a.causal; i.k_diff = a.k_diff;
+    launch_bwd<D>(i, st);
     return hipGetLastError();
 }
 

@@ -108,9 +108,11 @@ struct DpsArgs {
     float* o;
     float* lse;          // forward output / backward input (natural log) [BH, T]
     const float* d_o;
-    const float* o_in;
+    // fp32 tensors on the matrix cores: the backward forms u and delta from v1 and o_in itself and leaves dV1 in du
+    const float *v1, *o_in;
     float *dq, *dk1, *dk2, *du, *dv2;
-    // scratch, all fp32: r, w, dw, dr, dk2_part [BH,T,D]; lse1, delta, dlse1, delta1 [BH,T]
+    // scratch, all fp32: r, w, dw, dr, dk2_part [BH,T,D]; lse1, delta, dlse1, delta1 [BH,T] (dw, dlse1 and, in the forward,
+    // r: the VALU kernels only)
     float *r, *w, *dw, *dr, *dk2_part, *lse1, *delta, *dlse1, *delta1;
     int BH, T, D;
     float alpha;

@@ -398,6 +398,19 @@ def test_fp32_tensors_on_the_matrix_cores(D, causal, k_diff, tune):
         util.assert_close(f"{name} vs VALU kernels", a, b, **FP32)
 
 
+@pytest.mark.parametrize("D", [32, 64])
+@pytest.mark.parametrize("T,causal,k_diff", [(1, True, 1), (31, False, 31), (32, True, 32), (33, True, 0), (33, False, 33),
+                                             (128, True, 31), (129, True, 32), (161, True, 33), (290, True, 127)])
+def test_fp32_streamed_tiles_dealt_out_to_waves(T, causal, k_diff, D):
+    """32-row owner tiles whose streamed tiles are dealt out to four waves: fewer tiles than waves, exactly as many, one
+    more, one row in the last tile, windows that end on, before and behind a tile's edge; seven (batch, head) slices
+    (padding workgroups in the grid).  The bar of fp32 tensors."""
+    print(f"case dps fp32 waves T={T} causal={causal} k_diff={k_diff} D={D}", flush=True)
+    # (one key: its weight is 1 and dQ, dK1, dK2 are exactly zero, so only the absolute bar means anything)
+    check_all(orc.make_inputs(1, 7, T, D, torch.float32, seed=T + k_diff), 1 / math.sqrt(D), causal, k_diff, factorised=False,
+              rel=math.inf if T == 1 else 1e-4)
+
+
 def test_large_logits_with_convert_to_float32_hold_the_16_bit_bar():
     """convert_to_float32=True on 16-bit tensors: fp32 operands throughout (the fp32 matrix-core kernels), as the
     reference's flag asks of its kernels (dot_product_sum/trittention_triton.py:92-119).  Logits of a few hundred,
