@@ -1,6 +1,6 @@
 // Triple-dot-product trittention backward on MFMA (gfx950), 16-bit tensors.  This file: the kernel
-// for D = 64 with full causal windows or no mask, the scratch producers / consumers and the launcher;
-// tdp_bwd_rows_general.hpp: D = 128 and windowed masks.
+// for D = 64 with full causal windows, windows that no k-k band cuts, or no mask, the scratch producers /
+// consumers and the launcher; tdp_bwd_rows_general.hpp: D = 128 and the other windowed masks.
 //
 // With virtual query rows (q,k):  A = alpha*log2e * Q[q] (.) K2[k],  G = dO[q] (.) V2[k],
 //   S = A K1^T (log2 units),  P = exp2(S - LSE2[q]),  dP = G U^T,  dS = P (dP - Delta[q])
@@ -115,7 +115,8 @@ namespace tritt {
 //  * stages are fetched direct-to-LDS two ahead into three buffers and the workgroup barrier
 //    sits in the middle of a stage: by then the next stage has landed for every wave, so its
 //    first row operands are read during the second half and nothing waits at the stage boundary.
-template <typename E, int D, bool WITH_DQ, bool SV>
+// WIN: a query sees the rows q - wb .. q and the keys q - wa .. q (no k-k band): rounds and stages cover the tile's window.
+template <typename E, int D, bool WITH_DQ, bool SV, bool WIN>
 __device__ __forceinline__ void tdp_bwd_rows_body(const BwdParams<E>& p, const int block) {
     using M = Mma<E>;
     using v8 = typename M::v8;
@@ -170,10 +171,17 @@ __device__ __forceinline__ void tdp_bwd_rows_body(const BwdParams<E>& p, const i
     const int qlast = min(T - 1, q0 + BQ - 1);
     const int jend = p.causal ? qlast : T - 1;  // last j (and last k) any query of the tile needs
     const int jfull = p.causal ? q0 : T - 1;    // keys / rows 0 .. jfull are valid for every column
-    const int nst = jend / 64 + 1, nrounds = jend / 8 + 1;
-    const bool dead_tail = (jend & 63) < 32;  // the last stage's second step lies past every query's last key
-    const int per_split = (nrounds + p.splits - 1) / p.splits;
-    const int m_lo = split * per_split, m_hi = min(nrounds, m_lo + per_split);
+    const int nrounds = jend / 8 + 1;
+    // WIN: rows q - wb .. q and keys q - wa .. q belong to query q; the rounds and stages that hold none are left out
+    const int m_first = WIN ? max(0, q0 - p.wb) / 8 : 0;
+    // The stages start at the 32-key step of the first key any query sees, so that only the last one can hold a step
+    // without any (a second place where a step is left out costs 20 spilled registers).  Such a stage may reach 32 keys
+    // past Tp; what it fetches there (from inside the workspace) is only read by the step that is left out.
+    const int j0 = WIN ? max(0, q0 - p.wa) & ~31 : 0;
+    const int nst = (jend - j0) / 64 + 1;
+    const bool dead_tail = ((jend - j0) & 63) < 32;  // the last stage's second step lies past every query's last key
+    const int per_split = (nrounds - m_first + p.splits - 1) / p.splits;
+    const int m_lo = m_first + split * per_split, m_hi = min(nrounds, m_lo + per_split);
     if (m_lo >= m_hi) return;  // fewer rounds than shares (uniform over the workgroup, before any barrier)
     const int q = q0 + n;                        // this lane's column
     const bool q_ok = q < T;
@@ -200,7 +208,7 @@ __device__ __forceinline__ void tdp_bwd_rows_body(const BwdParams<E>& p, const i
         }
     }
     auto issue_stage = [&](int st, int buf) {
-        const int jb = st * 64;
+        const int jb = j0 + st * 64;
         E* dst = sStage + (buf * 4 + tensor) * TILE + (wave & 1) * 4 * 512;
         if (rowmajor && jb + 63 > T - 1) {
             const int pos = lane & 7, rr = lane >> 3;
@@ -224,8 +232,7 @@ __device__ __forceinline__ void tdp_bwd_rows_body(const BwdParams<E>& p, const i
         }
     };
 
-    // prologue: Q / dO tiles in both forms, first round, first three stages (the j sweep repeats
-    // every round, so stage numbers simply cycle: stage of running index x is x mod nst)
+    // prologue: Q / dO tiles in both forms, first round, first two stages
     for (int idx = tid; idx < BQ * D; idx += NTH) {
         const int r = idx / D, d = idx % D;
         const unsigned row = (unsigned)min(q0 + r, T - 1);
@@ -243,9 +250,14 @@ __device__ __forceinline__ void tdp_bwd_rows_body(const BwdParams<E>& p, const i
         float* all = sOb + BQ * LDQ;
         for (int idx = tid; idx < (NW / 2) * BQ * D; idx += NTH) all[idx] = 0.f;
     }
+    // the stage fetched next (the sweep repeats every round, so the stage numbers cycle)
+    int st_ahead = 0;
+    auto advance = [&]() { st_ahead = st_ahead + 1 < nst ? st_ahead + 1 : 0; };
     issue_round(m_lo, m_lo & 1);
-    issue_stage(0, 0);
-    issue_stage(1 % nst, 1);
+    issue_stage(st_ahead, 0);
+    advance();
+    issue_stage(st_ahead, 1);
+    advance();
     barrier_keep_loads<0>();  // stages 0 and 1 and the first round have landed for every wave
 
     // per-column constants that enter the score products as C operands; a column past the end of
@@ -283,8 +295,7 @@ __device__ __forceinline__ void tdp_bwd_rows_body(const BwdParams<E>& p, const i
     load_rows(0, 0);
 
     const bool late = (wave >> 2) & 1;  // second wave of its SIMD (waves w and w + 4 share one)
-    int gstage = 0;          // running stage index; buffer = gstage % NBUF
-    int st_ahead = 2 % nst;  // stage number of running index gstage + 2
+    int gstage = 0;  // running stage index; buffer = gstage % NBUF
     for (int m = m_lo; m < m_hi; ++m) {
         const int mb = m & 1;
         const int k = m * 8 + wave;  // this wave's K2/V2 row
@@ -328,9 +339,10 @@ __device__ __forceinline__ void tdp_bwd_rows_body(const BwdParams<E>& p, const i
             const E* sUT = sStage + (sb * 4 + 3) * TILE;
 #pragma unroll
             for (int half = 0; half < 2; ++half) {
-                const int jb = st * 64 + half * 32;
+                const int jb = j0 + st * 64 + half * 32;
                 // wave-uniform: some (q, j, k) of this step is invalid
-                const bool need_mask = (k > jfull) || (jb + 31 > jfull);
+                bool need_mask = (k > jfull) || (jb + 31 > jfull);
+                if constexpr (WIN) need_mask = need_mask || k < q0 + 31 - p.wb || jb < q0 + 31 - p.wa;
                 f32x16 s, dp;
                 __builtin_amdgcn_sched_barrier(0);
                 // Wave priority: low while this wave issues the score products (eight MFMAs and nothing else), high for
@@ -342,10 +354,18 @@ __device__ __forceinline__ void tdp_bwd_rows_body(const BwdParams<E>& p, const i
                 // (q, j, k) is invalid S starts from -3e4 instead.  Element i of a lane is key
                 // jb + key_of(0, i) + 8 g.
                 if (need_mask) {
-                    const int lim = (k <= jq) ? jq - jb - 8 * g : -1;
                     f32x16 c;
+                    if constexpr (WIN) {
+                        // keys lim - wa .. lim; a lane whose query does not see row k has lim = -1: lim - key is below
+                        // zero then, so past every window as an unsigned number
+                        const int lim = (unsigned)(jq - k) <= (unsigned)p.wb ? jq - jb - 8 * g : -1;
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) c[i] = key_of(0, i) <= lim ? -lse2 : -3.0e4f;
+                        for (int i = 0; i < 16; ++i) c[i] = (unsigned)(lim - key_of(0, i)) <= (unsigned)p.wa ? -lse2 : -3.0e4f;
+                    } else {
+                        const int lim = (k <= jq) ? jq - jb - 8 * g : -1;
+#pragma unroll
+                        for (int i = 0; i < 16; ++i) c[i] = key_of(0, i) <= lim ? -lse2 : -3.0e4f;
+                    }
                     s = M::mma(ak[0], bq[0], c);
                 } else {
                     s = M::mma(ak[0], bq[0], init_s);
@@ -357,7 +377,7 @@ __device__ __forceinline__ void tdp_bwd_rows_body(const BwdParams<E>& p, const i
                     // past that (this stage's barrier was crossed in the first half): fetch it now
                     if (st == 0 && m + 1 < m_hi) issue_round(m + 1, mb ^ 1);  // older than the stage loads
                     issue_stage(st_ahead, (gstage + 2) % NBUF);
-                    st_ahead = st_ahead + 1 < nst ? st_ahead + 1 : 0;
+                    advance();
                 }
                 __builtin_amdgcn_sched_barrier(0);
                 // a step past every query's last key (the second half of the last stage, for every other tile) has
@@ -520,9 +540,9 @@ __device__ __forceinline__ void tdp_bwd_rows_body(const BwdParams<E>& p, const i
     }
 }
 
-template <typename E, int D, bool WITH_DQ, bool SV = false>
+template <typename E, int D, bool WITH_DQ, bool SV, bool WIN>
 __global__ __launch_bounds__(512) void tdp_bwd_rows_kernel(BwdParams<E> p) {
-    tdp_bwd_rows_body<E, D, WITH_DQ, SV>(p, blockIdx.x);
+    tdp_bwd_rows_body<E, D, WITH_DQ, SV, WIN>(p, blockIdx.x);
 }
 
 // The same grid together with the fp32 workgroups of query tile 0 (tdp_f32_tiles.hpp: both roles, one workgroup per
@@ -532,13 +552,13 @@ __global__ __launch_bounds__(512) void tdp_bwd_rows_kernel(BwdParams<E> p) {
 // before them (small grids: the main blocks are as short as these, and a latency-bound workgroup that starts last
 // is the launch's tail).  They add to the same accumulators as every other workgroup, in fixed point, so the order
 // changes nothing.
-template <typename E, int D, bool WITH_DQ, bool SV>
+template <typename E, int D, bool WITH_DQ, bool SV, bool WIN>
 __global__ __launch_bounds__(512) void tdp_bwd_rows_tile0_kernel(BwdParams<E> p, F32BwdParams<E> r0, F32BwdParams<E> r1,
                                                                  int roles_mask, int main_blocks, int t0_x, int t0_first) {
     const int t0_blocks = t0_x * 2 * r0.split_rounds;
     const int block = (int)blockIdx.x - (t0_first ? t0_blocks : 0);  // main blocks: 0 .. main_blocks - 1
     if (block >= 0 && block < main_blocks) {
-        tdp_bwd_rows_body<E, D, WITH_DQ, SV>(p, block);
+        tdp_bwd_rows_body<E, D, WITH_DQ, SV, WIN>(p, block);
     } else {
         const int extra = t0_first ? (int)blockIdx.x : block - main_blocks;
         f32_tile0_block<E, D, D>(r0, r1, roles_mask, extra / t0_x, extra % t0_x);
@@ -709,6 +729,31 @@ static BwdLayout bwd_layout(int BH, int T, int D, bool fixed_point) {
     return l;
 }
 
+// Workgroups per query tile under a window at D = 64, by the time that the launch takes with s of them: one workgroup
+// fills a CU, and all tiles but those at the start of the sequence cost the same, so the launch takes the larger of
+// whole rounds of the full tiles' parts over the CUs and of the even share plus half a part of tail.  Work in 32-key steps
+// of eight rows; a part's own prologue, dQ's shares and tail are worth about nine of them.  Against one part per tile below
+// 1024 tiles and two from there on, training steps: B=2 H=4 T=2048 window 512 5.67 -> 5.3 ms (3 parts), B=2 H=8 T=2048
+// window 100 1.41 -> 1.31 ms (1), B=1 H=2 T=1999 window 77 232 -> 212 us (2); the rest of a dozen shapes within 1 %.
+static int windowed_splits(const MfmaBwdArgs& a) {
+    constexpr float kPart = 9.f;
+    constexpr int kCus = 256;
+    const int nqt = (a.T + 31) / 32, rows = std::min(a.k2_window, a.T - 1) + 32;
+    const int keys = std::min(std::min(a.k1_window, a.T - 1) + 32, a.kk_left + a.kk_right + 8);
+    const float w = (float)((rows + 7) / 8) * (float)((keys + 31) / 32);  // of a tile past the start of the sequence
+    const int full = a.BH * std::max(nqt - rows / 32, 0), light = a.BH * std::min(nqt, rows / 32);
+    const float total = ((float)full + 0.36f * (float)light) * w;
+    int best = 1;
+    float least = 3.0e38f;
+    for (int s : {1, 2, 3, 4, 6, 8, 12, 16}) {
+        const float part = kPart + w / (float)s;
+        const float t = std::max((float)((full * s + kCus - 1) / kCus) * part,
+                                 ((float)(full + light) * (float)s * kPart + total) / kCus + 0.5f * part);
+        if (t < least) least = t, best = s;
+    }
+    return best;
+}
+
 // SV: the caller's tensors are strided views, read where they lie (the kernels' SV instantiations)
 template <typename E, int D, bool SV>
 static hipError_t launch_bwd(const MfmaBwdArgs& a, hipStream_t st) {
@@ -725,7 +770,8 @@ static hipError_t launch_bwd(const MfmaBwdArgs& a, hipStream_t st) {
     // workgroups, and dQ is accumulated in fp32 like the row gradients.
     const int tiles = 8 * ((a.BH + 7) / 8) * ((a.T + 31) / 32);
     int splits = 1;
-    if (tiles < 1024) splits = std::min(16, (1024 + tiles - 1) / tiles);
+    if (D == 64 && a.windowed && !a.split) splits = windowed_splits(a);
+    else if (tiles < 1024) splits = std::min(16, (1024 + tiles - 1) / tiles);
     // a few waves of long tiles: the last tiles of each head are the costliest (the work of a tile grows with the
     // square of its position), and halving them shortens the tail by about 1 % (measured: B=4 H=8 T=1024, 2048)
     else if (tiles < 4096 && a.T >= 1024) splits = 2;
@@ -755,13 +801,21 @@ static hipError_t launch_bwd(const MfmaBwdArgs& a, hipStream_t st) {
     p.acc_q = dqacc; p.splits = splits; p.fixed_point = a.deterministic ? 1 : 0;
     p.scale_parts = (const unsigned*)(ws + l.scale_parts); p.poison = (unsigned*)(ws + l.poison);
 
-    // D = 64, full windows: three stage buffers of four 64x64 tiles, two rounds of 8 K2 / V2 rows, the Q and dO
+    // D = 64, full windows and windows that no k-k band cuts: three stage buffers of four 64x64 tiles, two rounds of 8 K2 / V2 rows, the Q and dO
     // tiles (twice: operand and epilogue layout), four dQ slices.  Otherwise: tdp_bwd_rows_general.hpp
     size_t smem;
     void (*kern_dq)(BwdParams<E>);
     void (*kern_nodq)(BwdParams<E>);
     int nthreads = 512, col_parts = 1;
     bool plain64 = false;  // the D = 64 kernel of this file
+    // The D = 64 kernel of this file takes windows that kk_left / kk_right do not cut (no pair inside the k1 and k2 windows
+    // of a query is further apart): its stages are the same for every round.  Training steps against the general kernel at
+    // equal splits: window 512 (B=2 H=4 T=2048) 6.4 -> 5.67 ms, 200 (B=1 H=4 T=1000) 520 -> 460 us, 128 (B=4 H=8 T=1024)
+    // 1.60 -> 1.55 ms.  A window of 64 is three steps, i.e. two stages of which one is half empty: 835 -> 868 us, so up to
+    // there the general kernel's 32-key stages stay.  With a k-k band of its own range of stages per round this kernel
+    // spills 100 bytes a lane and loses 10 to 40 %.
+    const bool kk_cuts = std::min(a.k2_window, a.T - 1) > a.kk_right || std::min(a.k1_window, a.T - 1) > a.kk_left;
+    const bool general_window = a.windowed && (D == 128 || kk_cuts || std::min(a.k1_window, a.k2_window) <= 64);
     if constexpr (D == 32) {
         // one shape, the banded instantiation for every mask (full windows are windows of T)
         smem = bwdg_smem(32, 8, 32, true);
@@ -791,7 +845,7 @@ static hipError_t launch_bwd(const MfmaBwdArgs& a, hipStream_t st) {
             kern_dq = tdp_bwd_rows_q16_kernel<E, true, true, SV>;
             kern_nodq = tdp_bwd_rows_q16_kernel<E, false, true, SV>;
         }
-    } else if (a.windowed) {
+    } else if (general_window) {
         smem = bwdg_smem(D, 8, 64, true);
         kern_dq = tdp_bwd_rows_general_kernel<E, (D < 64 ? 64 : D), true, 8, 64, true, false, SV>;
         kern_nodq = tdp_bwd_rows_general_kernel<E, (D < 64 ? 64 : D), false, 8, 64, true, false, SV>;
@@ -820,8 +874,8 @@ static hipError_t launch_bwd(const MfmaBwdArgs& a, hipStream_t st) {
     } else {
         smem = 2 * (size_t)(3 * 4 * 64 * 64 + 2 * 2 * 8 * 64 + 2 * (64 / 32) * 64 * 16) +
                4 * (size_t)(2 * 32 * (64 + 4) + 4 * 32 * 64);
-        kern_dq = tdp_bwd_rows_kernel<E, 64, true, SV>;
-        kern_nodq = tdp_bwd_rows_kernel<E, 64, false, SV>;
+        kern_dq = a.windowed ? tdp_bwd_rows_kernel<E, 64, true, SV, true> : tdp_bwd_rows_kernel<E, 64, true, SV, false>;
+        kern_nodq = a.windowed ? tdp_bwd_rows_kernel<E, 64, false, SV, true> : tdp_bwd_rows_kernel<E, 64, false, SV, false>;
         plain64 = true;
     }
     if (hipError_t e = ensure_dynamic_smem(reinterpret_cast<const void*>(kern_dq), smem); e != hipSuccess) return e;
@@ -877,7 +931,10 @@ static hipError_t launch_bwd(const MfmaBwdArgs& a, hipStream_t st) {
     auto launch_rows = [&](bool with_dq) {
         if constexpr (D == 64) {
             if (fuse_tile0) {  // the first launch takes tile 0 along
-                auto fused = with_dq ? tdp_bwd_rows_tile0_kernel<E, 64, true, SV> : tdp_bwd_rows_tile0_kernel<E, 64, false, SV>;
+                auto fused = a.windowed ? (with_dq ? tdp_bwd_rows_tile0_kernel<E, 64, true, SV, true>
+                                                   : tdp_bwd_rows_tile0_kernel<E, 64, false, SV, true>)
+                                        : (with_dq ? tdp_bwd_rows_tile0_kernel<E, 64, true, SV, false>
+                                                   : tdp_bwd_rows_tile0_kernel<E, 64, false, SV, false>);
                 launch_error = ensure_dynamic_smem(reinterpret_cast<const void*>(fused), std::max(smem, f32_bwd_smem<64>()));
                 if (launch_error != hipSuccess) return;
                 const int t0_x = 8 * xcd_slots(a.BH, 1);

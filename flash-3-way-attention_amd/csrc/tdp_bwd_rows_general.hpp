@@ -1,7 +1,7 @@
 // Triple-dot-product trittention backward on MFMA: the general form of the rows kernel (included by
-// tdp_bwd_mfma.hip after BwdParams).  It serves head dimensions 32 and 128 and, for head dimensions
-// 64 and 128, windowed causal masks (WIN): rounds and steps then cover the band only, and a key outside the
-// window of its (q, k) is masked like one past the causal bound.
+// tdp_bwd_mfma.hip after BwdParams).  It serves head dimensions 32 and 128, split operands and, at head
+// dimension 64, the windowed causal masks (WIN) that the kernel there leaves (k-k bands and windows up to 64).  WIN:
+// rounds and steps cover the band only, and a key outside the window of its (q, k) is masked like one past the causal bound.
 //
 // Same decomposition as tdp_bwd_rows_kernel (rows = one K2/V2 row k per wave and round, K1 / U
 // streamed over j, the columns of every tile = 32 queries).  The accumulators Yq / Tv of all 128
@@ -16,8 +16,8 @@
 // offset_operand) instead of two resident 16-register C tiles.  Stages are 32 keys: K1 and U rows
 // as 64 x 64 tiles (tile row = 32 * (d / 64) + key, the swizzle of direct_lds.hpp), K1^T and U^T
 // of the workgroup's columns as compact [NCOL d][32 keys] tiles; three buffers, fetched
-// direct-to-LDS two steps ahead, one workgroup barrier per step.  D = 64 (WIN only; the full-window
-// case has its own kernel): NW = 8, NCOL = 64, the row tiles have 32 rows.  D = 32: NW = 8,
+// direct-to-LDS two steps ahead, one workgroup barrier per step.  D = 64 (WIN and split operands; full
+// windows have their own kernel): NW = 8, NCOL = 64, the row tiles have 32 rows.  D = 32: NW = 8,
 // NCOL = 32, the row tiles have 32 rows of 64 bytes (swizzled like the transposed tiles).
 #pragma once
 

@@ -609,6 +609,27 @@ def test_mfma_backward_windows_bf16(seq_len, windows, D):
             assert util.rel_err(a, b) <= 5e-2, (name, util.rel_err(a, b))
 
 
+@pytest.mark.parametrize("splits", [0, 1, 3])
+@pytest.mark.parametrize("dtype,windows,seq_len", [
+    (torch.bfloat16, (65, 65, 65, 65), 97), (torch.bfloat16, (65, 128, None, None), 161), (torch.bfloat16, (96, 70, 200, 100), 289),
+    (torch.float16, (127, 129, 129, 129), 333), (torch.bfloat16, (200, 66, None, None), 224), (torch.bfloat16, (64, 64, 64, 64), 161),
+    (torch.bfloat16, (128, 128, 128, 127), 256), (torch.float16, (159, 160, None, None), 161)])
+def test_mfma_backward_wide_windows_d64(dtype, windows, seq_len, splits, tune):
+    """Windows that no k-k band cuts, at head dimension 64: lengths that end inside and on a stage, windows whose first key
+    lies in either half of one, unequal windows, and the neighbours that stay with the general kernel (a window of 64, a band
+    one key short).  The oracle's bars are those of the other windowed tests: one key too many or too few in a window of 65
+    is an error above a tenth."""
+    tune(_lib.TUNE_BWD_SPLITS, splits)
+    print(f"case mfma bwd wide windows T={seq_len} {windows} splits={splits}", flush=True)
+    inputs = orc.make_inputs(2, 2, seq_len, 64, dtype, seed=seq_len + splits)
+    z, _, grads = util.oracle_tdp(inputs, 1 / 8, True, windows)
+    out, g = util.run_tdp(inputs, 1 / 8, True, windows, flags=FORCE_MFMA)
+    util.assert_close("out", out, z, **LOWP)
+    for name, a, b in zip(util.NAMES, g, grads):
+        util.assert_mostly_close(name, a, b, **LOWP)
+        assert util.rel_err(a, b) <= 5e-2, (name, util.rel_err(a, b))
+
+
 @pytest.mark.parametrize("D", [64, 128])
 def test_mfma_windows_fp16_batched(D):
     """fp16, several batch entries and heads, odd window sizes: forward and all five gradients."""
