@@ -754,6 +754,28 @@ static int windowed_splits(const MfmaBwdArgs& a) {
     return best;
 }
 
+// Workgroups per query tile under a full causal mask at D = 64, for grids of less than 1024 tiles.  The work of a tile grows
+// with the square of its position and the heaviest parts start first, so a launch takes the longer of the even share of all
+// parts over the CUs and of its longest part (which starts late by what the parts before it differ: 1.15).  Work in 32-key
+// steps of eight rows; a part's own prologue, dQ's shares and tail are worth about seven of them.  Against parts that bring
+// the grid to 1024 workgroups whatever they cost, training steps: B=2 H=4 T=256 172 -> 158 us (16 -> 8 parts), B=4 H=8 T=128
+// 168 -> 154 us (8 -> 4), B=2 H=8 T=300 360 -> 352 us (7 -> 4), B=1 H=4 T=512 348 -> 341 us (8 -> 12); B=1 H=8 T=1000
+// keeps its four.  D = 32 and 128 measure within 1 % of their best at 1024 workgroups.
+static int causal_splits(const MfmaBwdArgs& a) {
+    constexpr float kPart = 7.f;
+    constexpr int kCus = 256;
+    const int nqt = (a.T + 31) / 32;
+    const float w = (float)((a.T + 7) / 8) * (float)nqt;  // the last tile's
+    const float total = (float)a.BH * w * (float)((nqt + 1) * (2 * nqt + 1)) / (float)(6 * nqt);  // a sum of squares
+    int best = 1;
+    float least = 3.0e38f;
+    for (int s : {1, 2, 3, 4, 6, 8, 12, 16}) {
+        const float t = std::max(1.15f * (kPart + w / (float)s), (total + (float)(a.BH * nqt * s) * kPart) / kCus);
+        if (t < least) least = t, best = s;
+    }
+    return best;
+}
+
 // SV: the caller's tensors are strided views, read where they lie (the kernels' SV instantiations)
 template <typename E, int D, bool SV>
 static hipError_t launch_bwd(const MfmaBwdArgs& a, hipStream_t st) {
@@ -771,6 +793,7 @@ static hipError_t launch_bwd(const MfmaBwdArgs& a, hipStream_t st) {
     const int tiles = 8 * ((a.BH + 7) / 8) * ((a.T + 31) / 32);
     int splits = 1;
     if (D == 64 && a.windowed && !a.split) splits = windowed_splits(a);
+    else if (D == 64 && a.causal && !a.split && tiles < 1024) splits = causal_splits(a);
     else if (tiles < 1024) splits = std::min(16, (1024 + tiles - 1) / tiles);
     // a few waves of long tiles: the last tiles of each head are the costliest (the work of a tile grows with the
     // square of its position), and halving them shortens the tail by about 1 % (measured: B=4 H=8 T=1024, 2048)

@@ -630,6 +630,20 @@ def test_mfma_backward_wide_windows_d64(dtype, windows, seq_len, splits, tune):
         assert util.rel_err(a, b) <= 5e-2, (name, util.rel_err(a, b))
 
 
+@pytest.mark.parametrize("B,H,seq_len", [(1, 1, 33), (1, 2, 65), (1, 9, 96), (4, 8, 64), (4, 9, 97), (2, 8, 129)])
+def test_mfma_backward_parts_by_cost_d64(B, H, seq_len):
+    """Full causal masks on grids too small for one part per query tile, where the launcher picks the parts by their cost (1 to
+    16 of them): lengths at a tile's edge, more parts than a tile has rounds, head counts that leave padding workgroups."""
+    print(f"case mfma bwd parts B={B} H={H} T={seq_len}", flush=True)
+    inputs = orc.make_inputs(B, H, seq_len, 64, torch.bfloat16, seed=seq_len + H)
+    z, _, grads = util.oracle_tdp(inputs, 1 / 8, True, (None,) * 4)
+    out, g = util.run_tdp(inputs, 1 / 8, True, (None,) * 4, flags=FORCE_MFMA)
+    util.assert_close("out", out, z, **LOWP)
+    for name, a, b in zip(util.NAMES, g, grads):
+        util.assert_mostly_close(name, a, b, **LOWP)
+        assert util.rel_err(a, b) <= 5e-2, (name, util.rel_err(a, b))
+
+
 @pytest.mark.parametrize("D", [64, 128])
 def test_mfma_windows_fp16_batched(D):
     """fp16, several batch entries and heads, odd window sizes: forward and all five gradients."""
