@@ -322,9 +322,14 @@ int tdp_bwd_generic(Arena& ar, bool run, const void* q, const void* k1, const vo
 // the vector ALUs; TRITT_TUNE_F32_VALU forces the latter
 bool use_f32_mfma_dps(int D) { return !knobs().f32_valu && f32_mfma_dps_supported(D); }
 
+// What a forward leaves for its backward beside o and lse (null pointers: nothing, the backward runs the inner pass again)
+struct DpsKept {
+    float *r, *lse1;
+};
+
 int dps_fwd_impl(Arena& ar, bool run, const void* q, const void* k1, const void* k2, const void* v1, const void* v2,
                  void* o, float* lse, int B, int H, int T, int D, int dtype, float alpha, int causal, int k_diff,
-                 hipStream_t st) {
+                 hipStream_t st, DpsKept kept = {}) {
     const size_t n = (size_t)B * H * T * D, rows = (size_t)B * H * T;
     float *copies[4], *u;
     F32Inputs in = plan_inputs(ar, q, k1, k2, v2, n, dtype, copies, &u);
@@ -333,6 +338,10 @@ int dps_fwd_impl(Arena& ar, bool run, const void* q, const void* k1, const void*
     if (!use_f32_mfma_dps(D)) a.r = ar.take<float>(n);
     a.w = ar.take<float>(n);
     a.lse1 = ar.take<float>(rows);
+    if (kept.r) {
+        a.r = kept.r;
+        a.lse1 = kept.lse1;
+    }
     if (!run) return TRITT_OK;
     if (ar.overflows()) return TRITT_ERR_WORKSPACE;
     fill_inputs(q, k1, k2, v1, v2, n, dtype, copies, u, st);
@@ -348,7 +357,7 @@ int dps_fwd_impl(Arena& ar, bool run, const void* q, const void* k1, const void*
 int dps_bwd_impl(Arena& ar, bool run, const void* q, const void* k1, const void* k2, const void* v1, const void* v2,
                  const void* o, const float* lse, const void* d_o, void* dq, void* dk1, void* dk2, void* dv1,
                  void* dv2, int B, int H, int T, int D, int dtype, float alpha, int causal, int k_diff,
-                 hipStream_t st) {
+                 hipStream_t st, DpsKept kept = {}) {
     const size_t n = (size_t)B * H * T * D, rows = (size_t)B * H * T;
     float *copies[4], *u;
     F32Inputs in = plan_inputs(ar, q, k1, k2, v2, n, dtype, copies, &u);
@@ -386,6 +395,10 @@ int dps_bwd_impl(Arena& ar, bool run, const void* q, const void* k1, const void*
         lse = lse32;
     } else if (in_place) {
         a.v1 = (const float*)v1; a.o_in = (const float*)o;
+        if (kept.r) {
+            a.kept = true;
+            a.r = kept.r; a.lse1 = kept.lse1;
+        }
     } else {
         rowdot(d_o, o, a.delta, (int)rows, D, dtype, st);
     }
@@ -429,6 +442,11 @@ bool use_mfma_bwd(int T, int D, int dtype, int causal, int w1, int w2, int kl, i
 bool use_mfma_dps(int D, int dtype, unsigned flags) {
     if (flags & TRITT_FLAG_FORCE_GENERIC) return false;
     return mfma_dps_supported(D, dtype != TRITT_F32);
+}
+
+// whether the forward can leave what DpsKept names: the matrix-core kernels on the caller's own type
+bool dps_keeps(int D, int dtype, unsigned flags) {
+    return use_mfma_dps(D, dtype, flags) || (dtype == TRITT_F32 && use_f32_mfma_dps(D));
 }
 
 bool any_null(std::initializer_list<const void*> ps) {
@@ -717,9 +735,9 @@ size_t tritt_dps_fwd_workspace_bytes(int B, int H, int T, int D, int dtype, unsi
     return ar.bytes();
 }
 
-int tritt_dps_fwd(const void* q, const void* k1, const void* k2, const void* v1, const void* v2, void* o, float* lse,
+static int dps_fwd_call(const void* q, const void* k1, const void* k2, const void* v1, const void* v2, void* o, float* lse,
                   int B, int H, int T, int D, int dtype, float alpha, int causal, int k_diff, void* workspace,
-                  size_t workspace_bytes, unsigned flags, void* stream) {
+                  size_t workspace_bytes, unsigned flags, void* stream, DpsKept kept) {
     if (empty_problem(B, H, T)) return check_common(1, 1, 1, D, dtype);
     int rc = check_common(B, H, T, D, dtype);
     if (rc != TRITT_OK) return rc;
@@ -733,13 +751,21 @@ int tritt_dps_fwd(const void* q, const void* k1, const void* k2, const void* v1,
     if (mfma) {
         MfmaDpsArgs a{};
         a.q = q; a.k1 = k1; a.k2 = k2; a.v1 = v1; a.v2 = v2; a.o_out = o; a.lse_out = lse; a.workspace = workspace;
+        a.kept_r = kept.r; a.kept_lse1 = kept.lse1;
         a.BH = B * H; a.T = T; a.D = D; a.alpha = alpha; a.causal = causal ? 1 : 0; a.k_diff = clampw(k_diff, T);
         a.is_bf16 = dtype == TRITT_BF16;
         return (int)mfma_dps_fwd(a, (hipStream_t)stream);
     }
     Arena ar(workspace, workspace_bytes);
     return dps_fwd_impl(ar, true, q, k1, k2, v1, v2, o, lse, B, H, T, D, dtype, alpha, causal, clampw(k_diff, T),
-                        (hipStream_t)stream);
+                        (hipStream_t)stream, kept);
+}
+
+int tritt_dps_fwd(const void* q, const void* k1, const void* k2, const void* v1, const void* v2, void* o, float* lse,
+                  int B, int H, int T, int D, int dtype, float alpha, int causal, int k_diff, void* workspace,
+                  size_t workspace_bytes, unsigned flags, void* stream) {
+    return dps_fwd_call(q, k1, k2, v1, v2, o, lse, B, H, T, D, dtype, alpha, causal, k_diff, workspace, workspace_bytes,
+                        flags, stream, DpsKept{});
 }
 
 size_t tritt_dps_bwd_workspace_bytes(int B, int H, int T, int D, int dtype, unsigned flags) {
@@ -752,10 +778,10 @@ size_t tritt_dps_bwd_workspace_bytes(int B, int H, int T, int D, int dtype, unsi
     return ar.bytes();
 }
 
-int tritt_dps_bwd(const void* q, const void* k1, const void* k2, const void* v1, const void* v2, const void* o,
+static int dps_bwd_call(const void* q, const void* k1, const void* k2, const void* v1, const void* v2, const void* o,
                   const float* lse, const void* d_o, void* dq, void* dk1, void* dk2, void* dv1, void* dv2, int B, int H,
                   int T, int D, int dtype, float alpha, int causal, int k_diff, void* workspace, size_t workspace_bytes,
-                  unsigned flags, void* stream) {
+                  unsigned flags, void* stream, DpsKept kept) {
     if (empty_problem(B, H, T)) return check_common(1, 1, 1, D, dtype);
     int rc = check_common(B, H, T, D, dtype);
     if (rc != TRITT_OK) return rc;
@@ -770,13 +796,22 @@ int tritt_dps_bwd(const void* q, const void* k1, const void* k2, const void* v1,
         MfmaDpsArgs a{};
         a.q = q; a.k1 = k1; a.k2 = k2; a.v1 = v1; a.v2 = v2; a.o = o; a.d_o = d_o; a.lse_in = lse;
         a.dq = dq; a.dk1 = dk1; a.dk2 = dk2; a.dv1 = dv1; a.dv2 = dv2; a.workspace = workspace;
+        a.kept_r = kept.r; a.kept_lse1 = kept.lse1;
         a.BH = B * H; a.T = T; a.D = D; a.alpha = alpha; a.causal = causal ? 1 : 0; a.k_diff = clampw(k_diff, T);
         a.is_bf16 = dtype == TRITT_BF16;
         return (int)mfma_dps_bwd(a, (hipStream_t)stream);
     }
     Arena ar(workspace, workspace_bytes);
     return dps_bwd_impl(ar, true, q, k1, k2, v1, v2, o, lse, d_o, dq, dk1, dk2, dv1, dv2, B, H, T, D, dtype, alpha,
-                        causal, clampw(k_diff, T), (hipStream_t)stream);
+                        causal, clampw(k_diff, T), (hipStream_t)stream, kept);
+}
+
+int tritt_dps_bwd(const void* q, const void* k1, const void* k2, const void* v1, const void* v2, const void* o,
+                  const float* lse, const void* d_o, void* dq, void* dk1, void* dk2, void* dv1, void* dv2, int B, int H,
+                  int T, int D, int dtype, float alpha, int causal, int k_diff, void* workspace, size_t workspace_bytes,
+                  unsigned flags, void* stream) {
+    return dps_bwd_call(q, k1, k2, v1, v2, o, lse, d_o, dq, dk1, dk2, dv1, dv2, B, H, T, D, dtype, alpha, causal, k_diff,
+                        workspace, workspace_bytes, flags, stream, DpsKept{});
 }
 
 // ---------------------------------------------------------------- strided entry points
@@ -884,10 +919,10 @@ size_t tritt_dps_fwd_strided_workspace_bytes(int B, int H, int T, int D, int dty
     return round256(tritt_dps_fwd_workspace_bytes(B, H, T, D, dtype, flags)) + v.bytes;
 }
 
-int tritt_dps_fwd_strided(const void* q, const void* k1, const void* k2, const void* v1, const void* v2,
+static int dps_fwd_strided_call(const void* q, const void* k1, const void* k2, const void* v1, const void* v2,
                           const tritt_layout* in_layouts, void* o, float* lse, int B, int H, int T, int D, int dtype,
                           float alpha, int causal, int k_diff, void* workspace, size_t workspace_bytes, unsigned flags,
-                          void* stream) {
+                          void* stream, DpsKept kept) {
     if (empty_problem(B, H, T)) return check_common(1, 1, 1, D, dtype);
     int rc = check_common(B, H, T, D, dtype);
     if (rc != TRITT_OK) return rc;
@@ -901,6 +936,7 @@ int tritt_dps_fwd_strided(const void* q, const void* k1, const void* k2, const v
         if (!workspace || workspace_bytes < plain) return TRITT_ERR_WORKSPACE;
         MfmaDpsArgs a{};
         a.q = q; a.k1 = k1; a.k2 = k2; a.v1 = v1; a.v2 = v2; a.o_out = o; a.lse_out = lse; a.workspace = workspace;
+        a.kept_r = kept.r; a.kept_lse1 = kept.lse1;
         a.BH = B * H; a.T = T; a.D = D; a.alpha = alpha; a.causal = causal ? 1 : 0; a.k_diff = clampw(k_diff, T);
         a.is_bf16 = dtype == TRITT_BF16;
         dps_views(a, in_layouts, nullptr, H, T, D);
@@ -912,8 +948,16 @@ int tritt_dps_fwd_strided(const void* q, const void* k1, const void* k2, const v
     if (rc != TRITT_OK) return rc;
     if (!workspace || workspace_bytes < plain + v.bytes) return TRITT_ERR_WORKSPACE;
     run_pack(v, B, H, T, D, dtype, (hipStream_t)stream);
-    return tritt_dps_fwd(v.ptr[0], v.ptr[1], v.ptr[2], v.ptr[3], v.ptr[4], o, lse, B, H, T, D, dtype, alpha, causal, k_diff,
-                         workspace, plain, flags, stream);
+    return dps_fwd_call(v.ptr[0], v.ptr[1], v.ptr[2], v.ptr[3], v.ptr[4], o, lse, B, H, T, D, dtype, alpha, causal, k_diff,
+                         workspace, plain, flags, stream, kept);
+}
+
+int tritt_dps_fwd_strided(const void* q, const void* k1, const void* k2, const void* v1, const void* v2,
+                          const tritt_layout* in_layouts, void* o, float* lse, int B, int H, int T, int D, int dtype,
+                          float alpha, int causal, int k_diff, void* workspace, size_t workspace_bytes, unsigned flags,
+                          void* stream) {
+    return dps_fwd_strided_call(q, k1, k2, v1, v2, in_layouts, o, lse, B, H, T, D, dtype, alpha, causal, k_diff, workspace,
+                                workspace_bytes, flags, stream, DpsKept{});
 }
 
 size_t tritt_dps_bwd_strided_workspace_bytes(int B, int H, int T, int D, int dtype, unsigned flags,
@@ -927,11 +971,11 @@ size_t tritt_dps_bwd_strided_workspace_bytes(int B, int H, int T, int D, int dty
     return round256(tritt_dps_bwd_workspace_bytes(B, H, T, D, dtype, flags)) + v.bytes;
 }
 
-int tritt_dps_bwd_strided(const void* q, const void* k1, const void* k2, const void* v1, const void* v2,
+static int dps_bwd_strided_call(const void* q, const void* k1, const void* k2, const void* v1, const void* v2,
                           const tritt_layout* in_layouts, const void* o, const float* lse, const void* d_o,
                           const tritt_layout* d_o_layout, void* dq, void* dk1, void* dk2, void* dv1, void* dv2, int B,
                           int H, int T, int D, int dtype, float alpha, int causal, int k_diff, void* workspace,
-                          size_t workspace_bytes, unsigned flags, void* stream) {
+                          size_t workspace_bytes, unsigned flags, void* stream, DpsKept kept) {
     if (empty_problem(B, H, T)) return check_common(1, 1, 1, D, dtype);
     int rc = check_common(B, H, T, D, dtype);
     if (rc != TRITT_OK) return rc;
@@ -948,6 +992,7 @@ int tritt_dps_bwd_strided(const void* q, const void* k1, const void* k2, const v
         MfmaDpsArgs a{};
         a.q = q; a.k1 = k1; a.k2 = k2; a.v1 = v1; a.v2 = v2; a.o = o; a.d_o = d_o; a.lse_in = lse;
         a.dq = dq; a.dk1 = dk1; a.dk2 = dk2; a.dv1 = dv1; a.dv2 = dv2; a.workspace = workspace;
+        a.kept_r = kept.r; a.kept_lse1 = kept.lse1;
         a.BH = B * H; a.T = T; a.D = D; a.alpha = alpha; a.causal = causal ? 1 : 0; a.k_diff = clampw(k_diff, T);
         a.is_bf16 = dtype == TRITT_BF16;
         dps_views(a, in_layouts, d_o_layout, H, T, D);
@@ -961,8 +1006,50 @@ int tritt_dps_bwd_strided(const void* q, const void* k1, const void* k2, const v
     if (rc != TRITT_OK) return rc;
     if (!workspace || workspace_bytes < plain + v.bytes) return TRITT_ERR_WORKSPACE;
     run_pack(v, B, H, T, D, dtype, (hipStream_t)stream);
-    return tritt_dps_bwd(v.ptr[0], v.ptr[1], v.ptr[2], v.ptr[3], v.ptr[4], o, lse, v.ptr[5], dq, dk1, dk2, dv1, dv2, B, H, T,
-                         D, dtype, alpha, causal, k_diff, workspace, plain, flags, stream);
+    return dps_bwd_call(v.ptr[0], v.ptr[1], v.ptr[2], v.ptr[3], v.ptr[4], o, lse, v.ptr[5], dq, dk1, dk2, dv1, dv2, B, H, T,
+                         D, dtype, alpha, causal, k_diff, workspace, plain, flags, stream, kept);
+}
+
+int tritt_dps_bwd_strided(const void* q, const void* k1, const void* k2, const void* v1, const void* v2,
+                          const tritt_layout* in_layouts, const void* o, const float* lse, const void* d_o,
+                          const tritt_layout* d_o_layout, void* dq, void* dk1, void* dk2, void* dv1, void* dv2, int B,
+                          int H, int T, int D, int dtype, float alpha, int causal, int k_diff, void* workspace,
+                          size_t workspace_bytes, unsigned flags, void* stream) {
+    return dps_bwd_strided_call(q, k1, k2, v1, v2, in_layouts, o, lse, d_o, d_o_layout, dq, dk1, dk2, dv1, dv2, B, H, T, D,
+                                dtype, alpha, causal, k_diff, workspace, workspace_bytes, flags, stream, DpsKept{});
+}
+
+int tritt_dps_keeps(int D, int dtype, unsigned flags) { return dps_keeps(D, dtype, flags) ? 1 : 0; }
+
+static int check_kept(const float* r, const float* lse1, int B, int H, int T, int D, int dtype, unsigned flags) {
+    if (empty_problem(B, H, T)) return TRITT_OK;
+    if (any_null({r, lse1}) || any_misaligned({r, lse1})) return TRITT_ERR_INVALID;
+    return dps_keeps(D, dtype, flags) ? TRITT_OK : TRITT_ERR_UNSUPPORTED;
+}
+
+int tritt_dps_fwd_keep(const void* q, const void* k1, const void* k2, const void* v1, const void* v2,
+                       const tritt_layout* in_layouts, void* o, float* lse, float* r, float* lse1, int B, int H, int T, int D,
+                       int dtype, float alpha, int causal, int k_diff, void* workspace, size_t workspace_bytes,
+                       unsigned flags, void* stream) {
+    if (int rc = check_kept(r, lse1, B, H, T, D, dtype, flags); rc != TRITT_OK) return rc;
+    return in_layouts ? dps_fwd_strided_call(q, k1, k2, v1, v2, in_layouts, o, lse, B, H, T, D, dtype, alpha, causal, k_diff,
+                                             workspace, workspace_bytes, flags, stream, DpsKept{r, lse1})
+                      : dps_fwd_call(q, k1, k2, v1, v2, o, lse, B, H, T, D, dtype, alpha, causal, k_diff, workspace,
+                                     workspace_bytes, flags, stream, DpsKept{r, lse1});
+}
+
+int tritt_dps_bwd_kept(const void* q, const void* k1, const void* k2, const void* v1, const void* v2,
+                       const tritt_layout* in_layouts, const void* o, const float* lse, const float* r, const float* lse1,
+                       const void* d_o, const tritt_layout* d_o_layout, void* dq, void* dk1, void* dk2, void* dv1, void* dv2,
+                       int B, int H, int T, int D, int dtype, float alpha, int causal, int k_diff, void* workspace,
+                       size_t workspace_bytes, unsigned flags, void* stream) {
+    if (int rc = check_kept(r, lse1, B, H, T, D, dtype, flags); rc != TRITT_OK) return rc;
+    const DpsKept kept{const_cast<float*>(r), const_cast<float*>(lse1)};  // only read
+    return in_layouts || d_o_layout
+               ? dps_bwd_strided_call(q, k1, k2, v1, v2, in_layouts, o, lse, d_o, d_o_layout, dq, dk1, dk2, dv1, dv2, B, H, T, D,
+                                      dtype, alpha, causal, k_diff, workspace, workspace_bytes, flags, stream, kept)
+               : dps_bwd_call(q, k1, k2, v1, v2, o, lse, d_o, dq, dk1, dk2, dv1, dv2, B, H, T, D, dtype, alpha, causal, k_diff,
+                              workspace, workspace_bytes, flags, stream, kept);
 }
 
 // The triple-dot backward on the 16-bit matrix-core path reads the six views where they lie when every row stride

@@ -895,6 +895,10 @@ struct PrepP {
     E *up1, *k1p1, *k2p1, *qp1, *dop1;  // packing P1
     E *up2, *k1p2, *k2p2, *qp2, *dop2;  // packing P2
     float *lse2, *delta;
+    // the forward's R, for W = R * V2
+    const float* r;
+    View<E, SV> v2;
+    E *w, *wp1;
     int BH, T, Tp;
     int H;  // heads per batch entry in the views' indexing
 };
@@ -946,7 +950,7 @@ __global__ __launch_bounds__(256) void dps_prep_kernel(PrepP<E, SV> p) {
             __syncthreads();
         }
     };
-    // blockIdx.y deals the tensors out (3 in the forward, 5 and the row vectors in the backward): a workgroup per
+    // blockIdx.y deals the tensors out (3 in the forward, 5, the row vectors and W in the backward): a workgroup per
     // tile walking them one after the other was five dependent round trips through LDS
     const int job = blockIdx.y;
     if (job == 0) emit(p.v1, p.up1, p.up2, true);
@@ -954,6 +958,24 @@ __global__ __launch_bounds__(256) void dps_prep_kernel(PrepP<E, SV> p) {
     if (job == 2) emit(p.k2, p.k2p1, p.k2p2, false);
     if (job == 3 && p.q) emit(p.q, p.qp1, p.qp2, false);
     if (job == 4 && p.d_o) emit(p.d_o, p.dop1, p.dop2, false);
+    if (job == 6 && p.r) {
+        for (int idx = threadIdx.x; idx < 32 * (D / 8); idx += 256) {
+            const int j = j0 + idx / (D / 8), d0 = (idx % (D / 8)) * 8;
+            v8 x;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] = (E)0.f;
+            if (j < T) {
+                const size_t off = base + (size_t)j * D + d0;
+                const float4 a = *reinterpret_cast<const float4*>(p.r + off), b = *reinterpret_cast<const float4*>(p.r + off + 4);
+                const v8 v = *reinterpret_cast<const v8*>(p.v2.row(at, j, T, D) + d0);
+                const float r[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+                for (int e = 0; e < 8; ++e) x[e] = (E)(r[e] * (float)v[e]);
+                *reinterpret_cast<v8*>(p.w + off) = x;
+            }
+            *reinterpret_cast<v8*>(p.wp1 + tb + p1_index<D>(j, d0)) = x;
+        }
+    }
     if (job == 5 && p.delta) {
         // Delta[j] = dO[j] . O[j]: the D / 8 lanes that hold a row's 16-byte pieces sit next to each other
         constexpr int cpr = D / 8;
@@ -1078,15 +1100,16 @@ hipError_t run_fwd(const MfmaDpsArgs& a, hipStream_t st, bool for_bwd) {
         pp.BH = a.BH; pp.T = a.T; pp.Tp = Tp; pp.H = a.H;
         hipLaunchKernelGGL((dps_prep_kernel<E, D, SV>), dim3(grid.x, 3), dim3(256), 0, st, pp);
     }
-    // inner: rows K2[t], keys K1, values U; R (fp32, backward only), W = R * V2 and W^T, lse1 (log2)
+    // inner: rows K2[t], keys K1, values U; R (fp32, for the backward only), W = R * V2 and W^T, lse1 (log2)
     AttnFwdP<E, SV> p{};
     p.x = caller_view<E, SV>(a, a.k2, a.lk2); p.kp = (const E*)(ws + l.k1p1); p.vp2 = (const E*)(ws + l.up2);
     p.mul = caller_view<E, SV>(a, a.v2, a.lv2);
-    p.out_f32 = for_bwd ? (float*)(ws + l.r) : nullptr;
+    float* const lse1 = a.kept_lse1 ? a.kept_lse1 : (float*)(ws + l.lse1);
+    p.out_f32 = for_bwd ? (float*)(ws + l.r) : a.kept_r;
     p.outm = for_bwd ? (E*)(ws + l.w) : nullptr;
     p.outm_p1 = for_bwd ? (E*)(ws + l.wp1) : nullptr;
     p.outm_p2 = (E*)(ws + l.wp2);
-    p.lse = (float*)(ws + l.lse1); p.lse_stride = Tp; p.lse_scale = 1.0f;
+    p.lse = lse1; p.lse_stride = Tp; p.lse_scale = 1.0f;
     p.BH = a.BH; p.H = a.H; p.T = a.T; p.Tp = Tp; p.scale_log2 = sl2; p.causal = a.causal; p.k_diff = a.k_diff;
     p.pair = pair_in;
     // Large grids take the kernel whose workgroups own 128 rows and share the streamed tiles through LDS
@@ -1111,7 +1134,7 @@ hipError_t run_fwd(const MfmaDpsArgs& a, hipStream_t st, bool for_bwd) {
     if (for_bwd) return hipGetLastError();
     // outer: rows Q[q], keys K2 with bias lse1, values W; O and LSE (natural log)
     AttnFwdP<E, SV> o{};
-    o.x = caller_view<E, SV>(a, a.q, a.lq); o.kp = (const E*)(ws + l.k2p1); o.vp2 = (const E*)(ws + l.wp2); o.bias = (const float*)(ws + l.lse1);
+    o.x = caller_view<E, SV>(a, a.q, a.lq); o.kp = (const E*)(ws + l.k2p1); o.vp2 = (const E*)(ws + l.wp2); o.bias = lse1;
     o.out = (E*)a.o_out; o.lse = a.lse_out; o.lse_stride = a.T; o.lse_scale = kLn2;
     o.BH = a.BH; o.H = a.H; o.T = a.T; o.Tp = Tp; o.scale_log2 = sl2; o.causal = a.causal; o.k_diff = a.T;
     o.pair = pair_out;
@@ -1150,10 +1173,21 @@ hipError_t run_bwd(const MfmaDpsArgs& a, hipStream_t st) {
     pp.qp2 = (E*)(ws + l.qp2); pp.dop2 = (E*)(ws + l.dop2);
     pp.lse2 = (float*)(ws + l.lse2); pp.delta = (float*)(ws + l.delta);
     pp.BH = a.BH; pp.T = a.T; pp.Tp = Tp; pp.H = a.H;
-    hipLaunchKernelGGL((dps_prep_kernel<E, D, SV>), dim3(grid.x, 6), dim3(256), 0, st, pp);
-    // recompute the inner pass: R, W, W^T, lse1
-    e = run_fwd<E, D, kW, SV>(a, st, true);
-    if (e != hipSuccess) return e;
+    // R, W, W^T, lse1 of the inner pass: from the forward where the caller kept R and lse1 (W = R * V2 is then formed by the
+    // prep launch), else by running that pass again.  Keeping them holds four bytes per element between the two calls and
+    // takes one of the backward's seven products and a launch away; training steps, bf16, run again -> kept: B=4 H=8
+    // T=1024 154 -> 142 us, B=1 H=8 T=8192 k_diff 2048 822 -> 784 us.
+    const float *r = (const float*)(ws + l.r), *lse1 = (const float*)(ws + l.lse1);
+    if (a.kept_r) {
+        r = a.kept_r; lse1 = a.kept_lse1;
+        pp.r = r; pp.v2 = caller_view<E, SV>(a, a.v2, a.lv2); pp.w = (E*)(ws + l.w); pp.wp1 = (E*)(ws + l.wp1);
+        pp.up2 = nullptr;  // the inner pass's values
+        hipLaunchKernelGGL((dps_prep_kernel<E, D, SV>), dim3(grid.x, 7), dim3(256), 0, st, pp);
+    } else {
+        hipLaunchKernelGGL((dps_prep_kernel<E, D, SV>), dim3(grid.x, 6), dim3(256), 0, st, pp);
+        e = run_fwd<E, D, kW, SV>(a, st, true);
+        if (e != hipSuccess) return e;
+    }
 
     // outer pass: X = Q, G = dO, K = K2 (bias lse1), V = W
     AttnBwdP<E, SV> o{};
@@ -1162,12 +1196,12 @@ hipError_t run_bwd(const MfmaDpsArgs& a, hipStream_t st) {
     o.kp = (const E*)(ws + l.k2p1); o.vp = (const E*)(ws + l.wp1); o.kp2 = (const E*)(ws + l.k2p2);
     o.xp = (const E*)(ws + l.qp1); o.gp = (const E*)(ws + l.dop1);
     o.xp2 = (const E*)(ws + l.qp2); o.gp2 = (const E*)(ws + l.dop2);
-    o.bias = (const float*)(ws + l.lse1); o.lse2 = (const float*)(ws + l.lse2); o.delta = (const float*)(ws + l.delta);
+    o.bias = lse1; o.lse2 = (const float*)(ws + l.lse2); o.delta = (const float*)(ws + l.delta);
     o.BH = a.BH; o.H = a.H; o.T = a.T; o.Tp = Tp; o.alpha = a.alpha; o.causal = a.causal; o.k_diff = a.T;
     o.pair = pair_out;
     o.dx = (E*)a.dq;
     o.dk_f32 = (float*)(ws + l.dk2p);
-    o.r_f32 = (const float*)(ws + l.r); o.v2 = caller_view<E, SV>(a, a.v2, a.lv2); o.dv2 = (E*)a.dv2;
+    o.r_f32 = r; o.v2 = caller_view<E, SV>(a, a.v2, a.lv2); o.dv2 = (E*)a.dv2;
     o.dr = (E*)(ws + l.dr); o.dr_p1 = (E*)(ws + l.drp1); o.dr_p2 = (E*)(ws + l.drp2); o.delta1 = (float*)(ws + l.delta1);
     // Large grids: the kernels whose workgroups own 128 rows and share the streamed tiles through LDS
     // (dps_bwd_shared.hpp), as the forward passes do (run_fwd).  They pay from 512 such workgroups on; measured
@@ -1207,7 +1241,7 @@ hipError_t run_bwd(const MfmaDpsArgs& a, hipStream_t st) {
     i.kp = (const E*)(ws + l.k1p1); i.vp = (const E*)(ws + l.up1); i.kp2 = (const E*)(ws + l.k1p2);
     i.xp = (const E*)(ws + l.k2p1); i.gp = (const E*)(ws + l.drp1);
     i.xp2 = (const E*)(ws + l.k2p2); i.gp2 = (const E*)(ws + l.drp2);
-    i.lse2 = (const float*)(ws + l.lse1); i.delta = (const float*)(ws + l.delta1);
+    i.lse2 = lse1; i.delta = (const float*)(ws + l.delta1);
     i.BH = a.BH; i.H = a.H; i.T = a.T; i.Tp = Tp; i.alpha = a.alpha; i.causal = a.causal; i.k_diff = a.k_diff;
     i.pair = pair_in;
     i.addend = (const float*)(ws + l.dk2p); i.dx = (E*)a.dk2;

@@ -110,6 +110,7 @@ struct DpsArgs {
     const float* d_o;
     // fp32 tensors on the matrix cores: the backward forms u and delta from v1 and o_in itself and leaves dV1 in du
     const float *v1, *o_in;
+    bool kept;           // backward on the matrix cores, fp32 tensors: r and lse1 are the forward's
     float *dq, *dk1, *dk2, *du, *dv2;
     // scratch, all fp32: r, w, dw, dr, dk2_part [BH,T,D]; lse1, delta, dlse1, delta1 [BH,T] (dw, dlse1 and, in the forward,
     // r: the VALU kernels only)
@@ -194,6 +195,9 @@ struct MfmaDpsArgs {
     const void *o, *d_o;  // backward inputs
     const float* lse_in;  // backward input
     void *dq, *dk1, *dk2, *dv1, *dv2;
+    // the inner pass's rows R [BH,T,D] and log-sum-exps [BH, T rounded up to 32] (log2 units): left here by the forward,
+    // taken from here by the backward instead of running that pass again; null: neither
+    float *kept_r, *kept_lse1;
     void* workspace;      // mfma_dps_{fwd,bwd}_workspace() bytes
     int BH, T, D;
     float alpha;

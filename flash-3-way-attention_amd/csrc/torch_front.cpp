@@ -84,6 +84,7 @@ struct Problem {
     bool causal;
     int64_t w[4];  // k1_window, k2_window, kk_left, kk_right; dot-product sum: k_diff in w[0]
     int64_t flags;
+    bool keep = false;  // dot-product sum: the forward leaves what its backward would form again
 };
 void save(AutogradContext* ctx, const Problem& p) {
     ctx->saved_data["p"] = std::vector<int64_t>{p.causal, p.w[0], p.w[1], p.w[2], p.w[3], p.flags};
@@ -92,6 +93,11 @@ void save(AutogradContext* ctx, const Problem& p) {
 Problem load(AutogradContext* ctx) {
     const std::vector<int64_t> v = ctx->saved_data["p"].toIntVector();
     return Problem{ctx->saved_data["s"].toDouble(), v[0] != 0, {v[1], v[2], v[3], v[4]}, v[5]};
+}
+// a saved tensor as the library takes one that has to be dense (a saved-tensor hook may bring it back in another layout)
+Tensor dense(const Tensor& t) {
+    Tensor d = t.contiguous();
+    return reinterpret_cast<uintptr_t>(d.data_ptr()) % 16 ? d.clone(at::MemoryFormat::Contiguous) : d;
 }
 Tensor gradient_like(const Tensor& q) { return at::empty(q.sizes(), q.options()); }
 
@@ -186,6 +192,18 @@ struct Dps : torch::autograd::Function<Dps> {
                                             : tritt_dps_fwd_strided_workspace_bytes(B, H, T, D, code, flags, l.at.data()),
                                     q);
         void* st = current_stream(q);
+        if (p.keep) {
+            const Tensor r = at::empty({B, H, T, D}, m.options()), lse1 = at::empty({B, H, (T + 31) / 32 * 32}, m.options());
+            check(tritt_dps_fwd_keep(q.data_ptr(), in[1].data_ptr(), in[2].data_ptr(), in[3].data_ptr(), in[4].data_ptr(),
+                                     l.dense ? nullptr : l.at.data(), o.data_ptr(), m.data_ptr<float>(), r.data_ptr<float>(),
+                                     lse1.data_ptr<float>(), B, H, T, D, code, (float)p.scale, p.causal, k_diff, ws.data_ptr(),
+                                     ws.numel(), flags, st),
+                  "tritt_dps_fwd_keep");
+            ctx->save_for_backward({in[0], in[1], in[2], in[3], in[4], o, m, r, lse1});
+            ctx->mark_non_differentiable({m});
+            save(ctx, p);
+            return {o, m};
+        }
         check(l.dense ? tritt_dps_fwd(q.data_ptr(), in[1].data_ptr(), in[2].data_ptr(), in[3].data_ptr(), in[4].data_ptr(),
                                       o.data_ptr(), m.data_ptr<float>(), B, H, T, D, code, (float)p.scale, p.causal, k_diff,
                                       ws.data_ptr(), ws.numel(), flags, st)
@@ -212,7 +230,7 @@ struct Dps : torch::autograd::Function<Dps> {
         const int code = dtype_code(q.scalar_type()), k_diff = (int)p.w[0];
         const unsigned flags = (unsigned)p.flags;
         const Layouts l = layouts_of(in);
-        const bool dense = l.dense && d_o.is_contiguous();
+        const bool all_dense = l.dense && d_o.is_contiguous();
         variable_list g(6);
         void* gp[5];
         for (int i = 0; i < 5; ++i) {
@@ -221,11 +239,20 @@ struct Dps : torch::autograd::Function<Dps> {
         }
         const tritt_layout ldo = layout_of(d_o);
         const tritt_layout *lp = l.dense ? nullptr : l.at.data(), *ldp = d_o.is_contiguous() ? nullptr : &ldo;
-        const Tensor ws = workspace(dense ? tritt_dps_bwd_workspace_bytes(B, H, T, D, code, flags)
-                                          : tritt_dps_bwd_strided_workspace_bytes(B, H, T, D, code, flags, lp, ldp),
+        const Tensor ws = workspace(all_dense ? tritt_dps_bwd_workspace_bytes(B, H, T, D, code, flags)
+                                              : tritt_dps_bwd_strided_workspace_bytes(B, H, T, D, code, flags, lp, ldp),
                                     q);
         void* st = current_stream(q);
-        check(dense ? tritt_dps_bwd(q.data_ptr(), in[1].data_ptr(), in[2].data_ptr(), in[3].data_ptr(), in[4].data_ptr(),
+        if (s.size() > 7) {
+            const Tensor r = dense(s[7]), lse1 = dense(s[8]);
+            check(tritt_dps_bwd_kept(q.data_ptr(), in[1].data_ptr(), in[2].data_ptr(), in[3].data_ptr(), in[4].data_ptr(), lp,
+                                     o.data_ptr(), m.data_ptr<float>(), r.data_ptr<float>(), lse1.data_ptr<float>(),
+                                     d_o.data_ptr(), ldp, gp[0], gp[1], gp[2], gp[3], gp[4], B, H, T, D, code, (float)p.scale,
+                                     p.causal, k_diff, ws.data_ptr(), ws.numel(), flags, st),
+                  "tritt_dps_bwd_kept");
+            return g;
+        }
+        check(all_dense ? tritt_dps_bwd(q.data_ptr(), in[1].data_ptr(), in[2].data_ptr(), in[3].data_ptr(), in[4].data_ptr(),
                                     o.data_ptr(), m.data_ptr<float>(), d_o.data_ptr(), gp[0], gp[1], gp[2], gp[3], gp[4], B, H,
                                     T, D, code, (float)p.scale, p.causal, k_diff, ws.data_ptr(), ws.numel(), flags, st)
                     : tritt_dps_bwd_strided(q.data_ptr(), in[1].data_ptr(), in[2].data_ptr(), in[3].data_ptr(),
@@ -343,6 +370,8 @@ PyObject* py_dps(PyObject*, PyObject* const* args, Py_ssize_t n) {
             !truth(args[8], &convert))
             Py_RETURN_NONE;
         if (convert) p.flags = TRITT_FLAG_FORCE_GENERIC;
+        if (at::GradMode::is_enabled() && tritt_dps_keeps((int)(*t)[0].size(3), dtype_code((*t)[0].scalar_type()), (unsigned)p.flags))
+            for (const Tensor& x : *t) p.keep = p.keep || x.requires_grad();
         variable_list r;
         {
             pybind11::gil_scoped_release release;

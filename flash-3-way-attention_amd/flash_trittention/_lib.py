@@ -52,6 +52,10 @@ _PROTOS = {
     "tritt_dps_fwd_strided_workspace_bytes": (_sz, [_i] * 5 + [_u, _lp]),
     "tritt_dps_fwd_strided": (_i, [_vp] * 5 + [_lp] + [_vp] * 2 + [_i] * 5 + [_f] + [_i] * 2 + [_vp, _sz, _u, _vp]),
     "tritt_dps_bwd_strided_workspace_bytes": (_sz, [_i] * 5 + [_u, _lp, _lp]),
+    "tritt_dps_keeps": (_i, [_i, _i, _u]),
+    "tritt_dps_fwd_keep": (_i, [_vp] * 5 + [_lp] + [_vp] * 4 + [_i] * 5 + [_f] + [_i] * 2 + [_vp, _sz, _u, _vp]),
+    "tritt_dps_bwd_kept": (_i, [_vp] * 5 + [_lp] + [_vp] * 5 + [_lp] + [_vp] * 5 + [_i] * 5 + [_f] + [_i] * 2
+                           + [_vp, _sz, _u, _vp]),
     "tritt_dps_bwd_strided": (_i, [_vp] * 5 + [_lp] + [_vp] * 3 + [_lp] + [_vp] * 5 + [_i] * 5 + [_f] + [_i] * 2
                               + [_vp, _sz, _u, _vp]),
 }

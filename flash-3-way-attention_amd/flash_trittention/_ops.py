@@ -83,7 +83,9 @@ def tdp_bwd_impl(q, k1, k2, v1, v2, o, lse, d_o, softmax_scale: float, causal: b
     return grads
 
 
-def dps_fwd_impl(q, k1, k2, v1, v2, softmax_scale: float, causal: bool, k_diff: int, flags: int):
+def dps_fwd_impl(q, k1, k2, v1, v2, softmax_scale: float, causal: bool, k_diff: int, flags: int, keep: bool = False):
+    """(o, m); with `keep` also what the backward would otherwise form again (`kept` of dps_bwd_impl), None where the
+    library has no such form."""
     _lib.require_gpu(q, "TrittentionTriton")
     q, k1, k2, v1, v2 = (_lib.view(t) for t in (q, k1, k2, v1, v2))
     lay = _lib.layouts((q, k1, k2, v1, v2))
@@ -93,8 +95,18 @@ def dps_fwd_impl(q, k1, k2, v1, v2, softmax_scale: float, causal: bool, k_diff: 
     o = _empty_like_bhtd(q)
     m = torch.empty((B, H, T), dtype=torch.float32, device=q.device)
     shape = (B, H, T, D, code, float(softmax_scale), int(causal), k_diff)
+    kept = None
     with _lib.on_device(q.device):
-        if lay is None:
+        if keep and lib.tritt_dps_keeps(D, code, flags):
+            kept = (torch.empty((B, H, T, D), dtype=torch.float32, device=q.device),
+                    torch.empty((B, H, (T + 31) // 32 * 32), dtype=torch.float32, device=q.device))
+            need = (_lib.workspace_bytes("tritt_dps_fwd_workspace_bytes", B, H, T, D, code, flags) if lay is None else
+                    _lib.workspace_bytes("tritt_dps_fwd_strided_workspace_bytes", B, H, T, D, code, flags, lay))
+            ws = _lib.workspace(need, q.device)
+            st = lib.tritt_dps_fwd_keep(_lib.ptr(q), _lib.ptr(k1), _lib.ptr(k2), _lib.ptr(v1), _lib.ptr(v2), lay,
+                                        _lib.ptr(o), _lib.ptr(m), *(_lib.ptr(t) for t in kept), *shape, _lib.ptr(ws),
+                                        ws.numel(), flags, _lib.stream_ptr(q.device))
+        elif lay is None:
             ws = _lib.workspace(_lib.workspace_bytes("tritt_dps_fwd_workspace_bytes", B, H, T, D, code, flags), q.device)
             st = lib.tritt_dps_fwd(_lib.ptr(q), _lib.ptr(k1), _lib.ptr(k2), _lib.ptr(v1), _lib.ptr(v2), _lib.ptr(o),
                                    _lib.ptr(m), *shape, _lib.ptr(ws), ws.numel(), flags, _lib.stream_ptr(q.device))
@@ -105,10 +117,10 @@ def dps_fwd_impl(q, k1, k2, v1, v2, softmax_scale: float, causal: bool, k_diff: 
                                            _lib.ptr(o), _lib.ptr(m), *shape, _lib.ptr(ws), ws.numel(), flags,
                                            _lib.stream_ptr(q.device))
     _lib.check(st, "tritt_dps_fwd")
-    return o, m
+    return (o, m, kept) if keep else (o, m)
 
 
-def dps_bwd_impl(q, k1, k2, v1, v2, o, m, d_o, softmax_scale: float, causal: bool, k_diff: int, flags: int):
+def dps_bwd_impl(q, k1, k2, v1, v2, o, m, d_o, softmax_scale: float, causal: bool, k_diff: int, flags: int, kept=None):
     B, H, T, D = q.shape
     q, k1, k2, v1, v2, d_o = (_lib.view(t) for t in (q, k1, k2, v1, v2, d_o))
     lay, lay_do = _lib.layouts((q, k1, k2, v1, v2)), _lib.layouts((d_o,))
@@ -118,7 +130,16 @@ def dps_bwd_impl(q, k1, k2, v1, v2, o, m, d_o, softmax_scale: float, causal: boo
     gptr = [_lib.ptr(t) for t in grads]
     shape = (B, H, T, D, code, float(softmax_scale), int(causal), k_diff)
     with _lib.on_device(q.device):
-        if lay is None and lay_do is None:
+        if kept is not None:
+            need = (_lib.workspace_bytes("tritt_dps_bwd_workspace_bytes", B, H, T, D, code, flags)
+                    if lay is None and lay_do is None else
+                    _lib.workspace_bytes("tritt_dps_bwd_strided_workspace_bytes", B, H, T, D, code, flags, lay, lay_do))
+            ws = _lib.workspace(need, q.device)
+            kept = [_lib.dense(t) for t in kept]
+            st = lib.tritt_dps_bwd_kept(_lib.ptr(q), _lib.ptr(k1), _lib.ptr(k2), _lib.ptr(v1), _lib.ptr(v2), lay,
+                                        _lib.ptr(o), _lib.ptr(m), *(_lib.ptr(t) for t in kept), _lib.ptr(d_o), lay_do,
+                                        *gptr, *shape, _lib.ptr(ws), ws.numel(), flags, _lib.stream_ptr(q.device))
+        elif lay is None and lay_do is None:
             ws = _lib.workspace(_lib.workspace_bytes("tritt_dps_bwd_workspace_bytes", B, H, T, D, code, flags), q.device)
             st = lib.tritt_dps_bwd(_lib.ptr(q), _lib.ptr(k1), _lib.ptr(k2), _lib.ptr(v1), _lib.ptr(v2), _lib.ptr(o),
                                    _lib.ptr(m), _lib.ptr(d_o), *gptr, *shape, _lib.ptr(ws), ws.numel(), flags,

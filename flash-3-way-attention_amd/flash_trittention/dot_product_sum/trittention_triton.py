@@ -48,9 +48,15 @@ class TrittentionTritonFunction(torch.autograd.Function):
         flags = _lib.FLAG_AUTO if compiling else getattr(getattr(ctx, "_forward_cls", None), "IMPL_FLAGS", _lib.FLAG_AUTO)
         if convert_to_float32 and not flags & _lib.FLAG_FORCE_MFMA:
             flags |= _lib.FLAG_FORCE_GENERIC  # fp32 operands throughout (trittention_triton.py:92-98 of the reference)
-        call = torch.ops.flash_trittention.dps_fwd if compiling else _ops.dps_fwd_impl
-        o, m = call(q, k1, k2, v1, v2, float(softmax_scale), bool(causal), k_diff, flags)
-        ctx.save_for_backward(q, k1, k2, v1, v2, o, m)
+        args = (q, k1, k2, v1, v2, float(softmax_scale), bool(causal), k_diff, flags)
+        kept = None
+        if compiling:
+            o, m = torch.ops.flash_trittention.dps_fwd(*args)
+        elif any(ctx.needs_input_grad):
+            o, m, kept = _ops.dps_fwd_impl(*args, keep=True)
+        else:
+            o, m = _ops.dps_fwd_impl(*args)
+        ctx.save_for_backward(q, k1, k2, v1, v2, o, m, *(kept or ()))
         ctx.causal = bool(causal)
         ctx.softmax_scale = float(softmax_scale)
         ctx.k_diff = k_diff
@@ -60,15 +66,17 @@ class TrittentionTritonFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_output, m_grad=None):
-        q, k1, k2, v1, v2, o, m = ctx.saved_tensors
+        q, k1, k2, v1, v2, o, m, *kept = ctx.saved_tensors
         assert grad_output.shape == o.shape, f"Shape mismatch: O={o.shape}, dO={grad_output.shape}"
         assert o.device == grad_output.device, "O and dO must be on the same device"
         assert o.dtype == grad_output.dtype, "O and dO must have the same dtype"
         if _ops.compiling():
             grad_output = grad_output.contiguous()
-        call = torch.ops.flash_trittention.dps_bwd if _ops.compiling() else _ops.dps_bwd_impl
-        dq, dk1, dk2, dv1, dv2 = call(q, k1, k2, v1, v2, o, m, grad_output, ctx.softmax_scale, ctx.causal, ctx.k_diff,
-                                      ctx.flags)
+        args = (q, k1, k2, v1, v2, o, m, grad_output, ctx.softmax_scale, ctx.causal, ctx.k_diff, ctx.flags)
+        if _ops.compiling():
+            dq, dk1, dk2, dv1, dv2 = torch.ops.flash_trittention.dps_bwd(*args)
+        else:
+            dq, dk1, dk2, dv1, dv2 = _ops.dps_bwd_impl(*args, kept=kept or None)
         return dq, dk1, dk2, dv1, dv2, None, None, None, None, None
 
 

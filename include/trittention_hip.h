@@ -253,6 +253,24 @@ int tritt_dps_bwd_strided(const void* q, const void* k1, const void* k2, const v
                           int B, int H, int T, int D, int dtype, float alpha, int causal, int k_diff,
                           void* workspace, size_t workspace_bytes, unsigned flags, void* stream);
 
+/* The dot-product-sum forward for training: what the inner pass (the attention of K2 over K1) leaves, `r` (fp32
+ * [B,H,T,D], its output) and `lse1` (fp32 [B,H,T rounded up to a multiple of 32], its log-sum-exps in log2 units), stays with
+ * the caller, and the backward reads it instead of running that pass again.  Both buffers 16-byte aligned; the backward takes
+ * them only from a forward of the same arguments.  tritt_dps_keeps tells whether a head dimension and type have this form
+ * (16-bit types with D = 32, 64, 128; fp32 with D = 32, 64); elsewhere the two calls return TRITT_ERR_UNSUPPORTED.  Layouts
+ * as in the strided calls, workspace sizes from the plain queries (from the strided ones if a layout is given). */
+int tritt_dps_keeps(int D, int dtype, unsigned flags);
+int tritt_dps_fwd_keep(const void* q, const void* k1, const void* k2, const void* v1, const void* v2,
+                       const tritt_layout* in_layouts, void* o, float* lse, float* r, float* lse1,
+                       int B, int H, int T, int D, int dtype, float alpha, int causal, int k_diff,
+                       void* workspace, size_t workspace_bytes, unsigned flags, void* stream);
+int tritt_dps_bwd_kept(const void* q, const void* k1, const void* k2, const void* v1, const void* v2,
+                       const tritt_layout* in_layouts, const void* o, const float* lse, const float* r, const float* lse1,
+                       const void* d_o, const tritt_layout* d_o_layout,
+                       void* dq, void* dk1, void* dk2, void* dv1, void* dv2,
+                       int B, int H, int T, int D, int dtype, float alpha, int causal, int k_diff,
+                       void* workspace, size_t workspace_bytes, unsigned flags, void* stream);
+
 /* Calibration for benchmarks (no counterpart in the reference).  Launches `blocks` workgroups of
  * eight waves that each issue iters * 4 independent 32x32x16 bf16 MFMAs and nothing else:
  * blocks * 8 * iters * 4 * 32768 flop.  Timed by the caller, it gives the rate the matrix pipes

@@ -166,3 +166,11 @@ def test_product_never_imports_oracle():
             if f.endswith((".py", ".hip", ".hpp", ".h")):
                 text = open(os.path.join(dirpath, f)).read()
                 assert "oracle" not in text, os.path.join(dirpath, f)
+
+
+def test_kept_inner_pass_where_there_is_none():
+    lib = _lib.lib()
+    assert lib.tritt_dps_keeps(64, _lib.TRITT_BF16, _lib.FLAG_AUTO) == 1
+    assert lib.tritt_dps_keeps(64, _lib.TRITT_BF16, _lib.FLAG_FORCE_GENERIC) == 0
+    assert lib.tritt_dps_keeps(16, _lib.TRITT_F32, _lib.FLAG_AUTO) == 0
+    assert lib.tritt_dps_keeps(128, _lib.TRITT_F32, _lib.FLAG_AUTO) == 0

@@ -426,3 +426,32 @@ def test_large_logits_with_convert_to_float32_hold_the_16_bit_bar():
     util.assert_close("m", m.cpu(), lse, rtol=1e-4, atol=1e-3)
     for name, leaf, want in zip(util.NAMES, leaves, grads):
         util.assert_mostly_close(name, leaf.grad.float().cpu(), want, **LOWP)
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 32), (torch.bfloat16, 64), (torch.float16, 128), (torch.float32, 32),
+                                     (torch.float32, 64)])
+@pytest.mark.parametrize("T,causal,k_diff", [(1, True, 1), (31, False, 31), (33, True, 7), (97, True, 97), (130, True, 64)])
+@pytest.mark.parametrize("fused", [False, True])
+@pytest.mark.parametrize("shared", [0, 1])
+def test_backward_from_the_kept_inner_pass(dtype, D, T, causal, k_diff, fused, shared, tune):
+    """A training step's forward leaves the inner pass's rows and log-sum-exps for its backward; the C ABI's plain backward
+    forms them again.  Both against the oracle's gradients, with the saved tensors untouched by a first backward."""
+    from flash_trittention import TrittentionTriton, _lib, _ops
+
+    print(f"case dps kept {dtype} D={D} T={T} causal={causal} k_diff={k_diff} fused={fused} shared={shared}", flush=True)
+    tune(_lib.TUNE_DPS_SHARED, shared)
+    scale, low = 1 / math.sqrt(D), dtype != torch.float32
+    inputs = orc.make_inputs(2, 3, T, D, dtype, seed=T + D)
+    z, _, grads = util.oracle_dps(inputs, scale, causal, k_diff, factorised=True)
+    *ins, d_o = (t.cuda() for t in inputs)
+    if fused:
+        ins = [t for t in torch.stack(ins, 2).permute(0, 3, 2, 1, 4).contiguous().permute(2, 0, 3, 1, 4)]
+    ins = [t.detach().requires_grad_(True) for t in ins]
+    out, m = TrittentionTriton(causal=causal, softmax_scale=scale, k_diff=k_diff)(*ins)
+    first = torch.autograd.grad(out, ins, d_o, retain_graph=True)
+    again = torch.autograd.grad(out, ins, d_o)
+    plain = _ops.dps_bwd_impl(*(t.detach() for t in ins), out.detach(), m, d_o, scale, causal, k_diff, _lib.FLAG_AUTO)
+    for name, a, b, c, want in zip(util.NAMES, first, again, plain, grads):
+        assert torch.equal(a, b), name
+        for got in (a.float().cpu(), c.float().cpu()):
+            (util.assert_mostly_close if low else util.assert_close)(name, got, want, **(LOWP if low else FP32))
