@@ -4,8 +4,8 @@
 // Under a windowed mask a query q only sees keys j in [q - wa, q] and k in [q - wb, q].  When the
 // windows are narrow, every key row a tile of 32 queries can touch (at most max(wa, wb) + 32 + 31 rows
 // of K1, U^T, K2 and V2) fits in LDS at once.  The workgroup loads that band ONCE, synchronises once,
-// and from then on its eight waves run independently with no barrier and no global load: each wave
-// walks its four queries one after another, per query the k-tiles of 32 inside [q - wb, q], per k-tile
+// and from then on its eight or sixteen waves run independently with no barrier and no global load: each
+// wave walks its four or two queries one after another, per query the k-tiles of 32 inside [q - wb, q], per k-tile
 // the 32-key steps of j inside the band of that tile.  Same formulation as the streaming kernel (virtual
 // rows (q, k), transposed scores, P fed back as the A operand); what changes is that a k-tile of a narrow
 // band has only a handful of steps, so everything per k-tile is kept cheap:
@@ -21,23 +21,24 @@
 
 namespace tritt {
 
-constexpr int kBandQ = 32;  // queries per workgroup: 8 waves x 4
+constexpr int kBandQ = 32;  // queries per workgroup
 
 // rows of the resident band: everything queries q0 .. q0+31 can touch (q0 is a multiple of 32, and so is the
 // first resident row)
 inline int band_rows(int wa, int wb) { return ((wa > wb ? wa : wb) + 31) / 32 * 32 + kBandQ; }
 
-template <int D>
+template <int D, int kW>
 constexpr size_t band_smem_bytes(int nr) {
-    return sizeof(uint16_t) * ((size_t)3 * nr * (D + 8) + (size_t)D * (nr + 8)) + sizeof(float) * (kBandQ * D + 8 * 32 + 5 * 16 * 64);
+    return sizeof(uint16_t) * ((size_t)3 * nr * (D + 8) + (size_t)D * (nr + 8)) + sizeof(float) * (kBandQ * D + kW * 32 + 5 * 16 * 64);
 }
 
-template <typename E, int D, bool MV = false>
-__global__ __launch_bounds__(512, 2) void tdp_fwd_band_kernel(FwdParams<E> p, int NR) {
+// kW: waves per workgroup (band_waves16)
+template <typename E, int D, int kW, bool MV = false>
+__global__ __launch_bounds__(64 * kW, kW / 4) void tdp_fwd_band_kernel(FwdParams<E> p, int NR) {
     using M = Mma<E>;
     using v8 = typename M::v8;
     using v2 = typename M::v2;
-    constexpr int KS = D / 16, DT = D / 32, LDK = D + 8;
+    constexpr int KS = D / 16, DT = D / 32, LDK = D + 8, kThreads = 64 * kW;
     const int LDU = NR + 8;
 
     extern __shared__ __align__(16) char smem[];
@@ -46,8 +47,8 @@ __global__ __launch_bounds__(512, 2) void tdp_fwd_band_kernel(FwdParams<E> p, in
     E* sV2 = sK2 + NR * LDK;
     E* sUT = sV2 + NR * LDK;               // [D][LDU]
     float* sQ = reinterpret_cast<float*>(sUT + D * LDU);  // [32][D]  Q * alpha*log2(e), fp32
-    float* sW = sQ + kBandQ * D;                                // [8][32] per-wave scratch
-    float* sTab = sW + 8 * 32;  // [5 slots][4][64 lanes][4]  band masks in the MFMA C layout; slot 4: zeros
+    float* sW = sQ + kBandQ * D;                                // [kW][32] per-wave scratch
+    float* sTab = sW + kW * 32;  // [5 slots][4][64 lanes][4]  band masks in the MFMA C layout; slot 4: zeros
 
     int bh, order;
     if (!xcd_tile(p.BH, p.nqt, blockIdx.x >> 3, blockIdx.x & 7, bh, order)) return;
@@ -75,7 +76,7 @@ __global__ __launch_bounds__(512, 2) void tdp_fwd_band_kernel(FwdParams<E> p, in
         const unsigned st_k1 = MV ? p.at_k1.st : in_st, st_k2 = MV ? p.at_k2.st : in_st, st_v2 = MV ? p.at_v2.st : in_st;
         const E* __restrict__ UT = p.ut + (size_t)bh * D * p.Tp;
         const int row_chunks = NR * (D / 8);
-        for (int c = tid; c < row_chunks; c += 512) {
+        for (int c = tid; c < row_chunks; c += kThreads) {
             const int r = c / (D / 8), ch = c % (D / 8);
             const unsigned row = (unsigned)min(rlo + r, T - 1);
             const uint4 a = *reinterpret_cast<const uint4*>(K1 + (size_t)(row * st_k1) + ch * 8);
@@ -86,7 +87,7 @@ __global__ __launch_bounds__(512, 2) void tdp_fwd_band_kernel(FwdParams<E> p, in
             *reinterpret_cast<uint4*>(sV2 + r * LDK + ch * 8) = v;
         }
         const int ut_chunks = D * (NR / 8);
-        for (int c = tid; c < ut_chunks; c += 512) {
+        for (int c = tid; c < ut_chunks; c += kThreads) {
             const int d = c / (NR / 8), cj = c % (NR / 8);
             const int j0 = rlo + cj * 8;
             uint4 u = {0u, 0u, 0u, 0u};
@@ -94,7 +95,7 @@ __global__ __launch_bounds__(512, 2) void tdp_fwd_band_kernel(FwdParams<E> p, in
             *reinterpret_cast<uint4*>(sUT + d * LDU + cj * 8) = u;
         }
     }
-    for (int idx = tid; idx < kBandQ * D; idx += 512) {
+    for (int idx = tid; idx < kBandQ * D; idx += kThreads) {
         const int r = idx / D, d = idx % D;
         sQ[idx] = (float)Q[(size_t)((unsigned)min(q0 + r, T - 1) * in_st) + d] * p.scale_log2;
     }
@@ -124,10 +125,10 @@ __global__ __launch_bounds__(512, 2) void tdp_fwd_band_kernel(FwdParams<E> p, in
         __builtin_amdgcn_wave_barrier();
     };
 
-    for (int qi = 0; qi < kBandQ / 8; ++qi) {
-        const int q = q0 + wave + 8 * qi;  // interleaved: the waves' loads stay even at the start of a sequence
+    for (int qi = 0; qi < kBandQ / kW; ++qi) {
+        const int q = q0 + wave + kW * qi;  // interleaved: the waves' loads stay even at the start of a sequence
         if (q >= T) break;
-        const float* sQw = sQ + (wave + 8 * qi) * D;
+        const float* sQw = sQ + (wave + kW * qi) * D;
 
         float Mrun = -INFINITY, Lrun = 0.f, Orun[DT];  // Lrun, Orun: per-lane partial sums
 #pragma unroll

@@ -951,8 +951,20 @@ static bool use_band_kernel(const MfmaFwdArgs& a) {
     if (a.split) return false;  // split operands: the streaming kernels only
     if (knobs().fwd_band < 0) return false;
     const int nr = band_rows(a.k1_window, a.k2_window);
-    const size_t smem = a.D == 32 ? band_smem_bytes<32>(nr) : a.D == 64 ? band_smem_bytes<64>(nr) : band_smem_bytes<128>(nr);
+    const size_t smem = a.D == 32 ? band_smem_bytes<32, 16>(nr) : a.D == 64 ? band_smem_bytes<64, 16>(nr) : band_smem_bytes<128, 8>(nr);
     return smem <= kBandSmemLimit;
+}
+
+// Sixteen waves per workgroup (two queries each) or eight (four each).  A wave's steps are a serial chain through LDS, matrix
+// and exp2 latencies, so the kernel wants four waves on a SIMD.  D = 64 takes sixteen: the band rarely leaves room for a second
+// workgroup, and does not repay it where it does.  D = 32 takes eight where two such workgroups fit a CU's LDS and the grid has
+// two for every CU.  At D = 128 a wave needs 195 registers: eight.  Forward, 8 -> 16 waves: D = 64 B=2 H=8 T=2048 windows 128 /
+// 32 209 -> 184 us, windows 16 / 8 64 -> 60 us, B=4 H=8 T=1024 windows 64 / 16 135 -> 111 us; D = 32 B=4 H=8 T=1024 windows
+// 300 751 -> 618 us, but where two fit, B=2 H=8 T=2048 windows 128 / 32, 119 -> 128 us.
+template <int D>
+static bool band_waves16(const MfmaFwdArgs& a, int nr) {
+    if (D != 32) return D == 64;
+    return 2 * band_smem_bytes<D, 8>(nr) > 160 * 1024 || a.BH * ((a.T + kBandQ - 1) / kBandQ) < 2 * 256;
 }
 
 // The layout the kernels are handed: the caller's strides, or those of a dense [BH][T][D] tensor (in_st == 0)
@@ -984,12 +996,15 @@ static hipError_t launch_band(const MfmaFwdArgs& a, hipStream_t st) {
     p.splits = 1;
     p.part = nullptr;
     const int nr = band_rows(p.wa, p.wb);
-    const size_t smem = band_smem_bytes<D>(nr);
-    auto kern = a.many_views ? tdp_fwd_band_kernel<E, D, true> : tdp_fwd_band_kernel<E, D, false>;
+    constexpr int kWide = D == 128 ? 8 : 16, kNarrow = D == 64 ? 16 : 8;
+    const bool wide = band_waves16<D>(a, nr);
+    const size_t smem = wide ? band_smem_bytes<D, kWide>(nr) : band_smem_bytes<D, kNarrow>(nr);
+    auto kern = wide ? (a.many_views ? tdp_fwd_band_kernel<E, D, kWide, true> : tdp_fwd_band_kernel<E, D, kWide, false>)
+                     : (a.many_views ? tdp_fwd_band_kernel<E, D, kNarrow, true> : tdp_fwd_band_kernel<E, D, kNarrow, false>);
     p.at_k1 = a.at_k1; p.at_k2 = a.at_k2; p.at_v2 = a.at_v2;
     hipError_t e = ensure_dynamic_smem(reinterpret_cast<const void*>(kern), smem);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(kern, dim3(8 * xcd_slots(a.BH, p.nqt)), dim3(512), smem, st, p, nr);
+    hipLaunchKernelGGL(kern, dim3(8 * xcd_slots(a.BH, p.nqt)), dim3(64 * (wide ? kWide : kNarrow)), smem, st, p, nr);
     return hipGetLastError();
 }
 

@@ -749,6 +749,20 @@ def test_band_resident_forward_matches_streaming_and_oracle(windows, D, tune):
         util.assert_mostly_close(name, a, b, **LOWP)
 
 
+@pytest.mark.parametrize("windows", [(40, 50, 9, 20), (300, 200, 60, 60)])
+@pytest.mark.parametrize("seq_len", [250, 256])
+def test_band_resident_forward_waves_of_a_workgroup_d32(windows, seq_len):
+    """512 query tiles at D = 32, where two workgroups of eight waves share a CU if the band is small; one head by itself takes
+    sixteen waves.  A query is one wave's work either way, so the head comes out bit for bit the same."""
+    print(f"case band waves {windows} T={seq_len}", flush=True)
+    inputs = orc.make_inputs(4, 16, seq_len, 32, torch.bfloat16, seed=seq_len)
+    out, _ = util.run_tdp(inputs, 32 ** -0.5, True, windows, backward=False, flags=FORCE_MFMA)
+    one = [t[1:2, 5:6].contiguous() for t in inputs]
+    alone, _ = util.run_tdp(one, 32 ** -0.5, True, windows, backward=False, flags=FORCE_MFMA)
+    assert torch.equal(out[1:2, 5:6], alone)
+    util.assert_close("out", alone, util.oracle_tdp(one, 32 ** -0.5, True, windows)[0], **LOWP)
+
+
 def test_band_resident_forward_large_logits():
     """Scores spanning hundreds under a narrow window: single waves leave the fast sweep and repeat their
     k-tile with the online softmax, and k-tiles with different reference maxima meet in the merge."""
