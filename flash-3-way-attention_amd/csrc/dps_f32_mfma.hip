@@ -44,7 +44,9 @@ __device__ __forceinline__ bool pair_valid(int causal, int k_diff, int r, int a)
 }
 
 // Rows row0 .. row0 + 31 of a head's row-major [T][D] operand (row0 is uniform).  A buffer resource of the rows that
-// exist: rows past T read as zeros, one lane offset serves all loads, and no 64-bit address is kept per lane.
+// exist: rows past T read as zeros, the loads share their lane offsets, and no 64-bit address is kept per lane.  Every
+// offset stands in the lane offset or the instruction: the scalar offset has no part in the range check, so a row reached
+// through it would be read from whatever lies behind the tensor, and a NaN there outlives its zero weight.
 template <int D>
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rows(const float* src, int row0, int T) {
     row0 = __builtin_amdgcn_readfirstlane(row0);
@@ -65,11 +67,14 @@ __device__ __forceinline__ void load_rows(float (&reg)[D / 2], const float* src,
 template <int D>
 __device__ __forceinline__ void load_cols(float (&reg)[D / 2], const float* src, int row0, int T, int n, int g) {
     const __amdgpu_buffer_rsrc_t rows = tile_rows<D>(src, row0, T);
+    // rows 0 .. 15 and 16 .. 31; opaque, so that the rows of a half are one register plus the instruction's offset
+    int lower = (4 * g * D + D / 32 * n) * 4, upper = lower + 16 * D * 4;
+    asm volatile("" : "+v"(lower), "+v"(upper));
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-        const int at = (4 * g * D + D / 32 * n) * 4, row = (8 * (i / 4) + i % 4) * D * 4;
+        const int at = i < 8 ? lower : upper, row = (8 * (i % 8 / 4) + i % 4) * D * 4;
         if constexpr (D == 64) {
-            const auto v = __builtin_amdgcn_raw_buffer_load_b64(rows, at + row % 4096, row / 4096 * 4096, 0);
+            const auto v = __builtin_amdgcn_raw_buffer_load_b64(rows, at + row, 0, 0);
             reg[2 * i] = __uint_as_float(v[0]);
             reg[2 * i + 1] = __uint_as_float(v[1]);
         } else {

@@ -1,7 +1,8 @@
 """Properties of the compiled device code that the sources rely on but the compiler does not check (CPU only: the
-kernels are cross-compiled to assembly, nothing runs).  The library's Makefile runs the same check on every build."""
+kernels are cross-compiled to assembly, nothing runs).  The library's Makefile runs the first check on every build."""
 import importlib.util
 import os
+import re
 import shutil
 import subprocess
 
@@ -18,17 +19,30 @@ def _checker():
     return mod.check
 
 
-@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not available")
-@pytest.mark.parametrize("unit", ["tdp_bwd_mfma.hip", "dps_mfma.hip"])
-def test_direct_lds_loads_own_m0(tmp_path, unit):
-    """The direct-to-LDS loads set M0 in inline assembly; nothing the compiler emits in those kernels may use M0, and
-    the LDS waits must stay counted (csrc/check_m0.py states the conditions)."""
+def _assembly(tmp_path, unit):
     out = tmp_path / "unit.s"
     flags = ["-O3", "-std=c++17", "--offload-arch=gfx950", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
              "-Wno-unused-command-line-argument", "--cuda-device-only", "-S"]
     subprocess.run([HIPCC, *flags, os.path.join(CSRC, unit), "-o", str(out)], check=True,
                    stderr=subprocess.DEVNULL, cwd=CSRC)
-    assert _checker()(out.read_text()) is None
+    return out.read_text()
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not available")
+@pytest.mark.parametrize("unit", ["tdp_bwd_mfma.hip", "dps_mfma.hip"])
+def test_direct_lds_loads_own_m0(tmp_path, unit):
+    """The direct-to-LDS loads set M0 in inline assembly; nothing the compiler emits in those kernels may use M0, and
+    the LDS waits must stay counted (csrc/check_m0.py states the conditions)."""
+    assert _checker()(_assembly(tmp_path, unit)) is None
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not available")
+def test_buffer_loads_keep_their_offset_in_the_range_check(tmp_path):
+    """The fp32 dot-product-sum kernels rely on buffer loads to return zeros for rows past the end of a head.  The range
+    check of a raw buffer leaves the scalar offset out, so that offset is zero in every one of them."""
+    loads = re.findall(r"^\s*buffer_load_dword\w*\s+(.*)$", _assembly(tmp_path, "dps_f32_mfma.hip"), re.M)
+    assert len(loads) > 100
+    assert [x for x in loads if not re.search(r"s\[\d+:\d+\], 0 offen\b", x)] == []
 
 
 def test_checker_rejects_foreign_users_of_m0():

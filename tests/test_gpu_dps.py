@@ -455,3 +455,53 @@ def test_backward_from_the_kept_inner_pass(dtype, D, T, causal, k_diff, fused, s
         assert torch.equal(a, b), name
         for got in (a.float().cpu(), c.float().cpu()):
             (util.assert_mostly_close if low else util.assert_close)(name, got, want, **(LOWP if low else FP32))
+
+
+def _behind_nan(t):
+    """`t` on the GPU as a dense tensor that NaN precedes and follows."""
+    guard = 1 << 14
+    whole = torch.full((t.numel() + 2 * guard,), float("nan"), dtype=t.dtype, device="cuda")
+    inside = whole[guard:guard + t.numel()].view(t.shape)
+    inside.copy_(t)
+    return inside
+
+
+@pytest.mark.parametrize("D", [32, 64])
+@pytest.mark.parametrize("T", [33, 40, 47, 49, 63])
+@pytest.mark.parametrize("keep", [False, True])
+def test_fp32_reads_nothing_past_the_last_row(T, D, keep):
+    """A ragged last tile is completed with zeros: with NaN behind every tensor and in all of the workspace, one such read
+    would show in the results, also where its weight is zero."""
+    from flash_trittention import _lib
+
+    lib, B, H, alpha = _lib.lib(), 1, 2, 1 / math.sqrt(D)
+    print(f"fp32 dot-product sum inside NaN: T={T} D={D} keep={keep}", flush=True)
+    inputs = orc.make_inputs(B, H, T, D, torch.float32, seed=T)
+    z, lse, grads = util.oracle_dps(inputs, alpha, True, T, factorised=True)
+    q, k1, k2, v1, v2, do = (_behind_nan(t) for t in inputs)
+    o, m = _behind_nan(torch.zeros(B, H, T, D)), _behind_nan(torch.zeros(B, H, T))
+    kept = [_behind_nan(torch.zeros(B, H, T, D)), _behind_nan(torch.zeros(B, H, (T + 31) // 32 * 32))] if keep else []
+    out = [_behind_nan(torch.zeros(B, H, T, D)) for _ in range(5)]
+    shape, stream = (B, H, T, D, _lib.TRITT_F32, alpha, 1, T), _lib.stream_ptr(q.device)
+    nan_bytes = lambda n: torch.full(((n + 3) // 4,), float("nan"), device="cuda")
+    ws = nan_bytes(lib.tritt_dps_fwd_workspace_bytes(B, H, T, D, _lib.TRITT_F32, 0))
+    tensors = [_lib.ptr(t) for t in (q, k1, k2, v1, v2)]
+    tail = (_lib.ptr(ws), 4 * ws.numel(), 0, stream)
+    if keep:
+        rc = lib.tritt_dps_fwd_keep(*tensors, None, _lib.ptr(o), _lib.ptr(m), *map(_lib.ptr, kept), *shape, *tail)
+    else:
+        rc = lib.tritt_dps_fwd(*tensors, _lib.ptr(o), _lib.ptr(m), *shape, *tail)
+    assert rc == 0, lib.tritt_status_string(rc)
+    wb = nan_bytes(lib.tritt_dps_bwd_workspace_bytes(B, H, T, D, _lib.TRITT_F32, 0))
+    tail, gp = (_lib.ptr(wb), 4 * wb.numel(), 0, stream), [_lib.ptr(t) for t in out]
+    if keep:
+        rc = lib.tritt_dps_bwd_kept(*tensors, None, _lib.ptr(o), _lib.ptr(m), *map(_lib.ptr, kept), _lib.ptr(do), None, *gp,
+                                    *shape, *tail)
+    else:
+        rc = lib.tritt_dps_bwd(*tensors, _lib.ptr(o), _lib.ptr(m), _lib.ptr(do), *gp, *shape, *tail)
+    assert rc == 0, lib.tritt_status_string(rc)
+    torch.cuda.synchronize()
+    util.assert_close("out", o.cpu(), z, **FP32)
+    util.assert_close("m", m.cpu(), lse, rtol=1e-5, atol=1e-4)
+    for name, a, b in zip(util.NAMES, out, grads):
+        util.assert_close(name, a.cpu(), b, **FP32)
