@@ -260,7 +260,7 @@ int tdp_bwd_generic(Arena& ar, bool run, const void* q, const void* k1, const vo
     a.BH = B * H; a.T = T; a.D = D; a.alpha = alpha;
     a.causal = causal; a.k1_window = w1; a.k2_window = w2; a.kk_left = kl; a.kk_right = kr;
     if (dtype != TRITT_F32) plan_f32_parts(ar, a);  // (o32 is null while measuring)
-    long long* fixed = mfma32 ? ar.take<long long>(f32_mfma_tdp_bwd_scratch_elems(B * H, T, D)) : nullptr;
+    long long* fixed = mfma32 ? ar.take<long long>(f32_mfma_tdp_bwd_scratch_elems(a)) : nullptr;
     // VALU kernels: fp32 results, the caller's tensors when they are fp32, scratch otherwise; `spare` stands in for the
     // unwanted (null) half of a gradient pair whose other half is wanted (one kernel writes both halves)
     float *dq32 = (float*)dq, *dk132 = (float*)dk1, *dk232 = (float*)dk2, *dv232 = (float*)dv2;

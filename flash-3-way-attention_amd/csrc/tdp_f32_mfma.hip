@@ -7,8 +7,8 @@
 // Formulation (the same virtual-query one as the 16-bit kernels).  A workgroup owns 32 consecutive queries;
 // its waves take consecutive rows b per round (one per wave; b = k, the K2 / V2 row, in the natural orientation) and
 // sweep the streamed index a (= j, K1 / U rows) in 32-row stages shared through LDS.  The rounds of a tile are dealt out
-// over several workgroups by their cost (F32Deal): the forward's parts are joined by f32_merge_kernel, the backward's
-// meet in fixed-point accumulators.
+// over several workgroups by their cost (F32Deal): the forward's parts are joined by f32_merge_kernel and dQ's by
+// f32_finish_kernel; the row gradients, sums over query tiles, meet in fixed-point accumulators.
 // For a fixed row b the scores of the 32 queries against 32 streamed rows are one 32x32 tile
 //   S^T[a, q] = sum_d KA[a, d] * (scale * Q[q, d] * KB[b, d])
 // i.e. D / 2 MFMAs (K = 2 each).  The tile leaves the MFMA with lane <-> query and registers <-> streamed rows,
@@ -62,7 +62,7 @@ __global__ __launch_bounds__(256) void f32_prep_kernel(const float* __restrict__
             dot = x[0] * y[0] + x[1] * y[1] + (x[2] * y[2] + x[3] * y[3]);
             const longlong2 z = make_longlong2(0, 0);
 #pragma unroll
-            for (int t = 0; t < 5; ++t) {
+            for (int t = 0; t < 4; ++t) {
                 longlong2* p = reinterpret_cast<longlong2*>(acc + t * n + off);
                 p[0] = z;
                 p[1] = z;
@@ -73,13 +73,18 @@ __global__ __launch_bounds__(256) void f32_prep_kernel(const float* __restrict__
         if (idx % kPieces == 0 && j < T) delta[(size_t)bh * T + j] = dot;
     }
 }
-// fixed point -> the gradients (null: not wanted); dV1 = dU SiLU'(V1), dQ = alpha times its sum.  Four elements per thread.
+// The sums -> the gradients (null: not wanted), four elements per thread: dK2, dV2, dK1 and dV1 = dU SiLU'(V1) from fixed
+// point, dQ = alpha times the sum of its tile's parts.  dQ's sum belongs to one tile, so its parts are joined in fp32 and in
+// order: a gradient may lie many powers of two below what the scale of a fixed-point sum is set by (operands of 0.01, T = 128:
+// dQ in steps of 2^-36 max |dO| is 6e-3 off, so joined 1e-6).  Costs what the accumulator did (training steps, accumulator ->
+// parts: B=2 H=4 T=500 D=64 4.32 -> 4.32 ms, B=4 H=8 T=128 522 -> 525 us, B=1 H=2 T=64 D=32 53.0 -> 53.5 us).
 template <typename E>
 __global__ __launch_bounds__(256) void f32_finish_kernel(const long long* __restrict__ acc, const E* __restrict__ v1,
                                                          E* __restrict__ dq, E* __restrict__ dk1, E* __restrict__ dk2,
                                                          E* __restrict__ dv1, E* __restrict__ dv2, size_t n, int T, int D,
                                                          const unsigned* __restrict__ scale_parts,
-                                                         const unsigned* __restrict__ poison, float alpha) {
+                                                         const unsigned* __restrict__ poison, float alpha,
+                                                         const float* __restrict__ part_q, F32Deal deal, TdpMask mask, int nw) {
     typedef __attribute__((ext_vector_type(4))) E e4;
     for (size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4; i < n; i += (size_t)gridDim.x * 1024) {
         const size_t row = i / D;
@@ -104,7 +109,17 @@ __global__ __launch_bounds__(256) void f32_finish_kernel(const long long* __rest
             const e4 x = *reinterpret_cast<const e4*>(v1 + i);
             put(dv1, 3, kPoisonDU, [&](int e) { return silu_grad_f((float)x[e]); });
         }
-        put(dq, 4, kPoisonDQ, [&](int) { return alpha; });
+        if (dq) {
+            const float* src = part_q + row * deal.max_parts * D + i % D;
+            const int parts = f32_tile_parts(deal, mask, (int)(row % T) / 32, T, nw);
+            f32x4v sum = *reinterpret_cast<const f32x4v*>(src);
+#pragma unroll 4
+            for (int s = 1; s < parts; ++s) sum += *reinterpret_cast<const f32x4v*>(src + s * D);
+            e4 r;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) r[e] = (E)(sum[e] * alpha);
+            *reinterpret_cast<e4*>(dq + i) = r;
+        }
     }
 }
 
@@ -186,7 +201,7 @@ hipError_t launch_f32_bwd_tiles(F32BwdParams<E> p, const E* k1, const E* u, cons
     constexpr size_t smem = f32_bwd_smem<D, NW>();
     if (hipError_t e = ensure_dynamic_smem(reinterpret_cast<const void*>(kern_dq), smem); e != hipSuccess) return e;
     if (hipError_t e = ensure_dynamic_smem(reinterpret_cast<const void*>(kern_nodq), smem); e != hipSuccess) return e;
-    // The rounds of a tile are dealt out to several workgroups (the launch with dQ: only when dQ has an accumulator).  The list
+    // The rounds of a tile are dealt out to several workgroups (the launch with dQ: only when dQ's shares have a place).  The list
     // of parts belongs to the mask it was made for, and the second launch exchanges the two key indices.
     const TdpMask exchanged{natural.causal, natural.wb, natural.wa, natural.rab, natural.lab};
     const F32Deal whole{0.f, 1, p.nqt};
@@ -197,7 +212,7 @@ hipError_t launch_f32_bwd_tiles(F32BwdParams<E> p, const E* k1, const E* u, cons
     place_inputs(p, at, false);
     p.acc_k = acc_k2; p.acc_v = acc_v2; p.bit_k = kPoisonDK2; p.bit_v = kPoisonDV2;
     p.mask = natural;
-    p.deal = want_q && !p.acc_q ? whole : deal_for(natural);
+    p.deal = want_q && !p.part_q && !p.acc_q ? whole : deal_for(natural);
     if (want_q) hipLaunchKernelGGL(kern_dq, grid_of(p.deal), dim3(64 * NW), smem, st, p);
     else if (want_k2) hipLaunchKernelGGL(kern_nodq, grid_of(p.deal), dim3(64 * NW), smem, st, p);
     // rows = (K1, U), streamed = (K2, V2): dK1, dU (the mask with the two key indices exchanged)
@@ -215,19 +230,23 @@ hipError_t launch_f32_bwd(const F32BwdCall& c, hipStream_t st) {
     const GenericTdpArgs& a = c.a;
     const size_t n = (size_t)a.BH * a.T * D, rows = (size_t)a.BH * a.T;
     const bool want_q = c.dq != nullptr, want_k2 = c.dk2 || c.dv2, want_k1 = c.dk1 || c.dv1;
-    // scratch: the accumulators of dK2, dV2, dK1, dU and dQ, the rows' poison words, the slices' scale partials
+    const TdpMask natural{a.causal, a.k1_window, a.k2_window, a.kk_left, a.kk_right};
+    const F32Deal deal_q = f32_bwd_deal(a.BH, a.T, D, natural);
+    // scratch: the accumulators of dK2, dV2, dK1 and dU, the rows' poison words, the slices' scale partials, dQ's parts
     long long* acc = c.scratch;
-    unsigned* poison = reinterpret_cast<unsigned*>(acc + 5 * n);
-    unsigned* parts = reinterpret_cast<unsigned*>(acc + 5 * n + (rows + 3) / 4 * 2);  // 16-byte aligned
+    unsigned* poison = reinterpret_cast<unsigned*>(acc + 4 * n);
+    unsigned* parts = reinterpret_cast<unsigned*>(acc + 4 * n + (rows + 3) / 4 * 2);  // 16-byte aligned
+    float* part_q = reinterpret_cast<float*>(parts + (size_t)a.BH * kScaleParts);
+    // a dQ of one part per tile needs no place of its own where the kernel can write the caller's type
+    const bool direct_q = c.elem == 0 && deal_q.max_parts == 1;
     hipLaunchKernelGGL(f32_prep_kernel<D>, dim3((a.T + 63) / 64, a.BH), dim3(256), 0, st, c.v1_f32, c.v1_f32 ? c.u_out : nullptr,
                        c.o, a.d_o, c.delta, acc, n, parts, poison, a.T);
     F32BwdParams<float> p{};
     p.q = a.q; p.d_o = a.d_o; p.lse = a.lse_in; p.delta = c.delta;
-    p.dq = nullptr; p.acc_q = acc + 4 * n; p.acc_q_rows = 0; p.stats_part = nullptr; p.split_rounds = 0;
+    p.dq = direct_q ? (float*)c.dq : nullptr; p.part_q = direct_q ? nullptr : part_q; p.acc_q = nullptr; p.acc_q_rows = 0; p.stats_part = nullptr; p.split_rounds = 0;
     p.scale_parts = parts; p.poison = poison; p.scale_bias = kF32FixedBias;
     p.T = a.T; p.BH = a.BH; p.nqt = (a.T + 31) / 32;
     p.alpha = a.alpha;
-    const TdpMask natural{a.causal, a.k1_window, a.k2_window, a.kk_left, a.kk_right};
     if (hipError_t e = launch_f32_bwd_tiles<float, D>(p, a.k1, a.u, a.k2, a.v2, acc, acc + n, acc + 2 * n, acc + 3 * n,
                                                       natural, want_q, want_k2, want_k1, st, dense_inputs(a.T, D), true);
         e != hipSuccess)
@@ -235,8 +254,9 @@ hipError_t launch_f32_bwd(const F32BwdCall& c, hipStream_t st) {
     const dim3 grid((unsigned)std::min<size_t>((n / 4 + 255) / 256, 8192));
     auto finish = [&](auto zero) {
         using E = decltype(zero);
-        hipLaunchKernelGGL(f32_finish_kernel<E>, grid, dim3(256), 0, st, acc, (const E*)c.v1, (E*)c.dq, (E*)c.dk1, (E*)c.dk2,
-                           (E*)c.dv1, (E*)c.dv2, n, a.T, D, parts, poison, a.alpha);
+        hipLaunchKernelGGL(f32_finish_kernel<E>, grid, dim3(256), 0, st, acc, (const E*)c.v1, direct_q ? nullptr : (E*)c.dq,
+                           (E*)c.dk1, (E*)c.dk2, (E*)c.dv1, (E*)c.dv2, n, a.T, D, parts, poison, a.alpha, part_q, deal_q,
+                           natural, f32_bwd_waves(D));
     };
     if (c.elem == 0) finish(0.f);
     else if (c.elem == 1) finish((__bf16)0.f);
@@ -359,9 +379,10 @@ hipError_t f32_mfma_tdp_fwd(const GenericTdpArgs& a, hipStream_t st) {
     return hipErrorInvalidValue;
 }
 
-size_t f32_mfma_tdp_bwd_scratch_elems(int BH, int T, int D) {
-    return 5 * (size_t)BH * T * D + ((size_t)BH * T + 3) / 4 * 2 +
-           (size_t)BH * kScaleParts / 2;
+size_t f32_mfma_tdp_bwd_scratch_elems(const GenericTdpArgs& a) {
+    const size_t rows = (size_t)a.BH * a.T;
+    const int parts_q = f32_bwd_deal(a.BH, a.T, a.D, TdpMask{a.causal, a.k1_window, a.k2_window, a.kk_left, a.kk_right}).max_parts;
+    return 4 * rows * a.D + (rows + 3) / 4 * 2 + (size_t)a.BH * kScaleParts / 2 + rows * a.D * parts_q / 2;
 }
 
 hipError_t f32_mfma_tdp_bwd(const F32BwdCall& c, hipStream_t st) {

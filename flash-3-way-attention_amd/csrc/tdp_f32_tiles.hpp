@@ -558,13 +558,15 @@ struct F32BwdParams {
     const float *lse, *delta;
     E* dq;                 // WITH_DQ, when acc_q is null
     void *acc_k, *acc_v;   // [BH][T][D] gradients of the rows: fixed point (long long) or float
-    void* acc_q;           // WITH_DQ: when non-null, dQ / alpha is added here instead of being written to dq
+    // WITH_DQ: when non-null, this workgroup's share of dQ / alpha is left in part_q[((bh T + q) max_parts + part) D]
+    float* part_q;
+    void* acc_q;           // WITH_DQ: else, when non-null, dQ / alpha is added here instead of being written to dq
     int acc_q_rows;        // 0: acc_q is [BH][T][D]; else it holds the first acc_q_rows queries only, [BH][rows][D]
     // when non-null, LSE and Delta of query tile 0 come from the partials the split STATS launch left here
     const float* stats_part;
     int split_rounds;      // tile 0 only: rounds dealt out to workgroups (see tdp_f32_tile0_kernel), else 0
-    // tdp_f32_bwd_kernel: the rounds of a tile dealt out to f32_tile_parts() workgroups.  max_parts above one needs acc_q
-    // where dQ is produced (each workgroup holds a share of it)
+    // tdp_f32_bwd_kernel: the rounds of a tile dealt out to f32_tile_parts() workgroups.  max_parts above one needs part_q
+    // or acc_q where dQ is produced (each workgroup holds a share of it)
     F32Deal deal;
     // fixed-point accumulators (common.hpp); scale_parts null: the accumulators are float
     const unsigned* scale_parts;
@@ -918,7 +920,9 @@ __device__ __forceinline__ void f32_bwd_body(const F32BwdParams<E>& p, int only_
             const int r = idx / DOUT, d = idx % DOUT;
             if (q0 + r < T) {
                 const size_t off = base + (size_t)(q0 + r) * D + c0 + d;
-                if (p.acc_q)
+                if (p.part_q)
+                    p.part_q[(((size_t)bh * T + q0 + r) * p.deal.max_parts + part) * D + c0 + d] = merged(d, r);
+                else if (p.acc_q)
                     shared_add(p.acc_q, p.acc_q_rows ? ((size_t)bh * p.acc_q_rows + q0 + r) * D + c0 + d : off,
                                merged(d, r), fscale, p.poison + (size_t)bh * T + q0 + r, kPoisonDQ);
                 else

@@ -1082,3 +1082,45 @@ def test_non_finite_dO_gives_non_finite_gradients(dtype, bad):
         a = a.clone()
         a[1, 2] = b[1, 2]
         assert torch.equal(a, b), f"{name}: another head changed"
+
+
+# ---- fp32 gradients hold their precision whatever the operands' size: dQ and dK shrink with the fourth power of the
+# operands while dO stays, so an accumulator with a step of its own, relative to dO, loses them.
+
+def _gradients_in_64_bits(inputs, alpha, heads, **windows):
+    out = []
+    for b, h in heads:
+        _, _, grads = orc.tdp_forward_backward_chunked(*(t[b, h].double() for t in inputs), alpha, True, **windows)
+        out.append(grads)
+    return out
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("c", [0.05, 0.02, 0.01])
+@pytest.mark.parametrize("splits", [0, 1])
+def test_fp32_dq_of_small_operands(D, c, splits, tune):
+    """128 query tiles and operands of size c: dQ against 64 bits, its tile dealt out to workgroups and in one.  Bar: a
+    rounding of 2^-24 in each of the D + 3 sums and products behind an element, and sqrt(T) of them in its sum (8.8e-5 at
+    D = 128)."""
+    print(f"case small operands, dQ: D={D} c={c} splits={splits}", flush=True)
+    tune(_lib.TUNE_BWD_SPLITS, splits)
+    B, H, T = 4, 8, 128
+    inputs = orc.make_inputs(B, H, T, D, torch.float32, seed=D)
+    inputs = [t * c for t in inputs[:5]] + [inputs[5]]
+    heads = [(0, 0), (1, 5), (3, 7)]
+    _, g = util.run_tdp(inputs, 1 / math.sqrt(D), True)
+    for (b, h), want in zip(heads, _gradients_in_64_bits(inputs, 1 / math.sqrt(D), heads)):
+        err = (g[0][b, h].double() - want[0]).norm() / want[0].norm()
+        print(f"    dq[{b}, {h}]: {err:.2e}", flush=True)
+        assert err <= 2.0 ** -24 * (D + 3) * math.sqrt(T), (b, h, err.item())
+
+
+def test_fp32_dq_beyond_the_range_of_dO():
+    """dQ far above |dO| (large keys and values) is finite: nothing bounds it by a multiple of max |dO|."""
+    inputs = orc.make_inputs(4, 8, 128, 64, torch.float32, seed=9)
+    inputs = [inputs[0] * 1e-6] + [t * 1e3 for t in inputs[1:5]] + [inputs[5] * 1e-4]
+    want = _gradients_in_64_bits(inputs, 1e-3, [(2, 3)])[0]
+    assert want[0].abs().max() > 2.0 ** 27 * inputs[5].abs().max()
+    _, g = util.run_tdp(inputs, 1e-3, True)
+    assert torch.isfinite(g[0]).all()
+    assert util.rel_err(g[0][2, 3].double(), want[0]) <= 1e-4
