@@ -8,7 +8,8 @@
 // its waves take consecutive rows b per round (one per wave; b = k, the K2 / V2 row, in the natural orientation) and
 // sweep the streamed index a (= j, K1 / U rows) in 32-row stages shared through LDS.  The rounds of a tile are dealt out
 // over several workgroups by their cost (F32Deal): the forward's parts are joined by f32_merge_kernel and dQ's by
-// f32_finish_kernel; the row gradients, sums over query tiles, meet in fixed-point accumulators.
+// f32_finish_kernel; the row gradients, sums over query tiles, meet in fixed-point accumulators, or are left by each tile of
+// a problem of a few tiles and joined like dQ (f32_tile_slabs).
 // For a fixed row b the scores of the 32 queries against 32 streamed rows are one 32x32 tile
 //   S^T[a, q] = sum_d KA[a, d] * (scale * Q[q, d] * KB[b, d])
 // i.e. D / 2 MFMAs (K = 2 each).  The tile leaves the MFMA with lane <-> query and registers <-> streamed rows,
@@ -28,20 +29,21 @@ namespace tritt {
 namespace {
 
 // One pass ahead of the backward kernels, 64 rows per workgroup: U = SiLU(V1) (u null: the caller has it), Delta =
-// rowsum(dO * O), the partial maxima of |dO| that fix the scale of a slice's accumulators, and the accumulators and poison
-// words cleared.  Five launches of 2-5 us each without it; grid (64-row blocks, BH).
+// rowsum(dO * O), the accumulators cleared (`planes` times n words) and, for fixed-point ones (scale_parts not null), the
+// partial maxima of |dO| that fix a slice's scale and the poison words cleared.  Five launches of 2-5 us each without it;
+// grid (64-row blocks, BH).
 template <int D>
 __global__ __launch_bounds__(256) void f32_prep_kernel(const float* __restrict__ v1, float* __restrict__ u,
                                                        const float* __restrict__ o, const float* __restrict__ d_o,
-                                                       float* __restrict__ delta, long long* __restrict__ acc, size_t n,
+                                                       float* __restrict__ delta, unsigned* __restrict__ acc, int planes, size_t n,
                                                        unsigned* __restrict__ scale_parts, unsigned* __restrict__ poison, int T) {
     __shared__ unsigned red[4];
     constexpr int kPieces = D / 4;
     const int bh = blockIdx.y, j0 = blockIdx.x * 64;
     const size_t base = (size_t)bh * T * D;
-    if (threadIdx.x < 64 && j0 + threadIdx.x < T) poison[(size_t)bh * T + j0 + threadIdx.x] = 0;
+    if (scale_parts && threadIdx.x < 64 && j0 + threadIdx.x < T) poison[(size_t)bh * T + j0 + threadIdx.x] = 0;
     // part s of a slice: its 64-row blocks s, s + kScaleParts, ...
-    for (int part = blockIdx.x; part < kScaleParts; part += gridDim.x) {
+    for (int part = blockIdx.x; scale_parts && part < kScaleParts; part += gridDim.x) {
         unsigned m = 0;
         for (int r0 = part * 64; r0 < T; r0 += kScaleParts * 64)
             m = max(m, block_absmax_bits<float>(d_o + base + (size_t)r0 * D, (size_t)min(64, T - r0) * kPieces, red));
@@ -60,13 +62,7 @@ __global__ __launch_bounds__(256) void f32_prep_kernel(const float* __restrict__
             }
             const f32x4v x = *reinterpret_cast<const f32x4v*>(o + off), y = *reinterpret_cast<const f32x4v*>(d_o + off);
             dot = x[0] * y[0] + x[1] * y[1] + (x[2] * y[2] + x[3] * y[3]);
-            const longlong2 z = make_longlong2(0, 0);
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                longlong2* p = reinterpret_cast<longlong2*>(acc + t * n + off);
-                p[0] = z;
-                p[1] = z;
-            }
+            for (int t = 0; t < planes; ++t) *reinterpret_cast<uint4*>(acc + t * n + off) = make_uint4(0u, 0u, 0u, 0u);
         }
 #pragma unroll
         for (int w = kPieces / 2; w > 0; w >>= 1) dot += __shfl_xor(dot, w, 64);
@@ -74,7 +70,7 @@ __global__ __launch_bounds__(256) void f32_prep_kernel(const float* __restrict__
     }
 }
 // The sums -> the gradients (null: not wanted), four elements per thread: dK2, dV2, dK1 and dV1 = dU SiLU'(V1) from fixed
-// point, dQ = alpha times the sum of its tile's parts.  dQ's sum belongs to one tile, so its parts are joined in fp32 and in
+// point (`slabs` > 0: from that many tiles' fp32 shares, in order), dQ = alpha times the sum of its tile's parts.  dQ's sum belongs to one tile, so its parts are joined in fp32 and in
 // order: a gradient may lie many powers of two below what the scale of a fixed-point sum is set by (operands of 0.01, T = 128:
 // dQ in steps of 2^-36 max |dO| is 6e-3 off, so joined 1e-6).  Costs what the accumulator did (training steps, accumulator ->
 // parts: B=2 H=4 T=500 D=64 4.32 -> 4.32 ms, B=4 H=8 T=128 522 -> 525 us, B=1 H=2 T=64 D=32 53.0 -> 53.5 us).
@@ -84,14 +80,25 @@ __global__ __launch_bounds__(256) void f32_finish_kernel(const long long* __rest
                                                          E* __restrict__ dv1, E* __restrict__ dv2, size_t n, int T, int D,
                                                          const unsigned* __restrict__ scale_parts,
                                                          const unsigned* __restrict__ poison, float alpha,
-                                                         const float* __restrict__ part_q, F32Deal deal, TdpMask mask, int nw) {
+                                                         const float* __restrict__ part_q, F32Deal deal, TdpMask mask, int nw,
+                                                         int slabs) {
     typedef __attribute__((ext_vector_type(4))) E e4;
     for (size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4; i < n; i += (size_t)gridDim.x * 1024) {
         const size_t row = i / D;
-        const double inv = fixed_scale_inverse(fixed_scale_field<false>(scale_parts, (int)(row / T), kF32FixedBias));
-        const unsigned bad = poison[row];
+        const double inv = slabs ? 0. : fixed_scale_inverse(fixed_scale_field<false>(scale_parts, (int)(row / T), kF32FixedBias));
+        const unsigned bad = slabs ? 0u : poison[row];
         auto put = [&](E* out, int which, unsigned bit, auto factor) {
             if (!out) return;
+            if (slabs) {
+                const float* src = reinterpret_cast<const float*>(acc) + (size_t)which * slabs * n + i;
+                f32x4v sum = *reinterpret_cast<const f32x4v*>(src);
+                for (int t = 1; t < slabs; ++t) sum += *reinterpret_cast<const f32x4v*>(src + t * n);
+                e4 r;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) r[e] = (E)(sum[e] * factor(e));
+                *reinterpret_cast<e4*>(out + i) = r;
+                return;
+            }
             const longlong2* p = reinterpret_cast<const longlong2*>(acc + which * n + i);
             const longlong2 lo = p[0], hi = p[1];
             const long long v[4] = {lo.x, lo.y, hi.x, hi.y};
@@ -188,6 +195,13 @@ F32Deal f32_bwd_deal(int BH, int T, int D, const TdpMask& mask) {
     return f32_deal(mask, BH, T, nw, nw == 4 ? 512 : 256, knobs().bwd_splits > 0 ? std::min(knobs().bwd_splits, 16) : 16);
 }
 
+// Problems of less than eight query tiles: every tile has row-gradient accumulators of its own, fp32, where each element gets
+// one share (a row belongs to one round, a round to one workgroup), and f32_finish_kernel adds the tiles'.  Nothing then has a
+// step or a range of its own: in steps of 2^-36 max |dO| operands of 0.02 left dK1 2.5e-3 off (T = 64, D = 32), shares of fp32
+// 4e-7 or less.  At most seven tiles' words, of at most 224 rows each.  Kernel time of a training step, fixed point -> this:
+// B=1 H=2 T=64 D=32 50.0 -> 49.1 us, B=1 H=2 T=100 D=64 157.7 -> 160.2 (the last launch adds four tiles' words).
+bool f32_tile_slabs(int BH, int T) { return (long long)BH * ((T + 31) / 32) < 8; }
+
 // both launches of the backward over query tiles 0 .. nqt - 1
 template <typename E, int D>
 hipError_t launch_f32_bwd_tiles(F32BwdParams<E> p, const E* k1, const E* u, const E* k2, const E* v2, void* acc_k2,
@@ -232,22 +246,27 @@ hipError_t launch_f32_bwd(const F32BwdCall& c, hipStream_t st) {
     const bool want_q = c.dq != nullptr, want_k2 = c.dk2 || c.dv2, want_k1 = c.dk1 || c.dv1;
     const TdpMask natural{a.causal, a.k1_window, a.k2_window, a.kk_left, a.kk_right};
     const F32Deal deal_q = f32_bwd_deal(a.BH, a.T, D, natural);
-    // scratch: the accumulators of dK2, dV2, dK1 and dU, the rows' poison words, the slices' scale partials, dQ's parts
+    // scratch: the accumulators of dK2, dV2, dK1 and dU, with fixed-point ones the rows' poison words and the slices' scale
+    // partials, and dQ's parts
+    const int slabs = f32_tile_slabs(a.BH, a.T) ? (a.T + 31) / 32 : 0;
     long long* acc = c.scratch;
-    unsigned* poison = reinterpret_cast<unsigned*>(acc + 4 * n);
-    unsigned* parts = reinterpret_cast<unsigned*>(acc + 4 * n + (rows + 3) / 4 * 2);  // 16-byte aligned
-    float* part_q = reinterpret_cast<float*>(parts + (size_t)a.BH * kScaleParts);
+    float* share = reinterpret_cast<float*>(acc);
+    unsigned* poison = slabs ? nullptr : reinterpret_cast<unsigned*>(acc + 4 * n);
+    unsigned* parts = slabs ? nullptr : reinterpret_cast<unsigned*>(acc + 4 * n + (rows + 3) / 4 * 2);  // 16-byte aligned
+    float* part_q = slabs ? share + 4 * slabs * n : reinterpret_cast<float*>(parts + (size_t)a.BH * kScaleParts);
     // a dQ of one part per tile needs no place of its own where the kernel can write the caller's type
     const bool direct_q = c.elem == 0 && deal_q.max_parts == 1;
     hipLaunchKernelGGL(f32_prep_kernel<D>, dim3((a.T + 63) / 64, a.BH), dim3(256), 0, st, c.v1_f32, c.v1_f32 ? c.u_out : nullptr,
-                       c.o, a.d_o, c.delta, acc, n, parts, poison, a.T);
+                       c.o, a.d_o, c.delta, reinterpret_cast<unsigned*>(acc), slabs ? 4 * slabs : 8, n, parts, poison, a.T);
     F32BwdParams<float> p{};
     p.q = a.q; p.d_o = a.d_o; p.lse = a.lse_in; p.delta = c.delta;
     p.dq = direct_q ? (float*)c.dq : nullptr; p.part_q = direct_q ? nullptr : part_q; p.acc_q = nullptr; p.acc_q_rows = 0; p.stats_part = nullptr; p.split_rounds = 0;
     p.scale_parts = parts; p.poison = poison; p.scale_bias = kF32FixedBias;
     p.T = a.T; p.BH = a.BH; p.nqt = (a.T + 31) / 32;
     p.alpha = a.alpha;
-    if (hipError_t e = launch_f32_bwd_tiles<float, D>(p, a.k1, a.u, a.k2, a.v2, acc, acc + n, acc + 2 * n, acc + 3 * n,
+    p.acc_tile = slabs ? n : 0;
+    auto acc_of = [&](int which) { return slabs ? (void*)(share + which * slabs * n) : (void*)(acc + which * n); };
+    if (hipError_t e = launch_f32_bwd_tiles<float, D>(p, a.k1, a.u, a.k2, a.v2, acc_of(0), acc_of(1), acc_of(2), acc_of(3),
                                                       natural, want_q, want_k2, want_k1, st, dense_inputs(a.T, D), true);
         e != hipSuccess)
         return e;
@@ -256,7 +275,7 @@ hipError_t launch_f32_bwd(const F32BwdCall& c, hipStream_t st) {
         using E = decltype(zero);
         hipLaunchKernelGGL(f32_finish_kernel<E>, grid, dim3(256), 0, st, acc, (const E*)c.v1, direct_q ? nullptr : (E*)c.dq,
                            (E*)c.dk1, (E*)c.dk2, (E*)c.dv1, (E*)c.dv2, n, a.T, D, parts, poison, a.alpha, part_q, deal_q,
-                           natural, f32_bwd_waves(D));
+                           natural, f32_bwd_waves(D), slabs);
     };
     if (c.elem == 0) finish(0.f);
     else if (c.elem == 1) finish((__bf16)0.f);
@@ -382,7 +401,10 @@ hipError_t f32_mfma_tdp_fwd(const GenericTdpArgs& a, hipStream_t st) {
 size_t f32_mfma_tdp_bwd_scratch_elems(const GenericTdpArgs& a) {
     const size_t rows = (size_t)a.BH * a.T;
     const int parts_q = f32_bwd_deal(a.BH, a.T, a.D, TdpMask{a.causal, a.k1_window, a.k2_window, a.kk_left, a.kk_right}).max_parts;
-    return 4 * rows * a.D + (rows + 3) / 4 * 2 + (size_t)a.BH * kScaleParts / 2 + rows * a.D * parts_q / 2;
+    const size_t fixed = 4 * rows * a.D + (rows + 3) / 4 * 2 + (size_t)a.BH * kScaleParts / 2;
+    // (one or two tiles' own accumulators are smaller than the fixed-point ones: the size stays monotone in T)
+    const size_t sums = f32_tile_slabs(a.BH, a.T) ? std::max(fixed, 2 * ((a.T + 31) / 32) * rows * a.D) : fixed;
+    return sums + rows * a.D * parts_q / 2;
 }
 
 hipError_t f32_mfma_tdp_bwd(const F32BwdCall& c, hipStream_t st) {

@@ -558,6 +558,7 @@ struct F32BwdParams {
     const float *lse, *delta;
     E* dq;                 // WITH_DQ, when acc_q is null
     void *acc_k, *acc_v;   // [BH][T][D] gradients of the rows: fixed point (long long) or float
+    size_t acc_tile;       // elements from one query tile's acc_k, acc_v to the next one's (0: all tiles add to the same)
     // WITH_DQ: when non-null, this workgroup's share of dQ / alpha is left in part_q[((bh T + q) max_parts + part) D]
     float* part_q;
     void* acc_q;           // WITH_DQ: else, when non-null, dQ / alpha is added here instead of being written to dq
@@ -855,7 +856,7 @@ __device__ __forceinline__ void f32_bwd_body(const F32BwdParams<E>& p, int only_
                     const float sum = half_sum_16x2(xk, xv);
                     const bool odd = n & 1;
                     const int i = half_sum_register(), d = c0 + DTO * c_row(g, i) + dt;
-                    shared_add(odd ? p.acc_v : p.acc_k, base + (size_t)b * D + d, odd ? sum : sum * kLn2, fscale,
+                    shared_add(odd ? p.acc_v : p.acc_k, (size_t)qt * p.acc_tile + base + (size_t)b * D + d, odd ? sum : sum * kLn2, fscale,
                                p.poison + (size_t)bh * T + b, odd ? p.bit_v : p.bit_k);
                     __builtin_amdgcn_sched_barrier(0);  // one tile's products and sums in registers at a time
                 }

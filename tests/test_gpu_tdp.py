@@ -1124,3 +1124,36 @@ def test_fp32_dq_beyond_the_range_of_dO():
     _, g = util.run_tdp(inputs, 1e-3, True)
     assert torch.isfinite(g[0]).all()
     assert util.rel_err(g[0][2, 3].double(), want[0]) <= 1e-4
+
+
+@pytest.mark.parametrize("B,H,T,D", [(1, 2, 64, 32), (1, 1, 200, 64), (1, 3, 61, 128), (7, 1, 32, 64), (1, 1, 5, 32)])
+@pytest.mark.parametrize("splits", [0, 1])
+@pytest.mark.parametrize("case", ["operands 0.05", "operands 0.01", "rows of dO over 1e6", "windows"])
+def test_fp32_gradients_of_a_few_tiles_are_fp32_throughout(B, H, T, D, splits, case, tune):
+    """Less than eight query tiles: all five gradients against 64 bits with small operands, and row by row where dO falls by
+    1e6 along the sequence and late rows see small incoming gradients only.  Bar as above; a row of dQ, and of what only
+    late queries add to, is held to the fp32 bar by itself."""
+    print(f"case few tiles: {B} {H} {T} {D} splits={splits} {case}", flush=True)
+    tune(_lib.TUNE_BWD_SPLITS, splits)
+    inputs = orc.make_inputs(B, H, T, D, torch.float32, seed=T + D)
+    windows = {}
+    if case.startswith("operands"):
+        inputs = [t * float(case.split()[1]) for t in inputs[:5]] + [inputs[5]]
+    elif case.startswith("rows"):
+        inputs[5] = inputs[5] * torch.logspace(0, -6, T).view(1, 1, T, 1)
+    else:
+        windows = dict(k1_window=20, k2_window=41, kk_left=3, kk_right=30)
+        inputs = [t * 0.02 for t in inputs[:5]] + [inputs[5]]
+    heads = [(0, 0), (B - 1, H - 1)]
+    alpha = 1 / math.sqrt(D)
+    order = [windows.get(k) for k in ("k1_window", "k2_window", "kk_left", "kk_right")]
+    _, g = util.run_tdp(inputs, alpha, True, order)
+    for (b, h), want in zip(heads, _gradients_in_64_bits(inputs, alpha, heads, **windows)):
+        for name, a, r in zip(util.NAMES, g, want):
+            a = a[b, h].double()
+            err = ((a - r).norm() / r.norm()).item()
+            rows = ((a - r).norm(dim=-1) / r.norm(dim=-1))[1:].max().item()  # row 0 of dQ, dK1, dK2 may be exactly zero
+            print(f"    {name}[{b}, {h}]: {err:.2e}, worst row {rows:.2e}", flush=True)
+            # (in the norm the rounding of dP - Delta of the first, largest rows counts, whose own gradients are nearly zero)
+            assert case.startswith("rows") or err <= 2.0 ** -24 * (D + 3) * math.sqrt(T), (name, b, h, err)
+            assert rows <= 1e-4, (name, b, h, rows)
