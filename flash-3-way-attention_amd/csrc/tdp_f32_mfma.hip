@@ -19,6 +19,7 @@
 // finished row b into the output, O^T[d, q] += Tv^T[d, q] * VB[b, d]) is lane-local.
 // One loop body serves every mask; only tiles on its edge evaluate it.
 #include <algorithm>
+#include <cmath>
 
 #include "common.hpp"
 #include "kernels.hpp"
@@ -29,26 +30,34 @@ namespace tritt {
 namespace {
 
 // One pass ahead of the backward kernels, 64 rows per workgroup: U = SiLU(V1) (u null: the caller has it), Delta =
-// rowsum(dO * O), the accumulators cleared (`planes` times n words) and, for fixed-point ones (scale_parts not null), the
-// partial maxima of |dO| that fix a slice's scale and the poison words cleared.  Five launches of 2-5 us each without it;
-// grid (64-row blocks, BH).
+// rowsum(dO * O), the accumulators cleared (`planes` times n words) and, for fixed-point ones (maxima not null), the
+// partial maxima that fix a slice's scales (F32RowScale; V1's are U's where the caller has that) and the poison words cleared.
+// Five launches of 2-5 us each without it; grid (64-row blocks, BH, 1 + the maxima's tensors: one of them after the other
+// in the blocks of z = 0 is 6 us longer).
 template <int D>
-__global__ __launch_bounds__(256) void f32_prep_kernel(const float* __restrict__ v1, float* __restrict__ u,
+__global__ __launch_bounds__(256) void f32_prep_kernel(const float* __restrict__ q, const float* __restrict__ k1,
+                                                       const float* __restrict__ k2, const float* __restrict__ v2,
+                                                       const float* __restrict__ u_in, const float* __restrict__ v1,
+                                                       float* __restrict__ u,
                                                        const float* __restrict__ o, const float* __restrict__ d_o,
                                                        float* __restrict__ delta, unsigned* __restrict__ acc, int planes, size_t n,
-                                                       unsigned* __restrict__ scale_parts, unsigned* __restrict__ poison, int T) {
+                                                       unsigned* __restrict__ maxima, unsigned* __restrict__ poison, int T) {
     __shared__ unsigned red[4];
     constexpr int kPieces = D / 4;
     const int bh = blockIdx.y, j0 = blockIdx.x * 64;
     const size_t base = (size_t)bh * T * D;
-    if (scale_parts && threadIdx.x < 64 && j0 + threadIdx.x < T) poison[(size_t)bh * T + j0 + threadIdx.x] = 0;
-    // part s of a slice: its 64-row blocks s, s + kScaleParts, ...
-    for (int part = blockIdx.x; scale_parts && part < kScaleParts; part += gridDim.x) {
-        unsigned m = 0;
-        for (int r0 = part * 64; r0 < T; r0 += kScaleParts * 64)
-            m = max(m, block_absmax_bits<float>(d_o + base + (size_t)r0 * D, (size_t)min(64, T - r0) * kPieces, red));
-        if (threadIdx.x == 0) scale_parts[bh * kScaleParts + part] = m;
+    if (blockIdx.z) {  // part s of a slice: its 64-row blocks s, s + kScaleParts, ...
+        const int t = blockIdx.z - 1;
+        const float* src = (t == kMaxDO ? d_o : t == kMaxQ ? q : t == kMaxK1 ? k1 : t == kMaxK2 ? k2 : t == kMaxV2 ? v2 : v1 ? v1 : u_in) + base;
+        for (int part = blockIdx.x; part < kScaleParts; part += gridDim.x) {
+            unsigned m = 0;
+            for (int r0 = part * 64; r0 < T; r0 += kScaleParts * 64)
+                m = max(m, block_absmax_bits<float>(src + (size_t)r0 * D, (size_t)min(64, T - r0) * kPieces, red));
+            if (threadIdx.x == 0) maxima[((size_t)t * gridDim.y + bh) * kScaleParts + part] = m;
+        }
+        return;
     }
+    if (maxima && threadIdx.x < 64 && j0 + threadIdx.x < T) poison[(size_t)bh * T + j0 + threadIdx.x] = 0;
     for (int idx = threadIdx.x; idx < 64 * kPieces; idx += 256) {  // whole waves: 64 kPieces is a multiple of 256
         const int j = j0 + idx / kPieces;
         const size_t off = base + (size_t)j * D + (idx % kPieces) * 4;
@@ -70,24 +79,25 @@ __global__ __launch_bounds__(256) void f32_prep_kernel(const float* __restrict__
     }
 }
 // The sums -> the gradients (null: not wanted), four elements per thread: dK2, dV2, dK1 and dV1 = dU SiLU'(V1) from fixed
-// point (`slabs` > 0: from that many tiles' fp32 shares, in order), dQ = alpha times the sum of its tile's parts.  dQ's sum belongs to one tile, so its parts are joined in fp32 and in
-// order: a gradient may lie many powers of two below what the scale of a fixed-point sum is set by (operands of 0.01, T = 128:
-// dQ in steps of 2^-36 max |dO| is 6e-3 off, so joined 1e-6).  Costs what the accumulator did (training steps, accumulator ->
-// parts: B=2 H=4 T=500 D=64 4.32 -> 4.32 ms, B=4 H=8 T=128 522 -> 525 us, B=1 H=2 T=64 D=32 53.0 -> 53.5 us).
+// point (`slabs` > 0: from that many tiles' fp32 shares, in order), dQ = alpha times the sum of its tile's parts.  dQ's sum
+// belongs to one tile, so its parts are joined in fp32 and in order: a gradient may lie many powers of two below what the
+// scale of a fixed-point sum is set by (B=4 H=8 T=128 D=64, operands of 0.01: dQ in steps of 2^-36 max |dO| is 1.8e-2 off, so
+// joined 3e-7).  Costs what the accumulator did (training steps, accumulator -> parts: B=2 H=4 T=500 D=64 4.32 -> 4.32 ms,
+// B=4 H=8 T=128 522 -> 525 us, B=1 H=2 T=64 D=32 53.0 -> 53.5 us).
 template <typename E>
 __global__ __launch_bounds__(256) void f32_finish_kernel(const long long* __restrict__ acc, const E* __restrict__ v1,
                                                          E* __restrict__ dq, E* __restrict__ dk1, E* __restrict__ dk2,
                                                          E* __restrict__ dv1, E* __restrict__ dv2, size_t n, int T, int D,
-                                                         const unsigned* __restrict__ scale_parts,
+                                                         const unsigned* __restrict__ fields,
                                                          const unsigned* __restrict__ poison, float alpha,
                                                          const float* __restrict__ part_q, F32Deal deal, TdpMask mask, int nw,
                                                          int slabs) {
     typedef __attribute__((ext_vector_type(4))) E e4;
     for (size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4; i < n; i += (size_t)gridDim.x * 1024) {
         const size_t row = i / D;
-        const double inv = slabs ? 0. : fixed_scale_inverse(fixed_scale_field<false>(scale_parts, (int)(row / T), kF32FixedBias));
+        const uint4 field = slabs ? make_uint4(0u, 0u, 0u, 0u) : reinterpret_cast<const uint4*>(fields)[row / T];
         const unsigned bad = slabs ? 0u : poison[row];
-        auto put = [&](E* out, int which, unsigned bit, auto factor) {
+        auto put = [&](E* out, int which, unsigned bit, unsigned f, auto factor) {
             if (!out) return;
             if (slabs) {
                 const float* src = reinterpret_cast<const float*>(acc) + (size_t)which * slabs * n + i;
@@ -102,6 +112,7 @@ __global__ __launch_bounds__(256) void f32_finish_kernel(const long long* __rest
             const longlong2* p = reinterpret_cast<const longlong2*>(acc + which * n + i);
             const longlong2 lo = p[0], hi = p[1];
             const long long v[4] = {lo.x, lo.y, hi.x, hi.y};
+            const double inv = fixed_scale_inverse(f);
             e4 r;
 #pragma unroll
             for (int e = 0; e < 4; ++e)
@@ -109,12 +120,12 @@ __global__ __launch_bounds__(256) void f32_finish_kernel(const long long* __rest
             *reinterpret_cast<e4*>(out + i) = r;
         };
         auto one = [](int) { return 1.0f; };
-        put(dk2, 0, kPoisonDK2, one);
-        put(dv2, 1, kPoisonDV2, one);
-        put(dk1, 2, kPoisonDK1, one);
+        put(dk2, 0, kPoisonDK2, field.x, one);
+        put(dv2, 1, kPoisonDV2, field.y, one);
+        put(dk1, 2, kPoisonDK1, field.z, one);
         if (dv1) {
             const e4 x = *reinterpret_cast<const e4*>(v1 + i);
-            put(dv1, 3, kPoisonDU, [&](int e) { return silu_grad_f((float)x[e]); });
+            put(dv1, 3, kPoisonDU, field.w, [&](int e) { return silu_grad_f((float)x[e]); });
         }
         if (dq) {
             const float* src = part_q + row * deal.max_parts * D + i % D;
@@ -225,6 +236,7 @@ hipError_t launch_f32_bwd_tiles(F32BwdParams<E> p, const E* k1, const E* u, cons
     p.ka = k1; p.va = u; p.kb = k2; p.vb = v2;
     place_inputs(p, at, false);
     p.acc_k = acc_k2; p.acc_v = acc_v2; p.bit_k = kPoisonDK2; p.bit_v = kPoisonDV2;
+    p.rows.fields_at = 0; p.rows.streamed_k = kMaxK1; p.rows.streamed_v = kMaxV1;
     p.mask = natural;
     p.deal = want_q && !p.part_q && !p.acc_q ? whole : deal_for(natural);
     if (want_q) hipLaunchKernelGGL(kern_dq, grid_of(p.deal), dim3(64 * NW), smem, st, p);
@@ -233,6 +245,7 @@ hipError_t launch_f32_bwd_tiles(F32BwdParams<E> p, const E* k1, const E* u, cons
     p.ka = k2; p.va = v2; p.kb = k1; p.vb = u;
     place_inputs(p, at, true);
     p.acc_k = acc_k1; p.acc_v = acc_u; p.bit_k = kPoisonDK1; p.bit_v = kPoisonDU;
+    p.rows.fields_at = 2; p.rows.streamed_k = kMaxK2; p.rows.streamed_v = kMaxV2;
     p.mask = exchanged;
     p.deal = deal_for(exchanged);
     if (want_k1) hipLaunchKernelGGL(kern_nodq, grid_of(p.deal), dim3(64 * NW), smem, st, p);
@@ -246,22 +259,32 @@ hipError_t launch_f32_bwd(const F32BwdCall& c, hipStream_t st) {
     const bool want_q = c.dq != nullptr, want_k2 = c.dk2 || c.dv2, want_k1 = c.dk1 || c.dv1;
     const TdpMask natural{a.causal, a.k1_window, a.k2_window, a.kk_left, a.kk_right};
     const F32Deal deal_q = f32_bwd_deal(a.BH, a.T, D, natural);
-    // scratch: the accumulators of dK2, dV2, dK1 and dU, with fixed-point ones the rows' poison words and the slices' scale
-    // partials, and dQ's parts
+    // scratch: the accumulators of dK2, dV2, dK1 and dU, with fixed-point ones the rows' poison words, the slices' partial
+    // maxima and exponent fields, and dQ's parts
     const int slabs = f32_tile_slabs(a.BH, a.T) ? (a.T + 31) / 32 : 0;
     long long* acc = c.scratch;
     float* share = reinterpret_cast<float*>(acc);
     unsigned* poison = slabs ? nullptr : reinterpret_cast<unsigned*>(acc + 4 * n);
-    unsigned* parts = slabs ? nullptr : reinterpret_cast<unsigned*>(acc + 4 * n + (rows + 3) / 4 * 2);  // 16-byte aligned
-    float* part_q = slabs ? share + 4 * slabs * n : reinterpret_cast<float*>(parts + (size_t)a.BH * kScaleParts);
+    unsigned* maxima = slabs ? nullptr : reinterpret_cast<unsigned*>(acc + 4 * n + (rows + 3) / 4 * 2);  // 16-byte aligned
+    unsigned* fields = slabs ? nullptr : maxima + (size_t)a.BH * kScaleParts * kMaxima;
+    float* part_q = slabs ? share + 4 * slabs * n : reinterpret_cast<float*>(fields + (size_t)a.BH * 4);
     // a dQ of one part per tile needs no place of its own where the kernel can write the caller's type
     const bool direct_q = c.elem == 0 && deal_q.max_parts == 1;
-    hipLaunchKernelGGL(f32_prep_kernel<D>, dim3((a.T + 63) / 64, a.BH), dim3(256), 0, st, c.v1_f32, c.v1_f32 ? c.u_out : nullptr,
-                       c.o, a.d_o, c.delta, reinterpret_cast<unsigned*>(acc), slabs ? 4 * slabs : 8, n, parts, poison, a.T);
+    hipLaunchKernelGGL(f32_prep_kernel<D>, dim3((a.T + 63) / 64, a.BH, slabs ? 1 : 1 + kMaxima), dim3(256), 0, st, a.q, a.k1, a.k2, a.v2, a.u, c.v1_f32,
+                       c.v1_f32 ? c.u_out : nullptr, c.o, a.d_o, c.delta, reinterpret_cast<unsigned*>(acc), slabs ? 4 * slabs : 8, n,
+                       maxima, poison, a.T);
     F32BwdParams<float> p{};
     p.q = a.q; p.d_o = a.d_o; p.lse = a.lse_in; p.delta = c.delta;
     p.dq = direct_q ? (float*)c.dq : nullptr; p.part_q = direct_q ? nullptr : part_q; p.acc_q = nullptr; p.acc_q_rows = 0; p.stats_part = nullptr; p.split_rounds = 0;
-    p.scale_parts = parts; p.poison = poison; p.scale_bias = kF32FixedBias;
+    p.scale_parts = nullptr; p.poison = poison;
+    auto log2_above = [](float x) {  // x <= 2^this
+        int e = 128;
+        if (std::isfinite(x)) std::frexp(x, &e);
+        return e;
+    };
+    p.rows.maxima = maxima; p.rows.fields = fields;
+    p.rows.free_v = 127 + 61 - log2_above((float)a.T);
+    p.rows.free_k = p.rows.free_v - 1 - log2_above((float)D) - log2_above(a.alpha);
     p.T = a.T; p.BH = a.BH; p.nqt = (a.T + 31) / 32;
     p.alpha = a.alpha;
     p.acc_tile = slabs ? n : 0;
@@ -274,7 +297,7 @@ hipError_t launch_f32_bwd(const F32BwdCall& c, hipStream_t st) {
     auto finish = [&](auto zero) {
         using E = decltype(zero);
         hipLaunchKernelGGL(f32_finish_kernel<E>, grid, dim3(256), 0, st, acc, (const E*)c.v1, direct_q ? nullptr : (E*)c.dq,
-                           (E*)c.dk1, (E*)c.dk2, (E*)c.dv1, (E*)c.dv2, n, a.T, D, parts, poison, a.alpha, part_q, deal_q,
+                           (E*)c.dk1, (E*)c.dk2, (E*)c.dv1, (E*)c.dv2, n, a.T, D, fields, poison, a.alpha, part_q, deal_q,
                            natural, f32_bwd_waves(D), slabs);
     };
     if (c.elem == 0) finish(0.f);
@@ -401,7 +424,7 @@ hipError_t f32_mfma_tdp_fwd(const GenericTdpArgs& a, hipStream_t st) {
 size_t f32_mfma_tdp_bwd_scratch_elems(const GenericTdpArgs& a) {
     const size_t rows = (size_t)a.BH * a.T;
     const int parts_q = f32_bwd_deal(a.BH, a.T, a.D, TdpMask{a.causal, a.k1_window, a.k2_window, a.kk_left, a.kk_right}).max_parts;
-    const size_t fixed = 4 * rows * a.D + (rows + 3) / 4 * 2 + (size_t)a.BH * kScaleParts / 2;
+    const size_t fixed = 4 * rows * a.D + (rows + 3) / 4 * 2 + (size_t)a.BH * (kScaleParts * kMaxima + 4) / 2;
     // (one or two tiles' own accumulators are smaller than the fixed-point ones: the size stays monotone in T)
     const size_t sums = f32_tile_slabs(a.BH, a.T) ? std::max(fixed, 2 * ((a.T + 31) / 32) * rows * a.D) : fixed;
     return sums + rows * a.D * parts_q / 2;

@@ -547,8 +547,41 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 2 : 3) void tdp_f32_fwd_kernel(F
 // The operand reads and the walk over rounds and stages are the forward's; four waves per workgroup and two workgroups to a
 // CU at D <= 64 (B=4 H=8 T=512 D=64: 18.5 -> 13.5 ms, B=2 H=4 T=500: 20.0 -> 3.5; eight waves, one workgroup: 15.1 / 4.0).
 // DOUT < D: a workgroup produces DOUT of the gradient columns (blockIdx.y picks them).
-// the fp32 tensors' accumulators resolve 2^-36 of the slice's max |dO| and cover sums up to 2^27 times it
+
+// Scales of the fp32 tensors' row-gradient accumulators.  A gradient shrinks with every operand in it while dO stays, so the
+// scale follows all of them: with the slice's largest finite |dO|, |Q|, |K1|, |K2|, |V1|, |V2| (`maxima`, kScaleParts words per
+// tensor and slice, [tensor][BH][parts]; |SiLU(x)| <= |x|), S the streamed operands and sum P = 1,
+//   |dV rows| <= T max|dO| max|VS|       |dK rows| <= alpha T max|Q| max|KS| 2 D max|dO| max|V1| max|V2|
+// and a sum of that size is placed at 2^61.  A tensor with a few large elements makes this bound far too wide: the step is
+// never coarser than 2^-36 of max |dO| (sums past 2^27 times it then set the row's poison word, common.hpp).
+// B=4 H=8 T=128 D=64 with operands of 1 / 0.05 / 0.02 / 0.01, dK2 against 64 bits: 4.5e-7 / 1.4e-4 / 5.3e-3 / 8.1e-2 with the
+// scale of dO alone, 4.5e-7 / 2.8e-7 / 3.1e-7 / 3.2e-7 with this one.  Kernel time of a training step, dO's scale -> this:
+// B=2 H=4 T=500 D=64 4335 -> 4330 us, B=1 H=2 T=128 D=64 160.4 -> 159.8, B=4 H=8 T=128 D=64 531 -> 539.
 constexpr int kF32FixedBias = 36;
+enum { kMaxDO, kMaxQ, kMaxK1, kMaxK2, kMaxV1, kMaxV2, kMaxima };
+struct F32RowScale {
+    const unsigned* maxima;      // null: one scale by max |dO| (or float accumulators)
+    unsigned* fields;            // [BH][4] for the launch that converts: dK2, dV2, dK1, dU
+    int fields_at;               // 0 or 2: this launch's pair
+    int streamed_k, streamed_v;  // kMax.. of the streamed tensors
+    int free_k, free_v;          // exponent field that a sum bounded by 1 would get, less what alpha, T and D take
+};
+__device__ __forceinline__ void f32_row_fields(const F32RowScale& s, int BH, int bh, int& field_k, int& field_v) {
+    // lane t * kScaleParts + i holds part i of tensor t, and at the end an exponent that all of that tensor is below
+    const int lane = threadIdx.x & 63, t = lane / kScaleParts;
+    static_assert(kScaleParts == 8 && kMaxima * kScaleParts <= 64, "one word per lane");
+    unsigned m = s.maxima[((size_t)min(t, kMaxima - 1) * BH + bh) * kScaleParts + lane % kScaleParts];
+#pragma unroll
+    for (int w = 1; w < kScaleParts; w *= 2) m = max(m, (unsigned)__shfl_xor((int)m, w, 64));
+    const int e = (int)(m >> 23) - 126;
+    auto exponent = [&](int tensor) { return __builtin_amdgcn_readlane(e, tensor * kScaleParts); };
+    const int d_o = exponent(kMaxDO), v1 = exponent(kMaxV1), v2 = exponent(kMaxV2);
+    const int least = max(min(kF32FixedBias + 254 - 126 - d_o, 254), 1);  // as fixed_scale_field
+    field_v = s.free_v - d_o - (s.streamed_v == kMaxV1 ? v1 : v2);
+    field_k = s.free_k - d_o - v1 - v2 - exponent(kMaxQ) - (s.streamed_k == kMaxK1 ? exponent(kMaxK1) : exponent(kMaxK2));
+    field_k = max(least, min(field_k, 254));
+    field_v = max(least, min(field_v, 254));
+}
 
 template <typename E>
 struct F32BwdParams {
@@ -573,6 +606,7 @@ struct F32BwdParams {
     const unsigned* scale_parts;
     unsigned* poison;
     int scale_bias;
+    F32RowScale rows;  // maxima not null: the scales of acc_k and acc_v instead of scale_parts'
     unsigned bit_k, bit_v;  // poison bits of acc_k / acc_v
     int T, BH, nqt;        // nqt: query tiles this launch covers (tiles 0 .. nqt - 1)
     float alpha;
@@ -646,8 +680,6 @@ __device__ __forceinline__ void f32_bwd_body(const F32BwdParams<E>& p, int only_
     const E* __restrict__ Qs = slice(p.q, p.at_q);
     const TdpMask mask = p.mask;
     const float scale_log2 = p.alpha * kLog2e;
-    const float fscale = p.scale_parts ? fixed_scale_value(fixed_scale_field(p.scale_parts, bh, p.scale_bias)) : 0.f;
-
     const int q0 = qt * 32, q1 = min(T - 1, q0 + 31);
     const int q = q0 + n;
     const Range rows = row_range(mask, q0, q1, T);
@@ -688,6 +720,18 @@ __device__ __forceinline__ void f32_bwd_body(const F32BwdParams<E>& p, int only_
         const size_t row = (size_t)min(q0 + r, T - 1);
         sQ[r * LD + d] = (float)Qs[row * p.at_q.st + d] * scale_log2;
         sDO[r * LD + d] = (float)slice(p.d_o, p.at_do)[row * p.at_do.st + d];
+    }
+    // (here, where the first stage's loads are on their way)
+    float fscale = p.scale_parts ? fixed_scale_value(fixed_scale_field(p.scale_parts, bh, p.scale_bias)) : 0.f, fscale_v = fscale;
+    if (p.rows.maxima) {
+        int field_k, field_v;
+        f32_row_fields(p.rows, p.BH, bh, field_k, field_v);
+        fscale = fixed_scale_value(field_k);
+        fscale_v = fixed_scale_value(field_v);
+        if (qt == 0 && part == 0 && threadIdx.x == 0) {
+            p.rows.fields[bh * 4 + p.rows.fields_at] = field_k;
+            p.rows.fields[bh * 4 + p.rows.fields_at + 1] = field_v;
+        }
     }
     // a query past the end of the sequence gets a huge LSE: its P is exactly 0
     float lse2 = 1.0e30f, delta = 0.f;
@@ -856,7 +900,7 @@ __device__ __forceinline__ void f32_bwd_body(const F32BwdParams<E>& p, int only_
                     const float sum = half_sum_16x2(xk, xv);
                     const bool odd = n & 1;
                     const int i = half_sum_register(), d = c0 + DTO * c_row(g, i) + dt;
-                    shared_add(odd ? p.acc_v : p.acc_k, (size_t)qt * p.acc_tile + base + (size_t)b * D + d, odd ? sum : sum * kLn2, fscale,
+                    shared_add(odd ? p.acc_v : p.acc_k, (size_t)qt * p.acc_tile + base + (size_t)b * D + d, odd ? sum : sum * kLn2, odd ? fscale_v : fscale,
                                p.poison + (size_t)bh * T + b, odd ? p.bit_v : p.bit_k);
                     __builtin_amdgcn_sched_barrier(0);  // one tile's products and sums in registers at a time
                 }

@@ -1096,23 +1096,39 @@ def _gradients_in_64_bits(inputs, alpha, heads, **windows):
 
 
 @pytest.mark.parametrize("D", [32, 64, 128])
-@pytest.mark.parametrize("c", [0.05, 0.02, 0.01])
+@pytest.mark.parametrize("case", ["0.05", "0.02", "0.01", "keys 1e-3", "values 1e-4", "outliers", "16-bit 0.02"])
 @pytest.mark.parametrize("splits", [0, 1])
-def test_fp32_dq_of_small_operands(D, c, splits, tune):
-    """128 query tiles and operands of size c: dQ against 64 bits, its tile dealt out to workgroups and in one.  Bar: a
-    rounding of 2^-24 in each of the D + 3 sums and products behind an element, and sqrt(T) of them in its sum (8.8e-5 at
-    D = 128)."""
-    print(f"case small operands, dQ: D={D} c={c} splits={splits}", flush=True)
+def test_fp32_gradients_of_small_operands(D, case, splits, tune):
+    """128 query tiles and operands of size c: all five gradients against 64 bits, the tiles dealt out to workgroups and in
+    one each; keys or values alone that small; one element of every tensor 30 times the others; 16-bit tensors on these
+    kernels.  Bar: a rounding of 2^-24 in each of the D + 3 sums and products behind an element,
+    and sqrt(T) of them in its sum (8.8e-5 at D = 128)."""
+    print(f"case small operands: D={D} {case} splits={splits}", flush=True)
     tune(_lib.TUNE_BWD_SPLITS, splits)
     B, H, T = 4, 8, 128
     inputs = orc.make_inputs(B, H, T, D, torch.float32, seed=D)
-    inputs = [t * c for t in inputs[:5]] + [inputs[5]]
+    scale = [1.0] * 6
+    if case == "outliers":
+        for d, t in enumerate(inputs[:5]):  # a column each: their product in one score would leave fp32 no digits
+            t[..., T // 3, d] *= 30
+    elif case.startswith("keys"):
+        scale[1] = scale[2] = 1e-3
+    elif case.startswith("values"):
+        scale[3] = scale[4] = 1e-4
+    else:
+        scale[:5] = [float(case.split()[-1])] * 5
+    inputs = [t * c for t, c in zip(inputs, scale)]
+    bar, flags = 2.0 ** -24 * (D + 3) * math.sqrt(T), 0
+    if case.startswith("16-bit"):
+        inputs = [t.bfloat16() for t in inputs]
+        bar, flags = 2.0 ** -8, _lib.FLAG_FORCE_GENERIC  # the rounding of the result
     heads = [(0, 0), (1, 5), (3, 7)]
-    _, g = util.run_tdp(inputs, 1 / math.sqrt(D), True)
+    _, g = util.run_tdp(inputs, 1 / math.sqrt(D), True, flags=flags)
     for (b, h), want in zip(heads, _gradients_in_64_bits(inputs, 1 / math.sqrt(D), heads)):
-        err = (g[0][b, h].double() - want[0]).norm() / want[0].norm()
-        print(f"    dq[{b}, {h}]: {err:.2e}", flush=True)
-        assert err <= 2.0 ** -24 * (D + 3) * math.sqrt(T), (b, h, err.item())
+        for name, a, r in zip(util.NAMES, g, want):
+            err = ((a[b, h].double() - r).norm() / r.norm()).item()
+            print(f"    {name}[{b}, {h}]: {err:.2e}  (max {r.abs().max().item():.1e})", flush=True)
+            assert err <= bar, (name, b, h, err)
 
 
 def test_fp32_dq_beyond_the_range_of_dO():
