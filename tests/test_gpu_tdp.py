@@ -1173,3 +1173,23 @@ def test_fp32_gradients_of_a_few_tiles_are_fp32_throughout(B, H, T, D, splits, c
             # (in the norm the rounding of dP - Delta of the first, largest rows counts, whose own gradients are nearly zero)
             assert case.startswith("rows") or err <= 2.0 ** -24 * (D + 3) * math.sqrt(T), (name, b, h, err)
             assert rows <= 1e-4, (name, b, h, rows)
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_fp32_forward_of_large_values_under_rising_scores(D):
+    """Keys whose scores are 2^35 above those of the tile before and values of 1e13 (outputs of 1e26): the unnormalised sums
+    stay far enough from the end of fp32's range, whatever maximum they are kept relative to."""
+    T, alpha = 96, 0.125
+    inputs = orc.make_inputs(1, 2, T, D, torch.float32, seed=D + 1)
+    q, k1, k2, v1, v2, _ = inputs
+    q *= 0.1
+    q[..., 0], k2[..., 0], k1[..., 0] = 1.0, 1.0, 0.0
+    k1[..., 32:64, 0] = 35 * math.log(2) / alpha
+    k1[..., 64:, 0] = 70 * math.log(2) / alpha
+    v1 *= 1e13
+    v2 *= 1e13
+    out, _ = util.run_tdp(inputs, alpha, True, backward=False)
+    assert torch.isfinite(out).all()
+    for h in range(2):
+        z, _, _ = orc.tdp_forward_backward_chunked(*(t[0, h].double() for t in inputs), alpha, True, need_grads=False)
+        assert util.rel_err(out[0, h].double(), z) <= 1e-4
