@@ -448,6 +448,10 @@ bool use_mfma_dps(int D, int dtype, unsigned flags) {
 bool dps_keeps(int D, int dtype, unsigned flags) {
     return use_mfma_dps(D, dtype, flags) || (dtype == TRITT_F32 && use_f32_mfma_dps(D));
 }
+// whether a forward may have left it: TRITT_TUNE_F32_VALU may have been set since (the backward then runs the inner pass)
+bool dps_kept_exists(int D, int dtype, unsigned flags) {
+    return use_mfma_dps(D, dtype, flags) || (dtype == TRITT_F32 && f32_mfma_dps_supported(D));
+}
 
 bool any_null(std::initializer_list<const void*> ps) {
     for (const void* p : ps)
@@ -1021,17 +1025,17 @@ int tritt_dps_bwd_strided(const void* q, const void* k1, const void* k2, const v
 
 int tritt_dps_keeps(int D, int dtype, unsigned flags) { return dps_keeps(D, dtype, flags) ? 1 : 0; }
 
-static int check_kept(const float* r, const float* lse1, int B, int H, int T, int D, int dtype, unsigned flags) {
+static int check_kept(const float* r, const float* lse1, int B, int H, int T, bool form) {
     if (empty_problem(B, H, T)) return TRITT_OK;
     if (any_null({r, lse1}) || any_misaligned({r, lse1})) return TRITT_ERR_INVALID;
-    return dps_keeps(D, dtype, flags) ? TRITT_OK : TRITT_ERR_UNSUPPORTED;
+    return form ? TRITT_OK : TRITT_ERR_UNSUPPORTED;
 }
 
 int tritt_dps_fwd_keep(const void* q, const void* k1, const void* k2, const void* v1, const void* v2,
                        const tritt_layout* in_layouts, void* o, float* lse, float* r, float* lse1, int B, int H, int T, int D,
                        int dtype, float alpha, int causal, int k_diff, void* workspace, size_t workspace_bytes,
                        unsigned flags, void* stream) {
-    if (int rc = check_kept(r, lse1, B, H, T, D, dtype, flags); rc != TRITT_OK) return rc;
+    if (int rc = check_kept(r, lse1, B, H, T, dps_keeps(D, dtype, flags)); rc != TRITT_OK) return rc;
     return in_layouts ? dps_fwd_strided_call(q, k1, k2, v1, v2, in_layouts, o, lse, B, H, T, D, dtype, alpha, causal, k_diff,
                                              workspace, workspace_bytes, flags, stream, DpsKept{r, lse1})
                       : dps_fwd_call(q, k1, k2, v1, v2, o, lse, B, H, T, D, dtype, alpha, causal, k_diff, workspace,
@@ -1043,7 +1047,7 @@ int tritt_dps_bwd_kept(const void* q, const void* k1, const void* k2, const void
                        const void* d_o, const tritt_layout* d_o_layout, void* dq, void* dk1, void* dk2, void* dv1, void* dv2,
                        int B, int H, int T, int D, int dtype, float alpha, int causal, int k_diff, void* workspace,
                        size_t workspace_bytes, unsigned flags, void* stream) {
-    if (int rc = check_kept(r, lse1, B, H, T, D, dtype, flags); rc != TRITT_OK) return rc;
+    if (int rc = check_kept(r, lse1, B, H, T, dps_kept_exists(D, dtype, flags)); rc != TRITT_OK) return rc;
     const DpsKept kept{const_cast<float*>(r), const_cast<float*>(lse1)};  // only read
     return in_layouts || d_o_layout
                ? dps_bwd_strided_call(q, k1, k2, v1, v2, in_layouts, o, lse, d_o, d_o_layout, dq, dk1, dk2, dv1, dv2, B, H, T, D,

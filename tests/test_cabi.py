@@ -174,3 +174,15 @@ def test_kept_inner_pass_where_there_is_none():
     assert lib.tritt_dps_keeps(64, _lib.TRITT_BF16, _lib.FLAG_FORCE_GENERIC) == 0
     assert lib.tritt_dps_keeps(16, _lib.TRITT_F32, _lib.FLAG_AUTO) == 0
     assert lib.tritt_dps_keeps(128, _lib.TRITT_F32, _lib.FLAG_AUTO) == 0
+
+
+def test_kept_inner_pass_is_taken_after_the_kernels_were_switched(tune):
+    """Between a forward that kept its inner pass and the backward the fp32 kernels may be switched: the backward still
+    takes what it is handed (it is refused here for its workspace, behind the check of the form)."""
+    lib, one = _lib.lib(), ctypes.c_void_p(256)
+    call = lambda D: lib.tritt_dps_bwd_kept(*[one] * 5, None, *[one] * 5, None, *[one] * 5, 1, 1, 64, D, _lib.TRITT_F32, 0.1, 1, 64,
+                                            None, 0, 0, None)
+    assert call(64) == -3 and call(128) == -4
+    tune(_lib.TUNE_F32_VALU, 1)
+    assert lib.tritt_dps_keeps(64, _lib.TRITT_F32, _lib.FLAG_AUTO) == 0
+    assert call(64) == -3 and call(128) == -4

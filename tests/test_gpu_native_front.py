@@ -164,3 +164,13 @@ def test_native_path_arguments_without_a_truth_value():
         flash_trittention(*ins, causal=torch.ones(2), **FULL)
     with pytest.raises(RuntimeError, match="ambiguous"):
         flash_trittention(*ins, convert_to_float32=torch.ones(2), **FULL)
+
+
+def test_kernels_switched_between_a_keeping_forward_and_its_backward(tune):
+    *ins, grad = make(torch.float32, False)
+    a = leaves(ins, (1,) * 5)
+    out, _ = TrittentionTriton(softmax_scale=0.2, k_diff=40)(*a)
+    want = torch.autograd.grad(out, a, grad, retain_graph=True)
+    tune(_lib.TUNE_F32_VALU, 1)
+    for x, y in zip(torch.autograd.grad(out, a, grad), want):
+        torch.testing.assert_close(x, y, rtol=1e-4, atol=2e-5)
