@@ -19,6 +19,7 @@
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
+#include <torch/version.h>
 
 #include <array>
 #include <optional>
@@ -394,4 +395,12 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", "torch tensors to the C 
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__native(void) { return PyModule_Create(&module); }
+// torch_version: what this was compiled against; torch's C++ interfaces change from one version to the next
+PyMODINIT_FUNC PyInit__native(void) {
+    PyObject* m = PyModule_Create(&module);
+    if (m && PyModule_AddStringConstant(m, "torch_version", TORCH_VERSION) < 0) {
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
+}

@@ -186,3 +186,35 @@ def test_kept_inner_pass_is_taken_after_the_kernels_were_switched(tune):
     tune(_lib.TUNE_F32_VALU, 1)
     assert lib.tritt_dps_keeps(64, _lib.TRITT_F32, _lib.FLAG_AUTO) == 0
     assert call(64) == -3 and call(128) == -4
+
+
+@pytest.mark.parametrize("broken", ["missing", "another torch"])
+def test_host_path_without_its_extension(broken, monkeypatch):
+    """An extension that is missing or built for another torch: the Functions and ctypes take the calls, with a warning."""
+    import sys
+    import types
+
+    import flash_trittention as ft
+
+    other = None if broken == "missing" else types.SimpleNamespace(torch_version="0.1", tdp=None, dps=None)
+    monkeypatch.setattr(_lib, "_native", None)
+    monkeypatch.delattr(ft, "_native", raising=False)
+    monkeypatch.setitem(sys.modules, "flash_trittention._native", other)
+    q = torch.randn(1, 1, 32, 32)
+    with pytest.warns(RuntimeWarning, match="_native.so is not used"), pytest.raises(RuntimeError, match="CPU implementation"):
+        ft.flash_trittention(q, q, q, q, q)
+    with pytest.raises(RuntimeError, match="CPU implementation"):
+        ft.TrittentionTriton()(q, q, q, q, q)
+
+
+def test_c_library_builds_without_torch(tmp_path):
+    """`make lib` looks for no torch, and `make` gives the library where there is none (dry run)."""
+    import subprocess
+
+    (tmp_path / "python3").write_text("#!/bin/sh\ncase \"$2\" in *torch*) echo asked >> " + str(tmp_path / "asked") +
+                                      ";; esac\nexit 1\n")
+    (tmp_path / "python3").chmod(0o755)
+    env = dict(os.environ, PATH=f"{tmp_path}:{os.environ['PATH']}")
+    out = subprocess.run(["make", "-n", "-B", "-C", _lib.CSRC_DIR, "lib"], env=env, check=True, capture_output=True, text=True)
+    assert "libtrittention_hip.so" in out.stdout and "torch_front" not in out.stdout
+    assert not (tmp_path / "asked").exists()
