@@ -110,10 +110,13 @@ def test_fp32_rounds_dealt_out_to_workgroups(D, T, splits, tune):
 
 
 @pytest.mark.parametrize("causal", [True, False])
-def test_fp32_head_dim_128_large_grid_on_the_matrix_cores(causal, tune):
-    """D = 128 with enough query tiles that each is walked by one workgroup (dQ written by that workgroup, its running
-    sum kept in LDS): against the fp32 VALU kernels of the same library, bitwise the same on a second run."""
-    print(f"case fp32 mfma D=128 large grid causal={causal}", flush=True)
+@pytest.mark.parametrize("splits", [0, 1])
+def test_fp32_head_dim_128_large_grid_on_the_matrix_cores(causal, splits, tune):
+    """D = 128 (dQ's running sum of a workgroup kept in LDS) on 136 query tiles, dealt out to workgroups whose shares of dQ
+    are joined, and with each tile walked by one workgroup that writes its dQ: against the fp32 VALU kernels of the same
+    library, bitwise the same on a second run."""
+    print(f"case fp32 mfma D=128 large grid causal={causal} splits={splits}", flush=True)
+    tune(_lib.TUNE_BWD_SPLITS, splits)
     inputs = orc.make_inputs(2, 4, 530, 128, torch.float32, seed=11)
     alpha = 1 / math.sqrt(128)
     out, g = util.run_tdp(inputs, alpha, causal)
@@ -1193,3 +1196,26 @@ def test_fp32_forward_of_large_values_under_rising_scores(D):
     for h in range(2):
         z, _, _ = orc.tdp_forward_backward_chunked(*(t[0, h].double() for t in inputs), alpha, True, need_grads=False)
         assert util.rel_err(out[0, h].double(), z) <= 1e-4
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("splits", [0, 1])
+@pytest.mark.parametrize("wanted", [0b11111, 0b00001, 0b10110])
+def test_narrow_windows_of_16_bit_tensors_in_fp32(D, splits, wanted, tune):
+    """Windows that leave a query at most 1024 pairs: every tile of the 16-bit backward runs on the fp32 kernels, in one
+    workgroup that writes its dQ itself (D = 128: from LDS) or in several that share an accumulator."""
+    from flash_trittention import _ops
+
+    print(f"case narrow 16-bit D={D} splits={splits} wanted={wanted:05b}", flush=True)
+    tune(_lib.TUNE_BWD_SPLITS, splits)
+    windows, T, alpha = (24, 22, 9, 13), 170, 1 / math.sqrt(D)
+    inputs = orc.make_inputs(2, 2, T, D, torch.bfloat16, seed=D + splits)
+    _, _, grads = util.oracle_tdp(inputs, alpha, True, windows)
+    *ins, d_o = (t.cuda() for t in inputs)
+    o, lse = _ops.tdp_fwd_impl(*ins, alpha, True, *windows, _lib.FLAG_AUTO)
+    got = _ops.tdp_bwd_impl(*ins, o, lse, d_o, alpha, True, *windows, _lib.FLAG_AUTO, wanted)
+    for i, (name, a, want) in enumerate(zip(util.NAMES, got, grads)):
+        assert (a is not None) == bool(wanted >> i & 1), name
+        if a is not None:
+            util.assert_mostly_close(name, a.float().cpu(), want, **LOWP)
+            assert util.rel_err(a.float().cpu(), want) <= 2e-2, name
