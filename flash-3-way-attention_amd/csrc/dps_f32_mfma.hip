@@ -10,8 +10,8 @@
 // end.  A step of 32 x 32 pairs is 64-128 MFMAs of 64 cycles, so the serial chain of steps of one wave is what a call
 // of a few hundred owner tiles waits for: with one wave per owner tile and the streamed tiles shared through LDS
 // (B = 2, H = 8, T = 1000, D = 64: half a wave per SIMD, up to 32 steps of 4.4 us one after another) a training step
-// took 589 us, now 205; larger grids gain from the loads and the missing barriers (B = 4, H = 16, T = 2048: 7.1 -> 3.1 ms,
-// 110 TFLOP/s executed of 157).  What bounds it now: the MFMAs at that rate, below it the chain.  Operands come from L2 straight into registers
+// took 589 us, now 193; larger grids gain from the loads and the missing barriers (B = 4, H = 16, T = 2048: 7.1 -> 2.7 ms,
+// 114 TFLOP/s executed of 157).  What bounds it now: the MFMAs at that rate, below it the chain.  Operands come from L2 straight into registers
 // (16 KB per step and wave: a quarter of what L2 gives a CU in the time of the step's MFMAs), without LDS and without a
 // barrier inside the loop; a register set is loaded again as soon as the product that reads it has been issued, so every
 // load has at least one product (2048 cycles) to arrive in.

@@ -51,7 +51,7 @@ struct GenericTdpArgs {
 hipError_t generic_tdp_fwd(const GenericTdpArgs& a, hipStream_t st);
 hipError_t generic_tdp_bwd(const GenericTdpArgs& a, hipStream_t st);
 
-// fp32 MFMA triple-dot kernels (D = 32 or 64, any mask): same operands as the VALU kernels
+// fp32 MFMA triple-dot kernels (D = 32, 64 or 128, any mask): same operands as the VALU kernels
 bool f32_mfma_tdp_supported(int D);
 // workgroups per query tile that the forward of this problem is dealt out to (BH, T, D and the mask of `a`)
 int f32_fwd_parts(const GenericTdpArgs& a);
@@ -66,7 +66,7 @@ struct F32BwdCall {
     const float* v1_f32;  // with u_out = a.u: fp32 V1, whose SiLU the call forms; null: a.u is there already
     float* u_out;
     float* delta;         // scratch [BH, T]
-    long long* scratch;   // f32_mfma_tdp_bwd_scratch_elems() 64-bit words: fixed-point accumulators and dQ's parts
+    long long* scratch;   // f32_mfma_tdp_bwd_scratch_elems() 64-bit words: the row gradients' accumulators and dQ's parts
     const void* v1;       // V1 in the caller's type (SiLU')
     void *dq, *dk1, *dk2, *dv1, *dv2;  // null: not wanted
     int elem;             // the caller's type: 0 float, 1 bf16, 2 f16

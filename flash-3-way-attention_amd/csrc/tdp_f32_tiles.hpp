@@ -540,7 +540,7 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 2 : 3) void tdp_f32_fwd_kernel(F
 //   dKB[b, d]  += alpha sum_q Yq^T[d, q] Q[q, d],   dVB[b, d] += sum_q Tv^T[d, q] dO[q, d]
 // The sums over the tile's 32 queries are lane reductions; the sums over query tiles (workgroups) go to shared
 // accumulators: 64-bit fixed point with integer atomics (the result does not depend on the order of arrival), or
-// fp32 atomics when the caller's accumulators are fp32.
+// fp32 atomics when the accumulators are fp32 (the caller's, or a tile's own: F32BwdParams::acc_tile).
 //
 // The tensors may be 16-bit (E = bf16 / f16): they are converted as they are staged, everything after that is
 // fp32.  That is how the 16-bit backward runs its first query tile: for the first few causal queries the softmax

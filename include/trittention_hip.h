@@ -115,8 +115,9 @@ int tritt_set_tuning(int knob, int value, int* previous);
  *   like every other entry point here, the call is bitwise reproducible from run to run
  *   (measured cost against fp32 atomics: none).  The fixed-point scale is a power of two chosen
  *   per (batch, head) slice from the largest finite |dO| of the slice: steps of 2^-30 of that
- *   magnitude (2^-36 on the fp32 matrix-core kernels), sums up to 2^33 (2^27) times it, so the
- *   backward is exactly homogeneous in dO for powers of two (loss scaling, mean-reduced losses)
+ *   magnitude, sums up to 2^33 times it (fp32 matrix-core kernels: from the largest magnitudes of
+ *   all six tensors, never coarser than 2^-36 of max |dO|; dQ, and below eight query tiles all
+ *   five gradients, are summed in fp32 there), so the backward is exactly homogeneous in dO for powers of two (loss scaling, mean-reduced losses)
  *   and has no absolute floor, like the reference's fp32 accumulators
  *   (triple_dot_product/kernels/bwd_dk1.py:239-258).  A share that is NaN, Inf or beyond the
  *   accumulator's range makes that row of that gradient NaN in the output.
