@@ -99,7 +99,7 @@ struct FirstTileArgs {
     int causal, k1_window, k2_window, kk_left, kk_right;
     bool want_q, want_k2, want_k1;
     int tiles;
-    bool split_rounds;  // tiles > 1: the rounds (of eight rows) of a query tile may be dealt out to workgroups; needs acc_q when dQ is wanted
+    bool deal_out;  // tiles > 1: the rounds of a query tile may be dealt out to workgroups
 };
 hipError_t f32_mfma_tdp_bwd_first_tile(const FirstTileArgs& a, hipStream_t st);
 // fp32 operands of the dot-product-sum kernels (two chained attention passes).

@@ -787,12 +787,23 @@ static hipError_t launch_bwd(const MfmaBwdArgs& a, hipStream_t st) {
     float *dk1acc = (float*)(ws + l.dk1acc), *duacc = (float*)(ws + l.duacc);
     float *dk2acc = (float*)(ws + l.dk2acc), *dv2acc = (float*)(ws + l.dv2acc);
 
+    // A windowed mask that leaves a query no more than about a thousand (j, k) pairs makes every softmax row nearly one-hot
+    // (see below, at query tile 0): then all query tiles take the fp32 kernel (the work of such masks is small: T times the
+    // pair count).  Its tiles cost the same but for the first ones, so their rounds are dealt out (F32Deal) where the tiles
+    // alone do not fill the chip's two workgroups per CU.  Backward, D = 64, H = 4, whole tiles -> dealt out: windows
+    // (16,16,8,8) 100 / 128 / 256 tiles 365 / 364 / 374 -> 218 / 256 / 393 us, (24,22,24,22) 128 / 256 tiles 507 / 516 -> 333 / 517;
+    // 1024 tiles 1143 -> 1218 and 1632 -> 1686, so not there.
+    const long long pairs = (long long)(a.k2_window + 1) * std::min(a.k1_window + 1, a.kk_left + a.kk_right + 1);
+    const bool all_in_f32 = a.causal && a.windowed && pairs <= 1024 && !a.split;
+    const bool deal_f32 = all_in_f32 && a.BH * ((a.T + 31) / 32) < 512;
+
     // A workgroup owns a 32-query tile and walks all of its rows.  When that leaves most of the chip idle, or
     // ends in a long tail (few heads, short sequences), the rows of a tile are dealt out to several
     // workgroups, and dQ is accumulated in fp32 like the row gradients.
     const int tiles = 8 * ((a.BH + 7) / 8) * ((a.T + 31) / 32);
     int splits = 1;
-    if (D == 64 && a.windowed && !a.split) splits = windowed_splits(a);
+    if (all_in_f32) splits = deal_f32 ? 2 : 1;  // (an accumulator for dQ, or none)
+    else if (D == 64 && a.windowed && !a.split) splits = windowed_splits(a);
     else if (D == 64 && a.causal && !a.split && tiles < 1024) splits = causal_splits(a);
     else if (tiles < 1024) splits = std::min(16, (1024 + tiles - 1) / tiles);
     // a few waves of long tiles: the last tiles of each head are the costliest (the work of a tile grows with the
@@ -908,11 +919,8 @@ static hipError_t launch_bwd(const MfmaBwdArgs& a, hipStream_t st) {
     // are nearly one-hot, and dS = P (dP - Delta) then cancels two numbers whose 16-bit operand rounding the
     // kernels here cannot resolve (query 0 has a gradient of exactly zero in dQ).  The kernels below start at
     // tile 1: the grid simply has one tile less, and the heaviest-first numbering never reaches tile 0.
-    // A windowed mask that leaves a query no more than about a thousand (j, k) pairs makes every row like that:
-    // then all query tiles take the fp32 kernel (the work of such masks is small: T times the pair count).
+    // (all_in_f32: every tile does)
     const bool first_in_f32 = a.causal != 0;
-    const long long pairs = (long long)(a.k2_window + 1) * std::min(a.k1_window + 1, a.kk_left + a.kk_right + 1);
-    const bool all_in_f32 = first_in_f32 && a.windowed && pairs <= 1024 && !a.split;
     // tile 0's backward workgroups ride at the end of the first rows launch below where that is the D = 64 kernel
     // (tdp_bwd_rows_tile0_kernel); otherwise they are a launch of their own
     bool fuse_tile0 = false;
@@ -931,7 +939,7 @@ static hipError_t launch_bwd(const MfmaBwdArgs& a, hipStream_t st) {
         f.k1_window = a.k1_window; f.k2_window = a.k2_window; f.kk_left = a.kk_left; f.kk_right = a.kk_right;
         f.want_q = want_q; f.want_k2 = want_k2; f.want_k1 = want_k1;
         f.tiles = all_in_f32 ? p.nqt : 1;
-        f.split_rounds = dqacc || !want_q;
+        f.deal_out = deal_f32;
         if constexpr (D == 64) {
             if (plain64 && !all_in_f32 && p.nqt > 1 && (want_q || want_k2 || want_k1)) {
                 if (hipError_t e = tile0_prepare<E, 64>(f, st, t0_r0, t0_r1, t0_roles, t0_rounds); e != hipSuccess) return e;

@@ -217,7 +217,7 @@ bool f32_tile_slabs(int BH, int T) { return (long long)BH * ((T + 31) / 32) < 8;
 template <typename E, int D>
 hipError_t launch_f32_bwd_tiles(F32BwdParams<E> p, const E* k1, const E* u, const E* k2, const E* v2, void* acc_k2,
                                 void* acc_v2, void* acc_k1, void* acc_u, const TdpMask& natural, bool want_q,
-                                bool want_k2, bool want_k1, hipStream_t st, const InputsAt& at, bool split) {
+                                bool want_k2, bool want_k1, hipStream_t st, const InputsAt& at, bool deal_out) {
     // a workgroup holds all D gradient columns and forms S and dP once (D = 128: dQ's running sum is kept in LDS)
     constexpr int DOUT = D;
     constexpr int NW = f32_bwd_waves(D);
@@ -230,7 +230,7 @@ hipError_t launch_f32_bwd_tiles(F32BwdParams<E> p, const E* k1, const E* u, cons
     // of parts belongs to the mask it was made for, and the second launch exchanges the two key indices.
     const TdpMask exchanged{natural.causal, natural.wb, natural.wa, natural.rab, natural.lab};
     const F32Deal whole{0.f, 1, p.nqt};
-    auto deal_for = [&](const TdpMask& m) { return split ? f32_bwd_deal(p.BH, p.T, D, m) : whole; };
+    auto deal_for = [&](const TdpMask& m) { return deal_out ? f32_bwd_deal(p.BH, p.T, D, m) : whole; };
     auto grid_of = [&](const F32Deal& d) { return dim3(8 * xcd_slots(p.BH, d.items), D / DOUT); };
     // rows = (K2, V2), streamed = (K1, U): dQ, dK2, dV2
     p.ka = k1; p.va = u; p.kb = k2; p.vb = v2;
@@ -403,11 +403,11 @@ static hipError_t first_tile_typed(const FirstTileArgs& a, hipStream_t st) {
     const E *k1 = (const E*)a.k1, *u = (const E*)a.u, *k2 = (const E*)a.k2, *v2 = (const E*)a.v2;
     const bool wq = a.want_q, wk2 = a.want_k2, wk1 = a.want_k1;
     if (a.D == 32)
-        return launch_f32_bwd_tiles<E, 32>(p, k1, u, k2, v2, a.acc_k2, a.acc_v2, a.acc_k1, a.acc_u, natural, wq, wk2, wk1, st, inputs_of(a), a.split_rounds);
+        return launch_f32_bwd_tiles<E, 32>(p, k1, u, k2, v2, a.acc_k2, a.acc_v2, a.acc_k1, a.acc_u, natural, wq, wk2, wk1, st, inputs_of(a), a.deal_out);
     if (a.D == 64)
-        return launch_f32_bwd_tiles<E, 64>(p, k1, u, k2, v2, a.acc_k2, a.acc_v2, a.acc_k1, a.acc_u, natural, wq, wk2, wk1, st, inputs_of(a), a.split_rounds);
+        return launch_f32_bwd_tiles<E, 64>(p, k1, u, k2, v2, a.acc_k2, a.acc_v2, a.acc_k1, a.acc_u, natural, wq, wk2, wk1, st, inputs_of(a), a.deal_out);
     if (a.D == 128)
-        return launch_f32_bwd_tiles<E, 128>(p, k1, u, k2, v2, a.acc_k2, a.acc_v2, a.acc_k1, a.acc_u, natural, wq, wk2, wk1, st, inputs_of(a), a.split_rounds);
+        return launch_f32_bwd_tiles<E, 128>(p, k1, u, k2, v2, a.acc_k2, a.acc_v2, a.acc_k1, a.acc_u, natural, wq, wk2, wk1, st, inputs_of(a), a.deal_out);
     return hipErrorInvalidValue;
 }
 hipError_t f32_mfma_tdp_bwd_first_tile(const FirstTileArgs& a, hipStream_t st) {

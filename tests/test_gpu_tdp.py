@@ -1219,3 +1219,17 @@ def test_narrow_windows_of_16_bit_tensors_in_fp32(D, splits, wanted, tune):
         if a is not None:
             util.assert_mostly_close(name, a.float().cpu(), want, **LOWP)
             assert util.rel_err(a.float().cpu(), want) <= 2e-2, name
+
+
+@pytest.mark.parametrize("tiles", [511, 512])
+def test_narrow_windows_either_side_of_dealing_out(tiles):
+    """The grid sizes around the rule that deals the tiles of such a mask out (dQ through an accumulator) or walks each in
+    one workgroup."""
+    windows, alpha = (16, 16, 8, 8), 0.125
+    inputs = orc.make_inputs(1, tiles // 7 if tiles == 511 else tiles // 8, 224 if tiles == 511 else 250, 64, torch.bfloat16, seed=3)
+    assert inputs[0].shape[1] * ((inputs[0].shape[2] + 31) // 32) == tiles
+    _, g = util.run_tdp(inputs, alpha, True, windows)
+    for h in (0, 31, inputs[0].shape[1] - 1):
+        _, _, grads = util.oracle_tdp([t[:, h:h + 1] for t in inputs], alpha, True, windows)
+        for name, a, want in zip(util.NAMES, g, grads):
+            util.assert_mostly_close(f"{name}[{h}]", a[:, h:h + 1], want, **LOWP)
