@@ -1233,3 +1233,41 @@ def test_narrow_windows_either_side_of_dealing_out(tiles):
         _, _, grads = util.oracle_tdp([t[:, h:h + 1] for t in inputs], alpha, True, windows)
         for name, a, want in zip(util.NAMES, g, grads):
             util.assert_mostly_close(f"{name}[{h}]", a[:, h:h + 1], want, **LOWP)
+
+
+@pytest.mark.parametrize("B,H,T,D,splits", [(1, 2, 64, 32, 0), (2, 4, 100, 64, 0), (1, 3, 97, 128, 1)])
+def test_fp32_training_step_replays_from_a_hip_graph(B, H, T, D, splits, tune):
+    """The fp32 backward clears what its workgroups add to and forms its scales in every call: replays on inputs of another
+    size each, with eager calls in between, are the eager results bit for bit."""
+    from flash_trittention.triple_dot_product.flash_trittention import flash_trittention
+
+    tune(_lib.TUNE_BWD_SPLITS, splits)
+    full = dict(softmax_scale=1 / math.sqrt(D), k1_window=None, k2_window=None, kk_left=None, kk_right=None)
+    static = [t.cuda().requires_grad_(True) for t in orc.make_inputs(B, H, T, D, torch.float32, seed=1)[:5]]
+    static_do = torch.zeros(B, H, T, D, device="cuda")
+
+    def step():
+        out = flash_trittention(*static, **full)
+        return out, *torch.autograd.grad(out, static, static_do)
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for _ in range(3):
+            step()
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = step()
+    for rep, c in enumerate((1.0, 1e-2, 30.0, 1.0)):
+        fresh = orc.make_inputs(B, H, T, D, torch.float32, seed=10 + rep)
+        with torch.no_grad():
+            for dst, src in zip(static, fresh[:5]):
+                dst.copy_(src * min(c, 2.0))
+            static_do.copy_(fresh[5] * c)
+        graph.replay()
+        torch.cuda.synchronize()
+        got = [t.clone() for t in captured]
+        for name, a, b in zip(("out",) + util.NAMES, got, step()):
+            assert torch.equal(a, b), (name, rep)
