@@ -168,9 +168,9 @@ struct F32Inputs {
     const float *q, *k1, *k2, *u, *v2;
 };
 F32Inputs plan_inputs(Arena& ar, const void* q, const void* k1, const void* k2, const void* v2, size_t n, int dtype,
-                      float** copies /* [4] scratch or null */, float** u) {
+                      float** copies /* [4] scratch or null */, float** u, bool need_u = true) {
     F32Inputs r{};
-    *u = ar.take<float>(n);
+    *u = need_u ? ar.take<float>(n) : nullptr;
     r.u = *u;
     if (dtype == TRITT_F32) {
         r.q = (const float*)q; r.k1 = (const float*)k1; r.k2 = (const float*)k2; r.v2 = (const float*)v2;
@@ -198,15 +198,22 @@ int clampw(int w, int T) { return w > T ? T : w; }
 // rounds of a query tile out over workgroups and are the faster ones at every size (B=1 H=1 T=16 D=64: forward 14 against
 // 27 us, backward 32 against 200 us), and on the vector ALUs (D = 8 and 16, and TRITT_TUNE_F32_VALU).
 bool use_f32_mfma() { return knobs().f32_valu == 0; }
-// room for the parts of a split fp32 matrix-core forward; a problem whose other scratch fits the library's static buffer
-// (tritt_tdp_fwd_static_scratch) takes no more parts than still fit
-void plan_f32_parts(Arena& ar, GenericTdpArgs& a) {
+// Scratch of an fp32 matrix-core forward beyond its operands: the images of the streamed tensors, unless the problem is so
+// short that they would cost more than they save, and the parts of a split one.  `compact` (tritt_tdp_fwd_static_scratch, for
+// problems whose images do not fit the library's static buffer): no images, and no more parts than still fit.
+bool f32_fwd_has_images(GenericTdpArgs a, int dtype) {
+    a.fwd_parts = f32_fwd_parts(a);
+    return dtype != TRITT_F32 || !f32_fwd_takes_v1(a);
+}
+void plan_f32_fwd(Arena& ar, GenericTdpArgs& a, int dtype, bool compact) {
     a.fwd_parts = 1;
     a.part = nullptr;
+    a.images = nullptr;
     if (!f32_mfma_tdp_supported(a.D) || !use_f32_mfma()) return;
+    if (!compact && f32_fwd_has_images(a, dtype)) a.images = ar.take<char>(f32_fwd_image_bytes(a));
     const size_t per_part = (size_t)a.BH * a.T * f32_fwd_part_floats(a.D) * sizeof(float), used = ar.bytes();
     size_t parts = (size_t)f32_fwd_parts(a);
-    if (used <= TRITT_STATIC_SCRATCH_BYTES) parts = std::min(parts, (TRITT_STATIC_SCRATCH_BYTES - used) / per_part);
+    if (compact) parts = std::min(parts, used < TRITT_STATIC_SCRATCH_BYTES ? (TRITT_STATIC_SCRATCH_BYTES - used) / per_part : 0);
     if (parts < 2) return;
     a.fwd_parts = (int)parts;
     a.part = ar.take<float>(parts * per_part / sizeof(float));
@@ -215,21 +222,23 @@ void plan_f32_parts(Arena& ar, GenericTdpArgs& a) {
 // ---------------------------------------------------------------- triple-dot, fp32 VALU path
 int tdp_fwd_generic(Arena& ar, bool run, const void* q, const void* k1, const void* k2, const void* v1,
                     const void* v2, void* o, float* lse, int B, int H, int T, int D, int dtype, float alpha,
-                    int causal, int w1, int w2, int kl, int kr, hipStream_t st) {
+                    int causal, int w1, int w2, int kl, int kr, hipStream_t st, bool compact) {
     const size_t n = (size_t)B * H * T * D;
-    float *copies[4], *u;
-    F32Inputs in = plan_inputs(ar, q, k1, k2, v2, n, dtype, copies, &u);
-    float* o32 = dtype == TRITT_F32 ? (float*)o : ar.take<float>(n);
     GenericTdpArgs a{};
     a.BH = B * H; a.T = T; a.D = D; a.alpha = alpha;
     a.causal = causal; a.k1_window = w1; a.k2_window = w2; a.kk_left = kl; a.kk_right = kr;
-    plan_f32_parts(ar, a);
+    const bool mfma32 = f32_mfma_tdp_supported(D) && use_f32_mfma();
+    // with images SiLU(V1) is one of them; a short problem's kernel applies SiLU itself (unless `compact` took parts away)
+    float *copies[4], *u;
+    F32Inputs in = plan_inputs(ar, q, k1, k2, v2, n, dtype, copies, &u,
+                               !mfma32 || dtype != TRITT_F32 || compact || !f32_fwd_has_images(a, dtype));
+    float* o32 = dtype == TRITT_F32 ? (float*)o : ar.take<float>(n);
+    plan_f32_fwd(ar, a, dtype, compact);
     if (!run) return TRITT_OK;
     if (ar.overflows()) return TRITT_ERR_WORKSPACE;
-    const bool mfma32 = f32_mfma_tdp_supported(D) && use_f32_mfma();
     a.q = in.q; a.k1 = in.k1; a.k2 = in.k2; a.u = in.u; a.v2 = in.v2;
     a.o = o32; a.lse = lse;
-    if (mfma32 && dtype == TRITT_F32 && f32_fwd_takes_v1(a)) {
+    if (mfma32 && dtype == TRITT_F32 && (a.images || f32_fwd_takes_v1(a))) {
         a.u = (const float*)v1;
         a.u_is_v1 = 1;
     } else {
@@ -259,7 +268,7 @@ int tdp_bwd_generic(Arena& ar, bool run, const void* q, const void* k1, const vo
     GenericTdpArgs a{};
     a.BH = B * H; a.T = T; a.D = D; a.alpha = alpha;
     a.causal = causal; a.k1_window = w1; a.k2_window = w2; a.kk_left = kl; a.kk_right = kr;
-    if (dtype != TRITT_F32) plan_f32_parts(ar, a);  // (o32 is null while measuring)
+    if (dtype != TRITT_F32) plan_f32_fwd(ar, a, dtype, false);  // (o32 is null while measuring)
     long long* fixed = mfma32 ? ar.take<long long>(f32_mfma_tdp_bwd_scratch_elems(a)) : nullptr;
     // VALU kernels: fp32 results, the caller's tensors when they are fp32, scratch otherwise; `spare` stands in for the
     // unwanted (null) half of a gradient pair whose other half is wanted (one kernel writes both halves)
@@ -622,21 +631,27 @@ static MfmaFwdArgs mfma_fwd_shape(int B, int H, int T, int D, int dtype, int cau
     return a;
 }
 
-size_t tritt_tdp_fwd_workspace_bytes(int B, int H, int T, int D, int dtype, int causal, int k1_window, int k2_window,
-                                     int kk_left, int kk_right, unsigned flags) {
+// compact: see plan_f32_fwd
+static size_t tdp_fwd_bytes(int B, int H, int T, int D, int dtype, int causal, int k1_window, int k2_window, int kk_left,
+                            int kk_right, unsigned flags, bool compact) {
     if (check_common(B, H, T, D, dtype) != TRITT_OK) return 0;
     if (use_mfma_fwd(T, D, dtype, causal, k1_window, k2_window, kk_left, kk_right, flags))
         return mfma_tdp_fwd_workspace(mfma_fwd_shape(B, H, T, D, dtype, causal, k1_window, k2_window, kk_left, kk_right, flags));
     Arena ar(nullptr);
     tdp_fwd_generic(ar, false, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, B, H, T, D, dtype, 0.f,
-                    causal, k1_window, k2_window, kk_left, kk_right, nullptr);
-    (void)flags;
+                    causal, k1_window, k2_window, kk_left, kk_right, nullptr, compact);
     return ar.bytes();
 }
 
-int tritt_tdp_fwd(const void* q, const void* k1, const void* k2, const void* v1, const void* v2, void* o, float* lse,
-                  int B, int H, int T, int D, int dtype, float alpha, int causal, int k1_window, int k2_window,
-                  int kk_left, int kk_right, void* workspace, size_t workspace_bytes, unsigned flags, void* stream) {
+size_t tritt_tdp_fwd_workspace_bytes(int B, int H, int T, int D, int dtype, int causal, int k1_window, int k2_window,
+                                     int kk_left, int kk_right, unsigned flags) {
+    return tdp_fwd_bytes(B, H, T, D, dtype, causal, k1_window, k2_window, kk_left, kk_right, flags, false);
+}
+
+static int tdp_fwd_call(const void* q, const void* k1, const void* k2, const void* v1, const void* v2, void* o, float* lse,
+                        int B, int H, int T, int D, int dtype, float alpha, int causal, int k1_window, int k2_window,
+                        int kk_left, int kk_right, void* workspace, size_t workspace_bytes, unsigned flags, void* stream,
+                        bool compact) {
     if (empty_problem(B, H, T)) return check_common(1, 1, 1, D, dtype);
     int rc = check_common(B, H, T, D, dtype);
     if (rc != TRITT_OK) return rc;
@@ -648,7 +663,7 @@ int tritt_tdp_fwd(const void* q, const void* k1, const void* k2, const void* v1,
     if ((flags & TRITT_FLAG_FORCE_MFMA) && !mfma) return TRITT_ERR_UNSUPPORTED;
     // the caller sized `o` for two tensors: a path that writes one would leave the residual undefined
     if ((flags & TRITT_FLAG_SPLIT_OPERANDS) && !(mfma && use_split(D, dtype, flags))) return TRITT_ERR_UNSUPPORTED;
-    const size_t need = tritt_tdp_fwd_workspace_bytes(B, H, T, D, dtype, causal, w1, w2, kl, kr, flags);
+    const size_t need = tdp_fwd_bytes(B, H, T, D, dtype, causal, w1, w2, kl, kr, flags, compact);
     if (need && (!workspace || workspace_bytes < need)) return TRITT_ERR_WORKSPACE;
     if (mfma) {
         MfmaFwdArgs a = mfma_fwd_shape(B, H, T, D, dtype, causal, w1, w2, kl, kr, flags);
@@ -658,7 +673,14 @@ int tritt_tdp_fwd(const void* q, const void* k1, const void* k2, const void* v1,
     }
     Arena ar(workspace, workspace_bytes);
     return tdp_fwd_generic(ar, true, q, k1, k2, v1, v2, o, lse, B, H, T, D, dtype, alpha, causal, w1, w2, kl, kr,
-                           (hipStream_t)stream);
+                           (hipStream_t)stream, compact);
+}
+
+int tritt_tdp_fwd(const void* q, const void* k1, const void* k2, const void* v1, const void* v2, void* o, float* lse,
+                  int B, int H, int T, int D, int dtype, float alpha, int causal, int k1_window, int k2_window,
+                  int kk_left, int kk_right, void* workspace, size_t workspace_bytes, unsigned flags, void* stream) {
+    return tdp_fwd_call(q, k1, k2, v1, v2, o, lse, B, H, T, D, dtype, alpha, causal, k1_window, k2_window, kk_left, kk_right,
+                        workspace, workspace_bytes, flags, stream, false);
 }
 
 size_t tritt_static_scratch_bytes(void) { return TRITT_STATIC_SCRATCH_BYTES; }
@@ -670,16 +692,18 @@ int tritt_tdp_fwd_static_scratch(const void* q, const void* k1, const void* k2, 
     if (empty_problem(B, H, T)) return check_common(1, 1, 1, D, dtype);
     int rc = check_common(B, H, T, D, dtype);
     if (rc != TRITT_OK) return rc;
-    const size_t need = tritt_tdp_fwd_workspace_bytes(B, H, T, D, dtype, causal, k1_window, k2_window, kk_left,
-                                                      kk_right, flags);
-    if (need > TRITT_STATIC_SCRATCH_BYTES) return TRITT_ERR_SCRATCH_LIMIT;
+    auto need = [&](bool compact) {
+        return tdp_fwd_bytes(B, H, T, D, dtype, causal, k1_window, k2_window, kk_left, kk_right, flags, compact);
+    };
+    const bool compact = need(false) > TRITT_STATIC_SCRATCH_BYTES;
+    if (compact && need(true) > TRITT_STATIC_SCRATCH_BYTES) return TRITT_ERR_SCRATCH_LIMIT;
     void* ws = nullptr;
     rc = static_scratch(&ws);
     if (rc != TRITT_OK) return rc;
     // every kernel of the forward writes the part of the scratch it later reads (the transposed SiLU(V1) copy
     // including its zero padding, the parts of a split forward): nothing has to be cleared between calls
-    return tritt_tdp_fwd(q, k1, k2, v1, v2, o, lse, B, H, T, D, dtype, alpha, causal, k1_window, k2_window, kk_left,
-                         kk_right, ws, TRITT_STATIC_SCRATCH_BYTES, flags, stream);
+    return tdp_fwd_call(q, k1, k2, v1, v2, o, lse, B, H, T, D, dtype, alpha, causal, k1_window, k2_window, kk_left, kk_right, ws,
+                        TRITT_STATIC_SCRATCH_BYTES, flags, stream, compact);
 }
 
 size_t tritt_tdp_bwd_workspace_bytes(int B, int H, int T, int D, int dtype, int causal, int k1_window, int k2_window,

@@ -46,7 +46,8 @@ struct GenericTdpArgs {
     // fp32 MFMA forward: workgroups per query tile at most (f32_fwd_parts) and, above 1, room for that many parts per row
     int fwd_parts;
     float* part;
-    int u_is_v1;  // forward: `u` is V1 and the kernel applies SiLU (where f32_fwd_takes_v1 says it may)
+    void* images;  // forward: room for the streamed tensors' images (f32_fwd_image_bytes), or null: they are split as they are staged
+    int u_is_v1;  // forward: `u` is V1 and SiLU is applied here (with images, or where f32_fwd_takes_v1 says so)
 };
 hipError_t generic_tdp_fwd(const GenericTdpArgs& a, hipStream_t st);
 hipError_t generic_tdp_bwd(const GenericTdpArgs& a, hipStream_t st);
@@ -57,6 +58,7 @@ bool f32_mfma_tdp_supported(int D);
 int f32_fwd_parts(const GenericTdpArgs& a);
 bool f32_fwd_takes_v1(const GenericTdpArgs& a);
 size_t f32_fwd_part_floats(int D);  // scratch per row and part
+size_t f32_fwd_image_bytes(const GenericTdpArgs& a);
 hipError_t f32_mfma_tdp_fwd(const GenericTdpArgs& a, hipStream_t st);
 // The backward: `a` holds the fp32 operands (u: written by the call when v1_f32 is given), lse_in and d_o; the gradients come
 // out in the caller's type.

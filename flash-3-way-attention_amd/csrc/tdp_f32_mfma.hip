@@ -24,7 +24,7 @@
 #include "common.hpp"
 #include "kernels.hpp"
 #include "mfma.hpp"
-#include "tdp_f32_tiles.hpp"
+#include "tdp_f32_split.hpp"
 
 namespace tritt {
 namespace {
@@ -142,7 +142,7 @@ __global__ __launch_bounds__(256) void f32_finish_kernel(const long long* __rest
 }
 
 // waves per workgroup
-constexpr int f32_fwd_waves(int D) { return D > 64 ? 8 : 4; }
+constexpr int f32_fwd_waves(int D) { return 4; }
 constexpr int f32_bwd_waves(int D) { return D > 64 ? 8 : 4; }
 
 // Joins the parts of a split forward, four columns per thread.
@@ -309,24 +309,28 @@ hipError_t launch_f32_bwd(const F32BwdCall& c, hipStream_t st) {
 F32Deal f32_fwd_deal(const GenericTdpArgs& a, int most) {
     auto w = [&](int x) { return std::min(x, a.T); };
     const TdpMask mask{a.causal, w(a.k1_window), w(a.k2_window), w(a.kk_left), w(a.kk_right)};
-    return f32_deal(mask, a.BH, a.T, f32_fwd_waves(a.D), a.D > 64 ? 256 : 768, knobs().fwd_splits > 0 ? std::min(knobs().fwd_splits, most) : most);
+    return f32_deal(mask, a.BH, a.T, f32_fwd_waves(a.D), a.D > 64 ? 256 : 512, knobs().fwd_splits > 0 ? std::min(knobs().fwd_splits, most) : most);
 }
 
 template <int D>
 hipError_t launch_f32_fwd(const GenericTdpArgs& a, hipStream_t st) {
-    F32Params<float> p{};
+    F32FwdParams p{};
     p.q = a.q; p.ka = a.k1; p.kb = a.k2; p.va = a.u; p.vb = a.v2;
-    place_inputs(p, dense_inputs(a.T, D), false);
     p.o = a.o; p.lse = a.lse;
-    p.d_o = nullptr; p.delta = nullptr; p.split_rounds = 0; p.zero_ptr = nullptr; p.zero_words = 0; p.deal = F32Deal{0.f, 1, p.nqt}; p.silu_va = a.u_is_v1 != 0;
+    p.silu_va = a.u_is_v1;
     p.T = a.T; p.BH = a.BH; p.nqt = (a.T + 31) / 32;
     p.scale_log2 = a.alpha * kLog2e;
     p.mask = TdpMask{a.causal, a.k1_window, a.k2_window, a.kk_left, a.kk_right};
     p.deal = a.part ? f32_fwd_deal(a, a.fwd_parts) : F32Deal{0.f, 1, p.nqt};
     p.part = a.part;
     constexpr int NW = f32_fwd_waves(D);
-    auto kern = tdp_f32_fwd_kernel<float, D, false, NW>;
-    constexpr size_t smem = f32_fwd_smem<D, NW>();
+    if (a.images) {
+        __bf16 *ka = (__bf16*)a.images, *va = ka + split_image_elems<D>(a.BH, a.T);
+        hipLaunchKernelGGL(f32_split_images_kernel<D>, dim3(p.nqt, a.BH, 2), dim3(256), 0, st, a.k1, a.u, ka, va, a.u_is_v1, a.T);
+        p.image_ka = ka; p.image_va = va;
+    }
+    auto kern = a.images ? tdp_f32_split_fwd_kernel<D, NW, true> : tdp_f32_split_fwd_kernel<D, NW, false>;
+    constexpr size_t smem = f32_split_fwd_smem<D, NW>();
     if (hipError_t e = ensure_dynamic_smem(reinterpret_cast<const void*>(kern), smem); e != hipSuccess) return e;
     hipLaunchKernelGGL(kern, dim3(8 * xcd_slots(a.BH, p.deal.items)), dim3(64 * NW), smem, st, p);
     if (p.deal.max_parts > 1) {
@@ -346,6 +350,9 @@ bool f32_fwd_takes_v1(const GenericTdpArgs& a) {
     return d.inv_target >= 0.25f && (long long)a.BH * d.items <= 768;
 }
 int f32_fwd_parts(const GenericTdpArgs& a) { return f32_fwd_deal(a, 16).max_parts; }
+size_t f32_fwd_image_bytes(const GenericTdpArgs& a) {
+    return 2 * sizeof(__bf16) * (a.D == 32 ? split_image_elems<32>(a.BH, a.T) : a.D == 64 ? split_image_elems<64>(a.BH, a.T) : split_image_elems<128>(a.BH, a.T));
+}
 size_t f32_fwd_part_floats(int D) { return D + 4; }
 
 bool f32_mfma_tdp_supported(int D) { return D == 32 || D == 64 || D == 128; }
@@ -353,16 +360,16 @@ bool f32_mfma_tdp_supported(int D) { return D == 32 || D == 64 || D == 128; }
 // The first query tiles of a 16-bit backward, in fp32 (see the comment above tdp_f32_bwd_kernel).
 template <typename E, int D>
 static hipError_t launch_stats(const FirstTileArgs& a, hipStream_t st) {
-    F32Params<E> p{};
+    F32StatsParams<E> p{};
     p.q = (const E*)a.q; p.ka = (const E*)a.k1; p.kb = (const E*)a.k2; p.va = (const E*)a.u; p.vb = (const E*)a.v2;
     place_inputs(p, inputs_of(a), false);
-    p.o = nullptr; p.lse = a.lse_f32; p.d_o = (const E*)a.d_o; p.delta = a.delta_f32;
-    p.split_rounds = 0; p.zero_ptr = nullptr; p.zero_words = 0; p.deal = F32Deal{0.f, 1, p.nqt}; p.silu_va = false;
+    p.lse = a.lse_f32; p.d_o = (const E*)a.d_o; p.delta = a.delta_f32;
+    p.split_rounds = 0; p.zero_ptr = nullptr; p.zero_words = 0;
     p.T = a.T; p.BH = a.BH; p.nqt = a.tiles;
     p.scale_log2 = a.alpha * kLog2e;
     p.mask = TdpMask{a.causal, a.k1_window, a.k2_window, a.kk_left, a.kk_right};
-    auto kern = tdp_f32_fwd_kernel<E, D, true, kF32Waves>;
-    constexpr size_t smem = f32_fwd_smem<D, kF32Waves>();
+    auto kern = tdp_f32_stats_kernel<E, D, kF32Waves>;
+    constexpr size_t smem = f32_stats_smem<D, kF32Waves>();
     if (hipError_t e = ensure_dynamic_smem(reinterpret_cast<const void*>(kern), smem); e != hipSuccess) return e;
     hipLaunchKernelGGL(kern, dim3(8 * xcd_slots(a.BH, p.nqt)), dim3(512), smem, st, p);
     return hipGetLastError();

@@ -71,30 +71,24 @@ __device__ __forceinline__ F32Item f32_item(const F32Deal& d, const TdpMask& m, 
     return it;
 }
 
+// statistics of the 16-bit backward's fp32 tiles: lse receives the fp32 log-sum-exp of the covered rows and delta their
+// rowsum(dO * O) with O in fp32
 template <typename E>
-struct F32Params {
+struct F32StatsParams {
     const E *q, *ka, *kb, *va, *vb;  // streamed = (ka, va), rows = (kb, vb)
     // where these five and d_o lie: H heads per batch entry and each tensor's strides (dense tensors: H = 1 and
-    // sb = T D, st = D); the outputs are dense
+    // sb = T D, st = D)
     int H;
     TensorAt at_q, at_ka, at_kb, at_va, at_vb, at_do;
-    E* o;
     float* lse;
-    // STATS mode (the 16-bit backward's fp32 tiles): O is not written; lse receives the fp32 log-sum-exp of the
-    // covered rows and delta their rowsum(dO * O) with O in fp32
     const E* d_o;
     float* delta;
-    // STATS over query tile 0 with the rounds dealt out to `split_rounds` workgroups (blockIdx.y): each writes its
+    // Query tile 0 alone, with its rounds dealt out to `split_rounds` workgroups (blockIdx.y): each writes its
     // partial (maximum, sum, sum_d dO * unnormalised O) to delta[((bh * 32 + q) * split_rounds + round) * 3 ..] and
     // the first one clears `zero_words` 4-byte words at zero_ptr + bh * zero_words
     int split_rounds;
     unsigned* zero_ptr;
     int zero_words;
-    bool silu_va;  // va is V1 itself: SiLU is applied as its stages go to LDS (not with STATS)
-    // deal.max_parts > 1 (never with STATS): the rounds of a tile are dealt out to f32_tile_parts() workgroups; each leaves
-    // its unnormalised output, reference maximum and row sum in part[((bh T + q) max_parts + y) (D + 4)] (O[D], M, L)
-    F32Deal deal;
-    float* part;
     int T, BH, nqt;  // nqt: query tiles this launch covers (tiles 0 .. nqt - 1)
     float scale_log2;
     TdpMask mask;  // in terms of the streamed index a and the row index b
@@ -133,13 +127,12 @@ __device__ __forceinline__ void stage_fetch_e(StageE<E, D, NW>& r, const E* __re
     }
 }
 template <typename E, int D, int NW>
-__device__ __forceinline__ void stage_store_e(const StageE<E, D, NW>& r, float* sk, float* sv, bool silu_v = false) {
+__device__ __forceinline__ void stage_store_e(const StageE<E, D, NW>& r, float* sk, float* sv) {
     using S = StageE<E, D, NW>;
     constexpr int kVec = D / S::VE, LD = D + 4;  // f32_pitch<D>()
     const int t = threadIdx.x & (S::kThreads - 1);
     const bool first = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) < NW / 2;
     float* dst = first ? sk : sv;
-    const bool silu = silu_v && !first;
 #pragma unroll
     for (int i = 0; i < S::kPer; ++i) {
         const int idx = t + i * S::kThreads;
@@ -151,10 +144,6 @@ __device__ __forceinline__ void stage_store_e(const StageE<E, D, NW>& r, float* 
             for (int k = 0; k < S::VE; k += 4) {
                 typedef __attribute__((ext_vector_type(4))) float f4;
                 f4 v = {(float)e[k], (float)e[k + 1], (float)e[k + 2], (float)e[k + 3]};
-                if (silu) {
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) v[j] = silu_f(v[j]);
-                }
                 *reinterpret_cast<f4*>(p + k) = v;
             }
         }
@@ -220,20 +209,13 @@ __device__ __forceinline__ bool open_round(Walk& w, const TdpMask& mask, int m, 
     return false;
 }
 
-// ------------------------------------------------------------------------------------------ forward
-// What bounds it: the fp32 matrix pipe, which fp32 MFMAs (64 cycles each) and vector instructions use in turn -- measured
-// busy(MFMA) + busy(VALU) = 97 % of the cycles -- so every vector instruction of the loop counts, and waves of different
-// workgroups have to fill each other's waits.  Hence: a workgroup is four waves (D <= 64; one per SIMD) that fit 168
-// registers, three workgroups to a CU; the B operand of the score product is formed once per round and held; the maximum is
-// only formed when a sum outgrows its reference; tiles inside the mask skip it; stages are fetched from a scalar base at
-// constant lane offsets.  Operand reads are as wide as the layout allows: the k-slots of four consecutive MFMAs are four
-// consecutive d (16 bytes of a row), and output row r of value tile dt is column d = DT r + dt, so that the operands of the
-// DT value tiles are DT consecutive columns.  Stages and row operands are fetched one step ahead across the rounds' ends,
-// one barrier per step.  B=4 H=8 T=512 D=64: 5.94 -> 3.26 ms (113 TFLOP/s, 72 % of the fp32 matrix rate), of which the parts
-// (F32Deal) make 2.4; B=2 H=4 T=500: 5.38 -> 0.88 ms.  Eight waves with the operand formed as it is used and 128 registers
-// (two workgroups to a CU) measured 3.49 ms, eight with it held (one workgroup) 3.66.
-template <typename E, int D, bool STATS, int NW>
-__global__ __launch_bounds__(64 * NW, NW == 8 ? 2 : 3) void tdp_f32_fwd_kernel(F32Params<E> p) {
+// ------------------------------------------------------------------------------------------ statistics
+// The forward over the fp32 query tiles of a 16-bit backward, for their log-sum-exp and Delta (F32StatsParams).  Operand reads
+// are as wide as the layout allows: the k-slots of four consecutive MFMAs are four consecutive d (16 bytes of a row), and
+// output row r of value tile dt is column d = DT r + dt, so that the operands of the DT value tiles are DT consecutive columns.
+// Stages and row operands are fetched one step ahead across the rounds' ends, one barrier per step.
+template <typename E, int D, int NW>
+__global__ __launch_bounds__(64 * NW, 2) void tdp_f32_stats_kernel(F32StatsParams<E> p) {
     constexpr int DT = D / 32, LD = f32_pitch<D>(), NT = 64 * NW;
     constexpr bool HOLD = D <= 64;
     using vDT = typename VecF<DT>::type;
@@ -248,15 +230,12 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 2 : 3) void tdp_f32_fwd_kernel(F
     float* sO = sK;                     // [NW][D][33] end of kernel: the waves' outputs (alias everything from the stages on)
 
     int bh, order;
-    if (!xcd_tile(p.BH, STATS ? p.nqt : p.deal.items, blockIdx.x >> 3, blockIdx.x & 7, bh, order)) return;
-    const F32Item item = STATS ? F32Item{p.nqt - 1 - order, 0, 1} : f32_item(p.deal, p.mask, order, p.nqt, p.T, NW);
-    const int qt = item.qt, part = item.part, step = item.parts;
-    if (part >= step) return;
+    if (!xcd_tile(p.BH, p.nqt, blockIdx.x >> 3, blockIdx.x & 7, bh, order)) return;
+    const int qt = p.nqt - 1 - order;
 
     const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int T = p.T;
-    const size_t base = (size_t)bh * T * D;
     const int b_ = bh / p.H, h_ = bh % p.H;
     auto slice = [&](const E* t, const TensorAt& at) { return t + (size_t)b_ * at.sb + (size_t)h_ * at.sh; };
     const E* __restrict__ KA = slice(p.ka, p.at_ka);
@@ -269,9 +248,8 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 2 : 3) void tdp_f32_fwd_kernel(F
     const int q0 = qt * 32, q1 = min(T - 1, q0 + 31);
     const int q = q0 + n;  // this lane's query (column of every tile)
     const Range rows = row_range(mask, q0, q1, T);
-    // rounds of NW rows: workgroup `part` of a tile takes every step-th one from the part-th on
-    int m_lo = rows.lo / NW + part, m_hi = rows.hi / NW;
-    if (STATS && p.split_rounds) {
+    int m_lo = rows.lo / NW, m_hi = rows.hi / NW;  // rounds of NW rows
+    if (p.split_rounds) {
         m_lo = max(m_lo, (int)blockIdx.y);  // this workgroup's round only (none at all if it is out of range)
         m_hi = min(m_hi, (int)blockIdx.y);
         if (blockIdx.y == 0)
@@ -310,7 +288,7 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 2 : 3) void tdp_f32_fwd_kernel(F
     };
 
     Walk w{};
-    bool have = open_round<NW>(w, mask, m_lo, m_hi, step, q0, q1, T);
+    bool have = open_round<NW>(w, mask, m_lo, m_hi, 1, q0, q1, T);
     if (have) {
         fetch_rows(w.m);
         stage_fetch_e<E, D, NW>(regs, KA, VA, w.st * 32, T, p.at_ka.st, p.at_va.st);
@@ -321,7 +299,7 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 2 : 3) void tdp_f32_fwd_kernel(F
     }
     if (have) {
         store_rows(0);
-        stage_store_e<E, D, NW>(regs, sK, sV, !STATS && p.silu_va);
+        stage_store_e<E, D, NW>(regs, sK, sV);
     }
     __syncthreads();
 
@@ -333,7 +311,7 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 2 : 3) void tdp_f32_fwd_kernel(F
         const float* cV = sV + buf * 32 * LD;
         const bool last = w.st == w.st_hi;  // of this round
         Walk nw{w.m, w.st + 1, w.st_hi};
-        const bool more = last ? open_round<NW>(nw, mask, w.m + step, m_hi, step, q0, q1, T) : true;
+        const bool more = last ? open_round<NW>(nw, mask, w.m + 1, m_hi, 1, q0, q1, T) : true;
         if (more) {
             stage_fetch_e<E, D, NW>(regs, KA, VA, nw.st * 32, T, p.at_ka.st, p.at_va.st);
             if (last) fetch_rows(nw.m);
@@ -446,7 +424,7 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 2 : 3) void tdp_f32_fwd_kernel(F
                 par ^= 1;
                 store_rows(par);
             }
-            stage_store_e<E, D, NW>(regs, sK + buf * 32 * LD, sV + buf * 32 * LD, !STATS && p.silu_va);
+            stage_store_e<E, D, NW>(regs, sK + buf * 32 * LD, sV + buf * 32 * LD);
             __syncthreads();
         }
         w = nw;
@@ -480,53 +458,28 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 2 : 3) void tdp_f32_fwd_kernel(F
     float L = 0.f;
 #pragma unroll
     for (int w = 0; w < NW; ++w) L += sL[w * 32 + n] * fast_exp2(sM[w * 32 + n] - M);
-    if constexpr (STATS) {
-        // Delta[q] = sum_d dO[q, d] O[q, d] with O in fp32: two threads of every wave per query, joined through LDS
-        float* red = sQ;  // [2 NW][32]
-        const int k16 = wave * 2 + g;
-        float dsum = 0.f;
-        if (q < T) {
-            const E* dor = slice(p.d_o, p.at_do) + (size_t)q * p.at_do.st;
-            for (int d = k16; d < D; d += 2 * NW) dsum += (float)dor[d] * merged(d, n);
-        }
-        red[k16 * 32 + n] = dsum;
-        __syncthreads();
-        if (wave == 0 && g == 0 && q < T) {
-            dsum = 0.f;
+    // Delta[q] = sum_d dO[q, d] O[q, d] with O in fp32: two threads of every wave per query, joined through LDS
+    float* red = sQ;  // [2 NW][32]
+    const int k16 = wave * 2 + g;
+    float dsum = 0.f;
+    if (q < T) {
+        const E* dor = slice(p.d_o, p.at_do) + (size_t)q * p.at_do.st;
+        for (int d = k16; d < D; d += 2 * NW) dsum += (float)dor[d] * merged(d, n);
+    }
+    red[k16 * 32 + n] = dsum;
+    __syncthreads();
+    if (wave == 0 && g == 0 && q < T) {
+        dsum = 0.f;
 #pragma unroll
-            for (int k = 0; k < 2 * NW; ++k) dsum += red[k * 32 + n];
-            if (p.split_rounds) {
-                float* part = p.delta + (((size_t)bh * 32 + n) * p.split_rounds + blockIdx.y) * 3;
-                part[0] = M; part[1] = L; part[2] = dsum;
-            } else {
-                p.delta[(size_t)bh * T + q] = dsum / L;
-            }
-        }
-        if (p.split_rounds) return;
-    } else if (p.deal.max_parts > 1) {
-        // perhaps one of several workgroups of the tile: its unnormalised output, reference and sum (f32_merge_kernel)
-        for (int idx = tid; idx < 32 * D; idx += NT) {
-            const int r = idx / D, d = idx % D;
-            if (q0 + r < T) p.part[(((size_t)bh * T + q0 + r) * p.deal.max_parts + part) * (D + 4) + d] = merged(d, r);
-        }
-        if (wave == 0 && g == 0 && q < T) {
-            float* ml = p.part + (((size_t)bh * T + q) * p.deal.max_parts + part) * (D + 4) + D;
-            ml[0] = M; ml[1] = L;
-        }
-        return;
-    } else {
-        for (int idx = tid; idx < 32 * D; idx += NT) {
-            const int r = idx / D, d = idx % D;
-            if (q0 + r < T) {
-                float Lr = 0.f, Mr = kNegBig;
-#pragma unroll
-                for (int w = 0; w < NW; ++w) Mr = fmaxf(Mr, sM[w * 32 + r]);
-#pragma unroll
-                for (int w = 0; w < NW; ++w) Lr += sL[w * 32 + r] * fast_exp2(sM[w * 32 + r] - Mr);
-                p.o[base + (size_t)(q0 + r) * D + d] = (E)(merged(d, r) / Lr);
-            }
+        for (int k = 0; k < 2 * NW; ++k) dsum += red[k * 32 + n];
+        if (p.split_rounds) {
+            float* part = p.delta + (((size_t)bh * 32 + n) * p.split_rounds + blockIdx.y) * 3;
+            part[0] = M; part[1] = L; part[2] = dsum;
+        } else {
+            p.delta[(size_t)bh * T + q] = dsum / L;
         }
     }
+    if (p.split_rounds) return;
     if (wave == 0 && g == 0 && q < T) p.lse[(size_t)bh * T + q] = (M + fast_log2(L)) * kLn2;
 }
 
@@ -588,7 +541,7 @@ __device__ __forceinline__ void f32_row_fields(const F32RowScale& s, int BH, int
 template <typename E>
 struct F32BwdParams {
     const E *q, *d_o, *ka, *kb, *va, *vb;
-    int H;  // layouts of the six inputs, as in F32Params
+    int H;  // layouts of the six inputs, as in F32StatsParams
     TensorAt at_q, at_ka, at_kb, at_va, at_vb, at_do;
     const float *lse, *delta;
     E* dq;                 // WITH_DQ, when acc_q is null
@@ -1012,13 +965,13 @@ constexpr size_t f32_bwd_smem() {
 }
 
 template <int D, int NW>
-constexpr size_t f32_fwd_smem() {
+constexpr size_t f32_stats_smem() {
     constexpr int loop = 4 * 32 * f32_pitch<D>() + 4 * NW * D, merge = NW * D * 33;
     return sizeof(float) * (size_t)(2 * NW * 32 + 32 * f32_pitch<D>() + (loop > merge ? loop : merge));
 }
 
 
-// where the six inputs lie (F32Params::H and at_*)
+// where the six inputs lie (F32StatsParams::H and at_*)
 struct InputsAt {
     int H;
     TensorAt q, d_o, k1, u, k2, v2;
@@ -1049,19 +1002,18 @@ hipError_t tile0_prepare(const FirstTileArgs& a, hipStream_t st, F32BwdParams<E>
     const TdpMask natural{a.causal, a.k1_window, a.k2_window, a.kk_left, a.kk_right};
     const bool own_dq_acc = a.want_q && !a.acc_q;  // dQ of the tile is summed over its rounds in a.dq0_acc
     {
-        F32Params<E> p{};
+        F32StatsParams<E> p{};
         p.q = (const E*)a.q; p.ka = (const E*)a.k1; p.kb = (const E*)a.k2; p.va = (const E*)a.u; p.vb = (const E*)a.v2;
         place_inputs(p, inputs_of(a), false);
-        p.o = nullptr; p.lse = nullptr; p.d_o = (const E*)a.d_o; p.delta = a.delta_f32;
+        p.lse = nullptr; p.d_o = (const E*)a.d_o; p.delta = a.delta_f32;
         p.split_rounds = rounds;
         p.zero_ptr = own_dq_acc ? (unsigned*)a.dq0_acc : nullptr;
         p.zero_words = own_dq_acc ? 32 * D * (a.scale_parts ? 2 : 1) : 0;
-        p.deal = F32Deal{0.f, 1, 1}; p.silu_va = false;
         p.T = a.T; p.BH = a.BH; p.nqt = 1;
         p.scale_log2 = a.alpha * kLog2e;
         p.mask = natural;
-        auto kern = tdp_f32_fwd_kernel<E, D, true, kF32Waves>;
-        constexpr size_t smem = f32_fwd_smem<D, kF32Waves>();
+        auto kern = tdp_f32_stats_kernel<E, D, kF32Waves>;
+        constexpr size_t smem = f32_stats_smem<D, kF32Waves>();
         if (hipError_t e = ensure_dynamic_smem(reinterpret_cast<const void*>(kern), smem); e != hipSuccess) return e;
         hipLaunchKernelGGL(kern, dim3(8 * xcd_slots(a.BH, 1), rounds), dim3(512), smem, st, p);
     }

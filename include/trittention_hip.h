@@ -139,11 +139,14 @@ int tritt_tdp_fwd(const void* q, const void* k1, const void* k2, const void* v1,
  * serving loops, harnesses that forbid hipMalloc): the scratch that tritt_tdp_fwd takes as
  * `workspace` lives in a static device array inside the library instead, of
  * TRITT_STATIC_SCRATCH_BYTES bytes per GPU, held until the process ends.  The call allocates
- * and frees nothing.  Problems whose tritt_tdp_fwd_workspace_bytes() exceeds that size are
+ * and frees nothing.  Problems that need more than that are
  * rejected with TRITT_ERR_SCRATCH_LIMIT before anything is launched (32 MiB covers the
- * forward up to B*H*T*D = 16 Mi 16-bit elements, e.g. B=1 H=16 T=4096 D=128).  All calls on
+ * forward up to B*H*T*D = 16 Mi 16-bit elements, e.g. B=1 H=16 T=4096 D=128, and 8 Mi fp32 ones:
+ * where an fp32 problem's tritt_tdp_fwd_workspace_bytes() is larger than the array, the call does
+ * without the copies of the streamed tensors that it is mostly made of).  All calls on
  * one GPU share the one array: calls that overlap in time on the same GPU (different
- * streams or threads) race; serialise them.  Results are identical to tritt_tdp_fwd's.
+ * streams or threads) race; serialise them.  Results are identical to tritt_tdp_fwd's (without
+ * those copies: the same sums, perhaps in other shares, a few fp32 roundings apart).
  * tritt_static_scratch_bytes() returns the limit the library was built with. */
 #define TRITT_STATIC_SCRATCH_BYTES ((size_t)32 << 20)
 size_t tritt_static_scratch_bytes(void);

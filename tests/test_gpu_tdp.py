@@ -1179,6 +1179,37 @@ def test_fp32_gradients_of_a_few_tiles_are_fp32_throughout(B, H, T, D, splits, c
 
 
 @pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("B,H,T", [(1, 1, 1), (3, 1, 31), (1, 3, 33), (2, 2, 97), (1, 9, 160)])
+@pytest.mark.parametrize("mask", ["causal", "none", "windows"])
+def test_fp32_forward_against_64_bits(B, H, T, D, mask):
+    """The forward of fp32 tensors around its 32-row tiles, one and several workgroups per tile, every kind of mask.  A score
+    is a sum of D products of unit variance, each rounded to 24 bits on its own, and the output a weighted mean of what the
+    weights' errors leave: 2^-24 (sqrt(D) + 2) in the norm."""
+    windows = dict(k1_window=37, k2_window=20, kk_left=9, kk_right=40) if mask == "windows" else {}
+    inputs = orc.make_inputs(B, H, T, D, torch.float32, seed=T + D)
+    alpha = 1 / math.sqrt(D)
+    out, _ = util.run_tdp(inputs, alpha, mask != "none", [windows.get(k) for k in ("k1_window", "k2_window", "kk_left", "kk_right")])
+    for b, h in [(0, 0), (B - 1, H - 1)]:
+        z, _, _ = orc.tdp_forward_backward_chunked(*(t[b, h].double() for t in inputs), alpha, mask != "none", need_grads=False, **windows)
+        err = ((out[b, h].double() - z).norm() / z.norm()).item()
+        print(f"    O[{b}, {h}] {B} {H} {T} {D} {mask}: {err:.2e}", flush=True)
+        assert err <= 2.0 ** -24 * (math.sqrt(D) + 2), (b, h, err)
+
+
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+@pytest.mark.parametrize("which", [0, 1, 2, 3, 4])
+def test_fp32_non_finite_operands_stay_with_their_queries(value, which):
+    """A non-finite element leaves the rows that cannot see it untouched and no row that sees it in all its weights finite."""
+    inputs = orc.make_inputs(1, 2, 100, 64, torch.float32, seed=3)
+    good, _ = util.run_tdp(inputs, 0.125, True)
+    inputs[which][0, 1, 40, 5] = value
+    out, _ = util.run_tdp(inputs, 0.125, True)
+    assert torch.equal(out[0, 0], good[0, 0]) and torch.equal(out[0, 1, :32], good[0, 1, :32])
+    hit = out[0, 1, 40:] if which else out[0, 1, 40:41]
+    assert not torch.isfinite(hit[..., 5] if which > 2 else hit).any()
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
 def test_fp32_forward_of_large_values_under_rising_scores(D):
     """Keys whose scores are 2^35 above those of the tile before and values of 1e13 (outputs of 1e26): the unnormalised sums
     stay far enough from the end of fp32's range, whatever maximum they are kept relative to."""
