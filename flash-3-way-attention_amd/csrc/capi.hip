@@ -269,7 +269,7 @@ int tdp_bwd_generic(Arena& ar, bool run, const void* q, const void* k1, const vo
     a.BH = B * H; a.T = T; a.D = D; a.alpha = alpha;
     a.causal = causal; a.k1_window = w1; a.k2_window = w2; a.kk_left = kl; a.kk_right = kr;
     if (dtype != TRITT_F32) plan_f32_fwd(ar, a, dtype, false);  // (o32 is null while measuring)
-    long long* fixed = mfma32 ? ar.take<long long>(f32_mfma_tdp_bwd_scratch_elems(a)) : nullptr;
+    void* scratch32 = mfma32 ? ar.take<char>(f32_mfma_tdp_bwd_scratch_bytes(a)) : nullptr;
     // VALU kernels: fp32 results, the caller's tensors when they are fp32, scratch otherwise; `spare` stands in for the
     // unwanted (null) half of a gradient pair whose other half is wanted (one kernel writes both halves)
     float *dq32 = (float*)dq, *dk132 = (float*)dk1, *dk232 = (float*)dk2, *dv232 = (float*)dv2;
@@ -298,7 +298,7 @@ int tdp_bwd_generic(Arena& ar, bool run, const void* q, const void* k1, const vo
         F32BwdCall c{};
         c.a = a; c.o = o32 ? o32 : (const float*)o;
         c.v1_f32 = dtype == TRITT_F32 ? (const float*)v1 : nullptr; c.u_out = u;
-        c.delta = delta; c.scratch = fixed; c.v1 = v1;
+        c.delta = delta; c.scratch = scratch32; c.v1 = v1;
         c.dq = dq; c.dk1 = dk1; c.dk2 = dk2; c.dv1 = dv1; c.dv2 = dv2;
         c.elem = dtype == TRITT_F32 ? 0 : dtype == TRITT_BF16 ? 1 : 2;
         return (int)f32_mfma_tdp_bwd(c, st);

@@ -68,12 +68,12 @@ struct F32BwdCall {
     const float* v1_f32;  // with u_out = a.u: fp32 V1, whose SiLU the call forms; null: a.u is there already
     float* u_out;
     float* delta;         // scratch [BH, T]
-    long long* scratch;   // f32_mfma_tdp_bwd_scratch_elems() 64-bit words: the row gradients' accumulators and dQ's parts
+    void* scratch;        // f32_mfma_tdp_bwd_scratch_bytes() bytes
     const void* v1;       // V1 in the caller's type (SiLU')
     void *dq, *dk1, *dk2, *dv1, *dv2;  // null: not wanted
     int elem;             // the caller's type: 0 float, 1 bf16, 2 f16
 };
-size_t f32_mfma_tdp_bwd_scratch_elems(const GenericTdpArgs& a);  // by BH, T, D and the mask
+size_t f32_mfma_tdp_bwd_scratch_bytes(const GenericTdpArgs& a);  // by BH, T, D and the mask
 hipError_t f32_mfma_tdp_bwd(const F32BwdCall& c, hipStream_t st);
 
 // The first `tiles` query tiles (32 queries each) of a 16-bit triple-dot backward, computed in fp32 from the

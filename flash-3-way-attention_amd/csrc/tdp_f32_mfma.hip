@@ -30,120 +30,141 @@ namespace tritt {
 namespace {
 
 // One pass ahead of the backward kernels, 64 rows per workgroup: U = SiLU(V1) (u null: the caller has it), Delta =
-// rowsum(dO * O), the accumulators cleared (`planes` times n words) and, for fixed-point ones (maxima not null), the
-// partial maxima that fix a slice's scales (F32RowScale; V1's are U's where the caller has that) and the poison words cleared.
-// Five launches of 2-5 us each without it; grid (64-row blocks, BH, 1 + the maxima's tensors: one of them after the other
-// in the blocks of z = 0 is 6 us longer).
+// rowsum(dO * O), the accumulators cleared (`planes` times n words), the images of the streamed tensors and, for fixed-point
+// accumulators (maxima not null), the partial maxima that fix a slice's scales (F32RowScale; V1's are U's where the caller has
+// that) and the poison words cleared.  grid (64-row blocks, BH, 1 + the maxima's tensors + the images): one of them after the
+// other in the blocks of z = 0 is 6 us longer, a launch for each 2-5 us.
+struct F32PrepParams {
+    const float *q, *k1, *k2, *v2, *u_in, *v1, *o, *d_o;
+    float *u, *delta;
+    unsigned* acc;
+    int planes;
+    size_t n;
+    unsigned *maxima, *poison;
+    __bf16* images[4];  // Q, dO, K1, U (null: not wanted)
+    int T;
+};
 template <int D>
-__global__ __launch_bounds__(256) void f32_prep_kernel(const float* __restrict__ q, const float* __restrict__ k1,
-                                                       const float* __restrict__ k2, const float* __restrict__ v2,
-                                                       const float* __restrict__ u_in, const float* __restrict__ v1,
-                                                       float* __restrict__ u,
-                                                       const float* __restrict__ o, const float* __restrict__ d_o,
-                                                       float* __restrict__ delta, unsigned* __restrict__ acc, int planes, size_t n,
-                                                       unsigned* __restrict__ maxima, unsigned* __restrict__ poison, int T) {
+__global__ __launch_bounds__(256) void f32_prep_kernel(F32PrepParams p) {
     __shared__ unsigned red[4];
     constexpr int kPieces = D / 4;
-    const int bh = blockIdx.y, j0 = blockIdx.x * 64;
+    const int bh = blockIdx.y, j0 = blockIdx.x * 64, T = p.T;
     const size_t base = (size_t)bh * T * D;
-    if (blockIdx.z) {  // part s of a slice: its 64-row blocks s, s + kScaleParts, ...
-        const int t = blockIdx.z - 1;
-        const float* src = (t == kMaxDO ? d_o : t == kMaxQ ? q : t == kMaxK1 ? k1 : t == kMaxK2 ? k2 : t == kMaxV2 ? v2 : v1 ? v1 : u_in) + base;
+    int z = blockIdx.z;
+    if (z && p.maxima && z <= kMaxima) {  // part s of a slice: its 64-row blocks s, s + kScaleParts, ...
+        const int t = z - 1;
+        const float* src = (t == kMaxDO ? p.d_o : t == kMaxQ ? p.q : t == kMaxK1 ? p.k1 : t == kMaxK2 ? p.k2 : t == kMaxV2 ? p.v2 : p.v1 ? p.v1 : p.u_in) + base;
         for (int part = blockIdx.x; part < kScaleParts; part += gridDim.x) {
             unsigned m = 0;
             for (int r0 = part * 64; r0 < T; r0 += kScaleParts * 64)
                 m = max(m, block_absmax_bits<float>(src + (size_t)r0 * D, (size_t)min(64, T - r0) * kPieces, red));
-            if (threadIdx.x == 0) maxima[((size_t)t * gridDim.y + bh) * kScaleParts + part] = m;
+            if (threadIdx.x == 0) p.maxima[((size_t)t * gridDim.y + bh) * kScaleParts + part] = m;
         }
         return;
     }
-    if (maxima && threadIdx.x < 64 && j0 + threadIdx.x < T) poison[(size_t)bh * T + j0 + threadIdx.x] = 0;
+    if (z) {
+        z -= p.maxima ? kMaxima + 1 : 1;
+        const float* src = z == 0 ? p.q : z == 1 ? p.d_o : z == 2 ? p.k1 : p.v1 ? p.v1 : p.u_in;
+        __bf16* dst = p.images[z];
+        const int tiles = (T + 31) / 32;
+        if (dst)
+            for (int tile = 2 * blockIdx.x; tile < min(2 * (int)blockIdx.x + 2, tiles); ++tile)
+                split_image_tile<D>(src + base, dst + ((size_t)bh * tiles + tile) * (3 * split_plane<D>()), tile * 32, T, z == 3 && p.v1);
+        return;
+    }
+    if (p.maxima && threadIdx.x < 64 && j0 + threadIdx.x < T) p.poison[(size_t)bh * T + j0 + threadIdx.x] = 0;
     for (int idx = threadIdx.x; idx < 64 * kPieces; idx += 256) {  // whole waves: 64 kPieces is a multiple of 256
         const int j = j0 + idx / kPieces;
         const size_t off = base + (size_t)j * D + (idx % kPieces) * 4;
         float dot = 0.f;
         if (j < T) {
-            if (u) {
-                f32x4v x = *reinterpret_cast<const f32x4v*>(v1 + off);
+            if (p.u) {
+                f32x4v x = *reinterpret_cast<const f32x4v*>(p.v1 + off);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) x[e] = silu_f(x[e]);
-                *reinterpret_cast<f32x4v*>(u + off) = x;
+                *reinterpret_cast<f32x4v*>(p.u + off) = x;
             }
-            const f32x4v x = *reinterpret_cast<const f32x4v*>(o + off), y = *reinterpret_cast<const f32x4v*>(d_o + off);
+            const f32x4v x = *reinterpret_cast<const f32x4v*>(p.o + off), y = *reinterpret_cast<const f32x4v*>(p.d_o + off);
             dot = x[0] * y[0] + x[1] * y[1] + (x[2] * y[2] + x[3] * y[3]);
-            for (int t = 0; t < planes; ++t) *reinterpret_cast<uint4*>(acc + t * n + off) = make_uint4(0u, 0u, 0u, 0u);
+            for (int t = 0; t < p.planes; ++t) *reinterpret_cast<uint4*>(p.acc + t * p.n + off) = make_uint4(0u, 0u, 0u, 0u);
         }
 #pragma unroll
         for (int w = kPieces / 2; w > 0; w >>= 1) dot += __shfl_xor(dot, w, 64);
-        if (idx % kPieces == 0 && j < T) delta[(size_t)bh * T + j] = dot;
+        if (idx % kPieces == 0 && j < T) p.delta[(size_t)bh * T + j] = dot;
     }
 }
-// The sums -> the gradients (null: not wanted), four elements per thread: dK2, dV2, dK1 and dV1 = dU SiLU'(V1) from fixed
-// point (`slabs` > 0: from that many tiles' fp32 shares, in order), dQ = alpha times the sum of its tile's parts.  dQ's sum
-// belongs to one tile, so its parts are joined in fp32 and in order: a gradient may lie many powers of two below what the
-// scale of a fixed-point sum is set by (B=4 H=8 T=128 D=64, operands of 0.01: dQ in steps of 2^-36 max |dO| is 1.8e-2 off, so
-// joined 3e-7).  Costs what the accumulator did (training steps, accumulator -> parts: B=2 H=4 T=500 D=64 4.32 -> 4.32 ms,
-// B=4 H=8 T=128 522 -> 525 us, B=1 H=2 T=64 D=32 53.0 -> 53.5 us).
+// The sums -> the gradients (null: not wanted), four elements per thread: dK2 and dV2 from fixed point (`slabs` > 0: from that
+// many tiles' fp32 shares, in order); dQ, dK1 and dV1 = dU SiLU'(V1) are the sums of their tile's parts, in fp32 and in order: a
+// gradient may lie many powers of two below what the scale of a fixed-point sum is set by.
+struct F32FinishParams {
+    const long long* acc;
+    const unsigned *fields, *poison;
+    const float *part_q, *part_k1, *part_u;
+    F32Deal deal_q, deal_k;
+    TdpMask mask;
+    int nw, slabs;
+    size_t n;
+    int T, D;
+    float alpha;
+};
 template <typename E>
-__global__ __launch_bounds__(256) void f32_finish_kernel(const long long* __restrict__ acc, const E* __restrict__ v1,
-                                                         E* __restrict__ dq, E* __restrict__ dk1, E* __restrict__ dk2,
-                                                         E* __restrict__ dv1, E* __restrict__ dv2, size_t n, int T, int D,
-                                                         const unsigned* __restrict__ fields,
-                                                         const unsigned* __restrict__ poison, float alpha,
-                                                         const float* __restrict__ part_q, F32Deal deal, TdpMask mask, int nw,
-                                                         int slabs) {
+__global__ __launch_bounds__(256) void f32_finish_kernel(F32FinishParams p, const E* __restrict__ v1, E* __restrict__ dq, E* __restrict__ dk1,
+                                                         E* __restrict__ dk2, E* __restrict__ dv1, E* __restrict__ dv2) {
     typedef __attribute__((ext_vector_type(4))) E e4;
-    for (size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4; i < n; i += (size_t)gridDim.x * 1024) {
-        const size_t row = i / D;
-        const uint4 field = slabs ? make_uint4(0u, 0u, 0u, 0u) : reinterpret_cast<const uint4*>(fields)[row / T];
-        const unsigned bad = slabs ? 0u : poison[row];
-        auto put = [&](E* out, int which, unsigned bit, unsigned f, auto factor) {
-            if (!out) return;
-            if (slabs) {
-                const float* src = reinterpret_cast<const float*>(acc) + (size_t)which * slabs * n + i;
-                f32x4v sum = *reinterpret_cast<const f32x4v*>(src);
-                for (int t = 1; t < slabs; ++t) sum += *reinterpret_cast<const f32x4v*>(src + t * n);
-                e4 r;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) r[e] = (E)(sum[e] * factor(e));
-                *reinterpret_cast<e4*>(out + i) = r;
-                return;
-            }
-            const longlong2* p = reinterpret_cast<const longlong2*>(acc + which * n + i);
-            const longlong2 lo = p[0], hi = p[1];
-            const long long v[4] = {lo.x, lo.y, hi.x, hi.y};
-            const double inv = fixed_scale_inverse(f);
+    for (size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4; i < p.n; i += (size_t)gridDim.x * 1024) {
+        const size_t row = i / p.D;
+        auto write = [&](E* out, const f32x4v& v) {
             e4 r;
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-                r[e] = (E)(((bad & bit) ? __builtin_nanf("") : (float)((double)v[e] * inv)) * factor(e));
+            for (int e = 0; e < 4; ++e) r[e] = (E)v[e];
             *reinterpret_cast<e4*>(out + i) = r;
         };
-        auto one = [](int) { return 1.0f; };
-        put(dk2, 0, kPoisonDK2, field.x, one);
-        put(dv2, 1, kPoisonDV2, field.y, one);
-        put(dk1, 2, kPoisonDK1, field.z, one);
-        if (dv1) {
-            const e4 x = *reinterpret_cast<const e4*>(v1 + i);
-            put(dv1, 3, kPoisonDU, field.w, [&](int e) { return silu_grad_f((float)x[e]); });
-        }
-        if (dq) {
-            const float* src = part_q + row * deal.max_parts * D + i % D;
-            const int parts = f32_tile_parts(deal, mask, (int)(row % T) / 32, T, nw);
+        auto shared = [&](E* out, int which, unsigned bit) {
+            if (!out) return;
+            if (p.slabs) {
+                const float* src = reinterpret_cast<const float*>(p.acc) + (size_t)which * p.slabs * p.n + i;
+                f32x4v sum = *reinterpret_cast<const f32x4v*>(src);
+                for (int t = 1; t < p.slabs; ++t) sum += *reinterpret_cast<const f32x4v*>(src + t * p.n);
+                write(out, sum);
+                return;
+            }
+            const longlong2* src = reinterpret_cast<const longlong2*>(p.acc + which * p.n + i);
+            const longlong2 lo = src[0], hi = src[1];
+            const long long v[4] = {lo.x, lo.y, hi.x, hi.y};
+            const double inv = fixed_scale_inverse(p.fields[row / p.T * 2 + which]);
+            const bool bad = p.poison[row] & bit;
+            f32x4v r;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) r[e] = bad ? __builtin_nanf("") : (float)((double)v[e] * inv);
+            write(out, r);
+        };
+        shared(dk2, 0, kPoisonDK2);
+        shared(dv2, 1, kPoisonDV2);
+        const int tile = (int)(row % p.T) / 32, d = (int)(i % p.D);
+        auto joined = [&](const float* part, const F32Deal& deal) {
+            const float* src = part + row * deal.max_parts * p.D + d;
+            const int parts = f32_tile_parts(deal, p.mask, tile, p.T, p.nw);
             f32x4v sum = *reinterpret_cast<const f32x4v*>(src);
 #pragma unroll 4
-            for (int s = 1; s < parts; ++s) sum += *reinterpret_cast<const f32x4v*>(src + s * D);
-            e4 r;
+            for (int s = 1; s < parts; ++s) sum += *reinterpret_cast<const f32x4v*>(src + s * p.D);
+            return sum;
+        };
+        if (dq) write(dq, joined(p.part_q, p.deal_q) * p.alpha);
+        if (dk1) write(dk1, joined(p.part_k1, p.deal_k) * p.alpha);
+        if (dv1) {
+            const e4 x = *reinterpret_cast<const e4*>(v1 + i);
+            f32x4v v = joined(p.part_u, p.deal_k);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) r[e] = (E)(sum[e] * alpha);
-            *reinterpret_cast<e4*>(dq + i) = r;
+            for (int e = 0; e < 4; ++e) v[e] *= silu_grad_f((float)x[e]);
+            if (!p.slabs && (p.poison[row] & kPoisonDU)) v = f32x4v{NAN, NAN, NAN, NAN};
+            write(dv1, v);
         }
     }
 }
 
 // waves per workgroup
-constexpr int f32_fwd_waves(int D) { return 4; }
-constexpr int f32_bwd_waves(int D) { return D > 64 ? 8 : 4; }
+constexpr int kSplitWaves = 4;
+constexpr int f32_tile_waves(int D) { return D > 64 ? 8 : 4; }  // launch_f32_bwd_tiles
 
 // Joins the parts of a split forward, four columns per thread.
 __global__ __launch_bounds__(256) void f32_merge_kernel(const float* __restrict__ part, float* __restrict__ o,
@@ -152,7 +173,7 @@ __global__ __launch_bounds__(256) void f32_merge_kernel(const float* __restrict_
     const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x, row = idx / (D / 4);
     const int d = (int)(idx % (D / 4)) * 4;
     if (row >= rows) return;
-    const int parts = f32_tile_parts(deal, mask, (int)(row % T) / 32, T, f32_fwd_waves(D));
+    const int parts = f32_tile_parts(deal, mask, (int)(row % T) / 32, T, kSplitWaves);
     const float* src = part + row * deal.max_parts * (D + 4);
     // four parts' loads in flight at a time (a part beyond the last one repeats it with weight zero)
     float m = kNegBig, l = 0.f;
@@ -187,23 +208,31 @@ __global__ __launch_bounds__(256) void f32_merge_kernel(const float* __restrict_
 // count of 4 / 16 per tile 4.1 / 3.9, by cost 3.3); below sixteen steps per slot a part's own cost (prologue, merge: two
 // or three steps' worth) asks for fewer, two per slot; a problem smaller than that gets one step per part (B=1 H=2 T=64
 // D=32: 27 -> 9 us).  At most sixteen parts per tile: 32 gained nothing and double the scratch of a split forward.
-F32Deal f32_deal(const TdpMask& mask, int BH, int T, int nw, int slots, int most) {
+// `share` of the chip: two kinds of tiles in one grid get half of those parts each.
+F32Deal f32_deal(const TdpMask& mask, int BH, int T, int nw, int slots, int most, bool keys = false, double share = 1.0) {
     const int nqt = (T + 31) / 32;
     long long total = 0;
     int rounds;
-    for (int qt = 0; qt < nqt; ++qt) total += f32_tile_steps(mask, qt * 32, std::min(T - 1, qt * 32 + 31), T, nw, &rounds);
-    const double per_slot = (double)total * BH / slots;
+    for (int qt = 0; qt < nqt; ++qt) {
+        const int first = qt * 32, last = std::min(T - 1, qt * 32 + 31);
+        total += keys ? f32_key_tile_steps(mask, first, last, T, nw, &rounds) : f32_tile_steps(mask, first, last, T, nw, &rounds);
+    }
+    const double per_slot = (double)total * BH / (slots * share);
     const double target = std::max({per_slot / 6.0, std::min(16.0, per_slot / 2.0), 1.0});
-    F32Deal d{(float)(1.0 / target), most, 0};
+    F32Deal d{(float)(1.0 / target), most, 0, keys};
     int parts = 1;
     for (int qt = 0; qt < nqt; ++qt) parts = std::max(parts, f32_tile_parts(d, mask, qt, T, nw));
     d.max_parts = parts;
     for (int qt = 0; qt < nqt; ++qt) d.items += f32_tile_parts(d, mask, qt, T, nw);
     return d;
 }
-F32Deal f32_bwd_deal(int BH, int T, int D, const TdpMask& mask) {
-    const int nw = f32_bwd_waves(D);
-    return f32_deal(mask, BH, T, nw, nw == 4 ? 512 : 256, knobs().bwd_splits > 0 ? std::min(knobs().bwd_splits, 16) : 16);
+int f32_most_parts() { return knobs().bwd_splits > 0 ? std::min(knobs().bwd_splits, 16) : 16; }
+F32Deal f32_tiles_deal(int BH, int T, int D, const TdpMask& mask) {  // launch_f32_bwd_tiles
+    const int nw = f32_tile_waves(D);
+    return f32_deal(mask, BH, T, nw, nw == 4 ? 512 : 256, f32_most_parts());
+}
+F32Deal f32_bwd_deal(int BH, int T, int D, const TdpMask& mask, bool keys) {
+    return f32_deal(mask, BH, T, kSplitWaves, D == 32 ? 512 : 256, f32_most_parts(), keys, 0.5);
 }
 
 // Problems of less than eight query tiles: every tile has row-gradient accumulators of its own, fp32, where each element gets
@@ -220,7 +249,7 @@ hipError_t launch_f32_bwd_tiles(F32BwdParams<E> p, const E* k1, const E* u, cons
                                 bool want_k2, bool want_k1, hipStream_t st, const InputsAt& at, bool deal_out) {
     // a workgroup holds all D gradient columns and forms S and dP once (D = 128: dQ's running sum is kept in LDS)
     constexpr int DOUT = D;
-    constexpr int NW = f32_bwd_waves(D);
+    constexpr int NW = f32_tile_waves(D);
     auto kern_dq = tdp_f32_bwd_kernel<E, D, DOUT, true, NW>;
     auto kern_nodq = tdp_f32_bwd_kernel<E, D, DOUT, false, NW>;
     constexpr size_t smem = f32_bwd_smem<D, NW>();
@@ -230,75 +259,124 @@ hipError_t launch_f32_bwd_tiles(F32BwdParams<E> p, const E* k1, const E* u, cons
     // of parts belongs to the mask it was made for, and the second launch exchanges the two key indices.
     const TdpMask exchanged{natural.causal, natural.wb, natural.wa, natural.rab, natural.lab};
     const F32Deal whole{0.f, 1, p.nqt};
-    auto deal_for = [&](const TdpMask& m) { return deal_out ? f32_bwd_deal(p.BH, p.T, D, m) : whole; };
+    auto deal_for = [&](const TdpMask& m) { return deal_out ? f32_tiles_deal(p.BH, p.T, D, m) : whole; };
     auto grid_of = [&](const F32Deal& d) { return dim3(8 * xcd_slots(p.BH, d.items), D / DOUT); };
     // rows = (K2, V2), streamed = (K1, U): dQ, dK2, dV2
     p.ka = k1; p.va = u; p.kb = k2; p.vb = v2;
     place_inputs(p, at, false);
     p.acc_k = acc_k2; p.acc_v = acc_v2; p.bit_k = kPoisonDK2; p.bit_v = kPoisonDV2;
-    p.rows.fields_at = 0; p.rows.streamed_k = kMaxK1; p.rows.streamed_v = kMaxV1;
     p.mask = natural;
-    p.deal = want_q && !p.part_q && !p.acc_q ? whole : deal_for(natural);
+    p.deal = want_q && !p.acc_q ? whole : deal_for(natural);
     if (want_q) hipLaunchKernelGGL(kern_dq, grid_of(p.deal), dim3(64 * NW), smem, st, p);
     else if (want_k2) hipLaunchKernelGGL(kern_nodq, grid_of(p.deal), dim3(64 * NW), smem, st, p);
     // rows = (K1, U), streamed = (K2, V2): dK1, dU (the mask with the two key indices exchanged)
     p.ka = k2; p.va = v2; p.kb = k1; p.vb = u;
     place_inputs(p, at, true);
     p.acc_k = acc_k1; p.acc_v = acc_u; p.bit_k = kPoisonDK1; p.bit_v = kPoisonDU;
-    p.rows.fields_at = 2; p.rows.streamed_k = kMaxK2; p.rows.streamed_v = kMaxV2;
     p.mask = exchanged;
     p.deal = deal_for(exchanged);
     if (want_k1) hipLaunchKernelGGL(kern_nodq, grid_of(p.deal), dim3(64 * NW), smem, st, p);
     return hipGetLastError();
 }
 
+// (a window beyond the sequence is no window; the workspace's query may name any)
+TdpMask f32_mask(const GenericTdpArgs& a) {
+    auto w = [&](int x) { return std::min(x, a.T); };
+    return {a.causal, w(a.k1_window), w(a.k2_window), w(a.kk_left), w(a.kk_right)};
+}
+
+// Scratch of a backward: the accumulators of dK2 and dV2, with fixed-point ones the rows' poison words, the slices' partial
+// maxima and exponent fields; the parts of dQ, dK1 and dU; the images of Q, dO, K1 and U.  base null: measuring (bytes = the end).
+struct F32BwdScratch {
+    F32Deal deal_q, deal_k;
+    int slabs;
+    long long* acc;
+    unsigned *poison, *maxima, *fields;
+    float *part_q, *part_k1, *part_u;
+    __bf16* images;
+    size_t image_elems, bytes;
+};
+template <int D>
+F32BwdScratch f32_bwd_scratch(const GenericTdpArgs& a, void* base) {
+    const TdpMask mask = f32_mask(a);
+    const size_t rows = (size_t)a.BH * a.T, n = rows * D;
+    F32BwdScratch s{};
+    s.deal_q = f32_bwd_deal(a.BH, a.T, D, mask, false);
+    s.deal_k = f32_bwd_deal(a.BH, a.T, D, mask, true);
+    s.slabs = f32_tile_slabs(a.BH, a.T) ? (a.T + 31) / 32 : 0;
+    size_t at = 0;
+    auto take = [&](size_t bytes) {
+        char* p = base ? (char*)base + at : nullptr;
+        at += (bytes + 255) & ~size_t(255);
+        return p;
+    };
+    // (one or two tiles' own accumulators are smaller than the fixed-point ones: the size stays monotone in T)
+    s.acc = (long long*)take(std::max((size_t)16 * n, (size_t)8 * s.slabs * n));
+    s.poison = (unsigned*)take(4 * rows);
+    s.maxima = (unsigned*)take((size_t)4 * a.BH * kScaleParts * kMaxima);
+    s.fields = (unsigned*)take((size_t)8 * a.BH);
+    s.part_q = (float*)take(4 * n * s.deal_q.max_parts);
+    s.part_k1 = (float*)take(4 * n * s.deal_k.max_parts);
+    s.part_u = (float*)take(4 * n * s.deal_k.max_parts);
+    s.image_elems = split_image_elems<D>(a.BH, a.T);
+    s.images = (__bf16*)take(4 * sizeof(__bf16) * s.image_elems);
+    s.bytes = at;
+    return s;
+}
+
 template <int D>
 hipError_t launch_f32_bwd(const F32BwdCall& c, hipStream_t st) {
     const GenericTdpArgs& a = c.a;
-    const size_t n = (size_t)a.BH * a.T * D, rows = (size_t)a.BH * a.T;
-    const bool want_q = c.dq != nullptr, want_k2 = c.dk2 || c.dv2, want_k1 = c.dk1 || c.dv1;
-    const TdpMask natural{a.causal, a.k1_window, a.k2_window, a.kk_left, a.kk_right};
-    const F32Deal deal_q = f32_bwd_deal(a.BH, a.T, D, natural);
-    // scratch: the accumulators of dK2, dV2, dK1 and dU, with fixed-point ones the rows' poison words, the slices' partial
-    // maxima and exponent fields, and dQ's parts
-    const int slabs = f32_tile_slabs(a.BH, a.T) ? (a.T + 31) / 32 : 0;
-    long long* acc = c.scratch;
-    float* share = reinterpret_cast<float*>(acc);
-    unsigned* poison = slabs ? nullptr : reinterpret_cast<unsigned*>(acc + 4 * n);
-    unsigned* maxima = slabs ? nullptr : reinterpret_cast<unsigned*>(acc + 4 * n + (rows + 3) / 4 * 2);  // 16-byte aligned
-    unsigned* fields = slabs ? nullptr : maxima + (size_t)a.BH * kScaleParts * kMaxima;
-    float* part_q = slabs ? share + 4 * slabs * n : reinterpret_cast<float*>(fields + (size_t)a.BH * 4);
+    const size_t n = (size_t)a.BH * a.T * D;
+    const bool want_q = c.dq != nullptr, want_keys = c.dk2 || c.dv2 || c.dk1 || c.dv1;
+    const F32BwdScratch s = f32_bwd_scratch<D>(a, c.scratch);
     // a dQ of one part per tile needs no place of its own where the kernel can write the caller's type
-    const bool direct_q = c.elem == 0 && deal_q.max_parts == 1;
-    hipLaunchKernelGGL(f32_prep_kernel<D>, dim3((a.T + 63) / 64, a.BH, slabs ? 1 : 1 + kMaxima), dim3(256), 0, st, a.q, a.k1, a.k2, a.v2, a.u, c.v1_f32,
-                       c.v1_f32 ? c.u_out : nullptr, c.o, a.d_o, c.delta, reinterpret_cast<unsigned*>(acc), slabs ? 4 * slabs : 8, n,
-                       maxima, poison, a.T);
-    F32BwdParams<float> p{};
-    p.q = a.q; p.d_o = a.d_o; p.lse = a.lse_in; p.delta = c.delta;
-    p.dq = direct_q ? (float*)c.dq : nullptr; p.part_q = direct_q ? nullptr : part_q; p.acc_q = nullptr; p.acc_q_rows = 0; p.stats_part = nullptr; p.split_rounds = 0;
-    p.scale_parts = nullptr; p.poison = poison;
+    const bool direct_q = c.elem == 0 && s.deal_q.max_parts == 1;
+    F32PrepParams prep{};
+    prep.q = a.q; prep.k1 = a.k1; prep.k2 = a.k2; prep.v2 = a.v2; prep.u_in = a.u; prep.v1 = c.v1_f32; prep.o = c.o; prep.d_o = a.d_o;
+    prep.u = c.v1_f32 ? c.u_out : nullptr; prep.delta = c.delta;
+    prep.acc = reinterpret_cast<unsigned*>(s.acc); prep.planes = s.slabs ? 2 * s.slabs : 4; prep.n = n;
+    prep.maxima = s.slabs ? nullptr : s.maxima; prep.poison = s.poison; prep.T = a.T;
+    for (int i = 0; i < 4; ++i) prep.images[i] = (i < 2 ? want_keys : want_q) ? s.images + i * s.image_elems : nullptr;
+    hipLaunchKernelGGL(f32_prep_kernel<D>, dim3((a.T + 63) / 64, a.BH, 1 + (s.slabs ? 0 : kMaxima) + 4), dim3(256), 0, st, prep);
+    F32SplitBwdParams p{};
+    p.q = a.q; p.d_o = a.d_o; p.k1 = a.k1; p.u = a.u; p.k2 = a.k2; p.v2 = a.v2;
+    p.image_q = prep.images[0]; p.image_do = prep.images[1]; p.image_k1 = prep.images[2]; p.image_u = prep.images[3];
+    p.lse = a.lse_in; p.delta = c.delta;
+    p.dq = direct_q ? (float*)c.dq : nullptr; p.part_q = direct_q ? nullptr : s.part_q;
+    p.part_k1 = s.part_k1; p.part_u = s.part_u;
+    p.acc_k = s.acc;
+    p.acc_v = s.slabs ? (void*)((float*)s.acc + s.slabs * n) : (void*)(s.acc + n);
+    p.acc_tile = s.slabs ? n : 0;
+    p.poison = s.poison;
     auto log2_above = [](float x) {  // x <= 2^this
         int e = 128;
         if (std::isfinite(x)) std::frexp(x, &e);
         return e;
     };
-    p.rows.maxima = maxima; p.rows.fields = fields;
+    p.rows.maxima = prep.maxima; p.rows.fields = s.fields;
     p.rows.free_v = 127 + 61 - log2_above((float)a.T);
     p.rows.free_k = p.rows.free_v - 1 - log2_above((float)D) - log2_above(a.alpha);
     p.T = a.T; p.BH = a.BH; p.nqt = (a.T + 31) / 32;
     p.alpha = a.alpha;
-    p.acc_tile = slabs ? n : 0;
-    auto acc_of = [&](int which) { return slabs ? (void*)(share + which * slabs * n) : (void*)(acc + which * n); };
-    if (hipError_t e = launch_f32_bwd_tiles<float, D>(p, a.k1, a.u, a.k2, a.v2, acc_of(0), acc_of(1), acc_of(2), acc_of(3),
-                                                      natural, want_q, want_k2, want_k1, st, dense_inputs(a.T, D), true);
-        e != hipSuccess)
-        return e;
+    p.mask = f32_mask(a);
+    p.deal_q = s.deal_q; p.deal_k = s.deal_k;
+    p.key_blocks = want_keys ? 8 * xcd_slots(a.BH, s.deal_k.items) : 0;
+    const int query_blocks = want_q ? 8 * xcd_slots(a.BH, s.deal_q.items) : 0;
+    auto kern = tdp_f32_split_bwd_kernel<D, kSplitWaves>;
+    constexpr size_t smem = f32_split_bwd_smem<D, kSplitWaves>();
+    if (hipError_t e = ensure_dynamic_smem(reinterpret_cast<const void*>(kern), smem); e != hipSuccess) return e;
+    if (p.key_blocks + query_blocks)
+        hipLaunchKernelGGL(kern, dim3(p.key_blocks + query_blocks), dim3(64 * kSplitWaves), smem, st, p);
+    F32FinishParams f{};
+    f.acc = s.acc; f.fields = s.fields; f.poison = s.poison; f.part_q = s.part_q; f.part_k1 = s.part_k1; f.part_u = s.part_u;
+    f.deal_q = s.deal_q; f.deal_k = s.deal_k; f.mask = p.mask; f.nw = kSplitWaves; f.slabs = s.slabs;
+    f.n = n; f.T = a.T; f.D = D; f.alpha = a.alpha;
     const dim3 grid((unsigned)std::min<size_t>((n / 4 + 255) / 256, 8192));
     auto finish = [&](auto zero) {
         using E = decltype(zero);
-        hipLaunchKernelGGL(f32_finish_kernel<E>, grid, dim3(256), 0, st, acc, (const E*)c.v1, direct_q ? nullptr : (E*)c.dq,
-                           (E*)c.dk1, (E*)c.dk2, (E*)c.dv1, (E*)c.dv2, n, a.T, D, fields, poison, a.alpha, part_q, deal_q,
-                           natural, f32_bwd_waves(D), slabs);
+        hipLaunchKernelGGL(f32_finish_kernel<E>, grid, dim3(256), 0, st, f, (const E*)c.v1, direct_q ? nullptr : (E*)c.dq,
+                           (E*)c.dk1, (E*)c.dk2, (E*)c.dv1, (E*)c.dv2);
     };
     if (c.elem == 0) finish(0.f);
     else if (c.elem == 1) finish((__bf16)0.f);
@@ -307,9 +385,7 @@ hipError_t launch_f32_bwd(const F32BwdCall& c, hipStream_t st) {
 }
 
 F32Deal f32_fwd_deal(const GenericTdpArgs& a, int most) {
-    auto w = [&](int x) { return std::min(x, a.T); };
-    const TdpMask mask{a.causal, w(a.k1_window), w(a.k2_window), w(a.kk_left), w(a.kk_right)};
-    return f32_deal(mask, a.BH, a.T, f32_fwd_waves(a.D), a.D > 64 ? 256 : 512, knobs().fwd_splits > 0 ? std::min(knobs().fwd_splits, most) : most);
+    return f32_deal(f32_mask(a), a.BH, a.T, kSplitWaves, a.D > 64 ? 256 : 512, knobs().fwd_splits > 0 ? std::min(knobs().fwd_splits, most) : most);
 }
 
 template <int D>
@@ -320,10 +396,10 @@ hipError_t launch_f32_fwd(const GenericTdpArgs& a, hipStream_t st) {
     p.silu_va = a.u_is_v1;
     p.T = a.T; p.BH = a.BH; p.nqt = (a.T + 31) / 32;
     p.scale_log2 = a.alpha * kLog2e;
-    p.mask = TdpMask{a.causal, a.k1_window, a.k2_window, a.kk_left, a.kk_right};
+    p.mask = f32_mask(a);
     p.deal = a.part ? f32_fwd_deal(a, a.fwd_parts) : F32Deal{0.f, 1, p.nqt};
     p.part = a.part;
-    constexpr int NW = f32_fwd_waves(D);
+    constexpr int NW = kSplitWaves;
     if (a.images) {
         __bf16 *ka = (__bf16*)a.images, *va = ka + split_image_elems<D>(a.BH, a.T);
         hipLaunchKernelGGL(f32_split_images_kernel<D>, dim3(p.nqt, a.BH, 2), dim3(256), 0, st, a.k1, a.u, ka, va, a.u_is_v1, a.T);
@@ -428,13 +504,8 @@ hipError_t f32_mfma_tdp_fwd(const GenericTdpArgs& a, hipStream_t st) {
     return hipErrorInvalidValue;
 }
 
-size_t f32_mfma_tdp_bwd_scratch_elems(const GenericTdpArgs& a) {
-    const size_t rows = (size_t)a.BH * a.T;
-    const int parts_q = f32_bwd_deal(a.BH, a.T, a.D, TdpMask{a.causal, a.k1_window, a.k2_window, a.kk_left, a.kk_right}).max_parts;
-    const size_t fixed = 4 * rows * a.D + (rows + 3) / 4 * 2 + (size_t)a.BH * (kScaleParts * kMaxima + 4) / 2;
-    // (one or two tiles' own accumulators are smaller than the fixed-point ones: the size stays monotone in T)
-    const size_t sums = f32_tile_slabs(a.BH, a.T) ? std::max(fixed, 2 * ((a.T + 31) / 32) * rows * a.D) : fixed;
-    return sums + rows * a.D * parts_q / 2;
+size_t f32_mfma_tdp_bwd_scratch_bytes(const GenericTdpArgs& a) {
+    return a.D == 32 ? f32_bwd_scratch<32>(a, nullptr).bytes : a.D == 64 ? f32_bwd_scratch<64>(a, nullptr).bytes : f32_bwd_scratch<128>(a, nullptr).bytes;
 }
 
 hipError_t f32_mfma_tdp_bwd(const F32BwdCall& c, hipStream_t st) {

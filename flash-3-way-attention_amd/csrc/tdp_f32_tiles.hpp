@@ -32,6 +32,22 @@ __device__ __forceinline__ Range streamed_range(const TdpMask& m, int q0, int q1
     return {max(0, max(q0 - m.wa, b - m.lab)), min(q1, b + m.rab)};
 }
 
+// The same with the roles of a backward's workgroups: they own queries (KEYS false: as above) or keys, [o0, o1], whose streamed
+// rows are then queries.
+template <bool KEYS>
+__device__ __forceinline__ Range own_row_range(const TdpMask& m, int o0, int o1, int T) {
+    if (!KEYS) return row_range(m, o0, o1, T);
+    if (!m.causal) return {0, T - 1};
+    // some q: max(a, b) <= q <= min(a + wa, b + wb)
+    return {max(0, o0 - min(m.rab, m.wb)), min(T - 1, o1 + min(m.lab, m.wa))};
+}
+template <bool KEYS>
+__device__ __forceinline__ Range own_streamed_range(const TdpMask& m, int o0, int o1, int b, int T) {
+    if (!KEYS) return streamed_range(m, o0, o1, b, T);
+    if (!m.causal) return {0, T - 1};
+    return {max(o0, b), min(T - 1, min(o1 + m.wa, b + m.wb))};
+}
+
 // Workgroups per query tile.  The work of a tile is its (round of nw rows, 32-row stage) steps, which under a causal mask
 // grows with the square of its position: a workgroup takes about 1 / inv_target of them, and a tile as many workgroups (its
 // parts) as that asks for.  The grid is the list of all parts, heaviest tiles first, without gaps: workgroups that find
@@ -40,6 +56,7 @@ __device__ __forceinline__ Range streamed_range(const TdpMask& m, int q0, int q1
 struct F32Deal {
     float inv_target;
     int max_parts, items;  // parts of the heaviest tile, and of all tiles of a slice
+    int keys = 0;          // the tiles own keys (f32_key_tile_steps): the first one is the heaviest
 };
 __host__ __device__ __forceinline__ int f32_tile_steps(const TdpMask& m, int q0, int q1, int T, int nw, int* rounds_out) {
     const Range r = row_range(m, q0, q1, T);
@@ -49,11 +66,26 @@ __host__ __device__ __forceinline__ int f32_tile_steps(const TdpMask& m, int q0,
     const int span = q1 - (q0 - m.wa > 0 ? q0 - m.wa : 0), band = m.lab + m.rab + nw;
     return rounds * ((span < band ? span : band) / 32 + 1);
 }
+__host__ __device__ __forceinline__ int f32_key_tile_steps(const TdpMask& m, int o0, int o1, int T, int nw, int* rounds_out) {
+    auto least = [](int x, int y) { return x < y ? x : y; };
+    const int stages = (T + 31) / 32;
+    if (!m.causal) {
+        *rounds_out = (T - 1) / nw + 1;
+        return *rounds_out * stages;
+    }
+    const int lo = o0 - least(m.rab, m.wb) > 0 ? o0 - least(m.rab, m.wb) : 0, hi = least(T - 1, o1 + least(m.lab, m.wa));
+    const int below = o1 / nw - lo / nw + 1, above = hi / nw - o1 / nw;  // rounds up to the tile's own rows, and past them
+    *rounds_out = below + above;
+    // queries o .. min(o + wa, b + wb) below, b .. the same above
+    const int end = least(T - 1, o1 + least(m.wa, m.wb)), longest = (end - o0) / 32 + 1, shortest = end > hi ? (end - hi) / 32 + 1 : 1;
+    return below * longest + above * (longest + shortest) / 2;
+}
 __host__ __device__ __forceinline__ int f32_tile_parts(const F32Deal& d, const TdpMask& m, int qt, int T, int nw) {
     if (d.max_parts <= 1) return 1;
     const int q0 = qt * 32, q1 = q0 + 31 < T - 1 ? q0 + 31 : T - 1;
     int rounds;
-    const int want = 1 + (int)((float)f32_tile_steps(m, q0, q1, T, nw, &rounds) * d.inv_target);
+    const int steps = d.keys ? f32_key_tile_steps(m, q0, q1, T, nw, &rounds) : f32_tile_steps(m, q0, q1, T, nw, &rounds);
+    const int want = 1 + (int)((float)steps * d.inv_target);
     const int most = rounds < d.max_parts ? rounds : d.max_parts;
     return want < most ? want : most;
 }
@@ -62,11 +94,13 @@ struct F32Item {
     int qt, part, parts;
 };
 __device__ __forceinline__ F32Item f32_item(const F32Deal& d, const TdpMask& m, int item, int nqt, int T, int nw) {
-    if (d.max_parts <= 1) return {nqt - 1 - item, 0, 1};
-    F32Item it{nqt - 1, item, f32_tile_parts(d, m, nqt - 1, T, nw)};
-    while (it.part >= it.parts && it.qt > 0) {
+    const int first = d.keys ? 0 : nqt - 1, step = d.keys ? 1 : -1, last = nqt - 1 - first;  // heaviest tiles first
+    if (d.max_parts <= 1) return {first + step * item, 0, 1};
+    F32Item it{first, item, f32_tile_parts(d, m, first, T, nw)};
+    while (it.part >= it.parts && it.qt != last) {
         it.part -= it.parts;
-        it.parts = f32_tile_parts(d, m, --it.qt, T, nw);
+        it.qt += step;
+        it.parts = f32_tile_parts(d, m, it.qt, T, nw);
     }
     return it;
 }
@@ -189,17 +223,33 @@ __device__ __forceinline__ bool all_valid(const TdpMask& m, int q0, int a0, int 
     return (b <= q0) & (q0 + 31 <= b + m.wb) & (a0 + 31 <= min(q0, b + m.rab)) & (a0 >= max(q0 + 31 - m.wa, b - m.lab));
 }
 
+// the same for a workgroup that owns queries (above) or keys o
+template <bool KEYS>
+__device__ __forceinline__ Interval own_interval(const TdpMask& m, int o, int b, int T) {
+    if (!KEYS) return valid_interval(m, o, b, T);
+    if (!m.causal) return o < T ? Interval{0, (unsigned)(T - 1)} : Interval{1 << 30, 0u};
+    const int lo = max(o, b), hi = min(min(o + m.wa, b + m.wb), T - 1);
+    const bool any = (b <= o + m.lab) & (o <= b + m.rab) & (lo <= hi);
+    return any ? Interval{lo, (unsigned)(hi - lo)} : Interval{1 << 30, 0u};
+}
+template <bool KEYS>
+__device__ __forceinline__ bool own_all_valid(const TdpMask& m, int o0, int a0, int b, int T) {
+    if (!KEYS) return all_valid(m, o0, a0, b, T);
+    if (!m.causal) return (a0 + 31 < T) & (o0 + 31 < T);
+    return (a0 >= max(o0 + 31, b)) & (a0 + 31 <= min(min(o0 + m.wa, b + m.wb), T - 1)) & (b <= o0 + m.lab) & (o0 + 31 <= b + m.rab);
+}
+
 // The (round of rows, stage of streamed rows) sequence a workgroup walks, one stage per step; rounds whose rows see no
 // streamed row at all are passed over.
 struct Walk {
     int m, st, st_hi;
 };
-template <int NW>
+template <int NW, bool KEYS = false>
 __device__ __forceinline__ bool open_round(Walk& w, const TdpMask& mask, int m, int m_hi, int step, int q0, int q1, int T) {
     for (; m <= m_hi; m += step) {
         // the union over the round's rows
-        const Range ra = streamed_range(mask, q0, q1, min(m * NW, T - 1), T);
-        const Range rb = streamed_range(mask, q0, q1, min(m * NW + NW - 1, T - 1), T);
+        const Range ra = own_streamed_range<KEYS>(mask, q0, q1, min(m * NW, T - 1), T);
+        const Range rb = own_streamed_range<KEYS>(mask, q0, q1, min(m * NW + NW - 1, T - 1), T);
         const int lo = min(ra.lo, rb.lo) / 32, hi = max(ra.hi, rb.hi) / 32;
         if (lo <= hi) {
             w = {m, lo, hi};
@@ -493,7 +543,7 @@ __global__ __launch_bounds__(64 * NW, 2) void tdp_f32_stats_kernel(F32StatsParam
 //   dKB[b, d]  += alpha sum_q Yq^T[d, q] Q[q, d],   dVB[b, d] += sum_q Tv^T[d, q] dO[q, d]
 // The sums over the tile's 32 queries are lane reductions; the sums over query tiles (workgroups) go to shared
 // accumulators: 64-bit fixed point with integer atomics (the result does not depend on the order of arrival), or
-// fp32 atomics when the accumulators are fp32 (the caller's, or a tile's own: F32BwdParams::acc_tile).
+// fp32 atomics when the accumulators are fp32.
 //
 // The tensors may be 16-bit (E = bf16 / f16): they are converted as they are staged, everything after that is
 // fp32.  That is how the 16-bit backward runs its first query tile: for the first few causal queries the softmax
@@ -503,41 +553,6 @@ __global__ __launch_bounds__(64 * NW, 2) void tdp_f32_stats_kernel(F32StatsParam
 // CU at D <= 64 (B=4 H=8 T=512 D=64: 18.5 -> 13.5 ms, B=2 H=4 T=500: 20.0 -> 3.5; eight waves, one workgroup: 15.1 / 4.0).
 // DOUT < D: a workgroup produces DOUT of the gradient columns (blockIdx.y picks them).
 
-// Scales of the fp32 tensors' row-gradient accumulators.  A gradient shrinks with every operand in it while dO stays, so the
-// scale follows all of them: with the slice's largest finite |dO|, |Q|, |K1|, |K2|, |V1|, |V2| (`maxima`, kScaleParts words per
-// tensor and slice, [tensor][BH][parts]; |SiLU(x)| <= |x|), S the streamed operands and sum P = 1,
-//   |dV rows| <= T max|dO| max|VS|       |dK rows| <= alpha T max|Q| max|KS| 2 D max|dO| max|V1| max|V2|
-// and a sum of that size is placed at 2^61.  A tensor with a few large elements makes this bound far too wide: the step is
-// never coarser than 2^-36 of max |dO| (sums past 2^27 times it then set the row's poison word, common.hpp).
-// B=4 H=8 T=128 D=64 with operands of 1 / 0.05 / 0.02 / 0.01, dK2 against 64 bits: 4.5e-7 / 1.4e-4 / 5.3e-3 / 8.1e-2 with the
-// scale of dO alone, 4.5e-7 / 2.8e-7 / 3.1e-7 / 3.2e-7 with this one.  Kernel time of a training step, dO's scale -> this:
-// B=2 H=4 T=500 D=64 4335 -> 4330 us, B=1 H=2 T=128 D=64 160.4 -> 159.8, B=4 H=8 T=128 D=64 531 -> 539.
-constexpr int kF32FixedBias = 36;
-enum { kMaxDO, kMaxQ, kMaxK1, kMaxK2, kMaxV1, kMaxV2, kMaxima };
-struct F32RowScale {
-    const unsigned* maxima;      // null: one scale by max |dO| (or float accumulators)
-    unsigned* fields;            // [BH][4] for the launch that converts: dK2, dV2, dK1, dU
-    int fields_at;               // 0 or 2: this launch's pair
-    int streamed_k, streamed_v;  // kMax.. of the streamed tensors
-    int free_k, free_v;          // exponent field that a sum bounded by 1 would get, less what alpha, T and D take
-};
-__device__ __forceinline__ void f32_row_fields(const F32RowScale& s, int BH, int bh, int& field_k, int& field_v) {
-    // lane t * kScaleParts + i holds part i of tensor t, and at the end an exponent that all of that tensor is below
-    const int lane = threadIdx.x & 63, t = lane / kScaleParts;
-    static_assert(kScaleParts == 8 && kMaxima * kScaleParts <= 64, "one word per lane");
-    unsigned m = s.maxima[((size_t)min(t, kMaxima - 1) * BH + bh) * kScaleParts + lane % kScaleParts];
-#pragma unroll
-    for (int w = 1; w < kScaleParts; w *= 2) m = max(m, (unsigned)__shfl_xor((int)m, w, 64));
-    const int e = (int)(m >> 23) - 126;
-    auto exponent = [&](int tensor) { return __builtin_amdgcn_readlane(e, tensor * kScaleParts); };
-    const int d_o = exponent(kMaxDO), v1 = exponent(kMaxV1), v2 = exponent(kMaxV2);
-    const int least = max(min(kF32FixedBias + 254 - 126 - d_o, 254), 1);  // as fixed_scale_field
-    field_v = s.free_v - d_o - (s.streamed_v == kMaxV1 ? v1 : v2);
-    field_k = s.free_k - d_o - v1 - v2 - exponent(kMaxQ) - (s.streamed_k == kMaxK1 ? exponent(kMaxK1) : exponent(kMaxK2));
-    field_k = max(least, min(field_k, 254));
-    field_v = max(least, min(field_v, 254));
-}
-
 template <typename E>
 struct F32BwdParams {
     const E *q, *d_o, *ka, *kb, *va, *vb;
@@ -546,22 +561,18 @@ struct F32BwdParams {
     const float *lse, *delta;
     E* dq;                 // WITH_DQ, when acc_q is null
     void *acc_k, *acc_v;   // [BH][T][D] gradients of the rows: fixed point (long long) or float
-    size_t acc_tile;       // elements from one query tile's acc_k, acc_v to the next one's (0: all tiles add to the same)
-    // WITH_DQ: when non-null, this workgroup's share of dQ / alpha is left in part_q[((bh T + q) max_parts + part) D]
-    float* part_q;
-    void* acc_q;           // WITH_DQ: else, when non-null, dQ / alpha is added here instead of being written to dq
+    void* acc_q;           // WITH_DQ: when non-null, dQ / alpha is added here instead of being written to dq
     int acc_q_rows;        // 0: acc_q is [BH][T][D]; else it holds the first acc_q_rows queries only, [BH][rows][D]
     // when non-null, LSE and Delta of query tile 0 come from the partials the split STATS launch left here
     const float* stats_part;
     int split_rounds;      // tile 0 only: rounds dealt out to workgroups (see tdp_f32_tile0_kernel), else 0
-    // tdp_f32_bwd_kernel: the rounds of a tile dealt out to f32_tile_parts() workgroups.  max_parts above one needs part_q
-    // or acc_q where dQ is produced (each workgroup holds a share of it)
+    // tdp_f32_bwd_kernel: the rounds of a tile dealt out to f32_tile_parts() workgroups.  max_parts above one needs
+    // acc_q where dQ is produced (each workgroup holds a share of it)
     F32Deal deal;
     // fixed-point accumulators (common.hpp); scale_parts null: the accumulators are float
     const unsigned* scale_parts;
     unsigned* poison;
     int scale_bias;
-    F32RowScale rows;  // maxima not null: the scales of acc_k and acc_v instead of scale_parts'
     unsigned bit_k, bit_v;  // poison bits of acc_k / acc_v
     int T, BH, nqt;        // nqt: query tiles this launch covers (tiles 0 .. nqt - 1)
     float alpha;
@@ -570,22 +581,36 @@ struct F32BwdParams {
 
 // Sums over the 32 lanes of a wave half, of 16 registers of two tensors at once: lane n ends with the sum of register
 // 8 (n>>4 & 1) + 4 (n>>3 & 1) + 2 (n>>2 & 1) + (n>>1 & 1), of x in even lanes and of y in odd ones.  Every exchange halves
-// what is left to exchange: 31 of them, where register after register takes 160.
-__device__ __forceinline__ float half_sum_16x2(f32x16 x, f32x16 y) {
-    const int n = threadIdx.x & 31;
+// what is left to exchange, and none goes through LDS: rows of 16 lanes are swapped between two registers, lanes of a row meet
+// by DPP (8 apart, mirrored in 8, 2 and 1 apart).  77 vector instructions; written with selects of vector elements and
+// __shfl_xor it was 850 (the compiler makes the selects into chains of compares) and 31 LDS round trips.
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+template <int CTRL>
+__device__ __forceinline__ float half_sum_step(bool up, float low, float high) {  // keeps `high` in the lanes `up`, `low` elsewhere
+    asm("" : "+v"(low), "+v"(high));  // (two values: not one element picked by `up`)
+    const float keep = up ? high : low, send = up ? low : high;
+    return keep + dpp<CTRL>(send);
+}
+__device__ __forceinline__ float half_sum_16(const f32x16& x, int n) {
+    float v[8];
 #pragma unroll
-    for (int w = 8; w >= 1; w >>= 1) {
-        const bool up = n & (2 * w);
-#pragma unroll
-        for (int i = 0; i < w; ++i) {
-            const float kx = up ? x[i + w] : x[i], sx = up ? x[i] : x[i + w];
-            const float ky = up ? y[i + w] : y[i], sy = up ? y[i] : y[i + w];
-            x[i] = kx + __shfl_xor(sx, 2 * w, 64);
-            y[i] = ky + __shfl_xor(sy, 2 * w, 64);
-        }
+    for (int i = 0; i < 8; ++i) {
+        // even rows of 16 lanes get their x[i] and their odd row's, odd rows both x[i + 8]
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x[i]), __float_as_uint(x[i + 8]), false, false);
+        v[i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
     }
-    const bool odd = n & 1;
-    return (odd ? y[0] : x[0]) + __shfl_xor(odd ? x[0] : y[0], 1, 64);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = half_sum_step<0x128>(n & 8, v[i], v[i + 4]);  // row_ror:8
+#pragma unroll
+    for (int i = 0; i < 2; ++i) v[i] = half_sum_step<0x141>(n & 4, v[i], v[i + 2]);  // row_half_mirror
+    return half_sum_step<0x4e>(n & 2, v[0], v[1]);                                    // quad_perm [2, 3, 0, 1]
+}
+__device__ __forceinline__ float half_sum_16x2(const f32x16& x, const f32x16& y) {
+    const int n = threadIdx.x & 31;
+    return half_sum_step<0xb1>(n & 1, half_sum_16(x, n), half_sum_16(y, n));           // quad_perm [1, 0, 3, 2]
 }
 __device__ __forceinline__ int half_sum_register() {  // the register whose sum this lane ends with
     return (threadIdx.x >> 1) & 15;
@@ -677,17 +702,7 @@ __device__ __forceinline__ void f32_bwd_body(const F32BwdParams<E>& p, int only_
         sDO[r * LD + d] = (float)slice(p.d_o, p.at_do)[row * p.at_do.st + d];
     }
     // (here, where the first stage's loads are on their way)
-    float fscale = p.scale_parts ? fixed_scale_value(fixed_scale_field(p.scale_parts, bh, p.scale_bias)) : 0.f, fscale_v = fscale;
-    if (p.rows.maxima) {
-        int field_k, field_v;
-        f32_row_fields(p.rows, p.BH, bh, field_k, field_v);
-        fscale = fixed_scale_value(field_k);
-        fscale_v = fixed_scale_value(field_v);
-        if (qt == 0 && part == 0 && threadIdx.x == 0) {
-            p.rows.fields[bh * 4 + p.rows.fields_at] = field_k;
-            p.rows.fields[bh * 4 + p.rows.fields_at + 1] = field_v;
-        }
-    }
+    const float fscale = p.scale_parts ? fixed_scale_value(fixed_scale_field(p.scale_parts, bh, p.scale_bias)) : 0.f;
     // a query past the end of the sequence gets a huge LSE: its P is exactly 0
     float lse2 = 1.0e30f, delta = 0.f;
     if (q < T) {
@@ -855,7 +870,7 @@ __device__ __forceinline__ void f32_bwd_body(const F32BwdParams<E>& p, int only_
                     const float sum = half_sum_16x2(xk, xv);
                     const bool odd = n & 1;
                     const int i = half_sum_register(), d = c0 + DTO * c_row(g, i) + dt;
-                    shared_add(odd ? p.acc_v : p.acc_k, (size_t)qt * p.acc_tile + base + (size_t)b * D + d, odd ? sum : sum * kLn2, odd ? fscale_v : fscale,
+                    shared_add(odd ? p.acc_v : p.acc_k, base + (size_t)b * D + d, odd ? sum : sum * kLn2, fscale,
                                p.poison + (size_t)bh * T + b, odd ? p.bit_v : p.bit_k);
                     __builtin_amdgcn_sched_barrier(0);  // one tile's products and sums in registers at a time
                 }
@@ -920,9 +935,7 @@ __device__ __forceinline__ void f32_bwd_body(const F32BwdParams<E>& p, int only_
             const int r = idx / DOUT, d = idx % DOUT;
             if (q0 + r < T) {
                 const size_t off = base + (size_t)(q0 + r) * D + c0 + d;
-                if (p.part_q)
-                    p.part_q[(((size_t)bh * T + q0 + r) * p.deal.max_parts + part) * D + c0 + d] = merged(d, r);
-                else if (p.acc_q)
+                if (p.acc_q)
                     shared_add(p.acc_q, p.acc_q_rows ? ((size_t)bh * p.acc_q_rows + q0 + r) * D + c0 + d : off,
                                merged(d, r), fscale, p.poison + (size_t)bh * T + q0 + r, kPoisonDQ);
                 else

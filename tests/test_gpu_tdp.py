@@ -1134,6 +1134,34 @@ def test_fp32_gradients_of_small_operands(D, case, splits, tune):
             assert err <= bar, (name, b, h, err)
 
 
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("B,H,T,mask", [(1, 1, 1, "causal"), (3, 3, 31, "none"), (3, 3, 33, "windows"), (1, 9, 65, "none"),
+                                        (2, 2, 97, "causal"), (1, 9, 97, "windows"), (2, 2, 130, "narrow"), (1, 3, 160, "causal")])
+def test_fp32_gradients_against_64_bits(B, H, T, D, mask):
+    """All five gradients of fp32 tensors around the 32-row tiles of queries and of keys, under every kind of mask (the windows of
+    the two key indices differ, and a narrow one leaves tiles of keys that few queries see), and again one at a time: a
+    workgroup that owns keys gives four of them, one that owns queries the fifth.  Bar as above; two rows at the least."""
+    print(f"case {B} {H} {T} {D} {mask}", flush=True)
+    windows = {"windows": dict(k1_window=70, k2_window=20, kk_left=9, kk_right=40), "narrow": dict(k1_window=3, k2_window=35, kk_left=2, kk_right=50)}.get(mask, {})
+    order = [windows.get(k) for k in ("k1_window", "k2_window", "kk_left", "kk_right")]
+    inputs, alpha, causal = orc.make_inputs(B, H, T, D, torch.float32, seed=T + D), 1 / math.sqrt(D), mask != "none"
+    _, g = util.run_tdp(inputs, alpha, causal, order)
+    for b, h in [(0, 0), (B - 1, H - 1)]:
+        _, _, grads = orc.tdp_forward_backward_chunked(*(t[b, h].double() for t in inputs), alpha, causal, **windows)
+        for name, a, r in zip(util.NAMES, g, grads):
+            # (a lone query's dQ and dK are the zeros that dP - Delta leaves: held to the size of dO)
+            err = ((a[b, h].double() - r).norm() / (r.norm() if T > 1 else inputs[5][b, h].double().norm())).item()
+            print(f"    {name}[{b}, {h}]: {err:.2e}", flush=True)
+            assert err <= 2.0 ** -24 * (D + 3) * math.sqrt(max(T, 2)), (name, b, h, err)
+    from flash_trittention import flash_trittention
+
+    for which in range(5):
+        leaves = [t.cuda().requires_grad_(i == which) for i, t in enumerate(inputs[:5])]
+        out = flash_trittention(*leaves, softmax_scale=alpha, causal=causal, **dict(zip(("k1_window", "k2_window", "kk_left", "kk_right"), order)))
+        out.backward(inputs[5].cuda())
+        assert torch.equal(leaves[which].grad.cpu(), g[which]), util.NAMES[which]
+
+
 def test_fp32_dq_beyond_the_range_of_dO():
     """dQ far above |dO| (large keys and values) is finite: nothing bounds it by a multiple of max |dO|."""
     inputs = orc.make_inputs(4, 8, 128, 64, torch.float32, seed=9)
