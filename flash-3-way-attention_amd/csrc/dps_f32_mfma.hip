@@ -1,39 +1,38 @@
-// Dot-product-sum trittention for fp32 tensors on the matrix cores (v_mfma_f32_32x32x2_f32), D = 32 or 64.
+// Dot-product-sum trittention for fp32 tensors on the matrix cores, D = 32 or 64: fp32 operands and sums, every product as six
+// bf16 products of three-way splits (f32_split.hpp).
 //
 // The same two chained attention passes as dps_kernels.hip (inner: lse1, R = softmax_s(alpha K1_s.K2_t) @ U;
 // outer: softmax_t(alpha Q_q.K2_t + lse1[t]) @ (R * V2); backward = the two attention backwards chained through
 // dR and dlse1): "attention with a per-key bias" forward, backward by owner rows and backward by owner columns, the
-// last two in one launch.  True fp32 operands, products and accumulation (the 1e-4 bar of fp32 tensors).
+// last two in one launch.
 //
 // Tiling.  A workgroup owns 32 rows (one per MFMA column = lane % 32) in all of its waves; the 32-row tiles of the other
 // operand are dealt out to the waves in turn, each wave sums its own share and the shares are joined through LDS at the
-// end.  A step of 32 x 32 pairs is 64-128 MFMAs of 64 cycles, so the serial chain of steps of one wave is what a call
-// of a few hundred owner tiles waits for: with one wave per owner tile and the streamed tiles shared through LDS
-// (B = 2, H = 8, T = 1000, D = 64: half a wave per SIMD, up to 32 steps of 4.4 us one after another) a training step
-// took 589 us, now 193; larger grids gain from the loads and the missing barriers (B = 4, H = 16, T = 2048: 7.1 -> 2.7 ms,
-// 114 TFLOP/s executed of 157).  What bounds it now: the MFMAs at that rate, below it the chain.  Operands come from L2 straight into registers
-// (16 KB per step and wave: a quarter of what L2 gives a CU in the time of the step's MFMAs), without LDS and without a
-// barrier inside the loop; a register set is loaded again as soon as the product that reads it has been issued, so every
-// load has at least one product (2048 cycles) to arrive in.
+// end: a call of a few hundred owner tiles waits for the serial chain of steps of one wave.  Streamed operands come from L2
+// straight into registers as floats (16 KB per step and wave), without LDS and without a barrier inside the loop, and are split
+// there; a register set is loaded again as soon as the product that reads it has been issued.
 //
-// A 32x32 score tile is D / 2 MFMAs with the contraction dealt out to the lane halves in pieces of four,
-//   S^T[a, r] = sum Ka[a][8 j + 4 g + e] * Xr[r][8 j + 4 g + e]       (A: 16-byte loads of a row, B: owner's registers)
-// It leaves the MFMA with lane <-> owner row and registers <-> streamed rows (row c_row(g, i) in register i), which
-// is the B-operand layout of the output products
+// What bounds it: vector issue.  A SIMD issues one vector or matrix instruction per five cycles or so, and a step has 11 of the
+// former for one MFMA of 32 cycles (a split takes 11 per pair of floats; the streamed rows are split once as rows and once as
+// columns).  Placing the splits between the MFMAs by hand or wave priorities around them changed nothing.  fp32 MFMAs -> this, training
+// step: B=2 H=8 T=1000 D=64 k_diff 128 192 -> 150 us, B=4 H=8 T=1024 D=64 424 -> 327, B=4 H=16 T=2048 D=64 2708 -> 2356, B=4 H=8 T=1024
+// D=32 229 -> 183; gradients against 64 bits at the first 5.4-6.1e-7 -> 3.7-4.8e-7.
+//
+// A 32x32 score tile S^T[a, r] = Ka[a] . Xr[r] takes the streamed row key_of_row(n) in A row n, so that it leaves the MFMAs with
+// lane <-> owner row and registers <-> streamed rows key_of(g, i): registers 8 h .. + 7 are the k-slots of rows 16 h .. of the
+// output products
 //   O^T[d, r] += sum_a V^T[d, a] P^T[a, r]                            (A: loads along a row, B = the P registers)
 // so P never moves between lanes and every per-owner quantity (running maximum, sums, LSE, Delta) is lane-local.
 // MFMA row n of output tile dt is column d = (D / 32) n + dt, so that a lane's loads are as wide as D allows.
 // One owner per output element: no atomics, bitwise reproducible.
 #include "common.hpp"
 #include "kernels.hpp"
+#include "f32_split.hpp"
 #include "mfma.hpp"
 
 namespace tritt {
 namespace {
 
-__device__ __forceinline__ f32x16 mma2(float a, float b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
-}
 __device__ __forceinline__ void pin_order() { __builtin_amdgcn_sched_barrier(0); }
 
 constexpr int kWaves = 4;  // per workgroup; every wave walks each kWaves-th tile of the workgroup's range
@@ -52,27 +51,28 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rows(const float* src, in
     row0 = __builtin_amdgcn_readfirstlane(row0);
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(src) + (size_t)row0 * D, 0, min(32, T - row0) * D * 4, 0x00020000);
 }
-// as A operand of a score product: lane n holds row n
+// operand of a score product: lane (n, g) holds columns 16 ks + 8 g .. + 7 of row `row`, which is n for the owner's rows (B) and
+// key_of_row(n) for the streamed ones (A)
 template <int D>
-__device__ __forceinline__ void load_rows(float (&reg)[D / 2], const float* src, int row0, int T, int n, int g) {
+__device__ __forceinline__ void load_rows(float (&reg)[D / 2], const float* src, int row0, int T, int row, int g) {
     const __amdgpu_buffer_rsrc_t rows = tile_rows<D>(src, row0, T);
 #pragma unroll
     for (int j = 0; j < D / 8; ++j) {
-        const auto v = __builtin_amdgcn_raw_buffer_load_b128(rows, (n * D + 4 * g) * 4 + 32 * j, 0, 0);
+        const auto v = __builtin_amdgcn_raw_buffer_load_b128(rows, (row * D + 8 * g) * 4 + 64 * (j / 2) + 16 * (j % 2), 0, 0);
 #pragma unroll
         for (int e = 0; e < 4; ++e) reg[4 * j + e] = __uint_as_float(v[e]);
     }
 }
-// as A operand of an output product: lane n holds columns DT n .. DT n + DT - 1 of rows c_row(g, 0 .. 15)
+// A operand of an output product: lane n holds columns DT n .. DT n + DT - 1 of rows key_of(g, 0 .. 15)
 template <int D>
 __device__ __forceinline__ void load_cols(float (&reg)[D / 2], const float* src, int row0, int T, int n, int g) {
     const __amdgpu_buffer_rsrc_t rows = tile_rows<D>(src, row0, T);
     // rows 0 .. 15 and 16 .. 31; opaque, so that the rows of a half are one register plus the instruction's offset
-    int lower = (4 * g * D + D / 32 * n) * 4, upper = lower + 16 * D * 4;
+    int lower = (8 * g * D + D / 32 * n) * 4, upper = lower + 16 * D * 4;
     asm volatile("" : "+v"(lower), "+v"(upper));
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-        const int at = i < 8 ? lower : upper, row = (8 * (i % 8 / 4) + i % 4) * D * 4;
+        const int at = i < 8 ? lower : upper, row = i % 8 * D * 4;
         if constexpr (D == 64) {
             const auto v = __builtin_amdgcn_raw_buffer_load_b64(rows, at + row, 0, 0);
             reg[2 * i] = __uint_as_float(v[0]);
@@ -87,13 +87,32 @@ __device__ __forceinline__ float load_vec(const float* src, int row0, int T, int
     const __amdgpu_buffer_rsrc_t rows = tile_rows<1>(src, row0, T);
     return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rows, 4 * n, 0, 0));
 }
-template <int D>
-__device__ __forceinline__ f32x16 score_tile(const float (&rows)[D / 2], const float (&own)[D / 2]) {
+__device__ __forceinline__ Split8 split_at(const float* x) {
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = x[e];
+    return split8(v);
+}
+// S^T of a tile; own(ks): the owner's operand of k-step ks.  The small products of all k-steps come first, and the split of a
+// k-step's streamed operand stands beside the products of the one before.
+template <int D, typename F>
+__device__ __forceinline__ f32x16 score_tile(const float (&rows)[D / 2], const F& own) {
+    constexpr int KS = D / 16;
     f32x16 s;
 #pragma unroll
     for (int i = 0; i < 16; ++i) s[i] = 0.f;
+    Split8 a = split_at(rows);
+    bf16x8 h[KS];
 #pragma unroll
-    for (int ks = 0; ks < D / 2; ++ks) s = mma2(rows[ks], own[ks], s);
+    for (int ks = 0; ks < KS; ++ks) {
+        Split8 next = a;
+        if (ks + 1 < KS) next = split_at(rows + 8 * (ks + 1 < KS ? ks + 1 : 0));
+        s = small_products(a, own(ks), s);
+        h[ks] = a.h;
+        a = next;
+    }
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) s = large_product(h[ks], own(ks).h, s);
     return s;
 }
 // acc^T[d, owner] += sum over the 32 streamed rows of cols[row, d] * w[row, owner]   (w in score-tile layout)
@@ -101,9 +120,19 @@ template <int D>
 __device__ __forceinline__ void output_tile(f32x16 (&acc)[D / 32], const float (&cols)[D / 2], const f32x16& w) {
     constexpr int DT = D / 32;
 #pragma unroll
-    for (int i = 0; i < 16; ++i)
+    for (int half = 0; half < 2; ++half) {
+        float x[8];
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) acc[dt] = mma2(cols[i * DT + dt], w[i], acc[dt]);
+        for (int e = 0; e < 8; ++e) x[e] = w[8 * half + e];
+        const Split8 b = split8(x);
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) {
+            float v[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = cols[(8 * half + e) * DT + dt];
+            acc[dt] = products_of_step(split8(v), b, acc[dt]);
+        }
+    }
 }
 template <int D>
 __device__ __forceinline__ void clear(f32x16 (&acc)[D / 32]) {
@@ -120,16 +149,24 @@ struct Shares {
     alignas(16) float part[kWaves][32 * LD];
     float row[kWaves][32], row2[kWaves][32];  // per owner row and wave
     alignas(16) float vec[kWaves][2][32];                 // one value per streamed row of a wave's step, on its way into the registers
-    alignas(16) float own[32 * LD];                       // the backward's owner rows X or K, scaled
+    // the backward's owner rows, split: the scaled X or K, and G or V.  Rows of 16 (D / 8 + 1) bytes: a wave's 16-byte reads of 32
+    // rows fall on distinct bank groups
+    static constexpr int kOwnLD = D + 8;
+    alignas(16) __bf16 own[2][3][32 * kOwnLD];
+    __device__ __forceinline__ Split8 own_operand(int which, int ks, int n, int g) const {
+        const int at = n * kOwnLD + 16 * ks + 8 * g;
+        return {*reinterpret_cast<const bf16x8*>(own[which][0] + at), *reinterpret_cast<const bf16x8*>(own[which][1] + at),
+                *reinterpret_cast<const bf16x8*>(own[which][2] + at)};
+    }
 
-    // lane n's values of the wave's 32 streamed rows, in score-tile order (register i: row c_row(g, i)).  Only the wave
+    // lane n's values of the wave's 32 streamed rows, in score-tile order (registers 4 i4 .. + 3: rows key_of(g, 4 i4) .. + 3).  Only the wave
     // itself writes and reads its slots and its LDS accesses stay in order.
     __device__ __forceinline__ void vec_put(int which, float v, int wave, int n) {
         vec[wave][which][n] = v;
         asm volatile("" ::: "memory");
     }
     __device__ __forceinline__ float4 vec_get(int which, int wave, int g, int i4) const {
-        return *reinterpret_cast<const float4*>(&vec[wave][which][8 * i4 + 4 * g]);
+        return *reinterpret_cast<const float4*>(&vec[wave][which][key_of(0, 4 * i4) + 8 * g]);
     }
     // this wave's registers, scaled per owner row
     __device__ __forceinline__ void put(const f32x16 (&acc)[D / 32], float f, int wave, int n, int g) {
@@ -171,7 +208,7 @@ struct FwdP {
 };
 template <int D>
 __global__ __launch_bounds__(64 * kWaves, 2) void attn_fwd_f32m_kernel(FwdP p) {
-    constexpr int DT = D / 32, KS = D / 2;
+    constexpr int DT = D / 32, KS = D / 16;
     __shared__ Shares<D> sh;
     const int T = p.T, ntiles = (T + 31) / 32;
     int bh, order;
@@ -190,33 +227,26 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attn_fwd_f32m_kernel(FwdP p) {
     int a0 = a_lo + 32 * wave;
     if (a0 <= a_hi) {
         float bias = p.bias ? load_vec(p.bias + vbase, a0, T, n) : 0.f;
-        float x[KS], rows[KS], cols[KS];
+        float x[D / 2], rows[D / 2], cols[D / 2];
         load_rows<D>(x, X, r0, T, n, g);
-        load_rows<D>(rows, K, a0, T, n, g);
+        load_rows<D>(rows, K, a0, T, key_of_row(n), g);
         load_cols<D>(cols, V, a0, T, n, g);
+        Split8 own[KS];
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) x[ks] *= p.scale_log2;
+        for (int ks = 0; ks < KS; ++ks) {
+            float v[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = x[8 * ks + e] * p.scale_log2;
+            own[ks] = split8(v);
+        }
         for (; a0 <= a_hi; a0 += 32 * kWaves) {
             const int next = min(a0 + 32 * kWaves, a_hi & ~31);  // (past the end: in bounds, not used)
             if (p.bias) sh.vec_put(0, bias, wave, n);
-            // two chains: with the one wave per SIMD of a small call an accumulating chain waits for each of its results
-            f32x16 s, t;
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                s[i] = 0.f;
-                t[i] = 0.f;
-            }
-#pragma unroll
-            for (int ks = 0; ks < KS; ks += 2) {
-                s = mma2(rows[ks], x[ks], s);
-                t = mma2(rows[ks + 1], x[ks + 1], t);
-            }
+            f32x16 s = score_tile<D>(rows, [&](int ks) -> const Split8& { return own[ks]; });
             pin_order();
-            load_rows<D>(rows, K, next, T, n, g);
+            load_rows<D>(rows, K, next, T, key_of_row(n), g);
             if (p.bias) bias = load_vec(p.bias + vbase, next, T, n);
             pin_order();
-#pragma unroll
-            for (int i = 0; i < 16; ++i) s[i] += t[i];
             if (p.bias) {
 #pragma unroll
                 for (int i4 = 0; i4 < 4; ++i4) {
@@ -227,7 +257,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attn_fwd_f32m_kernel(FwdP p) {
             if (a0 + 32 > T || (p.causal && (a0 + 31 > r0 || r0 + 31 - a0 > p.k_diff))) {
 #pragma unroll
                 for (int i = 0; i < 16; ++i) {
-                    const int a = a0 + c_row(g, i);
+                    const int a = a0 + key_of(g, i);
                     s[i] = ((a < T) & pair_valid(p.causal, p.k_diff, r, a)) ? s[i] : -INFINITY;
                 }
             }
@@ -308,38 +338,31 @@ struct BwdP {
     int BH, T, causal, k_diff;
 };
 
-// In the backward one of the owner's two operands is read from LDS in every step (8 reads for 32 MFMAs at D = 64): with it
-// in registers beside the accumulators, two operand sets, the other operand and the score tiles the kernel spills at 256.
+// In the backward the owner's two operands are read from LDS in every step, by all waves: in registers beside the accumulators,
+// two operand sets and the score tiles they do not fit.
 template <int D>
-__device__ __forceinline__ void own_put(Shares<D>& sh, const float* src, int row0, int T, float scale, int tid) {
+__device__ __forceinline__ void own_put(Shares<D>& sh, int which, const float* src, int row0, int T, float scale, int tid) {
+    for (int piece = tid; piece < 32 * D / 8; piece += 64 * kWaves) {
+        const int row = piece / (D / 8), c = piece % (D / 8) * 8;
+        const float* at = src + (size_t)min(row0 + row, T - 1) * D + c;
+        float v[8];
 #pragma unroll
-    for (int piece = tid; piece < Shares<D>::kPieces; piece += 64 * kWaves) {
-        const int row = piece / (D / 4), c = piece % (D / 4) * 4;
-        float4 x = *reinterpret_cast<const float4*>(src + (size_t)min(row0 + row, T - 1) * D + c);
-        x.x *= scale; x.y *= scale; x.z *= scale; x.w *= scale;
-        *reinterpret_cast<float4*>(sh.own + row * Shares<D>::LD + c) = x;
+        for (int e = 0; e < 8; ++e) v[e] = at[e] * scale;
+        const Split8 x = split8(v);
+        *reinterpret_cast<bf16x8*>(sh.own[which][0] + row * Shares<D>::kOwnLD + c) = x.h;
+        *reinterpret_cast<bf16x8*>(sh.own[which][1] + row * Shares<D>::kOwnLD + c) = x.m;
+        *reinterpret_cast<bf16x8*>(sh.own[which][2] + row * Shares<D>::kOwnLD + c) = x.l;
     }
 }
 template <int D>
-__device__ __forceinline__ f32x16 score_tile(const float (&rows)[D / 2], const Shares<D>& sh, int n, int g) {
-    f32x16 s;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) s[i] = 0.f;
+__device__ __forceinline__ f32x16 score_tile(const float (&rows)[D / 2], const Shares<D>& sh, int which, int n, int g) {
     asm volatile("" ::: "memory");  // (the reads stay inside the caller's loop)
-#pragma unroll
-    for (int j = 0; j < D / 8; ++j) {
-        const float4 x = *reinterpret_cast<const float4*>(sh.own + n * Shares<D>::LD + 8 * j + 4 * g);
-        s = mma2(rows[4 * j], x.x, s);
-        s = mma2(rows[4 * j + 1], x.y, s);
-        s = mma2(rows[4 * j + 2], x.z, s);
-        s = mma2(rows[4 * j + 3], x.w, s);
-    }
-    return s;
+    return score_tile<D>(rows, [&](int ks) { return sh.own_operand(which, ks, n, g); });
 }
 
 template <int D>
 __device__ __forceinline__ void bwd_rows(const BwdP& p, Shares<D>& sh, int bh, int tile, int tid, int wave, int n, int g) {
-    constexpr int DT = D / 32, KS = D / 2;
+    constexpr int DT = D / 32;
     const int T = p.T;
     const size_t base = (size_t)bh * T * D, vbase = (size_t)bh * T;
     const float *X = p.X + base, *G = p.G + base, *K = p.K + base, *V = p.V + base;
@@ -349,27 +372,28 @@ __device__ __forceinline__ void bwd_rows(const BwdP& p, Shares<D>& sh, int bh, i
     f32x16 acc[DT];
     clear<D>(acc);
     int a0 = a_lo + 32 * wave;
-    own_put<D>(sh, X, r0, T, scale_log2, tid);
+    own_put<D>(sh, 0, X, r0, T, scale_log2, tid);
+    own_put<D>(sh, 1, G, r0, T, 1.f, tid);
     __syncthreads();
     if (a0 <= a_hi) {
         float bias = p.bias ? load_vec(p.bias + vbase, a0, T, n) : 0.f;
-        float gg[KS], ra[KS], rb[KS];
-        load_rows<D>(ra, K, a0, T, n, g);
-        load_rows<D>(gg, G, r0, T, n, g);
-        load_rows<D>(rb, V, a0, T, n, g);
+        const int nk = key_of_row(n);
+        float ra[D / 2], rb[D / 2];
+        load_rows<D>(ra, K, a0, T, nk, g);
+        load_rows<D>(rb, V, a0, T, nk, g);
         const float lse2 = p.lse[vbase + rc] * p.lse_to_log2, dl = p.delta[vbase + rc];
         // two operand sets in turn: the K rows of the next step take the set the V rows are in now
-        auto step = [&](float (&A)[KS], float (&B)[KS]) {
+        auto step = [&](float (&A)[D / 2], float (&B)[D / 2]) {
             const int next = min(a0 + 32 * kWaves, a_hi & ~31);
             if (p.bias) sh.vec_put(0, bias, wave, n);
-            f32x16 s = score_tile<D>(A, sh, n, g);
+            f32x16 s = score_tile<D>(A, sh, 0, n, g);
             pin_order();
             load_cols<D>(A, K, a0, T, n, g);
             if (p.bias) bias = load_vec(p.bias + vbase, next, T, n);
             pin_order();
-            const f32x16 dp = score_tile<D>(B, gg);
+            const f32x16 dp = score_tile<D>(B, sh, 1, n, g);
             pin_order();
-            load_rows<D>(B, K, next, T, n, g);
+            load_rows<D>(B, K, next, T, nk, g);
             pin_order();
             if (p.bias) {
 #pragma unroll
@@ -384,13 +408,13 @@ __device__ __forceinline__ void bwd_rows(const BwdP& p, Shares<D>& sh, int bh, i
             if (edge) {
 #pragma unroll
                 for (int i = 0; i < 16; ++i) {
-                    const int a = a0 + c_row(g, i);
+                    const int a = a0 + key_of(g, i);
                     s[i] = ((a < T) & pair_valid(p.causal, p.k_diff, r, a)) ? s[i] : 0.f;
                 }
             }
             output_tile<D>(acc, A, s);
             pin_order();
-            load_rows<D>(A, V, next, T, n, g);
+            load_rows<D>(A, V, next, T, nk, g);
             pin_order();
         };
         while (true) {
@@ -420,7 +444,7 @@ __device__ __forceinline__ void bwd_rows(const BwdP& p, Shares<D>& sh, int bh, i
 
 template <int D>
 __device__ __forceinline__ void bwd_cols(const BwdP& p, Shares<D>& sh, int bh, int tile, int tid, int wave, int n, int g) {
-    constexpr int DT = D / 32, KS = D / 2;
+    constexpr int DT = D / 32;
     const int T = p.T;
     const size_t base = (size_t)bh * T * D, vbase = (size_t)bh * T;
     const float *X = p.X + base, *G = p.G + base, *K = p.K + base, *V = p.V + base;
@@ -432,26 +456,27 @@ __device__ __forceinline__ void bwd_cols(const BwdP& p, Shares<D>& sh, int bh, i
     clear<D>(accV);
     float db = 0.f;
     int rr0 = r_lo + 32 * wave;
-    own_put<D>(sh, K, c0, T, scale_log2, tid);
+    own_put<D>(sh, 0, K, c0, T, scale_log2, tid);
+    own_put<D>(sh, 1, V, c0, T, 1.f, tid);
     __syncthreads();
     if (rr0 <= r_hi) {
         float lse = load_vec(p.lse + vbase, rr0, T, n), delta = load_vec(p.delta + vbase, rr0, T, n);
-        float v[KS], ra[KS], rb[KS];
-        load_rows<D>(ra, X, rr0, T, n, g);
-        load_rows<D>(v, V, c0, T, n, g);
-        load_rows<D>(rb, G, rr0, T, n, g);
+        const int nk = key_of_row(n);
+        float ra[D / 2], rb[D / 2];
+        load_rows<D>(ra, X, rr0, T, nk, g);
+        load_rows<D>(rb, G, rr0, T, nk, g);
         const float b = p.bias ? p.bias[vbase + min(a, T - 1)] : 0.f;
         for (; rr0 <= r_hi; rr0 += 32 * kWaves) {
             const int next = min(rr0 + 32 * kWaves, r_hi & ~31);
             sh.vec_put(0, lse * p.lse_to_log2, wave, n);
             sh.vec_put(1, delta, wave, n);
-            f32x16 s = score_tile<D>(ra, sh, n, g);  // rows = streamed r, columns = owner a
+            f32x16 s = score_tile<D>(ra, sh, 0, n, g);  // rows = streamed r, columns = owner a
             pin_order();
             load_cols<D>(ra, X, rr0, T, n, g);
             lse = load_vec(p.lse + vbase, next, T, n);
             delta = load_vec(p.delta + vbase, next, T, n);
             pin_order();
-            f32x16 dp = score_tile<D>(rb, v);
+            f32x16 dp = score_tile<D>(rb, sh, 1, n, g);
             pin_order();
             load_cols<D>(rb, G, rr0, T, n, g);
             pin_order();
@@ -471,7 +496,7 @@ __device__ __forceinline__ void bwd_cols(const BwdP& p, Shares<D>& sh, int bh, i
             if (edge) {
 #pragma unroll
                 for (int i = 0; i < 16; ++i) {
-                    const int rr = rr0 + c_row(g, i);
+                    const int rr = rr0 + key_of(g, i);
                     const bool ok = (rr < T) & pair_valid(p.causal, p.k_diff, rr, a);
                     s[i] = ok ? s[i] : 0.f;
                     dp[i] = ok ? dp[i] : 0.f;
@@ -481,11 +506,11 @@ __device__ __forceinline__ void bwd_cols(const BwdP& p, Shares<D>& sh, int bh, i
             for (int i = 0; i < 16; ++i) db += s[i];
             output_tile<D>(accK, ra, s);
             pin_order();
-            load_rows<D>(ra, X, next, T, n, g);
+            load_rows<D>(ra, X, next, T, nk, g);
             pin_order();
             output_tile<D>(accV, rb, dp);
             pin_order();
-            load_rows<D>(rb, G, next, T, n, g);
+            load_rows<D>(rb, G, next, T, nk, g);
             pin_order();
         }
     }

@@ -555,3 +555,20 @@ def test_fp32_gradients_against_64_bits(D):
             norm, most = (err.norm() / r.norm()).item(), (err / r.abs().clamp_min(rms)).max().item()
             print(f"    {name}[{b}, {h}]: norm {norm:.2e}, element {most:.2e}", flush=True)
             assert norm <= 2.9e-6 and most <= 1.8e-4, name
+
+
+@pytest.mark.parametrize("D", [32, 64])
+@pytest.mark.parametrize("T,k_diff", [(31, 5), (33, 33), (65, 40), (129, 20), (257, 257)])
+def test_fp32_split_products_around_the_tiles(T, k_diff, D):
+    """The fp32 kernels around their 32-row tiles, fewer streamed tiles than waves and more, against 64 bits.  Every score and every
+    output is a sum whose D or T products keep 24 bits: 2^-24 (sqrt(D) + sqrt(T) + 2) in the norm for the output, four such
+    factors (P, dP - Delta, and what is chained through R) for a gradient."""
+    scale = 1 / math.sqrt(D)
+    inputs = orc.make_inputs(2, 3, T, D, torch.float32, seed=T + D)
+    out, m, g = util.run_dps(inputs, scale, True, k_diff)
+    for b, h in ((0, 0), (1, 2)):
+        z, lse, grads = _dps_in_64_bits(inputs, scale, k_diff, b, h)
+        for name, a, r in zip(("o", *util.NAMES), (out, *g), (z, *grads)):
+            err = ((a[b, h].double() - r).norm() / r.norm()).item()
+            print(f"    {name}[{b}, {h}] T={T} D={D}: {err:.2e}", flush=True)
+            assert err <= (1 if name == "o" else 4) * 2.0 ** -24 * (math.sqrt(D) + math.sqrt(T) + 2), name
