@@ -14,26 +14,33 @@
 //   * masks of the k-j band come from a table in LDS: the pattern of a 32x32 step depends only on
 //     (first key j - first key k), and at most four such offsets straddle an edge of the band; the
 //     table holds them in the MFMA C layout (0 or -3e4), read as the C operand of the score product.
-//     Steps cut by j <= q or j >= q - wa, and k-tiles cut by the k window, are masked element-wise.
+//     Steps cut by j <= q or j >= q - wa add another table's entries (by j - limit, the same for every row), k-tiles
+//     cut by the k window a penalty per row.
 //   * with reference 0 everywhere the merge of a k-tile into the running output needs no maximum, no
 //     rescaling and no row weights (masked rows have P = 0 exactly): O += V2[k] (.) Tv[(q,k)].
+// What bounds it: vector issue, one vector or matrix instruction per five cycles and SIMD, with 13-18 of the former for an MFMA:
+// exponentials, the operand of a k-tile (80 for 24 MFMAs) and its merge.  B=2 H=8 T=2048 D=64 fp16, windows 128 / 32 (a call): 176 us;
+// with the step loop on the scalar unit and V2 by transposed reads 167, with the limits' masks from a table 164, with K2 as floats
+// 155 (B=4 H=8 T=1024 windows 64 / 16: 109 -> 94; D = 32 B=4 H=8 T=2048 windows 300 / 100 953 -> 845).
 #pragma once
 
 namespace tritt {
 
 constexpr int kBandQ = 32;  // queries per workgroup
+constexpr int kCutRow = 72;  // entries of a limit's mask, j - limit = -32 .. 31 and what a copy is shifted by
 
 // rows of the resident band: everything queries q0 .. q0+31 can touch (q0 is a multiple of 32, and so is the
 // first resident row)
 inline int band_rows(int wa, int wb) { return ((wa > wb ? wa : wb) + 31) / 32 * 32 + kBandQ; }
 
 template <int D, int kW>
-constexpr size_t band_smem_bytes(int nr) {
-    return sizeof(uint16_t) * ((size_t)3 * nr * (D + 8) + (size_t)D * (nr + 8)) + sizeof(float) * (kBandQ * D + kW * 32 + 5 * 16 * 64);
+constexpr size_t band_smem_bytes(int nr, bool k2_float = false) {
+    return (k2_float ? sizeof(float) * nr * (D + 4) - sizeof(uint16_t) * nr * (D + 8) : 0) + sizeof(uint16_t) * ((size_t)3 * nr * (D + 8) + (size_t)D * (nr + 8)) + sizeof(float) * (kBandQ * D + kW * 32 + 5 * 16 * 64 + 2 * 4 * kCutRow);
 }
 
-// kW: waves per workgroup (band_waves16)
-template <typename E, int D, int kW, bool MV = false>
+// kW: waves per workgroup (band_waves16).  K2F: K2 lies in LDS as floats, converted once per workgroup and not once per query and
+// k-tile (32 of a k-tile's 340 vector instructions at D = 64)
+template <typename E, int D, int kW, bool MV = false, bool K2F = false>
 __global__ __launch_bounds__(64 * kW, kW / 4) void tdp_fwd_band_kernel(FwdParams<E> p, int NR) {
     using M = Mma<E>;
     using v8 = typename M::v8;
@@ -43,12 +50,15 @@ __global__ __launch_bounds__(64 * kW, kW / 4) void tdp_fwd_band_kernel(FwdParams
 
     extern __shared__ __align__(16) char smem[];
     E* sK1 = reinterpret_cast<E*>(smem);  // [NR][LDK]
-    E* sK2 = sK1 + NR * LDK;
-    E* sV2 = sK2 + NR * LDK;
+    E* sK2 = sK1 + NR * LDK;                // [NR][LDK], K2F: floats, [NR][D + 4]
+    E* sV2 = K2F ? reinterpret_cast<E*>(reinterpret_cast<float*>(sK2) + NR * (D + 4)) : sK2 + NR * LDK;
     E* sUT = sV2 + NR * LDK;               // [D][LDU]
     float* sQ = reinterpret_cast<float*>(sUT + D * LDU);  // [32][D]  Q * alpha*log2(e), fp32
     float* sW = sQ + kBandQ * D;                                // [kW][32] per-wave scratch
     float* sTab = sW + kW * 32;  // [5 slots][4][64 lanes][4]  band masks in the MFMA C layout; slot 4: zeros
+    // [2][4][kCutRow]  masks of the limits j <= q and j >= q - wa by j - limit (0 or -3e4); copy c is shifted by c entries, so that
+    // four consecutive ones are an aligned read whatever the limit
+    float* sCut = sTab + 5 * 16 * 64;
 
     int bh, order;
     if (!xcd_tile(p.BH, p.nqt, blockIdx.x >> 3, blockIdx.x & 7, bh, order)) return;
@@ -83,7 +93,14 @@ __global__ __launch_bounds__(64 * kW, kW / 4) void tdp_fwd_band_kernel(FwdParams
             const uint4 b = *reinterpret_cast<const uint4*>(K2 + (size_t)(row * st_k2) + ch * 8);
             const uint4 v = *reinterpret_cast<const uint4*>(V2 + (size_t)(row * st_v2) + ch * 8);
             *reinterpret_cast<uint4*>(sK1 + r * LDK + ch * 8) = a;
-            *reinterpret_cast<uint4*>(sK2 + r * LDK + ch * 8) = b;
+            if constexpr (K2F) {
+                const v8 x = __builtin_bit_cast(v8, b);
+                float* at = reinterpret_cast<float*>(sK2) + r * (D + 4) + ch * 8;
+                *reinterpret_cast<float4*>(at) = make_float4((float)x[0], (float)x[1], (float)x[2], (float)x[3]);
+                *reinterpret_cast<float4*>(at + 4) = make_float4((float)x[4], (float)x[5], (float)x[6], (float)x[7]);
+            } else {
+                *reinterpret_cast<uint4*>(sK2 + r * LDK + ch * 8) = b;
+            }
             *reinterpret_cast<uint4*>(sV2 + r * LDK + ch * 8) = v;
         }
         const int ut_chunks = D * (NR / 8);
@@ -109,9 +126,16 @@ __global__ __launch_bounds__(64 * kW, kW / 4) void tdp_fwd_band_kernel(FwdParams
             sTab[((sl * 4 + i / 4) * 64 + lane) * 4 + (i % 4)] = (sl == 4 || (dlt >= -lab && dlt <= rab)) ? 0.f : -3.0e4f;
         }
     }
+    for (int idx = tid; idx < 2 * 4 * kCutRow; idx += kThreads) {
+        const int x = idx % kCutRow + idx / kCutRow % 4 - 32;
+        sCut[idx] = (idx < 4 * kCutRow ? x <= 0 : x >= 0) ? 0.f : -3.0e4f;
+    }
     __syncthreads();
     // from here on the waves never meet again
 
+    // (the compiler takes the maximum of three on the vector ALU and then keeps the loop that starts from it there, under exec
+    // masks: 20 of 56 vector instructions per step)
+    auto uniform = [](int x) { return __builtin_amdgcn_readfirstlane(x); };
     float* sWw = sW + wave * 32;
     const int krow_off = key_of_row(n);
     auto rows_of = [&](float v, float (&out)[16]) {
@@ -135,7 +159,7 @@ __global__ __launch_bounds__(64 * kW, kW / 4) void tdp_fwd_band_kernel(FwdParams
         for (int dt = 0; dt < DT; ++dt) Orun[dt] = 0.f;
 
         // k >= q - wb, and some j with q - wa <= j <= k + rab
-        const int kt_a = max(0, max(q - wb, q - wa - rab)) / 32, kt_b = q / 32;
+        const int kt_a = uniform(max(0, max(q - wb, q - wa - rab)) / 32), kt_b = q / 32;
         for (int kt = kt_a; kt <= kt_b; ++kt) {
             const int k0 = kt * 32, k = k0 + n;
             // window of keys j of the virtual row (q, k); empty: hi < lo
@@ -144,21 +168,31 @@ __global__ __launch_bounds__(64 * kW, kW / 4) void tdp_fwd_band_kernel(FwdParams
             const bool kval = whi >= 0;
             // all 32 rows of the tile are inside the k window
             const bool rows_clean = (k0 + 31 <= q) && (q <= k0 + wb);
-            const int jlo_t = max(0, max(q - wa, k0 - lab)), jhi_t = min(q, k0 + 31 + rab);
+            const int jlo_t = uniform(max(0, max(q - wa, k0 - lab))), jhi_t = min(q, k0 + 31 + rab);
             const int jb_lo = jlo_t & ~31;
             if (jlo_t > jhi_t) continue;  // no (j, k) of this tile is inside the band of q
 
             v8 bq[KS];
 #pragma unroll
             for (int ks = 0; ks < KS; ++ks) {
-                const v8 kv = *reinterpret_cast<const v8*>(sK2 + (k0 - rlo + n) * LDK + ks * 16 + g * 8);
+                float kf[8];
+                if constexpr (K2F) {
+                    const float* at = reinterpret_cast<const float*>(sK2) + (k0 - rlo + n) * (D + 4) + ks * 16 + g * 8;
+                    const float4 lo = *reinterpret_cast<const float4*>(at), hi = *reinterpret_cast<const float4*>(at + 4);
+                    kf[0] = lo.x; kf[1] = lo.y; kf[2] = lo.z; kf[3] = lo.w;
+                    kf[4] = hi.x; kf[5] = hi.y; kf[6] = hi.z; kf[7] = hi.w;
+                } else {
+                    const v8 kv = *reinterpret_cast<const v8*>(sK2 + (k0 - rlo + n) * LDK + ks * 16 + g * 8);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) kf[e] = (float)kv[e];
+                }
                 const float* qp = sQw + ks * 16 + g * 8;
                 const float4 qa = *reinterpret_cast<const float4*>(qp), qb = *reinterpret_cast<const float4*>(qp + 4);
                 const float qf[8] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};
                 v8 r;
 #pragma unroll
                 for (int e = 0; e < 8; e += 2) {
-                    const v2 pr = M::pack((float)kv[e] * qf[e], (float)kv[e + 1] * qf[e + 1]);
+                    const v2 pr = M::pack(kf[e] * qf[e], kf[e + 1] * qf[e + 1]);
                     r[e] = pr[0];
                     r[e + 1] = pr[1];
                 }
@@ -187,7 +221,7 @@ __global__ __launch_bounds__(64 * kW, kW / 4) void tdp_fwd_band_kernel(FwdParams
             // ---- FAST sweep ---------------------------------------------------------------------
             // C operand of the score product = the mask, all of it additive: the k-j band from the table
             // (slot 4: all zeros), a per-lane penalty for rows outside the k window, and, on the steps the
-            // limits j <= q / j >= q - wa cut through, an element-wise one.  The first step starts the
+            // limits j <= q / j >= q - wa cut through, the limits' tables.  The first step starts the
             // value accumulators from a zero C operand instead of cleared registers.
             const float row_pen = kval ? 0.f : -3.0e4f;
             auto fast_step = [&](int jb, auto first_tag) {
@@ -206,11 +240,17 @@ __global__ __launch_bounds__(64 * kW, kW / 4) void tdp_fwd_band_kernel(FwdParams
 #pragma unroll
                     for (int i = 0; i < 16; ++i) s[i] += row_pen;
                 }
-                if (jb + 31 > q || jb < q - wa) {
-                    const int lo = q - wa - jb - 8 * g, span = wa;  // valid: 0 <= key_of(0, i) - lo <= wa
+                auto cut = [&](const float* masks, int limit) {  // |jb - limit| <= 31
+                    const int x = jb - limit + 32, c = x & 3;
+                    const float* at = masks + c * kCutRow + (x - c) + 8 * g;
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) s[i] = ((unsigned)(key_of(0, i) - lo) <= (unsigned)span) ? s[i] : -3.0e4f;
-                }
+                    for (int b = 0; b < 4; ++b) {
+                        const float4 f4 = *reinterpret_cast<const float4*>(at + key_of(0, 4 * b));
+                        s[4 * b] += f4.x; s[4 * b + 1] += f4.y; s[4 * b + 2] += f4.z; s[4 * b + 3] += f4.w;
+                    }
+                };
+                if (jb + 31 > q) cut(sCut, q);
+                if (jb < q - wa) cut(sCut + 4 * kCutRow, q - wa);
 #pragma unroll
                 for (int ks = 0; ks < KS; ++ks) s = M::mma(*reinterpret_cast<const v8*>(k1p + ks * 16), bq[ks], s);
                 v8 pa[2];
@@ -299,7 +339,16 @@ __global__ __launch_bounds__(64 * kW, kW / 4) void tdp_fwd_band_kernel(FwdParams
             }
 
             // ---- merge the 32 virtual rows (q, k) into the running output ---------------------------
-            const E* v2p = sV2 + (k0 - rlo) * LDK + n;
+            // V2 of rows c_row(g, i), column dt 32 + n: four rows of a column per transposed read (in every group of 16 lanes
+            // ds_read_b64_tr_b16 gives lane l element l % 4 of what lanes l / 4, 4 + l / 4, ... address)
+            const E* v2p = sV2 + (k0 - rlo + 4 * g + (lane & 15) / 4) * LDK + ((lane >> 4) & 1) * 16 + (lane & 3) * 4;
+            auto v2_rows = [&](int dt, int b, float (&v)[4]) {  // registers 4 b .. + 3
+                typedef __attribute__((ext_vector_type(4))) short s4;
+                typedef __attribute__((ext_vector_type(4))) E e4;
+                const e4 x = __builtin_bit_cast(e4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s4*)(v2p + 8 * b * LDK + dt * 32)));
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = (float)x[e];
+            };
             if (fast_ok && (Mrun == 0.f || Mrun == -INFINITY)) {
                 // everything so far is relative to reference 0 and masked rows hold exact zeros
                 Mrun = 0.f;
@@ -308,7 +357,12 @@ __global__ __launch_bounds__(64 * kW, kW / 4) void tdp_fwd_band_kernel(FwdParams
                 for (int dt = 0; dt < DT; ++dt) {
                     float part = 0.f;
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) part += (float)v2p[c_row(g, i) * LDK + dt * 32] * acc[dt][i];
+                    for (int b = 0; b < 4; ++b) {
+                        float v[4];
+                        v2_rows(dt, b, v);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) part += v[e] * acc[dt][4 * b + e];
+                    }
                     Orun[dt] += part;
                 }
             } else {
@@ -326,7 +380,12 @@ __global__ __launch_bounds__(64 * kW, kW / 4) void tdp_fwd_band_kernel(FwdParams
                 for (int dt = 0; dt < DT; ++dt) {
                     float part = 0.f;
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) part += wr[i] * (float)v2p[c_row(g, i) * LDK + dt * 32] * acc[dt][i];
+                    for (int b = 0; b < 4; ++b) {
+                        float v[4];
+                        v2_rows(dt, b, v);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) part += wr[4 * b + e] * v[e] * acc[dt][4 * b + e];
+                    }
                     Orun[dt] = Orun[dt] * f + part;
                 }
             }

@@ -945,7 +945,7 @@ static size_t ut_bytes(int BH, int T, int D) {
 // TRITT_FWD_SPLITS overrides the count (tests, tuning sweeps); read once per process (knobs())
 // The band-resident kernel takes windowed causal masks whose band fits in LDS (with room to spare for the
 // compiler's own use).  TRITT_FWD_BAND=0 switches it off (A/B runs).
-constexpr size_t kBandSmemLimit = 156 * 1024;
+constexpr size_t kBandSmemLimit = 156 * 1024 + sizeof(float) * 2 * 4 * kCutRow;
 static bool use_band_kernel(const MfmaFwdArgs& a) {
     if (!(a.windowed && a.causal)) return false;
     if (a.split) return false;  // split operands: the streaming kernels only
@@ -998,8 +998,11 @@ static hipError_t launch_band(const MfmaFwdArgs& a, hipStream_t st) {
     const int nr = band_rows(p.wa, p.wb);
     constexpr int kWide = D == 128 ? 8 : 16, kNarrow = D == 64 ? 16 : 8;
     const bool wide = band_waves16<D>(a, nr);
-    const size_t smem = wide ? band_smem_bytes<D, kWide>(nr) : band_smem_bytes<D, kNarrow>(nr);
-    auto kern = wide ? (a.many_views ? tdp_fwd_band_kernel<E, D, kWide, true> : tdp_fwd_band_kernel<E, D, kWide, false>)
+    constexpr bool kMayFloat = D == 64;
+    const bool k2_float = kMayFloat && wide && band_smem_bytes<D, kWide>(nr, true) <= kBandSmemLimit;
+    const size_t smem = wide ? band_smem_bytes<D, kWide>(nr, k2_float) : band_smem_bytes<D, kNarrow>(nr);
+    auto kern = k2_float ? (a.many_views ? tdp_fwd_band_kernel<E, D, kWide, true, kMayFloat> : tdp_fwd_band_kernel<E, D, kWide, false, kMayFloat>)
+              : wide ? (a.many_views ? tdp_fwd_band_kernel<E, D, kWide, true> : tdp_fwd_band_kernel<E, D, kWide, false>)
                      : (a.many_views ? tdp_fwd_band_kernel<E, D, kNarrow, true> : tdp_fwd_band_kernel<E, D, kNarrow, false>);
     p.at_k1 = a.at_k1; p.at_k2 = a.at_k2; p.at_v2 = a.at_v2;
     hipError_t e = ensure_dynamic_smem(reinterpret_cast<const void*>(kern), smem);
