@@ -322,6 +322,7 @@ __global__ __launch_bounds__(64 * NW, D > 64 ? 1 : 2) void tdp_f32_split_fwd_ker
     if (have) {
         form_operand(0);
         s = scores(sK);
+        __syncthreads();  // the first step's fetch of w2 overwrites the keys of w0
     }
     int buf = 0, slot0 = 0, slot1 = fresh1 ? 1 : 0;  // buffer of V(w0) (and of K(w0), K(w2)); places of the rounds' rows
     while (have) {
