@@ -805,7 +805,9 @@ static hipError_t launch_bwd(const MfmaBwdArgs& a, hipStream_t st) {
     if (all_in_f32) splits = deal_f32 ? 2 : 1;  // (an accumulator for dQ, or none)
     else if (D == 64 && a.windowed && !a.split) splits = windowed_splits(a);
     else if (D == 64 && a.causal && !a.split && tiles < 1024) splits = causal_splits(a);
-    else if (tiles < 1024) splits = std::min(16, (1024 + tiles - 1) / tiles);
+    // (D = 32 with split operands: workgroups of half the size, three to a CU.  B=2 H=8 T=512, training step: 4 / 6 / 8 / 12 / 16
+    // parts 1112 / 984 / 977 / 958 / 958 us; B=2 H=4 T=256, 4 / 8 / 16 parts 283 / 187 / 135; 704 tiles, 2 to 12 parts: 4.40-4.48 ms)
+    else if (tiles < 1024) splits = std::min(16, ((D == 32 && a.split ? 3072 : 1024) + tiles - 1) / tiles);
     // a few waves of long tiles: the last tiles of each head are the costliest (the work of a tile grows with the
     // square of its position), and halving them shortens the tail by about 1 % (measured: B=4 H=8 T=1024, 2048)
     else if (tiles < 4096 && a.T >= 1024) splits = 2;
@@ -851,14 +853,12 @@ static hipError_t launch_bwd(const MfmaBwdArgs& a, hipStream_t st) {
     const bool kk_cuts = std::min(a.k2_window, a.T - 1) > a.kk_right || std::min(a.k1_window, a.T - 1) > a.kk_left;
     const bool general_window = a.windowed && (D == 128 || kk_cuts || std::min(a.k1_window, a.k2_window) <= 64);
     if constexpr (D == 32) {
-        // one shape, the banded instantiation for every mask (full windows are windows of T)
-        smem = bwdg_smem(32, 8, 32, true);
-        kern_dq = tdp_bwd_rows_general_kernel<E, 32, true, 8, 32, true, false, SV>;
-        kern_nodq = tdp_bwd_rows_general_kernel<E, 32, false, 8, 32, true, false, SV>;
-        if (a.split) {
-            kern_dq = tdp_bwd_rows_general_kernel<E, 32, true, 8, 32, true, true, SV>;
-            kern_nodq = tdp_bwd_rows_general_kernel<E, 32, false, 8, 32, true, true, SV>;
-        }
+        // the banded instantiation for every mask (full windows are windows of T)
+        constexpr int NW = bwdg_waves_d32(false), NS = bwdg_waves_d32(true);
+        smem = bwdg_smem(32, a.split ? NS : NW, 32, true);
+        nthreads = 64 * (a.split ? NS : NW);
+        kern_dq = a.split ? tdp_bwd_rows_general_kernel<E, 32, true, NS, 32, true, true, SV> : tdp_bwd_rows_general_kernel<E, 32, true, NW, 32, true, false, SV>;
+        kern_nodq = a.split ? tdp_bwd_rows_general_kernel<E, 32, false, NS, 32, true, true, SV> : tdp_bwd_rows_general_kernel<E, 32, false, NW, 32, true, false, SV>;
     } else if (a.split) {
         // split operands: the general kernel (banded instantiation: full windows are windows of T)
         if constexpr (D == 64) {

@@ -57,6 +57,12 @@ __device__ __forceinline__ constexpr int swz_t(int r) { return (r >> 2) & 3; }
 
 constexpr int bwdg_stage_bytes(int d, int ncol) { return 2 * d * 64 + 2 * ncol * 64; }
 // rows of a round buffer: the round's NW rows, or what one 1 KB load brings in if that is more
+// D = 32: waves of a workgroup.  The kernel waits for its barriers and LDS reads with the two waves a SIMD that one workgroup of eight
+// gives, and a CU's LDS holds three.  In 128 registers (52-64 B per lane in scratch memory, in the prologue and between rounds) two
+// share a CU: training steps B=2 H=8 T=512 817 -> 714 us, B=4 H=8 T=1024 10.1 -> 8.76 ms, B=2 H=8 T=2048 windows 300 / 100 2.47 ->
+// 2.00 ms (four waves, three workgroups: 757 us, 9.65 and 2.00 ms).  Split operands need 160 registers: workgroups of four waves,
+// three to a CU, 1000 -> 958 us and 12.9 -> 12.1 ms (twelve parts per tile at the first; 128 registers and 150 B: 1340 us).
+constexpr int bwdg_waves_d32(bool split) { return split ? 4 : 8; }
 constexpr int bwdg_round_rows(int d, int nw) { return nw > 512 / d ? nw : 512 / d; }
 constexpr size_t bwdg_smem(int d, int nw, int ncol, bool with_dq) {
     return 3 * (size_t)bwdg_stage_bytes(d, ncol)               // stage buffers
@@ -72,7 +78,7 @@ constexpr size_t bwdg_smem(int d, int nw, int ncol, bool with_dq) {
 // 16-bit operand rounding.
 // SV: the caller's tensors are strided views (BwdParams::at_*); otherwise everything is dense.
 template <typename E, int D, bool WITH_DQ, int NW, int NCOL, bool WIN, bool SPLIT = false, bool SV = false>
-__global__ __launch_bounds__(64 * NW) void tdp_bwd_rows_general_kernel(BwdParams<E> p) {
+__global__ __launch_bounds__(64 * NW, D == 32 ? (SPLIT ? 3 : 4) : 1) void tdp_bwd_rows_general_kernel(BwdParams<E> p) {
     using M = Mma<E>;
     using v8 = typename M::v8;
     using v2 = typename M::v2;
@@ -88,7 +94,7 @@ __global__ __launch_bounds__(64 * NW) void tdp_bwd_rows_general_kernel(BwdParams
     constexpr int RR = bwdg_round_rows(D, NW);   // rows of a round buffer
     static_assert(D == 32 || D == 64 || D == 128, "head dimension");
     static_assert((NW == 8 && NCOL == 64 && D >= 64) || (D == 128 && NW == 4 && NCOL == 128) ||
-                  (D == 32 && NW == 8 && NCOL == 32), "workgroup shapes");
+                  (D == 32 && NCOL == 32), "workgroup shapes");
     static_assert(NBLK % NW == 0, "whole blocks per wave");
     static_assert(!SPLIT || D <= 64, "split operands: the lo halves of a D = 128 round do not fit the register file");
 
@@ -98,6 +104,7 @@ __global__ __launch_bounds__(64 * NW) void tdp_bwd_rows_general_kernel(BwdParams
     E* sVr = sKr + 2 * RR * D;
     // Q and dO tiles for the operand build.  64-column shapes (where LDS has the room): Q * alpha*log2(e) and dO in
     // fp32, so a product is one conversion and one multiply and S is rounded exactly as the forward rounded it.
+    // (D = 32 has the room and loses by it: B=2 H=8 T=512 714 -> 768 us, with split operands no change)
     constexpr bool QF = NCOL == 64;
     constexpr int LDQ = D + 4, QT_BYTES = QF ? BQ * LDQ * 4 : BQ * LDK * 2;
     char* qtiles = reinterpret_cast<char*>(sVr + 2 * RR * D);
@@ -530,10 +537,20 @@ __global__ __launch_bounds__(64 * NW) void tdp_bwd_rows_general_kernel(BwdParams
                         }
                     }
                 } else {
+                    // rows c_row(g, i) of column d: four per transposed read (in every group of 16 lanes ds_read_b64_tr_b16
+                    // gives lane l element l % 4 of what lanes l / 4, 4 + l / 4, ... address)
+                    typedef __attribute__((ext_vector_type(4))) short s4;
+                    typedef __attribute__((ext_vector_type(4))) E e4;
+                    const int at = (4 * g + (lane & 15) / 4) * LDK + c0 + dt * 32 + ((lane >> 4) & 1) * 16 + (lane & 3) * 4;
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) {
-                        sk += accQ[dt][i] * (float)sQb[c_row(g, i) * LDK + d];
-                        sv += accT[dt][i] * (float)sOb[c_row(g, i) * LDK + d];
+                    for (int b = 0; b < 4; ++b) {
+                        const e4 qv = __builtin_bit_cast(e4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s4*)(sQb + at + 8 * b * LDK)));
+                        const e4 ov = __builtin_bit_cast(e4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s4*)(sOb + at + 8 * b * LDK)));
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            sk += accQ[dt][4 * b + e] * (float)qv[e];
+                            sv += accT[dt][4 * b + e] * (float)ov[e];
+                        }
                     }
                 }
                 sk += __shfl_xor(sk, 32, 64);

@@ -1347,3 +1347,38 @@ def test_band_forward_where_its_limits_cut(dtype, D, w):
     for h in range(2):
         z, _, _ = orc.tdp_forward_backward_chunked(*(t[0, h] for t in f32), 1 / math.sqrt(D), True, need_grads=False, **kw)
         util.assert_close(f"out[{h}]", out[0, h], z, rtol=5e-2, atol=2e-2)
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("T,windows", [(250, (100, 40, 24, 7)), (100, (None,) * 4)])
+def test_fp32_training_step_is_the_same_bits_every_time(D, T, windows):
+    """Waves of a workgroup share LDS stages that are fetched while others still read the ones before: thirty runs, one result."""
+    inputs = orc.make_inputs(2, 4, T, D, torch.float32, seed=T + D)
+    first = None
+    for _ in range(30):
+        out, g = util.run_tdp(inputs, 1 / math.sqrt(D), True, windows)
+        first = first or (out, g)
+        assert torch.equal(out, first[0]) and all(torch.equal(a, b) for a, b in zip(g, first[1]))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,H,T,windows", [(1, 1, 33, (None,) * 4), (1, 3, 129, (40, 25, 9, 30)), (2, 8, 160, (None,) * 4), (5, 8, 97, (None,) * 4)])
+@pytest.mark.parametrize("splits", [0, 1, 16])
+def test_backward_d32_shapes_of_a_workgroup(B, H, T, windows, splits, dtype, tune):
+    """D = 32, with and without split operands: workgroups of four and of eight waves, one part per tile and as many as there
+    are, part counts that leave some without a round.  16-bit bar."""
+    from flash_trittention import flash_trittention
+
+    tune(_lib.TUNE_BWD_SPLITS, splits)
+    inputs = orc.make_inputs(B, H, T, 32, dtype, seed=T)
+    kw = dict(zip(("k1_window", "k2_window", "kk_left", "kk_right"), windows))
+    f32 = [t.float() for t in inputs]
+    for convert in (False, True):
+        leaves = [t.cuda().requires_grad_(True) for t in inputs[:5]]
+        out = flash_trittention(*leaves, softmax_scale=32 ** -0.5, causal=True, convert_to_float32=convert, **kw)
+        out.backward(inputs[5].cuda())
+        for b, h in {(0, 0), (B - 1, H - 1)}:
+            z, _, grads = orc.tdp_forward_backward_chunked(*(t[b, h] for t in f32), 32 ** -0.5, True, **kw)
+            util.assert_close(f"out[{b}, {h}] convert={convert}", out.detach()[b, h].float().cpu(), z, rtol=5e-2, atol=2e-2)
+            for name, leaf, want in zip(util.NAMES, leaves, grads):
+                util.assert_close(f"{name}[{b}, {h}] convert={convert}", leaf.grad[b, h].float().cpu(), want, rtol=5e-2, atol=2e-2)
