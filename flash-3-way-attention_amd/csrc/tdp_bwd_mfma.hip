@@ -540,35 +540,42 @@ __device__ __forceinline__ void tdp_bwd_rows_body(const BwdParams<E>& p, const i
     }
 }
 
-template <typename E, int D, bool WITH_DQ, bool SV, bool WIN>
-__global__ __launch_bounds__(512) void tdp_bwd_rows_kernel(BwdParams<E> p) {
-    tdp_bwd_rows_body<E, D, WITH_DQ, SV, WIN>(p, blockIdx.x);
-}
-
-// The same grid together with the fp32 workgroups of query tile 0 (tdp_f32_tiles.hpp: both roles, one workgroup per
-// round of eight rows; t0_x * 2 * rounds of them).  As a launch of their own they are 64 short workgroups between two
-// launches that fill the chip, 30 us in which most of it idles.  Here they come after the main blocks, beside the
-// last and lightest tiles of the launch (t0_first = 0: large grids, whose heavy tiles should start at once), or
-// before them (small grids: the main blocks are as short as these, and a latency-bound workgroup that starts last
-// is the launch's tail).  They add to the same accumulators as every other workgroup, in fixed point, so the order
-// changes nothing.
-template <typename E, int D, bool WITH_DQ, bool SV, bool WIN>
-__global__ __launch_bounds__(512) void tdp_bwd_rows_tile0_kernel(BwdParams<E> p, F32BwdParams<E> r0, F32BwdParams<E> r1,
-                                                                 int roles_mask, int main_blocks, int t0_x, int t0_first) {
-    const int t0_blocks = t0_x * 2 * r0.split_rounds;
-    const int block = (int)blockIdx.x - (t0_first ? t0_blocks : 0);  // main blocks: 0 .. main_blocks - 1
-    if (block >= 0 && block < main_blocks) {
-        tdp_bwd_rows_body<E, D, WITH_DQ, SV, WIN>(p, block);
-    } else {
-        const int extra = t0_first ? (int)blockIdx.x : block - main_blocks;
-        f32_tile0_block<E, D, D>(r0, r1, roles_mask, extra / t0_x, extra % t0_x);
+// Both roles in one grid: first_blocks workgroups of rows = (K2, V2) (with dQ, if that is wanted) and then those of rows = (K1, U).
+// They read the same tensors and add to different sums; as two launches each ended in a tail of its own.  With T0 (a causal mask)
+// the fp32 workgroups of query tile 0 (tdp_f32_tiles.hpp: both roles, one workgroup per round of eight rows; t0_x * 2 * rounds of
+// them) join the grid.  As a launch of their own they are 64 short workgroups between two launches that fill the chip, 30 us in
+// which most of it idles.  They come after the main blocks, beside the last and lightest tiles (t0_first = 0: large grids, whose
+// heavy tiles should start at once), or before them (small grids: the main blocks are as short as these, and a latency-bound
+// workgroup that starts last is the launch's tail).  They add to the same accumulators as every other workgroup, in fixed
+// point, so the order changes nothing.
+// Two launches -> one (and the pass ahead dealt out, bwd_prep_kernel), training steps: B=2 H=4 T=256 158.5 -> 147 us, B=4 H=8 T=256 428
+// -> 404, B=1 H=8 T=700 window 100 286 -> 259; B=4 H=8 T=1024 13.7 ms either way.
+template <typename E>
+struct BothRoles {
+    BwdParams<E> p1, p2;
+    int first_blocks, main_blocks;  // workgroups of the first role, of both
+    F32BwdParams<E> r0, r1;         // T0
+    int roles_mask, t0_x, t0_first;
+};
+template <typename E, int D, bool WITH_DQ, bool SV, bool WIN, bool T0>
+__global__ __launch_bounds__(512) void tdp_bwd_rows_kernel(BothRoles<E> a) {
+    const int t0_blocks = T0 ? a.t0_x * 2 * a.r0.split_rounds : 0;
+    const int block = (int)blockIdx.x - (T0 && a.t0_first ? t0_blocks : 0);  // main blocks: 0 .. main_blocks - 1
+    if (!T0 || (block >= 0 && block < a.main_blocks)) {
+        if (block < a.first_blocks) tdp_bwd_rows_body<E, D, WITH_DQ, SV, WIN>(a.p1, block);
+        else tdp_bwd_rows_body<E, D, false, SV, WIN>(a.p2, block - a.first_blocks);
+    } else if constexpr (T0) {
+        const int extra = a.t0_first ? (int)blockIdx.x : block - a.main_blocks;
+        f32_tile0_block<E, D, D>(a.r0, a.r1, a.roles_mask, extra / a.t0_x, extra % a.t0_x);
     }
 }
 
 // ------------------------------------------------------------------------------------------
 // scratch producers / consumers
-// U = SiLU(V1) row-major; U^T and K1^T as [D][Tp] (zero padded); Delta = rowsum(dO*O);
-// zero the fp32 accumulators.
+// U = SiLU(V1) row-major; U^T, K1^T, K2^T and V2^T as [D][Tp] (zero padded); Delta = rowsum(dO*O); the partial maxima of |dO|;
+// the accumulators and poison words cleared.  One kind of work per blockIdx.z (kPrepJobs): a workgroup that did all of it for its
+// 64 rows was a chain of four round trips, 13 us at B=2 H=4 T=256, where few workgroups share the chip.
+constexpr int kPrepJobs = 4;
 template <typename E>
 __global__ __launch_bounds__(256) void bwd_prep_kernel(const E* __restrict__ v1, const E* __restrict__ k1,
                                                        const E* __restrict__ k2, const E* __restrict__ v2,
@@ -590,43 +597,47 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(const E* __restrict__ v1,
     const int b_ = bh / H, h_ = bh % H;
     auto slice = [&](const E* t, const TensorAt& at) { return t + (size_t)b_ * at.sb + (size_t)h_ * at.sh; };
     v1 = slice(v1, at_v1); k1 = slice(k1, at_k1); k2 = slice(k2, at_k2); v2 = slice(v2, at_v2); d_o = slice(d_o, at_do);
+    const int job = blockIdx.z;
+    if (job < 2) {  // two tiles at a time (static LDS stays under 64 KB at D = 128): their loads are in flight together
+        constexpr int kTile = 64 * (128 + 2);
+        __shared__ E tiles[2 * kTile];
+        if (job == 0) {
+            transpose_load<E, true>(v1, u + base, tiles, j0, T, D, at_v1.st);
+            transpose_load<E, false>(k1, nullptr, tiles + kTile, j0, T, D, at_k1.st);
+        } else {
+            transpose_load<E, false>(k2, nullptr, tiles, j0, T, D, at_k2.st);
+            transpose_load<E, false>(v2, nullptr, tiles + kTile, j0, T, D, at_v2.st);
+        }
+        __syncthreads();
+        transpose_store<E>((job == 0 ? ut : k2t) + tbase, tiles, j0, Tp, D);
+        transpose_store<E>((job == 0 ? k1t : v2t) + tbase, tiles + kTile, j0, Tp, D);
+        return;
+    }
+    if (job == 2) {  // the accumulators: zero_width 4-byte words per row (D floats, or D 64-bit fixed-point sums)
+        if (scale_parts && threadIdx.x < 64 && j0 + threadIdx.x < T) poison[(size_t)bh * T + j0 + threadIdx.x] = 0;
+        const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
+        for (int idx = threadIdx.x; idx < 64 * (zero_width / 4); idx += 256) {
+            const int j = j0 + idx / (zero_width / 4);
+            if (j < T) {
+                const size_t off = ((size_t)bh * T + j) * zero_width + (idx % (zero_width / 4)) * 4;
+                *reinterpret_cast<float4*>(zero_a + off) = z4;
+                *reinterpret_cast<float4*>(zero_b + off) = z4;
+                *reinterpret_cast<float4*>(zero_c + off) = z4;
+                *reinterpret_cast<float4*>(zero_d + off) = z4;
+                if (zero_e) *reinterpret_cast<float4*>(zero_e + off) = z4;
+            }
+        }
+        return;
+    }
     if (scale_parts) {
-        // fixed-point accumulators: clear the poison words of this block's rows; the first blocks of a slice
-        // also leave the partial maxima of |dO| that fix the slice's scale (part s = 64-row blocks s, s + 8, ...)
+        // the first blocks of a slice leave the partial maxima of |dO| that fix the slice's scale (part s = 64-row blocks s,
+        // s + 8, ...)
         __shared__ unsigned red[4];
-        if (threadIdx.x < 64 && j0 + threadIdx.x < T) poison[(size_t)bh * T + j0 + threadIdx.x] = 0;
         for (int part = blockIdx.x; part < kScaleParts; part += gridDim.x) {
             unsigned m = 0;
             for (int r0 = part * 64; r0 < T; r0 += kScaleParts * 64)
                 m = max(m, block_absmax_bits<E>(d_o + (size_t)r0 * at_do.st, (size_t)min(64, T - r0) * D / 8, red, D / 8, at_do.st));
             if (threadIdx.x == 0) scale_parts[bh * kScaleParts + part] = m;
-        }
-    }
-    // two tiles at a time (static LDS stays under 64 KB at D = 128): their loads are in flight together
-    constexpr int kTile = 64 * (128 + 2);
-    __shared__ E tiles[2 * kTile];
-    transpose_load<E, true>(v1, u + base, tiles, j0, T, D, at_v1.st);
-    transpose_load<E, false>(k1, nullptr, tiles + kTile, j0, T, D, at_k1.st);
-    __syncthreads();
-    transpose_store<E>(ut + tbase, tiles, j0, Tp, D);
-    transpose_store<E>(k1t + tbase, tiles + kTile, j0, Tp, D);
-    __syncthreads();
-    transpose_load<E, false>(k2, nullptr, tiles, j0, T, D, at_k2.st);
-    transpose_load<E, false>(v2, nullptr, tiles + kTile, j0, T, D, at_v2.st);
-    __syncthreads();
-    transpose_store<E>(k2t + tbase, tiles, j0, Tp, D);
-    transpose_store<E>(v2t + tbase, tiles + kTile, j0, Tp, D);
-    // the accumulators: zero_width 4-byte words per row (D floats, or D 64-bit fixed-point sums)
-    const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int idx = threadIdx.x; idx < 64 * (zero_width / 4); idx += 256) {
-        const int j = j0 + idx / (zero_width / 4);
-        if (j < T) {
-            const size_t off = ((size_t)bh * T + j) * zero_width + (idx % (zero_width / 4)) * 4;
-            *reinterpret_cast<float4*>(zero_a + off) = z4;
-            *reinterpret_cast<float4*>(zero_b + off) = z4;
-            *reinterpret_cast<float4*>(zero_c + off) = z4;
-            *reinterpret_cast<float4*>(zero_d + off) = z4;
-            if (zero_e) *reinterpret_cast<float4*>(zero_e + off) = z4;
         }
     }
     // Delta[j] = dO[j] . O[j]: the D / 8 lanes that hold a row's 16-byte pieces sit next to each other
@@ -814,7 +825,7 @@ static hipError_t launch_bwd(const MfmaBwdArgs& a, hipStream_t st) {
     if (knobs().bwd_splits > 0) splits = std::min(16, knobs().bwd_splits);  // tuning sweeps
     float* dqacc = splits > 1 ? (float*)(ws + l.dqacc) : nullptr;
 
-    hipLaunchKernelGGL(bwd_prep_kernel<E>, dim3(Tp / 64, a.BH), dim3(256), 0, st, (const E*)a.v1, (const E*)a.k1,
+    hipLaunchKernelGGL(bwd_prep_kernel<E>, dim3(Tp / 64, a.BH, kPrepJobs), dim3(256), 0, st, (const E*)a.v1, (const E*)a.k1,
                        (const E*)a.k2, (const E*)a.v2, (const E*)a.o, (const E*)a.d_o, (E*)(ws + l.u),
                        (E*)(ws + l.ut), (E*)(ws + l.k1t), (E*)(ws + l.k2t), (E*)(ws + l.v2t),
                        (float*)(ws + l.delta), dk1acc, duacc, dk2acc, dv2acc, dqacc, a.T, Tp, D,
@@ -840,8 +851,9 @@ static hipError_t launch_bwd(const MfmaBwdArgs& a, hipStream_t st) {
     // D = 64, full windows and windows that no k-k band cuts: three stage buffers of four 64x64 tiles, two rounds of 8 K2 / V2 rows, the Q and dO
     // tiles (twice: operand and epilogue layout), four dQ slices.  Otherwise: tdp_bwd_rows_general.hpp
     size_t smem;
-    void (*kern_dq)(BwdParams<E>);
-    void (*kern_nodq)(BwdParams<E>);
+    void (*kern_dq)(BwdParams<E>) = nullptr;
+    void (*kern_nodq)(BwdParams<E>) = nullptr;
+    void (*kern_both)(BothRoles<E>) = nullptr;  // both roles in one grid
     int nthreads = 512, col_parts = 1;
     bool plain64 = false;  // the D = 64 kernel of this file
     // The D = 64 kernel of this file takes windows that kk_left / kk_right do not cut (no pair inside the k1 and k2 windows
@@ -908,12 +920,8 @@ static hipError_t launch_bwd(const MfmaBwdArgs& a, hipStream_t st) {
     } else {
         smem = 2 * (size_t)(3 * 4 * 64 * 64 + 2 * 2 * 8 * 64 + 2 * (64 / 32) * 64 * 16) +
                4 * (size_t)(2 * 32 * (64 + 4) + 4 * 32 * 64);
-        kern_dq = a.windowed ? tdp_bwd_rows_kernel<E, 64, true, SV, true> : tdp_bwd_rows_kernel<E, 64, true, SV, false>;
-        kern_nodq = a.windowed ? tdp_bwd_rows_kernel<E, 64, false, SV, true> : tdp_bwd_rows_kernel<E, 64, false, SV, false>;
         plain64 = true;
     }
-    if (hipError_t e = ensure_dynamic_smem(reinterpret_cast<const void*>(kern_dq), smem); e != hipSuccess) return e;
-    if (hipError_t e = ensure_dynamic_smem(reinterpret_cast<const void*>(kern_nodq), smem); e != hipSuccess) return e;
     const bool want_q = a.dq != nullptr, want_k2 = a.dk2 || a.dv2, want_k1 = a.dk1 || a.dv1;
     // Under a causal mask the first query tile goes through the fp32 kernel (tdp_f32_mfma.hip): its softmax rows
     // are nearly one-hot, and dS = P (dP - Delta) then cancels two numbers whose 16-bit operand rounding the
@@ -958,37 +966,32 @@ static hipError_t launch_bwd(const MfmaBwdArgs& a, hipStream_t st) {
     p.at_row_k = a.at_k2; p.at_row_v = a.at_v2; p.at_st_k = a.at_k1; p.at_st_v = at_u;
     p.acc_k = dk2acc; p.acc_v = dv2acc; p.bit_k = kPoisonDK2; p.bit_v = kPoisonDV2;
     p.wa = a.k1_window; p.wb = a.k2_window; p.lab = a.kk_left; p.rab = a.kk_right;
-    hipError_t launch_error = hipSuccess;
-    auto launch_rows = [&](bool with_dq) {
-        if constexpr (D == 64) {
-            if (fuse_tile0) {  // the first launch takes tile 0 along
-                auto fused = a.windowed ? (with_dq ? tdp_bwd_rows_tile0_kernel<E, 64, true, SV, true>
-                                                   : tdp_bwd_rows_tile0_kernel<E, 64, false, SV, true>)
-                                        : (with_dq ? tdp_bwd_rows_tile0_kernel<E, 64, true, SV, false>
-                                                   : tdp_bwd_rows_tile0_kernel<E, 64, false, SV, false>);
-                launch_error = ensure_dynamic_smem(reinterpret_cast<const void*>(fused), std::max(smem, f32_bwd_smem<64>()));
-                if (launch_error != hipSuccess) return;
-                const int t0_x = 8 * xcd_slots(a.BH, 1);
-                const int t0_first = tiles < 1024 ? 1 : 0;
-                hipLaunchKernelGGL(fused, dim3(grid.x + t0_x * 2 * t0_rounds), dim3(512), std::max(smem, f32_bwd_smem<64>()),
-                                   st, p, t0_r0, t0_r1, t0_roles, (int)grid.x, t0_x, t0_first);
-                fuse_tile0 = false;
-                return;
-            }
-        }
-        hipLaunchKernelGGL(with_dq ? kern_dq : kern_nodq, grid, dim3(nthreads), smem, st, p);
-    };
-    // a launch whose gradients the caller does not want (null outputs) is skipped
-    if (tiles_here > 0 && want_q) launch_rows(true);
-    else if (tiles_here > 0 && want_k2) launch_rows(false);
     // rows = (K1, U), streamed = (K2, V2): dK1, dU
-    p.row_k = (const E*)a.k1; p.row_v = u;
-    p.st_k = (const E*)a.k2; p.st_v = (const E*)a.v2; p.st_kt = k2t; p.st_vt = v2t;
-    p.at_row_k = a.at_k1; p.at_row_v = at_u; p.at_st_k = a.at_k2; p.at_st_v = a.at_v2;
-    p.acc_k = dk1acc; p.acc_v = duacc; p.bit_k = kPoisonDK1; p.bit_v = kPoisonDU;
-    p.wa = a.k2_window; p.wb = a.k1_window; p.lab = a.kk_right; p.rab = a.kk_left;  // the mask with j and k exchanged
-    if (tiles_here > 0 && want_k1) launch_rows(false);
-    if (launch_error != hipSuccess) return launch_error;
+    BwdParams<E> p2 = p;
+    p2.row_k = (const E*)a.k1; p2.row_v = u;
+    p2.st_k = (const E*)a.k2; p2.st_v = (const E*)a.v2; p2.st_kt = k2t; p2.st_vt = v2t;
+    p2.at_row_k = a.at_k1; p2.at_row_v = at_u; p2.at_st_k = a.at_k2; p2.at_st_v = a.at_v2;
+    p2.acc_k = dk1acc; p2.acc_v = duacc; p2.bit_k = kPoisonDK1; p2.bit_v = kPoisonDU;
+    p2.wa = a.k2_window; p2.wb = a.k1_window; p2.lab = a.kk_right; p2.rab = a.kk_left;  // the mask with j and k exchanged
+    // a role whose gradients the caller does not want (null outputs) is left out
+    const bool first = tiles_here > 0 && (want_q || want_k2), second = tiles_here > 0 && want_k1;
+    if (plain64) {
+        if constexpr (D == 64)
+            kern_both = a.windowed ? (fuse_tile0 ? (want_q ? tdp_bwd_rows_kernel<E, 64, true, SV, true, true> : tdp_bwd_rows_kernel<E, 64, false, SV, true, true>)
+                                                 : (want_q ? tdp_bwd_rows_kernel<E, 64, true, SV, true, false> : tdp_bwd_rows_kernel<E, 64, false, SV, true, false>))
+                                   : (fuse_tile0 ? (want_q ? tdp_bwd_rows_kernel<E, 64, true, SV, false, true> : tdp_bwd_rows_kernel<E, 64, false, SV, false, true>)
+                                                 : (want_q ? tdp_bwd_rows_kernel<E, 64, true, SV, false, false> : tdp_bwd_rows_kernel<E, 64, false, SV, false, false>));
+        if (fuse_tile0) smem = std::max(smem, f32_bwd_smem<64>());
+        BothRoles<E> both{p, p2, first ? (int)grid.x : 0, (first ? (int)grid.x : 0) + (second ? (int)grid.x : 0), t0_r0, t0_r1, t0_roles, 8 * xcd_slots(a.BH, 1), tiles < 1024 ? 1 : 0};
+        const int blocks = both.main_blocks + (fuse_tile0 ? both.t0_x * 2 * t0_rounds : 0);
+        if (hipError_t e = ensure_dynamic_smem(reinterpret_cast<const void*>(kern_both), smem); e != hipSuccess) return e;
+        if (first || second) hipLaunchKernelGGL(kern_both, dim3(blocks), dim3(512), smem, st, both);
+    } else {
+        if (hipError_t e = ensure_dynamic_smem(reinterpret_cast<const void*>(kern_dq), smem); e != hipSuccess) return e;
+        if (hipError_t e = ensure_dynamic_smem(reinterpret_cast<const void*>(kern_nodq), smem); e != hipSuccess) return e;
+        if (first) hipLaunchKernelGGL(want_q ? kern_dq : kern_nodq, grid, dim3(nthreads), smem, st, p);
+        if (second) hipLaunchKernelGGL(kern_nodq, grid, dim3(nthreads), smem, st, p2);
+    }
 
     const size_t n = (size_t)a.BH * a.T * D;
     size_t gridf = (n + 255) / 256;
