@@ -217,8 +217,10 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attn_fwd_f32m_kernel(FwdP p) {
     const float *X = p.X + base, *K = p.K + base, *V = p.V + base;
     const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // heavy first: under a causal mask the last owner tiles stream the most rows
-    const int r0 = (p.causal ? ntiles - 1 - order : order) * 32, r = r0 + n;
+    // heavy first: under a causal mask the last owner tiles stream the most rows.  A grid that the CUs take whole, two workgroups
+    // each, goes in the other direction from the middle on, so that a heavy tile shares its CU with a light one
+    const bool whole = p.BH * ntiles <= 512 && order >= (ntiles + 1) / 2;
+    const int r0 = (!p.causal ? order : whole ? order - (ntiles + 1) / 2 : ntiles - 1 - order) * 32, r = r0 + n;
     const int a_lo = p.causal ? max(0, r0 - p.k_diff) & ~31 : 0, a_hi = p.causal ? min(T - 1, r0 + 31) : T - 1;
 
     f32x16 acc[DT];
