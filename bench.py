@@ -6,7 +6,7 @@ B=4 H=8 T=1024 D=64 bf16 causal (inputs resident in HBM before the timed
 region).  Prints ONE JSON line.  `value` is the algorithmic TFLOP/s of the
 whole step: 16*D*N / time with N = B*H*T(T+1)(2T+1)/6 valid (q,j,k) triples
 (forward 4*D*N, backward 12*D*N).  `roofline` covers the dominant kernel (the backward rows
-kernel, launched twice per step), `roofline_fwd` the forward kernel; both divide by the
+kernel, one launch per step), `roofline_fwd` the forward kernel; both divide by the
 MI355X dense bf16 MFMA peak.
 `cpu_baseline` times the CPU oracle (the reference's naive dense formulation)
 on a bounded sample on this box's host cores.
@@ -34,10 +34,11 @@ TRAFFIC_SOURCE = "profiles/tdp_fwd_bwd_B4_H8_T1024_D64_bf16_counters.txt (rocpro
 # 27.4 MiB fetched + 15.0 MiB written: the algorithmic 20 + 4 MiB, and 28 bytes per lane that the kernel's prologue
 # spills (a million lanes: ~11 MiB written once; spill-free builds of the kernel measured 2 % slower)
 TRAFFIC_FWD = 44.4e6
-# average of the two launches: 587 / 527 MiB written (64-bit atomics; the first launch also spills 16-20 bytes per lane), 36 / 39 MiB fetched (some runs: up to 440 MiB in the first
-# launch, when its accumulators fall out of their XCD's L2; the bytes are L2 <-> fabric traffic, which the 256 MB Infinity
-# Cache absorbs)
-TRAFFIC_BWD_ROWS = 624e6
+# both roles of the rows kernel: 587 + 527 MiB written (64-bit atomics; 16-20 bytes per lane of the role with dQ are
+# spilled), 36 + 39 MiB fetched (some runs: up to 440 MiB, when its accumulators fall out of their XCD's L2; the bytes
+# are L2 <-> fabric traffic, which the 256 MB Infinity Cache absorbs).  Measured when each role was a launch of its own;
+# their sum.
+TRAFFIC_BWD_ROWS = 1248e6
 
 
 def triples(B, H, T, causal=True):
@@ -503,18 +504,16 @@ def main():
                    "peak_used": "2.5 PFLOP/s bf16 dense (256 CUs x 4096 flop/clk x 2.4 GHz nominal)",
                    # measured in this run: what a pure-MFMA kernel reaches, and the clock that implies
                    "mfma_probe": probe},
-        # dominant kernel by time: the rows kernel of the backward, launched twice (dQ,dK2,dV2 then dK1,dU; the
-        # first launch is tdp_bwd_rows_tile0_kernel, the same body with the 128 fp32 workgroups of query tile 0 in
-        # its grid, the second tdp_bwd_rows_kernel).  Each launch is credited half of the backward's algorithmic
-        # flops (6*D*N) and half of the event-timed backward (the prep/finish kernels in that time are < 1 %).
+        # dominant kernel by time: the rows kernel of the backward, one launch with both roles (dQ,dK2,dV2 and dK1,dU)
+        # and the 128 fp32 workgroups of query tile 0 in its grid.  It is credited the backward's algorithmic flops
+        # and the event-timed backward (the prep/finish kernels in that time are < 1 %).
         "roofline": {"bound": "mfma",
-                     "kernel": "tdp_bwd_rows_tile0_kernel<bf16,64,true> + tdp_bwd_rows_kernel<bf16,64,false> (the rows "
-                               "kernel's two launches, averaged)",
+                     "kernel": "tdp_bwd_rows_kernel<bf16,64> (both roles and query tile 0 in one launch)",
                      "achieved": bwd_tf, "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
                      "frac": bwd_tf / PEAK_BF16_TFLOPS, "traffic": TRAFFIC_BWD_ROWS if default_workload else None,
                      "traffic_source": TRAFFIC_SOURCE if default_workload else None,
                      "frac_of_sustained_mfma_rate": bwd_tf / probe["tflops"],
-                     "flops_per_launch": f_bwd // 2, "ms_per_launch": ms_bwd / 2},
+                     "flops_per_launch": f_bwd, "ms_per_launch": ms_bwd},
         "roofline_fwd": {"bound": "mfma", "kernel": "tdp_fwd_mfma_kernel<bf16,64,NT=2,8 waves>",
                          "achieved": fwd_tf, "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
                          "frac": fwd_tf / PEAK_BF16_TFLOPS, "traffic": TRAFFIC_FWD if default_workload else None,

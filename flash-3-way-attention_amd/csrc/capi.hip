@@ -194,7 +194,7 @@ void fill_inputs(const void* q, const void* k1, const void* k2, const void* v1, 
 
 int clampw(int w, int T) { return w > T ? T : w; }
 
-// The fp32 path has two sets of kernels: on the matrix cores (v_mfma_f32_32x32x2_f32; D = 32, 64 and 128), which deal the
+// The fp32 path has two sets of kernels: on the matrix cores (products of split operands; D = 32, 64 and 128), which deal the
 // rounds of a query tile out over workgroups and are the faster ones at every size (B=1 H=1 T=16 D=64: forward 14 against
 // 27 us, backward 32 against 200 us), and on the vector ALUs (D = 8 and 16, and TRITT_TUNE_F32_VALU).
 bool use_f32_mfma() { return knobs().f32_valu == 0; }
@@ -327,7 +327,7 @@ int tdp_bwd_generic(Arena& ar, bool run, const void* q, const void* k1, const vo
 }
 
 // ---------------------------------------------------------------- dot-product-sum
-// fp32 path: the attention kernels on the fp32 matrix cores where they exist (D = 32, 64), else one lane per row on
+// fp32 path: the attention kernels on the matrix cores where they exist (D = 32, 64), else one lane per row on
 // the vector ALUs; TRITT_TUNE_F32_VALU forces the latter
 bool use_f32_mfma_dps(int D) { return !knobs().f32_valu && f32_mfma_dps_supported(D); }
 

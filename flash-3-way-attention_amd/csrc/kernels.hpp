@@ -43,7 +43,7 @@ struct GenericTdpArgs {
     int BH, T, D;
     float alpha;
     int causal, k1_window, k2_window, kk_left, kk_right;
-    // fp32 MFMA forward: workgroups per query tile at most (f32_fwd_parts) and, above 1, room for that many parts per row
+    // fp32 matrix-core forward: workgroups per query tile at most (f32_fwd_parts) and, above 1, room for that many parts per row
     int fwd_parts;
     float* part;
     void* images;  // forward: room for the streamed tensors' images (f32_fwd_image_bytes), or null: they are split as they are staged
@@ -52,7 +52,7 @@ struct GenericTdpArgs {
 hipError_t generic_tdp_fwd(const GenericTdpArgs& a, hipStream_t st);
 hipError_t generic_tdp_bwd(const GenericTdpArgs& a, hipStream_t st);
 
-// fp32 MFMA triple-dot kernels (D = 32, 64 or 128, any mask): same operands as the VALU kernels
+// fp32 matrix-core triple-dot kernels (D = 32, 64 or 128, any mask): same operands as the VALU kernels
 bool f32_mfma_tdp_supported(int D);
 // workgroups per query tile that the forward of this problem is dealt out to (BH, T, D and the mask of `a`)
 int f32_fwd_parts(const GenericTdpArgs& a);
@@ -123,7 +123,7 @@ struct DpsArgs {
 };
 hipError_t dps_fwd(const DpsArgs& a, hipStream_t st);
 hipError_t dps_bwd(const DpsArgs& a, hipStream_t st);
-// the same two calls with the attention kernels on the fp32 matrix cores (D = 32 or 64)
+// the same two calls with the attention kernels on the matrix cores (D = 32 or 64)
 bool f32_mfma_dps_supported(int D);
 hipError_t f32_mfma_dps_fwd(const DpsArgs& a, hipStream_t st);
 hipError_t f32_mfma_dps_bwd(const DpsArgs& a, hipStream_t st);

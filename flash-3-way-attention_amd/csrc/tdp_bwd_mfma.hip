@@ -7,10 +7,9 @@
 // six contractions are needed per valid (q,j,k):
 //   S, dP, dS K1 (-> dQ, dK2), P U (-> dV2), and by the symmetry (K1,U,j) <-> (K2,V2,k) of the
 //   whole problem, dS K2 (-> dK1) and P V2 (-> dU).
-// One kernel template, tdp_bwd_rows_kernel, is launched twice, each launch recomputing S and dP
-// (8 products executed for 6):
-//   launch 1: rows = (K2, V2), streamed = (K1, U):  dQ (owner-computes), dK2, dV2
-//   launch 2: rows = (K1, U),  streamed = (K2, V2): dK1, dU
+// tdp_bwd_rows_kernel runs two roles in one grid, each of which recomputes S and dP (8 products executed for 6):
+//   first:  rows = (K2, V2), streamed = (K1, U):  dQ (owner-computes), dK2, dV2
+//   second: rows = (K1, U),  streamed = (K2, V2): dK1, dU
 // See the comment above the kernel.
 #include <algorithm>
 #include <cstdlib>
@@ -929,8 +928,8 @@ static hipError_t launch_bwd(const MfmaBwdArgs& a, hipStream_t st) {
     // tile 1: the grid simply has one tile less, and the heaviest-first numbering never reaches tile 0.
     // (all_in_f32: every tile does)
     const bool first_in_f32 = a.causal != 0;
-    // tile 0's backward workgroups ride at the end of the first rows launch below where that is the D = 64 kernel
-    // (tdp_bwd_rows_tile0_kernel); otherwise they are a launch of their own
+    // tile 0's backward workgroups are part of the rows kernel's grid where that is the D = 64 one (BothRoles);
+    // otherwise they are a launch of their own
     bool fuse_tile0 = false;
     [[maybe_unused]] F32BwdParams<E> t0_r0{}, t0_r1{};
     [[maybe_unused]] int t0_roles = 0, t0_rounds = 0;

@@ -1,19 +1,21 @@
-// Triple-dot-product trittention in true fp32 on the matrix cores (v_mfma_f32_32x32x2_f32), D = 32, 64 or 128,
-// every mask.  This is the path of fp32 tensors: fp32 operands, fp32 products, fp32 accumulation (the 1e-4
-// relative bar), at the fp32 matrix rate (157 TFLOP/s peak) instead of the fp32 vector rate of the VALU kernels.
+// Triple-dot-product trittention for fp32 tensors on the matrix cores, D = 32, 64 or 128, every mask: fp32 operands and sums,
+// every product as six bf16 products of three-way splits (f32_split.hpp; nearer to 64 bits than a chain of fp32 MFMAs, at up
+// to 2.4 PFLOP/s / 6 instead of 157 TFLOP/s).  This file: the passes ahead and behind, the deal of tiles to workgroups and the
+// launchers; tdp_f32_split.hpp: the forward and the backward kernel; tdp_f32_tiles.hpp: the deal's device side and the fp32
+// query tiles of a 16-bit backward.
 //
 // All tensors here are fp32 [BH, T, D]; U = SiLU(V1) (see capi.hip).
 //
-// Formulation (the same virtual-query one as the 16-bit kernels).  A workgroup owns 32 consecutive queries;
-// its waves take consecutive rows b per round (one per wave; b = k, the K2 / V2 row, in the natural orientation) and
-// sweep the streamed index a (= j, K1 / U rows) in 32-row stages shared through LDS.  The rounds of a tile are dealt out
-// over several workgroups by their cost (F32Deal): the forward's parts are joined by f32_merge_kernel and dQ's by
-// f32_finish_kernel; the row gradients, sums over query tiles, meet in fixed-point accumulators, or are left by each tile of
-// a problem of a few tiles and joined like dQ (f32_tile_slabs).
+// Formulation (the same virtual-query one as the 16-bit kernels).  A workgroup owns 32 consecutive rows (queries; the
+// backward has workgroups that own keys as well); its waves take consecutive rows b of (K2, V2) per round, one per wave, and
+// sweep the streamed index a in 32-row stages shared through LDS.  The rounds of a tile are dealt out over several workgroups
+// by their cost (F32Deal): the forward's parts are joined by f32_merge_kernel and those of dQ, dK1 and dU by f32_finish_kernel;
+// dK2 and dV2, sums over tiles, meet in fixed-point accumulators, or are left by each tile of a problem of a few tiles and
+// joined like the others (f32_tile_slabs).
 // For a fixed row b the scores of the 32 queries against 32 streamed rows are one 32x32 tile
 //   S^T[a, q] = sum_d KA[a, d] * (scale * Q[q, d] * KB[b, d])
-// i.e. D / 2 MFMAs (K = 2 each).  The tile leaves the MFMA with lane <-> query and registers <-> streamed rows,
-// which is exactly the B-operand layout of the next product
+// The tile leaves the MFMA with lane <-> query and registers <-> streamed rows, which is (but for the order of the streamed
+// rows) the B-operand layout of the next product
 //   Tv^T[d, q] += sum_a VA^T[d, a] * P^T[a, q]
 // so P is never moved between lanes, and every per-query quantity (running maximum, row sum, the merge of a
 // finished row b into the output, O^T[d, q] += Tv^T[d, q] * VB[b, d]) is lane-local.

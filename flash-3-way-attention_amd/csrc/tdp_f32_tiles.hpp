@@ -1,6 +1,6 @@
-// The device side of the fp32 matrix-core triple-dot kernels (tdp_f32_mfma.hip holds the description and the launchers),
-// as a header: the 16-bit backward appends the workgroups of its fp32 query tile 0 to the grid of its own first launch
-// (tdp_bwd_mfma.hip), so both translation units instantiate these bodies.
+// The deal of query and key tiles to workgroups, shared by the fp32 triple-dot kernels (tdp_f32_mfma.hip has the description),
+// and the fp32 query tiles of a 16-bit backward on v_mfma_f32_32x32x2_f32: their statistics pass and their backward, as a
+// header because the 16-bit backward appends the workgroups of query tile 0 to its own grid (tdp_bwd_mfma.hip).
 #pragma once
 #include <algorithm>
 
@@ -534,8 +534,8 @@ __global__ __launch_bounds__(64 * NW, 2) void tdp_f32_stats_kernel(F32StatsParam
 }
 
 // ------------------------------------------------------------------------------------------ backward
-// Launched twice, like the 16-bit backward: rows = (K2, V2), streamed = (K1, U) gives dQ, dK2, dV2; with the roles
-// exchanged, dK1 and dU.  Per (query tile, row b, 32 streamed rows):
+// The fp32 query tiles of a 16-bit backward, in two roles: rows = (K2, V2), streamed = (K1, U) gives dQ, dK2, dV2; with the
+// roles exchanged, dK1 and dU.  Per (query tile, row b, 32 streamed rows):
 //   S^T, dP^T (D / 2 MFMAs each),  P = exp2(S - LSE2[q]),  dS = P (dP - Delta[q])   (both lane-local)
 //   Yq^T[d, q] += KA^T[d, a] dS^T[a, q]      Tv^T[d, q] += VA^T[d, a] P^T[a, q]      (DOUT / 2 MFMAs each)
 // and when the row is finished
