@@ -8,7 +8,8 @@
 // over 64 is 1.44e-7 off on fp32 MFMAs, 1.10e-7 with the six products of each k-step in turn (products_of_step) and 0.50e-7
 // with all the small ones ahead of the large ones (small_products, large_product); over 1024, 5.7e-7 and 4.9e-7.
 //
-// Infinite operands: h is infinite and m NaN, so every result that they enter is NaN (fp32 MFMAs leave some of them infinite).
+// Infinite operands, and those above 3.39e38, which h rounds to infinity: m is NaN, so every result that they enter is NaN (fp32
+// MFMAs leave some of them infinite).
 #pragma once
 #include "mfma.hpp"
 
