@@ -25,6 +25,8 @@
 // so P never moves between lanes and every per-owner quantity (running maximum, sums, LSE, Delta) is lane-local.
 // MFMA row n of output tile dt is column d = (D / 32) n + dt, so that a lane's loads are as wide as D allows.
 // One owner per output element: no atomics, bitwise reproducible.
+#include <type_traits>
+
 #include "common.hpp"
 #include "kernels.hpp"
 #include "f32_split.hpp"
@@ -87,26 +89,45 @@ __device__ __forceinline__ float load_vec(const float* src, int row0, int T, int
     const __amdgpu_buffer_rsrc_t rows = tile_rows<1>(src, row0, T);
     return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rows, 4 * n, 0, 0));
 }
+// ANY: the values may be infinite (split8_any).  Testing every value of a step for that would cost a tenth of its vector
+// instructions, so a wave forms its share with split8, whose third plane is NaN for such a value, and forms it again if a NaN
+// came out of it (B=2 H=8 T=1000 D=64 k_diff 128, backward 119.5 -> 120.5 us, forward 40.6 both).
+template <bool ANY, typename X>
+__device__ __forceinline__ Split8 split_value(const X& x) {
+    if constexpr (ANY) return split8_any(x);
+    else return split8(x);
+}
+template <bool ANY>
 __device__ __forceinline__ Split8 split_at(const float* x) {
     float v[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] = x[e];
-    return split8(v);
+    return split_value<ANY>(v);
+}
+template <int DT>
+__device__ __forceinline__ bool any_nan(const f32x16 (&acc)[DT]) {
+    float sum[4] = {0.f, 0.f, 0.f, 0.f};  // (infinities that cancel are taken for one: the share is formed again for nothing)
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) sum[i % 4] += acc[dt][i];
+    const float all = sum[0] + sum[1] + (sum[2] + sum[3]);
+    return __any(all != all);
 }
 // S^T of a tile; own(ks): the owner's operand of k-step ks.  The small products of all k-steps come first, and the split of a
 // k-step's streamed operand stands beside the products of the one before.
-template <int D, typename F>
+template <int D, bool ANY, typename F>
 __device__ __forceinline__ f32x16 score_tile(const float (&rows)[D / 2], const F& own) {
     constexpr int KS = D / 16;
     f32x16 s;
 #pragma unroll
     for (int i = 0; i < 16; ++i) s[i] = 0.f;
-    Split8 a = split_at(rows);
+    Split8 a = split_at<ANY>(rows);
     bf16x8 h[KS];
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
         Split8 next = a;
-        if (ks + 1 < KS) next = split_at(rows + 8 * (ks + 1 < KS ? ks + 1 : 0));
+        if (ks + 1 < KS) next = split_at<ANY>(rows + 8 * (ks + 1 < KS ? ks + 1 : 0));
         s = small_products(a, own(ks), s);
         h[ks] = a.h;
         a = next;
@@ -116,7 +137,7 @@ __device__ __forceinline__ f32x16 score_tile(const float (&rows)[D / 2], const F
     return s;
 }
 // acc^T[d, owner] += sum over the 32 streamed rows of cols[row, d] * w[row, owner]   (w in score-tile layout)
-template <int D>
+template <int D, bool ANY>
 __device__ __forceinline__ void output_tile(f32x16 (&acc)[D / 32], const float (&cols)[D / 2], const f32x16& w) {
     constexpr int DT = D / 32;
 #pragma unroll
@@ -124,13 +145,13 @@ __device__ __forceinline__ void output_tile(f32x16 (&acc)[D / 32], const float (
         float x[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) x[e] = w[8 * half + e];
-        const Split8 b = split8(x);
+        const Split8 b = split_value<ANY>(x);
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
             float v[8];
 #pragma unroll
             for (int e = 0; e < 8; ++e) v[e] = cols[(8 * half + e) * DT + dt];
-            acc[dt] = products_of_step(split8(v), b, acc[dt]);
+            acc[dt] = products_of_step(split_value<ANY>(v), b, acc[dt]);
         }
     }
 }
@@ -224,72 +245,79 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attn_fwd_f32m_kernel(FwdP p) {
     const int a_lo = p.causal ? max(0, r0 - p.k_diff) & ~31 : 0, a_hi = p.causal ? min(T - 1, r0 + 31) : T - 1;
 
     f32x16 acc[DT];
-    clear<D>(acc);
-    float m = -INFINITY, l = 0.f;
-    int a0 = a_lo + 32 * wave;
-    if (a0 <= a_hi) {
-        float bias = p.bias ? load_vec(p.bias + vbase, a0, T, n) : 0.f;
-        float x[D / 2], rows[D / 2], cols[D / 2];
-        load_rows<D>(x, X, r0, T, n, g);
-        load_rows<D>(rows, K, a0, T, key_of_row(n), g);
-        load_cols<D>(cols, V, a0, T, n, g);
-        Split8 own[KS];
+    float m, l;
+    auto share = [&](auto any) {  // this wave's
+        constexpr bool ANY = decltype(any)::value;
+        clear<D>(acc);
+        m = -INFINITY;
+        l = 0.f;
+        int a0 = a_lo + 32 * wave;
+        if (a0 <= a_hi) {
+            float bias = p.bias ? load_vec(p.bias + vbase, a0, T, n) : 0.f;
+            float x[D / 2], rows[D / 2], cols[D / 2];
+            load_rows<D>(x, X, r0, T, n, g);
+            load_rows<D>(rows, K, a0, T, key_of_row(n), g);
+            load_cols<D>(cols, V, a0, T, n, g);
+            Split8 own[KS];
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            float v[8];
+            for (int ks = 0; ks < KS; ++ks) {
+                float v[8];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] = x[8 * ks + e] * p.scale_log2;
-            own[ks] = split8(v);
-        }
-        for (; a0 <= a_hi; a0 += 32 * kWaves) {
-            const int next = min(a0 + 32 * kWaves, a_hi & ~31);  // (past the end: in bounds, not used)
-            if (p.bias) sh.vec_put(0, bias, wave, n);
-            f32x16 s = score_tile<D>(rows, [&](int ks) -> const Split8& { return own[ks]; });
-            pin_order();
-            load_rows<D>(rows, K, next, T, key_of_row(n), g);
-            if (p.bias) bias = load_vec(p.bias + vbase, next, T, n);
-            pin_order();
-            if (p.bias) {
-#pragma unroll
-                for (int i4 = 0; i4 < 4; ++i4) {
-                    const float4 b = sh.vec_get(0, wave, g, i4);
-                    s[4 * i4] += b.x; s[4 * i4 + 1] += b.y; s[4 * i4 + 2] += b.z; s[4 * i4 + 3] += b.w;
-                }
+                for (int e = 0; e < 8; ++e) v[e] = x[8 * ks + e] * p.scale_log2;
+                own[ks] = split_value<ANY>(v);
             }
-            if (a0 + 32 > T || (p.causal && (a0 + 31 > r0 || r0 + 31 - a0 > p.k_diff))) {
+            for (; a0 <= a_hi; a0 += 32 * kWaves) {
+                const int next = min(a0 + 32 * kWaves, a_hi & ~31);  // (past the end: in bounds, not used)
+                if (p.bias) sh.vec_put(0, bias, wave, n);
+                f32x16 s = score_tile<D, ANY>(rows, [&](int ks) -> const Split8& { return own[ks]; });
+                pin_order();
+                load_rows<D>(rows, K, next, T, key_of_row(n), g);
+                if (p.bias) bias = load_vec(p.bias + vbase, next, T, n);
+                pin_order();
+                if (p.bias) {
+#pragma unroll
+                    for (int i4 = 0; i4 < 4; ++i4) {
+                        const float4 b = sh.vec_get(0, wave, g, i4);
+                        s[4 * i4] += b.x; s[4 * i4 + 1] += b.y; s[4 * i4 + 2] += b.z; s[4 * i4 + 3] += b.w;
+                    }
+                }
+                if (a0 + 32 > T || (p.causal && (a0 + 31 > r0 || r0 + 31 - a0 > p.k_diff))) {
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) {
+                        const int a = a0 + key_of(g, i);
+                        s[i] = ((a < T) & pair_valid(p.causal, p.k_diff, r, a)) ? s[i] : -INFINITY;
+                    }
+                }
+                float mx = s[0];
+#pragma unroll
+                for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
+                mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+                const float m_new = fmaxf(m, mx);
+                const float f = m_new == -INFINITY ? 1.f : fast_exp2(m - m_new);  // nothing seen yet: keep the zeros
+                float ps = 0.f;
 #pragma unroll
                 for (int i = 0; i < 16; ++i) {
-                    const int a = a0 + key_of(g, i);
-                    s[i] = ((a < T) & pair_valid(p.causal, p.k_diff, r, a)) ? s[i] : -INFINITY;
+                    s[i] = s[i] == -INFINITY ? 0.f : fast_exp2(s[i] - m_new);
+                    ps += s[i];
                 }
+                ps += __shfl_xor(ps, 32, 64);
+                l = l * f + ps;
+                m = m_new;
+                if (__any(f != 1.f)) {
+#pragma unroll
+                    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                        for (int i = 0; i < 16; ++i) acc[dt][i] *= f;
+                }
+                output_tile<D, ANY>(acc, cols, s);
+                pin_order();
+                load_cols<D>(cols, V, next, T, n, g);
+                pin_order();
             }
-            float mx = s[0];
-#pragma unroll
-            for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
-            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-            const float m_new = fmaxf(m, mx);
-            const float f = m_new == -INFINITY ? 1.f : fast_exp2(m - m_new);  // nothing seen yet: keep the zeros
-            float ps = 0.f;
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                s[i] = s[i] == -INFINITY ? 0.f : fast_exp2(s[i] - m_new);
-                ps += s[i];
-            }
-            ps += __shfl_xor(ps, 32, 64);
-            l = l * f + ps;
-            m = m_new;
-            if (__any(f != 1.f)) {
-#pragma unroll
-                for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) acc[dt][i] *= f;
-            }
-            output_tile<D>(acc, cols, s);
-            pin_order();
-            load_cols<D>(cols, V, next, T, n, g);
-            pin_order();
         }
-    }
+    };
+    share(std::false_type{});
+    if (any_nan(acc)) share(std::true_type{});
     if (g == 0) sh.row[wave][n] = m;
     __syncthreads();
     float M = sh.row[0][n];
@@ -350,16 +378,16 @@ __device__ __forceinline__ void own_put(Shares<D>& sh, int which, const float* s
         float v[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] = at[e] * scale;
-        const Split8 x = split8(v);
+        const Split8 x = split8_any(v);
         *reinterpret_cast<bf16x8*>(sh.own[which][0] + row * Shares<D>::kOwnLD + c) = x.h;
         *reinterpret_cast<bf16x8*>(sh.own[which][1] + row * Shares<D>::kOwnLD + c) = x.m;
         *reinterpret_cast<bf16x8*>(sh.own[which][2] + row * Shares<D>::kOwnLD + c) = x.l;
     }
 }
-template <int D>
+template <int D, bool ANY>
 __device__ __forceinline__ f32x16 score_tile(const float (&rows)[D / 2], const Shares<D>& sh, int which, int n, int g) {
     asm volatile("" ::: "memory");  // (the reads stay inside the caller's loop)
-    return score_tile<D>(rows, [&](int ks) { return sh.own_operand(which, ks, n, g); });
+    return score_tile<D, ANY>(rows, [&](int ks) { return sh.own_operand(which, ks, n, g); });
 }
 
 template <int D>
@@ -372,62 +400,67 @@ __device__ __forceinline__ void bwd_rows(const BwdP& p, Shares<D>& sh, int bh, i
     const int a_lo = p.causal ? max(0, r0 - p.k_diff) & ~31 : 0, a_hi = p.causal ? min(T - 1, r0 + 31) : T - 1;
     const float scale_log2 = p.alpha * kLog2e;
     f32x16 acc[DT];
-    clear<D>(acc);
-    int a0 = a_lo + 32 * wave;
     own_put<D>(sh, 0, X, r0, T, scale_log2, tid);
     own_put<D>(sh, 1, G, r0, T, 1.f, tid);
     __syncthreads();
-    if (a0 <= a_hi) {
-        float bias = p.bias ? load_vec(p.bias + vbase, a0, T, n) : 0.f;
-        const int nk = key_of_row(n);
-        float ra[D / 2], rb[D / 2];
-        load_rows<D>(ra, K, a0, T, nk, g);
-        load_rows<D>(rb, V, a0, T, nk, g);
-        const float lse2 = p.lse[vbase + rc] * p.lse_to_log2, dl = p.delta[vbase + rc];
-        // two operand sets in turn: the K rows of the next step take the set the V rows are in now
-        auto step = [&](float (&A)[D / 2], float (&B)[D / 2]) {
-            const int next = min(a0 + 32 * kWaves, a_hi & ~31);
-            if (p.bias) sh.vec_put(0, bias, wave, n);
-            f32x16 s = score_tile<D>(A, sh, 0, n, g);
-            pin_order();
-            load_cols<D>(A, K, a0, T, n, g);
-            if (p.bias) bias = load_vec(p.bias + vbase, next, T, n);
-            pin_order();
-            const f32x16 dp = score_tile<D>(B, sh, 1, n, g);
-            pin_order();
-            load_rows<D>(B, K, next, T, nk, g);
-            pin_order();
-            if (p.bias) {
+    auto share = [&](auto any) {
+        constexpr bool ANY = decltype(any)::value;
+        clear<D>(acc);
+        int a0 = a_lo + 32 * wave;
+        if (a0 <= a_hi) {
+            float bias = p.bias ? load_vec(p.bias + vbase, a0, T, n) : 0.f;
+            const int nk = key_of_row(n);
+            float ra[D / 2], rb[D / 2];
+            load_rows<D>(ra, K, a0, T, nk, g);
+            load_rows<D>(rb, V, a0, T, nk, g);
+            const float lse2 = p.lse[vbase + rc] * p.lse_to_log2, dl = p.delta[vbase + rc];
+            // two operand sets in turn: the K rows of the next step take the set the V rows are in now
+            auto step = [&](float (&A)[D / 2], float (&B)[D / 2]) {
+                const int next = min(a0 + 32 * kWaves, a_hi & ~31);
+                if (p.bias) sh.vec_put(0, bias, wave, n);
+                f32x16 s = score_tile<D, ANY>(A, sh, 0, n, g);
+                pin_order();
+                load_cols<D>(A, K, a0, T, n, g);
+                if (p.bias) bias = load_vec(p.bias + vbase, next, T, n);
+                pin_order();
+                const f32x16 dp = score_tile<D, ANY>(B, sh, 1, n, g);
+                pin_order();
+                load_rows<D>(B, K, next, T, nk, g);
+                pin_order();
+                if (p.bias) {
 #pragma unroll
-                for (int i4 = 0; i4 < 4; ++i4) {
-                    const float4 b = sh.vec_get(0, wave, g, i4);
-                    s[4 * i4] += b.x; s[4 * i4 + 1] += b.y; s[4 * i4 + 2] += b.z; s[4 * i4 + 3] += b.w;
+                    for (int i4 = 0; i4 < 4; ++i4) {
+                        const float4 b = sh.vec_get(0, wave, g, i4);
+                        s[4 * i4] += b.x; s[4 * i4 + 1] += b.y; s[4 * i4 + 2] += b.z; s[4 * i4 + 3] += b.w;
+                    }
                 }
-            }
-            const bool edge = a0 + 32 > T || (p.causal && (a0 + 31 > r0 || r0 + 31 - a0 > p.k_diff));
+                const bool edge = a0 + 32 > T || (p.causal && (a0 + 31 > r0 || r0 + 31 - a0 > p.k_diff));
 #pragma unroll
-            for (int i = 0; i < 16; ++i) s[i] = fast_exp2(s[i] - lse2) * (dp[i] - dl);
-            if (edge) {
+                for (int i = 0; i < 16; ++i) s[i] = fast_exp2(s[i] - lse2) * (dp[i] - dl);
+                if (edge) {
 #pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    const int a = a0 + key_of(g, i);
-                    s[i] = ((a < T) & pair_valid(p.causal, p.k_diff, r, a)) ? s[i] : 0.f;
+                    for (int i = 0; i < 16; ++i) {
+                        const int a = a0 + key_of(g, i);
+                        s[i] = ((a < T) & pair_valid(p.causal, p.k_diff, r, a)) ? s[i] : 0.f;
+                    }
                 }
+                output_tile<D, ANY>(acc, A, s);
+                pin_order();
+                load_rows<D>(A, V, next, T, nk, g);
+                pin_order();
+            };
+            while (true) {
+                step(ra, rb);
+                a0 += 32 * kWaves;
+                if (a0 > a_hi) break;
+                step(rb, ra);
+                a0 += 32 * kWaves;
+                if (a0 > a_hi) break;
             }
-            output_tile<D>(acc, A, s);
-            pin_order();
-            load_rows<D>(A, V, next, T, nk, g);
-            pin_order();
-        };
-        while (true) {
-            step(ra, rb);
-            a0 += 32 * kWaves;
-            if (a0 > a_hi) break;
-            step(rb, ra);
-            a0 += 32 * kWaves;
-            if (a0 > a_hi) break;
         }
-    }
+    };
+    share(std::false_type{});
+    if (any_nan(acc)) share(std::true_type{});
     sh.put(acc, p.alpha, wave, n, g);
     __syncthreads();
 #pragma unroll
@@ -454,68 +487,74 @@ __device__ __forceinline__ void bwd_cols(const BwdP& p, Shares<D>& sh, int bh, i
     const int r_lo = p.causal ? c0 : 0, r_hi = p.causal ? (int)min((long)T - 1, (long)c0 + 31 + p.k_diff) : T - 1;
     const float scale_log2 = p.alpha * kLog2e;
     f32x16 accK[DT], accV[DT];
-    clear<D>(accK);
-    clear<D>(accV);
-    float db = 0.f;
-    int rr0 = r_lo + 32 * wave;
+    float db;
     own_put<D>(sh, 0, K, c0, T, scale_log2, tid);
     own_put<D>(sh, 1, V, c0, T, 1.f, tid);
     __syncthreads();
-    if (rr0 <= r_hi) {
-        float lse = load_vec(p.lse + vbase, rr0, T, n), delta = load_vec(p.delta + vbase, rr0, T, n);
-        const int nk = key_of_row(n);
-        float ra[D / 2], rb[D / 2];
-        load_rows<D>(ra, X, rr0, T, nk, g);
-        load_rows<D>(rb, G, rr0, T, nk, g);
-        const float b = p.bias ? p.bias[vbase + min(a, T - 1)] : 0.f;
-        for (; rr0 <= r_hi; rr0 += 32 * kWaves) {
-            const int next = min(rr0 + 32 * kWaves, r_hi & ~31);
-            sh.vec_put(0, lse * p.lse_to_log2, wave, n);
-            sh.vec_put(1, delta, wave, n);
-            f32x16 s = score_tile<D>(ra, sh, 0, n, g);  // rows = streamed r, columns = owner a
-            pin_order();
-            load_cols<D>(ra, X, rr0, T, n, g);
-            lse = load_vec(p.lse + vbase, next, T, n);
-            delta = load_vec(p.delta + vbase, next, T, n);
-            pin_order();
-            f32x16 dp = score_tile<D>(rb, sh, 1, n, g);
-            pin_order();
-            load_cols<D>(rb, G, rr0, T, n, g);
-            pin_order();
-            const bool edge = rr0 + 32 > T || (p.causal && (rr0 < c0 + 31 || rr0 + 31 - c0 > p.k_diff));
+    auto share = [&](auto any) {
+        constexpr bool ANY = decltype(any)::value;
+        clear<D>(accK);
+        clear<D>(accV);
+        db = 0.f;
+        int rr0 = r_lo + 32 * wave;
+        if (rr0 <= r_hi) {
+            float lse = load_vec(p.lse + vbase, rr0, T, n), delta = load_vec(p.delta + vbase, rr0, T, n);
+            const int nk = key_of_row(n);
+            float ra[D / 2], rb[D / 2];
+            load_rows<D>(ra, X, rr0, T, nk, g);
+            load_rows<D>(rb, G, rr0, T, nk, g);
+            const float b = p.bias ? p.bias[vbase + min(a, T - 1)] : 0.f;
+            for (; rr0 <= r_hi; rr0 += 32 * kWaves) {
+                const int next = min(rr0 + 32 * kWaves, r_hi & ~31);
+                sh.vec_put(0, lse * p.lse_to_log2, wave, n);
+                sh.vec_put(1, delta, wave, n);
+                f32x16 s = score_tile<D, ANY>(ra, sh, 0, n, g);  // rows = streamed r, columns = owner a
+                pin_order();
+                load_cols<D>(ra, X, rr0, T, n, g);
+                lse = load_vec(p.lse + vbase, next, T, n);
+                delta = load_vec(p.delta + vbase, next, T, n);
+                pin_order();
+                f32x16 dp = score_tile<D, ANY>(rb, sh, 1, n, g);
+                pin_order();
+                load_cols<D>(rb, G, rr0, T, n, g);
+                pin_order();
+                const bool edge = rr0 + 32 > T || (p.causal && (rr0 < c0 + 31 || rr0 + 31 - c0 > p.k_diff));
 #pragma unroll
-            for (int i4 = 0; i4 < 4; ++i4) {
-                const float4 l2 = sh.vec_get(0, wave, g, i4), dl = sh.vec_get(1, wave, g, i4);
-                const float l2s[4] = {l2.x, l2.y, l2.z, l2.w}, dls[4] = {dl.x, dl.y, dl.z, dl.w};
+                for (int i4 = 0; i4 < 4; ++i4) {
+                    const float4 l2 = sh.vec_get(0, wave, g, i4), dl = sh.vec_get(1, wave, g, i4);
+                    const float l2s[4] = {l2.x, l2.y, l2.z, l2.w}, dls[4] = {dl.x, dl.y, dl.z, dl.w};
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int i = 4 * i4 + e;
-                    const float pr = fast_exp2(s[i] + b - l2s[e]);
-                    s[i] = pr * (dp[i] - dls[e]);
-                    dp[i] = pr;
+                    for (int e = 0; e < 4; ++e) {
+                        const int i = 4 * i4 + e;
+                        const float pr = fast_exp2(s[i] + b - l2s[e]);
+                        s[i] = pr * (dp[i] - dls[e]);
+                        dp[i] = pr;
+                    }
                 }
-            }
-            if (edge) {
+                if (edge) {
 #pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    const int rr = rr0 + key_of(g, i);
-                    const bool ok = (rr < T) & pair_valid(p.causal, p.k_diff, rr, a);
-                    s[i] = ok ? s[i] : 0.f;
-                    dp[i] = ok ? dp[i] : 0.f;
+                    for (int i = 0; i < 16; ++i) {
+                        const int rr = rr0 + key_of(g, i);
+                        const bool ok = (rr < T) & pair_valid(p.causal, p.k_diff, rr, a);
+                        s[i] = ok ? s[i] : 0.f;
+                        dp[i] = ok ? dp[i] : 0.f;
+                    }
                 }
-            }
 #pragma unroll
-            for (int i = 0; i < 16; ++i) db += s[i];
-            output_tile<D>(accK, ra, s);
-            pin_order();
-            load_rows<D>(ra, X, next, T, nk, g);
-            pin_order();
-            output_tile<D>(accV, rb, dp);
-            pin_order();
-            load_rows<D>(rb, G, next, T, nk, g);
-            pin_order();
+                for (int i = 0; i < 16; ++i) db += s[i];
+                output_tile<D, ANY>(accK, ra, s);
+                pin_order();
+                load_rows<D>(ra, X, next, T, nk, g);
+                pin_order();
+                output_tile<D, ANY>(accV, rb, dp);
+                pin_order();
+                load_rows<D>(rb, G, next, T, nk, g);
+                pin_order();
+            }
         }
-    }
+    };
+    share(std::false_type{});
+    if (any_nan(accK) || any_nan(accV)) share(std::true_type{});
     db += __shfl_xor(db, 32, 64);
     if (g == 0) sh.row[wave][n] = db;
     sh.put(accK, p.alpha, wave, n, g);

@@ -8,8 +8,12 @@
 // over 64 is 1.44e-7 off on fp32 MFMAs, 1.10e-7 with the six products of each k-step in turn (products_of_step) and 0.50e-7
 // with all the small ones ahead of the large ones (small_products, large_product); over 1024, 5.7e-7 and 4.9e-7.
 //
-// Infinite operands, and those above 3.39e38, which h rounds to infinity: m is NaN, so every result that they enter is NaN (fp32
-// MFMAs leave some of them infinite).
+// Operands that are infinite or above kSplitMax (h would be rounded to infinity and m, x - h, be no number): split8_any.  It gives
+// an infinite one as (+-1, 0, +-infinity), of whose six products with a finite operand only l h is infinite, with the sign and the
+// zero case of the fp32 product, and with an infinite one l h and h l; and a finite one h rounded toward zero.  split8 is for values
+// that cannot be that large (probabilities), for a triple-dot backward's dS (an infinite one makes NaN of what it enters), and
+// where a result is looked at for NaN and formed again (dps_f32_mfma.hip).  Small operands: bf16 ends at 2^-133, so below 2^-109
+// (1.5e-33) l loses digits and below 2^-117 all of them.
 #pragma once
 #include "mfma.hpp"
 
@@ -33,6 +37,31 @@ __device__ __forceinline__ Split8 split8(const X& x) {
         s.h[e] = h[0]; s.h[e + 1] = h[1];
         s.m[e] = m[0]; s.m[e + 1] = m[1];
         s.l[e] = l[0]; s.l[e + 1] = l[1];
+    }
+    return s;
+}
+constexpr float kSplitMax = 0x1.fep127f;  // the largest bf16 number
+template <typename X>
+__device__ __forceinline__ float largest8(const X& x) {
+    float most = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) most = fmaxf(most, fabsf(x[e]));
+    return most;
+}
+template <typename X>
+__device__ __forceinline__ Split8 split8_any(const X& x) {
+    Split8 s = split8(x);
+    if (__builtin_expect(largest8(x) > kSplitMax, 0)) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            if (!(fabsf(x[e]) > kSplitMax)) continue;
+            const bool infinite = fabsf(x[e]) == INFINITY;
+            const float h = copysignf(infinite ? 1.f : kSplitMax, x[e]), r = infinite ? 0.f : x[e] - h;
+            const __bf16 m = (__bf16)r;
+            s.h[e] = (__bf16)h;
+            s.m[e] = m;
+            s.l[e] = (__bf16)(infinite ? x[e] : r - (float)m);
+        }
     }
     return s;
 }

@@ -572,3 +572,40 @@ def test_fp32_split_products_around_the_tiles(T, k_diff, D):
             err = ((a[b, h].double() - r).norm() / r.norm()).item()
             print(f"    {name}[{b}, {h}] T={T} D={D}: {err:.2e}", flush=True)
             assert err <= (1 if name == "o" else 4) * 2.0 ** -24 * (math.sqrt(D) + math.sqrt(T) + 2), name
+
+
+@pytest.mark.parametrize("D", [32, 64])
+@pytest.mark.parametrize("T,k_diff", [(100, 100), (257, 60)])
+def test_fp32_operands_at_the_end_of_the_range(T, k_diff, D):
+    """A K1 row whose scores are all -infinity has weight 0 and the others are as without it (0 times infinity is a NaN in its own
+    column of dK2: nothing is asked there).  Without a mask an infinite V1 element makes its column infinite, with the sign of V2,
+    and nothing else; one between the largest bf16 number and fp32's keeps its digits.  Bars as above."""
+    scale, h = 1 / math.sqrt(D), 1
+    bar = 2.0 ** -24 * (math.sqrt(D) + math.sqrt(T) + 2)
+    base = orc.make_inputs(1, 2, T, D, torch.float32, seed=T + D)
+    inputs = [t.clone() for t in base]
+    inputs[2][0, h, :, 5] = -inputs[2][0, h, :, 5].abs()
+    inputs[1][0, h, 40, 5] = math.inf
+    out, _, g = util.run_dps(inputs, scale, True, k_diff)
+    z, _, grads = _dps_in_64_bits(inputs, scale, k_diff, 0, h)
+    others = [d for d in range(D) if d != 5]
+    for name, a, r in zip(("o", *util.NAMES), (out, *g), (z, *grads)):
+        a, r = (a[0, h][:, others].double(), r[:, others]) if name == "dk2" else (a[0, h].double(), r)
+        err = ((a - r).norm() / r.norm()).item()
+        print(f"    {name} T={T} D={D}: {err:.2e}", flush=True)
+        assert err <= (1 if name == "o" else 4) * bar, (name, err)
+
+    inputs = [t.clone() for t in base]
+    inputs[4][0, h, :, 5] = -inputs[4][0, h, :, 5].abs()
+    good, _, _ = util.run_dps(inputs, scale, False, T, backward=False)
+    inputs[3][0, h, 40, 5] = math.inf
+    out, _, _ = util.run_dps(inputs, scale, False, T, backward=False)
+    assert (out[0, h, :, 5] == -math.inf).all()
+    out[0, h, :, 5] = good[0, h, :, 5]
+    assert torch.equal(out, good)
+    inputs[2][0, h], inputs[3][0, h, 40, 5] = 0.0, 3.395e38
+    inputs[4][0, h, :, 5] *= 1e-20
+    out, _, _ = util.run_dps(inputs, scale, False, T, backward=False)
+    z, _, _ = orc.dps_forward_backward(*(t[0, h].double() for t in inputs), scale, False, factorised=True)
+    err = ((out[0, h, :, 5].double() - z[:, 5]).norm() / z[:, 5].norm()).item()
+    assert err <= bar, err

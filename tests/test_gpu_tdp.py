@@ -1238,6 +1238,53 @@ def test_fp32_non_finite_operands_stay_with_their_queries(value, which):
 
 
 @pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("B,H,T", [(1, 2, 100), (4, 8, 130)])
+@pytest.mark.parametrize("which", [1, 2])
+def test_fp32_key_at_infinity_is_left_out(which, B, H, T, D):
+    """A key whose scores are all -infinity has weight 0 and the others are as without it, forward and backward, where the streamed
+    tensors are split as they are staged and where they come as images.  0 times infinity is a NaN in that key's own column of what its
+    row enters: there, and in the whole row of a fixed-point sum, nothing is asked.  Bars of the tests against 64 bits above."""
+    print(f"case key at infinity {which} {B} {H} {T} {D}", flush=True)
+    inputs, alpha, at = orc.make_inputs(B, H, T, D, torch.float32, seed=D), 1 / math.sqrt(D), (B - 1, H - 1)
+    inputs[0][at][:, 5], inputs[3 - which][at][:, 5] = -inputs[0][at][:, 5].abs(), inputs[3 - which][at][:, 5].abs()
+    inputs[which][at][40, 5] = math.inf
+    out, g = util.run_tdp(inputs, alpha, True)
+    z, _, grads = orc.tdp_forward_backward_chunked(*(t[at].double() for t in inputs), alpha)
+    err = ((out[at].double() - z).norm() / z.norm()).item()
+    assert err <= 2.0 ** -24 * (math.sqrt(D) + 2), err
+    others = [d for d in range(D) if d != 5]
+    for name, a, r in zip(util.NAMES, g, grads):
+        if name == "dk2" and which == 1:
+            continue
+        a, r = (a[at].double(), r) if name in ("dv1", "dv2", f"dk{which}") else (a[at][:, others].double(), r[:, others])
+        err = ((a - r).norm() / r.norm()).item()
+        print(f"    {name}: {err:.2e}", flush=True)
+        assert err <= 2.0 ** -24 * (D + 3) * math.sqrt(T), (name, err)
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("B,H,T", [(1, 2, 100)])
+def test_fp32_values_at_the_end_of_the_range(B, H, T, D):
+    """Without a mask (0 times infinity is a NaN, and a masked weight is 0) an infinite V1 element makes its column infinite, with
+    the sign of V2, and nothing else; one between the largest bf16 number and fp32's keeps its digits (equal weights: 2^-24 for
+    each of the T rows, and V2's product)."""
+    inputs, alpha, at = orc.make_inputs(B, H, T, D, torch.float32, seed=D), 1 / math.sqrt(D), (B - 1, H - 1)
+    inputs[4][at][:, 5] = -inputs[4][at][:, 5].abs()
+    good, _ = util.run_tdp(inputs, alpha, False, backward=False)
+    inputs[3][at][40, 5] = math.inf
+    out, _ = util.run_tdp(inputs, alpha, False, backward=False)
+    assert (out[at][:, 5] == -math.inf).all()
+    out[at][:, 5] = good[at][:, 5]
+    assert torch.equal(out, good)
+    inputs[0][at], inputs[3][at][40, 5] = 0.0, 3.395e38
+    inputs[4][at][:, 5] *= 1e-20
+    out, _ = util.run_tdp(inputs, alpha, False, backward=False)
+    z, _, _ = orc.tdp_forward_backward_chunked(*(t[at].double() for t in inputs), alpha, False, need_grads=False)
+    err = ((out[at][:, 5].double() - z[:, 5]).norm() / z[:, 5].norm()).item()
+    assert err <= 2.0 ** -24 * (math.sqrt(T) + 2), err
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
 def test_fp32_forward_of_large_values_under_rising_scores(D):
     """Keys whose scores are 2^35 above those of the tile before and values of 1e13 (outputs of 1e26): the unnormalised sums
     stay far enough from the end of fp32's range, whatever maximum they are kept relative to."""
