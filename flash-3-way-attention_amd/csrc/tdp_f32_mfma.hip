@@ -177,7 +177,7 @@ __global__ __launch_bounds__(256) void f32_merge_kernel(const float* __restrict_
     if (row >= rows) return;
     const int parts = f32_tile_parts(deal, mask, (int)(row % T) / 32, T, kSplitWaves);
     const float* src = part + row * deal.max_parts * (D + 4);
-    // four parts' loads in flight at a time (a part beyond the last one repeats it with weight zero)
+    // four parts' loads in flight at a time (for a part beyond the last one that one's, not used: zero times an infinite output is NaN)
     float m = kNegBig, l = 0.f;
     f32x4v acc = {0.f, 0.f, 0.f, 0.f};
     for (int s0 = 0; s0 < parts; s0 += 4) {
@@ -197,7 +197,7 @@ __global__ __launch_bounds__(256) void f32_merge_kernel(const float* __restrict_
         for (int k = 0; k < 4; ++k) {
             const float w = fast_exp2(ms[k] - top);
             l += w * ls[k];
-            acc += os[k] * w;
+            if (s0 + k < parts) acc += os[k] * w;
         }
         m = top;
     }
