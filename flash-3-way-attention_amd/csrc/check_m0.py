@@ -18,7 +18,7 @@ def check(text):
     lines = [ln.split(";")[0].strip() for ln in text.splitlines()]
     lines = [ln for ln in lines if ln and not ln.startswith(".")]
     uses = [i for i, ln in enumerate(lines) if re.search(r"\bm0\b", ln)]
-    if len(uses) < 50:
+    if len(uses) < 100:
         return "expected the direct loads of the kernels, found %d uses of m0" % len(uses)
     for i in uses:
         if not lines[i].startswith("s_mov_b32 m0,"):
