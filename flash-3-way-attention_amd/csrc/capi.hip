@@ -198,25 +198,34 @@ int clampw(int w, int T) { return w > T ? T : w; }
 // rounds of a query tile out over workgroups and are the faster ones at every size (B=1 H=1 T=16 D=64: forward 14 against
 // 27 us, backward 32 against 200 us), and on the vector ALUs (D = 8 and 16, and TRITT_TUNE_F32_VALU).
 bool use_f32_mfma() { return knobs().f32_valu == 0; }
-// Scratch of an fp32 matrix-core forward beyond its operands: the images of the streamed tensors, unless the problem is so
-// short that they would cost more than they save, and the parts of a split one.  `compact` (tritt_tdp_fwd_static_scratch, for
-// problems whose images do not fit the library's static buffer): no images, and no more parts than still fit.
-bool f32_fwd_has_images(GenericTdpArgs a, int dtype) {
-    a.fwd_parts = f32_fwd_parts(a);
-    return dtype != TRITT_F32 || !f32_fwd_takes_v1(a);
-}
-void plan_f32_fwd(Arena& ar, GenericTdpArgs& a, int dtype, bool compact) {
-    a.fwd_parts = 1;
-    a.part = nullptr;
-    a.images = nullptr;
-    if (!f32_mfma_tdp_supported(a.D) || !use_f32_mfma()) return;
-    if (!compact && f32_fwd_has_images(a, dtype)) a.images = ar.take<char>(f32_fwd_image_bytes(a));
-    const size_t per_part = (size_t)a.BH * a.T * f32_fwd_part_floats(a.D) * sizeof(float), used = ar.bytes();
+// How an fp32 matrix-core forward runs: the parts that its tiles are dealt out in, whether the streamed tensors come as images
+// (unless the problem is so short that they would cost more than they save), and whether it applies SiLU to V1 itself.  `used`:
+// the scratch of its operands, SiLU(V1) among them.  Where that fits the library's static buffer (tritt_tdp_fwd_static_scratch)
+// the parts have to fit as well, in every call, so that both entry points form the same sums; more parts gain nothing at such
+// sizes but at D = 128 (forward, bounded -> as many as the deal asks for: B=4 H=8 T=1024 D=64 2 -> 9 parts 14.4 -> 14.7 ms, D = 32 6 ->
+// 10 parts 8.1 -> 8.3, B=2 H=12 T=2048 D=64 windows 40 1 -> 3 parts 430 -> 484 us; B=1 H=16 T=2048 D=128 1 -> 5 parts 134 -> 131 ms).
+// `compact`: that buffer has no room for the images; the streamed tensors are split as they are staged, which gives the same bits.
+struct F32FwdPlan {
+    int parts = 1;
+    bool images = false, silu = false;
+};
+F32FwdPlan f32_fwd_plan(GenericTdpArgs a, int dtype, size_t used, bool compact) {
+    F32FwdPlan p;
+    if (!f32_mfma_tdp_supported(a.D) || !use_f32_mfma()) return p;
+    const size_t per_part = (size_t)a.BH * a.T * f32_fwd_part_floats(a.D) * sizeof(float);
     size_t parts = (size_t)f32_fwd_parts(a);
-    if (compact) parts = std::min(parts, used < TRITT_STATIC_SCRATCH_BYTES ? (TRITT_STATIC_SCRATCH_BYTES - used) / per_part : 0);
-    if (parts < 2) return;
-    a.fwd_parts = (int)parts;
-    a.part = ar.take<float>(parts * per_part / sizeof(float));
+    if (used <= TRITT_STATIC_SCRATCH_BYTES) parts = std::min(parts, (TRITT_STATIC_SCRATCH_BYTES - used) / per_part);
+    p.parts = (int)std::max<size_t>(parts, 1);
+    a.fwd_parts = p.parts;
+    const bool takes_v1 = dtype == TRITT_F32 && f32_fwd_takes_v1(a);
+    p.images = !compact && !takes_v1;
+    p.silu = takes_v1 || (dtype == TRITT_F32 && p.images);
+    return p;
+}
+void take_f32_fwd(Arena& ar, GenericTdpArgs& a, const F32FwdPlan& p) {
+    a.fwd_parts = p.parts;
+    a.images = p.images ? ar.take<char>(f32_fwd_image_bytes(a)) : nullptr;
+    a.part = p.parts > 1 ? ar.take<float>((size_t)p.parts * a.BH * a.T * f32_fwd_part_floats(a.D)) : nullptr;
 }
 
 // ---------------------------------------------------------------- triple-dot, fp32 VALU path
@@ -228,17 +237,18 @@ int tdp_fwd_generic(Arena& ar, bool run, const void* q, const void* k1, const vo
     a.BH = B * H; a.T = T; a.D = D; a.alpha = alpha;
     a.causal = causal; a.k1_window = w1; a.k2_window = w2; a.kk_left = kl; a.kk_right = kr;
     const bool mfma32 = f32_mfma_tdp_supported(D) && use_f32_mfma();
-    // with images SiLU(V1) is one of them; a short problem's kernel applies SiLU itself (unless `compact` took parts away)
+    Arena operands(nullptr);
+    for (int i = 0; i < (dtype == TRITT_F32 ? 1 : 6); ++i) operands.take<float>(n);  // U; the other copies and O
+    const F32FwdPlan plan = f32_fwd_plan(a, dtype, operands.bytes(), compact);
     float *copies[4], *u;
-    F32Inputs in = plan_inputs(ar, q, k1, k2, v2, n, dtype, copies, &u,
-                               !mfma32 || dtype != TRITT_F32 || compact || !f32_fwd_has_images(a, dtype));
+    F32Inputs in = plan_inputs(ar, q, k1, k2, v2, n, dtype, copies, &u, !plan.silu);
     float* o32 = dtype == TRITT_F32 ? (float*)o : ar.take<float>(n);
-    plan_f32_fwd(ar, a, dtype, compact);
+    take_f32_fwd(ar, a, plan);
     if (!run) return TRITT_OK;
     if (ar.overflows()) return TRITT_ERR_WORKSPACE;
     a.q = in.q; a.k1 = in.k1; a.k2 = in.k2; a.u = in.u; a.v2 = in.v2;
     a.o = o32; a.lse = lse;
-    if (mfma32 && dtype == TRITT_F32 && (a.images || f32_fwd_takes_v1(a))) {
+    if (plan.silu) {
         a.u = (const float*)v1;
         a.u_is_v1 = 1;
     } else {
@@ -268,7 +278,7 @@ int tdp_bwd_generic(Arena& ar, bool run, const void* q, const void* k1, const vo
     GenericTdpArgs a{};
     a.BH = B * H; a.T = T; a.D = D; a.alpha = alpha;
     a.causal = causal; a.k1_window = w1; a.k2_window = w2; a.kk_left = kl; a.kk_right = kr;
-    if (dtype != TRITT_F32) plan_f32_fwd(ar, a, dtype, false);  // (o32 is null while measuring)
+    if (dtype != TRITT_F32) take_f32_fwd(ar, a, f32_fwd_plan(a, dtype, ar.bytes(), false));  // (o32 is null while measuring)
     void* scratch32 = mfma32 ? ar.take<char>(f32_mfma_tdp_bwd_scratch_bytes(a)) : nullptr;
     // VALU kernels: fp32 results, the caller's tensors when they are fp32, scratch otherwise; `spare` stands in for the
     // unwanted (null) half of a gradient pair whose other half is wanted (one kernel writes both halves)
@@ -631,7 +641,7 @@ static MfmaFwdArgs mfma_fwd_shape(int B, int H, int T, int D, int dtype, int cau
     return a;
 }
 
-// compact: see plan_f32_fwd
+// compact: see f32_fwd_plan
 static size_t tdp_fwd_bytes(int B, int H, int T, int D, int dtype, int causal, int k1_window, int k2_window, int kk_left,
                             int kk_right, unsigned flags, bool compact) {
     if (check_common(B, H, T, D, dtype) != TRITT_OK) return 0;

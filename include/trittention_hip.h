@@ -145,8 +145,7 @@ int tritt_tdp_fwd(const void* q, const void* k1, const void* k2, const void* v1,
  * where an fp32 problem's tritt_tdp_fwd_workspace_bytes() is larger than the array, the call does
  * without the copies of the streamed tensors that it is mostly made of).  All calls on
  * one GPU share the one array: calls that overlap in time on the same GPU (different
- * streams or threads) race; serialise them.  Results are identical to tritt_tdp_fwd's (without
- * those copies: the same sums, perhaps in other shares, a few fp32 roundings apart).
+ * streams or threads) race; serialise them.  Results are identical to tritt_tdp_fwd's.
  * tritt_static_scratch_bytes() returns the limit the library was built with. */
 #define TRITT_STATIC_SCRATCH_BYTES ((size_t)32 << 20)
 size_t tritt_static_scratch_bytes(void);
