@@ -386,8 +386,9 @@ hipError_t launch_f32_bwd(const F32BwdCall& c, hipStream_t st) {
     return hipGetLastError();
 }
 
+int f32_fwd_slots(int D) { return D > 64 ? 256 : 512; }
 F32Deal f32_fwd_deal(const GenericTdpArgs& a, int most) {
-    return f32_deal(f32_mask(a), a.BH, a.T, kSplitWaves, a.D > 64 ? 256 : 512, knobs().fwd_splits > 0 ? std::min(knobs().fwd_splits, most) : most);
+    return f32_deal(f32_mask(a), a.BH, a.T, kSplitWaves, f32_fwd_slots(a.D), knobs().fwd_splits > 0 ? std::min(knobs().fwd_splits, most) : most);
 }
 
 template <int D>
@@ -421,11 +422,25 @@ hipError_t launch_f32_fwd(const GenericTdpArgs& a, hipStream_t st) {
 
 }  // namespace
 
-// SiLU as the value stages go to LDS costs about 1600 cycles of the waves that move them, every time a tile streams a row;
-// where a workgroup has no more than a few stages to walk that is less than a launch of its own (2-5 us)
+// A short problem's streamed tensors are split, and V1 goes through SiLU, as their stages are put in LDS: 0.4 / 0.7 / 1.3 us a step at
+// D = 32 / 64 / 128, every time a tile streams a row, where the launch that makes images takes 2-2.5 us.  `walk`: steps of the longest
+// workgroup, or the average of a place on the chip where that is more.  Forward, split as staged against images, D = 32 / 64 / 128:
+// B=1 H=2 T=64 (walk 2) 12.7 15.7 24.0 against 14.8 16.8 24.2 us, B=4 H=8 T=64 (2.5, D = 128: 5) 18.5 29.5 66.5 against 19.3 29.1 62.2,
+// B=1 H=2 T=1000 windows 16 (3, 6) 22.0 33.9 79.1 against 23.5 35.0 76.8, B=1 H=2 T=128 (8) 22.9 30.8 52.8 against 22.1 27.3 43.7,
+// T=256 (32) 59.8 87.5 161 against 49.0 65.3 114; T=72 (6) 19.7 26.2 43.3 against 19.8 24.1 37.3.
 bool f32_fwd_takes_v1(const GenericTdpArgs& a) {
     const F32Deal d = f32_fwd_deal(a, std::max(1, a.fwd_parts));
-    return d.inv_target >= 0.25f && (long long)a.BH * d.items <= 768;
+    const TdpMask mask = f32_mask(a);
+    double total = 0, walk = 0;
+    for (int qt = 0; qt * 32 < a.T; ++qt) {
+        int rounds;
+        const int steps = f32_tile_steps(mask, qt * 32, std::min(a.T - 1, qt * 32 + 31), a.T, kSplitWaves, &rounds);
+        total += steps;
+        const int parts = f32_tile_parts(d, mask, qt, a.T, kSplitWaves);
+        walk = std::max(walk, (double)((rounds + parts - 1) / parts) * steps / rounds);
+    }
+    walk = std::max(walk, total * a.BH / f32_fwd_slots(a.D));
+    return walk * (a.D + 32) <= 330;
 }
 int f32_fwd_parts(const GenericTdpArgs& a) { return f32_fwd_deal(a, 16).max_parts; }
 size_t f32_fwd_image_bytes(const GenericTdpArgs& a) {

@@ -1238,7 +1238,7 @@ def test_fp32_non_finite_operands_stay_with_their_queries(value, which):
 
 
 @pytest.mark.parametrize("D", [32, 64, 128])
-@pytest.mark.parametrize("B,H,T", [(1, 2, 100), (4, 8, 130)])
+@pytest.mark.parametrize("B,H,T", [(1, 2, 64), (1, 2, 100), (4, 8, 130)])
 @pytest.mark.parametrize("which", [1, 2])
 def test_fp32_key_at_infinity_is_left_out(which, B, H, T, D):
     """A key whose scores are all -infinity has weight 0 and the others are as without it, forward and backward, where the streamed
@@ -1263,7 +1263,7 @@ def test_fp32_key_at_infinity_is_left_out(which, B, H, T, D):
 
 
 @pytest.mark.parametrize("D", [32, 64, 128])
-@pytest.mark.parametrize("B,H,T", [(1, 2, 100), (4, 8, 130)])
+@pytest.mark.parametrize("B,H,T", [(1, 2, 64), (1, 2, 100), (4, 8, 130)])
 def test_fp32_values_at_the_end_of_the_range(B, H, T, D):
     """Without a mask (0 times infinity is a NaN, and a masked weight is 0) an infinite V1 element makes its column infinite, with
     the sign of V2, and nothing else; one between the largest bf16 number and fp32's keeps its digits (equal weights: 2^-24 for
