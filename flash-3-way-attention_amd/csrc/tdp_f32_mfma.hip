@@ -37,7 +37,7 @@ namespace {
 // that) and the poison words cleared.  grid (64-row blocks, BH, 1 + the maxima's tensors + the images): one of them after the
 // other in the blocks of z = 0 is 6 us longer, a launch for each 2-5 us.
 struct F32PrepParams {
-    const float *q, *k1, *k2, *v2, *u_in, *v1, *o, *d_o;
+    const float *q, *k1, *v2, *u_in, *v1, *o, *d_o;
     float *u, *delta;
     unsigned* acc;
     int planes;
@@ -55,7 +55,7 @@ __global__ __launch_bounds__(256) void f32_prep_kernel(F32PrepParams p) {
     int z = blockIdx.z;
     if (z && p.maxima && z <= kMaxima) {  // part s of a slice: its 64-row blocks s, s + kScaleParts, ...
         const int t = z - 1;
-        const float* src = (t == kMaxDO ? p.d_o : t == kMaxQ ? p.q : t == kMaxK1 ? p.k1 : t == kMaxK2 ? p.k2 : t == kMaxV2 ? p.v2 : p.v1 ? p.v1 : p.u_in) + base;
+        const float* src = (t == kMaxDO ? p.d_o : t == kMaxQ ? p.q : t == kMaxK1 ? p.k1 : t == kMaxV2 ? p.v2 : p.v1 ? p.v1 : p.u_in) + base;
         for (int part = blockIdx.x; part < kScaleParts; part += gridDim.x) {
             unsigned m = 0;
             for (int r0 = part * 64; r0 < T; r0 += kScaleParts * 64)
@@ -335,7 +335,7 @@ hipError_t launch_f32_bwd(const F32BwdCall& c, hipStream_t st) {
     // a dQ of one part per tile needs no place of its own where the kernel can write the caller's type
     const bool direct_q = c.elem == 0 && s.deal_q.max_parts == 1;
     F32PrepParams prep{};
-    prep.q = a.q; prep.k1 = a.k1; prep.k2 = a.k2; prep.v2 = a.v2; prep.u_in = a.u; prep.v1 = c.v1_f32; prep.o = c.o; prep.d_o = a.d_o;
+    prep.q = a.q; prep.k1 = a.k1; prep.v2 = a.v2; prep.u_in = a.u; prep.v1 = c.v1_f32; prep.o = c.o; prep.d_o = a.d_o;
     prep.u = c.v1_f32 ? c.u_out : nullptr; prep.delta = c.delta;
     prep.acc = reinterpret_cast<unsigned*>(s.acc); prep.planes = s.slabs ? 2 * s.slabs : 4; prep.n = n;
     prep.maxima = s.slabs ? nullptr : s.maxima; prep.poison = s.poison; prep.T = a.T;

@@ -521,16 +521,16 @@ constexpr size_t f32_split_fwd_smem() {
 // between the MFMAs -> 11.0, the sums over lanes by swaps and DPP -> 10.1.  D = 32 forms its scores in turn: two waves a SIMD
 // fill each other's gaps (scores ahead need 212 B of scratch per lane there; 19.7 -> 18.4 ms).
 // Scales of the fp32 tensors' row-gradient accumulators.  A gradient shrinks with every operand in it while dO stays, so the
-// scale follows all of them: with the slice's largest finite |dO|, |Q|, |K1|, |K2|, |V1|, |V2| (`maxima`, kScaleParts words per
-// tensor and slice, [tensor][BH][parts]; |SiLU(x)| <= |x|), S the streamed operands and sum P = 1,
-//   |dV rows| <= T max|dO| max|VS|       |dK rows| <= alpha T max|Q| max|KS| 2 D max|dO| max|V1| max|V2|
+// scale follows all of them: with the slice's largest finite |dO|, |Q|, |K1|, |V1|, |V2| (`maxima`, kScaleParts words per
+// tensor and slice, [tensor][BH][parts]; |SiLU(x)| <= |x|) and sum P = 1,
+//   |dV2| <= T max|dO| max|V1|       |dK2| <= alpha T max|Q| max|K1| 2 D max|dO| max|V1| max|V2|
 // and a sum of that size is placed at 2^61.  A tensor with a few large elements makes this bound far too wide: the step is
 // never coarser than 2^-36 of max |dO| (sums past 2^27 times it then set the row's poison word, common.hpp).
 // B=4 H=8 T=128 D=64 with operands of 1 / 0.05 / 0.02 / 0.01, dK2 against 64 bits: 4.5e-7 / 1.4e-4 / 5.3e-3 / 8.1e-2 with the
 // scale of dO alone, 4.5e-7 / 2.8e-7 / 3.1e-7 / 3.2e-7 with this one.  Kernel time of a training step, dO's scale -> this:
 // B=2 H=4 T=500 D=64 4335 -> 4330 us, B=1 H=2 T=128 D=64 160.4 -> 159.8, B=4 H=8 T=128 D=64 531 -> 539.
 constexpr int kF32FixedBias = 36;
-enum { kMaxDO, kMaxQ, kMaxK1, kMaxK2, kMaxV1, kMaxV2, kMaxima };
+enum { kMaxDO, kMaxQ, kMaxK1, kMaxV1, kMaxV2, kMaxima };
 struct F32RowScale {
     const unsigned* maxima;      // null: one scale by max |dO| (or float accumulators)
     unsigned* fields;            // [BH][2] for the launch that converts: dK2, dV2
