@@ -1227,7 +1227,9 @@ def test_fp32_forward_against_64_bits(B, H, T, D, mask):
 @pytest.mark.parametrize("value", [float("nan"), float("inf")])
 @pytest.mark.parametrize("which", [0, 1, 2, 3, 4])
 def test_fp32_non_finite_operands_stay_with_their_queries(value, which):
-    """A non-finite element leaves the rows that cannot see it untouched and no row that sees it in all its weights finite."""
+    """A non-finite element leaves no row that sees it in all its weights finite, other heads and the query tiles ahead of it as
+    they are, and in its own tile of 32 the rows that cannot see it as exact as before (a NaN score moves the tile's references:
+    2^-24 (sqrt(D) + 2) in the norm), except that a value meets them with weight 0 and leaves a NaN in its own column."""
     inputs = orc.make_inputs(1, 2, 100, 64, torch.float32, seed=3)
     good, _ = util.run_tdp(inputs, 0.125, True)
     inputs[which][0, 1, 40, 5] = value
@@ -1235,6 +1237,13 @@ def test_fp32_non_finite_operands_stay_with_their_queries(value, which):
     assert torch.equal(out[0, 0], good[0, 0]) and torch.equal(out[0, 1, :32], good[0, 1, :32])
     hit = out[0, 1, 40:] if which else out[0, 1, 40:41]
     assert not torch.isfinite(hit[..., 5] if which > 2 else hit).any()
+    if which > 2:
+        others = [d for d in range(64) if d != 5]
+        assert torch.equal(out[0, 1][:, others], good[0, 1][:, others])
+    else:
+        for rows in [slice(32, 40)] + ([slice(41, 100)] if which == 0 else []):
+            err = ((out[0, 1, rows] - good[0, 1, rows]).norm() / good[0, 1, rows].norm()).item()
+            assert err <= 2.0 ** -24 * 10, (rows, err)
 
 
 @pytest.mark.parametrize("D", [32, 64, 128])
