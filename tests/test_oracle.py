@@ -13,6 +13,7 @@ import torch.nn.functional as F
 
 from oracle import brute
 from oracle import trittention_oracle as orc
+from tests import util
 
 torch.manual_seed(0)
 DT = torch.float64
@@ -238,3 +239,20 @@ def test_rounded_silu_is_the_dense_formula_on_rounded_gated_values():
     z3.backward(do)
     sg = torch.sigmoid(v1)
     torch.testing.assert_close(g[3], ul.grad * sg * (1 + v1 * (1 - sg)), rtol=1e-6, atol=1e-7)
+
+
+@pytest.mark.parametrize("D,w", util.BAND_CASES)
+def test_bar_of_the_band_limits_sees_a_mask_one_key_off(D, w):
+    """Every one of the eight masks with one limit a key further out or in moves some query's row by more than twice the bar that
+    the band-resident forward is held to (where it is another mask at all)."""
+    T, windows = util.band_windows(w)
+    inputs = orc.make_inputs(1, 1, T, D, torch.bfloat16, seed=w)
+    z, masked = util.band_oracle(inputs, 0, windows), orc.tdp_mask(T, *windows)
+    for i in range(4):
+        for step in (-1, 1):
+            other = list(windows)
+            other[i] += step
+            if other[i] < 0 or torch.equal(masked, orc.tdp_mask(T, *other)):
+                continue
+            off = (util.band_oracle(inputs, 0, other) - z).norm(dim=1) / z.norm(dim=1)
+            assert off.max().item() > 2 * util.BAND_BAR, (i, step)

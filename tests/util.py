@@ -147,3 +147,21 @@ def check_offsets_beyond_32_bits(variant, B, H, T, D, windows=(None,) * 4, rtol=
     finally:
         del leaves, do, out
         torch.cuda.empty_cache()
+
+
+# the band-resident forward's limits: head dimensions and windows, and the bar of a query's row.  Four roundings of at most 2^-9
+# (the scores' operand, P, U, the output) are 2^-9 sqrt(4 / 3) of a row in the norm; the bar is seven times that, for rows of a
+# few pairs that nearly cancel
+BAND_CASES = [(64, 1), (64, 31), (64, 33), (64, 128), (64, 129), (64, 192), (64, 193), (32, 40), (128, 64)]
+BAND_BAR = 2.0 ** -6
+
+
+def band_windows(w):
+    """(sequence length, windows): both windows and both sides of the k-k band differ."""
+    return 2 * w + 77, (w, max(1, w - 3), w // 3, w // 2 + 1)
+
+
+def band_oracle(inputs, h, windows):
+    D = inputs[0].shape[-1]
+    kw = dict(zip(("k1_window", "k2_window", "kk_left", "kk_right"), windows))
+    return orc.tdp_forward_backward_chunked(*(t[0, h].float() for t in inputs), D ** -0.5, True, need_grads=False, **kw)[0]
