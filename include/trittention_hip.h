@@ -105,9 +105,9 @@ int tritt_set_tuning(int knob, int value, int* previous);
  * tritt_tdp_bwd replaces FlashTrittention.backward and its five launches
  *   (triple_dot_product/flash_trittention.py:141-393, kernels/bwd_{dq,dk1,dk2,dv1,dv2}.py),
  *   including Delta = rowsum(dO*O) and the SiLU' factor on dV1.  Any of dq, dk1, dk2, dv1, dv2 may
- *   be NULL: that gradient is not wanted, and a kernel launch that only serves unwanted gradients
- *   is skipped (the launches produce {dq, dk2, dv2} and {dk1, dv1}; the fp32 kernels {dq},
- *   {dk2, dv2} and {dk1, dv1}).  On the 16-bit MFMA path
+ *   be NULL: that gradient is not wanted, and workgroups that only serve unwanted gradients
+ *   are left out (they produce {dq, dk2, dv2} or {dk1, dv1}; those of the fp32 kernels {dq} or
+ *   the other four).  On the 16-bit MFMA path
  *   (16-bit tensors, D = 32, 64 or 128, any mask) the workgroups of different query tiles add their
  *   shares of dK1/dV1/dK2/dV2 (and of dQ, when a small grid splits a tile's rows) to common
  *   accumulators.  The shares are added as 64-bit fixed point with integer atomics, whose result
@@ -116,9 +116,9 @@ int tritt_set_tuning(int knob, int value, int* previous);
  *   (measured cost against fp32 atomics: none).  The fixed-point scale is a power of two chosen
  *   per (batch, head) slice from the largest finite |dO| of the slice: steps of 2^-30 of that
  *   magnitude, sums up to 2^33 times it (fp32 matrix-core kernels: from the largest magnitudes of
- *   all six tensors, never coarser than 2^-36 of max |dO|; dQ, and below eight query tiles all
+ *   dO, Q, K1, V1 and V2, never coarser than 2^-36 of max |dO|; dQ, dK1 and dV1, and below eight query tiles all
  *   five gradients, are summed in fp32 there), so the backward is exactly homogeneous in dO for powers of two (loss scaling, mean-reduced losses)
- *   and has no absolute floor, like the reference's fp32 accumulators
+ *   and has no absolute floor (fp32 tensors: down to |dO| of 1e-30), like the reference's fp32 accumulators
  *   (triple_dot_product/kernels/bwd_dk1.py:239-258).  A share that is NaN, Inf or beyond the
  *   accumulator's range makes that row of that gradient NaN in the output.
  *   TRITT_FLAG_FLOAT_ATOMICS selects fp32 atomics instead (reproducible to rounding only;

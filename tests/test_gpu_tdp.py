@@ -1162,6 +1162,23 @@ def test_fp32_gradients_against_64_bits(B, H, T, D, mask):
         assert torch.equal(leaves[which].grad.cpu(), g[which]), util.NAMES[which]
 
 
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("B,H,T,power", [(2, 4, 200, -100), (1, 2, 64, -100), (1, 2, 64, -113)])
+def test_fp32_gradients_of_the_smallest_dO(B, H, T, power, D):
+    """dO of 2^-100 (8e-31) keeps every gradient's digits.  Split products end at 2^-133: at 2^-113 (1e-34) each dS, about
+    sqrt(D) 2^-113 over the T^2 pairs of a row, is cut off by up to 2^-134, and so many of them are summed: 2^-21 T^2 / sqrt(D)
+    on top of the bar above."""
+    print(f"case dO 2^{power}: {B} {H} {T} {D}", flush=True)
+    inputs, alpha = orc.make_inputs(B, H, T, D, torch.float32, seed=D), 1 / math.sqrt(D)
+    _, g = util.run_tdp(list(inputs[:5]) + [inputs[5] * 2.0 ** power], alpha, True)
+    bar = 2.0 ** -24 * (D + 3) * math.sqrt(T) + (2.0 ** -21 * T * T / math.sqrt(D) if power < -109 else 0)
+    _, _, grads = orc.tdp_forward_backward_chunked(*(t[-1, -1].double() for t in inputs), alpha)
+    for name, a, r in zip(util.NAMES, g, grads):
+        err = ((a[-1, -1].double() * 2.0 ** -power - r).norm() / r.norm()).item()
+        print(f"    {name}: {err:.2e}", flush=True)
+        assert err <= bar, (name, err)
+
+
 def test_fp32_dq_beyond_the_range_of_dO():
     """dQ far above |dO| (large keys and values) is finite: nothing bounds it by a multiple of max |dO|."""
     inputs = orc.make_inputs(4, 8, 128, 64, torch.float32, seed=9)
