@@ -31,14 +31,13 @@ NOMINAL_CLOCK_MHZ = 2400.0  # the clock behind the published peak
 # default workload only, scaled by a plain 256 MiB copy (summary and commands:
 # profiles/tdp_fwd_bwd_B4_H8_T1024_D64_bf16_counters.txt).  Reported only when the workload is the default one.
 TRAFFIC_SOURCE = "profiles/tdp_fwd_bwd_B4_H8_T1024_D64_bf16_counters.txt (rocprofv3 --pmc, default workload only)"
-# 27.4 MiB fetched + 15.0 MiB written: the algorithmic 20 + 4 MiB, and 28 bytes per lane that the kernel's prologue
+# 29.0 MiB fetched + 15.5 MiB written: the algorithmic 20 + 4 MiB, and 28 bytes per lane that the kernel's prologue
 # spills (a million lanes: ~11 MiB written once; spill-free builds of the kernel measured 2 % slower)
-TRAFFIC_FWD = 44.4e6
-# both roles of the rows kernel: 587 + 527 MiB written (64-bit atomics; 16-20 bytes per lane of the role with dQ are
-# spilled), 36 + 39 MiB fetched (some runs: up to 440 MiB, when its accumulators fall out of their XCD's L2; the bytes
-# are L2 <-> fabric traffic, which the 256 MB Infinity Cache absorbs).  Measured when each role was a launch of its own;
-# their sum.
-TRAFFIC_BWD_ROWS = 1248e6
+TRAFFIC_FWD = 46.7e6
+# both roles of the rows kernel: 1107 MiB written (64-bit atomics; 56 bytes of scratch memory per lane), 68 MiB fetched (as
+# two launches some runs fetched up to 440 MiB, when the accumulators fell out of their XCD's L2; the bytes are L2 <->
+# fabric traffic, which the 256 MB Infinity Cache absorbs)
+TRAFFIC_BWD_ROWS = 1232e6
 
 
 def triples(B, H, T, causal=True):

@@ -88,7 +88,7 @@ __device__ __forceinline__ float acc_scale(const BwdParams<E>& p, int bh) {
 namespace tritt {
 
 // ------------------------------------------------------------------------------------------
-// Written for launch 1 (rows = K2/V2 indexed by k, streamed = K1/U indexed by j); launch 2 is the
+// Written for the first role (rows = K2/V2 indexed by k, streamed = K1/U indexed by j); the second is the
 // same code with the two roles exchanged.
 //
 // Owner = 32 consecutive queries (the columns of every MFMA tile of the workgroup).  The eight
@@ -742,9 +742,11 @@ static BwdLayout bwd_layout(int BH, int T, int D, bool fixed_point) {
 // Workgroups per query tile under a window at D = 64, by the time that the launch takes with s of them: one workgroup
 // fills a CU, and all tiles but those at the start of the sequence cost the same, so the launch takes the larger of
 // whole rounds of the full tiles' parts over the CUs and of the even share plus half a part of tail.  Work in 32-key steps
-// of eight rows; a part's own prologue, dQ's shares and tail are worth about nine of them.  Against one part per tile below
-// 1024 tiles and two from there on, training steps: B=2 H=4 T=2048 window 512 5.67 -> 5.3 ms (3 parts), B=2 H=8 T=2048
-// window 100 1.41 -> 1.31 ms (1), B=1 H=2 T=1999 window 77 232 -> 212 us (2); the rest of a dozen shapes within 1 %.
+// of eight rows; a part's own prologue, dQ's shares and tail are worth about nine of them.  The model is that of one role's
+// workgroups in a launch of their own.  In the grid that holds both roles its choice (backward, chosen / best): B=2 H=4 T=2048
+// window 512 6 parts 4.09 ms / 3 parts 4.00, B=1 H=8 T=700 window 100 3 parts 214 us, B=2 H=8 T=2048 window 100 1 part 1.02 ms (both
+// the best), B=1 H=4 T=1500 window 300 6 parts 724 / 3 parts 707, B=4 H=8 T=1024 window 200 2 parts 2.00 / 1 part 1.92, B=1 H=2
+// T=1999 window 77 2 parts 141 / 1 part 130.
 static int windowed_splits(const MfmaBwdArgs& a) {
     constexpr float kPart = 9.f;
     constexpr int kCus = 256;
@@ -767,10 +769,11 @@ static int windowed_splits(const MfmaBwdArgs& a) {
 // Workgroups per query tile under a full causal mask at D = 64, for grids of less than 1024 tiles.  The work of a tile grows
 // with the square of its position and the heaviest parts start first, so a launch takes the longer of the even share of all
 // parts over the CUs and of its longest part (which starts late by what the parts before it differ: 1.15).  Work in 32-key
-// steps of eight rows; a part's own prologue, dQ's shares and tail are worth about seven of them.  Against parts that bring
-// the grid to 1024 workgroups whatever they cost, training steps: B=2 H=4 T=256 172 -> 158 us (16 -> 8 parts), B=4 H=8 T=128
-// 168 -> 154 us (8 -> 4), B=2 H=8 T=300 360 -> 352 us (7 -> 4), B=1 H=4 T=512 348 -> 341 us (8 -> 12); B=1 H=8 T=1000
-// keeps its four.  D = 32 and 128 measure within 1 % of their best at 1024 workgroups.
+// steps of eight rows; a part's own prologue, dQ's shares and tail are worth about seven of them.  The model is that of one role's
+// workgroups in a launch of their own.  In the grid that holds both roles its choice (backward, chosen / best): B=2 H=4 T=256 8 parts 109 us
+// / 6 parts 104, B=4 H=8 T=128 4 parts 107 / 2 parts 98, B=4 H=8 T=256 3 parts 316 / 2 parts 306, B=2 H=8 T=300 4 parts 266 / 3 parts
+// 262, B=1 H=4 T=512 12 parts 253 / 8 parts 250, B=1 H=2 T=128 16 parts 41 / 12 parts 39; B=1 H=8 T=1000 and B=2 H=4 T=600 within 1 % of
+// the best.  D = 32 and 128 measure within 1 % of their best at 1024 workgroups.
 static int causal_splits(const MfmaBwdArgs& a) {
     constexpr float kPart = 7.f;
     constexpr int kCus = 256;

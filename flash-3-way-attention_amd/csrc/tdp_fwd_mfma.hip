@@ -998,6 +998,8 @@ static hipError_t launch_band(const MfmaFwdArgs& a, hipStream_t st) {
     const int nr = band_rows(p.wa, p.wb);
     constexpr int kWide = D == 128 ? 8 : 16, kNarrow = D == 64 ? 16 : 8;
     const bool wide = band_waves16<D>(a, nr);
+    // K2 as floats: D = 64 B=2 H=8 T=2048 windows 128 / 32 159.8 -> 156.3 us, B=4 H=8 T=1024 64 / 16 97.8 -> 95.6.  At D = 32 the workgroups
+    // of sixteen waves gain 1 % (windows 300 / 100 447 -> 442) and at D = 128 none (175.6 both): not worth their instantiations
     constexpr bool kMayFloat = D == 64;
     const bool k2_float = kMayFloat && wide && band_smem_bytes<D, kWide>(nr, true) <= kBandSmemLimit;
     const size_t smem = wide ? band_smem_bytes<D, kWide>(nr, k2_float) : band_smem_bytes<D, kNarrow>(nr);
