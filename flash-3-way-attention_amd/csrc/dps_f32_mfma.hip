@@ -89,14 +89,10 @@ __device__ __forceinline__ float load_vec(const float* src, int row0, int T, int
     const __amdgpu_buffer_rsrc_t rows = tile_rows<1>(src, row0, T);
     return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rows, 4 * n, 0, 0));
 }
-// ANY: the values may be infinite (split8_any).  Testing every value of a step for that would cost a tenth of its vector
-// instructions, so a wave forms its share with split8, whose third plane is NaN for such a value, and forms it again if a NaN
-// came out of it (B=2 H=8 T=1000 D=64 k_diff 128, backward 119.5 -> 120.5 us, forward 40.6 both).
-template <bool ANY, typename X>
-__device__ __forceinline__ Split8 split_value(const X& x) {
-    if constexpr (ANY) return split8_any(x);
-    else return split8(x);
-}
+// ANY: the values may be infinite.  Testing every value of a step for that would cost a tenth of its vector instructions, so a wave
+// forms its share with split8, whose third plane is NaN for such a value, and forms it again if a NaN came out of it
+// (B=2 H=8 T=300 D=64 forward 23.6 -> 24.0, backward 48.3 -> 48.8 us, B=4 H=8 T=512 k_diff 100 34.2 -> 33.1 and 89.5 -> 89.7; the branch
+// taken for unlikely: D = 32 backward of T=300 33.9 -> 33.2).
 template <bool ANY>
 __device__ __forceinline__ Split8 split_at(const float* x) {
     float v[8];
@@ -317,7 +313,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attn_fwd_f32m_kernel(FwdP p) {
         }
     };
     share(std::false_type{});
-    if (any_nan(acc)) share(std::true_type{});
+    if (__builtin_expect(any_nan(acc), 0)) share(std::true_type{});
     if (g == 0) sh.row[wave][n] = m;
     __syncthreads();
     float M = sh.row[0][n];
@@ -371,17 +367,23 @@ struct BwdP {
 // In the backward the owner's two operands are read from LDS in every step, by all waves: in registers beside the accumulators,
 // two operand sets and the score tiles they do not fit.
 template <int D>
-__device__ __forceinline__ void own_put(Shares<D>& sh, int which, const float* src, int row0, int T, float scale, int tid) {
+__device__ __forceinline__ void own_put(Shares<D>& sh, const float* src0, const float* src1, int row0, int T, float scale0, int tid) {
     for (int piece = tid; piece < 32 * D / 8; piece += 64 * kWaves) {
         const int row = piece / (D / 8), c = piece % (D / 8) * 8;
-        const float* at = src + (size_t)min(row0 + row, T - 1) * D + c;
-        float v[8];
+        const size_t at = (size_t)min(row0 + row, T - 1) * D + c;
+        float v[2][8];  // (both loaded ahead of the first split, which branches)
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = at[e] * scale;
-        const Split8 x = split8_any(v);
-        *reinterpret_cast<bf16x8*>(sh.own[which][0] + row * Shares<D>::kOwnLD + c) = x.h;
-        *reinterpret_cast<bf16x8*>(sh.own[which][1] + row * Shares<D>::kOwnLD + c) = x.m;
-        *reinterpret_cast<bf16x8*>(sh.own[which][2] + row * Shares<D>::kOwnLD + c) = x.l;
+        for (int e = 0; e < 8; ++e) {
+            v[0][e] = src0[at + e] * scale0;
+            v[1][e] = src1[at + e];
+        }
+#pragma unroll
+        for (int which = 0; which < 2; ++which) {
+            const Split8 x = split8_any(v[which]);
+            *reinterpret_cast<bf16x8*>(sh.own[which][0] + row * Shares<D>::kOwnLD + c) = x.h;
+            *reinterpret_cast<bf16x8*>(sh.own[which][1] + row * Shares<D>::kOwnLD + c) = x.m;
+            *reinterpret_cast<bf16x8*>(sh.own[which][2] + row * Shares<D>::kOwnLD + c) = x.l;
+        }
     }
 }
 template <int D, bool ANY>
@@ -400,8 +402,7 @@ __device__ __forceinline__ void bwd_rows(const BwdP& p, Shares<D>& sh, int bh, i
     const int a_lo = p.causal ? max(0, r0 - p.k_diff) & ~31 : 0, a_hi = p.causal ? min(T - 1, r0 + 31) : T - 1;
     const float scale_log2 = p.alpha * kLog2e;
     f32x16 acc[DT];
-    own_put<D>(sh, 0, X, r0, T, scale_log2, tid);
-    own_put<D>(sh, 1, G, r0, T, 1.f, tid);
+    own_put<D>(sh, X, G, r0, T, scale_log2, tid);
     __syncthreads();
     auto share = [&](auto any) {
         constexpr bool ANY = decltype(any)::value;
@@ -460,7 +461,7 @@ __device__ __forceinline__ void bwd_rows(const BwdP& p, Shares<D>& sh, int bh, i
         }
     };
     share(std::false_type{});
-    if (any_nan(acc)) share(std::true_type{});
+    if (__builtin_expect(any_nan(acc), 0)) share(std::true_type{});
     sh.put(acc, p.alpha, wave, n, g);
     __syncthreads();
 #pragma unroll
@@ -488,8 +489,7 @@ __device__ __forceinline__ void bwd_cols(const BwdP& p, Shares<D>& sh, int bh, i
     const float scale_log2 = p.alpha * kLog2e;
     f32x16 accK[DT], accV[DT];
     float db;
-    own_put<D>(sh, 0, K, c0, T, scale_log2, tid);
-    own_put<D>(sh, 1, V, c0, T, 1.f, tid);
+    own_put<D>(sh, K, V, c0, T, scale_log2, tid);
     __syncthreads();
     auto share = [&](auto any) {
         constexpr bool ANY = decltype(any)::value;
@@ -554,7 +554,7 @@ __device__ __forceinline__ void bwd_cols(const BwdP& p, Shares<D>& sh, int bh, i
         }
     };
     share(std::false_type{});
-    if (any_nan(accK) || any_nan(accV)) share(std::true_type{});
+    if (__builtin_expect(any_nan(accK) || any_nan(accV), 0)) share(std::true_type{});
     db += __shfl_xor(db, 32, 64);
     if (g == 0) sh.row[wave][n] = db;
     sh.put(accK, p.alpha, wave, n, g);

@@ -52,7 +52,7 @@ __device__ __forceinline__ float largest8(const X& x) {
 template <typename X>
 __device__ __forceinline__ Split8 split8_any(const X& x) {
     Split8 s = split8(x);
-    if (__builtin_expect(largest8(x) > kSplitMax, 0)) {
+    if (__builtin_expect(__any(largest8(x) > kSplitMax), 0)) {  // (a uniform branch: its body is placed out of the way)
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             if (!(fabsf(x[e]) > kSplitMax)) continue;
@@ -65,6 +65,11 @@ __device__ __forceinline__ Split8 split8_any(const X& x) {
         }
     }
     return s;
+}
+template <bool ANY, typename X>
+__device__ __forceinline__ Split8 split_value(const X& x) {
+    if constexpr (ANY) return split8_any(x);
+    else return split8(x);
 }
 __device__ __forceinline__ f32x16 small_products(const Split8& a, const Split8& b, f32x16 c) {
     using M = Mma<__bf16>;

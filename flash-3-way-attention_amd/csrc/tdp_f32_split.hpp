@@ -145,6 +145,26 @@ __device__ __forceinline__ void split_products(Split8 (&s)[KS], const float* own
     }
 }
 
+// A backward that does not hold its operands (D = 128) has no round to test them in: whether the workgroup has met an own or a row
+// operand above 2^63 (below, no product of the two is too large for split8).  A word per wave; that wave's staging writes it ahead
+// of the barrier after which the operands are read, and a later one only sets it.  Backward of B=2 H=4 T=500 against no test: 6 % more
+// with every product tested as it is formed (4.87 -> 5.17 ms), 1 % with this (4.97 -> 5.00).  With the words instead of the test of
+// split_products the forward and D = 32, 64 were up to 2 % slower.
+constexpr float kSplitFactor = 0x1p63f;
+template <int NW>
+struct LargeOperands {
+    static_assert(NW == 4, "one 16-byte read");
+    int* words;  // [NW], 16-byte aligned
+    __device__ __forceinline__ void start(float most) const { words[threadIdx.x >> 6] = __any(most > kSplitFactor); }
+    __device__ __forceinline__ void more(float most) const {
+        if (__builtin_expect(__any(most > kSplitFactor), 0)) words[threadIdx.x >> 6] = 1;
+    }
+    __device__ __forceinline__ bool any() const {
+        const int4 w = *reinterpret_cast<const int4*>(words);
+        return __builtin_amdgcn_readfirstlane(w.x | w.y | w.z | w.w) != 0;
+    }
+};
+
 // Split of a pair of floats in two slots of vector work: s's elements e, e + 1
 struct SplitPair {
     f32x2 r;
@@ -598,7 +618,8 @@ __device__ __forceinline__ void f32_split_bwd_body(const F32SplitBwdParams& p, c
     constexpr bool AHEAD = D == 64, HOLD = D <= 64;
     constexpr int NBUF = AHEAD ? 3 : 2;
     extern __shared__ __align__(16) float smem_f[];
-    float* sKo = smem_f;                 // [32][LD]  own rows: KO * alpha * log2(e)
+    const LargeOperands<NW> large{reinterpret_cast<int*>(smem_f)};  // [NW]  not HOLD
+    float* sKo = smem_f + NW;            // [32][LD]  own rows: KO * alpha * log2(e)
     float* sVo = sKo + 32 * LD;          // [32][LD]  VO
     float* sKb = sVo + 32 * LD;          // [3][NW][D]  rows of a round
     float* sVb = sKb + 3 * NW * D;       // [3][NW][D]
@@ -665,6 +686,12 @@ __device__ __forceinline__ void f32_split_bwd_body(const F32SplitBwdParams& p, c
             row_v[i] = VB[at];
         }
     };
+    auto rows_most = [&] {
+        float most = 0.f;
+#pragma unroll
+        for (int i = 0; i < kRowPer; ++i) most = fmaxf(most, fmaxf(fabsf(row_k[i]), fabsf(row_v[i])));
+        return most;
+    };
     auto store_rows = [&](int slot) {
 #pragma unroll
         for (int i = 0; i < kRowPer; ++i)
@@ -680,11 +707,14 @@ __device__ __forceinline__ void f32_split_bwd_body(const F32SplitBwdParams& p, c
     }
     const float* KO = (KEYS ? p.k1 : p.q) + base;
     const float* VO = (KEYS ? p.u : p.d_o) + base;
+    [[maybe_unused]] float most = 0.f;
     for (int idx = tid; idx < 32 * D; idx += NT) {
         const int r = idx / D, d = idx % D;
         const size_t at = (size_t)min(o0 + r, T - 1) * D + d;
-        sKo[r * LD + d] = KO[at] * scale_log2;
-        sVo[r * LD + d] = VO[at];
+        const float ko = KO[at] * scale_log2, vo = VO[at];
+        sKo[r * LD + d] = ko;
+        sVo[r * LD + d] = vo;
+        if (!HOLD) most = fmaxf(most, fmaxf(fabsf(ko), fabsf(vo)));
     }
     float fscale_k = 0.f, fscale_v = 0.f;
     if (KEYS && p.rows.maxima) {
@@ -704,8 +734,10 @@ __device__ __forceinline__ void f32_split_bwd_body(const F32SplitBwdParams& p, c
     }
     if (have) {
         store_rows(0);
+        if (!HOLD) most = fmaxf(most, rows_most());
         complete(0);
     }
+    if (!HOLD) large.start(most);
     bool fresh1 = have1 && w1.m != w0.m;  // w1 is the first step of its round
     if (AHEAD && have1) {
         fetch(w1.st, 1);
@@ -774,7 +806,8 @@ __device__ __forceinline__ void f32_split_bwd_body(const F32SplitBwdParams& p, c
         }(std::make_integer_sequence<int, KS>{});
     };
     // the same without held operands
-    auto scores_formed = [&](int buf, int slot, f32x16& s, f32x16& dp) {
+    auto scores_formed = [&](int buf, int slot, f32x16& s, f32x16& dp, auto any) {
+        constexpr bool ANY = decltype(any)::value;
         const __bf16 *tk = sK + buf * STAGE, *tv = sV + buf * STAGE;
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
@@ -785,8 +818,8 @@ __device__ __forceinline__ void f32_split_bwd_body(const F32SplitBwdParams& p, c
         asm volatile("" : "+v"(own), "+v"(at));  // (opaque: every read is one of them plus an immediate offset)
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
-            s = products_of_step(split_rows<D>(tk, row_base, ks), split8_any(row_product(sKo + own, sKb + at, ks)), s);
-            dp = products_of_step(split_rows<D>(tv, row_base, ks), split8_any(row_product(sVo + own, sVb + at, ks)), dp);
+            s = products_of_step(split_rows<D>(tk, row_base, ks), split_value<ANY>(row_product(sKo + own, sKb + at, ks)), s);
+            dp = products_of_step(split_rows<D>(tv, row_base, ks), split_value<ANY>(row_product(sVo + own, sVb + at, ks)), dp);
             __builtin_amdgcn_sched_barrier(0);  // one k-step's operands in registers at a time
         }
     };
@@ -827,7 +860,8 @@ __device__ __forceinline__ void f32_split_bwd_body(const F32SplitBwdParams& p, c
             if (HOLD && fresh) form_operands(slot0);
             fresh = fresh1;
             if constexpr (HOLD) scores(buf, s, dp, [](auto) {});
-            else scores_formed(buf, slot0, s, dp);
+            else if (__builtin_expect(large.any(), 0)) scores_formed(buf, slot0, s, dp, std::true_type{});
+            else scores_formed(buf, slot0, s, dp, std::false_type{});
         }
         const int b = w0.m * NW + wave, a0 = w0.st * 32;
         const bool row_ok = b <= rows.hi && b >= rows.lo;
@@ -965,7 +999,10 @@ __device__ __forceinline__ void f32_split_bwd_body(const F32SplitBwdParams& p, c
                 if (fresh2) store_rows(slot2);
                 if (have2) complete(buf2);
             } else {
-                if (fresh1) store_rows(slot1);
+                if (fresh1) {
+                    store_rows(slot1);
+                    if (!HOLD) large.more(rows_most());
+                }
                 complete(buf1);
             }
             __syncthreads();
@@ -1023,7 +1060,7 @@ template <int D, int NW>
 constexpr size_t f32_split_bwd_smem() {
     constexpr int bufs = D == 64 ? 3 : 2;
     constexpr size_t loop = sizeof(float) * (6 * NW * D + bufs * 64) + bufs * 2 * 3 * sizeof(__bf16) * split_plane<D>(), merge = sizeof(float) * NW * D * 33;
-    return sizeof(float) * 2 * 32 * f32_pitch<D>() + (loop > merge ? loop : merge);
+    return sizeof(float) * (NW + 2 * 32 * f32_pitch<D>()) + (loop > merge ? loop : merge);
 }
 
 }  // namespace
