@@ -1,9 +1,9 @@
-// Included by dps_mfma.hip inside namespace tritt::{anonymous}: the two backward attention-with-bias kernels in the
+// Included by dps_mfma.hip inside namespace tritt::{anonymous}: the two backward attention-with-bias kernels of D = 128 in the
 // shape of dps_fwd_shared.hpp.  A workgroup of kW waves owns 32 * kW rows (row kernel: query-like rows; column
 // kernel: key-like rows), one tile of 32 per wave, and walks the streamed 32-row tiles once for all of them; a
 // tile's packed operands land in an LDS ring by direct-to-LDS loads, kNS - 1 tiles ahead, and every wave reads its
 // MFMA operands (and the tile's per-row vectors) from there.  No partial result crosses waves, so nothing is merged;
-// the operand fetches from L2 drop by kW.  Taken by large grids (see run_bwd).
+// the operand fetches from L2 drop by kW.  Taken by large grids (see launch_bwd_d128).
 #pragma once
 
 template <int D, int kW, int kNS, int kTensors>
@@ -106,9 +106,9 @@ __global__ __launch_bounds__(64 * kW, 2) void attn_bwd_row_shared_kernel(AttnBwd
             dp[i] = 0.f;
         }
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) s = M::mma(*reinterpret_cast<const v8*>(st + ks * 1024 + lane * 16), xb[ks], s);
+        for (int ks = 0; ks < KS; ++ks) s = M::mma(*reinterpret_cast<const v8*>(st + ks * 1024 + p1_piece(lane, ks) * 16), xb[ks], s);
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) dp = M::mma(*reinterpret_cast<const v8*>(st + (KS + ks) * 1024 + lane * 16), gb[ks], dp);
+        for (int ks = 0; ks < KS; ++ks) dp = M::mma(*reinterpret_cast<const v8*>(st + (KS + ks) * 1024 + p1_piece(lane, ks) * 16), gb[ks], dp);
         float b[16];
         if constexpr (BIAS) {
             tile_vector(reinterpret_cast<const float*>(st + S::CH * 1024 + wave * 256), g, b);
@@ -169,7 +169,7 @@ __global__ __launch_bounds__(64 * kW, 2) void attn_bwd_row_shared_kernel(AttnBwd
 // streamed per tile: X and G in packing P1 (scores, dP) and in packing P2 (dK, dV), the rows' LSE and Delta
 // (D = 128: two owner operands and four accumulators of 32 registers each leave no room for 256 registers a lane)
 template <typename E, int D, int kW, int kNS, bool LINK, bool SV>
-__global__ __launch_bounds__(64 * kW, (D <= 64 ? 2 : 1)) void attn_bwd_col_shared_kernel(AttnBwdP<E, SV> p) {
+__global__ __launch_bounds__(64 * kW, 1) void attn_bwd_col_shared_kernel(AttnBwdP<E, SV> p) {
     using M = Mma<E>;
     using v8 = typename M::v8;
     using S = BwdSharedShape<D, kW, kNS, 4>;
@@ -258,9 +258,9 @@ __global__ __launch_bounds__(64 * kW, (D <= 64 ? 2 : 1)) void attn_bwd_col_share
             dp[i] = 0.f;
         }
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) s = M::mma(*reinterpret_cast<const v8*>(st + ks * 1024 + lane * 16), kb[ks], s);
+        for (int ks = 0; ks < KS; ++ks) s = M::mma(*reinterpret_cast<const v8*>(st + ks * 1024 + p1_piece(lane, ks) * 16), kb[ks], s);
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) dp = M::mma(*reinterpret_cast<const v8*>(st + (KS + ks) * 1024 + lane * 16), vbv[ks], dp);
+        for (int ks = 0; ks < KS; ++ks) dp = M::mma(*reinterpret_cast<const v8*>(st + (KS + ks) * 1024 + p1_piece(lane, ks) * 16), vbv[ks], dp);
         float ls[16], dl[16];
         tile_vector(reinterpret_cast<const float*>(st + S::CH * 1024 + wave * 256), g, ls);
         tile_vector(reinterpret_cast<const float*>(st + S::CH * 1024 + (kW + wave) * 256), g, dl);

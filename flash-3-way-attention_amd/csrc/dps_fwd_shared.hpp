@@ -6,7 +6,7 @@
 // the streamed tiles, the operand fetches from L2 drop by kW and no partial softmax has to be merged.
 //
 // A packed tile is CH = 2 * D / 16 blocks of 64 lanes x 16 B, each exactly what one operand read of a wave wants, so
-// the blocks land in LDS as they lie in memory and lane i reads 16 B at block + 16 i: conflict-free without a swizzle.
+// the blocks land in LDS as they lie in memory and every 16 lanes read 16 pieces side by side: no bank conflicts.
 // Every wave fetches CH / kW blocks of each tile and its own copy of the bias (64 floats by one 4-byte load per
 // lane), so all waves issue the same number of loads per tile and one wait count serves them all.
 #pragma once
@@ -114,7 +114,7 @@ __global__ __launch_bounds__(64 * kW, 2) void attn_fwd_shared_kernel(AttnFwdP<E,
         for (int i = 0; i < 16; ++i) s[i] = 0.f;
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks)
-            s = M::mma(*reinterpret_cast<const v8*>(st + ks * 1024 + lane * 16), xb[ks], s);
+            s = M::mma(*reinterpret_cast<const v8*>(st + ks * 1024 + p1_piece(lane, ks) * 16), xb[ks], s);
         float b[16];
         if constexpr (BIAS) {
             const float* sb = reinterpret_cast<const float*>(st + S::CH * 1024 + wave * 256);
@@ -183,7 +183,11 @@ __global__ __launch_bounds__(64 * kW, 2) void attn_fwd_shared_kernel(AttnFwdP<E,
 
     if (rw0 >= Tp) return;  // no row of this wave exists, not even as padding of the packed outputs
     const float inv = 1.0f / l;
-    if (g == 0 && r < T) p.lse[(size_t)bh * p.lse_stride + r] = (m + fast_log2(l)) * p.lse_scale;
+    if (g == 0 && r < T) {
+        const float lse = (m + fast_log2(l)) * p.lse_scale;
+        p.lse[(size_t)bh * p.lse_stride + r] = lse;
+        if (p.term) p.term[(size_t)bh * p.lse_stride + r] = lse * p.term_scale;
+    }
     float* sT = reinterpret_cast<float*>(smem_raw + wave * S::kOutTile);  // [D][kLdr], this wave's alone
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)

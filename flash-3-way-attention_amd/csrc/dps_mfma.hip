@@ -7,13 +7,14 @@
 //   outer:  O[q] = softmax_t(alpha Q_q.K2_t + lse1[t]) @ W,  LSE[q] = logsumexp_t(.)
 // and the backward is the two attention backwards chained through (dR, dlse1).
 //
-// Three kernels, each a generic "attention with a per-key bias" building block on 32x32x16 MFMA:
-//   attn_fwd_mfma_kernel       owner = 32 query-like rows;  out, out*mul, (out*mul)^T, lse
-//   attn_bwd_row_mfma_kernel   owner = 32 query-like rows;  dX
-//   attn_bwd_col_mfma_kernel   owner = 32 key-like rows;    dK, dV, dbias (+ the element-wise link
-//                              between the two passes when it runs the outer pass)
-// A workgroup is kW (2 or 4) waves that share one owner tile and split the streamed 32-row tiles between
-// them round-robin (their partial results meet in LDS).
+// Generic "attention with a per-key bias" building blocks on 32x32x16 MFMA, each in a form for small grids and one for large:
+//   forward        owner = 32 query-like rows;  out, out*mul, (out*mul)^T, lse
+//   backward rows  owner = 32 query-like rows;  dX
+//   backward cols  owner = 32 key-like rows;    dK, dV, dbias (+ the element-wise link
+//                  between the two passes when it runs the outer pass)
+// Here: the forward and, for D = 128, the two backward kernels whose workgroups are kW (2 or 4) waves that share one owner
+// tile and split the streamed 32-row tiles between them round-robin (their partial results meet in LDS).
+// dps_bwd_tiles.hpp: the backward at D = 32 and 64; dps_fwd_shared.hpp, dps_bwd_shared.hpp: large grids otherwise.
 // Every tile is computed transposed where needed so that the owner index sits on the MFMA column
 // (= lane) axis: softmax statistics, LSE and Delta stay lane-local, and with the permuted row order
 // of mfma.hpp the probabilities leave one MFMA in exactly the operand layout of the next.
@@ -22,7 +23,7 @@
 // 16-byte pieces from 32 different rows costs one cache-line lookup per row, and that address
 // traffic, not MFMA or bandwidth, was what bound these kernels).  Two packings of a [T][D] tensor,
 // both in tiles of 32 rows and both exactly Tp x D elements:
-//   P1 (k-slots run along d; rows permuted by key_of_row):  [tile][ks][lane][8]
+//   P1 (k-slots run along d; rows permuted by key_of_row):  [tile][ks][p1_piece(lane, ks)][8]
 //   P2 (k-slots run along the row index; "transposed use"): [tile][dt][kk][lane][8]
 // The prep kernel writes them for the inputs, the producing epilogues for W and dR.  Every output
 // element has one owner: no atomics, bitwise reproducible.
@@ -57,10 +58,15 @@ __device__ __forceinline__ int launch_tiles(int pair, int nt) { return pair ? (n
 __device__ __forceinline__ int owner_tiles(int pair, int nt, int tile) { return (pair && tile != nt - 1 - tile) ? 2 : 1; }
 __device__ __forceinline__ int owner_tile(int nt, int tile, int part) { return part ? nt - 1 - tile : tile; }
 
+// Packing P1 keeps the 16 bytes of an operand load's lane at piece p1_piece(lane, ks) of the k-step's block.  The order
+// inside a block is free as far as operand loads go (the 64 pieces are one kilobyte either way); this one lets the
+// transposed LDS reads of a packed tile (dps_bwd_tiles.hpp) touch every bank once.
+__device__ __forceinline__ int p1_piece(int lane, int ks) { return lane ^ ((lane >> 5) << 2) ^ ((ks & 1) << 3); }
 // element offsets of (row, d) in the two packings
 template <int D>
 __device__ __forceinline__ size_t p1_index(int row, int d) {
-    return ((size_t)((row >> 5) * (D / 16) + (d >> 4)) * 64 + ((d >> 3) & 1) * 32 + row_of_key(row & 31)) * 8 + (d & 7);
+    const int lane = ((d >> 3) & 1) * 32 + row_of_key(row & 31);
+    return ((size_t)((row >> 5) * (D / 16) + (d >> 4)) * 64 + p1_piece(lane, d >> 4)) * 8 + (d & 7);
 }
 template <int D>
 __device__ __forceinline__ size_t p2_index(int row, int d) {
@@ -70,7 +76,7 @@ __device__ __forceinline__ size_t p2_index(int row, int d) {
 // the operand loads: lane's 16 bytes of (tile t, k-step ks) / (tile t, d-tile dt, half kk)
 template <typename E, int D>
 __device__ __forceinline__ const E* p1_at(const E* z, int t, int ks, int lane) {
-    return z + ((size_t)(t * (D / 16) + ks) * 64 + lane) * 8;
+    return z + ((size_t)(t * (D / 16) + ks) * 64 + p1_piece(lane, ks)) * 8;
 }
 template <typename E, int D>
 __device__ __forceinline__ const E* p2_at(const E* z, int t, int dt, int kk, int lane) {
@@ -162,6 +168,8 @@ struct AttnFwdP {
     E* outm_p2;         // out * mul, packing P2, or null
     float* lse;         // [BH][lse_stride]
     int lse_stride;
+    float* term;        // lse * term_scale as well, or null
+    float term_scale;
     int BH;
     int H;              // heads per batch entry in the views' indexing
     float lse_scale;    // lse = lse_scale * log2-sum-exp2
@@ -331,7 +339,11 @@ __global__ __launch_bounds__(64 * kW, 2) void attn_fwd_mfma_kernel(AttnFwdP<E, S
         ll += e[w] * sL[w * 32 + rr];
     }
     const float inv = 1.0f / ll;
-    if (dg == 0 && row < T) p.lse[(size_t)bh * p.lse_stride + row] = (mm + fast_log2(ll)) * p.lse_scale;
+    if (dg == 0 && row < T) {
+        const float lse = (mm + fast_log2(ll)) * p.lse_scale;
+        p.lse[(size_t)bh * p.lse_stride + row] = lse;
+        if (p.term) p.term[(size_t)bh * p.lse_stride + row] = lse * p.term_scale;
+    }
 #pragma unroll
     for (int c = dg; c < D / 8; c += 2 * kW) {  // 16-byte pieces dg, dg + 2 kW, ... of the row
         const int d0 = 8 * c;
@@ -386,7 +398,8 @@ struct AttnBwdP {
     const E *kp, *vp, *kp2, *xp, *gp, *xp2, *gp2;
     const float* bias;       // [BH][Tp] log2 units or null
     const float* lse2;       // [BH][Tp] log2 units
-    const float* delta;      // [BH][Tp]
+    const float* delta;      // [BH][Tp]; dps_bwd_tiles.hpp: -Delta
+    const float* term;       // dps_bwd_tiles.hpp: the streamed rows' term of the exponents / bwd_scale(alpha), [BH][Tp]
     int BH, T, Tp;
     int H;                   // heads per batch entry in the views' indexing
     float alpha;
@@ -551,28 +564,22 @@ __device__ __forceinline__ void attn_bwd_row_body(const AttnBwdP<E, SV>& p) {
 }
 
 template <typename E, int D, int kW, bool SV>
-__global__ __launch_bounds__(64 * kW, (D <= 64 ? 2 : 1)) void attn_bwd_row_mfma_kernel(AttnBwdP<E, SV> p) {
+__global__ __launch_bounds__(64 * kW, 1) void attn_bwd_row_mfma_kernel(AttnBwdP<E, SV> p) {
     attn_bwd_row_body<E, D, kW, SV>(p);
 }
 // Two row passes in one grid (blockIdx.y picks the pass): the outer pass's dQ and the inner pass's dK2 depend on
 // nothing of each other, and one pass alone gives a SIMD a single latency-bound wave.
 template <typename E, int D, int kW, bool SV>
-__global__ __launch_bounds__(64 * kW, (D <= 64 ? 2 : 1)) void attn_bwd_row_pair_kernel(AttnBwdP<E, SV> p0, AttnBwdP<E, SV> p1) {
+__global__ __launch_bounds__(64 * kW, 1) void attn_bwd_row_pair_kernel(AttnBwdP<E, SV> p0, AttnBwdP<E, SV> p1) {
     attn_bwd_row_body<E, D, kW, SV>(blockIdx.y == 0 ? p0 : p1);
 }
 
 // --------------------------------------------------------------------------- backward, columns
-// RING: every wave fetches its streamed tiles into a two-slot LDS ring of its own (direct-to-LDS loads, one tile ahead)
-// and reads the MFMA operands and the rows' statistics from there at the point of use, instead of holding the next
-// tile in registers: the kernel then fits 256 registers and two waves per SIMD (D = 64: 36 KB of LDS per wave).
-template <int D>
-constexpr int col_ring_tile_bytes() { return 4 * (D / 16) * 1024 + 2 * 256; }
-template <typename E, int D, int kW, bool LINK, bool SV, bool RING = false>
-__global__ __launch_bounds__(64 * kW, ((D <= 32 || RING) ? 2 : 1)) void attn_bwd_col_mfma_kernel(AttnBwdP<E, SV> p) {
+template <typename E, int D, int kW, bool LINK, bool SV>
+__global__ __launch_bounds__(64 * kW, 1) void attn_bwd_col_mfma_kernel(AttnBwdP<E, SV> p) {
     using M = Mma<E>;
     using v8 = typename M::v8;
     constexpr int KS = D / 16, DT = D / 32;
-    constexpr int kTileBytes = col_ring_tile_bytes<D>();
     extern __shared__ __align__(16) char smem_raw[];
     float* sO = reinterpret_cast<float*>(smem_raw);  // [kW][D][kLdr]
     float* sB = sO + kW * D * kLdr;                  // [kW][32]  dbias partials
@@ -620,82 +627,6 @@ __global__ __launch_bounds__(64 * kW, ((D <= 32 || RING) ? 2 : 1)) void attn_bwd
     float db = 0.f;
 
     const int t_first = r_lo / 32 + wave, t_last = r_hi / 32;
-    if constexpr (RING) {
-        char* ring = smem_raw + wave * 2 * kTileBytes;  // the merge tiles alias the rings: barrier before they are written
-        const char* XPc = reinterpret_cast<const char*>(uniform_ptr(XP));
-        const char* GPc = reinterpret_cast<const char*>(uniform_ptr(GP));
-        const char* XP2c = reinterpret_cast<const char*>(uniform_ptr(XP2));
-        const char* GP2c = reinterpret_cast<const char*>(uniform_ptr(GP2));
-        auto fetch = [&](int t, int slot) {
-            char* dst = ring + __builtin_amdgcn_readfirstlane(slot * kTileBytes);
-            const size_t tile_off = (size_t)__builtin_amdgcn_readfirstlane(t) * KS * 1024;
-#pragma unroll
-            for (int c = 0; c < KS; ++c) {
-                direct_load_16(uniform_ptr(XPc + tile_off + c * 1024), lane * 16, dst + c * 1024);
-                direct_load_16(uniform_ptr(GPc + tile_off + c * 1024), lane * 16, dst + (KS + c) * 1024);
-                direct_load_16(uniform_ptr(XP2c + tile_off + c * 1024), lane * 16, dst + (2 * KS + c) * 1024);
-                direct_load_16(uniform_ptr(GP2c + tile_off + c * 1024), lane * 16, dst + (3 * KS + c) * 1024);
-            }
-            const unsigned voff = (unsigned)min(t * 32 + lane, Tp - 1) * 4;
-            direct_load_4(lse2, voff, dst + 4 * KS * 1024);
-            direct_load_4(delta, voff, dst + 4 * KS * 1024 + 256);
-        };
-        if (t_first <= t_last) fetch(t_first, 0);
-        int slot = 0;
-        for (int t = t_first; t <= t_last; t += kW) {
-            const int r0 = t * 32;
-            // tile t has landed, and this wave's reads of the other slot are done: it may be overwritten
-            asm volatile("" ::: "memory");
-            __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (0 << 8) | (0 << 14));
-            asm volatile("" ::: "memory");
-            if (t + kW <= t_last) fetch(t + kW, slot ^ 1);
-            const char* st = ring + slot * kTileBytes;
-            slot ^= 1;
-            f32x16 s, dp;
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                s[i] = 0.f;
-                dp[i] = 0.f;
-            }
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks) s = M::mma(*reinterpret_cast<const v8*>(st + ks * 1024 + lane * 16), kb[ks], s);
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks) dp = M::mma(*reinterpret_cast<const v8*>(st + (KS + ks) * 1024 + lane * 16), vbv[ks], dp);
-            float ls[16], dl[16];
-            tile_vector(reinterpret_cast<const float*>(st + 4 * KS * 1024), g, ls);
-            tile_vector(reinterpret_cast<const float*>(st + 4 * KS * 1024 + 256), g, dl);
-            const bool edge = (r0 + 31 >= T) || (c0 + 31 >= T) || (p.causal && ((c0 + 31 > r0) || (r0 + 31 - c0 > p.k_diff)));
-            float pr[16], ds[16];
-            if (edge) {
-#pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    const int r = r0 + key_of(g, i);
-                    const bool ok = pair_ok(T, p.causal, p.k_diff, r, a);
-                    pr[i] = ok ? fast_exp2(fmaf(s[i], scale_log2, ba - ls[i])) : 0.f;
-                    ds[i] = ok ? pr[i] * (dp[i] - dl[i]) : 0.f;
-                    db += ds[i];
-                }
-            } else {
-#pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    pr[i] = fast_exp2(fmaf(s[i], scale_log2, ba - ls[i]));
-                    ds[i] = pr[i] * (dp[i] - dl[i]);
-                    db += ds[i];
-                }
-            }
-            v8 pb[2], dsb[2];
-            pack16<E>(pr, pb);
-            pack16<E>(ds, dsb);
-#pragma unroll
-            for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-                for (int kk = 0; kk < 2; ++kk) {
-                    acck[dt] = M::mma(*reinterpret_cast<const v8*>(st + (2 * KS + dt * 2 + kk) * 1024 + lane * 16), dsb[kk], acck[dt]);
-                    accv[dt] = M::mma(*reinterpret_cast<const v8*>(st + (3 * KS + dt * 2 + kk) * 1024 + lane * 16), pb[kk], accv[dt]);
-                }
-        }
-        __syncthreads();  // every wave is done with its ring: the merge tiles go on top of them
-    } else {
     // streamed operands and the per-row statistics of a tile are fetched one tile ahead, into the
     // registers the previous tile has just consumed
     v8 xn[KS], gn[KS], x2n[DT][2], g2n[DT][2];
@@ -780,7 +711,6 @@ __global__ __launch_bounds__(64 * kW, ((D <= 32 || RING) ? 2 : 1)) void attn_bwd
             }
         if (more) fetch_cols(t + kW);
     }
-    }  // operands from registers
     db += __shfl_xor(db, 32, 64);
 
     const int aa = tid & 31, dg = tid >> 5, row = c0 + aa;
@@ -881,6 +811,7 @@ __global__ __launch_bounds__(64 * kW, ((D <= 32 || RING) ? 2 : 1)) void attn_bwd
 }
 
 #include "dps_bwd_shared.hpp"
+#include "dps_bwd_tiles.hpp"
 
 // --------------------------------------------------------------------------------------- prep
 // Operand-packed copies of the inputs (U = SiLU(V1); rows past T are written as zeros), U row-major, and
@@ -895,6 +826,10 @@ struct PrepP {
     E *up1, *k1p1, *k2p1, *qp1, *dop1;  // packing P1
     E *up2, *k1p2, *k2p2, *qp2, *dop2;  // packing P2
     float *lse2, *delta;
+    float *row_term, *key_term;  // dps_bwd_tiles.hpp: -lse2 and, from lse1 in log2 units, lse1, both times term_scale
+    const float* lse1;
+    float term_scale;
+    float delta_sign;  // -1: delta receives -Delta (dps_bwd_tiles.hpp starts its dP products from it)
     // the forward's R, for W = R * V2
     const float* r;
     View<E, SV> v2;
@@ -991,8 +926,11 @@ __global__ __launch_bounds__(256) void dps_prep_kernel(PrepP<E, SV> p) {
 #pragma unroll
             for (int off = cpr >> 1; off > 0; off >>= 1) part += __shfl_xor(part, off, 64);
             if (c == 0) {
-                p.delta[(size_t)bh * Tp + j] = part;
-                p.lse2[(size_t)bh * Tp + j] = j < T ? p.lse[(size_t)bh * T + j] * kLog2e : 0.f;
+                p.delta[(size_t)bh * Tp + j] = part * p.delta_sign;
+                const float lse2 = j < T ? p.lse[(size_t)bh * T + j] * kLog2e : 0.f;
+                p.lse2[(size_t)bh * Tp + j] = lse2;
+                if (p.row_term) p.row_term[(size_t)bh * Tp + j] = -lse2 * p.term_scale;
+                if (p.key_term && p.lse1) p.key_term[(size_t)bh * Tp + j] = j < T ? p.lse1[(size_t)bh * Tp + j] * p.term_scale : 0.f;
             }
         }
     }
@@ -1000,7 +938,7 @@ __global__ __launch_bounds__(256) void dps_prep_kernel(PrepP<E, SV> p) {
 
 struct Layout {
     size_t up2, k1p1, k2p1, wp2, lse1;                                            // forward
-    size_t u, up1, k1p2, k2p2, qp1, qp2, dop1, dop2, w, wp1, dr, drp1, drp2, r, dk2p, lse2, delta, delta1;  // backward
+    size_t u, up1, k1p2, k2p2, qp1, qp2, dop1, dop2, w, wp1, dr, drp1, drp2, r, dk2p, lse2, delta, delta1, row_term, key_term;  // backward
     size_t total;
 };
 Layout layout(int BH, int T, int D, bool bwd) {
@@ -1021,22 +959,28 @@ Layout layout(int BH, int T, int D, bool bwd) {
     if (bwd) {
         l.u = take(n * 2);
         l.up1 = take(nt * 2);
-        l.k1p2 = take(nt * 2);
-        l.k2p2 = take(nt * 2);
         l.qp1 = take(nt * 2);
-        l.qp2 = take(nt * 2);
         l.dop1 = take(nt * 2);
-        l.dop2 = take(nt * 2);
         l.w = take(n * 2);
         l.wp1 = take(nt * 2);
         l.dr = take(n * 2);
         l.drp1 = take(nt * 2);
-        l.drp2 = take(nt * 2);
+        if (D > 64) {  // the kernels of D = 32 and 64 read packing P1 both ways
+            l.k1p2 = take(nt * 2);
+            l.k2p2 = take(nt * 2);
+            l.qp2 = take(nt * 2);
+            l.dop2 = take(nt * 2);
+            l.drp2 = take(nt * 2);
+        }
         l.r = take(n * 4);
         l.dk2p = take(n * 4);
         l.lse2 = take(nv * 4);
         l.delta = take(nv * 4);
         l.delta1 = take(nv * 4);
+        if (D <= 64) {
+            l.row_term = take(nv * 4);
+            l.key_term = take(nv * 4);
+        }
     }
     l.total = (off + 255) & ~size_t(255);
     return l;
@@ -1044,11 +988,8 @@ Layout layout(int BH, int T, int D, bool bwd) {
 
 template <int D, int kW>
 constexpr size_t fwd_smem() { return 4 * (size_t)(kW * D * kLdr + 2 * kW * 32); }
-template <int D, int kW, bool RING = false>
-constexpr size_t col_smem() {
-    const size_t merge = 4 * (size_t)(kW * D * kLdr + kW * 32 + 2 * kW * 32), ring = (size_t)kW * 2 * col_ring_tile_bytes<D>();
-    return RING && ring > merge ? ring : merge;
-}
+template <int D, int kW>
+constexpr size_t col_smem() { return 4 * (size_t)(kW * D * kLdr + kW * 32 + 2 * kW * 32); }
 template <int D, int kW>
 constexpr size_t row_smem() { return 4 * (size_t)(kW * D * kLdr); }
 
@@ -1068,7 +1009,6 @@ dim3 attn_grid(const MfmaDpsArgs& a, int Tp, bool pair) {
     return dim3(8 * xcd_slots(a.BH, pair ? (nt + 1) / 2 : nt));
 }
 
-// one of the caller's tensors / a row-major tensor of the workspace as the kernels take them
 // one of the caller's tensors / a row-major tensor of the workspace as the kernels take them
 template <typename E, bool SV>
 View<E, SV> dense_view(const MfmaDpsArgs& a, const void* p) {
@@ -1110,6 +1050,8 @@ hipError_t run_fwd(const MfmaDpsArgs& a, hipStream_t st, bool for_bwd) {
     p.outm_p1 = for_bwd ? (E*)(ws + l.wp1) : nullptr;
     p.outm_p2 = (E*)(ws + l.wp2);
     p.lse = lse1; p.lse_stride = Tp; p.lse_scale = 1.0f;
+    if constexpr (D <= 64)
+        if (for_bwd) { p.term = (float*)(ws + l.key_term); p.term_scale = 1.f / bwd_scale(a.alpha); }
     p.BH = a.BH; p.H = a.H; p.T = a.T; p.Tp = Tp; p.scale_log2 = sl2; p.causal = a.causal; p.k_diff = a.k_diff;
     p.pair = pair_in;
     // Large grids take the kernel whose workgroups own 128 rows and share the streamed tiles through LDS
@@ -1143,24 +1085,80 @@ hipError_t run_fwd(const MfmaDpsArgs& a, hipStream_t st, bool for_bwd) {
     return hipGetLastError();
 }
 
+// D = 32 and 64: the outer column pass, then the other three passes in one grid (dps_bwd_tiles.hpp)
+template <typename E, int D, int kOT, int kSH, bool SV>
+hipError_t launch_bwd_tiles(const AttnBwdP<E, SV>& outer, const AttnBwdP<E, SV>& inner, hipStream_t st) {
+    constexpr size_t smem = BwdTiles<D, kOT, kSH>::smem;
+    auto link = attn_bwd_link_kernel<E, D, kOT, kSH, SV>;
+    auto rest = attn_bwd_rest_kernel<E, D, kOT, kSH, SV>;
+    hipError_t e = allow_smem(link, smem);
+    if (e == hipSuccess) e = allow_smem(rest, smem);
+    if (e != hipSuccess) return e;
+    const int slots = xcd_slots(outer.BH, (outer.Tp / 32 + kOT - 1) / kOT);
+    hipLaunchKernelGGL(link, dim3(8 * slots), dim3(256), smem, st, outer);
+    AttnBwdP<E, SV> outer_rows = outer;
+    outer_rows.term = inner.term;  // the outer column pass streams rows, the outer row pass the keys
+    hipLaunchKernelGGL(rest, dim3(8 * 3 * slots), dim3(256), smem, st, outer_rows, inner);
+    return hipGetLastError();
+}
+
+// D = 128: the passes one after the other
+template <typename E, int D, int kW, bool SV>
+hipError_t launch_bwd_d128(const MfmaDpsArgs& a, const AttnBwdP<E, SV>& o, const AttnBwdP<E, SV>& i, int Tp, hipStream_t st) {
+    auto krow = attn_bwd_row_mfma_kernel<E, D, kW, SV>;
+    auto kcol_link = attn_bwd_col_mfma_kernel<E, D, kW, true, SV>;
+    auto kcol = attn_bwd_col_mfma_kernel<E, D, kW, false, SV>;
+    hipError_t e = allow_smem(krow, row_smem<D, kW>());
+    if (e == hipSuccess) e = allow_smem(kcol_link, col_smem<D, kW>());
+    if (e == hipSuccess) e = allow_smem(kcol, col_smem<D, kW>());
+    if (e != hipSuccess) return e;
+    // Large grids: the kernels whose workgroups own 128 rows and share the streamed tiles through LDS
+    // (dps_bwd_shared.hpp), as the forward passes do (run_fwd).  They pay from 512 such workgroups on; measured
+    // backward, bf16, B=4 H=8 T=4096, one owner tile per workgroup -> shared tiles: 2120 -> 1935 us.
+    constexpr int kSW = 4, kRowNS = 4, kColNS = 3;
+    using RowShape = BwdSharedShape<D, kSW, kRowNS, 3>;
+    using ColShape = BwdSharedShape<D, kSW, kColNS, 4>;
+    const int owners = (Tp / 32 + kSW - 1) / kSW;
+    if (knobs().dps_shared ? knobs().dps_shared > 0 : (long long)a.BH * owners >= 512) {
+        const dim3 grid(8 * xcd_slots(a.BH, owners));
+        auto srow_out = attn_bwd_row_shared_kernel<E, D, kSW, kRowNS, true, SV>;
+        auto scol_out = attn_bwd_col_shared_kernel<E, D, kSW, kColNS, true, SV>;
+        auto srow_in = attn_bwd_row_shared_kernel<E, D, kSW, kRowNS, false, SV>;
+        auto scol_in = attn_bwd_col_shared_kernel<E, D, kSW, kColNS, false, SV>;
+        if (e = allow_smem(srow_out, RowShape::smem); e != hipSuccess) return e;
+        if (e = allow_smem(scol_out, ColShape::smem); e != hipSuccess) return e;
+        if (e = allow_smem(srow_in, RowShape::smem); e != hipSuccess) return e;
+        if (e = allow_smem(scol_in, ColShape::smem); e != hipSuccess) return e;
+        hipLaunchKernelGGL(srow_out, grid, dim3(64 * kSW), RowShape::smem, st, o);
+        hipLaunchKernelGGL(scol_out, grid, dim3(64 * kSW), ColShape::smem, st, o);
+        hipLaunchKernelGGL(srow_in, grid, dim3(64 * kSW), RowShape::smem, st, i);
+        hipLaunchKernelGGL(scol_in, grid, dim3(64 * kSW), ColShape::smem, st, i);
+        return hipGetLastError();
+    }
+    // the two row passes share a launch when their grids are the same (attn_bwd_row_pair_kernel); the outer one then
+    // waits for the outer column pass, which the inner one needs
+    const bool rows_together = o.pair == i.pair;
+    const dim3 grid_out = attn_grid(a, Tp, o.pair), grid_in = attn_grid(a, Tp, i.pair);
+    if (!rows_together) hipLaunchKernelGGL(krow, grid_out, dim3(64 * kW), (row_smem<D, kW>()), st, o);
+    hipLaunchKernelGGL(kcol_link, grid_out, dim3(64 * kW), (col_smem<D, kW>()), st, o);
+    if (rows_together) {
+        auto krow2 = attn_bwd_row_pair_kernel<E, D, kW, SV>;
+        if (e = allow_smem(krow2, row_smem<D, kW>()); e != hipSuccess) return e;
+        hipLaunchKernelGGL(krow2, dim3(grid_in.x, 2), dim3(64 * kW), (row_smem<D, kW>()), st, o, i);
+    } else {
+        hipLaunchKernelGGL(krow, grid_in, dim3(64 * kW), (row_smem<D, kW>()), st, i);
+    }
+    hipLaunchKernelGGL(kcol, grid_in, dim3(64 * kW), (col_smem<D, kW>()), st, i);
+    return hipGetLastError();
+}
+
 template <typename E, int D, int kW, bool SV>
 hipError_t run_bwd(const MfmaDpsArgs& a, hipStream_t st) {
     const int Tp = (a.T + 31) / 32 * 32;
     const Layout l = layout(a.BH, a.T, D, true);
     char* ws = static_cast<char*>(a.workspace);
     const dim3 grid(8 * xcd_slots(a.BH, Tp / 32));
-    const bool pair_in = pair_tiles(a, a.k_diff, grid.x, true), pair_out = pair_tiles(a, a.T, grid.x, true);
-    auto krow = attn_bwd_row_mfma_kernel<E, D, kW, SV>;
-    // the column kernel's operands through per-wave LDS rings (see the kernel) where four waves split the streamed tiles,
-    // i.e. from T = 2048 on; measured backward, bf16: B=1 H=8 T=4096 306 -> 291 us, B=2 H=8 T=2048 199 -> 191 us; with two
-    // waves (B=4 H=8 T=1024) 136.5 -> 138.7 us, so those keep the operands in registers
-    constexpr bool kRing = D == 64 && kW == 4;
-    auto kcol_link = attn_bwd_col_mfma_kernel<E, D, kW, true, SV, kRing>;
-    auto kcol = attn_bwd_col_mfma_kernel<E, D, kW, false, SV, kRing>;
-    hipError_t e = allow_smem(krow, row_smem<D, kW>());
-    if (e == hipSuccess) e = allow_smem(kcol_link, col_smem<D, kW, kRing>());
-    if (e == hipSuccess) e = allow_smem(kcol, col_smem<D, kW, kRing>());
-    if (e != hipSuccess) return e;
+    constexpr bool kTiles = D <= 64;
 
     PrepP<E, SV> pp{};
     pp.v1 = caller_view<E, SV>(a, a.v1, a.lv1); pp.k1 = caller_view<E, SV>(a, a.k1, a.lk1); pp.k2 = caller_view<E, SV>(a, a.k2, a.lk2);
@@ -1169,9 +1167,15 @@ hipError_t run_bwd(const MfmaDpsArgs& a, hipStream_t st) {
     pp.u = (E*)(ws + l.u);
     pp.up1 = (E*)(ws + l.up1); pp.k1p1 = (E*)(ws + l.k1p1); pp.k2p1 = (E*)(ws + l.k2p1);
     pp.qp1 = (E*)(ws + l.qp1); pp.dop1 = (E*)(ws + l.dop1);
-    pp.up2 = (E*)(ws + l.up2); pp.k1p2 = (E*)(ws + l.k1p2); pp.k2p2 = (E*)(ws + l.k2p2);
-    pp.qp2 = (E*)(ws + l.qp2); pp.dop2 = (E*)(ws + l.dop2);
-    pp.lse2 = (float*)(ws + l.lse2); pp.delta = (float*)(ws + l.delta);
+    pp.up2 = (E*)(ws + l.up2);
+    if constexpr (!kTiles) {
+        pp.k1p2 = (E*)(ws + l.k1p2); pp.k2p2 = (E*)(ws + l.k2p2);
+        pp.qp2 = (E*)(ws + l.qp2); pp.dop2 = (E*)(ws + l.dop2);
+    }
+    pp.lse2 = (float*)(ws + l.lse2); pp.delta = (float*)(ws + l.delta); pp.delta_sign = kTiles ? -1.f : 1.f;
+    if constexpr (kTiles) {
+        pp.row_term = (float*)(ws + l.row_term); pp.key_term = (float*)(ws + l.key_term); pp.term_scale = 1.f / bwd_scale(a.alpha);
+    }
     pp.BH = a.BH; pp.T = a.T; pp.Tp = Tp; pp.H = a.H;
     // R, W, W^T, lse1 of the inner pass: from the forward where the caller kept R and lse1 (W = R * V2 is then formed by the
     // prep launch), else by running that pass again.  Keeping them holds four bytes per element between the two calls and
@@ -1179,13 +1183,13 @@ hipError_t run_bwd(const MfmaDpsArgs& a, hipStream_t st) {
     // T=1024 154 -> 142 us, B=1 H=8 T=8192 k_diff 2048 822 -> 784 us.
     const float *r = (const float*)(ws + l.r), *lse1 = (const float*)(ws + l.lse1);
     if (a.kept_r) {
-        r = a.kept_r; lse1 = a.kept_lse1;
+        r = a.kept_r; lse1 = a.kept_lse1; pp.lse1 = lse1;
         pp.r = r; pp.v2 = caller_view<E, SV>(a, a.v2, a.lv2); pp.w = (E*)(ws + l.w); pp.wp1 = (E*)(ws + l.wp1);
         pp.up2 = nullptr;  // the inner pass's values
         hipLaunchKernelGGL((dps_prep_kernel<E, D, SV>), dim3(grid.x, 7), dim3(256), 0, st, pp);
     } else {
         hipLaunchKernelGGL((dps_prep_kernel<E, D, SV>), dim3(grid.x, 6), dim3(256), 0, st, pp);
-        e = run_fwd<E, D, kW, SV>(a, st, true);
+        const hipError_t e = run_fwd<E, D, kW, SV>(a, st, true);
         if (e != hipSuccess) return e;
     }
 
@@ -1193,81 +1197,45 @@ hipError_t run_bwd(const MfmaDpsArgs& a, hipStream_t st) {
     AttnBwdP<E, SV> o{};
     o.x = caller_view<E, SV>(a, a.q, a.lq); o.g = caller_view<E, SV>(a, a.d_o, a.ldo); o.k = caller_view<E, SV>(a, a.k2, a.lk2);
     o.v = dense_view<E, SV>(a, ws + l.w);
-    o.kp = (const E*)(ws + l.k2p1); o.vp = (const E*)(ws + l.wp1); o.kp2 = (const E*)(ws + l.k2p2);
+    o.kp = (const E*)(ws + l.k2p1); o.vp = (const E*)(ws + l.wp1);
     o.xp = (const E*)(ws + l.qp1); o.gp = (const E*)(ws + l.dop1);
-    o.xp2 = (const E*)(ws + l.qp2); o.gp2 = (const E*)(ws + l.dop2);
     o.bias = lse1; o.lse2 = (const float*)(ws + l.lse2); o.delta = (const float*)(ws + l.delta);
     o.BH = a.BH; o.H = a.H; o.T = a.T; o.Tp = Tp; o.alpha = a.alpha; o.causal = a.causal; o.k_diff = a.T;
-    o.pair = pair_out;
     o.dx = (E*)a.dq;
     o.dk_f32 = (float*)(ws + l.dk2p);
     o.r_f32 = r; o.v2 = caller_view<E, SV>(a, a.v2, a.lv2); o.dv2 = (E*)a.dv2;
-    o.dr = (E*)(ws + l.dr); o.dr_p1 = (E*)(ws + l.drp1); o.dr_p2 = (E*)(ws + l.drp2); o.delta1 = (float*)(ws + l.delta1);
-    // Large grids: the kernels whose workgroups own 128 rows and share the streamed tiles through LDS
-    // (dps_bwd_shared.hpp), as the forward passes do (run_fwd).  They pay from 512 such workgroups on; measured
-    // backward, bf16 D = 64, one owner tile per workgroup -> shared tiles: B=8 H=16 T=2048 1650 -> 972 us, B=4 H=8
-    // T=4096 1245 -> 825 us, B=8 H=16 T=1024 510 -> 376 us, B=4 H=8 T=2048 (512 workgroups) 387 -> 313 us, B=1 H=8
-    // T=8192 (512) 1040 -> 1000 us, but B=1 H=8 T=4096 (256) 306 -> 506 us and B=4 H=8 T=1024 (256) 136 -> 175 us;
-    // D = 128, B=4 H=8 T=4096: 2120 -> 1935 us.
-    constexpr int kSW = 4, kRowNS = 4, kColNS = D > 64 ? 3 : 4;
-    using RowShape = BwdSharedShape<D, kSW, kRowNS, 3>;
-    using ColShape = BwdSharedShape<D, kSW, kColNS, 4>;
-    const int owners = (Tp / 32 + kSW - 1) / kSW;
-    bool shared = false;
-    if constexpr (D >= 64) shared = knobs().dps_shared ? knobs().dps_shared > 0 : (long long)a.BH * owners >= 512;
-    const dim3 grid_shared(8 * xcd_slots(a.BH, owners));
-    if constexpr (D >= 64) {
-        if (shared) {
-            auto srow_out = attn_bwd_row_shared_kernel<E, D, kSW, kRowNS, true, SV>;
-            auto scol_out = attn_bwd_col_shared_kernel<E, D, kSW, kColNS, true, SV>;
-            if (e = allow_smem(srow_out, RowShape::smem); e != hipSuccess) return e;
-            if (e = allow_smem(scol_out, ColShape::smem); e != hipSuccess) return e;
-            hipLaunchKernelGGL(srow_out, grid_shared, dim3(64 * kSW), RowShape::smem, st, o);
-            hipLaunchKernelGGL(scol_out, grid_shared, dim3(64 * kSW), ColShape::smem, st, o);
-        }
-    }
-    // the two row passes share a launch when their grids are the same (attn_bwd_row_pair_kernel); the outer one then
-    // waits for the outer column pass, which the inner one needs
-    const bool rows_together = !shared && pair_out == pair_in;
-    if (!shared) {
-        if (!rows_together) hipLaunchKernelGGL(krow, attn_grid(a, Tp, pair_out), dim3(64 * kW), (row_smem<D, kW>()), st, o);
-        hipLaunchKernelGGL(kcol_link, attn_grid(a, Tp, pair_out), dim3(64 * kW), (col_smem<D, kW, kRing>()), st, o);
-    }
+    o.dr = (E*)(ws + l.dr); o.dr_p1 = (E*)(ws + l.drp1); o.delta1 = (float*)(ws + l.delta1);
 
     // inner pass: X = K2, G = dR, K = K1, V = U
     AttnBwdP<E, SV> i{};
     i.x = caller_view<E, SV>(a, a.k2, a.lk2); i.g = dense_view<E, SV>(a, ws + l.dr); i.k = caller_view<E, SV>(a, a.k1, a.lk1);
     i.v = dense_view<E, SV>(a, ws + l.u);
-    i.kp = (const E*)(ws + l.k1p1); i.vp = (const E*)(ws + l.up1); i.kp2 = (const E*)(ws + l.k1p2);
+    i.kp = (const E*)(ws + l.k1p1); i.vp = (const E*)(ws + l.up1);
     i.xp = (const E*)(ws + l.k2p1); i.gp = (const E*)(ws + l.drp1);
-    i.xp2 = (const E*)(ws + l.k2p2); i.gp2 = (const E*)(ws + l.drp2);
     i.lse2 = lse1; i.delta = (const float*)(ws + l.delta1);
     i.BH = a.BH; i.H = a.H; i.T = a.T; i.Tp = Tp; i.alpha = a.alpha; i.causal = a.causal; i.k_diff = a.k_diff;
-    i.pair = pair_in;
     i.addend = (const float*)(ws + l.dk2p); i.dx = (E*)a.dk2;
     i.dk = (E*)a.dk1; i.v1 = caller_view<E, SV>(a, a.v1, a.lv1); i.dv = (E*)a.dv1;
-    if constexpr (D >= 64) {
-        if (shared) {
-            auto srow_in = attn_bwd_row_shared_kernel<E, D, kSW, kRowNS, false, SV>;
-            auto scol_in = attn_bwd_col_shared_kernel<E, D, kSW, kColNS, false, SV>;
-            if (e = allow_smem(srow_in, RowShape::smem); e != hipSuccess) return e;
-            if (e = allow_smem(scol_in, ColShape::smem); e != hipSuccess) return e;
-            hipLaunchKernelGGL(srow_in, grid_shared, dim3(64 * kSW), RowShape::smem, st, i);
-            hipLaunchKernelGGL(scol_in, grid_shared, dim3(64 * kSW), ColShape::smem, st, i);
-        }
+
+    if constexpr (kTiles) {
+        o.term = (const float*)(ws + l.row_term);
+        i.term = (const float*)(ws + l.key_term);
+        // 128 rows per workgroup (a wave per owner tile) on large grids, 64 (two waves share an owner tile) on small ones:
+        // the first fetch half as much from L2 and join nothing, the second are twice as many and level out better.  From 512
+        // to 1023 workgroups of 128 rows the grid is resident at once, so the longer the sequence, the more its longest
+        // blocks stand out.  Training steps, bf16, 64 rows -> 128: B=4 H=8 T=1024 (256 workgroups) 112 -> 145 us, B=8 H=16
+        // T=500 (512) 162 -> 157, B=1 H=8 T=8192 k_diff 2048 (512) 583 -> 600, D = 32 487 -> 518, B=8 H=16 T=1024 (1024)
+        // 422 -> 358, T=2048 1209 -> 985.
+        const long long blocks = (long long)a.BH * ((Tp / 32 + 3) / 4);
+        const bool wide = knobs().dps_shared ? knobs().dps_shared > 0 : blocks >= 1024 || (blocks >= 512 && a.T < 4096);
+        return wide ? launch_bwd_tiles<E, D, 4, 1, SV>(o, i, st) : launch_bwd_tiles<E, D, 2, 2, SV>(o, i, st);
+    } else {
+        o.kp2 = (const E*)(ws + l.k2p2); o.xp2 = (const E*)(ws + l.qp2); o.gp2 = (const E*)(ws + l.dop2); o.dr_p2 = (E*)(ws + l.drp2);
+        i.kp2 = (const E*)(ws + l.k1p2); i.xp2 = (const E*)(ws + l.k2p2); i.gp2 = (const E*)(ws + l.drp2);
+        o.pair = pair_tiles(a, a.T, grid.x, true);
+        i.pair = pair_tiles(a, a.k_diff, grid.x, true);
+        return launch_bwd_d128<E, D, kW, SV>(a, o, i, Tp, st);
     }
-    if (!shared) {
-        if (rows_together) {
-            auto krow2 = attn_bwd_row_pair_kernel<E, D, kW, SV>;
-            if (e = allow_smem(krow2, row_smem<D, kW>()); e != hipSuccess) return e;
-            const dim3 g1 = attn_grid(a, Tp, pair_in);
-            hipLaunchKernelGGL(krow2, dim3(g1.x, 2), dim3(64 * kW), (row_smem<D, kW>()), st, o, i);
-        } else {
-            hipLaunchKernelGGL(krow, attn_grid(a, Tp, pair_in), dim3(64 * kW), (row_smem<D, kW>()), st, i);
-        }
-        hipLaunchKernelGGL(kcol, attn_grid(a, Tp, pair_in), dim3(64 * kW), (col_smem<D, kW, kRing>()), st, i);
-    }
-    return hipGetLastError();
 }
 
 }  // namespace

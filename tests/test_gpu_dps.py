@@ -609,3 +609,44 @@ def test_fp32_operands_at_the_end_of_the_range(T, k_diff, D):
     z, _, _ = orc.dps_forward_backward(*(t[0, h].double() for t in inputs), scale, False, factorised=True)
     err = ((out[0, h, :, 5].double() - z[:, 5]).norm() / z[:, 5].norm()).item()
     assert err <= bar, err
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 64), (torch.float16, 64), (torch.bfloat16, 32)])
+@pytest.mark.parametrize("T,causal,k_diff", [(31, True, 31), (32, True, 0), (33, True, 32), (65, True, 31), (129, True, 33), (160, True, 160),
+                                             (161, True, 63), (257, True, 64), (96, False, 96), (130, False, 130)])
+@pytest.mark.parametrize("blocks", [-1, 1])
+def test_backward_tiles(dtype, D, T, causal, k_diff, blocks, tune):
+    """The backward passes at D = 32 and 64 in both shapes (workgroups of 64 rows whose tiles two waves share, and of 128) where
+    a tile, a band or an owner block ends, against the oracle; and, where the streamed terms are divided by a scale that is
+    negative, tiny or zero (the oracle masks its scores ahead of the scale), against the library's fp32 kernels."""
+    from flash_trittention import _lib
+
+    print(f"case dps backward tiles {dtype} D={D} T={T} causal={causal} k_diff={k_diff} blocks={blocks}", flush=True)
+    tune(_lib.TUNE_DPS_SHARED, blocks)
+    inputs, alpha = orc.make_inputs(1, 3, T, D, dtype, seed=T + k_diff), 1 / math.sqrt(D)
+    got, want = util.run_dps(inputs, alpha, causal, k_diff, flags=_lib.FLAG_FORCE_MFMA)[2], util.oracle_dps(inputs, alpha, causal, k_diff)[2]
+    for name, a, b in zip(util.NAMES, got, want):
+        util.assert_close(name, a, b, **LOWP)
+    for alpha in (-0.2, 1e-30, 0.0) if T in (65, 130) else ():
+        got, want = (util.run_dps(inputs, alpha, causal, k_diff, flags=f)[2] for f in (_lib.FLAG_FORCE_MFMA, _lib.FLAG_FORCE_GENERIC))
+        for name, a, b in zip(util.NAMES, got, want):
+            util.assert_close(f"{name} at {alpha}", a, b.float().cpu(), **LOWP)
+
+
+@pytest.mark.parametrize("blocks", [-1, 1])
+def test_an_infinite_gradient_row_stays_in_its_tiles(blocks, tune):
+    """One row of dO that is not finite reaches dQ of its own 32 rows and the key gradients of the tiles at and before it: keys of later
+    tiles, and under a band those before it, keep the gradients they have without that row."""
+    from flash_trittention import _lib
+
+    print(f"case dps infinite row blocks={blocks}", flush=True)
+    T, k_diff = 320, 32
+    tune(_lib.TUNE_DPS_SHARED, blocks)
+    inputs = orc.make_inputs(1, 2, T, 64, torch.bfloat16, seed=8)
+    plain = util.run_dps(inputs, 0.125, True, k_diff)[2]
+    inputs[5][:, :, 170] = math.inf
+    got = util.run_dps(inputs, 0.125, True, k_diff)[2]
+    assert not torch.isfinite(got[0][:, :, 170]).any()
+    for name, a, b in zip(util.NAMES, got, plain):
+        assert torch.isfinite(b).all() and torch.equal(a[:, :, 192:], b[:, :, 192:]), name
+    assert torch.equal(got[0][:, :, :160], plain[0][:, :, :160])
