@@ -265,13 +265,14 @@ __global__ __launch_bounds__(64 * WAVES, MINW) void tdp_fwd_mfma_kernel(FwdParam
     };
 
     // ---- prologue: Q tile, first k-tile, first stage ------------------------------------------
+    // (all asked for before any of it is waited for)
+    issue_ktile(kt_lo);
+    issue_stage(first_stage(kt_lo));
     for (int idx = tid; idx < BQ * D; idx += NTH) {
         const int r = idx / D, d = idx % D;
         sQ[r * LDQ + d] = (float)Q[(size_t)((unsigned)min(q0 + r, T - 1) * in_st) + d] * p.scale_log2;
     }
     if (tid < 2) sFlag[tid] = 0;  // two flags, used by alternate k-tiles
-    issue_ktile(kt_lo);
-    issue_stage(first_stage(kt_lo));
     commit_ktile(0);
     commit_stage(0);
     __syncthreads();
