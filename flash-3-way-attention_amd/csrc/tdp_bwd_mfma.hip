@@ -233,7 +233,7 @@ __device__ __forceinline__ void tdp_bwd_rows_body(const BwdParams<E>& p, const i
 
     // Prologue: first round and first two stages, Q / dO tiles in both forms, the rows' statistics.  Everything is asked for
     // before anything is waited for: a workgroup has a CU to itself, and nothing else runs under these round trips (element
-    // by element and one tensor after the other, a training step B=2 H=4 T=256 took 147.3 us, now 145.1).
+    // by element and one tensor after the other, a training step B=2 H=4 T=256 took 147.3 us, then 145.1).
     // the stage fetched next (the sweep repeats every round, so the stage numbers cycle)
     int st_ahead = 0;
     auto advance = [&]() { st_ahead = st_ahead + 1 < nst ? st_ahead + 1 : 0; };
@@ -755,18 +755,21 @@ static BwdLayout bwd_layout(int BH, int T, int D, bool fixed_point) {
     return l;
 }
 
-// Workgroups per query tile under a window at D = 64, by the time that the launch takes with s of them: one workgroup
-// fills a CU, and all tiles but those at the start of the sequence cost the same, so the launch takes the larger of
-// whole rounds of the full tiles' parts over the CUs and of the even share plus half a part of tail.  Work in 32-key steps
-// of eight rows; a part's own prologue, dQ's shares and tail are worth about nine of them.  The model is that of one role's
-// workgroups in a launch of their own.  In the grid that holds both roles its choice (backward, chosen / best): B=2 H=4 T=2048
-// window 512 6 parts 4.09 ms / 3 parts 4.00, B=1 H=8 T=700 window 100 3 parts 214 us, B=2 H=8 T=2048 window 100 1 part 1.02 ms (both
-// the best), B=1 H=4 T=1500 window 300 6 parts 724 / 3 parts 707, B=4 H=8 T=1024 window 200 2 parts 2.00 / 1 part 1.92, B=1 H=2
-// T=1999 window 77 2 parts 141 / 1 part 130.
+// the roles that a backward's wanted gradients need: {dq, dk2, dv2}, {dk1, dv1}
+static int wanted_roles(const MfmaBwdArgs& a) { return std::max(1, (a.dq || a.dk2 || a.dv2 ? 1 : 0) + (a.dk1 || a.dv1 ? 1 : 0)); }
+
+// Workgroups per query tile under a window at D = 64, by the time that the grid of both roles takes with s of them: one
+// workgroup fills a CU, and all tiles but those at the start of the sequence cost the same, so it takes the larger of
+// whole rounds of the full tiles' parts over the CUs and of the even share plus a third of a part of tail.  Work in 32-key steps
+// of eight rows; a part's own prologue, dQ's shares and tail are worth about nine of them.  Training steps, the parts it
+// chooses (the best otherwise): B=2 H=4 T=2048 window 512 3 parts 5.52 ms (1 to 12: 6.01 5.64 5.52 5.57 5.59 5.65 5.70), B=1 H=8
+// T=700 window 100 3 parts 259 us, B=2 H=8 T=2048 window 100 1 part 1.23 ms, B=1 H=4 T=1500 window 300 3 parts 934 us, B=4 H=8
+// T=1024 window 200 1 part 2.52 ms, B=1 H=2 T=1999 window 77 1 part 167 us, all the best; B=1 H=16 T=1024 window 400 3 parts 3.10 ms
+// (1 part 3.05).
 static int windowed_splits(const MfmaBwdArgs& a) {
     constexpr float kPart = 9.f;
     constexpr int kCus = 256;
-    const int nqt = (a.T + 31) / 32, rows = std::min(a.k2_window, a.T - 1) + 32;
+    const int nqt = (a.T + 31) / 32, rows = std::min(a.k2_window, a.T - 1) + 32, roles = wanted_roles(a);
     const int keys = std::min(std::min(a.k1_window, a.T - 1) + 32, a.kk_left + a.kk_right + 8);
     const float w = (float)((rows + 7) / 8) * (float)((keys + 31) / 32);  // of a tile past the start of the sequence
     const int full = a.BH * std::max(nqt - rows / 32, 0), light = a.BH * std::min(nqt, rows / 32);
@@ -775,23 +778,23 @@ static int windowed_splits(const MfmaBwdArgs& a) {
     float least = 3.0e38f;
     for (int s : {1, 2, 3, 4, 6, 8, 12, 16}) {
         const float part = kPart + w / (float)s;
-        const float t = std::max((float)((full * s + kCus - 1) / kCus) * part,
-                                 ((float)(full + light) * (float)s * kPart + total) / kCus + 0.5f * part);
+        const float t = std::max((float)((roles * full * s + kCus - 1) / kCus) * part,
+                                 (float)roles * ((float)(full + light) * (float)s * kPart + total) / kCus + 0.3f * part);
         if (t < least) least = t, best = s;
     }
     return best;
 }
 
 // Workgroups per query tile under a full causal mask at D = 64, for grids of less than 1024 tiles.  The work of a tile grows
-// with the square of its position and the heaviest parts start first, so a launch takes the longer of the even share of all
-// parts over the CUs and of its longest part (which starts late by what the parts before it differ: 1.15).  Work in 32-key
-// steps of eight rows; a part's own prologue, dQ's shares and tail are worth about seven of them.  The model is that of one role's
-// workgroups in a launch of their own.  In the grid that holds both roles its choice (backward, chosen / best): B=2 H=4 T=256 8 parts 109 us
-// / 6 parts 104, B=4 H=8 T=128 4 parts 107 / 2 parts 98, B=4 H=8 T=256 3 parts 316 / 2 parts 306, B=2 H=8 T=300 4 parts 266 / 3 parts
-// 262, B=1 H=4 T=512 12 parts 253 / 8 parts 250, B=1 H=2 T=128 16 parts 41 / 12 parts 39; B=1 H=8 T=1000 and B=2 H=4 T=600 within 1 % of
-// the best.  D = 32 and 128 measure within 1 % of their best at 1024 workgroups.
+// with the square of its position and the heaviest parts start first, so the grid of both roles takes the longer of the even
+// share of all parts over the CUs and of its longest part (which starts late by what the parts before it differ, and shares
+// the chip with the other role's: 1.5).  Work in 32-key steps of eight rows; a part's own prologue, dQ's shares and tail are
+// worth about twelve of them.  Training steps, the parts it chooses (the best otherwise): B=2 H=4 T=256 6 parts 141 us (2 to 16: 190 151
+// 144 141 145 152 154), B=4 H=8 T=128 2 parts 130 us, T=256 2 parts 402, B=2 H=8 T=300 3 parts 337, B=1 H=2 T=128 100 us, all the
+// best; B=1 H=4 T=512 8 parts 330 (12 parts 329), B=1 H=8 T=1000 3.49 ms (6 parts 3.48), B=1 H=16 T=700 2.47 ms (3 parts 2.45).
+// D = 32 and 128 measure within 1 % of their best at 1024 workgroups.
 static int causal_splits(const MfmaBwdArgs& a) {
-    constexpr float kPart = 7.f;
+    constexpr float kPart = 12.f;
     constexpr int kCus = 256;
     const int nqt = (a.T + 31) / 32;
     const float w = (float)((a.T + 7) / 8) * (float)nqt;  // the last tile's
@@ -799,7 +802,7 @@ static int causal_splits(const MfmaBwdArgs& a) {
     int best = 1;
     float least = 3.0e38f;
     for (int s : {1, 2, 3, 4, 6, 8, 12, 16}) {
-        const float t = std::max(1.15f * (kPart + w / (float)s), (total + (float)(a.BH * nqt * s) * kPart) / kCus);
+        const float t = std::max(1.5f * (kPart + w / (float)s), (float)wanted_roles(a) * (total + (float)(a.BH * nqt * s) * kPart) / kCus);
         if (t < least) least = t, best = s;
     }
     return best;
