@@ -58,15 +58,15 @@ __device__ __forceinline__ float wave_max(float v) {
 // One 64-row block of a row-major [T][D] tensor, transposed into dst[d][Tp] (rows past T become zeros), through
 // an LDS tile so that both the reads (8 consecutive d of a row) and the writes (8 consecutive rows of a column)
 // are whole 16-byte pieces: an element-wise transposed copy touches one cache line per lane and is bound by the
-// address traffic of the vector memory path.  256 threads; `tile` holds 64 x (D + 2) elements; the caller
+// address traffic of the vector memory path.  NT threads; `tile` holds 64 x (D + 2) elements; the caller
 // synchronises the workgroup between transpose_load and transpose_store (and again before reusing the tile).
 // SILU applies x -> SiLU(x) on the way and, with `rows` non-null, also stores the result row-major.
-template <typename E, bool SILU>
+template <typename E, bool SILU, int NT = 256>
 __device__ __forceinline__ void transpose_load(const E* __restrict__ src, E* __restrict__ rows, E* tile, int j0, int T,
                                                int D, unsigned src_stride = 0 /* elements between rows of src; 0: D */) {
     typedef __attribute__((ext_vector_type(8))) E e8;
     const int ld = D + 2, cpr = D / 8;
-    for (int idx = threadIdx.x; idx < 64 * cpr; idx += 256) {
+    for (int idx = threadIdx.x; idx < 64 * cpr; idx += NT) {
         const int jj = idx / cpr, c = idx % cpr, j = j0 + jj;
         e8 x;
 #pragma unroll
@@ -83,11 +83,11 @@ __device__ __forceinline__ void transpose_load(const E* __restrict__ src, E* __r
         for (int e = 0; e < 8; ++e) tile[jj * ld + c * 8 + e] = x[e];
     }
 }
-template <typename E>
+template <typename E, int NT = 256>
 __device__ __forceinline__ void transpose_store(E* __restrict__ dst, const E* tile, int j0, int Tp, int D) {
     typedef __attribute__((ext_vector_type(8))) E e8;
     const int ld = D + 2;
-    for (int idx = threadIdx.x; idx < D * 8; idx += 256) {
+    for (int idx = threadIdx.x; idx < D * 8; idx += NT) {
         const int d = idx >> 3, cj = idx & 7;
         e8 y;
 #pragma unroll
@@ -170,15 +170,15 @@ __device__ __forceinline__ void shared_add(void* acc, size_t idx, float v, float
     }
 }
 // block-wide maximum of the finite |x| bit patterns of `count` 16-byte pieces (E8 = 8 elements of E, or 4 floats)
-// starting at src; every thread of the 256-thread block returns the same value; `red` = 4 words of LDS
+// starting at src; every thread of the NT-thread block returns the same value; `red` = NT / 64 words of LDS
 // (row_pieces > 0: the pieces form rows of row_pieces pieces that lie `pitch` elements apart)
-template <typename E>
+template <typename E, int NT = 256>
 __device__ __forceinline__ unsigned block_absmax_bits(const E* __restrict__ src, size_t count, unsigned* red,
                                                       unsigned row_pieces = 0, unsigned pitch = 0) {
     constexpr int PER = 16 / sizeof(E);
     typedef __attribute__((ext_vector_type(PER))) E ev;
     unsigned m = 0;
-    for (size_t i = threadIdx.x; i < count; i += 256) {
+    for (size_t i = threadIdx.x; i < count; i += NT) {
         const size_t at = row_pieces ? (i / row_pieces) * pitch + (i % row_pieces) * PER : i * PER;
         const ev x = *reinterpret_cast<const ev*>(src + at);
 #pragma unroll
@@ -189,7 +189,10 @@ __device__ __forceinline__ unsigned block_absmax_bits(const E* __restrict__ src,
     __syncthreads();
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
     __syncthreads();
-    return max(max(red[0], red[1]), max(red[2], red[3]));
+    unsigned all = red[0];
+#pragma unroll
+    for (int w = 1; w < NT / 64; ++w) all = max(all, red[w]);
+    return all;
 }
 
 // Window parameters of the triple-dot causal mask, expressed for a "staged"

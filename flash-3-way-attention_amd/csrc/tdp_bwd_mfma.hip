@@ -592,81 +592,80 @@ __global__ __launch_bounds__(512) void tdp_bwd_rows_kernel(BothRoles<E> a) {
 // 64 rows was a chain of four round trips, 13 us at B=2 H=4 T=256, where few workgroups share the chip.
 constexpr int kPrepJobs = 4;
 template <typename E>
-__global__ __launch_bounds__(256) void bwd_prep_kernel(const E* __restrict__ v1, const E* __restrict__ k1,
-                                                       const E* __restrict__ k2, const E* __restrict__ v2,
-                                                       const E* __restrict__ o, const E* __restrict__ d_o,
-                                                       E* __restrict__ u, E* __restrict__ ut, E* __restrict__ k1t,
-                                                       E* __restrict__ k2t, E* __restrict__ v2t,
-                                                       float* __restrict__ delta, float* __restrict__ zero_a,
-                                                       float* __restrict__ zero_b, float* __restrict__ zero_c,
-                                                       float* __restrict__ zero_d, float* __restrict__ zero_e, int T,
-                                                       int Tp, int D, int zero_width,
-                                                       unsigned* __restrict__ scale_parts,
-                                                       unsigned* __restrict__ poison,
-                                                       const E* __restrict__ o_res, int H, TensorAt at_v1,
-                                                       TensorAt at_k1, TensorAt at_k2, TensorAt at_v2, TensorAt at_do) {
+struct BwdPrep {
     // v1, k1, k2, v2 and d_o lie where the caller has them (H heads per batch entry, strides in elements; a dense
     // call passes H = 1 and dense strides); everything else is dense
-    const int bh = blockIdx.y, j0 = blockIdx.x * 64;
+    const E *v1, *k1, *k2, *v2, *o, *d_o;
+    E *u, *ut, *k1t, *k2t, *v2t;
+    float *delta, *zero_a, *zero_b, *zero_c, *zero_d, *zero_e;
+    int T, Tp, BH, D, zero_width;
+    unsigned *scale_parts, *poison;
+    const E* o_res;
+    int H;
+    TensorAt at_v1, at_k1, at_k2, at_v2, at_do;
+};
+constexpr int kPrepTile = 64 * (128 + 2);  // elements of a transposed tile
+// one kind of work for 64 rows (block bx of a slice's nbx); `lds`: two tiles
+template <typename E, int NT>
+__device__ __forceinline__ void bwd_prep_block(const BwdPrep<E>& p, int bx, int bh, int job, int nbx, E* lds) {
+    const int j0 = bx * 64, T = p.T, Tp = p.Tp, D = p.D;
     const size_t base = (size_t)bh * T * D, tbase = (size_t)bh * D * Tp;
-    const int b_ = bh / H, h_ = bh % H;
+    const int b_ = bh / p.H, h_ = bh % p.H;
     auto slice = [&](const E* t, const TensorAt& at) { return t + (size_t)b_ * at.sb + (size_t)h_ * at.sh; };
-    v1 = slice(v1, at_v1); k1 = slice(k1, at_k1); k2 = slice(k2, at_k2); v2 = slice(v2, at_v2); d_o = slice(d_o, at_do);
-    const int job = blockIdx.z;
-    if (job < 2) {  // two tiles at a time (static LDS stays under 64 KB at D = 128): their loads are in flight together
-        constexpr int kTile = 64 * (128 + 2);
-        __shared__ E tiles[2 * kTile];
+    if (job < 2) {  // two tiles at a time: their loads are in flight together
         if (job == 0) {
-            transpose_load<E, true>(v1, u + base, tiles, j0, T, D, at_v1.st);
-            transpose_load<E, false>(k1, nullptr, tiles + kTile, j0, T, D, at_k1.st);
+            transpose_load<E, true, NT>(slice(p.v1, p.at_v1), p.u + base, lds, j0, T, D, p.at_v1.st);
+            transpose_load<E, false, NT>(slice(p.k1, p.at_k1), nullptr, lds + kPrepTile, j0, T, D, p.at_k1.st);
         } else {
-            transpose_load<E, false>(k2, nullptr, tiles, j0, T, D, at_k2.st);
-            transpose_load<E, false>(v2, nullptr, tiles + kTile, j0, T, D, at_v2.st);
+            transpose_load<E, false, NT>(slice(p.k2, p.at_k2), nullptr, lds, j0, T, D, p.at_k2.st);
+            transpose_load<E, false, NT>(slice(p.v2, p.at_v2), nullptr, lds + kPrepTile, j0, T, D, p.at_v2.st);
         }
         __syncthreads();
-        transpose_store<E>((job == 0 ? ut : k2t) + tbase, tiles, j0, Tp, D);
-        transpose_store<E>((job == 0 ? k1t : v2t) + tbase, tiles + kTile, j0, Tp, D);
+        transpose_store<E, NT>((job == 0 ? p.ut : p.k2t) + tbase, lds, j0, Tp, D);
+        transpose_store<E, NT>((job == 0 ? p.k1t : p.v2t) + tbase, lds + kPrepTile, j0, Tp, D);
         return;
     }
     if (job == 2) {  // the accumulators: zero_width 4-byte words per row (D floats, or D 64-bit fixed-point sums)
-        if (scale_parts && threadIdx.x < 64 && j0 + threadIdx.x < T) poison[(size_t)bh * T + j0 + threadIdx.x] = 0;
+        const int zero_width = p.zero_width;
+        if (p.scale_parts && threadIdx.x < 64 && j0 + threadIdx.x < T) p.poison[(size_t)bh * T + j0 + threadIdx.x] = 0;
         const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
-        for (int idx = threadIdx.x; idx < 64 * (zero_width / 4); idx += 256) {
+        for (int idx = threadIdx.x; idx < 64 * (zero_width / 4); idx += NT) {
             const int j = j0 + idx / (zero_width / 4);
             if (j < T) {
                 const size_t off = ((size_t)bh * T + j) * zero_width + (idx % (zero_width / 4)) * 4;
-                *reinterpret_cast<float4*>(zero_a + off) = z4;
-                *reinterpret_cast<float4*>(zero_b + off) = z4;
-                *reinterpret_cast<float4*>(zero_c + off) = z4;
-                *reinterpret_cast<float4*>(zero_d + off) = z4;
-                if (zero_e) *reinterpret_cast<float4*>(zero_e + off) = z4;
+                *reinterpret_cast<float4*>(p.zero_a + off) = z4;
+                *reinterpret_cast<float4*>(p.zero_b + off) = z4;
+                *reinterpret_cast<float4*>(p.zero_c + off) = z4;
+                *reinterpret_cast<float4*>(p.zero_d + off) = z4;
+                if (p.zero_e) *reinterpret_cast<float4*>(p.zero_e + off) = z4;
             }
         }
         return;
     }
-    if (scale_parts) {
+    const E* __restrict__ d_o = slice(p.d_o, p.at_do);
+    if (p.scale_parts) {
         // the first blocks of a slice leave the partial maxima of |dO| that fix the slice's scale (part s = 64-row blocks s,
         // s + 8, ...)
-        __shared__ unsigned red[4];
-        for (int part = blockIdx.x; part < kScaleParts; part += gridDim.x) {
+        unsigned* red = reinterpret_cast<unsigned*>(lds);
+        for (int part = bx; part < kScaleParts; part += nbx) {
             unsigned m = 0;
             for (int r0 = part * 64; r0 < T; r0 += kScaleParts * 64)
-                m = max(m, block_absmax_bits<E>(d_o + (size_t)r0 * at_do.st, (size_t)min(64, T - r0) * D / 8, red, D / 8, at_do.st));
-            if (threadIdx.x == 0) scale_parts[bh * kScaleParts + part] = m;
+                m = max(m, block_absmax_bits<E, NT>(d_o + (size_t)r0 * p.at_do.st, (size_t)min(64, T - r0) * D / 8, red, D / 8, p.at_do.st));
+            if (threadIdx.x == 0) p.scale_parts[bh * kScaleParts + part] = m;
         }
     }
     // Delta[j] = dO[j] . O[j]: the D / 8 lanes that hold a row's 16-byte pieces sit next to each other
     typedef __attribute__((ext_vector_type(8))) E e8;
     const int cpr = D / 8;
-    for (int idx = threadIdx.x; idx < 64 * cpr; idx += 256) {
+    for (int idx = threadIdx.x; idx < 64 * cpr; idx += NT) {
         const int j = j0 + idx / cpr, c = idx % cpr;
         float part = 0.f;
         if (j < T) {
             const size_t off = base + (size_t)j * D + c * 8;
-            const e8 a = *reinterpret_cast<const e8*>(o + off);
-            const e8 b = *reinterpret_cast<const e8*>(d_o + (size_t)j * at_do.st + c * 8);
-            if (o_res) {  // split operands: the output to 16 mantissa bits (rounded value + rounding residual)
-                const e8 r = *reinterpret_cast<const e8*>(o_res + off);
+            const e8 a = *reinterpret_cast<const e8*>(p.o + off);
+            const e8 b = *reinterpret_cast<const e8*>(d_o + (size_t)j * p.at_do.st + c * 8);
+            if (p.o_res) {  // split operands: the output to 16 mantissa bits (rounded value + rounding residual)
+                const e8 r = *reinterpret_cast<const e8*>(p.o_res + off);
 #pragma unroll
                 for (int e = 0; e < 8; ++e) part += ((float)a[e] + (float)r[e]) * (float)b[e];
             } else {
@@ -675,8 +674,27 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(const E* __restrict__ v1,
             }
         }
         for (int off = cpr >> 1; off > 0; off >>= 1) part += __shfl_xor(part, off, 64);
-        if (c == 0 && j < T) delta[(size_t)bh * T + j] = part;
+        if (c == 0 && j < T) p.delta[(size_t)bh * T + j] = part;
     }
+}
+template <typename E>
+__global__ __launch_bounds__(256) void bwd_prep_kernel(BwdPrep<E> p) {
+    __shared__ __align__(16) E tiles[2 * kPrepTile];
+    bwd_prep_block<E, 256>(p, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, tiles);
+}
+// The same, and the fp32 statistics of query tile 0 (tdp_f32_tiles.hpp) in the same grid: neither waits for the other (the tile's
+// workgroups form SiLU(V1) as they stage it), and as a launch of their own they were a few latency-bound workgroups in 12 us
+// between this one and the main kernel.  They come first; the others follow as x, job, slice.
+template <typename E, int D>
+__global__ __launch_bounds__(512, 2) void bwd_prep_stats_kernel(BwdPrep<E> p, F32StatsParams<E> s, int stats_x, int nbx) {
+    const int stats_blocks = stats_x * s.split_rounds;
+    if ((int)blockIdx.x < stats_blocks) {
+        f32_stats_block<E, D, kF32Waves, true>(s, blockIdx.x % stats_x, blockIdx.x / stats_x);
+        return;
+    }
+    extern __shared__ __align__(16) float smem_f[];
+    const int idx = blockIdx.x - stats_blocks;
+    bwd_prep_block<E, 512>(p, idx % nbx, idx / (nbx * kPrepJobs), idx / nbx % kPrepJobs, nbx, reinterpret_cast<E*>(smem_f));
 }
 
 // fp32 accumulators -> output tensors; dV1 = dU * SiLU'(V1)
@@ -846,16 +864,19 @@ static hipError_t launch_bwd(const MfmaBwdArgs& a, hipStream_t st) {
     if (knobs().bwd_splits > 0) splits = std::min(16, knobs().bwd_splits);  // tuning sweeps
     float* dqacc = splits > 1 ? (float*)(ws + l.dqacc) : nullptr;
 
-    hipLaunchKernelGGL(bwd_prep_kernel<E>, dim3(Tp / 64, a.BH, kPrepJobs), dim3(256), 0, st, (const E*)a.v1, (const E*)a.k1,
-                       (const E*)a.k2, (const E*)a.v2, (const E*)a.o, (const E*)a.d_o, (E*)(ws + l.u),
-                       (E*)(ws + l.ut), (E*)(ws + l.k1t), (E*)(ws + l.k2t), (E*)(ws + l.v2t),
-                       (float*)(ws + l.delta), dk1acc, duacc, dk2acc, dv2acc, dqacc, a.T, Tp, D,
-                       a.deterministic ? 2 * D : D, a.deterministic ? (unsigned*)(ws + l.scale_parts) : nullptr,
-                       (unsigned*)(ws + l.poison),
-                       a.split ? (const E*)a.o + (size_t)a.BH * a.T * D : (const E*)nullptr, SV ? a.H : 1,
-                       SV ? a.at_v1 : dense_at(1, a.T, D), SV ? a.at_k1 : dense_at(1, a.T, D),
-                       SV ? a.at_k2 : dense_at(1, a.T, D), SV ? a.at_v2 : dense_at(1, a.T, D),
-                       SV ? a.at_do : dense_at(1, a.T, D));
+    BwdPrep<E> prep{};
+    prep.v1 = (const E*)a.v1; prep.k1 = (const E*)a.k1; prep.k2 = (const E*)a.k2; prep.v2 = (const E*)a.v2;
+    prep.o = (const E*)a.o; prep.d_o = (const E*)a.d_o;
+    prep.u = (E*)(ws + l.u); prep.ut = (E*)(ws + l.ut); prep.k1t = (E*)(ws + l.k1t); prep.k2t = (E*)(ws + l.k2t); prep.v2t = (E*)(ws + l.v2t);
+    prep.delta = (float*)(ws + l.delta);
+    prep.zero_a = dk1acc; prep.zero_b = duacc; prep.zero_c = dk2acc; prep.zero_d = dv2acc; prep.zero_e = dqacc;
+    prep.T = a.T; prep.Tp = Tp; prep.BH = a.BH; prep.D = D; prep.zero_width = a.deterministic ? 2 * D : D;
+    prep.scale_parts = a.deterministic ? (unsigned*)(ws + l.scale_parts) : nullptr; prep.poison = (unsigned*)(ws + l.poison);
+    prep.o_res = a.split ? (const E*)a.o + (size_t)a.BH * a.T * D : nullptr;
+    prep.H = SV ? a.H : 1;
+    const TensorAt dense = dense_at(1, a.T, D);
+    prep.at_v1 = SV ? a.at_v1 : dense; prep.at_k1 = SV ? a.at_k1 : dense; prep.at_k2 = SV ? a.at_k2 : dense;
+    prep.at_v2 = SV ? a.at_v2 : dense; prep.at_do = SV ? a.at_do : dense;
 
     BwdParams<E> p;
     p.H = SV ? a.H : 1;
@@ -950,6 +971,7 @@ static hipError_t launch_bwd(const MfmaBwdArgs& a, hipStream_t st) {
     // tile 1: the grid simply has one tile less, and the heaviest-first numbering never reaches tile 0.
     // (all_in_f32: every tile does)
     const bool first_in_f32 = a.causal != 0;
+    auto launch_prep = [&] { hipLaunchKernelGGL(bwd_prep_kernel<E>, dim3(Tp / 64, a.BH, kPrepJobs), dim3(256), 0, st, prep); };
     // tile 0's backward workgroups are part of the rows kernel's grid where that is the D = 64 one (BothRoles);
     // otherwise they are a launch of their own
     bool fuse_tile0 = false;
@@ -971,12 +993,23 @@ static hipError_t launch_bwd(const MfmaBwdArgs& a, hipStream_t st) {
         f.deal_out = deal_f32;
         if constexpr (D == 64) {
             if (plain64 && !all_in_f32 && p.nqt > 1 && (want_q || want_k2 || want_k1)) {
-                if (hipError_t e = tile0_prepare<E, 64>(f, st, t0_r0, t0_r1, t0_roles, t0_rounds); e != hipSuccess) return e;
+                t0_rounds = tile0_rounds(f);
+                auto kern = bwd_prep_stats_kernel<E, 64>;
+                constexpr size_t prep_smem = std::max(f32_stats_smem<64, kF32Waves>(), 2 * kPrepTile * sizeof(E));
+                if (hipError_t e = ensure_dynamic_smem(reinterpret_cast<const void*>(kern), prep_smem); e != hipSuccess) return e;
+                const int stats_x = 8 * xcd_slots(a.BH, 1);
+                hipLaunchKernelGGL(kern, dim3(stats_x * t0_rounds + Tp / 64 * a.BH * kPrepJobs), dim3(512), prep_smem, st, prep,
+                                   tile0_stats<E, 64>(f, t0_rounds, a.v1, prep.at_v1), stats_x, Tp / 64);
+                tile0_backward<E, 64>(f, t0_r0, t0_r1, t0_roles);
                 fuse_tile0 = true;
             }
         }
-        if (!fuse_tile0)
+        if (!fuse_tile0) {
+            launch_prep();
             if (hipError_t e = f32_mfma_tdp_bwd_first_tile(f, st); e != hipSuccess) return e;
+        }
+    } else {
+        launch_prep();
     }
     const int tiles_here = all_in_f32 ? 0 : p.nqt - (first_in_f32 ? 1 : 0);
     p.grid_tiles = std::max(tiles_here, 1);  // the tiles the grid covers: nqt - 1 .. nqt - grid_tiles

@@ -473,8 +473,13 @@ template <typename E, int D>
 static hipError_t launch_tile0_split(const FirstTileArgs& a, hipStream_t st) {
     constexpr int DOUT = D > 64 ? 64 : D;
     F32BwdParams<E> r0, r1;
-    int roles, rounds;
-    if (hipError_t e = tile0_prepare<E, D>(a, st, r0, r1, roles, rounds); e != hipSuccess) return e;
+    int roles;
+    const int rounds = tile0_rounds(a);
+    auto stats = tdp_f32_stats_kernel<E, D, kF32Waves>;
+    constexpr size_t stats_smem = f32_stats_smem<D, kF32Waves>();
+    if (hipError_t e = ensure_dynamic_smem(reinterpret_cast<const void*>(stats), stats_smem); e != hipSuccess) return e;
+    hipLaunchKernelGGL(stats, dim3(8 * xcd_slots(a.BH, 1), rounds), dim3(512), stats_smem, st, tile0_stats<E, D>(a, rounds, nullptr, TensorAt{}));
+    tile0_backward<E, D>(a, r0, r1, roles);
     auto kern = tdp_f32_tile0_kernel<E, D, DOUT>;
     constexpr size_t smem = f32_bwd_smem<D>();
     if (hipError_t e = ensure_dynamic_smem(reinterpret_cast<const void*>(kern), smem); e != hipSuccess) return e;

@@ -160,7 +160,8 @@ __device__ __forceinline__ void stage_fetch_e(StageE<E, D, NW>& r, const E* __re
         }
     }
 }
-template <typename E, int D, int NW>
+// SILU: the second tensor is V1; its SiLU, rounded to E, is stored
+template <typename E, int D, int NW, bool SILU = false>
 __device__ __forceinline__ void stage_store_e(const StageE<E, D, NW>& r, float* sk, float* sv) {
     using S = StageE<E, D, NW>;
     constexpr int kVec = D / S::VE, LD = D + 4;  // f32_pitch<D>()
@@ -178,6 +179,12 @@ __device__ __forceinline__ void stage_store_e(const StageE<E, D, NW>& r, float* 
             for (int k = 0; k < S::VE; k += 4) {
                 typedef __attribute__((ext_vector_type(4))) float f4;
                 f4 v = {(float)e[k], (float)e[k + 1], (float)e[k + 2], (float)e[k + 3]};
+                if constexpr (SILU) {
+                    if (!first) {
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) v[j] = (float)(E)silu_f(v[j]);
+                    }
+                }
                 *reinterpret_cast<f4*>(p + k) = v;
             }
         }
@@ -264,8 +271,9 @@ __device__ __forceinline__ bool open_round(Walk& w, const TdpMask& mask, int m, 
 // are as wide as the layout allows: the k-slots of four consecutive MFMAs are four consecutive d (16 bytes of a row), and
 // output row r of value tile dt is column d = DT r + dt, so that the operands of the DT value tiles are DT consecutive columns.
 // Stages and row operands are fetched one step ahead across the rounds' ends, one barrier per step.
-template <typename E, int D, int NW>
-__global__ __launch_bounds__(64 * NW, 2) void tdp_f32_stats_kernel(F32StatsParams<E> p) {
+// SILU: p.va is V1 (a launch that does not wait for U)
+template <typename E, int D, int NW, bool SILU>
+__device__ __forceinline__ void f32_stats_block(const F32StatsParams<E>& p, int block, int round) {
     constexpr int DT = D / 32, LD = f32_pitch<D>(), NT = 64 * NW;
     constexpr bool HOLD = D <= 64;
     using vDT = typename VecF<DT>::type;
@@ -280,7 +288,7 @@ __global__ __launch_bounds__(64 * NW, 2) void tdp_f32_stats_kernel(F32StatsParam
     float* sO = sK;                     // [NW][D][33] end of kernel: the waves' outputs (alias everything from the stages on)
 
     int bh, order;
-    if (!xcd_tile(p.BH, p.nqt, blockIdx.x >> 3, blockIdx.x & 7, bh, order)) return;
+    if (!xcd_tile(p.BH, p.nqt, block >> 3, block & 7, bh, order)) return;
     const int qt = p.nqt - 1 - order;
 
     const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, g = lane >> 5;
@@ -300,9 +308,9 @@ __global__ __launch_bounds__(64 * NW, 2) void tdp_f32_stats_kernel(F32StatsParam
     const Range rows = row_range(mask, q0, q1, T);
     int m_lo = rows.lo / NW, m_hi = rows.hi / NW;  // rounds of NW rows
     if (p.split_rounds) {
-        m_lo = max(m_lo, (int)blockIdx.y);  // this workgroup's round only (none at all if it is out of range)
-        m_hi = min(m_hi, (int)blockIdx.y);
-        if (blockIdx.y == 0)
+        m_lo = max(m_lo, round);  // this workgroup's round only (none at all if it is out of range)
+        m_hi = min(m_hi, round);
+        if (round == 0)
             for (int idx = tid; idx < p.zero_words; idx += NT) p.zero_ptr[(size_t)bh * p.zero_words + idx] = 0u;
     }
 
@@ -349,7 +357,7 @@ __global__ __launch_bounds__(64 * NW, 2) void tdp_f32_stats_kernel(F32StatsParam
     }
     if (have) {
         store_rows(0);
-        stage_store_e<E, D, NW>(regs, sK, sV);
+        stage_store_e<E, D, NW, SILU>(regs, sK, sV);
     }
     __syncthreads();
 
@@ -474,7 +482,7 @@ __global__ __launch_bounds__(64 * NW, 2) void tdp_f32_stats_kernel(F32StatsParam
                 par ^= 1;
                 store_rows(par);
             }
-            stage_store_e<E, D, NW>(regs, sK + buf * 32 * LD, sV + buf * 32 * LD);
+            stage_store_e<E, D, NW, SILU>(regs, sK + buf * 32 * LD, sV + buf * 32 * LD);
             __syncthreads();
         }
         w = nw;
@@ -523,7 +531,7 @@ __global__ __launch_bounds__(64 * NW, 2) void tdp_f32_stats_kernel(F32StatsParam
 #pragma unroll
         for (int k = 0; k < 2 * NW; ++k) dsum += red[k * 32 + n];
         if (p.split_rounds) {
-            float* part = p.delta + (((size_t)bh * 32 + n) * p.split_rounds + blockIdx.y) * 3;
+            float* part = p.delta + (((size_t)bh * 32 + n) * p.split_rounds + round) * 3;
             part[0] = M; part[1] = L; part[2] = dsum;
         } else {
             p.delta[(size_t)bh * T + q] = dsum / L;
@@ -531,6 +539,10 @@ __global__ __launch_bounds__(64 * NW, 2) void tdp_f32_stats_kernel(F32StatsParam
     }
     if (p.split_rounds) return;
     if (wave == 0 && g == 0 && q < T) p.lse[(size_t)bh * T + q] = (M + fast_log2(L)) * kLn2;
+}
+template <typename E, int D, int NW>
+__global__ __launch_bounds__(64 * NW, 2) void tdp_f32_stats_kernel(F32StatsParams<E> p) {
+    f32_stats_block<E, D, NW, false>(p, blockIdx.x, blockIdx.y);
 }
 
 // ------------------------------------------------------------------------------------------ backward
@@ -1005,31 +1017,32 @@ void place_inputs(P& p, const InputsAt& at, bool exchanged) {
     p.at_kb = exchanged ? at.k1 : at.k2; p.at_vb = exchanged ? at.u : at.v2;
 }
 
-// Query tile 0 alone, first half: launches the STATS pass (its rounds dealt out to workgroups) and fills in the
-// parameters of the backward pass over the tile for both roles.  The backward workgroups themselves are
-// (8 xcd_slots(BH, 1)) x (2 rounds) calls of f32_tile0_block: tdp_f32_tile0_kernel, or the tail of another grid.
+// Query tile 0 alone, first half: the parameters of the STATS pass (its rounds dealt out to `rounds` workgroups; V1 is the
+// streamed value tensor where it is given) ...
 template <typename E, int D>
-hipError_t tile0_prepare(const FirstTileArgs& a, hipStream_t st, F32BwdParams<E>& r0, F32BwdParams<E>& r1, int& roles,
-                         int& rounds) {
-    rounds = (std::min(a.T, 32) + kF32Waves - 1) / kF32Waves;
-    const TdpMask natural{a.causal, a.k1_window, a.k2_window, a.kk_left, a.kk_right};
+F32StatsParams<E> tile0_stats(const FirstTileArgs& a, int rounds, const void* v1, const TensorAt& at_v1) {
     const bool own_dq_acc = a.want_q && !a.acc_q;  // dQ of the tile is summed over its rounds in a.dq0_acc
-    {
-        F32StatsParams<E> p{};
-        p.q = (const E*)a.q; p.ka = (const E*)a.k1; p.kb = (const E*)a.k2; p.va = (const E*)a.u; p.vb = (const E*)a.v2;
-        place_inputs(p, inputs_of(a), false);
-        p.lse = nullptr; p.d_o = (const E*)a.d_o; p.delta = a.delta_f32;
-        p.split_rounds = rounds;
-        p.zero_ptr = own_dq_acc ? (unsigned*)a.dq0_acc : nullptr;
-        p.zero_words = own_dq_acc ? 32 * D * (a.scale_parts ? 2 : 1) : 0;
-        p.T = a.T; p.BH = a.BH; p.nqt = 1;
-        p.scale_log2 = a.alpha * kLog2e;
-        p.mask = natural;
-        auto kern = tdp_f32_stats_kernel<E, D, kF32Waves>;
-        constexpr size_t smem = f32_stats_smem<D, kF32Waves>();
-        if (hipError_t e = ensure_dynamic_smem(reinterpret_cast<const void*>(kern), smem); e != hipSuccess) return e;
-        hipLaunchKernelGGL(kern, dim3(8 * xcd_slots(a.BH, 1), rounds), dim3(512), smem, st, p);
-    }
+    F32StatsParams<E> p{};
+    p.q = (const E*)a.q; p.ka = (const E*)a.k1; p.kb = (const E*)a.k2; p.va = (const E*)(v1 ? v1 : a.u); p.vb = (const E*)a.v2;
+    place_inputs(p, inputs_of(a), false);
+    if (v1) p.at_va = at_v1;
+    p.lse = nullptr; p.d_o = (const E*)a.d_o; p.delta = a.delta_f32;
+    p.split_rounds = rounds;
+    p.zero_ptr = own_dq_acc ? (unsigned*)a.dq0_acc : nullptr;
+    p.zero_words = own_dq_acc ? 32 * D * (a.scale_parts ? 2 : 1) : 0;
+    p.T = a.T; p.BH = a.BH; p.nqt = 1;
+    p.scale_log2 = a.alpha * kLog2e;
+    p.mask = TdpMask{a.causal, a.k1_window, a.k2_window, a.kk_left, a.kk_right};
+    return p;
+}
+inline int tile0_rounds(const FirstTileArgs& a) { return (std::min(a.T, 32) + kF32Waves - 1) / kF32Waves; }
+
+// ... and those of the backward pass over the tile for both roles, which is (8 xcd_slots(BH, 1)) x (2 rounds) calls of
+// f32_tile0_block: tdp_f32_tile0_kernel, or the tail of another grid.
+template <typename E, int D>
+void tile0_backward(const FirstTileArgs& a, F32BwdParams<E>& r0, F32BwdParams<E>& r1, int& roles) {
+    const int rounds = tile0_rounds(a);
+    const TdpMask natural{a.causal, a.k1_window, a.k2_window, a.kk_left, a.kk_right};
     r0 = F32BwdParams<E>{};
     r0.q = (const E*)a.q; r0.d_o = (const E*)a.d_o; r0.lse = nullptr; r0.delta = nullptr;
     r0.stats_part = a.delta_f32; r0.split_rounds = rounds; r0.deal = F32Deal{0.f, 1, 1};
@@ -1045,7 +1058,6 @@ hipError_t tile0_prepare(const FirstTileArgs& a, hipStream_t st, F32BwdParams<E>
     r1.acc_k = a.acc_k1; r1.acc_v = a.acc_u; r1.bit_k = kPoisonDK1; r1.bit_v = kPoisonDU;
     r1.mask = TdpMask{natural.causal, natural.wb, natural.wa, natural.rab, natural.lab};
     roles = ((a.want_q || a.want_k2) ? 1 : 0) | (a.want_k1 ? 2 : 0) | (a.want_q ? 4 : 0);
-    return hipGetLastError();
 }
 
 }  // namespace
