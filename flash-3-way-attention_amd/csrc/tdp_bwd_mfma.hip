@@ -991,23 +991,25 @@ static hipError_t launch_bwd(const MfmaBwdArgs& a, hipStream_t st) {
         f.want_q = want_q; f.want_k2 = want_k2; f.want_k1 = want_k1;
         f.tiles = all_in_f32 ? p.nqt : 1;
         f.deal_out = deal_f32;
+        if (f.tiles > 1) {
+            launch_prep();
+        } else {  // (also where every tile takes the fp32 kernel and there is one)
+            t0_rounds = tile0_rounds(f);
+            auto kern = bwd_prep_stats_kernel<E, D>;
+            constexpr size_t prep_smem = std::max(f32_stats_smem<D, kF32Waves>(), 2 * kPrepTile * sizeof(E));
+            if (hipError_t e = ensure_dynamic_smem(reinterpret_cast<const void*>(kern), prep_smem); e != hipSuccess) return e;
+            const int stats_x = 8 * xcd_slots(a.BH, 1);
+            hipLaunchKernelGGL(kern, dim3(stats_x * t0_rounds + Tp / 64 * a.BH * kPrepJobs), dim3(512), prep_smem, st, prep,
+                               tile0_stats<E, D>(f, t0_rounds, a.v1, prep.at_v1), stats_x, Tp / 64);
+        }
         if constexpr (D == 64) {
             if (plain64 && !all_in_f32 && p.nqt > 1 && (want_q || want_k2 || want_k1)) {
-                t0_rounds = tile0_rounds(f);
-                auto kern = bwd_prep_stats_kernel<E, 64>;
-                constexpr size_t prep_smem = std::max(f32_stats_smem<64, kF32Waves>(), 2 * kPrepTile * sizeof(E));
-                if (hipError_t e = ensure_dynamic_smem(reinterpret_cast<const void*>(kern), prep_smem); e != hipSuccess) return e;
-                const int stats_x = 8 * xcd_slots(a.BH, 1);
-                hipLaunchKernelGGL(kern, dim3(stats_x * t0_rounds + Tp / 64 * a.BH * kPrepJobs), dim3(512), prep_smem, st, prep,
-                                   tile0_stats<E, 64>(f, t0_rounds, a.v1, prep.at_v1), stats_x, Tp / 64);
                 tile0_backward<E, 64>(f, t0_r0, t0_r1, t0_roles);
                 fuse_tile0 = true;
             }
         }
-        if (!fuse_tile0) {
-            launch_prep();
+        if (!fuse_tile0)
             if (hipError_t e = f32_mfma_tdp_bwd_first_tile(f, st); e != hipSuccess) return e;
-        }
     } else {
         launch_prep();
     }

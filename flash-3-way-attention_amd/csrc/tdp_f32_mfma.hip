@@ -468,17 +468,13 @@ static hipError_t launch_stats(const FirstTileArgs& a, hipStream_t st) {
     return hipGetLastError();
 }
 
-// Query tile 0 alone: the STATS pass and the backward pass, each with its rounds dealt out to workgroups.
+// Query tile 0 alone, its rounds dealt out to workgroups (the STATS pass runs in the grid of the pass ahead).
 template <typename E, int D>
 static hipError_t launch_tile0_split(const FirstTileArgs& a, hipStream_t st) {
     constexpr int DOUT = D > 64 ? 64 : D;
     F32BwdParams<E> r0, r1;
     int roles;
     const int rounds = tile0_rounds(a);
-    auto stats = tdp_f32_stats_kernel<E, D, kF32Waves>;
-    constexpr size_t stats_smem = f32_stats_smem<D, kF32Waves>();
-    if (hipError_t e = ensure_dynamic_smem(reinterpret_cast<const void*>(stats), stats_smem); e != hipSuccess) return e;
-    hipLaunchKernelGGL(stats, dim3(8 * xcd_slots(a.BH, 1), rounds), dim3(512), stats_smem, st, tile0_stats<E, D>(a, rounds, nullptr, TensorAt{}));
     tile0_backward<E, D>(a, r0, r1, roles);
     auto kern = tdp_f32_tile0_kernel<E, D, DOUT>;
     constexpr size_t smem = f32_bwd_smem<D>();
