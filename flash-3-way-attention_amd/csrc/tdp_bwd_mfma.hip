@@ -994,13 +994,24 @@ static hipError_t launch_bwd(const MfmaBwdArgs& a, hipStream_t st) {
         if (f.tiles > 1) {
             launch_prep();
         } else {  // (also where every tile takes the fp32 kernel and there is one)
+            // One grid for this pass and the tile's statistics up to 2048 workgroups of the first; there it has the chip's two
+            // waves per SIMD that the statistics' registers leave, which on large grids costs more than a launch: B=4 H=16
+            // T=2048 D=32 window 40 (8192 of them) 1298 us as two, 1308 as one; B=4 H=8 T=1024 (2048) the same
             t0_rounds = tile0_rounds(f);
-            auto kern = bwd_prep_stats_kernel<E, D>;
-            constexpr size_t prep_smem = std::max(f32_stats_smem<D, kF32Waves>(), 2 * kPrepTile * sizeof(E));
-            if (hipError_t e = ensure_dynamic_smem(reinterpret_cast<const void*>(kern), prep_smem); e != hipSuccess) return e;
-            const int stats_x = 8 * xcd_slots(a.BH, 1);
-            hipLaunchKernelGGL(kern, dim3(stats_x * t0_rounds + Tp / 64 * a.BH * kPrepJobs), dim3(512), prep_smem, st, prep,
-                               tile0_stats<E, D>(f, t0_rounds, a.v1, prep.at_v1), stats_x, Tp / 64);
+            const int stats_x = 8 * xcd_slots(a.BH, 1), prep_blocks = Tp / 64 * a.BH * kPrepJobs;
+            constexpr size_t stats_smem = f32_stats_smem<D, kF32Waves>();
+            if (prep_blocks <= 2048) {
+                auto kern = bwd_prep_stats_kernel<E, D>;
+                constexpr size_t prep_smem = std::max(stats_smem, 2 * kPrepTile * sizeof(E));
+                if (hipError_t e = ensure_dynamic_smem(reinterpret_cast<const void*>(kern), prep_smem); e != hipSuccess) return e;
+                hipLaunchKernelGGL(kern, dim3(stats_x * t0_rounds + prep_blocks), dim3(512), prep_smem, st, prep,
+                                   tile0_stats<E, D>(f, t0_rounds, a.v1, prep.at_v1), stats_x, Tp / 64);
+            } else {
+                launch_prep();
+                auto kern = tdp_f32_stats_kernel<E, D, kF32Waves>;
+                if (hipError_t e = ensure_dynamic_smem(reinterpret_cast<const void*>(kern), stats_smem); e != hipSuccess) return e;
+                hipLaunchKernelGGL(kern, dim3(stats_x, t0_rounds), dim3(512), stats_smem, st, tile0_stats<E, D>(f, t0_rounds, nullptr, TensorAt{}));
+            }
         }
         if constexpr (D == 64) {
             if (plain64 && !all_in_f32 && p.nqt > 1 && (want_q || want_k2 || want_k1)) {

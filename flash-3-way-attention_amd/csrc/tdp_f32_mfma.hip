@@ -468,7 +468,7 @@ static hipError_t launch_stats(const FirstTileArgs& a, hipStream_t st) {
     return hipGetLastError();
 }
 
-// Query tile 0 alone, its rounds dealt out to workgroups (the STATS pass runs in the grid of the pass ahead).
+// Query tile 0 alone, its rounds dealt out to workgroups (the launcher of the backward has run its STATS pass).
 template <typename E, int D>
 static hipError_t launch_tile0_split(const FirstTileArgs& a, hipStream_t st) {
     constexpr int DOUT = D > 64 ? 64 : D;

@@ -1456,3 +1456,31 @@ def test_backward_d32_shapes_of_a_workgroup(B, H, T, windows, splits, dtype, tun
             util.assert_close(f"out[{b}, {h}] convert={convert}", out.detach()[b, h].float().cpu(), z, rtol=5e-2, atol=2e-2)
             for name, leaf, want in zip(util.NAMES, leaves, grads):
                 util.assert_close(f"{name}[{b}, {h}] convert={convert}", leaf.grad[b, h].float().cpu(), want, rtol=5e-2, atol=2e-2)
+
+
+@pytest.mark.parametrize("B,H,T,D,windows,split", [
+    (1, 3, 1, 32, (None,) * 4, False), (2, 5, 31, 32, (200, 32, 62, 5), False), (1, 2, 32, 64, (None,) * 4, False), (1, 2, 33, 64, (8, 8, 2, 2), False),
+    (1, 3, 65, 128, (None,) * 4, False), (2, 4, 97, 32, (None,) * 4, True), (129, 4, 33, 32, (None,) * 4, False), (65, 8, 40, 128, (None,) * 4, False)])
+def test_statistics_of_the_first_queries(B, H, T, D, windows, split):
+    """The fp32 statistics of query tile 0 ride in the grid of the backward's first pass (up to 2048 workgroups of it; the last two
+    shapes pass that) and stage V1 instead of SiLU(V1): one tile and several, narrow masks that leave every tile to the fp32 kernel, split operands, dense
+    tensors and slices of one projection.  Oracle: the first two and the last slice."""
+    from flash_trittention import flash_trittention
+
+    print(f"case tdp first queries {B, H, T, D} {windows} split={split}", flush=True)
+    inputs = orc.make_inputs(B, H, T, D, torch.bfloat16, seed=T + D)
+    alpha, picks = 1 / math.sqrt(D), sorted({(0, 0), (0, 1), (B - 1, H - 1)})
+    *ins, d_o = (t.cuda() for t in inputs)
+    fused = [t for t in torch.stack(ins, 2).permute(0, 3, 2, 1, 4).contiguous().permute(2, 0, 3, 1, 4)]
+    got = []
+    for tensors in (ins, fused):
+        leaves = [t.detach().requires_grad_(True) for t in tensors]
+        out = flash_trittention(*leaves, softmax_scale=alpha, **dict(zip(("k1_window", "k2_window", "kk_left", "kk_right"), windows)),
+                                causal=True, convert_to_float32=split)
+        got.append(torch.autograd.grad(out, leaves, d_o))
+    for name, a, b in zip(util.NAMES, *got):
+        assert torch.equal(a, b), name
+    for b, h in picks:
+        _, want = util.oracle_tdp([t[b:b + 1, h:h + 1] for t in inputs], alpha, True, windows)[::2]
+        for name, a, w in zip(util.NAMES, got[0], want):
+            util.assert_close(name, a[b:b + 1, h:h + 1].float().cpu(), w, **LOWP)
