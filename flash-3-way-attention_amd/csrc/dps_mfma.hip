@@ -1244,11 +1244,11 @@ bool mfma_dps_supported(int D, int dtype_is_16bit) { return dtype_is_16bit && (D
 size_t mfma_dps_fwd_workspace(int BH, int T, int D) { return layout(BH, T, D, false).total; }
 size_t mfma_dps_bwd_workspace(int BH, int T, int D) { return layout(BH, T, D, true).total; }
 
-// Waves per workgroup (they split the streamed tiles of an owner tile), measured at B*H = 32..64, bf16, forward /
-// backward in us, (waves, paired) = (2, no) | (4, no) | (4, yes):  T=512: 29 / 100 | 32 / 118 | 31 / 115;
-// T=1024: 42 / 137 | 39 / 145 | 38 / 142;  T=2048: 65 / 208 | 54 / 199 | 52 / 197;  T=4096: 112 / 351 | 84 / 309 | 81 / 308.
-// Two waves at D = 128 (fewer partial results to merge); at D = 64 four waves from T = 2048 on, and from T = 1024 in
-// the forward, or when the grid is too small to give every CU four workgroups of two waves.
+// Waves per workgroup of the forward passes and of D = 128 (they split the streamed tiles of an owner tile), measured at
+// B*H = 32..64, bf16, forward in us, (waves, paired) = (2, no) | (4, no) | (4, yes):  T=512: 29 | 32 | 31;  T=1024: 42 | 39 | 38;
+// T=2048: 65 | 54 | 52;  T=4096: 112 | 84 | 81.  Two waves at D = 128 (fewer partial results to merge); at D = 64 four waves from
+// T = 1024 on, or when the grid is too small to give every CU four workgroups of two waves.  `backward`: the inner forward pass
+// that a backward without a kept one repeats, two waves below T = 2048.
 static bool two_waves(const MfmaDpsArgs& a, bool backward) {
     if (a.D == 128) return true;
     if (a.D == 64 && knobs().dps_waves) return knobs().dps_waves == 2;

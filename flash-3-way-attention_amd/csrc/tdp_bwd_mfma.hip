@@ -683,7 +683,7 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(BwdPrep<E> p) {
     bwd_prep_block<E, 256>(p, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, tiles);
 }
 // The same, and the fp32 statistics of query tile 0 (tdp_f32_tiles.hpp) in the same grid: neither waits for the other (the tile's
-// workgroups form SiLU(V1) as they stage it), and as a launch of their own they were a few latency-bound workgroups in 12 us
+// workgroups form SiLU(V1) as they stage it), and as a launch of their own they were a few latency-bound workgroups in 8 to 21 us
 // between this one and the main kernel.  They come first; the others follow as x, job, slice.
 template <typename E, int D>
 __global__ __launch_bounds__(512, 2) void bwd_prep_stats_kernel(BwdPrep<E> p, F32StatsParams<E> s, int stats_x, int nbx) {
@@ -994,13 +994,15 @@ static hipError_t launch_bwd(const MfmaBwdArgs& a, hipStream_t st) {
         if (f.tiles > 1) {
             launch_prep();
         } else {  // (also where every tile takes the fp32 kernel and there is one)
-            // One grid for this pass and the tile's statistics up to 2048 workgroups of the first; there it has the chip's two
-            // waves per SIMD that the statistics' registers leave, which on large grids costs more than a launch: B=4 H=16
-            // T=2048 D=32 window 40 (8192 of them) 1298 us as two, 1308 as one; B=4 H=8 T=1024 (2048) the same
+            // One grid for this pass and the tile's statistics up to 2048 workgroups of the first (D = 128: 1024); there it has
+            // the chip's two waves per SIMD that the statistics' registers leave, which on large grids costs more than a launch.
+            // B=4 H=16 T=2048 D=32 window 40 (8192 of them) 1298 us as two, 1308 as one; the kernels alone, as two (without the gap between
+            // them) -> as one, at 512 / 1024 / 2048 workgroups, T=1024: D=32 20.2 -> 14.3 / 25.7 -> 14.1 / 25.8 -> 20.2 us,
+            // D=64 27.7 -> 17.7 / 29.2 -> 20.6 / 34.5 -> 34.2, D=128 34.3 -> 22.5 / 42.0 -> 28.3 / 65.7 -> 73.2.
             t0_rounds = tile0_rounds(f);
             const int stats_x = 8 * xcd_slots(a.BH, 1), prep_blocks = Tp / 64 * a.BH * kPrepJobs;
             constexpr size_t stats_smem = f32_stats_smem<D, kF32Waves>();
-            if (prep_blocks <= 2048) {
+            if (prep_blocks <= (D == 128 ? 1024 : 2048)) {
                 auto kern = bwd_prep_stats_kernel<E, D>;
                 constexpr size_t prep_smem = std::max(stats_smem, 2 * kPrepTile * sizeof(E));
                 if (hipError_t e = ensure_dynamic_smem(reinterpret_cast<const void*>(kern), prep_smem); e != hipSuccess) return e;
