@@ -1179,8 +1179,8 @@ hipError_t run_bwd(const MfmaDpsArgs& a, hipStream_t st) {
     pp.BH = a.BH; pp.T = a.T; pp.Tp = Tp; pp.H = a.H;
     // R, W, W^T, lse1 of the inner pass: from the forward where the caller kept R and lse1 (W = R * V2 is then formed by the
     // prep launch), else by running that pass again.  Keeping them holds four bytes per element between the two calls and
-    // takes one of the backward's seven products and a launch away; training steps, bf16, run again -> kept: B=4 H=8
-    // T=1024 154 -> 142 us, B=1 H=8 T=8192 k_diff 2048 822 -> 784 us.
+    // takes one of the backward's seven products and a launch away; the backward, bf16, run again -> kept: B=4 H=8
+    // T=1024 92 -> 84 us, B=1 H=8 T=8192 670 -> 569 us.
     const float *r = (const float*)(ws + l.r), *lse1 = (const float*)(ws + l.lse1);
     if (a.kept_r) {
         r = a.kept_r; lse1 = a.kept_lse1; pp.lse1 = lse1;
