@@ -971,6 +971,7 @@ static hipError_t launch_bwd(const MfmaBwdArgs& a, hipStream_t st) {
     // tile 1: the grid simply has one tile less, and the heaviest-first numbering never reaches tile 0.
     // (all_in_f32: every tile does)
     const bool first_in_f32 = a.causal != 0;
+    const int f32_tiles = all_in_f32 ? p.nqt : 1;
     auto launch_prep = [&] { hipLaunchKernelGGL(bwd_prep_kernel<E>, dim3(Tp / 64, a.BH, kPrepJobs), dim3(256), 0, st, prep); };
     // tile 0's backward workgroups are part of the rows kernel's grid where that is the D = 64 one (BothRoles);
     // otherwise they are a launch of their own
@@ -989,7 +990,7 @@ static hipError_t launch_bwd(const MfmaBwdArgs& a, hipStream_t st) {
         f.alpha = a.alpha; f.causal = a.causal;
         f.k1_window = a.k1_window; f.k2_window = a.k2_window; f.kk_left = a.kk_left; f.kk_right = a.kk_right;
         f.want_q = want_q; f.want_k2 = want_k2; f.want_k1 = want_k1;
-        f.tiles = all_in_f32 ? p.nqt : 1;
+        f.tiles = f32_tiles;
         f.deal_out = deal_f32;
         if (f.tiles > 1) {
             launch_prep();
@@ -1069,7 +1070,8 @@ static hipError_t launch_bwd(const MfmaBwdArgs& a, hipStream_t st) {
                        (const float*)duacc, (const float*)dk2acc, (const float*)dv2acc, (const float*)dqacc, a.alpha,
                        (E*)a.dq, (const E*)a.v1, (E*)a.dk1, (E*)a.dv1, (E*)a.dk2, (E*)a.dv2, n,
                        a.deterministic ? 1 : 0,
-                       (first_in_f32 && !all_in_f32 && !dqacc) ? (const float*)(ws + l.dq0acc) : nullptr, a.T, D,
+                       // (one fp32 tile and no accumulator for all of dQ, also where that tile is all there is)
+                       (first_in_f32 && f32_tiles == 1 && !dqacc) ? (const float*)(ws + l.dq0acc) : nullptr, a.T, D,
                        p.scale_parts, p.poison, p.H, SV ? a.at_v1 : dense_at(1, a.T, D));
     return hipGetLastError();
 }

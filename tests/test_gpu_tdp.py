@@ -1484,3 +1484,28 @@ def test_statistics_of_the_first_queries(B, H, T, D, windows, split):
         _, want = util.oracle_tdp([t[b:b + 1, h:h + 1] for t in inputs], alpha, True, windows)[::2]
         for name, a, w in zip(util.NAMES, got[0], want):
             util.assert_close(name, a[b:b + 1, h:h + 1].float().cpu(), w, **LOWP)
+
+
+@pytest.mark.parametrize("B,H,T,D,windows,splits", [
+    (64, 8, 32, 64, (16, 16, None, None), 0), (512, 1, 31, 32, (8, 20, 3, 9), 0), (65, 8, 17, 128, (16, 5, 4, 2), 0), (1, 3, 32, 64, (16, 16, None, None), 1),
+    (2, 2, 1, 32, (0, 0, 0, 0), 1), (1, 3, 29, 128, (7, 8, 30, 30), 1)])
+def test_query_gradient_of_one_tile_under_a_narrow_window(B, H, T, D, windows, splits, tune):
+    """Where a narrow window gives every query tile to the fp32 kernel and there is one, its dQ is summed over rounds, in an accumulator of
+    its own where the backward keeps none for dQ (from 512 slices on, or by TRITT_TUNE_BWD_SPLITS): it has to reach the caller's
+    tensor.  Memory that the gradients may be given holds NaN before the call."""
+    from flash_trittention import _lib, flash_trittention
+
+    print(f"case tdp one tile {B, H, T, D} {windows} splits={splits}", flush=True)
+    tune(_lib.TUNE_BWD_SPLITS, splits)
+    inputs = orc.make_inputs(B, H, T, D, torch.bfloat16, seed=T + D)
+    alpha = 1 / math.sqrt(D)
+    *leaves, d_o = (t.cuda() for t in inputs)
+    leaves = [t.requires_grad_(True) for t in leaves]
+    out = flash_trittention(*leaves, softmax_scale=alpha, **dict(zip(("k1_window", "k2_window", "kk_left", "kk_right"), windows)), causal=True)
+    poison = [torch.full_like(out, math.nan) for _ in range(8)]
+    del poison
+    got = torch.autograd.grad(out, leaves, d_o)
+    for b, h in sorted({(0, 0), (B // 2, H // 2), (B - 1, H - 1)}):
+        want = util.oracle_tdp([t[b:b + 1, h:h + 1] for t in inputs], alpha, True, windows)[2]
+        for name, a, w in zip(util.NAMES, got, want):
+            util.assert_close(f"{name}[{b}, {h}]", a[b:b + 1, h:h + 1].float().cpu(), w, **LOWP)
