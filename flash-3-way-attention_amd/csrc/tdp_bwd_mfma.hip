@@ -16,6 +16,7 @@
 #include <cstring>
 #include <type_traits>
 
+#include "bwd_parts.hpp"
 #include "direct_lds.hpp"
 #include "kernels.hpp"
 #include "mfma.hpp"
@@ -773,59 +774,6 @@ static BwdLayout bwd_layout(int BH, int T, int D, bool fixed_point) {
     return l;
 }
 
-// the roles that a backward's wanted gradients need: {dq, dk2, dv2}, {dk1, dv1}
-static int wanted_roles(const MfmaBwdArgs& a) { return std::max(1, (a.dq || a.dk2 || a.dv2 ? 1 : 0) + (a.dk1 || a.dv1 ? 1 : 0)); }
-
-// Workgroups per query tile under a window at D = 64, by the time that the grid of both roles takes with s of them: one
-// workgroup fills a CU, and all tiles but those at the start of the sequence cost the same, so it takes the larger of
-// whole rounds of the full tiles' parts over the CUs and of the even share plus a third of a part of tail.  Work in 32-key steps
-// of eight rows; a part's own prologue, dQ's shares and tail are worth about nine of them.  Training steps, the parts it
-// chooses (the best otherwise): B=2 H=4 T=2048 window 512 3 parts 5.52 ms (1 to 12: 6.01 5.64 5.52 5.57 5.59 5.65 5.70), B=1 H=8
-// T=700 window 100 3 parts 259 us, B=2 H=8 T=2048 window 100 1 part 1.23 ms, B=1 H=4 T=1500 window 300 3 parts 934 us, B=4 H=8
-// T=1024 window 200 1 part 2.52 ms, B=1 H=2 T=1999 window 77 1 part 167 us, all the best; B=1 H=16 T=1024 window 400 3 parts 3.10 ms
-// (1 part 3.05).
-static int windowed_splits(const MfmaBwdArgs& a) {
-    constexpr float kPart = 9.f;
-    constexpr int kCus = 256;
-    const int nqt = (a.T + 31) / 32, rows = std::min(a.k2_window, a.T - 1) + 32, roles = wanted_roles(a);
-    const int keys = std::min(std::min(a.k1_window, a.T - 1) + 32, a.kk_left + a.kk_right + 8);
-    const float w = (float)((rows + 7) / 8) * (float)((keys + 31) / 32);  // of a tile past the start of the sequence
-    const int full = a.BH * std::max(nqt - rows / 32, 0), light = a.BH * std::min(nqt, rows / 32);
-    const float total = ((float)full + 0.36f * (float)light) * w;
-    int best = 1;
-    float least = 3.0e38f;
-    for (int s : {1, 2, 3, 4, 6, 8, 12, 16}) {
-        const float part = kPart + w / (float)s;
-        const float t = std::max((float)((roles * full * s + kCus - 1) / kCus) * part,
-                                 (float)roles * ((float)(full + light) * (float)s * kPart + total) / kCus + 0.3f * part);
-        if (t < least) least = t, best = s;
-    }
-    return best;
-}
-
-// Workgroups per query tile under a full causal mask at D = 64, for grids of less than 1024 tiles.  The work of a tile grows
-// with the square of its position and the heaviest parts start first, so the grid of both roles takes the longer of the even
-// share of all parts over the CUs and of its longest part (which starts late by what the parts before it differ, and shares
-// the chip with the other role's: 1.5).  Work in 32-key steps of eight rows; a part's own prologue, dQ's shares and tail are
-// worth about twelve of them.  Training steps, the parts it chooses (the best otherwise): B=2 H=4 T=256 6 parts 141 us (2 to 16: 190 151
-// 144 141 145 152 154), B=4 H=8 T=128 2 parts 130 us, T=256 2 parts 402, B=2 H=8 T=300 3 parts 337, B=1 H=2 T=128 100 us, all the
-// best; B=1 H=4 T=512 8 parts 330 (12 parts 329), B=1 H=8 T=1000 3.49 ms (6 parts 3.48), B=1 H=16 T=700 2.47 ms (3 parts 2.45).
-// D = 32 and 128 measure within 1 % of their best at 1024 workgroups.
-static int causal_splits(const MfmaBwdArgs& a) {
-    constexpr float kPart = 12.f;
-    constexpr int kCus = 256;
-    const int nqt = (a.T + 31) / 32;
-    const float w = (float)((a.T + 7) / 8) * (float)nqt;  // the last tile's
-    const float total = (float)a.BH * w * (float)((nqt + 1) * (2 * nqt + 1)) / (float)(6 * nqt);  // a sum of squares
-    int best = 1;
-    float least = 3.0e38f;
-    for (int s : {1, 2, 3, 4, 6, 8, 12, 16}) {
-        const float t = std::max(1.5f * (kPart + w / (float)s), (float)wanted_roles(a) * (total + (float)(a.BH * nqt * s) * kPart) / kCus);
-        if (t < least) least = t, best = s;
-    }
-    return best;
-}
-
 // SV: the caller's tensors are strided views, read where they lie (the kernels' SV instantiations)
 template <typename E, int D, bool SV>
 static hipError_t launch_bwd(const MfmaBwdArgs& a, hipStream_t st) {
@@ -847,14 +795,25 @@ static hipError_t launch_bwd(const MfmaBwdArgs& a, hipStream_t st) {
     const bool all_in_f32 = a.causal && a.windowed && pairs <= 1024 && !a.split;
     const bool deal_f32 = all_in_f32 && a.BH * ((a.T + 31) / 32) < 512;
 
+    // The D = 64 kernel of this file takes windows that kk_left / kk_right do not cut (no pair inside the k1 and k2 windows
+    // of a query is further apart): its stages are the same for every round.  Training steps against the general kernel at
+    // equal splits: window 512 (B=2 H=4 T=2048) 6.4 -> 5.67 ms, 200 (B=1 H=4 T=1000) 520 -> 460 us, 128 (B=4 H=8 T=1024)
+    // 1.60 -> 1.55 ms.  A window of 64 is three steps, i.e. two stages of which one is half empty: 835 -> 868 us, so up to
+    // there the general kernel's 32-key stages stay.  With a k-k band of its own range of stages per round this kernel
+    // spills 100 bytes a lane and loses 10 to 40 %.
+    const bool kk_cuts = std::min(a.k2_window, a.T - 1) > a.kk_right || std::min(a.k1_window, a.T - 1) > a.kk_left;
+    const bool general_window = a.windowed && (D == 128 || kk_cuts || std::min(a.k1_window, a.k2_window) <= 64);
+
     // A workgroup owns a 32-query tile and walks all of its rows.  When that leaves most of the chip idle, or
     // ends in a long tail (few heads, short sequences), the rows of a tile are dealt out to several
     // workgroups, and dQ is accumulated in fp32 like the row gradients.
     const int tiles = 8 * ((a.BH + 7) / 8) * ((a.T + 31) / 32);
+    const int roles = (a.dq || a.dk2 || a.dv2 ? 1 : 0) + (a.dk1 || a.dv1 ? 1 : 0);
+    const BwdPartsCall call{a.BH, a.T, a.k1_window, a.k2_window, a.kk_left, a.kk_right, std::max(1, roles), !general_window};
     int splits = 1;
     if (all_in_f32) splits = deal_f32 ? 2 : 1;  // (an accumulator for dQ, or none)
-    else if (D == 64 && a.windowed && !a.split) splits = windowed_splits(a);
-    else if (D == 64 && a.causal && !a.split && tiles < 1024) splits = causal_splits(a);
+    else if (D == 64 && a.windowed && !a.split) splits = windowed_parts(call);
+    else if (D == 64 && a.causal && !a.split && tiles < 1024) splits = causal_parts(call);
     // (D = 32 with split operands: workgroups of half the size, three to a CU.  B=2 H=8 T=512, training step: 4 / 6 / 8 / 12 / 16
     // parts 1112 / 984 / 977 / 958 / 958 us; B=2 H=4 T=256, 4 / 8 / 16 parts 283 / 187 / 135; 704 tiles, 2 to 12 parts: 4.40-4.48 ms)
     else if (tiles < 1024) splits = std::min(16, ((D == 32 && a.split ? 3072 : 1024) + tiles - 1) / tiles);
@@ -898,14 +857,6 @@ static hipError_t launch_bwd(const MfmaBwdArgs& a, hipStream_t st) {
     void (*kern_both)(BothRoles<E>) = nullptr;  // both roles in one grid
     int nthreads = 512, col_parts = 1;
     bool plain64 = false;  // the D = 64 kernel of this file
-    // The D = 64 kernel of this file takes windows that kk_left / kk_right do not cut (no pair inside the k1 and k2 windows
-    // of a query is further apart): its stages are the same for every round.  Training steps against the general kernel at
-    // equal splits: window 512 (B=2 H=4 T=2048) 6.4 -> 5.67 ms, 200 (B=1 H=4 T=1000) 520 -> 460 us, 128 (B=4 H=8 T=1024)
-    // 1.60 -> 1.55 ms.  A window of 64 is three steps, i.e. two stages of which one is half empty: 835 -> 868 us, so up to
-    // there the general kernel's 32-key stages stay.  With a k-k band of its own range of stages per round this kernel
-    // spills 100 bytes a lane and loses 10 to 40 %.
-    const bool kk_cuts = std::min(a.k2_window, a.T - 1) > a.kk_right || std::min(a.k1_window, a.T - 1) > a.kk_left;
-    const bool general_window = a.windowed && (D == 128 || kk_cuts || std::min(a.k1_window, a.k2_window) <= 64);
     if constexpr (D == 32) {
         // the banded instantiation for every mask (full windows are windows of T)
         constexpr int NW = bwdg_waves_d32(false), NS = bwdg_waves_d32(true);

@@ -1,0 +1,75 @@
+"""The rules that choose how many workgroups share a query tile of the 16-bit triple-dot backward at D = 64 (csrc/bwd_parts.hpp), on
+the CPU: what they choose against times measured for every count, training steps in us on MI355X, bf16, counts 1 2 3 4 6 8 12 16."""
+import ctypes
+import os
+import shutil
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "flash-3-way-attention_amd", "csrc")
+COUNTS = (1, 2, 3, 4, 6, 8, 12, 16)
+# ((B, H, T, window, k-k band on either side or 0), times)
+LAUNCHES = [  # a launch per role: windows up to 64 and those that a k-k band cuts
+    ((1, 2, 512, 200, 50), (445.7, 291.6, 236.3, 207.8, 169.5, 156.7, 172.6, 164.6)),
+    ((1, 2, 512, 400, 100), (1030, 579.0, 447.1, 372.8, 293.6, 255.5, 214.9, 221.2)),
+    ((1, 2, 1999, 50, 0), (200.0, 150.1, 181.1, 160.1, 170.8, 201.7, 202.0, 205.6)),
+    ((1, 2, 1999, 100, 25), (263.4, 191.1, 228.6, 209.3, 207.6, 243.4, 244.1, 246.7)),
+    ((1, 4, 300, 100, 25), (253.9, 178.3, 149.8, 140.2, 119.8, 123.2, 127.2, 126.4)),
+    ((1, 4, 300, 200, 50), (446.2, 293.1, 237.0, 208.0, 169.9, 157.1, 165.5, 166.6)),
+    ((1, 8, 700, 64, 16), (181.7, 195.5, 167.6, 186.1, 187.0, 220.8, 224.1, 229.2)),
+    ((1, 8, 700, 100, 25), (264.5, 293.0, 231.9, 272.4, 247.9, 289.7, 290.3, 297.6)),
+    ((1, 8, 700, 200, 50), (520.3, 506.8, 435.3, 460.3, 432.8, 450.3, 476.1, 488.5)),
+    ((1, 8, 2048, 400, 100), (2588, 2662, 2558, 2677, 2546, 2687, 2755, 2871)),
+    ((2, 8, 300, 100, 25), (262.4, 194.0, 217.6, 214.0, 222.5, 240.5, 243.4, 256.0)),
+    ((2, 8, 1000, 200, 50), (1083, 1130, 1077, 1174, 1140, 1228, 1304, 1361)),
+    ((4, 8, 200, 100, 25), (268.7, 232.3, 235.7, 246.5, 258.3, 280.7, 285.8, 303.3)),
+    ((4, 8, 1024, 200, 50), (2042, 2014, 2014, 2220, 2141, 2323, 2488, 2602)),
+    ((4, 16, 600, 400, 100), (3889, 3959, 4024, 4324, 4183, 4386, 4559, 4753)),
+]
+ONE_GRID = [  # both roles in one grid
+    ((1, 2, 512, 200, 0), (327.2, 210.9, 168.0, 151.4, 163.4, 148.6, 160.4, 155.7)),
+    ((1, 2, 1999, 200, 0), (421.2, 411.8, 418.1, 443.3, 432.4, 462.7, 515.0, 499.6)),
+    ((1, 4, 300, 100, 0), (203.5, 144.6, 123.3, 120.8, 122.3, 125.5, 123.2, 129.5)),
+    ((1, 4, 1500, 100, 0), (331.8, 296.4, 294.0, 320.4, 310.2, 370.8, 358.9, 362.2)),
+    ((1, 8, 700, 512, 0), (1354, 1130, 1141, 1141, 1154, 1166, 1186, 1218)),
+    ((1, 8, 2048, 512, 0), (5658, 5298, 5235, 5272, 5338, 5375, 5450, 5693)),
+    ((2, 8, 300, 200, 0), (371.9, 329.2, 328.3, 333.9, 337.3, 356.5, 390.7, 387.5)),
+    ((2, 8, 2048, 300, 0), (4998, 5201, 5108, 5102, 5053, 5403, 5530, 5674)),
+    ((4, 8, 1024, 200, 0), (2491, 2565, 2584, 2753, 2702, 2886, 3269, 3183)),
+    ((4, 16, 600, 512, 0), (6355, 6527, 6535, 6518, 6601, 6705, 6871, 7075)),
+]
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    cxx = shutil.which("g++") or shutil.which("c++")
+    if cxx is None:
+        pytest.skip("no C++ compiler")
+    at = tmp_path_factory.mktemp("parts")
+    (at / "rules.cpp").write_text(
+        '#include "bwd_parts.hpp"\n'
+        'extern "C" int windowed(int BH, int T, int w, int kk, int roles, int one_grid) {\n'
+        '    return tritt::windowed_parts({BH, T, w, w, kk, kk, roles, one_grid != 0});\n}\n')
+    subprocess.run([cxx, "-O1", "-std=c++17", "-shared", "-fPIC", "-I", CSRC, str(at / "rules.cpp"), "-o", str(at / "rules.so")], check=True)
+    return ctypes.CDLL(str(at / "rules.so"))
+
+
+def _against_best(times, parts):
+    return times[COUNTS.index(parts)] / min(times)
+
+
+@pytest.mark.parametrize("table,one_grid,most,mean", [(LAUNCHES, 0, 1.2, 1.06), (ONE_GRID, 1, 1.1, 1.03)])
+def test_parts_under_a_window(rules, table, one_grid, most, mean):
+    """The models are coarse (up to a fifth off where a launch is a few rounds); the one of the other kind of launch misses the bars."""
+    lost = [_against_best(times, rules.windowed(B * H, T, w, kk or T, 2, one_grid)) for (B, H, T, w, kk), times in table]
+    assert max(lost) <= most and sum(lost) / len(lost) <= mean, lost
+    wrong = [_against_best(times, rules.windowed(B * H, T, w, kk or T, 2, 1 - one_grid)) for (B, H, T, w, kk), times in table]
+    assert max(wrong) > most or sum(wrong) / len(wrong) > mean, wrong
+
+
+def test_wanted_roles_count_in_one_grid_alone(rules):
+    """A backward that wants the gradients of one role fills half of the common grid and needs more parts; a launch per role does not change."""
+    for (B, H, T, w, kk), _ in LAUNCHES + ONE_GRID:
+        assert rules.windowed(B * H, T, w, kk or T, 1, 0) == rules.windowed(B * H, T, w, kk or T, 2, 0)
+    assert rules.windowed(8, 2048, 512, 2048, 1, 1) > rules.windowed(8, 2048, 512, 2048, 2, 1)
