@@ -42,13 +42,15 @@ inline int windowed_parts(const BwdPartsCall& a) {
     return best;
 }
 
-// Under a full causal mask, for grids of less than 1024 tiles (both roles in one grid).  The work of a tile grows
-// with the square of its position and the heaviest parts start first, so the grid of both roles takes the longer of the even
-// share of all parts over the CUs and of its longest part (which starts late by what the parts before it differ, and shares
-// the chip with the other role's: 1.5).  Work in 32-key steps of eight rows; a part's own prologue, dQ's shares and tail are
-// worth about twelve of them.  Training steps, the parts it chooses (the best otherwise): B=2 H=4 T=256 6 parts 141 us (2 to 16: 190 151
-// 144 141 145 152 154), B=4 H=8 T=128 2 parts 130 us, T=256 2 parts 402, B=2 H=8 T=300 3 parts 337, B=1 H=2 T=128 100 us, all the
-// best; B=1 H=4 T=512 8 parts 330 (12 parts 329), B=1 H=8 T=1000 3.49 ms (6 parts 3.48), B=1 H=16 T=700 2.47 ms (3 parts 2.45).
+// Under a full causal mask, for grids of less than 1024 tiles (both roles in one grid).  The work of a tile grows with the square
+// of its position and the heaviest parts start first, so the grid of both roles takes the even share of all parts over the CUs
+// and 0.3 of its longest part of tail, and no less than 1.5 of its longest part (which starts late by what the parts before it
+// differ, and shares the chip with the other role's).  Work in 32-key steps of eight rows; a part's own prologue, dQ's shares and
+// tail are worth about twelve of them.  Training steps, the parts it chooses and the best: B=2 H=4 T=256 6 parts 144 us (1 to 16: 298
+// 190 150 145 144 147 155 156), B=4 H=8 T=128 2 parts 127, T=256 2 parts 376, B=1 H=2 T=1500 16 parts 2.84 ms, B=1 H=8 T=700 6
+// parts 1.22, all the best; B=1 H=2 T=512 12 parts 234 us (16: 229), B=4 H=8 T=64 3 parts 74 (4: 71), T=700 3 parts 4.94 ms (1: 4.86).
+// Without the tail (the longer of the two alone) B=1 H=8 T=700 took 3 parts and 1.26 ms, B=1 H=2 T=1500 6 parts and 2.98, B=2 H=8
+// T=1500 1 part and 21.4 (with it 6: 20.8; 2: 20.6).
 // D = 32 and 128 measure within 1 % of their best at 1024 workgroups.
 inline int causal_parts(const BwdPartsCall& a) {
     constexpr float kPart = 12.f;
@@ -59,7 +61,8 @@ inline int causal_parts(const BwdPartsCall& a) {
     int best = 1;
     float least = 3.0e38f;
     for (int s : {1, 2, 3, 4, 6, 8, 12, 16}) {
-        const float t = std::max(1.5f * (kPart + w / (float)s), (float)a.roles * (total + (float)(a.BH * nqt * s) * kPart) / kCus);
+        const float part = kPart + w / (float)s;
+        const float t = std::max(1.5f * part, (float)a.roles * (total + (float)(a.BH * nqt * s) * kPart) / kCus + 0.3f * part);
         if (t < least) least = t, best = s;
     }
     return best;

@@ -40,6 +40,34 @@ ONE_GRID = [  # both roles in one grid
     ((4, 16, 600, 512, 0), (6355, 6527, 6535, 6518, 6601, 6705, 6871, 7075)),
 ]
 
+CAUSAL = [  # (B, H, T), both roles in one grid
+    ((1, 2, 128), (123.9, 87.75, 76.87, 69.79, 65.09, 60.14, 60.16, 61.09)),
+    ((1, 2, 512), (876.4, 490.8, 362.2, 308.3, 249.9, 243.2, 233.5, 228.8)),
+    ((1, 2, 777), (1945, 1078, 787.4, 666.2, 606.8, 589.7, 570.4, 600.0)),
+    ((1, 2, 1500), (6918, 4099, 3327, 3274, 2981, 2879, 2888, 2844)),
+    ((1, 4, 256), (292.8, 181.4, 142.7, 126.9, 120.2, 112.9, 114.8, 114.3)),
+    ((1, 4, 1024), (3336, 2067, 1917, 1836, 1765, 1755, 1762, 1774)),
+    ((1, 4, 1659), (10478, 8297, 7445, 7394, 7278, 7219, 7215, 7165)),
+    ((1, 8, 64), (69.74, 57.37, 54.09, 53.81, 54.5, 54.38, 53.66, 53.87)),
+    ((1, 8, 128), (127.1, 90.89, 80.12, 72.67, 72.71, 75.32, 72.05, 76.11)),
+    ((1, 8, 256), (298.4, 190.4, 150.3, 145.1, 144.2, 147.4, 154.6, 156.3)),
+    ((1, 8, 700), (1762, 1326, 1263, 1224, 1220, 1256, 1254, 1293)),
+    ((1, 8, 1500), (12533, 10948, 10724, 10694, 10731, 10640, 10703, 10814)),
+    ((2, 8, 128), (131.0, 95.78, 94.54, 90.34, 92.7, 95.68, 99.26, 102.9)),
+    ((2, 8, 256), (325.6, 225.9, 226.1, 225.8, 236.6, 242.4, 259.9, 265.0)),
+    ((2, 8, 512), (1137, 1054, 1030, 1037, 1045, 1061, 1095, 1118)),
+    ((2, 8, 815), (4101, 3841, 3828, 3811, 3816, 3838, 3880, 3908)),
+    ((2, 8, 1500), (21375, 20634, 20703, 20637, 20758, 20687, 20797, 21266)),
+    ((4, 8, 64), (89.53, 77.96, 73.95, 71.53, 72.36, 77.78, 78.22, 79.11)),
+    ((4, 8, 128), (156.3, 126.7, 135.2, 135.8, 139.3, 150.4, 153.7, 163.3)),
+    ((4, 8, 256), (387.8, 376.3, 387.3, 402.1, 414.9, 430.6, 462.6, 471.4)),
+    ((4, 8, 512), (2030, 1977, 1989, 2038, 2041, 2082, 2156, 2198)),
+    ((4, 8, 700), (4855, 4954, 4939, 4935, 4968, 4973, 5068, 5071)),
+    ((4, 16, 64), (118.0, 108.6, 114.5, 112.1, 113.1, 122.7, 124.3, 125.4)),
+    ((4, 16, 128), (231.8, 242.8, 240.9, 246.4, 258.2, 283.0, 285.3, 309.1)),
+    ((4, 16, 256), (688.0, 712.4, 722.2, 748.7, 776.9, 813.0, 874.0, 890.6)),
+]
+
 
 @pytest.fixture(scope="module")
 def rules(tmp_path_factory):
@@ -50,7 +78,8 @@ def rules(tmp_path_factory):
     (at / "rules.cpp").write_text(
         '#include "bwd_parts.hpp"\n'
         'extern "C" int windowed(int BH, int T, int w, int kk, int roles, int one_grid) {\n'
-        '    return tritt::windowed_parts({BH, T, w, w, kk, kk, roles, one_grid != 0});\n}\n')
+        '    return tritt::windowed_parts({BH, T, w, w, kk, kk, roles, one_grid != 0});\n}\n'
+        'extern "C" int causal(int BH, int T, int roles) { return tritt::causal_parts({BH, T, T, T, T, T, roles, true}); }\n')
     subprocess.run([cxx, "-O1", "-std=c++17", "-shared", "-fPIC", "-I", CSRC, str(at / "rules.cpp"), "-o", str(at / "rules.so")], check=True)
     return ctypes.CDLL(str(at / "rules.so"))
 
@@ -73,3 +102,8 @@ def test_wanted_roles_count_in_one_grid_alone(rules):
     for (B, H, T, w, kk), _ in LAUNCHES + ONE_GRID:
         assert rules.windowed(B * H, T, w, kk or T, 1, 0) == rules.windowed(B * H, T, w, kk or T, 2, 0)
     assert rules.windowed(8, 2048, 512, 2048, 1, 1) > rules.windowed(8, 2048, 512, 2048, 2, 1)
+
+
+def test_parts_under_a_causal_mask(rules):
+    lost = [_against_best(times, rules.causal(B * H, T, 2)) for (B, H, T), times in CAUSAL]
+    assert max(lost) <= 1.035 and sum(lost) / len(lost) <= 1.01, lost
