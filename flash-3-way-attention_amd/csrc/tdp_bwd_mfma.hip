@@ -622,8 +622,13 @@ __device__ __forceinline__ void bwd_prep_block(const BwdPrep<E>& p, int bx, int 
             transpose_load<E, false, NT>(slice(p.v2, p.at_v2), nullptr, lds + kPrepTile, j0, T, D, p.at_v2.st);
         }
         __syncthreads();
-        transpose_store<E, NT>((job == 0 ? p.ut : p.k2t) + tbase, lds, j0, Tp, D);
-        transpose_store<E, NT>((job == 0 ? p.k1t : p.v2t) + tbase, lds + kPrepTile, j0, Tp, D);
+        if (job == 0) {  // (a destination chosen by the job goes through scratch: 24 bytes a lane)
+            transpose_store<E, NT>(p.ut + tbase, lds, j0, Tp, D);
+            transpose_store<E, NT>(p.k1t + tbase, lds + kPrepTile, j0, Tp, D);
+        } else {
+            transpose_store<E, NT>(p.k2t + tbase, lds, j0, Tp, D);
+            transpose_store<E, NT>(p.v2t + tbase, lds + kPrepTile, j0, Tp, D);
+        }
         return;
     }
     if (job == 2) {  // the accumulators: zero_width 4-byte words per row (D floats, or D 64-bit fixed-point sums)

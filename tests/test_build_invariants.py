@@ -19,13 +19,19 @@ def _checker():
     return mod.check
 
 
+_compiled = {}
+
+
 def _assembly(tmp_path, unit):
+    if unit in _compiled:
+        return _compiled[unit]
     out = tmp_path / "unit.s"
     flags = ["-O3", "-std=c++20", "--offload-arch=gfx950", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
              "-Wno-unused-command-line-argument", "--cuda-device-only", "-S"]
     subprocess.run([HIPCC, *flags, os.path.join(CSRC, unit), "-o", str(out)], check=True,
                    stderr=subprocess.DEVNULL, cwd=CSRC)
-    return out.read_text()
+    _compiled[unit] = out.read_text()
+    return _compiled[unit]
 
 
 @pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not available")
@@ -34,6 +40,16 @@ def test_direct_lds_loads_own_m0(tmp_path, unit):
     """The direct-to-LDS loads set M0 in inline assembly; nothing the compiler emits in those kernels may use M0, and
     the LDS waits must stay counted (csrc/check_m0.py states the conditions)."""
     assert _checker()(_assembly(tmp_path, unit)) is None
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not available")
+def test_passes_ahead_of_the_backward_use_no_scratch(tmp_path):
+    """The pass that prepares the triple-dot backward's operands is a copy: pointers that the compiler keeps in scratch memory and loads
+    back by an index cost it more than its registers ever would."""
+    kernels = re.findall(r"\.amdhsa_kernel (\S+)(.*?)\.end_amdhsa_kernel", _assembly(tmp_path, "tdp_bwd_mfma.hip"), re.S)
+    scratch = {name: int(re.search(r"\.amdhsa_private_segment_fixed_size (\d+)", body)[1])
+               for name, body in kernels if "bwd_prep" in name or "bwd_finish" in name}
+    assert len(scratch) == 10 and set(scratch.values()) == {0}, scratch
 
 
 @pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not available")
