@@ -951,15 +951,20 @@ static hipError_t launch_bwd(const MfmaBwdArgs& a, hipStream_t st) {
         if (f.tiles > 1) {
             launch_prep();
         } else {  // (also where every tile takes the fp32 kernel and there is one)
-            // One grid for this pass and the tile's statistics up to 2048 workgroups of the first (D = 128: 1024); there it has
-            // the chip's two waves per SIMD that the statistics' registers leave, which on large grids costs more than a launch.
-            // B=4 H=16 T=2048 D=32 window 40 (8192 of them) 1298 us as two, 1308 as one; the kernels alone, as two (without the gap between
-            // them) -> as one, at 512 / 1024 / 2048 workgroups, T=1024: D=32 20.2 -> 14.3 / 25.7 -> 14.1 / 25.8 -> 20.2 us,
-            // D=64 27.7 -> 17.7 / 29.2 -> 20.6 / 34.5 -> 34.2, D=128 34.3 -> 22.5 / 42.0 -> 28.3 / 65.7 -> 73.2.
+            // One grid for this pass and the tile's statistics saves the gap between two launches (3 to 4 us) and lets the pass use
+            // the CUs that the statistics leave idle.  What it costs: the pass runs in workgroups of the statistics' registers and
+            // LDS, of which a CU holds two at D = 32 (121 registers), one at D = 64 (168) and 128 (154 KB).  So at D = 64 and 128
+            // the limit follows `idle`, the CUs that the statistics' last round leaves.  Backward, bf16, window 70, two launches -> one, D = 64:
+            // 64 slices (idle 0) T=128 (512 workgroups of the pass) 178.7 -> 179.3 us, T=512 (2048) 656 -> 659; 128 slices (0) T=128 (1024)
+            // 315 -> 320; 56 (32) T=200 (896) 274 -> 273, T=512 (1792) 605 -> 610; 80 (192) T=200 (1280) 380 -> 371; 32 (128) T=1024
+            // (2048) 682 -> 681, T=2048 (4096) 1345 -> 1351.  D = 128: 64 slices (0) T=48 (256) 190 -> 187, T=128 (512) 394 -> 401; 120
+            // (32) T=48 (480) 322 -> 321, T=128 (960) 713 -> 730; 32 (128) T=512 (1024) 873 -> 865, T=1024 (2048) 1693 -> 1694; 8 (224)
+            // T=2048 (1024) 875 -> 859.  D = 32: 32 slices T=1024 (2048) 511 -> 503, 64 T=2048 (8192) 1655 -> 1673.
             t0_rounds = tile0_rounds(f);
             const int stats_x = 8 * xcd_slots(a.BH, 1), prep_blocks = Tp / 64 * a.BH * kPrepJobs;
+            const int idle = 255 - (stats_x * t0_rounds + 255) % 256, limit = std::min(2048, D == 32 ? 2048 : D == 64 ? 512 + 12 * idle : 384 + 5 * idle);
             constexpr size_t stats_smem = f32_stats_smem<D, kF32Waves>();
-            if (prep_blocks <= (D == 128 ? 1024 : 2048)) {
+            if (prep_blocks <= limit) {
                 auto kern = bwd_prep_stats_kernel<E, D>;
                 constexpr size_t prep_smem = std::max(stats_smem, 2 * kPrepTile * sizeof(E));
                 if (hipError_t e = ensure_dynamic_smem(reinterpret_cast<const void*>(kern), prep_smem); e != hipSuccess) return e;

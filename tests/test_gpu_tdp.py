@@ -1460,10 +1460,11 @@ def test_backward_d32_shapes_of_a_workgroup(B, H, T, windows, splits, dtype, tun
 
 @pytest.mark.parametrize("B,H,T,D,windows,split", [
     (1, 3, 1, 32, (None,) * 4, False), (2, 5, 31, 32, (200, 32, 62, 5), False), (1, 2, 32, 64, (None,) * 4, False), (1, 2, 33, 64, (8, 8, 2, 2), False),
-    (1, 3, 65, 128, (None,) * 4, False), (2, 4, 97, 32, (None,) * 4, True), (129, 4, 33, 32, (None,) * 4, False), (65, 8, 40, 128, (None,) * 4, False)])
+    (1, 3, 65, 128, (None,) * 4, False), (2, 4, 97, 32, (None,) * 4, True), (129, 4, 33, 32, (None,) * 4, False), (65, 8, 40, 128, (None,) * 4, False),
+    (8, 8, 128, 64, (None,) * 4, False), (8, 8, 129, 64, (None,) * 4, False), (8, 8, 65, 128, (None,) * 4, False)])
 def test_statistics_of_the_first_queries(B, H, T, D, windows, split):
-    """The fp32 statistics of query tile 0 ride in the grid of the backward's first pass (up to 2048 workgroups of it, 1024 at D = 128; the last two
-    shapes pass that) and stage V1 instead of SiLU(V1): one tile and several, narrow masks that leave every tile to the fp32 kernel, split operands, dense
+    """The fp32 statistics of query tile 0 ride in the grid of the backward's first pass (up to 2048 workgroups of it, at D = 64 and 128
+    fewer where they leave no CU idle; the last five shapes but (8, 8, 128, 64) pass the limit) and stage V1 instead of SiLU(V1): one tile and several, narrow masks that leave every tile to the fp32 kernel, split operands, dense
     tensors and slices of one projection.  Oracle: the first two and the last slice."""
     from flash_trittention import flash_trittention
 
