@@ -814,11 +814,12 @@ static hipError_t launch_bwd(const MfmaBwdArgs& a, hipStream_t st) {
     // workgroups, and dQ is accumulated in fp32 like the row gradients.
     const int tiles = 8 * ((a.BH + 7) / 8) * ((a.T + 31) / 32);
     const int roles = (a.dq || a.dk2 || a.dv2 ? 1 : 0) + (a.dk1 || a.dv1 ? 1 : 0);
-    const BwdPartsCall call{a.BH, a.T, a.k1_window, a.k2_window, a.kk_left, a.kk_right, std::max(1, roles), !general_window};
+    const BwdPartsCall call{a.BH, a.T, a.k1_window, a.k2_window, a.kk_left, a.kk_right, std::max(1, roles)};
     int splits = 1;
     if (all_in_f32) splits = deal_f32 ? 2 : 1;  // (an accumulator for dQ, or none)
-    else if (D == 64 && a.windowed && !a.split) splits = windowed_parts(call);
-    else if (D == 64 && a.causal && !a.split && tiles < 1024) splits = causal_parts(call);
+    else if (D == 64 && a.windowed && !a.split) splits = general_window ? launch_parts(call) : one_grid_parts(call);
+    // (D = 32 and 128 under a causal mask measure within 1 % of their best at 1024 workgroups)
+    else if (D == 64 && a.causal && !a.split && tiles < 1024) splits = one_grid_parts(call);
     // (D = 32 with split operands: workgroups of half the size, three to a CU.  B=2 H=8 T=512, training step: 4 / 6 / 8 / 12 / 16
     // parts 1112 / 984 / 977 / 958 / 958 us; B=2 H=4 T=256, 4 / 8 / 16 parts 283 / 187 / 135; 704 tiles, 2 to 12 parts: 4.40-4.48 ms)
     else if (tiles < 1024) splits = std::min(16, ((D == 32 && a.split ? 3072 : 1024) + tiles - 1) / tiles);
