@@ -1220,14 +1220,19 @@ hipError_t run_bwd(const MfmaDpsArgs& a, hipStream_t st) {
     if constexpr (kTiles) {
         o.term = (const float*)(ws + l.row_term);
         i.term = (const float*)(ws + l.key_term);
-        // 128 rows per workgroup (a wave per owner tile) on large grids, 64 (two waves share an owner tile) on small ones:
-        // the first fetch half as much from L2 and join nothing, the second are twice as many and level out better.  From 512
-        // to 1023 workgroups of 128 rows the grid is resident at once, so the longer the sequence, the more its longest
-        // blocks stand out.  Training steps, bf16, 64 rows -> 128: B=4 H=8 T=1024 (256 workgroups) 112 -> 145 us, B=8 H=16
-        // T=500 (512) 162 -> 157, B=1 H=8 T=8192 k_diff 2048 (512) 583 -> 600, D = 32 487 -> 518, B=8 H=16 T=1024 (1024)
-        // 422 -> 358, T=2048 1209 -> 985.
+        // 128 rows per workgroup (a wave per owner tile) on large grids, 64 (two waves share an owner tile) on small ones: the first
+        // fetch half as much from L2 and join nothing, the second are twice as many and level out better.  At D = 64 two workgroups
+        // fit a CU: 512 of 128 rows are the whole first launch at once, which then lasts as long as its longest blocks, and the
+        // more so the longer the sequence; from about 700 on their order levels it.  At D = 32 three fit and the fetches are half as
+        // much, so the line lies higher.  The backward alone, bf16, 64 rows -> 128 (workgroups of 128 rows), D = 64: B=4 H=8 T=1024 (256) 80 -> 91 us, B=4 H=16
+        // T=700 (384) 98 -> 97, T=1024 (512) 143 -> 135, B=2 H=16 T=2048 (512) 191 -> 185, T=3072 (768) 366 -> 351, B=1 H=16 T=4096
+        // (512) 303 -> 303, with k_diff 300 213 -> 218, T=6144 (768) 614 -> 592, B=1 H=8 T=8192 (512) 533 -> 545, T=9000 k_diff 300 (568)
+        // 390 -> 448, T=12288 (768) 1122 -> 1078, B=8 H=16 T=1024 (1024) 300 -> 274.  D = 32: B=8 H=16 T=500 (512) 68 -> 67, B=4 H=16
+        // T=1150 (576) 96 -> 100, T=1900 (960) 185 -> 181, B=2 H=16 T=2048 (512) 114 -> 120, k_diff 300 94 -> 102, T=3072 (768) 205 -> 209,
+        // T=4096 (1024) 337 -> 333, B=1 H=16 T=7600 (960) 533 -> 538, k_diff 300 330 -> 350.
         const long long blocks = (long long)a.BH * ((Tp / 32 + 3) / 4);
-        const bool wide = knobs().dps_shared ? knobs().dps_shared > 0 : blocks >= 1024 || (blocks >= 512 && a.T < 4096);
+        const int many = D == 64 ? (a.T < 4096 ? 512 : 700) : a.T < 800 ? 512 : a.T < 4096 ? 900 : 1024;
+        const bool wide = knobs().dps_shared ? knobs().dps_shared > 0 : blocks >= many;
         return wide ? launch_bwd_tiles<E, D, 4, 1, SV>(o, i, st) : launch_bwd_tiles<E, D, 2, 2, SV>(o, i, st);
     } else {
         o.kp2 = (const E*)(ws + l.k2p2); o.xp2 = (const E*)(ws + l.qp2); o.gp2 = (const E*)(ws + l.dop2); o.dr_p2 = (E*)(ws + l.drp2);

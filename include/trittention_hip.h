@@ -87,7 +87,7 @@ const char* tritt_status_string(int status);
  *                           tiles (a long and a short one), -1 = never
  *   TRITT_TUNE_DPS_SHARED   dot-product-sum on the 16-bit matrix cores: 1 = always the kernels whose workgroups own 128 rows
  *                           and share the streamed tiles through LDS, -1 = never (0: the forward passes from 1024 such
- *                           workgroups on, the backward from 512 on, at D <= 64 only below T = 4096 until 1024);
+ *                           workgroups on, the backward from 512 on, of long sequences at D <= 64 from 700 to 1024 on);
  *                           the backward at D <= 64 otherwise takes workgroups of 64 rows */
 enum { TRITT_TUNE_FWD_SPLITS = 0, TRITT_TUNE_FWD_BAND = 1, TRITT_TUNE_BWD_SPLITS = 2, TRITT_TUNE_BWD128_WAVES = 3,
        TRITT_TUNE_F32_VALU = 4, TRITT_TUNE_DPS_WAVES = 5, TRITT_TUNE_DPS_PAIR = 6, TRITT_TUNE_DPS_SHARED = 7,

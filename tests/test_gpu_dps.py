@@ -248,6 +248,22 @@ def test_large_grids_take_the_shared_tile_kernels(B, H, fwd_shared, tune):
             util.assert_close(name, a[b:b + 1, h:h + 1], ref, **LOWP)
 
 
+@pytest.mark.parametrize("B,H,T,D,wide", [(1, 16, 4096, 64, False), (2, 16, 2048, 64, True), (1, 16, 5700, 64, True), (2, 16, 2048, 32, False),
+                                          (8, 16, 500, 32, True), (4, 16, 1793, 32, True), (1, 16, 7600, 32, False)])
+def test_rows_of_a_backward_workgroup_by_default(B, H, T, D, wide, tune):
+    """Backward workgroups own 128 rows from 512 of them on, but at D = 64 from 700 on where T >= 4096 and at D = 32 from 900 on where T >= 800, from
+    1024 on where T >= 4096.  Below 1024 the forward passes are those of the knob at -1, and a backward of 64 rows is bit for bit what that gives."""
+    from flash_trittention import _lib
+
+    print(f"case dps default rows {B, H, T, D}", flush=True)
+    inputs = orc.make_inputs(B, H, T, D, torch.bfloat16, seed=T)
+    default = util.run_dps(inputs, D ** -0.5, True, 200)
+    tune(_lib.TUNE_DPS_SHARED, -1)
+    forced = util.run_dps(inputs, D ** -0.5, True, 200)
+    assert torch.equal(default[0], forced[0]) and torch.equal(default[1], forced[1])
+    assert all(torch.equal(a, b) for a, b in zip(default[2], forced[2])) == (not wide)
+
+
 def test_rejects_mismatched_shapes():
     from flash_trittention import TrittentionTriton
 
