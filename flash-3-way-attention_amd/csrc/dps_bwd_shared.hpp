@@ -106,9 +106,9 @@ __global__ __launch_bounds__(64 * kW, 2) void attn_bwd_row_shared_kernel(AttnBwd
             dp[i] = 0.f;
         }
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) s = M::mma(*reinterpret_cast<const v8*>(st + ks * 1024 + p1_piece(lane, ks) * 16), xb[ks], s);
+        for (int ks = 0; ks < KS; ++ks) s = M::mma(*reinterpret_cast<const v8*>(st + ks * 1024 + p1_piece<D>(lane, ks) * 16), xb[ks], s);
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) dp = M::mma(*reinterpret_cast<const v8*>(st + (KS + ks) * 1024 + p1_piece(lane, ks) * 16), gb[ks], dp);
+        for (int ks = 0; ks < KS; ++ks) dp = M::mma(*reinterpret_cast<const v8*>(st + (KS + ks) * 1024 + p1_piece<D>(lane, ks) * 16), gb[ks], dp);
         float b[16];
         if constexpr (BIAS) {
             tile_vector(reinterpret_cast<const float*>(st + S::CH * 1024 + wave * 256), g, b);
@@ -258,9 +258,9 @@ __global__ __launch_bounds__(64 * kW, 1) void attn_bwd_col_shared_kernel(AttnBwd
             dp[i] = 0.f;
         }
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) s = M::mma(*reinterpret_cast<const v8*>(st + ks * 1024 + p1_piece(lane, ks) * 16), kb[ks], s);
+        for (int ks = 0; ks < KS; ++ks) s = M::mma(*reinterpret_cast<const v8*>(st + ks * 1024 + p1_piece<D>(lane, ks) * 16), kb[ks], s);
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) dp = M::mma(*reinterpret_cast<const v8*>(st + (KS + ks) * 1024 + p1_piece(lane, ks) * 16), vbv[ks], dp);
+        for (int ks = 0; ks < KS; ++ks) dp = M::mma(*reinterpret_cast<const v8*>(st + (KS + ks) * 1024 + p1_piece<D>(lane, ks) * 16), vbv[ks], dp);
         float ls[16], dl[16];
         tile_vector(reinterpret_cast<const float*>(st + S::CH * 1024 + wave * 256), g, ls);
         tile_vector(reinterpret_cast<const float*>(st + S::CH * 1024 + (kW + wave) * 256), g, dl);

@@ -114,7 +114,7 @@ __global__ __launch_bounds__(64 * kW, 2) void attn_fwd_shared_kernel(AttnFwdP<E,
         for (int i = 0; i < 16; ++i) s[i] = 0.f;
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks)
-            s = M::mma(*reinterpret_cast<const v8*>(st + ks * 1024 + p1_piece(lane, ks) * 16), xb[ks], s);
+            s = M::mma(*reinterpret_cast<const v8*>(st + ks * 1024 + p1_piece<D>(lane, ks) * 16), xb[ks], s);
         float b[16];
         if constexpr (BIAS) {
             const float* sb = reinterpret_cast<const float*>(st + S::CH * 1024 + wave * 256);

@@ -23,7 +23,7 @@
 // 16-byte pieces from 32 different rows costs one cache-line lookup per row, and that address
 // traffic, not MFMA or bandwidth, was what bound these kernels).  Two packings of a [T][D] tensor,
 // both in tiles of 32 rows and both exactly Tp x D elements:
-//   P1 (k-slots run along d; rows permuted by key_of_row):  [tile][ks][p1_piece(lane, ks)][8]
+//   P1 (k-slots run along d; rows permuted by key_of_row):  [tile][ks][p1_piece<D>(lane, ks)][8]
 //   P2 (k-slots run along the row index; "transposed use"): [tile][dt][kk][lane][8]
 // The prep kernel writes them for the inputs, the producing epilogues for W and dR.  Every output
 // element has one owner: no atomics, bitwise reproducible.
@@ -58,15 +58,18 @@ __device__ __forceinline__ int launch_tiles(int pair, int nt) { return pair ? (n
 __device__ __forceinline__ int owner_tiles(int pair, int nt, int tile) { return (pair && tile != nt - 1 - tile) ? 2 : 1; }
 __device__ __forceinline__ int owner_tile(int nt, int tile, int part) { return part ? nt - 1 - tile : tile; }
 
-// Packing P1 keeps the 16 bytes of an operand load's lane at piece p1_piece(lane, ks) of the k-step's block.  The order
+// Packing P1 keeps the 16 bytes of an operand load's lane at piece p1_piece<D>(lane, ks) of the k-step's block.  The order
 // inside a block is free as far as operand loads go (the 64 pieces are one kilobyte either way); this one lets the
-// transposed LDS reads of a packed tile (dps_bwd_tiles.hpp) touch every bank once.
-__device__ __forceinline__ int p1_piece(int lane, int ks) { return lane ^ ((lane >> 5) << 2) ^ ((ks & 1) << 3); }
+// transposed LDS reads of a packed tile (dps_bwd_tiles.hpp) touch every bank once.  At D = 128 nothing reads it that way.
+template <int D>
+__device__ __forceinline__ int p1_piece(int lane, int ks) {
+    return D > 64 ? lane : lane ^ ((lane >> 5) << 2) ^ ((ks & 1) << 3);
+}
 // element offsets of (row, d) in the two packings
 template <int D>
 __device__ __forceinline__ size_t p1_index(int row, int d) {
     const int lane = ((d >> 3) & 1) * 32 + row_of_key(row & 31);
-    return ((size_t)((row >> 5) * (D / 16) + (d >> 4)) * 64 + p1_piece(lane, d >> 4)) * 8 + (d & 7);
+    return ((size_t)((row >> 5) * (D / 16) + (d >> 4)) * 64 + p1_piece<D>(lane, d >> 4)) * 8 + (d & 7);
 }
 template <int D>
 __device__ __forceinline__ size_t p2_index(int row, int d) {
@@ -76,7 +79,7 @@ __device__ __forceinline__ size_t p2_index(int row, int d) {
 // the operand loads: lane's 16 bytes of (tile t, k-step ks) / (tile t, d-tile dt, half kk)
 template <typename E, int D>
 __device__ __forceinline__ const E* p1_at(const E* z, int t, int ks, int lane) {
-    return z + ((size_t)(t * (D / 16) + ks) * 64 + p1_piece(lane, ks)) * 8;
+    return z + (size_t)(t * (D / 16) + ks) * 512 + p1_piece<D>(lane, ks) * 8;
 }
 template <typename E, int D>
 __device__ __forceinline__ const E* p2_at(const E* z, int t, int dt, int kk, int lane) {
@@ -228,9 +231,16 @@ __global__ __launch_bounds__(64 * kW, 2) void attn_fwd_mfma_kernel(AttnFwdP<E, S
     // just consumed (each wave runs only a handful of tiles, so two dependent global round trips per
     // tile would be most of its time).
     v8 kn[KS], vn[DT][2];
+    // What is kept through the loop decides how many waves a SIMD holds: a lane's offset inside a tile is one number for even and
+    // one for odd k-steps, opaque (else the compiler keeps a pointer per k-step), and so is the thread's number after the loop.
+    // Registers at D = 32 / 64 / 128: 166 / 206 / 256 and scratch without, 126 / 166 / 232 with both.  Forward, bf16: B=1 H=8 T=8192
+    // k_diff 100 157 -> 146 us (D = 32 115 -> 105), B=2 H=8 T=500 17.1 -> 16.2, D = 128 B=4 H=8 T=1024 70.7 -> 66.1.
+    unsigned k_even = p1_piece<D>(lane, 0) * 16, k_odd = p1_piece<D>(lane, 1) * 16;
+    if constexpr (D <= 64) asm volatile("" : "+v"(k_even), "+v"(k_odd));
     auto fetch_k = [&](int t) {
+        const char* kt = reinterpret_cast<const char*>(KP) + (size_t)t * (KS * 1024);
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) kn[ks] = ld8<E>(p1_at<E, D>(KP, t, ks, lane));
+        for (int ks = 0; ks < KS; ++ks) kn[ks] = ld8<E>(reinterpret_cast<const E*>(kt + (D <= 64 && (ks & 1) ? k_odd : k_even) + ks * 1024));
     };
     auto fetch_v = [&](int t) {
 #pragma unroll
@@ -254,10 +264,11 @@ __global__ __launch_bounds__(64 * kW, 2) void attn_fwd_mfma_kernel(AttnFwdP<E, S
         }
     };
     const int t_first = a_lo / 32 + wave, t_last = a_hi / 32;
-    if (t_first <= t_last) {
-        fetch_k(t_first);
-        fetch_b(t_first);
-        fetch_v(t_first);
+    {
+        const int t = min(t_first, t_last);  // (also where the wave has no tile: no path leaves the registers without a value)
+        fetch_k(t);
+        fetch_b(t);
+        fetch_v(t);
     }
     for (int t = t_first; t <= t_last; t += kW) {
         const int a0 = t * 32;
@@ -327,7 +338,9 @@ __global__ __launch_bounds__(64 * kW, 2) void attn_fwd_mfma_kernel(AttnFwdP<E, S
     }
     spill_tiles<D>(sO, wave, acc, n, g);
     __syncthreads();
-    const int rr = tid & 31, dg = tid >> 5, row = r0 + rr;
+    int mtid = tid;
+    asm volatile("" : "+v"(mtid));  // none of the addresses below is formed ahead of the loop and kept through it
+    const int rr = mtid & 31, dg = mtid >> 5, row = r0 + rr;
     float mm = -INFINITY;
 #pragma unroll
     for (int w = 0; w < kW; ++w) mm = fmaxf(mm, sM[w * 32 + rr]);
@@ -345,8 +358,9 @@ __global__ __launch_bounds__(64 * kW, 2) void attn_fwd_mfma_kernel(AttnFwdP<E, S
         if (p.term) p.term[(size_t)bh * p.lse_stride + row] = lse * p.term_scale;
     }
 #pragma unroll
-    for (int c = dg; c < D / 8; c += 2 * kW) {  // 16-byte pieces dg, dg + 2 kW, ... of the row
-        const int d0 = 8 * c;
+    for (int i = 0; i < (D / 8 + 2 * kW - 1) / (2 * kW); ++i) {  // 16-byte pieces dg, dg + 2 kW, ... of the row
+        const int d0 = 8 * (dg + 2 * kW * i);
+        if (d0 >= D) break;
         float o[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) {

@@ -53,6 +53,17 @@ def test_passes_ahead_of_the_backward_use_no_scratch(tmp_path):
 
 
 @pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not available")
+def test_dot_product_sum_forward_keeps_its_waves(tmp_path):
+    """The dot-product-sum forward of small grids: a SIMD holds four of its waves at D = 32 (128 registers a lane), three at D = 64 (168) and two at
+    D = 128 (256), without scratch memory."""
+    kernels = re.findall(r"\.amdhsa_kernel (\S*attn_fwd_mfma_kernel\S*)(.*?)\.end_amdhsa_kernel", _assembly(tmp_path, "dps_mfma.hip"), re.S)
+    assert len(kernels) == 16
+    for name, body in kernels:
+        registers, scratch = (int(re.search(rf"\.amdhsa_{what} (\d+)", body)[1]) for what in ("next_free_vgpr", "private_segment_fixed_size"))
+        assert scratch == 0 and registers <= (128 if "Li32E" in name else 168 if "Li64E" in name else 256), (name, registers, scratch)
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not available")
 def test_buffer_loads_keep_their_offset_in_the_range_check(tmp_path):
     """The fp32 dot-product-sum kernels rely on buffer loads to return zeros for rows past the end of a head.  The range
     check of a raw buffer leaves the scalar offset out, so that offset is zero in every one of them."""
