@@ -1,6 +1,6 @@
 // Workgroups per query tile ("parts") of the 16-bit triple-dot backward at D = 64 under a causal mask, by the time that a launch
 // takes with s of them.  Host code alone, of plain numbers.  Work is counted in 32-key steps of eight rows; one workgroup fills a CU;
-// a part's own prologue, dQ's shares and tail are worth about nine steps.
+// a part's own prologue, dQ's shares and tail are worth about twelve steps beside the other role's parts, nine in a launch alone.
 #pragma once
 #include <algorithm>
 
@@ -14,14 +14,15 @@ struct BwdPartsCall {
 constexpr int kBwdParts[] = {1, 2, 3, 4, 6, 8, 12, 16};
 
 // Both roles in one grid (tdp_bwd_rows_kernel), heaviest tiles first, from tile 1 on (tile 0 takes the fp32 kernel).  It takes the
-// longest of: 1.1 of a heaviest part; the even share of all parts over the CUs and 0.2 of a heaviest part of tail; and, where many
+// longest of: 1.3 of a heaviest part; the even share of all parts over the CUs and 0.3 of a heaviest part of tail; and, where many
 // tiles cost the same, whole rounds of those.  Training steps, bf16, the parts it chooses (the best): B=2 H=4 T=256 6 parts 144 us (1
 // to 16: 298 190 150 145 144 147 155 156), B=4 H=8 T=128 2 parts 127, T=256 2 parts 376, B=1 H=2 T=1500 16 parts 2.84 ms, B=1 H=8 T=700
-// 6 parts 1.22, B=2 H=4 T=2048 window 512 3 parts 5.23, B=4 H=8 T=1024 window 200 1 part 2.49, B=1 H=8 T=90 window 70 6 parts 70 us, T=128
-// window 100 6 parts 97; B=1 H=2 T=512 12 parts 234 (16: 229), B=6 H=8 T=160 window 70 1 part 231 (2: 221), B=1 H=2 T=512 window 200
-// 6 parts 163 (8: 149).  Over 190 shapes it is 0.6 % from the best in the mean.
+// 6 parts 1.22, B=2 H=4 T=2048 window 512 3 parts 5.23, B=4 H=8 T=1024 window 200 1 part 2.49, B=1 H=8 T=90 window 70 8 parts 71 us (6:
+// 70), T=128 window 100 6 parts 97; B=1 H=2 T=512 12 parts 234 (16: 229), B=6 H=8 T=160 window 70 1 part 231 (2: 221), B=2 H=8 T=1000
+// window 200 1 part 1.40 ms (2: 1.35), B=1 H=2 T=512 window 200 6 parts 163 us (8: 149).  Over 190 shapes it is 0.6 % from the best in the
+// mean.  (A sum of squares in the place of the tiles' own work, and no tail, were 1.2 to 2.1 % from it and up to 16.)
 inline int one_grid_parts(const BwdPartsCall& a) {
-    constexpr float kPart = 9.f;
+    constexpr float kPart = 12.f;
     constexpr int kCus = 256;
     auto work = [&](int q0) {
         const int q1 = std::min(q0 + 31, a.T - 1);
@@ -44,8 +45,8 @@ inline int one_grid_parts(const BwdPartsCall& a) {
     for (int s : kBwdParts) {
         const float part = kPart + most / (float)s;
         const long long rounds = (a.roles * a.BH * full * s + kCus - 1) / kCus;
-        const float share = grid * (total + (float)((nqt - 1) * s) * kPart) / kCus + 0.2f * part;
-        const float t = std::max(std::max(1.1f * part, share), (float)rounds * part);
+        const float share = grid * (total + (float)((nqt - 1) * s) * kPart) / kCus + 0.3f * part;
+        const float t = std::max(std::max(1.3f * part, share), (float)rounds * part);
         if (t < least) least = t, best = s;
     }
     return best;
