@@ -11,8 +11,8 @@
 // 1260 cycles of a SIMD where its MFMAs take 512.  Timing-only ablations (B=1 H=8 T=8192, outer columns 168 us): no loads
 // 148, no barriers 153, no exp2 152, no transposed reads 157.  Reading the next rows a barrier earlier (246 registers instead
 // of 202) changed nothing.  Against one 32-row tile per workgroup with operands fetched per wave and the passes as launches of
-// their own (four-wave workgroups of 128 rows on large grids), training steps, bf16, D = 64: B=4 H=8 T=1024 142 -> 111 us, B=1
-// H=8 T=8192 k_diff 2048 786 -> 600; the three passes that depend on nothing of each other in one
+// their own (four-wave workgroups of 128 rows on large grids), training steps in turn, bf16, D = 64: B=4 H=8 T=1024 142 -> 110 us,
+// B=1 H=8 T=8192 k_diff 2048 795 -> 622 (both in workgroups of 64 rows); the three passes that depend on nothing of each other in one
 // grid instead of one after the other, and half the bytes per tile, are most of it.
 #pragma once
 

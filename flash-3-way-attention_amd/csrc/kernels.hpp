@@ -84,11 +84,11 @@ struct FirstTileArgs {
     // the other five lie where the caller has them: H heads per batch entry and these strides (H = 0: all dense)
     int H;
     TensorAt at_q, at_do, at_k1, at_k2, at_v2;
-    // scratch, [BH][T] floats each: the covered rows' LSE and Delta, recomputed in fp32 (tiles == 1: delta_f32 holds
-    // the per-round partials of tile 0 instead, [BH][32][4][3])
+    // tiles > 1: scratch, [BH][T] floats each: the covered rows' LSE and Delta, recomputed in fp32.  tiles == 1: delta_f32 holds the
+    // per-round partials of tile 0 instead, [BH][32][4][3], and is an input (see below)
     float *lse_f32, *delta_f32;
-    void* dq0_acc;                            // tiles == 1 and acc_q null: [BH][32][D] accumulator of the tile's dQ / alpha
-    void* dq;                                 // written when acc_q is null
+    void* dq0_acc;                            // tiles == 1 and acc_q null: [BH][32][D] accumulator of the tile's dQ / alpha, cleared
+    void* dq;                                 // tiles > 1 and acc_q null: written
     void *acc_k2, *acc_v2, *acc_k1, *acc_u;   // fixed point (long long) or float
     void* acc_q;                              // dQ / alpha accumulator of a split backward, or null
     // fixed-point accumulators (common.hpp): the slices' scale partials, the rows' poison words and the bias of the
@@ -103,6 +103,8 @@ struct FirstTileArgs {
     int tiles;
     bool deal_out;  // tiles > 1: the rounds of a query tile may be dealt out to workgroups
 };
+// tiles > 1: the statistics and the backward of the tiles.  tiles == 1: the backward alone; a launch ahead on the stream has run the
+// statistics with tile0_stats' parameters (tdp_f32_tiles.hpp), which leaves the partials in delta_f32 and clears dq0_acc.
 hipError_t f32_mfma_tdp_bwd_first_tile(const FirstTileArgs& a, hipStream_t st);
 // fp32 operands of the dot-product-sum kernels (two chained attention passes).
 struct DpsArgs {

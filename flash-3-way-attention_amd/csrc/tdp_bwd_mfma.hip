@@ -599,7 +599,7 @@ struct BwdPrep {
     const E *v1, *k1, *k2, *v2, *o, *d_o;
     E *u, *ut, *k1t, *k2t, *v2t;
     float *delta, *zero_a, *zero_b, *zero_c, *zero_d, *zero_e;
-    int T, Tp, BH, D, zero_width;
+    int T, Tp, D, zero_width;
     unsigned *scale_parts, *poison;
     const E* o_res;
     int H;
@@ -835,7 +835,7 @@ static hipError_t launch_bwd(const MfmaBwdArgs& a, hipStream_t st) {
     prep.u = (E*)(ws + l.u); prep.ut = (E*)(ws + l.ut); prep.k1t = (E*)(ws + l.k1t); prep.k2t = (E*)(ws + l.k2t); prep.v2t = (E*)(ws + l.v2t);
     prep.delta = (float*)(ws + l.delta);
     prep.zero_a = dk1acc; prep.zero_b = duacc; prep.zero_c = dk2acc; prep.zero_d = dv2acc; prep.zero_e = dqacc;
-    prep.T = a.T; prep.Tp = Tp; prep.BH = a.BH; prep.D = D; prep.zero_width = a.deterministic ? 2 * D : D;
+    prep.T = a.T; prep.Tp = Tp; prep.D = D; prep.zero_width = a.deterministic ? 2 * D : D;
     prep.scale_parts = a.deterministic ? (unsigned*)(ws + l.scale_parts) : nullptr; prep.poison = (unsigned*)(ws + l.poison);
     prep.o_res = a.split ? (const E*)a.o + (size_t)a.BH * a.T * D : nullptr;
     prep.H = SV ? a.H : 1;

@@ -117,7 +117,7 @@ struct F32StatsParams {
     float* lse;
     const E* d_o;
     float* delta;
-    // Query tile 0 alone, with its rounds dealt out to `split_rounds` workgroups (blockIdx.y): each writes its
+    // Query tile 0 alone, with its rounds dealt out to `split_rounds` workgroups (f32_stats_block's `round`): each writes its
     // partial (maximum, sum, sum_d dO * unnormalised O) to delta[((bh * 32 + q) * split_rounds + round) * 3 ..] and
     // the first one clears `zero_words` 4-byte words at zero_ptr + bh * zero_words
     int split_rounds;
