@@ -51,6 +51,11 @@ __host__ __device__ __forceinline__ float bwd_scale(float alpha) {
 // The streamed term comes divided by the scale and is what the score product starts from (the C operand, read from LDS
 // straight into the accumulator), so an exponent is one fused multiply-add; -Delta is what the dP product starts from.
 // NEG: the vector holds +LSE / scale; the owner's score operand and the scale are taken negative instead.
+// An exponent is thereby rounded two or three times at its terms' size where a sum formed ahead of the score is once or twice.  P's 16
+// bits hide that up to |LSE| of 2^12: against 64 bits errors are those of such a sum with operands 16 times normal ones, and with
+// one element of 1e4 in Q, K1 or K2 in bf16; in fp16 that element makes dV1 4.0e-4 instead of 3.4e-4, one of 6e4 1.8e-3 instead of
+// 0.9e-3 (a rounded LSE).  Forming the score products of such tiles once more from zero gives the latter figures; telling them apart
+// costs every workgroup a pass over the terms, 1 us and 1 to 5 % of a call of this package's sizes, and was taken back.
 template <typename E, int D, int kOT, int kSH, bool COL, bool BIAS, bool LINK, bool NEG, bool SV>
 __device__ __forceinline__ void attn_bwd_tiles_body(const AttnBwdP<E, SV>& p, int bh, int tile) {
     using M = Mma<E>;

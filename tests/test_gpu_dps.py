@@ -653,6 +653,31 @@ def test_backward_tiles(dtype, D, T, causal, k_diff, blocks, tune):
             util.assert_close(f"{name} at {alpha}", a, b.float().cpu(), **LOWP)
 
 
+@pytest.mark.parametrize("dtype,D", [(torch.float16, 32), (torch.float16, 64)])
+@pytest.mark.parametrize("blocks", [-1, 1])
+@pytest.mark.parametrize("which", [0, 1, 2])
+def test_large_scores_of_the_backward(which, blocks, dtype, D, tune):
+    """One element of 6e4 in Q, K1 or K2.  The backward's exponents are differences of numbers of the scores' size: dV1 and dV2, which depend on P
+    alone, stay as near 64 bits as roundings at that size allow (an ulp of LSE in the exponent, 2^-23 |LSE| of P relative, for each pass,
+    beside four roundings of 2^-11)."""
+    from flash_trittention import _lib
+
+    print(f"case dps large scores which={which} blocks={blocks} D={D}", flush=True)
+    tune(_lib.TUNE_DPS_SHARED, blocks)
+    T, alpha = 200, D ** -0.5
+    inputs = orc.make_inputs(1, 2, T, D, dtype, seed=D)
+    inputs[which][:, :, 100, 3] = 6e4
+    out, m, grads = util.run_dps(inputs, alpha, True, T, flags=_lib.FLAG_FORCE_MFMA)
+    lse = m.abs().max().item()
+    assert lse > 1e3
+    bar = 2 ** -9 + 2 * lse * 2.0 ** -23
+    for h in range(2):
+        _, _, want = orc.dps_forward_backward(*(t[0, h].double() for t in inputs), alpha, True, factorised=True)
+        for name, a, w in list(zip(util.NAMES, grads, want))[3:]:
+            err = ((a[0, h].double() - w).norm() / w.norm()).item()
+            assert err <= bar, (name, h, err, bar)
+
+
 @pytest.mark.parametrize("blocks", [-1, 1])
 def test_an_infinite_gradient_row_stays_in_its_tiles(blocks, tune):
     """One row of dO that is not finite reaches dQ of its own 32 rows and the key gradients of the tiles at and before it (the band limits
